@@ -112,6 +112,11 @@ void pl_set_error(const char* fmt, ...);
 // The compute units of the current device (launch-size choices go by it).
 int pl_compute_units();
 
+// The 32-bit product (gemm_f32.hip): y[n, N] = x[n, K] . w[N, K]^T, rows of x and y `ldx` and `ldy` values apart; `batch` of them,
+// whose operands and results begin `sx`, `sw` and `sy` values apart.
+int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, int ldx, int ldy, int batch, long sx,
+                long sw, long sy, hipStream_t stream);
+
 #define PL_REQUIRE(cond, ...)            \
     do {                                 \
         if (!(cond)) {                   \

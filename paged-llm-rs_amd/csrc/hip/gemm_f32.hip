@@ -1,0 +1,331 @@
+// y[n, N] = x[n, K] . w[N, K]^T of 32-bit operands on the matrix cores' 32-bit instruction (v_mfma_f32_16x16x4_f32): the
+// product of the true 32-bit path.  Operands, products and sums are 32-bit; nothing is rounded to fewer bits.
+//
+// A row's result does not depend on what else is in the batch, bit for bit, whichever of the kernels below runs: K is cut
+// into at most 16 parts by K alone, a part is one chain of matrix instructions from its first k to its last, and the parts
+// are added in ascending order.  (Inside 16 consecutive k an instruction takes k, k + 4, k + 8, k + 12: the four
+// consecutive values a lane holds are its operands of four instructions.)
+#include "common.hpp"
+
+#define PL_F32_PARTS 16
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// The length of a part: whole double steps of the tiled kernel, whole rounds of the kernel for few rows.
+static inline int f32_part_len(int K) { return pl_ceil_div(pl_ceil_div(K, PL_F32_PARTS), 64) * 64; }
+
+// The values k .. k + 3 of a row of K; past its end whatever stands at the end (f32_end clears it).  VEC: rows and K are
+// multiples of four values and the base is aligned.
+template <bool VEC>
+__device__ __forceinline__ f32x4 f32_load4(const float* row, int k, int K) {
+    if (VEC) return *reinterpret_cast<const f32x4*>(row + min(k, K - 4));
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = row[min(k + i, K - 1)];
+    return v;
+}
+
+__device__ __forceinline__ f32x4 f32_end(f32x4 v, int k, int K) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < K ? v[i] : 0.f;
+    return v;
+}
+
+// 16 k of TM tiles of 16 columns of w against TN tiles of 16 rows of x.
+template <int TM, int TN>
+__device__ __forceinline__ void f32_multiply(const f32x4 (&a)[TM], const f32x4 (&b)[TN], f32x4 (&acc)[TM][TN]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][q], b[j][q], acc[i][j], 0, 0, 0);
+}
+
+__device__ __forceinline__ void f32_store4(float* to, f32x4 v, int col, int N, bool whole) {
+    if (whole) {
+        if (col < N) *reinterpret_cast<f32x4*>(to) = v;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (col + q < N) to[q] = v[q];
+    }
+}
+
+// ---- few rows ----------------------------------------------------------------------------------------------------------------
+// Bound by the weights' bytes.  A workgroup of sixteen waves owns 16 columns and TN x 16 rows of x; a wave takes one part
+// of K straight from memory in the instruction's layout, 64 k a round, and the parts meet in LDS.  Also the product of many
+// rows whose rows are not made of aligned groups of four values (VEC false, a row tile a blockIdx.y).
+template <int TN, bool VEC>
+__global__ void __launch_bounds__(PL_F32_PARTS * PL_WAVE)
+gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int n, int N, int K,
+                    int ldx, int ldy, long sx, long sw, long sy, int part_len) {
+    constexpr int ROUND = TN > 2 ? 2 : 4;                               // steps of 16 k asked for together
+    __shared__ __attribute__((aligned(16))) float parts[PL_F32_PARTS][TN * 16][16];       // [part][row of x][column of w]
+    x += blockIdx.z * sx;
+    w += blockIdx.z * sw;
+    y += blockIdx.z * sy;
+    const int lane = threadIdx.x % PL_WAVE, wave = threadIdx.x / PL_WAVE;
+    const int r = lane % 16, c = lane / 16;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * TN * 16;
+    const float* wr = w + static_cast<size_t>(min(n0 + r, N - 1)) * K;
+    const float* xr[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) xr[j] = x + static_cast<size_t>(min(m0 + j * 16 + r, n - 1)) * ldx;
+
+    const int first = wave * part_len, last = min(K, first + part_len);
+    if (first < last) {
+        f32x4 acc[1][TN];
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[0][j] = zero;
+        f32x4 a[ROUND][1], b[ROUND][TN];
+        auto ask = [&](int k) {
+#pragma unroll
+            for (int u = 0; u < ROUND; ++u) {
+                a[u][0] = f32_load4<VEC>(wr, k + u * 16 + c * 4, K);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[u][j] = f32_load4<VEC>(xr[j], k + u * 16 + c * 4, K);
+            }
+        };
+        ask(first);
+        int k = first;
+        for (; k + ROUND * 16 < last; k += ROUND * 16) {
+            // (a step's registers are filled again as soon as it is multiplied; every load is unconditional, since a load in
+            // a branch would make the compiler wait for all that are on their way, and nothing past the part is asked for)
+#pragma unroll
+            for (int u = 0; u < ROUND; ++u) {
+                f32_multiply<1, TN>(a[u], b[u], acc);
+                const int next = k + (ROUND + u) * 16 + c * 4;
+                a[u][0] = f32_load4<VEC>(wr, next, K);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[u][j] = f32_load4<VEC>(xr[j], next, K);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < ROUND; ++u) {
+            if (k + u * 16 < last) {
+                a[u][0] = f32_end(a[u][0], k + u * 16 + c * 4, K);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[u][j] = f32_end(b[u][j], k + u * 16 + c * 4, K);
+                f32_multiply<1, TN>(a[u], b[u], acc);
+            }
+        }
+        // (a lane holds four columns of one row of x)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(&parts[wave][j * 16 + r][c * 4]) = acc[0][j];
+    }
+    __syncthreads();
+    const int used = (K + part_len - 1) / part_len;
+    const int row = threadIdx.x / 4, col = n0 + threadIdx.x % 4 * 4;       // four columns of one row
+    if (row < TN * 16 && m0 + row < n) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        for (int p = 0; p < used; ++p) sum += *reinterpret_cast<const f32x4*>(&parts[p][row][threadIdx.x % 4 * 4]);
+        const bool whole = N % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+        f32_store4(y + static_cast<size_t>(m0 + row) * ldy + col, sum, col, N, whole);
+    }
+}
+
+// ---- many rows ---------------------------------------------------------------------------------------------------------------
+// Bound by the matrix cores: a workgroup of four waves, two by two, owns TILE rows of x and TILE columns; 32 k a stage through
+// four stages of LDS, filled three steps ahead by loads that write LDS themselves (global_load_lds_dwordx4: a wave's load is
+// eight whole 128-byte pieces of rows).  Lane l of a load brings piece (l % 8) ^ (row % 8) of its row into slot l % 8, so that
+// the lanes that read one piece of eight rows find it in different banks.  What a step costs beside its products (1,024 cycles
+// at tiles of 64) is its barrier and what the addresses and the loads take to issue: with one workgroup a compute unit 1,024 x
+// 2,048 takes 41 us where the products alone take 27; 2,048 rows of 4,096 x 1,024 run at 113 TFLOP/s, and 104 to 125 in the
+// library's product.  Tiles of 128 run as fast as tiles of 64 there and leave more of the chip idle elsewhere, and operands
+// straight from L2 into registers (no LDS) half as fast: a compute unit's L1 then gives out each line twice.
+#define F32_BK 32
+#define F32_STAGES 4
+
+// 16 bytes a lane from `offset` bytes behind `base` (the same for the wave) to LDS, lane after lane from byte `to` on.  Assembly,
+// so that the compiler does not count the load and make every later read of LDS wait for all of them.
+__device__ __forceinline__ void f32_load_to_lds(const void* base, uint32_t offset, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(base) : "memory", "m0");
+}
+
+// K a multiple of 64 (two steps).
+template <int TILE>
+__global__ void __launch_bounds__(256)
+gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int n, int N, int K,
+                      int ldx, int ldy, long sx, long sw, long sy, int part_len, int row_tiles, int col_tiles) {
+    constexpr int TM = TILE / 32, TN = TM;                      // tiles of 16 a wave: columns, rows
+    constexpr int STAGE = 2 * TILE * F32_BK, LOADS = TILE / 16;
+    extern __shared__ __attribute__((aligned(16))) float f32_lds[];         // [stage][rows of x, then columns of w][32]
+    // Workgroups go to the eight XCDs in turn: an XCD gets whole columns of tiles, so that a row of w is read into one
+    // L2 only, and walks the rows of x first.
+    const int col_tile = blockIdx.x % 8 + 8 * (blockIdx.x / 8 / row_tiles), row_tile = blockIdx.x / 8 % row_tiles;
+    if (col_tile >= col_tiles) return;      // (the whole workgroup)
+    const int m0 = row_tile * TILE, n0 = col_tile * TILE;
+    const int lane = threadIdx.x % PL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PL_WAVE);
+    const int r = lane % 16, c = lane / 16;
+    y += blockIdx.z * sy;
+    const float* x0 = x + blockIdx.z * sx + static_cast<size_t>(m0) * ldx;
+    const float* w0 = w + blockIdx.z * sw + static_cast<size_t>(n0) * K;
+
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const float*)f32_lds));
+    uint32_t offset[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = (wave + 4 * i) * 8 + lane / 8;          // of the stage: rows of x for i < TN, columns of w behind them
+        const int piece = (lane % 8 ^ row % 8) * 4;
+        offset[i] = 4u * (i < TN ? static_cast<uint32_t>(min(row, n - 1 - m0)) * ldx + piece
+                                 : static_cast<uint32_t>(min(row - TILE, N - 1 - n0)) * K + piece);
+    }
+    const int steps = K / F32_BK;
+    auto ask = [&](int step) {              // (past the end: the last step again, so that the counts stay)
+        const int k = min(step, steps - 1) * F32_BK;
+        const uint32_t to = lds0 + (static_cast<uint32_t>(step) % F32_STAGES * STAGE + wave * 8 * F32_BK) * 4u;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) f32_load_to_lds((i < TN ? x0 : w0) + k, offset[i], to + i * 32 * F32_BK * 4u);
+    };
+    int a_at[2], b_at[2];                   // this lane's operands in a stage, for either half of a step
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int slot = ((c + 4 * h) ^ r % 8) * 4;
+        a_at[h] = (TILE + wave % 2 * TM * 16 + r) * F32_BK + slot;
+        b_at[h] = (wave / 2 * TN * 16 + r) * F32_BK + slot;
+    }
+    // The operands of a step are read out of LDS one step early, while the step before is multiplied: two sets of registers
+    // that take turns.
+    f32x4 a[2][2][TM], b[2][2][TN];         // [set][half of the step]
+    auto read = [&](int set, int step) {
+        const float* at = f32_lds + static_cast<uint32_t>(step) % F32_STAGES * STAGE;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[set][h][i] = *reinterpret_cast<const f32x4*>(at + a_at[h] + i * 16 * F32_BK);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[set][h][j] = *reinterpret_cast<const f32x4*>(at + b_at[h] + j * 16 * F32_BK);
+        }
+    };
+    f32x4 acc[TM][TN], total[TM][TN];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) total[i][j] = zero;
+    // One step.  The loads of the step after this one have landed in this wave (one later step's may be on their way); after
+    // the barrier every wave's have, and every wave has multiplied the step before, whose stage is filled next.
+    auto one_step = [&](int set, int step) {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | LOADS);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        ask(step + 3);
+        read(set ^ 1, step + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        f32_multiply<TM, TN>(a[set][0], b[set][0], acc);
+        f32_multiply<TM, TN>(a[set][1], b[set][1], acc);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ask(0);
+    ask(1);
+    ask(2);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | 2 * LOADS);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    const int part_steps = part_len / F32_BK;
+    for (int s0 = 0; s0 < steps; s0 += part_steps) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = zero;
+        const int stop = min(steps, s0 + part_steps);           // (both are even)
+        for (int s = s0; s < stop; s += 2) {
+            one_step(0, s);
+            one_step(1, s + 1);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) total[i][j] += acc[i][j];
+    }
+    // (the loads asked for past the end still write LDS: they have to have landed before the workgroup ends)
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    const bool whole = N % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int row = m0 + (wave / 2 * TN + j) * 16 + r;
+        if (row >= n) continue;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int col = n0 + (wave % 2 * TM + i) * 16 + c * 4;
+            f32_store4(y + static_cast<size_t>(row) * ldy + col, total[i][j], col, N, whole);
+        }
+    }
+}
+
+namespace {
+
+struct F32Product {
+    const float *x, *w;
+    float* y;
+    int n, N, K, ldx, ldy, batch;
+    long sx, sw, sy;
+};
+
+template <int TN, bool VEC>
+void launch_few(const F32Product& g, hipStream_t stream) {
+    const dim3 grid(pl_ceil_div(g.N, 16), pl_ceil_div(g.n, TN * 16), g.batch);
+    gemm_f32_few_kernel<TN, VEC><<<grid, PL_F32_PARTS * PL_WAVE, 0, stream>>>(g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw,
+                                                                              g.sy, f32_part_len(g.K));
+}
+
+template <int TILE>
+void launch_tiled(const F32Product& g, hipStream_t stream) {
+    constexpr size_t lds = sizeof(float) * F32_STAGES * 2 * TILE * F32_BK;
+    static_assert(lds <= 64 * 1024, "a workgroup's LDS");
+    const int row_tiles = pl_ceil_div(g.n, TILE), col_tiles = pl_ceil_div(g.N, TILE);
+    const dim3 grid(pl_ceil_div(col_tiles, 8) * 8 * row_tiles, 1, g.batch);
+    gemm_f32_tiled_kernel<TILE><<<grid, 256, lds, stream>>>(g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw, g.sy,
+                                                            f32_part_len(g.K), row_tiles, col_tiles);
+}
+
+}  // namespace
+
+// `batch` products, their operands and results sx, sw and sy values apart.  Which kernel: up to 16 rows the one for few rows,
+// whose workgroups hold all rows and read every weight once; against many columns its 16 columns a workgroup reads the rows
+// too often from nine rows on, and from 17 rows on earlier (us, few / tiles of 32: 16 rows, 6,144 x 1,024 12.2 / 12.8, 151,936 x
+// 1,024 172 / 141; 32 rows, 4,096 x 1,024 10.2 / 13.1, 6,144 x 1,024 17.0 / 12.9; 64 rows, 4,096 x 1,024 14.1 / 13.2).
+// Tiles of 64 rows by 64 columns or of 32 by 32: the shorter estimate for the compute unit with most of them, a small tile
+// costing 1.15 times as much for what it does (700 rows, tiles of 64 / 32: 1,024 x 2,048 43.7 / 34.7, 4,096 x 1,024 62.3 /
+// 59.5; 2,048 rows, 1,024 x 2,048 76.7 / 87.6, 4,096 x 1,024 152 / 178).
+int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, int ldx, int ldy, int batch, long sx,
+                long sw, long sy, hipStream_t stream) {
+    const F32Product g{x, w, y, n, N, K, ldx, ldy, batch, sx, sw, sy};
+    const bool vec = K % 4 == 0 && ldx % 4 == 0 && sx % 4 == 0 && sw % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    // (a row of a tile is addressed by 32 bits from the tile's first)
+    const bool tiles = vec && K % 64 == 0 && K < (1 << 22) && ldx < (1 << 22);
+    const long units = pl_compute_units();
+    const auto busiest = [&](int tile) {
+        return (static_cast<long>(pl_ceil_div(n, tile)) * pl_ceil_div(N, tile) * batch + units - 1) / units * tile * tile;
+    };
+    const bool few = n <= 8 || (n <= 16 && N < 32768) || (n <= 32 && N <= 4096);
+    PL_REQUIRE(static_cast<long>(pl_ceil_div(n, 32)) * (pl_ceil_div(N, 32) + 8) < (1L << 31) && pl_ceil_div(n, 64) <= 65535,
+               "gemm: %d x %d results are more than one launch covers", n, N);
+    if (few || !tiles) {
+        if (vec) {
+            if (n <= 16) launch_few<1, true>(g, stream);
+            else if (n <= 32) launch_few<2, true>(g, stream);
+            else launch_few<4, true>(g, stream);
+        } else if (n <= 16) {
+            launch_few<1, false>(g, stream);
+        } else {
+            launch_few<4, false>(g, stream);
+        }
+    } else if (busiest(64) * 20 <= busiest(32) * 23) {
+        launch_tiled<64>(g, stream);
+    } else {
+        launch_tiled<32>(g, stream);
+    }
+    PL_CHECK_LAUNCH("gemm_f32");
+    return 0;
+}

@@ -1,19 +1,17 @@
-// y[n, N] = x[n, K] . w[N, K]^T with 32-bit multiply-add on the vector units.
+// y[n, N] = x[n, K] . w[N, K]^T with 32-bit products and sums whatever the operands are: 32-bit ones go to gemm_f32.hip,
+// bfloat16 ones (the fallback for shapes that the fast kernels refuse) are multiplied here on the vector units.
 //
-// This is the matrix product of the true 32-bit path: no matrix-core mode, no
-// reduced precision anywhere.  Each output element is the sum over k in
-// ascending order, whatever n is, so a row's result does not depend on what
-// else is in the batch.  The same kernel over bfloat16 inputs (products and
-// sums in 32-bit) is the fallback for shapes the fast kernels refuse.
+// Each output element is the sum over k in ascending order, whatever n is, so a row's result does not depend on what
+// else is in the batch.
 #include "common.hpp"
 
 #define TILE_M 64
 #define TILE_N 64
 #define TILE_K 16
 
-template <typename T, typename OUT>
+template <typename OUT>
 __global__ void __launch_bounds__(256)
-gemm_nt_kernel(const T* __restrict__ x, const T* __restrict__ w, OUT* __restrict__ y, int n, int N,
+gemm_nt_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, OUT* __restrict__ y, int n, int N,
                int K, int ldx, int ldy, long sx = 0, long sw = 0, long sy = 0) {
     // (a batch of products, one a blockIdx.z: operands and result `sx`, `sw`, `sy` elements further on)
     x += blockIdx.z * sx;
@@ -78,14 +76,14 @@ extern "C" int pl_gemm_plain(const void* x, const void* w, void* y, int n, int N
     dim3 grid(pl_ceil_div(N, TILE_N), pl_ceil_div(n, TILE_M));
     PL_REQUIRE(grid.y <= 65535, "gemm: %d rows are more than one launch covers", n);
     if (dtype == PL_DTYPE_F32) {
-        gemm_nt_kernel<float, float><<<grid, 256, 0, stream>>>(
-            static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), n, N, K, ldx, ldy);
+        return pl_gemm_f32(static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), n, N, K, ldx, ldy,
+                           1, 0, 0, 0, stream);
     } else if (dtype == PL_DTYPE_BF16) {
         if (out_f32)
-            gemm_nt_kernel<bf16_t, float><<<grid, 256, 0, stream>>>(
+            gemm_nt_kernel<float><<<grid, 256, 0, stream>>>(
                 static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<float*>(y), n, N, K, ldx, ldy);
         else
-            gemm_nt_kernel<bf16_t, bf16_t><<<grid, 256, 0, stream>>>(
+            gemm_nt_kernel<bf16_t><<<grid, 256, 0, stream>>>(
                 static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<bf16_t*>(y), n, N, K, ldx, ldy);
     } else {
         PL_REQUIRE(false, "gemm: dtype code %d", dtype);
@@ -106,14 +104,14 @@ extern "C" int pl_gemm_heads(const void* x, const void* w, void* y, int n, int h
     PL_REQUIRE(grid.y <= 65535, "gemm over heads: %d rows are more than one launch covers", n);
     const long sw = static_cast<long>(N) * K;
     if (dtype == PL_DTYPE_F32) {
-        gemm_nt_kernel<float, float><<<grid, 256, 0, stream>>>(
-            static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), n, N, K, ldx, ldy, sx, sw, sy);
+        return pl_gemm_f32(static_cast<const float*>(x), static_cast<const float*>(w), static_cast<float*>(y), n, N, K, ldx, ldy,
+                           heads, sx, sw, sy, stream);
     } else if (dtype == PL_DTYPE_BF16) {
         if (out_f32)
-            gemm_nt_kernel<bf16_t, float><<<grid, 256, 0, stream>>>(
+            gemm_nt_kernel<float><<<grid, 256, 0, stream>>>(
                 static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<float*>(y), n, N, K, ldx, ldy, sx, sw, sy);
         else
-            gemm_nt_kernel<bf16_t, bf16_t><<<grid, 256, 0, stream>>>(
+            gemm_nt_kernel<bf16_t><<<grid, 256, 0, stream>>>(
                 static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), static_cast<bf16_t*>(y), n, N, K, ldx, ldy, sx, sw, sy);
     } else {
         PL_REQUIRE(false, "gemm over heads: dtype code %d", dtype);

@@ -292,7 +292,8 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor | None = None, activation: s
 
 def gemm_plain(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None,
                out_dtype: torch.dtype | None = None) -> torch.Tensor:
-    """y = x . w^T with 32-bit multiply-add on the vector units (no matrix-core mode)."""
+    """y = x . w^T with 32-bit products and sums: 32-bit operands on the matrix cores' 32-bit instruction, bfloat16 ones on
+    the vector units.  A row of the result does not depend on what else is in the batch."""
     n, K = x.shape
     N = w.shape[0]
     _need(x, "matrix product input")
@@ -1536,7 +1537,7 @@ def head_weights(w: torch.Tensor) -> torch.Tensor:
 def gemm_heads(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """A product a head: out[t, h, :N] = x[t, h, :K] . W[h]^T with ``w = head_weights(W)``, W [heads, N, K].  ``x`` [n, heads, >= K] and ``out``
     [n, heads, >= N] may be views whose rows and heads lie further apart than their own sizes (the last axis
-    contiguous); a view's values behind K or N are neither read nor written.  In 32-bit on the vector units
+    contiguous); a view's values behind K or N are neither read nor written.  In 32-bit by the 32-bit product
     (sums in ascending k: the true 32-bit path); in bfloat16 the library's batched product on the matrix cores."""
     _need(w, "weights a head")
     heads, N, K = w.shape if w.dtype == torch.float32 else (w.shape[0], w.shape[2], w.shape[1])

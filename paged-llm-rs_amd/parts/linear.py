@@ -82,7 +82,7 @@ class Linear:
             raise TensorError(f"a {self.weight.dtype} linear given {x.dtype}")
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.float32:
-            # the true 32-bit path: vector-unit multiply-add only
+            # the true 32-bit path: 32-bit operands, products and sums
             y = kernels.gemm_plain(x, self.weight, out_dtype=torch.float32)
             return kernels.swiglu(y, activation=activation) if swiglu else y
         if kernels.skinny_applies(x, self.weight, self.strips is not None):

@@ -231,6 +231,30 @@ def test_gemm_plain(dtype, n, N, K):
     assert torch.equal(alone, kernels.gemm_plain(x, w, out_dtype=torch.float32)[:1])
 
 
+@pytest.mark.parametrize("N,K", [(1, 4), (15, 60), (33, 64), (70, 1026), (100, 1088), (4100, 192), (130, 3072), (32800, 128)])
+def test_the_32_bit_product_of_few_and_of_many_rows(N, K):
+    """Row counts on both sides of every rule that chooses the kernel (one, two and four tiles of 16 rows, tiles of 32 and of
+    64), widths that are whole double steps of the tiled kernel and ones that are not: the same bits for a row whatever else
+    is in the batch, and 64-bit arithmetic within what sums of at most 16 parts, each a chain of K / 16 products, can
+    be off (every rounding 2^-24 of a partial sum: some sqrt(K / 16 + 16) of them, and a factor of four)."""
+    from paged_llm_rs_amd import kernels
+
+    x = torch.randn(2050 if N < 200 else 200, K, device=DEV)
+    w = torch.randn(N, K, device=DEV)
+    full = kernels.gemm_plain(x, w)
+    assert rel(full, x.double() @ w.double().T) < 4 * math.sqrt(K / 16 + 16) * 2.0 ** -24
+    for n in (1, 8, 9, 16, 17, 32, 33, 64, 65, 130):
+        assert torch.equal(kernels.gemm_plain(x[-n:].contiguous(), w), full[-n:]), f"{n} rows"
+    x[1, K // 2], w[N // 2, 0], x[3] = math.inf, math.nan, 1e-41      # (and numbers too small to have an exponent)
+    for n in (4, 200):
+        y = kernels.gemm_plain(x[:n].contiguous(), w)
+        same = torch.equal(y[0][torch.arange(N, device=DEV) != N // 2], full[0][torch.arange(N, device=DEV) != N // 2])
+        assert same and not bool(y[1].isfinite().any()) and bool(y[:, N // 2].isnan().all())
+        if K % 64 == 0 and N > 1:
+            small = torch.arange(N, device=DEV) != N // 2
+            assert rel(y[3][small], x[3].double() @ w[small].double().T) < 1e-3
+
+
 @pytest.mark.parametrize("n", [1, 2, 8, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(16, 32), (331, 104), (4096, 1024), (1024, 3072), (50, 8), (1000, 2056)])
 def test_gemm_skinny(n, N, K):
