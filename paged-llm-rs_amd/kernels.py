@@ -36,6 +36,8 @@ def _signatures(lib) -> None:
         "pl_swiglu": [p, p, i, i, i, i, p],
         "pl_gemm_plain": [p, p, p, i, i, i, i, i, i, i, p],
         "pl_paged_attention_plain": [p, i, p, p, p, p, i, i, p, p, i, i, i, i, f, i, i, p, p, f, i, p, i, p],
+        "pl_paged_attention_f32_applies": [p, i, p, p, p, i],
+        "pl_paged_attention_f32": [p, i, p, p, p, p, p, i, p, i, i, p, p, i, i, i, i, f, i, p, p, f, i, p, i, p, p, i, p],
         "pl_gemm_heads": [p, p, p, i, i, i, i, i, ctypes.c_long, i, ctypes.c_long, i, i, p],
         "pl_head_prepare": [p, p, i, i, i, f, p, p, p, p, i, i, i, i, f, i, p, p, p, i, i, i, p, p, p, i, i, i, i, i, i, i,
                             p, i, p, f, p],
@@ -370,6 +372,69 @@ def paged_attention_plain(q: torch.Tensor, q_row_stride: int, out: torch.Tensor,
         block_table.data_ptr(), block_table.shape[1], block_size, k_pool.data_ptr(), v_pool.data_ptr(),
         n, nq, nkv, d, float(scale), int(window or 0), _code(q, "query buffer"), _ptr(sinks), _ptr(slopes),
         *_more_args(more, nq, n), _stream()))
+    return out
+
+
+# The 32-bit kernel's segments of keys, and the room that they may take where a second kernel folds them.
+F32_SEGMENT = 64
+F32_SPLIT_BYTES = 64 << 20
+
+
+def f32_splits(rows: int, live_seqs: int, nq: int, nkv: int, d: int, max_ctx: int) -> bool:
+    """Whether the 32-bit kernel leaves the segments of every row in memory for a second kernel to fold.  It costs that
+    kernel (some 5 us) and the segments' trip, and it pays where the tiles alone leave compute units without work: a few
+    tokens, whose keys a few workgroups would take in at what a compute unit gets from memory (8 tokens at contexts up to 512,
+    16 heads over 8 of 128: 25 us whole, 14 split), or few tiles before more than 1,024 keys."""
+    group = nq // nkv
+    tokens, head_tiles = (16 // group, 1) if group <= 16 else (1, -(-group // 16))
+    tiles = min(rows, rows // tokens + live_seqs) * nkv * head_tiles
+    segments = -(-max_ctx // F32_SEGMENT)
+    return (tiles < compute_units() and segments > 1 and (rows <= 16 or segments > 16)
+            and rows * nq * segments * (d + 2) * 4 <= F32_SPLIT_BYTES)
+
+
+def paged_attention_f32(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, positions: torch.Tensor, q_start: torch.Tensor,
+                        q_len: torch.Tensor, ctx_len: torch.Tensor, block_table: torch.Tensor, block_size: int,
+                        k_pool: torch.Tensor, v_pool: torch.Tensor, nq: int, nkv: int, d: int, scale: float, max_ctx: int,
+                        window: int = 0, live_seqs: int | None = None, sinks: torch.Tensor | None = None,
+                        slopes: torch.Tensor | None = None, more: AttentionMore | None = None,
+                        split: bool | None = None) -> torch.Tensor:
+    """32-bit attention of any rows on the matrix cores' 32-bit instruction.  Request s brings the rows q_start[s] ..
+    q_start[s] + q_len[s] - 1, which end at position ctx_len[s] - 1 (``positions`` says the same row by row); no context
+    is longer than ``max_ctx``.  ``live_seqs``: only so many of the requests, the first ones, bring tokens.  ``split``: whether
+    a second kernel folds the keys' segments (``f32_splits`` where not given); the result is the same bit for bit.  What is
+    left: as for ``paged_attention_plain``."""
+    n = positions.numel()
+    S = block_table.shape[0]
+    _need(q, "query buffer", None, torch.float32)
+    if q.dim() != 2 or q.shape[0] != n or q.shape[1] != q_row_stride or q_row_stride < nq * d:
+        raise TensorError(f"query buffer has shape {tuple(q.shape)} for {n} tokens and row stride {q_row_stride}")
+    _need(out, "attention output", (n, nq * d), torch.float32)
+    _need(positions, "positions", (n,), torch.int32)
+    _need(block_table, "block table", None, torch.int32)
+    for t, what in ((q_start, "first row of each request"), (q_len, "tokens of each request"),
+                    (ctx_len, "context length of each request")):
+        _need(t, what, (S,), torch.int32)
+    for pool, what in ((k_pool, "key pool"), (v_pool, "value pool")):
+        _need(pool, what, None, torch.float32)
+        if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % block_size != 0:
+            raise TensorError(f"{what} has shape {tuple(pool.shape)}, expected [pages*{block_size}, {nkv * d}]")
+    live = S if live_seqs is None else int(live_seqs)
+    if not 0 < live <= S:
+        raise TensorError(f"{live} requests with tokens of {S}")
+    sinks, slopes = _head_numbers(sinks, "sinks", nq), _head_numbers(slopes, "distance slopes", nq)
+    if split is None:
+        split = f32_splits(n, live, nq, nkv, d, int(max_ctx))
+    part_acc = part_ml = None
+    segments = -(-int(max_ctx) // F32_SEGMENT)
+    if split:
+        part_acc = torch.empty((n * nq * segments * d,), dtype=torch.float32, device=q.device)
+        part_ml = torch.empty((n * nq * segments * 2,), dtype=torch.float32, device=q.device)
+    _check(library().pl_paged_attention_f32(
+        q.data_ptr(), q_row_stride, out.data_ptr(), positions.data_ptr(), q_start.data_ptr(), q_len.data_ptr(),
+        ctx_len.data_ptr(), live, block_table.data_ptr(), block_table.shape[1], block_size, k_pool.data_ptr(),
+        v_pool.data_ptr(), n, nq, nkv, d, float(scale), int(window or 0), _ptr(sinks), _ptr(slopes),
+        *_more_args(more, nq, n), _ptr(part_acc), _ptr(part_ml), segments, _stream()))
     return out
 
 
@@ -728,9 +793,15 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                     scale: float, window: int = 0, sinks: torch.Tensor | None = None,
                     slopes: torch.Tensor | None = None, more: AttentionMore | None = None) -> torch.Tensor:
     """Attention for every token of a step.  ``qkv`` rows begin with the rotated queries.
-    In bfloat16 the long portions go to the tiled kernel and the tokens of short ones
+    In 32-bit every row goes to the kernel on the matrix cores' 32-bit instruction, where the head size is a multiple of four up
+    to 256, and otherwise to the plain one.  In bfloat16 the long portions go to the tiled kernel and the tokens of short ones
     (decoded tokens among them) to the kernel for single tokens, or, where many query heads share a key
     head, to the tiled kernel with a group's heads as its rows; all read the same pages."""
+    if qkv.dtype == torch.float32 and _attention_mode == "kernel" and library().pl_paged_attention_f32_applies(
+            qkv.data_ptr(), qkv.shape[1], out.data_ptr(), kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), d):
+        return paged_attention_f32(qkv, qkv.shape[1], out, batch.positions, batch.q_start, batch.q_len, batch.ctx_len,
+                                   kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, batch.max_ctx_len,
+                                   window, getattr(batch, "live_seqs", None), sinks, slopes, more)
     if qkv.dtype != torch.bfloat16 or _attention_mode != "kernel" or d % 16 or d > 256:
         return paged_attention_plain(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                      kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window,
@@ -1302,7 +1373,7 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
                                          out.data_ptr(), batch.q_start.data_ptr(), batch.q_len.data_ptr(),
                                          batch.state_slots.data_ptr(), batch.num_seqs, H, G, N, V, below, stream))
     if chunked:
-        chunks = n // SSD_CHUNK + batch.num_seqs + 1
+        chunks = n // library().pl_recurrent_chunk_tokens(dim) + batch.num_seqs + 1
         f32 = dict(dtype=torch.float32, device=qkv.device)
         sums, before = torch.empty((chunks, H * N * V), **f32), torch.empty((chunks, H * N * V), **f32)
         ends = torch.empty((chunks, H), **f32)

@@ -1590,6 +1590,116 @@ def test_a_norm_handed_forward_from_one_product_to_the_next(n, H, deep, N2, swig
         assert rel(got, own.double()) < 1e-2
 
 
+def attention_with_everything(q, keys, values, pos, g, scale, window, sinks, slopes, more, row):
+    """One token in 64 bits: q [nq, d], keys and values [ctx, nkv, d]; a key set to None's place (NaN rows never seen) is masked."""
+    if window > 0:
+        first = max(0, pos + 1 - window)
+    elif window < 0:
+        first = pos - pos % -window
+    else:
+        first = 0
+    at = [j for j in range(pos + 1) if j >= first or j < more.keep]
+    out = []
+    for h in range(q.shape[0]):
+        s = keys[at, h // g] @ q[h] * scale
+        if more.cap > 0:
+            s = more.cap * torch.tanh(s / more.cap)
+        if slopes is not None:
+            s = s - float(slopes[h]) * (pos - torch.tensor(at, dtype=torch.float64))
+        top = max(float(s.max()), float(sinks[h]) if sinks is not None else -math.inf)
+        e = torch.exp(s - top)
+        total = e.sum() + (math.exp(float(sinks[h]) - top) if sinks is not None else 0.0)
+        o = (e[:, None] * values[at, h // g]).sum(0) / total
+        if more.gate is not None:
+            o = o * torch.sigmoid(more.gate[row, h].double().cpu())
+        out.append(o)
+    return torch.stack(out)
+
+
+F32_CASES = [
+    # nq, nkv, d, block size, [(context after the step, tokens of the step)], window, kept first keys
+    (4, 2, 16, 16, [(5, 5), (17, 17), (33, 1), (64, 1), (65, 1)], 0, 0),          # a head in part of a stretch, edges of segments
+    (16, 8, 128, 16, [(512, 1), (300, 1), (129, 3), (1, 1), (70, 37)], 0, 0),
+    (6, 2, 64, 1, [(200, 9), (64, 64)], 70, 0),                                     # five tokens a tile; a window over pages of one
+    (3, 3, 100, 8, [(140, 33), (7, 2)], -32, 0),                                    # blocks; sixteen tokens a tile, 100 of 128 values
+    (40, 2, 256, 32, [(90, 2), (200, 1)], 0, 0),                                    # two tiles of heads a token
+    (20, 1, 20, 4, [(300, 5)], 33, 6),                                              # kept keys in front of a window
+    (8, 1, 192, 128, [(260, 70)], 100, 70),                                         # kept keys of two segments
+    (16, 1, 36, 16, [(130, 130)], 0, 0),
+]
+
+
+@pytest.mark.parametrize("extras", [False, True])
+@pytest.mark.parametrize("nq,nkv,d,bs,requests,window,keep", F32_CASES)
+def test_the_32_bit_attention_kernel(nq, nkv, d, bs, requests, window, keep, extras):
+    """Every token against 64-bit arithmetic (some 2^-24 a rounding: 3e-6 of the result), the two ways to fold and the
+    tokens of a step one request at a time to the bit; free rows, a page that is not there and rows of padding hold NaNs."""
+    from paged_llm_rs_amd import kernels
+
+    ctx = [c for c, _ in requests]
+    bt, k_pool, v_pool, keys, values = build_paged(nkv, d, bs, ctx, torch.float32, seed=d + bs)
+    gen = torch.Generator().manual_seed(nq * d)
+    rows = sum(t for _, t in requests) + 2
+    stride = (nq + 2 * nkv) * d
+    q = (2 * torch.randn(rows, stride, generator=gen)).to(DEV)
+    sinks = torch.randn(nq, generator=gen).to(DEV) if extras else None
+    slopes = (0.02 * torch.rand(nq, generator=gen)).to(DEV) if extras else None
+    gate = torch.randn(rows, nq, generator=gen).to(DEV) if extras else None
+    more = kernels.AttentionMore(cap=5.0 if extras and window >= 0 else None, keep=keep, gate=gate)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    starts, at = [], 0
+    for _, t in requests:
+        starts.append(at)
+        at += t
+    positions = i32([c - t + k for c, t in requests for k in range(t)] + [-1, -1])
+    # one more request that holds the padding
+    table = torch.cat([bt, torch.full_like(bt[:1], -1)])
+    args = dict(q_start=i32(starts + [at]), q_len=i32([t for _, t in requests] + [2]), ctx_len=i32(ctx + [0]))
+    scale = d ** -0.5
+
+    def run(split, rows_of=None, **over):
+        a = {**args, **over}
+        qs, ps, gs = (q, positions, gate) if rows_of is None else (q[rows_of].contiguous(), positions[rows_of].contiguous(),
+                                                                   None if gate is None else gate[rows_of].contiguous())
+        out = torch.full((qs.shape[0], nq * d), 7.0, device=DEV)
+        m = kernels.AttentionMore(cap=more.cap, keep=keep, gate=gs)
+        return kernels.paged_attention_f32(qs, stride, out, ps, a["q_start"], a["q_len"], a["ctx_len"], a.get("table", table), bs,
+                                           k_pool, v_pool, nq, nkv, d, scale, max(ctx), window, live_seqs=a.get("live", len(ctx)),
+                                           sinks=sinks, slopes=slopes, more=m, split=split)
+
+    out = run(False)
+    assert torch.equal(out, run(True)), "the two ways to fold"
+    assert bool((out[-2:] == 7.0).all()), "rows of padding are not written"
+    plain = torch.full_like(out, 7.0)
+    seq_of = i32([s for s, (_, t) in enumerate(requests) for _ in range(t)] + [len(ctx)] * 2)
+    kernels.paged_attention_plain(q, stride, plain, positions, seq_of, table, bs, k_pool, v_pool, nq, nkv, d, scale, window,
+                                  sinks=sinks, slopes=slopes, more=more)
+    assert rel(out, plain) < 3e-6
+    for s, (c, t) in enumerate(requests):
+        for k in sorted({0, t - 1, t // 2}):
+            want = attention_with_everything(q[starts[s] + k, :nq * d].double().cpu().reshape(nq, d), keys[s], values[s], c - t + k,
+                                             nq // nkv, scale, window, sinks, slopes, more, starts[s] + k)
+            assert rel(out[starts[s] + k].reshape(nq, d), want) < 3e-6, f"request {s}, token {k}"
+        # the request's last token alone, and its last three
+        for last in (1, min(3, t)):
+            mine = torch.arange(starts[s] + t - last, starts[s] + t, device=DEV)
+            alone = run(last == 1, mine, q_start=i32([0]), q_len=i32([last]), ctx_len=i32([c]), table=table[s:s + 1].contiguous(), live=1)
+            assert torch.equal(alone, out[mine]), f"request {s}: its last {last}"
+    # an infinity among a late token's values reaches the tokens that see it and no other
+    s = max(range(len(ctx)), key=lambda i: requests[i][1])
+    c, t = requests[s]
+    if t > 2:
+        key = c - 2
+        slot = int(table[s, key // bs]) * bs + key % bs
+        v_pool[slot, :d] = math.inf
+        bad = run(False)
+        assert torch.equal(bad, run(True))
+        assert torch.equal(bad[starts[s]:starts[s] + t - 2], out[starts[s]:starts[s] + t - 2])
+        group = nq // nkv
+        assert not bool(bad[starts[s] + t - 1].view(nq, d)[:group].isfinite().any())
+        assert torch.equal(bad[starts[s] + t - 1].view(nq, d)[group:], out[starts[s] + t - 1].view(nq, d)[group:])
+
+
 SINK_CASES = [
     # nq, nkv, d, block size, [(context length after the step, tokens of the step)], window
     (4, 2, 48, 16, [(300, 40), (136, 1), (137, 1), (20, 20), (5, 2)], 136),      # token tiles and single tokens, a window
