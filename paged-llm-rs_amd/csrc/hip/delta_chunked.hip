@@ -380,6 +380,9 @@ static int launch_delta(const DeltaArgs& da, int seqs, int max_q_len, hipStream_
 
 // The requests of the step that bring at least `from` tokens.  Kn, Qn: room for (rows / chunk + requests)
 // chunks of H * chunk * (D rounded up to 4) floats; Tm, Aq: of H * chunk * chunk; scal: of H * 3 * chunk.
+// How many tokens a chunk has for heads of q and k of size D (the longer rows of large heads leave LDS for fewer).
+extern "C" int pl_recurrent_chunk_tokens(int D) { return D <= 128 ? 64 : 32; }
+
 extern "C" int pl_delta_chunked(const float* qkv, int qkv_stride, int q_off, int k_off, int v_off,
                                 const float* gates, int gates_stride, int g1_off, int g2_off,
                                 const float* a_log, const float* dt_bias,

@@ -226,6 +226,11 @@ extern "C" int pl_recurrent_scan(int kind, const float* qkv, int qkv_stride, int
     if (seqs == 0) return 0;
     ScanArgs a{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, p1, p2, p3, cap,
                state, state_stride, s_off, n_off, m_off, out, q_start, q_len, state_slots, H, G, D, V, below};
+    // (the scan kernel is left with states whose columns are no whole aligned quads)
+    if (pl_state_step(kind, a, seqs, stream)) {
+        PL_CHECK_LAUNCH("recurrent_scan (step)");
+        return 0;
+    }
     if (kind == PL_SCAN_LIGHTNING) return launch_scan<PL_SCAN_LIGHTNING>(a, seqs, stream);
     if (kind == PL_SCAN_MLSTM) return launch_scan<PL_SCAN_MLSTM>(a, seqs, stream);
     if (kind == PL_SCAN_SSD) return launch_scan<PL_SCAN_SSD>(a, seqs, stream);

@@ -37,3 +37,5 @@ __device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.f) - 
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 
+// The kernel for requests of few tokens that spreads a state over four waves (ssd.hip), for the kinds lightning, mlstm and delta.
+bool pl_state_step(int kind, const ScanArgs& a, int seqs, hipStream_t stream);

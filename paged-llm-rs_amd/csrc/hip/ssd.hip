@@ -4,7 +4,7 @@
 // q, k and v of the scan's arguments are C, B and x; C and B have G heads, head h reads head h / (H / G).
 //
 // Linear attention with a fixed decay a head (kind retention) is the same recurrence with e^(-a dt) = decay, dt = 1 in front of
-// B x^T and no D: the chunked kernels serve it as FIXED instances (p1 holds the decays), retention_step is its kernel for few tokens.
+// B x^T and no D: the chunked kernels serve it too (p1 holds the decays), retention_step is its kernel for few tokens.
 // Its q and k turn with their positions: retention_turn does that to a step's rows in front of the chunked kernels,
 // retention_step to what it reads.
 //
@@ -253,6 +253,192 @@ __global__ __launch_bounds__(256) void retention_turn_kernel(float* __restrict__
     }
 }
 
+// The other recurrences, token by token (kinds lightning, mlstm and delta): a workgroup of four waves owns 64 columns of a head's
+// state for one request, as above.  Bound by the chain of a token: state and rows on their way together, one round through
+// LDS for the read-out (delta: two more, for the unit vectors and for what the memory says to the key).  A wave with a
+// column of the state a lane (the scan kernel) asks for D rows one after the other and adds them up alone: 20 to 25 us for one token of
+// two requests (8 heads of 128 by 128, 4 of 128 by 256), and some 7 here.
+template <int R, int KIND>
+__global__ __launch_bounds__(256) void state_step_kernel(ScanArgs a) {
+    __shared__ ssd_f32x4 part[4][16], memory[4][16];
+    __shared__ __attribute__((aligned(16))) float qs[16 * R], ks[16 * R];
+    __shared__ float sums[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.y, s = blockIdx.z;
+    const int slot = a.state_slots[s];
+    const int count = a.q_len[s];
+    if (slot < 0 || count <= 0 || (a.below > 0 && count >= a.below)) return;
+    const int start = a.q_start[s];
+    const int N = a.D, V = a.V, H = a.H, g = h / (H / a.G), tiles = gridDim.x;
+    const int n0 = (4 * wave + (lane >> 4)) * R;
+    const int v0 = blockIdx.x * 64 + 4 * (lane & 15);
+    const bool owns = v0 < V;                                   // (V is a multiple of 4)
+    float* slot_state = a.state + static_cast<size_t>(slot) * a.state_stride;
+    float* Sg = slot_state + a.s_off + static_cast<size_t>(h) * N * V;
+    ssd_f32x4 S[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+        S[i] = (owns && n0 + i < N) ? *reinterpret_cast<const ssd_f32x4*>(Sg + static_cast<size_t>(n0 + i) * V + v0) : ssd_f32x4{0.f, 0.f, 0.f, 0.f};
+    // (every tile of columns has a copy of the normaliser and of the maximum of its own: see the scan kernel)
+    float* ng = slot_state + a.n_off + (static_cast<size_t>(h) * tiles + blockIdx.x) * N + tid;
+    float* mg = slot_state + a.m_off + h * tiles + blockIdx.x;
+    float nv = 0.f, m = 0.f;
+    if (KIND == PL_SCAN_MLSTM) {
+        if (tid < N) nv = *ng;
+        m = *mg;
+    }
+    const float c1 = KIND == PL_SCAN_DELTA ? expf(a.p1[h]) : a.p1[h], c2 = KIND == PL_SCAN_LIGHTNING ? 0.f : a.p2[h];
+    const float q_scale = 1.f / sqrtf(static_cast<float>(N));
+    for (int i = N + tid; i < 16 * R; i += 256) qs[i] = ks[i] = 0.f;
+    for (int t = 0; t < count; ++t) {
+        const float* row = a.qkv + static_cast<size_t>(start + t) * a.qkv_stride;
+        ssd_f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (owns) {
+            const float* vr = row + a.v_off + h * V + v0;
+            v = ssd_f32x4{vr[0], vr[1], vr[2], vr[3]};
+        }
+        float q = 0.f, k = 0.f, x1 = 0.f, x2 = 0.f;
+        if (tid < N) {
+            q = row[a.q_off + g * N + tid];
+            k = row[a.k_off + g * N + tid];
+        }
+        if (KIND != PL_SCAN_LIGHTNING) {
+            const float* gates = a.gates + static_cast<size_t>(start + t) * a.gates_stride;
+            x1 = gates[a.g1_off + h];
+            x2 = gates[a.g2_off + h];
+        }
+        if (KIND == PL_SCAN_LIGHTNING) {
+            q = silu_f(q);
+            k = silu_f(k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = silu_f(v[e]);
+        }
+        if (KIND == PL_SCAN_MLSTM) q *= q_scale;
+        if (KIND == PL_SCAN_DELTA) {
+            const float qq = wave_sum(q * q), kk = wave_sum(k * k);
+            if (lane == 0) {
+                sums[0][wave] = qq;
+                sums[1][wave] = kk;
+            }
+        }
+        if (tid < N) {
+            qs[tid] = q;
+            ks[tid] = k;
+        }
+        __syncthreads();
+        float kr[R], qr[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            kr[i] = ks[n0 + i];
+            qr[i] = qs[n0 + i];
+        }
+        float keep = c1, add = 1.f, below = 0.f;
+        if (KIND == PL_SCAN_MLSTM) {
+            const float gi = a.cap * tanhf((x1 + c1) / a.cap), gf = logsigmoid_f(a.cap * tanhf((x2 + c2) / a.cap));
+            const float top = fmaxf(gf + m, gi);
+            keep = expf(gf + m - top);
+            add = expf(gi - top);
+            m = top;
+            below = expf(-top);
+            nv = keep * nv + add * k;
+            const float nq = wave_sum(nv * q);
+            if (lane == 0) sums[0][wave] = nq;
+        }
+        if (KIND == PL_SCAN_DELTA) {
+            const float qq = sums[0][0] + sums[0][1] + sums[0][2] + sums[0][3], kk = sums[1][0] + sums[1][1] + sums[1][2] + sums[1][3];
+            const float by_q = 1.f / sqrtf(qq + 1e-6f) * q_scale, by_k = 1.f / sqrtf(kk + 1e-6f);
+            keep = expf(-c1 * softplus_f(x2 + c2));
+            ssd_f32x4 says = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                kr[i] *= by_k;
+                qr[i] *= by_q;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    S[i][e] *= keep;
+                    says[e] += S[i][e] * kr[i];
+                }
+            }
+#pragma unroll
+            for (int off = 16; off < 64; off <<= 1)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) says[e] += __shfl_xor(says[e], off, 64);
+            if (lane < 16) memory[wave][lane] = says;
+            __syncthreads();
+            const float beta = sigmoid_f(x1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float said = 0.f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) said += memory[w][lane & 15][e];
+                v[e] = beta * (v[e] - said);
+            }
+            keep = 1.f;
+        }
+        ssd_f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= add;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                S[i][e] = keep * S[i][e] + kr[i] * v[e];
+                o[e] += S[i][e] * qr[i];
+            }
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], off, 64);
+        if (lane < 16) part[wave][lane] = o;
+        __syncthreads();
+        if (wave == 0 && lane < 16 && owns) {
+            ssd_f32x4 y = part[0][lane];
+#pragma unroll
+            for (int w = 1; w < 4; ++w)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] += part[w][lane][e];
+            if (KIND == PL_SCAN_MLSTM) {
+                const float nq = sums[0][0] + sums[0][1] + sums[0][2] + sums[0][3];
+                const float by = 1.f / (fmaxf(fabsf(nq), below) + 1e-6f);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] *= by;
+            }
+            *reinterpret_cast<ssd_f32x4*>(a.out + static_cast<size_t>(start + t) * (H * V) + h * V + v0) = y;
+        }
+        // (what the first wave reads here, `part` and mlstm's `sums`, is written again behind the next token's first barrier, which
+        // the first wave reaches behind its reads; delta's `sums` were read by everybody before this token's last barrier)
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+        if (owns && n0 + i < N) *reinterpret_cast<ssd_f32x4*>(Sg + static_cast<size_t>(n0 + i) * V + v0) = S[i];
+    if (KIND == PL_SCAN_MLSTM) {
+        if (tid < N) *ng = nv;
+        if (tid == 0) *mg = m;
+    }
+}
+
+template <int KIND>
+static void launch_step(const ScanArgs& a, int seqs, hipStream_t stream) {
+    const dim3 grid(pl_ceil_div(a.V, 64), a.H, seqs);
+    if (a.D <= 16) state_step_kernel<1, KIND><<<grid, 256, 0, stream>>>(a);
+    else if (a.D <= 32) state_step_kernel<2, KIND><<<grid, 256, 0, stream>>>(a);
+    else if (a.D <= 64) state_step_kernel<4, KIND><<<grid, 256, 0, stream>>>(a);
+    else if (a.D <= 128) state_step_kernel<8, KIND><<<grid, 256, 0, stream>>>(a);
+    else state_step_kernel<16, KIND><<<grid, 256, 0, stream>>>(a);
+}
+
+// The kernel above needs whole aligned quads of columns.  False: it does not apply, and nothing was launched.
+bool pl_state_step(int kind, const ScanArgs& a, int seqs, hipStream_t stream) {
+    if (a.V % 4 != 0 || a.state_stride % 4 != 0 || a.s_off % 4 != 0 || reinterpret_cast<uintptr_t>(a.state) % 16 != 0 ||
+        reinterpret_cast<uintptr_t>(a.out) % 16 != 0)
+        return false;
+    if (kind == PL_SCAN_LIGHTNING) launch_step<PL_SCAN_LIGHTNING>(a, seqs, stream);
+    else if (kind == PL_SCAN_MLSTM) launch_step<PL_SCAN_MLSTM>(a, seqs, stream);
+    else if (kind == PL_SCAN_DELTA) launch_step<PL_SCAN_DELTA>(a, seqs, stream);
+    else return false;
+    return true;
+}
+
 // ---- many tokens -----------------------------------------------------------------------------------------
 
 struct SsdArgs {
@@ -260,6 +446,10 @@ struct SsdArgs {
     float* U;        // [chunks, H, N, V]  a chunk's weighted sum of B x^T
     float* Sin;      // [chunks, H, N, V]  the state before a chunk
     float* ends;     // [chunks, H]        b at the chunk's end
+    // the matrix memory's, null for the others
+    float* Uk;       // [chunks, H, N]     a chunk's weighted sum of B, for the normaliser
+    float* nin;      // [chunks, H, N]     the normaliser before a chunk
+    float* tops;     // [chunks, H, 2]     the largest w_t - b_t of a chunk; the running maximum before it
 };
 
 // A request's chunks have numbers of their own among all chunks of the step: requests lie one behind the
@@ -267,32 +457,53 @@ struct SsdArgs {
 __device__ __forceinline__ int ssd_chunk(const ScanArgs& a, int s, int c) { return a.q_start[s] / SSD_CHUNK + s + c; }
 
 // By one wave, all its lanes: the running sums b (64-bit) and the step sizes of a chunk's L <= 64 tokens; the sum
-// over the chunk comes back.  Lanes past the chunk hold the last sum and a step of zero.
-template <bool FIXED>
-__device__ __forceinline__ double ssd_gates(const ScanArgs& a, int h, int row0, int L, int lane, double& b, float& dt) {
-    dt = 0.f;
-    if (FIXED) {
+// over the chunk comes back.  Lanes past the chunk hold the last sum and a step of zero.  The matrix memory has in the
+// place of the step size the log weight of a token's write less b (64-bit; -inf past the chunk).
+template <int KIND>
+__device__ __forceinline__ double ssd_gates(const ScanArgs& a, int h, int row0, int L, int lane, double& b, double& dt) {
+    dt = KIND == PL_SCAN_MLSTM ? -INFINITY : 0.0;
+    if (KIND == PL_SCAN_RETENTION || KIND == PL_SCAN_LIGHTNING) {
         const double each = log(static_cast<double>(a.p1[h]));
-        if (lane < L) dt = 1.f;
+        if (lane < L) dt = 1.0;
         b = each * (min(lane, L - 1) + 1);
         return each * L;
     }
-    if (lane < L) dt = softplus_f(a.gates[static_cast<size_t>(row0 + lane) * a.gates_stride + a.g1_off + h] + a.p2[h]);
-    double sum = -static_cast<double>(expf(a.p1[h])) * static_cast<double>(dt);
+    double sum = 0.0;
+    if (KIND == PL_SCAN_MLSTM) {
+        if (lane < L) {
+            const float* gates = a.gates + static_cast<size_t>(row0 + lane) * a.gates_stride;
+            dt = a.cap * tanhf((gates[a.g1_off + h] + a.p1[h]) / a.cap);
+            sum = logsigmoid_f(a.cap * tanhf((gates[a.g2_off + h] + a.p2[h]) / a.cap));
+        }
+    } else {
+        if (lane < L) dt = softplus_f(a.gates[static_cast<size_t>(row0 + lane) * a.gates_stride + a.g1_off + h] + a.p2[h]);
+        sum = -static_cast<double>(expf(a.p1[h])) * dt;
+    }
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
         const double other = __shfl_up(sum, off, 64);
         if (lane >= off) sum += other;
     }
     b = sum;
+    if (KIND == PL_SCAN_MLSTM) dt -= b;
     return __shfl(sum, L - 1, 64);
 }
 
-// (FIXED: one decay a head, p1, and steps of one.)
+// What the rows hold becomes q, k and v: linear attention takes them through silu, the matrix memory scales its queries.
+template <int KIND>
+__device__ __forceinline__ float ssd_kv(float x) { return KIND == PL_SCAN_LIGHTNING ? silu_f(x) : x; }
+template <int KIND>
+__device__ __forceinline__ float ssd_q(float x, float scale) { return KIND == PL_SCAN_MLSTM ? x * scale : ssd_kv<KIND>(x); }
+
+// (Retention and lightning: one decay a head, p1, and steps of one.  The matrix memory, mlstm: with w_t the log weight of token
+// t's write and m the maximum that holds its exponentials, m_t = b_t + max(m_0, max_{u<=t} (w_u - b_u)), which is the very
+// sequence that the token-by-token form walks through, every exponent is at or below zero:
+//     y_t = (sum_{u<=t} e^(w_u - b_u - c_t) (q_t . k_u) v_u + e^(m_0 - c_t) S_0^T q_t) / max(|n . q|, e^(-m_t)),  c_t = m_t - b_t,
+// with n . q the same sum without v_u and S_0.)
 
 // summary: a wave a tile of 32 rows of N (and the tile four further on, where N has more than 128), 64 columns of V.
 // Both operands come straight from memory, a token a row: 128 bytes a half wave.
-template <bool FIXED>
+template <int KIND>
 __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
     const ScanArgs& a = sa.a;
     __shared__ float weight[SSD_CHUNK];
@@ -313,14 +524,25 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
 #pragma unroll
     for (int k = 0; k < SSD_CHUNK / 2; ++k) {
         const float* x = rows + static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.v_off + h * V;
-        xa[k] = x[va];
-        xb[k] = two ? x[vb] : 0.f;
+        xa[k] = ssd_kv<KIND>(x[va]);
+        xb[k] = two ? ssd_kv<KIND>(x[vb]) : 0.f;
     }
     if (wave == 0) {
-        double b;
-        float dt;
-        const double end = ssd_gates<FIXED>(a, h, row0, L, lane, b, dt);
-        weight[lane] = expf(static_cast<float>(end - b)) * dt;          // (zero past the chunk's tokens)
+        double b, dt;
+        const double end = ssd_gates<KIND>(a, h, row0, L, lane, b, dt);
+        if (KIND == PL_SCAN_MLSTM) {
+            double top = dt;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) top = fmax(top, __shfl_xor(top, off, 64));
+            weight[lane] = expf(static_cast<float>(dt - top));
+            if (vt == 0 && lane == 0) {
+                sa.tops[2 * idx] = static_cast<float>(top);
+                // the maximum that the request's first chunk starts from: the carry reads it here, not in the slot it writes
+                if (c == 0) sa.tops[2 * idx + 1] = a.state[static_cast<size_t>(slot) * a.state_stride + a.m_off + h * tiles];
+            }
+        } else {
+            weight[lane] = expf(static_cast<float>(end - b)) * static_cast<float>(dt);  // (zero past the chunk's tokens)
+        }
         if (vt == 0 && lane == 0) sa.ends[idx] = static_cast<float>(end);
     }
     __syncthreads();
@@ -336,7 +558,14 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
         float ka[SSD_CHUNK / 2];
 #pragma unroll
         for (int k = 0; k < SSD_CHUNK / 2; ++k)
-            ka[k] = rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n];
+            ka[k] = ssd_kv<KIND>(rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n]);
+        if (KIND == PL_SCAN_MLSTM && vt == 0) {
+            float sum = 0.f;
+#pragma unroll
+            for (int k = 0; k < SSD_CHUNK / 2; ++k) sum += weight[2 * k + half] * ka[k];
+            sum += __shfl_xor(sum, 32, 64);
+            if (half == 0 && n0 + l32 < N) sa.Uk[idx * N + n0 + l32] = sum;
+        }
         ssd_f32x16 da, db;
 #pragma unroll
         for (int r = 0; r < 16; ++r) da[r] = db[r] = 0.f;
@@ -357,6 +586,7 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
 
 // carry: the state before every chunk, and the request's state after its last; a thread an element, the sums of the next
 // chunks on their way while the ones before are taken in.
+template <int KIND>
 __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
     const ScanArgs& a = sa.a;
     const int N = a.D, V = a.V, H = a.H;
@@ -365,38 +595,55 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
     if (slot < 0 || count < a.below) return;
     const int chunks = (count + SSD_CHUNK - 1) / SSD_CHUNK;
     const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= N * V) return;
+    // the normaliser's N values ride along in the threads behind the matrix's
+    const bool element = e < N * V, of_n = KIND == PL_SCAN_MLSTM && e >= N * V && e < N * (V + 1);
+    if (!element && !of_n) return;
     const size_t NV = static_cast<size_t>(N) * V;
-    float* at = a.state + static_cast<size_t>(slot) * a.state_stride + a.s_off + h * NV + e;
+    const int tiles = (V + 63) / 64;       // (n and m have a copy a tile of columns in the slot; all are equal)
+    float* slot_state = a.state + static_cast<size_t>(slot) * a.state_stride;
+    const int en = e - N * V;
+    float* at = of_n ? slot_state + a.n_off + static_cast<size_t>(h) * tiles * N + en : slot_state + a.s_off + h * NV + e;
     const size_t first = static_cast<size_t>(ssd_chunk(a, s, 0)) * H + h;
-    const float* __restrict__ U = sa.U + first * NV + e;
-    float* __restrict__ Sin = sa.Sin + first * NV + e;
+    const float* __restrict__ U = of_n ? sa.Uk + first * N + en : sa.U + first * NV + e;
+    float* __restrict__ Sin = of_n ? sa.nin + first * N + en : sa.Sin + first * NV + e;
     const float* __restrict__ ends = sa.ends + first;
-    const size_t step = NV * H;
+    const size_t step = (of_n ? N : NV) * H;
     float S = *at;
+    float m = KIND == PL_SCAN_MLSTM ? sa.tops[2 * first + 1] : 0.f;
     constexpr int AHEAD = 8;
     for (int c0 = 0; c0 < chunks; c0 += AHEAD) {
-        float u[AHEAD], keep[AHEAD];
+        float u[AHEAD], keep[AHEAD], most[AHEAD];
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int c = min(c0 + i, chunks - 1);
             u[i] = U[c * step];
             keep[i] = ends[static_cast<size_t>(c) * H];
+            most[i] = KIND == PL_SCAN_MLSTM ? sa.tops[2 * (first + static_cast<size_t>(c) * H)] : 0.f;
         }
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i)
             if (c0 + i < chunks) {
                 Sin[(c0 + i) * step] = S;
-                S = expf(keep[i]) * S + u[i];
+                if (KIND == PL_SCAN_MLSTM) {
+                    if (c0 + i > 0 && e == 0) sa.tops[2 * (first + static_cast<size_t>(c0 + i) * H) + 1] = m;
+                    const float top = fmaxf(m, most[i]);
+                    S = expf(m - top) * S + expf(most[i] - top) * u[i];
+                    m = keep[i] + top;
+                } else {
+                    S = expf(keep[i]) * S + u[i];
+                }
             }
     }
     *at = S;
+    if (of_n)
+        for (int t = 1; t < tiles; ++t) at[static_cast<size_t>(t) * N] = S;
+    if (KIND == PL_SCAN_MLSTM && e < tiles) slot_state[a.m_off + h * tiles + e] = m;
 }
 
 // output: the read-outs of one chunk, head and tile of 64 columns.  Four waves; wave 2 ti + j owns the tokens 32 ti .. + 31 and, of the
 // scores, the earlier tokens 32 j .. + 31, of the read-outs, the columns 32 j .. + 31.
-// LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes.
-template <bool FIXED>
+// LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes, two numbers a token.
+template <int KIND>
 __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int aligned) {
     const ScanArgs& a = sa.a;
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -410,9 +657,13 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
     const int g = h / (H / a.G);
     const int Np = (N + 7) & ~7, P = Np + 4;
     constexpr int PA = SSD_CHUNK + 4;
+    // mlstm: bd holds c_t, dtd the w_u - b_u, before_w what multiplies S_0^T q_t, below what the read-out is divided by
     double* bd = reinterpret_cast<double*>(lds);
-    float* dts = lds + 2 * SSD_CHUNK;
-    float* Cs = dts + SSD_CHUNK;
+    double* dtd = bd + SSD_CHUNK;
+    float* before_w = lds + 4 * SSD_CHUNK;
+    float* below = before_w + SSD_CHUNK;
+    float* Cs = below + SSD_CHUNK;
+    const float q_scale = 1.f / sqrtf(static_cast<float>(N));
     float* Bs = Cs + SSD_CHUNK * P;
     float* As = Bs;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -431,6 +682,13 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
                 cv = *reinterpret_cast<const ssd_f32x4*>(row + a.q_off);
                 bv = *reinterpret_cast<const ssd_f32x4*>(row + a.k_off);
             }
+            if (KIND == PL_SCAN_LIGHTNING || KIND == PL_SCAN_MLSTM) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    cv[j] = ssd_q<KIND>(cv[j], q_scale);
+                    bv[j] = ssd_kv<KIND>(bv[j]);
+                }
+            }
             *reinterpret_cast<ssd_f32x4*>(Cs + t * P + i) = cv;
             *reinterpret_cast<ssd_f32x4*>(Bs + t * P + i) = bv;
         }
@@ -439,8 +697,8 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             const int t = e / Np, i = e - t * Np;
             const bool in = t < L && i < N;
             const float* row = rows + static_cast<size_t>(in ? t : 0) * a.qkv_stride + g * N + (in ? i : 0);
-            Cs[t * P + i] = in ? row[a.q_off] : 0.f;
-            Bs[t * P + i] = in ? row[a.k_off] : 0.f;
+            Cs[t * P + i] = in ? ssd_q<KIND>(row[a.q_off], q_scale) : 0.f;
+            Bs[t * P + i] = in ? ssd_kv<KIND>(row[a.k_off]) : 0.f;
         }
     }
     const int v = vt * 64 + 32 * tj + l32, vc = min(v, V - 1);
@@ -451,7 +709,7 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         x[k] = 0.f;
         if (columns && (k < 16 || ti == 1)) {
             const int u = 8 * (k >> 2) + 4 * half + (k & 3);
-            x[k] = rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc];
+            x[k] = ssd_kv<KIND>(rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc]);
         }
     }
     const float* S0 = sa.Sin + idx * N * V + vc;
@@ -465,11 +723,24 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
     float s0[32];
     if (columns) ask(0, s0);
     if (wave == 0) {
-        double b;
-        float dt;
-        ssd_gates<FIXED>(a, h, row0, L, lane, b, dt);
+        double b, dt;
+        ssd_gates<KIND>(a, h, row0, L, lane, b, dt);
+        if (KIND == PL_SCAN_MLSTM) {
+            const double m0 = sa.tops[2 * idx + 1];
+            double top = fmax(m0, dt);
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const double other = __shfl_up(top, off, 64);
+                if (lane >= off) top = fmax(top, other);
+            }
+            before_w[lane] = expf(static_cast<float>(m0 - top));
+            below[lane] = static_cast<float>(-(b + top));               // -m_t, until the weighted scores are there
+            b = top;
+        } else {
+            before_w[lane] = expf(static_cast<float>(b));
+        }
         bd[lane] = b;
-        dts[lane] = dt;
+        dtd[lane] = dt;
     }
     __syncthreads();
 
@@ -487,12 +758,13 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             for (int e = 0; e < 4; ++e) acc = ssd_mfma(cv[e], bv[e], acc);
         }
         const int u = 32 * tj + l32;
-        const double bu = bd[u];
-        const float du = dts[u];
+        const double bu = bd[u], du = dtd[u];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int t = 32 * ti + 8 * (r >> 2) + 4 * half + (r & 3);
-            acc[r] = (u <= t && t < L) ? acc[r] * (expf(static_cast<float>(bd[t] - bu)) * du) : 0.f;
+            const float w = KIND == PL_SCAN_MLSTM ? expf(static_cast<float>(du - bd[t]))
+                                                  : expf(static_cast<float>(bd[t] - bu)) * static_cast<float>(du);
+            acc[r] = (u <= t && t < L) ? acc[r] * w : 0.f;
         }
     }
     __syncthreads();                                                  // nobody reads B any more
@@ -521,9 +793,24 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             }
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] *= expf(static_cast<float>(bd[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)]));
+        for (int r = 0; r < 16; ++r) y[r] *= before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
     }
     __syncthreads();                                                  // the weighted scores are written
+    if (KIND == PL_SCAN_MLSTM) {
+        // n . q of a token, by four lanes: the weighted scores' sum and e^(m_0 - c_t) (n_0 . q_t)
+        const int t = tid >> 2, part = tid & 3;
+        float sum = 0.f, dot = 0.f;
+        if (t < L) {
+            const float* n0 = sa.nin + idx * N;
+            for (int u = part; u <= t; u += 4) sum += As[t * PA + u];
+            for (int i = part; i < N; i += 4) dot += n0[i] * Cs[t * P + i];
+        }
+        sum += before_w[t] * dot;
+        sum += __shfl_xor(sum, 1, 64);
+        sum += __shfl_xor(sum, 2, 64);
+        if (part == 0) below[t] = 1.f / (fmaxf(fabsf(sum), expf(below[t])) + 1e-6f);
+        __syncthreads();
+    }
     if (!columns) return;
     // ---- the weighted scores times x, and D x ----
     {
@@ -537,13 +824,17 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             }
         }
     }
-    const float skip = FIXED ? 0.f : a.p3[h];
+    const float skip = KIND == PL_SCAN_SSD ? a.p3[h] : 0.f;
     float* out = a.out + static_cast<size_t>(row0) * (H * V) + h * V;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int t = 32 * ti + 8 * (r >> 2) + 4 * half + (r & 3);
         // (token t's own x is the one this lane holds in the same place of its half of the chunk)
-        if (t < L && v < V) out[static_cast<size_t>(t) * (H * V) + v] = FIXED ? y[r] : y[r] + skip * (ti == 0 ? x[r] : x[16 + r]);
+        if (t >= L || v >= V) continue;
+        float o = y[r];
+        if (KIND == PL_SCAN_SSD) o += skip * (ti == 0 ? x[r] : x[16 + r]);
+        if (KIND == PL_SCAN_MLSTM) o *= below[t];
+        out[static_cast<size_t>(t) * (H * V) + v] = o;
     }
 }
 
@@ -583,22 +874,22 @@ extern "C" int pl_ssd_step(const float* qkv, int qkv_stride, int q_off, int k_of
     return 0;
 }
 
-template <bool FIXED>
+template <int KIND>
 static int launch_chunks(const SsdArgs& sa, int seqs, int max_q_len, hipStream_t stream) {
     const ScanArgs& a = sa.a;
     const int N = a.D, V = a.V, tiles = pl_ceil_div(V, 64);
     const dim3 grid(pl_ceil_div(max_q_len, SSD_CHUNK), a.H * tiles, seqs);
-    ssd_summary_kernel<FIXED><<<grid, 256, 0, stream>>>(sa);
+    ssd_summary_kernel<KIND><<<grid, 256, 0, stream>>>(sa);
     PL_CHECK_LAUNCH("ssd_chunked (summary)");
-    ssd_carry_kernel<<<dim3(pl_ceil_div(N * V, 256), a.H, seqs), 256, 0, stream>>>(sa);
+    ssd_carry_kernel<KIND><<<dim3(pl_ceil_div(N * (KIND == PL_SCAN_MLSTM ? V + 1 : V), 256), a.H, seqs), 256, 0, stream>>>(sa);
     PL_CHECK_LAUNCH("ssd_chunked (carry)");
     const int P = ((N + 7) & ~7) + 4;
-    const size_t lds = (3 * SSD_CHUNK + SSD_CHUNK * static_cast<size_t>(P) + SSD_CHUNK * static_cast<size_t>(P > SSD_CHUNK + 4 ? P : SSD_CHUNK + 4)) * sizeof(float);
+    const size_t lds = (6 * SSD_CHUNK + SSD_CHUNK * static_cast<size_t>(P) + SSD_CHUNK * static_cast<size_t>(P > SSD_CHUNK + 4 ? P : SSD_CHUNK + 4)) * sizeof(float);
     if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ssd_output_kernel<FIXED>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ssd_output_kernel<KIND>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
     }
-    ssd_output_kernel<FIXED><<<grid, 256, lds, stream>>>(sa, ssd_aligned(a) ? 1 : 0);
+    ssd_output_kernel<KIND><<<grid, 256, lds, stream>>>(sa, ssd_aligned(a) ? 1 : 0);
     PL_CHECK_LAUNCH("ssd_chunked (output)");
     return 0;
 }
@@ -616,8 +907,8 @@ extern "C" int pl_ssd_chunked(const float* qkv, int qkv_stride, int q_off, int k
     PL_REQUIRE(static_cast<long long>(H) * tiles <= 65535 && seqs >= 0 && seqs <= 65535, "ssd_chunked: %d heads of %d columns, %d requests", H, V, seqs);
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g_off, 0, a_log, dt_bias, skip, 0.f, state, state_stride,
-                      0, 0, 0, out, q_start, q_len, state_slots, H, G, N, V, from}, U, Sin, ends};
-    return launch_chunks<false>(sa, seqs, max_q_len, stream);
+                      0, 0, 0, out, q_start, q_len, state_slots, H, G, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
+    return launch_chunks<PL_SCAN_SSD>(sa, seqs, max_q_len, stream);
 }
 
 // Retention: S = decay S + k v^T, o = S^T q, q and k turning with their positions (HalfTurn; freq null: not at all).
@@ -666,6 +957,31 @@ extern "C" int pl_retention_chunked(const float* qkv, int qkv_stride, int q_off,
     PL_REQUIRE(static_cast<long long>(H) * pl_ceil_div(V, 64) <= 65535 && seqs >= 0 && seqs <= 65535, "retention_chunked: %d heads of %d columns, %d requests", H, V, seqs);
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, nullptr, 0, 0, 0, decay, nullptr, nullptr, 0.f, state, state_stride,
-                      0, 0, 0, out, q_start, q_len, state_slots, H, H, N, V, from}, U, Sin, ends};
-    return launch_chunks<true>(sa, seqs, max_q_len, stream);
+                      0, 0, 0, out, q_start, q_len, state_slots, H, H, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
+    return launch_chunks<PL_SCAN_RETENTION>(sa, seqs, max_q_len, stream);
+}
+
+// Linear attention with a fixed decay a head and silu on q, k and v (kind lightning), and the matrix memory with exponential gates
+// (kind mlstm): the requests of the step that bring at least `from` tokens; the others are the token-by-token kernel's.
+// U, Sin: room for (rows / 64 + requests) chunks of H * D * V floats; Uk, nin: of H * D (mlstm); scal: of H * 4.
+extern "C" int pl_recurrent_chunked(int kind, const float* qkv, int qkv_stride, int q_off, int k_off, int v_off,
+                                    const float* gates, int gates_stride, int g1_off, int g2_off,
+                                    const float* p1, const float* p2, float cap,
+                                    float* state, long state_stride, int s_off, int n_off, int m_off,
+                                    float* out, const int* q_start, const int* q_len, const int* state_slots,
+                                    int seqs, int max_q_len, int H, int D, int V, int from, int chunks,
+                                    float* U, float* Uk, float* Sin, float* nin, float* scal, hipStream_t stream) {
+    PL_REQUIRE(kind == PL_SCAN_LIGHTNING || kind == PL_SCAN_MLSTM, "recurrent_chunked: kind %d", kind);
+    PL_REQUIRE(H > 0 && D > 0 && D <= 256 && V > 0 && from >= 1, "recurrent_chunked: %d heads of %d by %d, from %d tokens", H, D, V, from);
+    PL_REQUIRE(p1 != nullptr && (kind == PL_SCAN_LIGHTNING || (gates != nullptr && p2 != nullptr && cap > 0.f)),
+               "recurrent_chunked: the gates of kind %d are missing", kind);
+    PL_REQUIRE(U != nullptr && Sin != nullptr && scal != nullptr && (kind == PL_SCAN_LIGHTNING || (Uk != nullptr && nin != nullptr)),
+               "recurrent_chunked: no room for the chunks' sums");
+    PL_REQUIRE(static_cast<long long>(H) * pl_ceil_div(V, 64) <= 65535 && seqs <= 65535, "recurrent_chunked: %d heads of %d columns, %d requests", H, V, seqs);
+    if (seqs == 0 || max_q_len < from) return 0;
+    const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, p1, p2, nullptr, cap, state, state_stride,
+                      s_off, n_off, m_off, out, q_start, q_len, state_slots, H, H, D, V, from},
+                     U, Sin, scal, Uk, nin, scal + static_cast<size_t>(chunks) * H};
+    return kind == PL_SCAN_LIGHTNING ? launch_chunks<PL_SCAN_LIGHTNING>(sa, seqs, max_q_len, stream)
+                                     : launch_chunks<PL_SCAN_MLSTM>(sa, seqs, max_q_len, stream);
 }

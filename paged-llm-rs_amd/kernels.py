@@ -65,7 +65,7 @@ def _signatures(lib) -> None:
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
                               i, i, i, i, i, i, p],
         "pl_recurrent_chunked": [i, p, i, i, i, i, p, i, i, i, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
-                                 i, i, i, i, i, i, p, p, p, p, p, p],
+                                 i, i, i, i, i, i, i, p, p, p, p, p, p],
         "pl_ssd_step": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p],
         "pl_ssd_step_applies": [i, ctypes.c_long],
         "pl_ssd_chunked": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p, p, p],
@@ -1324,7 +1324,8 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
               0 if gates is None else gates.shape[1], g1_off, g2_off, _ptr(p1), _ptr(p2), float(cap),
               state.data_ptr(), stride, 0, hdv, hdv + heads * tiles * dim, out.data_ptr(), batch.q_start.data_ptr(),
               batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
-    _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
+    if not chunked or batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0:
+        _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
     if chunked and kind == "delta":
         tokens = library().pl_recurrent_chunk_tokens(dim)
         chunks = (n // tokens + batch.num_seqs + 1) * heads
@@ -1340,19 +1341,19 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
             vdim, SCAN_CHUNKED_FROM, unit_k.data_ptr(), unit_q.data_ptr(), inverse.data_ptr(), masked.data_ptr(),
             scalars.data_ptr(), _stream()))
     elif chunked:
-        chunks = n // library().pl_recurrent_chunk_tokens(dim) + batch.num_seqs + 1
+        chunks = n // SSD_CHUNK + batch.num_seqs + 1
         f32 = dict(dtype=torch.float32, device=qkv.device)
         sums, before = torch.empty((chunks, hdv), **f32), torch.empty((chunks, hdv), **f32)
         k_sums, n_before = (torch.empty((chunks, heads * dim), **f32), torch.empty((chunks, heads * dim), **f32)) \
             if kind == "mlstm" else (None, None)
         scalars = torch.empty((chunks, heads * 4), **f32)
-        _check(library().pl_recurrent_chunked(*common, batch.max_q_len, heads, dim, vdim, SCAN_CHUNKED_FROM,
+        _check(library().pl_recurrent_chunked(*common, batch.max_q_len, heads, dim, vdim, SCAN_CHUNKED_FROM, chunks,
                                               sums.data_ptr(), _ptr(k_sums), before.data_ptr(), _ptr(n_before),
                                               scalars.data_ptr(), _stream()))
     return out
 
 
-SSD_CHUNK = 64       # tokens of a chunk of the state space's kernels
+SSD_CHUNK = 64       # tokens of a chunk of the kernels in chunks (the delta rule's say their own: pl_recurrent_chunk_tokens)
 
 
 def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch, H: int, G: int, N: int, V: int, gates,
@@ -1373,7 +1374,7 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
                                          out.data_ptr(), batch.q_start.data_ptr(), batch.q_len.data_ptr(),
                                          batch.state_slots.data_ptr(), batch.num_seqs, H, G, N, V, below, stream))
     if chunked:
-        chunks = n // library().pl_recurrent_chunk_tokens(dim) + batch.num_seqs + 1
+        chunks = n // SSD_CHUNK + batch.num_seqs + 1
         f32 = dict(dtype=torch.float32, device=qkv.device)
         sums, before = torch.empty((chunks, H * N * V), **f32), torch.empty((chunks, H * N * V), **f32)
         ends = torch.empty((chunks, H), **f32)

@@ -30,6 +30,8 @@ class _ScanMixer:
     """What they have in common: the fused projection and where its pieces lie in a row."""
 
     graph_safe = True
+    # requests that bring fewer tokens than this go token by token, which a step launches only where there are any
+    short_portion = kernels.SCAN_CHUNKED_FROM
 
     def _fuse(self, params: dict, names: list) -> None:
         self.columns, at = {}, 0
@@ -174,9 +176,6 @@ class StateSpace(_ScanMixer):
     gated by silu(z) first and normed then, in equal parts of all heads' values together.
     Tensors: ``in``, ``conv`` [channels, taps], ``conv.b``, ``dt_bias``, ``A_log``, ``D`` (one a head), ``norm``, ``o``."""
 
-    # requests that bring fewer tokens than this go through the scan token by token, which a step launches only where there are any
-    short_portion = kernels.SCAN_CHUNKED_FROM
-
     @staticmethod
     def declare(spec, hidden: int) -> list:
         H, inner = spec.num_heads, spec.num_heads * spec.value_dim
@@ -230,9 +229,6 @@ class StateSpace(_ScanMixer):
 class Retention(_ScanMixer):
     """Linear attention with a fixed decay a head and rotated queries and keys, no activations and no denominator; every head's read-out
     divided by its root mean square, times silu(gate).  Tensors: ``q``, ``k``, ``v``, ``g``, ``o``."""
-
-    # requests that bring fewer tokens than this go token by token, which a step launches only where there are any
-    short_portion = kernels.SCAN_CHUNKED_FROM
 
     @staticmethod
     def declare(spec, hidden: int) -> list:

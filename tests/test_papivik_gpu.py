@@ -334,3 +334,104 @@ def test_the_command_line_runs_the_design(tmp_path):
     assert done.returncode == 0, done.stderr[-2000:]
     lines = [json.loads(x) for x in done.stdout.splitlines() if x.startswith("{")]
     assert len(lines) == 2 and all(len(x["tokens"]) == 5 for x in lines), done.stdout
+
+
+# --- the recurrences' kernels alone ---------------------------------------------------------------------------------------
+
+class ScanStep:
+    """The part of a step's descriptor that the recurrences' kernels read; one more request holds rows of padding."""
+
+    def __init__(self, counts, slots, padding=2):
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32).cuda()
+        starts = np.concatenate([[0], np.cumsum(counts)])
+        self.num_tokens, self.num_seqs, self.max_q_len = int(starts[-1]) + padding, len(counts) + 1, max(max(counts), padding)
+        self.q_start, self.q_len, self.state_slots = i32(starts.tolist()), i32(list(counts) + [padding]), i32(list(slots) + [-1])
+        self.positions, self.seq_of = (torch.zeros(self.num_tokens, dtype=torch.int32).cuda() for _ in range(2))   # (not read)
+        self.counts = np.asarray(counts)
+
+    def tokens_of_short_requests(self, limit):
+        return int(self.counts[self.counts < limit].sum())
+
+
+def scan_in_64_bits(kind, q, k, v, x1, x2, p1, p2, cap):
+    """q, k [T, G, D], v [T, H, V], gates [T, H]: one request from an empty state, token by token."""
+    T, H, V = v.shape
+    D, silu = q.shape[2], torch.nn.functional.silu
+    q, k = (t.repeat_interleave(H // t.shape[1], 1) for t in (q, k))
+    S, n, m, out = torch.zeros(H, D, V, dtype=torch.float64), torch.zeros(H, D, dtype=torch.float64), torch.zeros(H, dtype=torch.float64), []
+    for t in range(T):
+        qt, kt, vt = q[t], k[t], v[t]
+        if kind == "lightning":
+            qt, kt, vt = silu(qt), silu(kt), silu(vt)
+            S = p1[:, None, None] * S + kt[:, :, None] * vt[:, None, :]
+            out.append((S * qt[:, :, None]).sum(1))
+        elif kind == "mlstm":
+            i, f = cap * torch.tanh((x1[t] + p1) / cap), torch.nn.functional.logsigmoid(cap * torch.tanh((x2[t] + p2) / cap))
+            top = torch.maximum(f + m, i)
+            keep, add, m = torch.exp(f + m - top), torch.exp(i - top), top
+            S = keep[:, None, None] * S + (add[:, None] * kt)[:, :, None] * vt[:, None, :]
+            n = keep[:, None] * n + add[:, None] * kt
+            qt = qt * D ** -0.5
+            out.append((S * qt[:, :, None]).sum(1) / (torch.maximum((n * qt).sum(-1).abs(), torch.exp(-m)) + 1e-6)[:, None])
+        else:
+            qt = qt / torch.sqrt((qt * qt).sum(-1, keepdim=True) + 1e-6) * D ** -0.5
+            kt = kt / torch.sqrt((kt * kt).sum(-1, keepdim=True) + 1e-6)
+            S = torch.exp(-torch.exp(p1) * torch.nn.functional.softplus(x2[t] + p2))[:, None, None] * S
+            u = torch.sigmoid(x1[t])[:, None] * (vt - (S * kt[:, :, None]).sum(1))
+            S = S + kt[:, :, None] * u[:, None, :]
+            out.append((S * qt[:, :, None]).sum(1))
+    return torch.stack(out)
+
+
+@pytest.mark.parametrize("kind", ["lightning", "mlstm", "delta"])
+@pytest.mark.parametrize("H,D,V", [(2, 16, 64), (1, 17, 4), (4, 1, 12), (3, 64, 60), (2, 100, 68), (4, 128, 128), (2, 129, 256), (1, 256, 72),
+                                   (2, 40, 70), (3, 20, 1)])
+def test_the_recurrences_kernels_in_portions(kind, H, D, V):
+    """Portions long enough for chunks (on both sides of one, two and three chunks), short ones and single tokens, from and into
+    the slots, against the recurrence in 64 bits; state columns that are whole quads (a kernel of four waves a state) and ones that
+    are not (the scan kernel).  Every sum is 32-bit: 3e-5 of the largest read-out, as for the state space's kernels."""
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator().manual_seed(H * 1000 + D + V)
+    G = H // 2 if kind == "delta" and H % 2 == 0 else H
+    T, cap, off = [194, 64, 3, 1, 65, 33], 5.0, 4
+    q, k = ([torch.randn((t, G, D), generator=g) for t in T] for _ in range(2))
+    v = [torch.randn((t, H, V), generator=g) for t in T]
+    x1, x2 = ([2 * torch.randn((t, H), generator=g) for t in T] for _ in range(2))
+    p1 = 1 - 0.5 * torch.rand((H,), generator=g) if kind == "lightning" else 0.5 * torch.randn((H,), generator=g)
+    p2 = 2 + torch.randn((H,), generator=g)
+    want = [scan_in_64_bits(kind, *(x[i].double() for x in (q, k, v, x1, x2)), p1.double(), p2.double(), cap).reshape(-1, H * V)
+            for i in range(len(T))]
+    scale = max(float(w.abs().max()) for w in want)
+    floats = kernels.scan_state_floats(kind, H, D, V)
+
+    def run(plan, slots):
+        state = torch.full((8, (floats + 8) // 4 * 4), 7.0).cuda()
+        state[:, :floats] = 0
+        at, got = {i: 0 for i in range(len(T))}, {i: [] for i in range(len(T))}
+        for step in plan:
+            b = ScanStep([c for _, c in step], [slots[i] for i, _ in step])
+            rows = torch.zeros((b.num_tokens, off + H * V + 2 * G * D))
+            gates = torch.zeros((b.num_tokens, 2 * H + 4))
+            r = 0
+            for i, c in step:
+                span = slice(at[i], at[i] + c)
+                rows[r:r + c, off:] = torch.cat([v[i][span].flatten(1), k[i][span].flatten(1), q[i][span].flatten(1)], -1)
+                gates[r:r + c, 4:] = torch.cat([x1[i][span], x2[i][span]], -1)
+                r += c
+            out = kernels.recurrent_scan(kind, rows.cuda(), off + H * V + G * D, off + H * V, off, state[:, :floats], b, H, G, D, V,
+                                         gates=None if kind == "lightning" else gates.cuda(), g1_off=4, g2_off=4 + H, p1=p1.cuda(),
+                                         p2=None if kind == "lightning" else p2.cuda(), cap=cap, chunked=True).double().cpu()
+            r = 0
+            for i, c in step:
+                got[i].append(out[r:r + c])
+                at[i] += c
+                r += c
+        assert (state[:, floats:] == 7.0).all(), "nothing beside the state is touched"
+        for i, pieces in got.items():
+            err = float((torch.cat(pieces) - want[i]).abs().max()) / scale
+            assert err <= 3e-5, (i, err)
+
+    run([[(i, t) for i, t in enumerate(T)]], [5, 0, 3, 1, 7, 2])
+    run([[(0, 15), (1, 16), (2, 1), (4, 63)], [(0, 64), (2, 1), (1, 48), (5, 2)], [(0, 1), (3, 1), (4, 2), (2, 1)], [(0, 114), (5, 31)]],
+        [0, 1, 2, 3, 4, 5])
