@@ -225,6 +225,8 @@ struct ad_extras_t<0> {
 struct ad_true_t { static constexpr bool value = true; };
 struct ad_false_t { static constexpr bool value = false; };
 
+#define AD_MERGE_AT_ONCE 8      // shares whose results are on their way together when they are put together
+
 template <int LPK, int GT, int U, int WV, int EX = 0>
 __global__ void __launch_bounds__(64 * WV)
 paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
@@ -234,7 +236,7 @@ paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t
                               const int* __restrict__ block_table, int max_blocks, int block_size,
                               bf16_t* __restrict__ k_pool, bf16_t* __restrict__ v_pool, int nq,
                               int nkv, int d, float scale_log2e, int window, int splits, int tiles, int g,
-                              uint32_t splits_magic, ad_fuse_t fuse, ad_extras_t<EX> extras) {
+                              uint32_t splits_magic, ad_fuse_t fuse, int* __restrict__ arrivals, ad_extras_t<EX> extras) {
     const float* const sinks = extras.sinks;
     const float* const slopes = extras.slopes;
     constexpr int KPW = PL_WAVE / LPK;  // keys a wave handles with one load
@@ -573,6 +575,23 @@ paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t
             }
         }
     }
+    auto finish = [&](int h, int dd, float big, float sum, float a) {
+        float opened = 1.f;
+        if constexpr (EX == 2) {
+            if (extras.more.gate != nullptr) opened = pl_head_gate(extras.more, t, h);
+        }
+        if constexpr (EX != 0) {
+            if (sinks != nullptr) {
+                // a sink: one more term of the denominator, unscaled, with no value behind it
+                const float sk = sinks[h] * 1.4426950408889634f;
+                const float top = fmaxf(big, sk);
+                const float keep = big == -INFINITY ? 0.f : exp2f(big - top);
+                sum = sum * keep + exp2f(sk - top);
+                a *= keep;
+            }
+        }
+        out[(static_cast<size_t>(t) * nq + h) * d + dd] = from_float<bf16_t>(sum > 0.f ? a / sum * opened : 0.f);
+    };
     __syncthreads();
     for (int idx = threadIdx.x; idx < heads * d; idx += blockDim.x) {
         const int hq = idx / d, dd = idx % d;
@@ -591,36 +610,57 @@ paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t
         }
         const int h = h0 + hq;
         if (splits == 1) {
-            float opened = 1.f;
-            if constexpr (EX == 2) {
-                if (extras.more.gate != nullptr) opened = pl_head_gate(extras.more, t, h);
-            }
-            if constexpr (EX != 0) {
-                if (sinks != nullptr) {
-                    // a sink: one more term of the denominator, unscaled, with no value behind it
-                    const float sk = sinks[h] * 1.4426950408889634f;
-                    const float top = fmaxf(big, sk);
-                    const float keep = big == -INFINITY ? 0.f : exp2f(big - top);
-                    sum = sum * keep + exp2f(sk - top);
-                    a *= keep;
-                }
-            }
-            out[(static_cast<size_t>(t) * nq + h) * d + dd] = from_float<bf16_t>(sum > 0.f ? a / sum * opened : 0.f);
+            finish(h, dd, big, sum, a);
         } else {
             const size_t pi = (static_cast<size_t>(t) * nq + h) * splits + split;
-            part_acc[pi * d + dd] = a;
+            pl_share(part_acc + pi * d + dd, a);
             if (dd == 0) {
-                part_ml[pi * 2] = big;
-                part_ml[pi * 2 + 1] = sum;
+                pl_share(part_ml + pi * 2, big);
+                pl_share(part_ml + pi * 2 + 1, sum);
             }
         }
+    }
+    if (splits == 1 || arrivals == nullptr) return;
+    // The last of the shares to arrive puts them together, in their order whichever it is.
+    pl_shares_written();
+    __syncthreads();
+    if (threadIdx.x == 0) pages_lds[0] = pl_arrive(arrivals + static_cast<size_t>(t) * nq + h0, splits) ? 1 : 0;
+    __syncthreads();
+    if (pages_lds[0] == 0) return;
+    for (int idx = threadIdx.x; idx < heads * d; idx += blockDim.x) {
+        const int hq = idx / d, dd = idx % d, h = h0 + hq;
+        const size_t base = (static_cast<size_t>(t) * nq + h) * splits;
+        float big = -INFINITY, sum = 0.f, a = 0.f;
+        for (int s0 = 0; s0 < splits; s0 += AD_MERGE_AT_ONCE) {
+            float ms[AD_MERGE_AT_ONCE], ls[AD_MERGE_AT_ONCE], as[AD_MERGE_AT_ONCE];
+#pragma unroll
+            for (int i = 0; i < AD_MERGE_AT_ONCE; ++i) {
+                const size_t at = base + min(s0 + i, splits - 1);
+                ms[i] = pl_shared(part_ml + at * 2);
+                ls[i] = pl_shared(part_ml + at * 2 + 1);
+                as[i] = pl_shared(part_acc + at * d + dd);
+            }
+            float top = big;
+#pragma unroll
+            for (int i = 0; i < AD_MERGE_AT_ONCE; ++i) top = fmaxf(top, s0 + i < splits ? ms[i] : -INFINITY);
+            const float keep = big == -INFINITY ? 0.f : exp2f(big - top);
+            sum *= keep;
+            a *= keep;
+            big = top;
+#pragma unroll
+            for (int i = 0; i < AD_MERGE_AT_ONCE; ++i) {
+                const float w = (s0 + i < splits && ms[i] != -INFINITY) ? exp2f(ms[i] - big) : 0.f;
+                sum = fmaf(ls[i], w, sum);
+                a = fmaf(as[i], w, a);
+            }
+        }
+        finish(h, dd, big, sum, a);
     }
 }
 
 // Merges the splits of one (token, query head): out = sum_s a_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).
-// (The merge is a kernel of its own because the end of a kernel is the cheapest way on this chip to make
-// one workgroup's results visible to another: a device-wide fence inside a kernel writes back and
-// invalidates a whole L2.)  One thread an output element; every load is asked for before any is used.
+// For launches without room for their workgroups' arrivals.  One thread an output element; every load is asked for before
+// any is used.
 #define AD_MAX_SPLITS 64
 
 template <int SP, bool EX = false>
@@ -687,7 +727,7 @@ static int launch_decode_keys(const void* q, int q_stride, void* out, float* par
                               const int* positions, const int* seq_of, const int* q_len, int short_limit, int num_seqs,
                               int short_rows, const int* block_table, int max_blocks, int block_size, void* k_pool,
                               void* v_pool, int n, int nq, int nkv, int d, float scale, int window, int splits,
-                              const ad_fuse_t& fuse, const float* sinks, const float* slopes,
+                              const ad_fuse_t& fuse, int* arrivals, const float* sinks, const float* slopes,
                               const PlAttentionMore& more, hipStream_t stream) {
     constexpr int WV = AD_WAVES;
     const int g = nq / nkv;
@@ -711,7 +751,7 @@ static int launch_decode_keys(const void* q, int q_stride, void* out, float* par
         static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out), part_acc, part_ml, positions, seq_of,      \
         q_len, short_limit, compact ? num_seqs : 0, block_table, max_blocks, block_size, static_cast<bf16_t*>(k_pool), \
         static_cast<bf16_t*>(v_pool), nq, nkv, d, scale * 1.4426950408889634f, window, splits, tiles, g,              \
-        static_cast<uint32_t>((0x100000000ull + splits - 1) / static_cast<unsigned>(splits)), fuse, with)
+        static_cast<uint32_t>((0x100000000ull + splits - 1) / static_cast<unsigned>(splits)), fuse, arrivals, with)
     if (extras == 2) {
         const ad_extras_t<2> with{sinks, slopes, more};
         AD_LAUNCH(2);
@@ -724,7 +764,7 @@ static int launch_decode_keys(const void* q, int q_stride, void* out, float* par
     }
 #undef AD_LAUNCH
     PL_CHECK_LAUNCH("paged_attention_decode");
-    if (splits > 1) {
+    if (splits > 1 && arrivals == nullptr) {
         const dim3 mgrid = dim3(pl_ceil_div(nq * d, 256), compact ? short_rows : n);
 #define AD_MERGE(SP)                                                                                              \
     do {                                                                                                          \
@@ -759,13 +799,13 @@ static int launch_decode(const void* q, int q_stride, void* out, float* part_acc
                          const int* positions, const int* seq_of, const int* q_len, int short_limit, int num_seqs,
                          int short_rows, const int* block_table, int max_blocks, int block_size, void* k_pool,
                          void* v_pool, int n, int nq, int nkv, int d, float scale, int window, int splits,
-                         const ad_fuse_t& fuse, const float* sinks, const float* slopes,
+                         const ad_fuse_t& fuse, int* arrivals, const float* sinks, const float* slopes,
                               const PlAttentionMore& more, hipStream_t stream) {
     const long long workgroups = static_cast<long long>(nkv) * pl_ceil_div(nq / nkv, GT) * n * splits;
 #define AD_KEYS_CALL(U)                                                                                            \
     return launch_decode_keys<LPK, GT, U>(q, q_stride, out, part_acc, part_ml, positions, seq_of, q_len,          \
                                           short_limit, num_seqs, short_rows, block_table, max_blocks, block_size,  \
-                                          k_pool, v_pool, n, nq, nkv, d, scale, window, splits, fuse, sinks, slopes, more, stream)
+                                          k_pool, v_pool, n, nq, nkv, d, scale, window, splits, fuse, arrivals, sinks, slopes, more, stream)
     if constexpr (GT <= 2) {
         if (workgroups <= pl_compute_units()) AD_KEYS_CALL(8);
         AD_KEYS_CALL(4);
@@ -780,12 +820,12 @@ static int dispatch_gt(int gt, const void* q, int q_stride, void* out, float* pa
                        const int* positions, const int* seq_of, const int* q_len, int short_limit, int num_seqs,
                        int short_rows, const int* block_table, int max_blocks, int block_size, void* k_pool,
                        void* v_pool, int n, int nq, int nkv, int d, float scale, int window, int splits,
-                       const ad_fuse_t& fuse, const float* sinks, const float* slopes,
+                       const ad_fuse_t& fuse, int* arrivals, const float* sinks, const float* slopes,
                               const PlAttentionMore& more, hipStream_t stream) {
 #define AD_CALL(G)                                                                                              \
     return launch_decode<LPK, G>(q, q_stride, out, part_acc, part_ml, positions, seq_of, q_len, short_limit,   \
                                  num_seqs, short_rows, block_table, max_blocks, block_size, k_pool, v_pool, n, nq, nkv, d, scale,    \
-                                 window, splits, fuse, sinks, slopes, more, stream)
+                                 window, splits, fuse, arrivals, sinks, slopes, more, stream)
     switch (gt) {
         case 1: AD_CALL(1);
         case 2: AD_CALL(2);
@@ -804,6 +844,8 @@ static int dispatch_gt(int gt, const void* q, int q_stride, void* out, float* pa
 // the raw projection and are normalised (gains, eps) and rotated (tables, rot a multiple of 16) here.  2: as 1, and
 // each token's key and value are taken raw from its row [q | k | v], used, and written into the cache; every
 // request then has to bring exactly one token.
+// `arrivals`: n * nq zeros, and zeros again behind the launch, for the shares' workgroups to meet at; null: the shares are put
+// together by a second kernel.
 extern "C" int pl_paged_attention_decode(const void* q, int q_stride, void* out, float* part_acc, float* part_ml,
                                          const int* positions, const int* seq_of, const int* q_len, int short_limit,
                                          int num_seqs, int short_rows,
@@ -812,7 +854,7 @@ extern "C" int pl_paged_attention_decode(const void* q, int q_stride, void* out,
                                          int splits, int fuse_mode, const void* q_gain, const void* k_gain,
                                          int gain_dtype, float eps, const float* cos_table, const float* sin_table,
                                          int rot, const float* sinks, const float* slopes, float cap, int keep,
-                                         const float* gate, int gate_stride, hipStream_t stream) {
+                                         const float* gate, int gate_stride, int* arrivals, hipStream_t stream) {
     const PlAttentionMore more{cap, keep, gate, gate_stride};
     PL_REQUIRE(cap >= 0.f && keep >= 0 && (gate == nullptr || gate_stride >= nq) && (keep == 0 || window >= 0),
                "decode attention: a cap of %g, %d first keys kept beside a window of %d, gates in rows of %d",
@@ -841,7 +883,7 @@ extern "C" int pl_paged_attention_decode(const void* q, int q_stride, void* out,
 #define AD_LPK(L)                                                                                                  \
     return dispatch_gt<L>(gt, q, q_stride, out, part_acc, part_ml, positions, seq_of, q_len, short_limit,        \
                           num_seqs, short_rows, block_table, max_blocks, block_size, k_pool, v_pool, n, nq, nkv, d, scale, window,      \
-                          splits, fuse, sinks, slopes, more, stream)
+                          splits, fuse, arrivals, sinks, slopes, more, stream)
     if (chunks <= 2) AD_LPK(2);
     if (chunks <= 4) AD_LPK(4);
     if (chunks <= 8) AD_LPK(8);

@@ -33,6 +33,11 @@ class StepEntry:
     fed_row: int = -1
 
 
+# Steps of up to so many rows bring room for the arrivals of attention workgroups that share the keys of a row (an int32 a row and
+# query head, up to so many heads); the keys of larger steps' rows are seldom shared out, and a second kernel puts them together.
+ARRIVAL_ROWS, ARRIVAL_HEADS = 1024, 64
+
+
 class StepBatch:
     """Device tensors of one step (all int32)."""
 
@@ -55,6 +60,10 @@ class StepBatch:
                             else np.asarray(tokens_each, dtype=np.int64))
         self.padded = padded
         self.short_bounds = dict(short_bounds or {})
+        # Zeros between any two kernels (``kernels.paged_attention_decode``).  They belong to this step alone: steps on other
+        # streams, of this cache or of another, count in their own.
+        self.arrivals = (torch.zeros(num_tokens * ARRIVAL_HEADS, dtype=torch.int32, device=packed.device)
+                         if packed.is_cuda and num_tokens <= ARRIVAL_ROWS else None)
 
         def view(name, *shape):
             begin, count = layout[name]

@@ -58,8 +58,8 @@ def _signatures(lib) -> None:
         "pl_gemm_stream_splits": [i, i, i, i],
         "pl_gemm_finish": [p, p, ctypes.c_longlong, i, i, i, i, i, p],
         "pl_paged_attention_decode": [p, i, p, p, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, i, f, i, i,
-                                      i, p, p, i, f, p, p, i, p, p, f, i, p, i, p],
-        "pl_paged_attention_prefill": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, p, p, f, i, p, i, p],
+                                      i, p, p, i, f, p, p, i, p, p, f, i, p, i, p, p],
+        "pl_paged_attention_prefill": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, p, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped_applies": [i, i, i, i],
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
@@ -476,6 +476,19 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     return out
 
 
+def _arrivals_ptr(arrivals, count: int) -> int:
+    """Room for ``count`` arrivals, or none (the kernels then leave the merging of shares to a second one)."""
+    if arrivals is None or arrivals.numel() < count:
+        return 0
+    return _need(arrivals, "arrivals", None, torch.int32).data_ptr()
+
+
+def _arrivals(batch, nq: int):
+    """The step's room for the arrivals of its shares' workgroups, where it has enough for ``nq`` heads."""
+    room = getattr(batch, "arrivals", None)
+    return room if room is not None and room.numel() >= batch.num_tokens * nq else None
+
+
 _attention_mode = "kernel"
 
 # A request that brings fewer tokens than this to a step has each of them served
@@ -541,8 +554,11 @@ def paged_attention_decode(q: torch.Tensor, q_row_stride: int, out: torch.Tensor
                            window: int = 0, splits: int = 1, q_len: torch.Tensor | None = None,
                            short_limit: int = 0, fuse: "QkFusion | None" = None, live_seqs: int | None = None,
                            short_rows: int = 0, sinks: torch.Tensor | None = None,
-                           slopes: torch.Tensor | None = None, more: AttentionMore | None = None) -> torch.Tensor:
-    """bfloat16 attention of single tokens over their requests' pages, split along the context.
+                           slopes: torch.Tensor | None = None, more: AttentionMore | None = None,
+                           arrivals: torch.Tensor | None = None) -> torch.Tensor:
+    """bfloat16 attention of single tokens over their requests' pages, split along the context.  ``arrivals``: at least n * nq
+    int32 zeros (zeros again behind the launch, for the next one on the same stream) where the workgroups of a token's shares
+    count themselves, the last of which puts them together; without, a second kernel does.
     With ``q_len`` the tokens of requests with ``short_limit`` tokens or more are left out; ``short_rows``
     then bounds the tokens that the other requests bring (0: not known) and ``live_seqs`` says how many
     requests, the first ones, bring tokens, so that the launch has workgroups for those tokens only.
@@ -592,7 +608,7 @@ def paged_attention_decode(q: torch.Tensor, q_row_stride: int, out: torch.Tensor
         block_table.data_ptr(), block_table.shape[1], block_size,
         k_pool.data_ptr(), v_pool.data_ptr(), n, nq, nkv, d, float(scale), int(window or 0), int(splits),
         mode, _ptr(q_gain), _ptr(k_gain), gain_code, float(eps), _ptr(cos), _ptr(sin), int(rot), _ptr(sinks),
-        _ptr(slopes), *_more_args(more, nq, n), _stream()))
+        _ptr(slopes), *_more_args(more, nq, n), _arrivals_ptr(arrivals, n * nq), _stream()))
     return out
 
 
@@ -614,13 +630,14 @@ def paged_attention_prefill(q: torch.Tensor, q_row_stride: int, out: torch.Tenso
                             scale: float, window: int = 0, short_limit: int = 0, max_ctx: int | None = None,
                             splits: int | None = None, live_seqs: int | None = None,
                             sinks: torch.Tensor | None = None, slopes: torch.Tensor | None = None,
-                            more: AttentionMore | None = None) -> torch.Tensor:
+                            more: AttentionMore | None = None, arrivals: torch.Tensor | None = None) -> torch.Tensor:
     """bfloat16 attention of prompt portions on the matrix cores.  Request s brings the rows
     q_start[s] .. q_start[s]+q_len[s]-1 at the positions ctx_len[s]-q_len[s] .. ctx_len[s]-1;
     requests with fewer than ``short_limit`` tokens are skipped.  ``max_ctx`` (the longest context
     of the step) lets the keys of a token tile be dealt to several workgroups where the tiles alone
     would leave compute units idle; ``splits`` sets their number by hand.  ``live_seqs``: only so many
-    of the requests, the first ones, bring tokens (the rest is padding and gets no workgroups)."""
+    of the requests, the first ones, bring tokens (the rest is padding and gets no workgroups).  ``arrivals``: as for
+    ``paged_attention_decode``."""
     n = q.shape[0]
     S = block_table.shape[0]
     _need(q, "query buffer", None, torch.bfloat16)
@@ -650,7 +667,7 @@ def paged_attention_prefill(q: torch.Tensor, q_row_stride: int, out: torch.Tenso
         q.data_ptr(), q_row_stride, out.data_ptr(), q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(),
         int(short_limit), live, int(max_q_len), block_table.data_ptr(), block_table.shape[1], block_size,
         k_pool.data_ptr(), v_pool.data_ptr(), nq, nkv, d, float(scale), int(window or 0), int(splits),
-        part_acc.data_ptr() if splits > 1 else None, part_ml.data_ptr() if splits > 1 else None, n,
+        _arrivals_ptr(arrivals, n * nq), part_acc.data_ptr() if splits > 1 else None, part_ml.data_ptr() if splits > 1 else None, n,
         _ptr(_head_numbers(sinks, "sinks", nq)), _ptr(_head_numbers(slopes, "distance slopes", nq)),
         *_more_args(more, nq, n), _stream()))
     return out
@@ -778,7 +795,7 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
         splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d)
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
-                                      fuse=prepare)
+                                      fuse=prepare, arrivals=_arrivals(batch, nq))
     qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
                           batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
                           nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)
@@ -817,7 +834,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
         paged_attention_prefill(qkv, stride, out, batch.q_start, batch.q_len, batch.ctx_len, batch.max_q_len,
                                 kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window,
                                 short_limit=0 if all_tiled else SHORT_PORTION, max_ctx=batch.max_ctx_len,
-                                live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more)
+                                live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more,
+                                arrivals=_arrivals(batch, nq))
         if short_tokens == 0 or all_tiled:
             return out
     mixed = batch.max_q_len >= SHORT_PORTION
@@ -837,7 +855,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                                   kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                   q_len=batch.q_len if mixed else None, short_limit=SHORT_PORTION if mixed else 0,
                                   live_seqs=getattr(batch, "live_seqs", None), short_rows=short_tokens,
-                                  sinks=sinks, slopes=slopes, more=more)
+                                  sinks=sinks, slopes=slopes, more=more, arrivals=_arrivals(batch, nq))
 
 
 class HandedNorm:

@@ -1590,6 +1590,49 @@ def test_a_norm_handed_forward_from_one_product_to_the_next(n, H, deep, N2, swig
         assert rel(got, own.double()) < 1e-2
 
 
+@pytest.mark.parametrize("window", [0, 40])
+def test_shares_that_meet_in_the_kernel_and_shares_merged_by_a_second(window):
+    """Single tokens and portions in one to eight shares, with room for the workgroups' arrivals and without,
+    over contexts that leave some shares without keys: the same up to the order in which shares past the eighth join (one
+    rounding to bfloat16), the same bits again in the next launch, and the room is zeros again behind every one."""
+    from paged_llm_rs_amd import kernels
+
+    bs, requests = 16, [(300, 1), (9, 1), (700, 3), (70, 40), (1000, 130), (64, 64), (1, 1)]
+    ctx = [c for c, _ in requests]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    q_len = i32([t for _, t in requests])
+    q_start = i32([0] + torch.cumsum(q_len, 0)[:-1].tolist())
+    n = int(q_len.sum())
+    positions = i32([c - t + k for c, t in requests for k in range(t)])
+    seq_of = i32([s for s, (_, t) in enumerate(requests) for _ in range(t)])
+    for nq, nkv, d in ((4, 2, 128), (6, 3, 64), (16, 2, 128), (3, 1, 80)):
+        bt, k_pool, v_pool, _, _ = build_paged(nkv, d, bs, ctx, torch.bfloat16, seed=d)
+        give_back_pages_behind_the_window(bt, k_pool, v_pool, bs, requests, window)
+        stride = (nq + 2 * nkv) * d
+        q = torch.randn(n, stride, device=DEV).bfloat16()
+        sinks = torch.randn(nq, device=DEV)
+        arrivals = torch.zeros(n * nq, dtype=torch.int32, device=DEV)
+        paged = (bt, bs, k_pool, v_pool, nq, nkv, d, d ** -0.5, window)
+
+        def single(splits, **more):
+            out = torch.full((n, nq * d), 7.0, device=DEV).bfloat16()
+            return kernels.paged_attention_decode(q, stride, out, positions, seq_of, *paged, splits, sinks=sinks, **more)
+
+        def tiled(splits, **more):
+            out = torch.full((n, nq * d), 7.0, device=DEV).bfloat16()
+            return kernels.paged_attention_prefill(q, stride, out, q_start, q_len, i32(ctx), 130, *paged, short_limit=3, splits=splits,
+                                                   sinks=sinks, **more)
+
+        for kernel in (single, tiled):
+            for splits in (1, 2, 3, 4, 8) + ((16,) if kernel is single else ()):
+                want = kernel(splits)
+                got = kernel(splits, arrivals=arrivals)
+                assert rel(got, want) < 2e-3, (kernel.__name__, nq, d, splits)
+                assert torch.equal(got == 7.0, want == 7.0), "rows that are not the kernel's stay as they were"
+                assert torch.equal(got, kernel(splits, arrivals=arrivals)), (kernel.__name__, nq, d, splits)
+                assert not bool(arrivals.any())
+
+
 def attention_with_everything(q, keys, values, pos, g, scale, window, sinks, slopes, more, row):
     """One token in 64 bits: q [nq, d], keys and values [ctx, nkv, d]; a key set to None's place (NaN rows never seen) is masked."""
     if window > 0:
