@@ -72,9 +72,8 @@ def _signatures(lib) -> None:
         "pl_retention_turn": [p, i, i, i, i, i, i, p, i, f, f, p, p],
         "pl_retention_step": [p, i, i, i, i, p, p, i, f, f, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, p],
         "pl_retention_chunked": [p, i, i, i, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p, p, p, p],
-        "pl_recurrent_chunk_tokens": [i],
         "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i,
-                             p, p, p, p, p, p],
+                             p, p, p, p, p, p, p],
         "pl_short_conv": [p, i, i, i, p, i, p, ctypes.c_long, i, p, p, p, p, p, i, p, i, i, p],
         "pl_conv_history": [p, i, i, i, i, p, ctypes.c_long, i, p, p, p, i, p],
         "pl_gated_group_norm": [p, i, i, i, p, i, f, p, i, i, i, i, p, i, p],
@@ -1345,18 +1344,17 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
     if not chunked or batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0:
         _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
     if chunked and kind == "delta":
-        tokens = library().pl_recurrent_chunk_tokens(dim)
-        chunks = (n // tokens + batch.num_seqs + 1) * heads
+        chunks = (n // SSD_CHUNK + batch.num_seqs + 1) * heads
         f32 = dict(dtype=torch.float32, device=qkv.device)
-        padded = (dim + 3) // 4 * 4
-        unit_k, unit_q = torch.empty((chunks, tokens * padded), **f32), torch.empty((chunks, tokens * padded), **f32)
-        inverse, masked = torch.empty((chunks, tokens * tokens), **f32), torch.empty((chunks, tokens * tokens), **f32)
-        scalars = torch.empty((chunks, 3 * tokens), **f32)
+        padded = (dim + 63) // 64 * 64
+        unit_k, unit_q, weighted_k = (torch.empty((chunks, SSD_CHUNK * padded), **f32) for _ in range(3))
+        inverse, masked = torch.empty((chunks, SSD_CHUNK * SSD_CHUNK), **f32), torch.empty((chunks, SSD_CHUNK * SSD_CHUNK), **f32)
+        scalars = torch.empty((chunks, 2 * SSD_CHUNK), **f32)
         _check(library().pl_delta_chunked(
             qkv.data_ptr(), width, q_off, k_off, v_off, gates.data_ptr(), gates.shape[1], g1_off, g2_off,
             p1.data_ptr(), p2.data_ptr(), state.data_ptr(), stride, out.data_ptr(), batch.q_start.data_ptr(),
             batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs, batch.max_q_len, heads, qk_heads, dim,
-            vdim, SCAN_CHUNKED_FROM, unit_k.data_ptr(), unit_q.data_ptr(), inverse.data_ptr(), masked.data_ptr(),
+            vdim, SCAN_CHUNKED_FROM, unit_k.data_ptr(), unit_q.data_ptr(), weighted_k.data_ptr(), inverse.data_ptr(), masked.data_ptr(),
             scalars.data_ptr(), _stream()))
     elif chunked:
         chunks = n // SSD_CHUNK + batch.num_seqs + 1
@@ -1371,7 +1369,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
     return out
 
 
-SSD_CHUNK = 64       # tokens of a chunk of the kernels in chunks (the delta rule's say their own: pl_recurrent_chunk_tokens)
+SSD_CHUNK = 64       # tokens of a chunk of the kernels in chunks
 
 
 def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch, H: int, G: int, N: int, V: int, gates,
