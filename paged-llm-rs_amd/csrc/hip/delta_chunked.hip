@@ -57,9 +57,9 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
     const size_t idx = static_cast<size_t>(delta_chunk_number(a, s, c_at)) * H + h;
     const int P = Dp + 4;
     double* bd = reinterpret_cast<double*>(lds);        // [64] b_t, the sum of log decays
-    float* be = lds + 2 * DL_C;                         // [64] beta_t
-    float* nrm = be + DL_C;                             // [2][64]
-    float* qs = nrm + 2 * DL_C;                         // [64][P]
+    double* nrm = bd + DL_C;                            // [2][64]
+    float* be = lds + 6 * DL_C;                         // [64] beta_t
+    float* qs = be + DL_C;                              // [64][P]
     float* ks = qs + DL_C * P;                          // [64][P]
     float* M = qs;                                      // [64][DL_T], where q lay
     float* T = ks;                                      // [64][DL_T], where k lay
@@ -98,9 +98,10 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
     {
         // four lanes a row of q and one of k
         const int t = tid >> 2, part = tid & 3;
-        float qq = 0.f, kk = 0.f;
+        // (a norm's rounding would stand in all of its row: 64-bit sums)
+        double qq = 0.0, kk = 0.0;
         for (int i = part; i < Dp; i += 4) {
-            const float q = qs[t * P + i], k = ks[t * P + i];
+            const double q = qs[t * P + i], k = ks[t * P + i];
             qq += q * q;
             kk += k * k;
         }
@@ -109,8 +110,8 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
         qq += __shfl_xor(qq, 2, 64);
         kk += __shfl_xor(kk, 2, 64);
         if (part == 0) {
-            nrm[t] = 1.f / sqrtf(qq + 1e-6f) * (1.f / sqrtf(static_cast<float>(D)));
-            nrm[DL_C + t] = 1.f / sqrtf(kk + 1e-6f);
+            nrm[t] = 1.0 / sqrt((qq + 1e-6) * D);
+            nrm[DL_C + t] = 1.0 / sqrt(kk + 1e-6);
         }
     }
     __syncthreads();
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
     float* Qn = da.Qn + idx * DL_C * Dp;
     for (int e = tid; e < DL_C * Dp; e += 256) {
         const int t = e / Dp, i = e - t * Dp;
-        const float q = qs[t * P + i] * nrm[t], k = ks[t * P + i] * nrm[DL_C + t];
+        const float q = static_cast<float>(qs[t * P + i] * nrm[t]), k = static_cast<float>(ks[t * P + i] * nrm[DL_C + t]);
         qs[t * P + i] = q;
         ks[t * P + i] = k;
         Qn[e] = q;
@@ -135,15 +136,27 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
     dl_f32x4 kk[4], qk[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) kk[j] = qk[j] = dl_f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < Dp; i += 16) {
-        const dl_f32x4 ka = dl_read4(ks + (16 * wave + r) * P + i + 4 * c), qa = dl_read4(qs + (16 * wave + r) * P + i + 4 * c);
+    for (int i = 0; i < Dp; i += 64) {                  // (64 of D a chain, the chains added)
+        dl_f32x4 kc[4], qc[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j <= wave) {
-                const dl_f32x4 kb = dl_read4(ks + (16 * j + r) * P + i + 4 * c);
-                kk[j] = dl_multiply(ka, kb, kk[j]);
-                qk[j] = dl_multiply(qa, kb, qk[j]);
-            }
+        for (int j = 0; j < 4; ++j) kc[j] = qc[j] = dl_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int at = i + 16 * e + 4 * c;
+            const dl_f32x4 ka = dl_read4(ks + (16 * wave + r) * P + at), qa = dl_read4(qs + (16 * wave + r) * P + at);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j <= wave) {
+                    const dl_f32x4 kb = dl_read4(ks + (16 * j + r) * P + at);
+                    kc[j] = dl_multiply(ka, kb, kc[j]);
+                    qc[j] = dl_multiply(qa, kb, qc[j]);
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            kk[j] += kc[j];
+            qk[j] += qc[j];
+        }
     }
     __syncthreads();                                    // q and k are done with
     float* Aq = da.Aq + idx * DL_C * DL_C;
@@ -345,7 +358,7 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs da) {
 static int launch_delta(const DeltaArgs& da, int seqs, int max_q_len, hipStream_t stream) {
     const ScanArgs& a = da.a;
     const int Dp = pl_ceil_div(a.D, 64) * 64, P = Dp + 4;
-    const size_t lds_p = (5 * DL_C + 2 * static_cast<size_t>(DL_C) * (P > DL_T ? P : DL_T)) * sizeof(float);
+    const size_t lds_p = (7 * DL_C + 2 * static_cast<size_t>(DL_C) * (P > DL_T ? P : DL_T)) * sizeof(float);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prepare_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(lds_p));
     PL_REQUIRE(e == hipSuccess, "delta_chunked: %zu bytes of LDS refused: %s", lds_p, hipGetErrorString(e));
