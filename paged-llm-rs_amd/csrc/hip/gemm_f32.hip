@@ -57,72 +57,98 @@ __device__ __forceinline__ void f32_store4(float* to, f32x4 v, int col, int N, b
 // Bound by the weights' bytes.  A workgroup of sixteen waves owns 16 columns and TN x 16 rows of x; a wave takes one part
 // of K straight from memory in the instruction's layout, 64 k a round, and the parts meet in LDS.  Also the product of many
 // rows whose rows are not made of aligned groups of four values (VEC false, a row tile a blockIdx.y).
-template <int TN, bool VEC>
-__global__ void __launch_bounds__(PL_F32_PARTS * PL_WAVE)
+//
+// With at most 8 rows of x half of the instruction's 16 would be copies.  SHARE 2 gives that half to another part of K: a wave takes
+// two parts of 8 columns, rows 0 .. 7 of its operands from one part and 8 .. 15 from the next, and of the result keeps the two
+// blocks of 8 x 8 whose operands belong together (each element the same chain as before); SHARE 4 four parts of 4 columns
+// for at most 4 rows.  A product has two or four times as many workgroups of fewer waves, and reads no row of x twice.
+//
+// GATED: w is [gate | up], N rows each; half of a workgroup's columns are columns of gate, the other half the same of up, and
+// y[n, N] = act(x . gate^T) * (x . up^T), each sum and then the pair as the product and the activation kernel would make them.
+template <int TN, bool VEC, int SHARE, bool GATED>
+__global__ void __launch_bounds__(PL_F32_PARTS / SHARE * PL_WAVE)
 gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int n, int N, int K,
-                    int ldx, int ldy, long sx, long sw, long sy, int part_len) {
+                    int ldx, int ldy, long sx, long sw, long sy, int part_len, int act) {
+    static_assert(SHARE == 1 || TN == 1, "parts share the instruction of one tile of rows");
+    static_assert(!GATED || SHARE < 4, "four columns of gate and of up make a store");
     constexpr int ROUND = TN > 2 ? 2 : 4;                               // steps of 16 k asked for together
-    __shared__ __attribute__((aligned(16))) float parts[PL_F32_PARTS][TN * 16][16];       // [part][row of x][column of w]
+    constexpr int COLS = 16 / SHARE, ROWS = TN * 16 / SHARE, OUT = GATED ? COLS / 2 : COLS;    // (OUT: columns of y)
+    __shared__ __attribute__((aligned(16))) float parts[PL_F32_PARTS][ROWS][COLS];       // [part][row of x][column of w]
     x += blockIdx.z * sx;
     w += blockIdx.z * sw;
     y += blockIdx.z * sy;
     const int lane = threadIdx.x % PL_WAVE, wave = threadIdx.x / PL_WAVE;
     const int r = lane % 16, c = lane / 16;
-    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * TN * 16;
-    const float* wr = w + static_cast<size_t>(min(n0 + r, N - 1)) * K;
+    const int n0 = blockIdx.x * OUT, m0 = blockIdx.y * ROWS;
+    const float* wr = w + (static_cast<size_t>(min(n0 + r % OUT, N - 1)) + (GATED && r % COLS >= OUT ? N : 0)) * K;
     const float* xr[TN];
 #pragma unroll
-    for (int j = 0; j < TN; ++j) xr[j] = x + static_cast<size_t>(min(m0 + j * 16 + r, n - 1)) * ldx;
+    for (int j = 0; j < TN; ++j) xr[j] = x + static_cast<size_t>(min(m0 + (j * 16 + r) % ROWS, n - 1)) * ldx;
 
-    const int first = wave * part_len, last = min(K, first + part_len);
+    // (the wave's first part; a lane's own begins `mine` behind it and ends at `end`)
+    const int first = wave * SHARE * part_len, last = min(K, first + part_len);
+    const int mine = r / COLS * part_len, end = SHARE == 1 ? K : min(K, first + mine + part_len);
     if (first < last) {
         f32x4 acc[1][TN];
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[0][j] = zero;
         f32x4 a[ROUND][1], b[ROUND][TN];
-        auto ask = [&](int k) {
+        auto ask = [&](int u, int k) {
+            a[u][0] = f32_load4<VEC>(wr, k + mine + c * 4, K);
 #pragma unroll
-            for (int u = 0; u < ROUND; ++u) {
-                a[u][0] = f32_load4<VEC>(wr, k + u * 16 + c * 4, K);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) b[u][j] = f32_load4<VEC>(xr[j], k + u * 16 + c * 4, K);
-            }
+            for (int j = 0; j < TN; ++j) b[u][j] = f32_load4<VEC>(xr[j], k + mine + c * 4, K);
         };
-        ask(first);
+        auto clear = [&](int u, int k) {
+            a[u][0] = f32_end(a[u][0], k + mine + c * 4, end);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[u][j] = f32_end(b[u][j], k + mine + c * 4, end);
+        };
+#pragma unroll
+        for (int u = 0; u < ROUND; ++u) ask(u, first + u * 16);
         int k = first;
         for (; k + ROUND * 16 < last; k += ROUND * 16) {
-            // (a step's registers are filled again as soon as it is multiplied; every load is unconditional, since a load in
-            // a branch would make the compiler wait for all that are on their way, and nothing past the part is asked for)
+            // (two steps' registers, a row's 128 bytes, are filled again as soon as they are multiplied; every load is
+            // unconditional, since a load in a branch would make the compiler wait for all that are on their way, and nothing past
+            // the part is asked for)
 #pragma unroll
-            for (int u = 0; u < ROUND; ++u) {
-                f32_multiply<1, TN>(a[u], b[u], acc);
-                const int next = k + (ROUND + u) * 16 + c * 4;
-                a[u][0] = f32_load4<VEC>(wr, next, K);
+            for (int u = 0; u < ROUND; u += 2) {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) b[u][j] = f32_load4<VEC>(xr[j], next, K);
+                for (int e = u; e < u + 2; ++e) {
+                    if (SHARE > 1) clear(e, k + e * 16);
+                    f32_multiply<1, TN>(a[e], b[e], acc);
+                }
+#pragma unroll
+                for (int e = u; e < u + 2; ++e) ask(e, k + (ROUND + e) * 16);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
 #pragma unroll
         for (int u = 0; u < ROUND; ++u) {
             if (k + u * 16 < last) {
-                a[u][0] = f32_end(a[u][0], k + u * 16 + c * 4, K);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) b[u][j] = f32_end(b[u][j], k + u * 16 + c * 4, K);
+                clear(u, k + u * 16);
                 f32_multiply<1, TN>(a[u], b[u], acc);
             }
         }
-        // (a lane holds four columns of one row of x)
+        // (a lane holds four columns of one row of x; the other blocks mix two parts)
+        if (c * 4 / COLS == r / COLS) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4*>(&parts[wave][j * 16 + r][c * 4]) = acc[0][j];
+            for (int j = 0; j < TN; ++j)
+                *reinterpret_cast<f32x4*>(&parts[wave * SHARE + r / COLS][(j * 16 + r) % ROWS][c * 4 % COLS]) = acc[0][j];
+        }
     }
     __syncthreads();
     const int used = (K + part_len - 1) / part_len;
-    const int row = threadIdx.x / 4, col = n0 + threadIdx.x % 4 * 4;       // four columns of one row
-    if (row < TN * 16 && m0 + row < n) {
-        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < used; ++p) sum += *reinterpret_cast<const f32x4*>(&parts[p][row][threadIdx.x % 4 * 4]);
+    const int row = threadIdx.x * 4 / OUT, at = threadIdx.x * 4 % OUT, col = n0 + at;         // four columns of one row
+    if (row < ROWS && m0 + row < n) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f}, up = {0.f, 0.f, 0.f, 0.f};
+        for (int p = 0; p < used; ++p) {
+            sum += *reinterpret_cast<const f32x4*>(&parts[p][row][at]);
+            if (GATED) up += *reinterpret_cast<const f32x4*>(&parts[p][row][OUT % COLS + at]);
+        }
+        if (GATED)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum[q] = pl_activate<true>(sum[q], act) * up[q];
         const bool whole = N % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
         f32_store4(y + static_cast<size_t>(m0 + row) * ldy + col, sum, col, N, whole);
     }
@@ -271,11 +297,11 @@ struct F32Product {
     long sx, sw, sy;
 };
 
-template <int TN, bool VEC>
-void launch_few(const F32Product& g, hipStream_t stream) {
-    const dim3 grid(pl_ceil_div(g.N, 16), pl_ceil_div(g.n, TN * 16), g.batch);
-    gemm_f32_few_kernel<TN, VEC><<<grid, PL_F32_PARTS * PL_WAVE, 0, stream>>>(g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw,
-                                                                              g.sy, f32_part_len(g.K));
+template <int TN, bool VEC, int SHARE = 1, bool GATED = false>
+void launch_few(const F32Product& g, hipStream_t stream, int act = 0) {
+    const dim3 grid(pl_ceil_div(g.N, 16 / SHARE / (GATED ? 2 : 1)), pl_ceil_div(g.n, TN * 16 / SHARE), g.batch);
+    gemm_f32_few_kernel<TN, VEC, SHARE, GATED><<<grid, PL_F32_PARTS / SHARE * PL_WAVE, 0, stream>>>(
+        g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw, g.sy, f32_part_len(g.K), act);
 }
 
 template <int TILE>
@@ -294,6 +320,10 @@ void launch_tiled(const F32Product& g, hipStream_t stream) {
 // whose workgroups hold all rows and read every weight once; against many columns its 16 columns a workgroup reads the rows
 // too often from nine rows on, and from 17 rows on earlier (us, few / tiles of 32: 16 rows, 6,144 x 1,024 12.2 / 12.8, 151,936 x
 // 1,024 172 / 141; 32 rows, 4,096 x 1,024 10.2 / 13.1, 6,144 x 1,024 17.0 / 12.9; 64 rows, 4,096 x 1,024 14.1 / 13.2).
+// Parts share the instruction where 16 columns a workgroup leave half of the chip idle (us, sixteen parts a workgroup / shared:
+// 1,024 x 3,072, 1 row 10.0 / 6.1, 4 rows 11.0 / 6.3, 8 rows 12.4 / 9.1; 1,024 x 2,048, 8 rows 8.9 / 6.9).  Wider ones read x
+// too often then (8 rows, 4,096 x 1,024 6.6 / 7.4, 151,936 x 1,024 125 / 164), unless there is one row (4,096 x 1,024 6.3 / 5.7,
+// 6,144 x 1,024 9.0 / 7.3, 151,936 x 1,024 113 / 101).
 // Tiles of 64 rows by 64 columns or of 32 by 32: the shorter estimate for the compute unit with most of them, a small tile
 // costing 1.15 times as much for what it does (700 rows, tiles of 64 / 32: 1,024 x 2,048 43.7 / 34.7, 4,096 x 1,024 62.3 /
 // 59.5; 2,048 rows, 1,024 x 2,048 76.7 / 87.6, 4,096 x 1,024 152 / 178).
@@ -313,7 +343,10 @@ int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, i
                "gemm: %d x %d results are more than one launch covers", n, N);
     if (few || !tiles) {
         if (vec) {
-            if (n <= 16) launch_few<1, true>(g, stream);
+            const bool idle = static_cast<long>(pl_ceil_div(N, 16)) * batch * 2 <= units;
+            if (n == 1 || (n <= 4 && idle)) launch_few<1, true, 4>(g, stream);
+            else if (n <= 8 && idle) launch_few<1, true, 2>(g, stream);
+            else if (n <= 16) launch_few<1, true>(g, stream);
             else if (n <= 32) launch_few<2, true>(g, stream);
             else launch_few<4, true>(g, stream);
         } else if (n <= 16) {
@@ -327,5 +360,24 @@ int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, i
         launch_tiled<32>(g, stream);
     }
     PL_CHECK_LAUNCH("gemm_f32");
+    return 0;
+}
+
+// y[n, I] = act(x . gate^T) * (x . up^T), w [gate | up] of I rows each: one launch instead of two for up to 16 rows whose product
+// is the kernel for few rows; the same bits as pl_gemm_f32 and then pl_swiglu.
+static bool f32_gated_applies(const void* x, const void* w, int n, int I, int K) {
+    return n >= 1 && n <= 16 && (n <= 8 || I < 16384) && I >= 1 && I < (1 << 30) && K >= 4 && K % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(w) % 16 == 0;
+}
+
+extern "C" int pl_gemm_f32_gated_applies(const void* x, const void* w, int n, int I, int K) { return f32_gated_applies(x, w, n, I, K) ? 1 : 0; }
+
+extern "C" int pl_gemm_f32_gated(const float* x, const float* w, float* y, int n, int I, int K, int act, hipStream_t stream) {
+    PL_REQUIRE(f32_gated_applies(x, w, n, I, K), "gated product: %d rows, %d x %d", n, I, K);
+    PL_REQUIRE(act >= PL_ACT_SILU && act <= PL_ACT_RELU2, "gated product: activation code %d", act);
+    const F32Product g{x, w, y, n, I, K, K, I, 1, 0, 0, 0};
+    if (n == 1) launch_few<1, true, 2, true>(g, stream, act);
+    else launch_few<1, true, 1, true>(g, stream, act);
+    PL_CHECK_LAUNCH("gemm_f32 (gated)");
     return 0;
 }

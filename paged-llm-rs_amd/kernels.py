@@ -34,6 +34,8 @@ def _signatures(lib) -> None:
         "pl_add_bias": [p, p, i, i, i, i, p],
         "pl_qk_norm_rope_kv_write": [p, p, p, i, f, p, p, i, p, p, p, i, i, p, p, i, i, i, i, i, i, i, p],
         "pl_swiglu": [p, p, i, i, i, i, p],
+        "pl_gemm_f32_gated": [p, p, p, i, i, i, i, p],
+        "pl_gemm_f32_gated_applies": [p, p, i, i, i],
         "pl_gemm_plain": [p, p, p, i, i, i, i, i, i, i, p],
         "pl_paged_attention_plain": [p, i, p, p, p, p, i, i, p, p, i, i, i, i, f, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_f32_applies": [p, i, p, p, p, i],
@@ -307,6 +309,22 @@ def gemm_plain(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None
         raise TensorError(f"matrix product output {out_dtype} from input {x.dtype}")
     _check(library().pl_gemm_plain(x.data_ptr(), w.data_ptr(), out.data_ptr(), n, N, K, K, N,
                                    _code(x, "matrix product input"), 1 if out_dtype == torch.float32 else 0, _stream()))
+    return out
+
+
+def gemm_plain_gated(x: torch.Tensor, w: torch.Tensor, activation: str = "silu") -> torch.Tensor:
+    """act(x . gate^T) * (x . up^T) of 32-bit operands, ``w`` [gate | up]: one kernel for few rows, otherwise the product and
+    the activation; the same bits."""
+    n, K = x.shape
+    if w.shape[0] % 2:
+        raise TensorError(f"fused gate/up projection has odd width {w.shape[0]}")
+    inter = w.shape[0] // 2
+    _need(x, "matrix product input", dtype=torch.float32)
+    _need(w, "weight", (2 * inter, K), torch.float32)
+    if not library().pl_gemm_f32_gated_applies(x.data_ptr(), w.data_ptr(), n, inter, K):
+        return swiglu(gemm_plain(x, w), activation=activation)
+    out = torch.empty((n, inter), dtype=torch.float32, device=x.device)
+    _check(library().pl_gemm_f32_gated(x.data_ptr(), w.data_ptr(), out.data_ptr(), n, inter, K, activation_code(activation), _stream()))
     return out
 
 

@@ -83,8 +83,9 @@ class Linear:
         out_dtype = out_dtype or x.dtype
         if x.dtype == torch.float32:
             # the true 32-bit path: 32-bit operands, products and sums
-            y = kernels.gemm_plain(x, self.weight, out_dtype=torch.float32)
-            return kernels.swiglu(y, activation=activation) if swiglu else y
+            if swiglu:
+                return kernels.gemm_plain_gated(x, self.weight, activation)
+            return kernels.gemm_plain(x, self.weight, out_dtype=torch.float32)
         if kernels.skinny_applies(x, self.weight, self.strips is not None):
             if add_into is not None and not swiglu:
                 if hand is not None and not kernels.hands_norm_forward(x.shape[0], self.out_features, self.in_features):

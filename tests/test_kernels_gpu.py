@@ -243,7 +243,7 @@ def test_the_32_bit_product_of_few_and_of_many_rows(N, K):
     w = torch.randn(N, K, device=DEV)
     full = kernels.gemm_plain(x, w)
     assert rel(full, x.double() @ w.double().T) < 4 * math.sqrt(K / 16 + 16) * 2.0 ** -24
-    for n in (1, 8, 9, 16, 17, 32, 33, 64, 65, 130):
+    for n in (1, 2, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 130):
         assert torch.equal(kernels.gemm_plain(x[-n:].contiguous(), w), full[-n:]), f"{n} rows"
     x[1, K // 2], w[N // 2, 0], x[3] = math.inf, math.nan, 1e-41      # (and numbers too small to have an exponent)
     for n in (4, 200):
@@ -253,6 +253,22 @@ def test_the_32_bit_product_of_few_and_of_many_rows(N, K):
         if K % 64 == 0 and N > 1:
             small = torch.arange(N, device=DEV) != N // 2
             assert rel(y[3][small], x[3].double() @ w[small].double().T) < 1e-3
+
+
+@pytest.mark.parametrize("I,K", [(1, 4), (7, 64), (30, 1028), (100, 100), (2052, 192), (16400, 64), (61, 1026)])
+@pytest.mark.parametrize("activation", ["silu", "gelu"])
+def test_the_32_bit_gated_product(I, K, activation):
+    """One kernel for few rows (one row, up to 8, up to 16) and the product with the activation behind it are the same bits, also
+    where a width or an address is not made of groups of four."""
+    from paged_llm_rs_amd import kernels
+
+    w = torch.randn(2 * I, K, device=DEV)
+    x = torch.randn(17, K, device=DEV)
+    want = kernels.swiglu(kernels.gemm_plain(x, w), activation=activation)
+    for n in (1, 2, 8, 9, 16, 17):
+        assert torch.equal(kernels.gemm_plain_gated(x[-n:].contiguous(), w, activation), want[-n:]), f"{n} rows"
+    beside = torch.randn(4 * K + 1, device=DEV)[1:].view(4, K)        # (not aligned)
+    assert torch.equal(kernels.gemm_plain_gated(beside, w, activation), kernels.swiglu(kernels.gemm_plain(beside, w), activation=activation))
 
 
 @pytest.mark.parametrize("n", [1, 2, 8, 16, 17, 33, 64])
