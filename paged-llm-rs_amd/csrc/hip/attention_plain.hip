@@ -7,8 +7,8 @@
 // because the cache write precedes attention inside a layer.  Keys are walked
 // in ascending order in tiles of 64 with a running maximum and sum, so the
 // result for a position does not depend on how the request was cut into steps
-// or on what else is in the batch.  It is the attention of the true 32-bit
-// path and the fallback for shapes the matrix-core kernels refuse.
+// or on what else is in the batch.  It is the fallback for shapes that the
+// matrix-core kernels refuse (attention_f32.hip on the true 32-bit path, the bfloat16 ones elsewhere).
 //
 // Two optional extras, a number a query head each: `slopes` (slope_h * (i - j) is taken off the score of key
 // j for the query at position i) and `sinks` (exp(sink_h) joins the softmax's denominator once: a score

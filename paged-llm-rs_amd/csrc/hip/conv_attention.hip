@@ -100,82 +100,120 @@ __global__ __launch_bounds__(64) void conv_qk_prepare_heads_kernel(ConvQkArgs a)
 }
 
 // Many tokens (prompt portions): one workgroup a token; its waves take the token's heads (query, key and value heads alike) in turn, and
-// the angles' cosines and sines are worked out once for the token.
-template <typename T>
+// the angles' cosines and sines are worked out once for the token.  A wave needs nobody else for a head: a lane holds NI of its values,
+// asks for all taps of them together (TAPS known) and finds the ones to turn them with in the wave's own LDS.  Bound by the chain of a
+// head's work (3,000 tokens, four taps, 16 query heads over 8 of 128: 36 us; 150 MB through the caches, 61 MB of them from memory).  With
+// the loads one by one and two barriers a round of four heads it took 75 us.
+template <typename T, int NI, int TAPS>
 __global__ __launch_bounds__(256) void conv_qk_prepare_kernel(ConvQkArgs a) {
-    __shared__ float heads[4][256];
+    __shared__ float heads[4][64 * NI];
     __shared__ float cs[128], sn[128];
-    const int t = blockIdx.x, wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int t = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const int pos = a.positions[t];
     if (pos < 0) return;
     const int s = a.seq_of[t];
     const int slot = a.state_slots[s];
     if (slot < 0) return;
     const int H = a.H, G = a.G, D = a.D, V = a.V, Dp = a.Dp;
-    const int channels = H * D + G * D + G * V;
+    const int channels = H * D + G * D + G * V, taps = TAPS > 0 ? TAPS : a.taps;
     const float* hist = a.state + static_cast<size_t>(slot) * a.state_stride + a.hist_off;
     const int r = t - a.q_start[s];
     const int half = a.rot / 2;
     for (int i = threadIdx.x; i < half; i += 256) sincosf(static_cast<float>(pos) * a.freq[i], &sn[i], &cs[i]);
-    __syncthreads();
     int page_row = -1;
     {
         const int page = a.block_table[static_cast<size_t>(s) * a.max_blocks + pos / a.block_size];
         if (page >= 0) page_row = page * a.block_size + pos % a.block_size;
     }
+    const auto tap_row = [&](int jt) {
+        const int back = taps - 1 - jt, src = r - back;
+        return src >= 0 ? a.rows + static_cast<size_t>(t - back) * a.stride + a.off : hist + static_cast<size_t>(taps - 1 + src) * channels;
+    };
     float* head = heads[wave];
-    for (int base = 0; base < H + 2 * G; base += 4) {
-        // which head this wave prepares now: a query head, a key head or a value head (the last round may leave
-        // waves without one; they still meet the others at the barriers)
-        const int which = base + wave;
-        const bool busy = which < H + 2 * G;
+    __syncthreads();
+    for (int which = wave; which < H + 2 * G; which += 4) {
         const int kind = which < H ? 0 : (which < H + G ? 1 : 2);
         const int index = kind == 0 ? which : (kind == 1 ? which - H : which - H - G);
         const int width = kind == 2 ? V : D;
         const int c0 = kind == 0 ? index * D : (kind == 1 ? H * D + index * D : H * D + G * D + index * V);
-        float ss = 0.f;
-        for (int e = lane; busy && e < width; e += 64) {
-            const int c = c0 + e;
-            float acc = 0.f;
-            for (int jt = 0; jt < a.taps; ++jt) {
-                const int back = a.taps - 1 - jt;
-                const int src = r - back;
-                const float u = src >= 0 ? a.rows[static_cast<size_t>(t - back) * a.stride + a.off + c]
-                                         : hist[static_cast<size_t>(a.taps - 1 + src) * channels + c];
-                acc += a.conv_w[jt * channels + c] * u;
-            }
-            head[e] = acc;
-            ss += acc * acc;
+        float x[NI];
+        int at[NI];                     // (past the head's end: its last value again, which is cleared)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            x[i] = 0.f;
+            at[i] = c0 + min(lane + 64 * i, width - 1);
         }
-        if (busy && kind != 2) {
+        if constexpr (TAPS > 0) {
+            float u[TAPS][NI], w[TAPS][NI];
+#pragma unroll
+            for (int jt = 0; jt < TAPS; ++jt) {
+                const float* row = tap_row(jt);
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    u[jt][i] = row[at[i]];
+                    w[jt][i] = a.conv_w[jt * channels + at[i]];
+                }
+            }
+#pragma unroll
+            for (int jt = 0; jt < TAPS; ++jt)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) x[i] += w[jt][i] * u[jt][i];
+        } else {
+            for (int jt = 0; jt < taps; ++jt) {
+                const float* row = tap_row(jt);
+#pragma unroll
+                for (int i = 0; i < NI; ++i) x[i] += a.conv_w[jt * channels + at[i]] * row[at[i]];
+            }
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if (lane + 64 * i >= width) x[i] = 0.f;
+            ss += x[i] * x[i];
+        }
+        if (kind != 2) {
             ss = wave_sum(ss);
             const float inv = 1.f / sqrtf(ss / static_cast<float>(D) + a.eps);
             const float* gain = kind == 0 ? a.q_gain : a.k_gain;
-            for (int e = lane; e < width; e += 64) head[e] = head[e] * inv * gain[e];
-        }
-        __syncthreads();
-        T* dst = nullptr;
-        if (!busy)
-            dst = nullptr;
-        else if (kind == 0)
-            dst = static_cast<T*>(a.q_out) + (static_cast<size_t>(t) * H + index) * Dp;
-        else if (page_row >= 0)
-            dst = static_cast<T*>(kind == 1 ? a.k_pool : a.v_pool) + (static_cast<size_t>(page_row) * G + index) * Dp;
-        if (dst != nullptr) {
-            for (int e = lane; e < Dp; e += 64) {
-                float x = 0.f;
-                if (e < width) {
-                    x = head[e];
-                    if (kind != 2 && e < a.rot) {
-                        const int i = e < half ? e : e - half;
-                        x = e < half ? head[e] * cs[i] - head[e + half] * sn[i] : head[e] * cs[i] + head[e - half] * sn[i];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) x[i] = x[i] * inv * gain[min(lane + 64 * i, width - 1)];
+            if (a.rot > 0) {
+#pragma unroll
+                for (int i = 0; i < NI; ++i) head[lane + 64 * i] = x[i];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const int e = lane + 64 * i;
+                    if (e < a.rot) {
+                        const int k = e < half ? e : e - half;
+                        x[i] = e < half ? x[i] * cs[k] - head[e + half] * sn[k] : x[i] * cs[k] + head[e - half] * sn[k];
                     }
                 }
-                dst[e] = from_float<T>(x);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
         }
-        __syncthreads();
+        if (kind != 0 && page_row < 0) continue;
+        T* dst = kind == 0 ? static_cast<T*>(a.q_out) + (static_cast<size_t>(t) * H + index) * Dp
+                           : static_cast<T*>(kind == 1 ? a.k_pool : a.v_pool) + (static_cast<size_t>(page_row) * G + index) * Dp;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+            if (lane + 64 * i < Dp) dst[lane + 64 * i] = from_float<T>(x[i]);
     }
+}
+
+template <typename T, int NI>
+static void launch_conv_qk(const ConvQkArgs& a, int n, hipStream_t stream) {
+    if (a.taps == 4) conv_qk_prepare_kernel<T, NI, 4><<<n, 256, 0, stream>>>(a);
+    else conv_qk_prepare_kernel<T, NI, 0><<<n, 256, 0, stream>>>(a);
+}
+
+template <typename T>
+static void launch_conv_qk(const ConvQkArgs& a, int n, hipStream_t stream) {
+    if (a.Dp <= 64) launch_conv_qk<T, 1>(a, n, stream);
+    else if (a.Dp <= 128) launch_conv_qk<T, 2>(a, n, stream);
+    else launch_conv_qk<T, 4>(a, n, stream);
 }
 
 extern "C" int pl_conv_qk_prepare(const float* rows, int stride, int off, const float* conv_w, int taps,
@@ -200,10 +238,10 @@ extern "C" int pl_conv_qk_prepare(const float* rows, int stride, int off, const 
     const dim3 grid(n, H + 2 * G);
     if (dtype == PL_DTYPE_F32) {
         if (few) conv_qk_prepare_heads_kernel<float><<<grid, 64, 0, stream>>>(a);
-        else conv_qk_prepare_kernel<float><<<n, 256, 0, stream>>>(a);
+        else launch_conv_qk<float>(a, n, stream);
     } else if (dtype == PL_DTYPE_BF16) {
         if (few) conv_qk_prepare_heads_kernel<bf16_t><<<grid, 64, 0, stream>>>(a);
-        else conv_qk_prepare_kernel<bf16_t><<<n, 256, 0, stream>>>(a);
+        else launch_conv_qk<bf16_t>(a, n, stream);
     }
     else
         PL_REQUIRE(false, "conv_qk_prepare: dtype code %d", dtype);

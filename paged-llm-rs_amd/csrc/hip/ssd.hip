@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void retention_turn_kernel(float* __restrict__
 // state for one request, as above.  Bound by the chain of a token: state and rows on their way together, one round through
 // LDS for the read-out (delta: two more, for the unit vectors and for what the memory says to the key).  A wave with a
 // column of the state a lane (the scan kernel) asks for D rows one after the other and adds them up alone: 20 to 25 us for one token of
-// two requests (8 heads of 128 by 128, 4 of 128 by 256), and some 7 here.
+// two requests (8 heads of 128 by 128, 4 of 128 by 256), and 5.5 here.
 template <int R, int KIND>
 __global__ __launch_bounds__(256) void state_step_kernel(ScanArgs a) {
     __shared__ ssd_f32x4 part[4][16], memory[4][16];

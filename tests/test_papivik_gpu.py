@@ -435,3 +435,59 @@ def test_the_recurrences_kernels_in_portions(kind, H, D, V):
     run([[(i, t) for i, t in enumerate(T)]], [5, 0, 3, 1, 7, 2])
     run([[(0, 15), (1, 16), (2, 1), (4, 63)], [(0, 64), (2, 1), (1, 48), (5, 2)], [(0, 1), (3, 1), (4, 2), (2, 1)], [(0, 114), (5, 31)]],
         [0, 1, 2, 3, 4, 5])
+
+
+@pytest.mark.parametrize("H,G,D,V,Dp,taps,rot", [(3, 1, 128, 128, 128, 4, 128), (2, 2, 100, 130, 132, 4, 62), (4, 2, 40, 64, 64, 4, 0),
+                                                 (2, 1, 200, 256, 256, 3, 200), (5, 1, 64, 20, 64, 1, 2), (2, 1, 130, 7, 130, 6, 130)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_preparation_of_convolved_heads_in_large_and_in_small_steps(H, G, D, V, Dp, taps, rot, dtype):
+    """A step of more than 512 rows (a workgroup a token) and its requests one at a time (a wave a head): the same values into the query
+    buffer and the pages, which are otherwise left alone; a request whose page is not there, rows of padding.  The kernels may contract
+    differently: some 16 roundings of 2^-24 of a value before its rotation (the largest is below 32), and one unit of bfloat16."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator().manual_seed(D + taps)
+    channels, off, counts, before = H * D + G * D + G * V, 4, [400, 70, 45, 1], [0, 2, 130, 5]
+    n = sum(counts) + 2
+    rows = torch.randn((n, off + channels), generator=g).cuda()
+    weight = torch.randn((taps, channels), generator=g).cuda()
+    history = torch.randn((5, taps * channels), generator=g).cuda()[:, :(taps - 1) * channels]
+    gains = [torch.randn((D,), generator=g).cuda() for _ in range(2)]
+    freq = torch.rand((rot // 2,), generator=g).cuda() if rot else None
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32).cuda()
+    bs = 16
+    table = torch.randperm(4 * 26, generator=g).reshape(4, 26).int()
+    table[1, 2] = -1
+
+    def run(which):
+        spans = [range(sum(counts[:i]), sum(counts[:i + 1])) for i in which]
+        mine = torch.cat([rows[s.start:s.stop] for s in spans] + [rows[-2:]]).contiguous()
+        starts = np.concatenate([[0], np.cumsum([counts[i] for i in which])]).tolist()
+        batch = SimpleNamespace(
+            num_tokens=len(mine), num_seqs=len(which) + 1, q_start=i32(starts), q_len=i32([counts[i] for i in which] + [2]),
+            state_slots=i32([[3, 0, 4, 1][i] for i in which] + [-1]), max_q_len=max(counts),
+            positions=i32([before[i] + k for i in which for k in range(counts[i])] + [-1, -1]),
+            seq_of=i32([s for s, i in enumerate(which) for _ in range(counts[i])] + [len(which)] * 2))
+        pools = [torch.full((4 * 26 * bs, G * Dp), 7.0, dtype=dtype, device="cuda") for _ in range(2)]
+        kv = SimpleNamespace(k_pool=pools[0], v_pool=pools[1], block_size=bs,
+                             block_table=torch.cat([table[which], torch.full((1, 26), -1, dtype=torch.int32)]).cuda())
+        out = torch.full((len(mine), H * Dp), 7.0, dtype=dtype, device="cuda")
+        kernels.conv_qk_prepare(mine, off, weight, history, *gains, 1e-6, freq, rot, batch, kv, H, G, D, V, Dp, out)
+        return out, pools
+
+    def close(x, y):
+        assert float(y.abs().max()) < 32
+        return torch.allclose(x.float(), y.float(), rtol=2.0 ** -7 if dtype == torch.bfloat16 else 0, atol=16 * 32 * 2.0 ** -24)
+
+    whole, pools = run([0, 1, 2, 3])
+    assert len(whole) >= 512 and bool((whole[-2:] == 7.0).all())
+    merged = [torch.full_like(p, 7.0) for p in pools]
+    for i in range(4):
+        out, parts = run([i])
+        assert close(out[:-2], whole[sum(counts[:i]):sum(counts[:i + 1])]), i
+        for m, p in zip(merged, parts):
+            m.copy_(torch.where(p != 7.0, p, m))
+    for m, p in zip(merged, pools):
+        assert torch.equal(m == 7.0, p == 7.0) and close(m, p)
