@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64) void conv_qk_prepare_heads_kernel(ConvQkArgs a)
 // Many tokens (prompt portions): one workgroup a token; its waves take the token's heads (query, key and value heads alike) in turn, and
 // the angles' cosines and sines are worked out once for the token.  A wave needs nobody else for a head: a lane holds NI of its values,
 // asks for all taps of them together (TAPS known) and finds the ones to turn them with in the wave's own LDS.  Bound by the chain of a
-// head's work (3,000 tokens, four taps, 16 query heads over 8 of 128: 36 us; 150 MB through the caches, 61 MB of them from memory).  With
+// head's work (3,000 tokens, four taps, 16 query heads over 8 of 128: 36 us for 49 MB of rows, read four times over through the caches, and 25 MB written).  With
 // the loads one by one and two barriers a round of four heads it took 75 us.
 template <typename T, int NI, int TAPS>
 __global__ __launch_bounds__(256) void conv_qk_prepare_kernel(ConvQkArgs a) {

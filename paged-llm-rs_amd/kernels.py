@@ -401,7 +401,7 @@ def f32_splits(rows: int, live_seqs: int, nq: int, nkv: int, d: int, max_ctx: in
     """Whether the 32-bit kernel leaves the segments of every row in memory for a second kernel to fold.  It costs that
     kernel (some 5 us) and the segments' trip, and it pays where the tiles alone leave compute units without work: a few
     tokens, whose keys a few workgroups would take in at what a compute unit gets from memory (8 tokens at contexts up to 512,
-    16 heads over 8 of 128: 25 us whole, 14.7 split), or few tiles before more than 1,024 keys."""
+    16 heads over 8 of 128: 24 us whole, 18.5 split with its second kernel), or few tiles before more than 1,024 keys."""
     group = nq // nkv
     tokens, head_tiles = (16 // group, 1) if group <= 16 else (1, -(-group // 16))
     tiles = min(rows, rows // tokens + live_seqs) * nkv * head_tiles
