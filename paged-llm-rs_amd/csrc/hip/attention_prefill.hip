@@ -178,9 +178,6 @@ struct ap_more_t {
 template <>
 struct ap_more_t<false> {};
 
-// With room for arrivals the shares of a token tile, up to so many, meet in this kernel.
-#define AP_MEET_MAX 4
-
 template <int DT, int NW, int KS, int FEED, bool GR, bool MORE>
 __global__ void __launch_bounds__(64 * NW * KS, DT <= 4 ? AP_OCC : 1)
 paged_attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
@@ -189,7 +186,7 @@ paged_attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_
                                int num_seqs, const int* __restrict__ block_table, int max_blocks,
                                int block_size, const bf16_t* __restrict__ k_pool,
                                const bf16_t* __restrict__ v_pool, int nq, int nkv, int d, float scale_log2e,
-                               int window, int total_work, int splits, int* __restrict__ arrivals, float* __restrict__ part_acc,
+                               int window, int total_work, int splits, float* __restrict__ part_acc,
                                float* __restrict__ part_ml, int compact, const float* __restrict__ sinks,
                                const float* __restrict__ slopes, ap_more_t<MORE> with) {
     constexpr int DP = 32 * DT;
@@ -453,10 +450,8 @@ paged_attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_
     };
     const int k_first = key_of(0);
     const int k_end = tile_first_no < tile_end_no ? key_of(tile_end_no - 1 - tile_first_no) + AP_BN : k_first;
-    // (with arrivals only the shares that hold tiles take part, and one that holds them all stores its output itself)
-    const int shares = !GR && arrivals != nullptr ? (key_tiles + tiles_a_split - 1) / tiles_a_split : splits;
     if (k_first >= k_end) {          // more splits than key tiles: nothing to add
-        if ((GR || arrivals == nullptr) && kt0 == 0 && q_ok) {
+        if (kt0 == 0 && q_ok) {
             float* ml = part_ml + ((static_cast<size_t>(row0 + wq) * nq + q_head) * splits + split) * 2;
             if (h == 0) {
                 ml[0] = -INFINITY;
@@ -866,97 +861,30 @@ paged_attention_prefill_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[dt][r] = o[dt][r] * w0 + hand[(dt * 16 + r) * PL_WAVE + lane] * w1;
     }
-    // o[dt][4*j + i] is element 32*dt + 8*j + 4*h + i of query r32
-    float m_log2 = m == -INFINITY ? -INFINITY : m * scale_log2e;           // in the exponent's own unit
-    if (shares > 1) {
-        const size_t at = (static_cast<size_t>(row0 + wq) * nq + q_head) * splits + split;
-        float* arow = part_acc + at * d;
-        if (GR || arrivals == nullptr) {
-            if (!q_ok) return;
-            if (h == 0) {
-                part_ml[at * 2] = m_log2;
-                part_ml[at * 2 + 1] = lsum;
-            }
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e0 = 32 * dt + 8 * j + 4 * h;
-                    if (e0 < d) *reinterpret_cast<f32x4*>(arow + e0) = f32x4{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
-                }
-            return;
-        }
-        // A wave meets the waves of the other shares that hold its queries; the last of them puts the shares together, in
-        // their order whichever it is.
-        if (!wave_active) return;
-        if (q_ok) {
-            if (h == 0) {
-                pl_share(part_ml + at * 2, m_log2);
-                pl_share(part_ml + at * 2 + 1, lsum);
-            }
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int e0 = 32 * dt + 8 * j + 4 * h;
-                    if (e0 < d) pl_share4(arow + e0, o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]);
-                }
-        }
-        pl_shares_written();
-        int last = 0;
-        // (the wave's first query names the counter)
-        const size_t first_query = static_cast<size_t>(row0 + q0 + wave * 32) * nq + head;
-        if (lane == 0) last = pl_arrive(arrivals + first_query, shares) ? 1 : 0;
-        if (__builtin_amdgcn_readfirstlane(last) == 0) return;
-        if (!q_ok) return;
-        const size_t first_share = at - split;
-        float ms[AP_MEET_MAX], ls[AP_MEET_MAX], big = -INFINITY;
-#pragma unroll
-        for (int s = 0; s < AP_MEET_MAX; ++s) {
-            const float2 ml = pl_shared2(part_ml + (first_share + min(s, shares - 1)) * 2);
-            ms[s] = s < shares ? ml.x : -INFINITY;
-            ls[s] = ml.y;
-            big = fmaxf(big, ms[s]);
-        }
-        float sum = 0.f;
-#pragma unroll
-        for (int s = 0; s < AP_MEET_MAX; ++s) {
-            ms[s] = ms[s] == -INFINITY ? 0.f : exp2f(ms[s] - big);
-            if (s < shares) sum = fmaf(ls[s], ms[s], sum);
-        }
-        // (its own share comes back from memory like the others': its registers are free for what is on its way)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            float2 v[AP_MEET_MAX][8];
-#pragma unroll
-            for (int s = 0; s < AP_MEET_MAX; ++s)
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int e0 = 32 * dt + 8 * (r / 2) + 4 * h;
-                    v[s][r] = pl_shared2(part_acc + (first_share + min(s, shares - 1)) * d + (e0 < d ? e0 + r % 2 * 2 : 0));
-                }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
-#pragma unroll
-            for (int s = 0; s < AP_MEET_MAX; ++s)
-                if (s < shares) {
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) {
-                        o[dt][2 * r] = fmaf(v[s][r].x, ms[s], o[dt][2 * r]);
-                        o[dt][2 * r + 1] = fmaf(v[s][r].y, ms[s], o[dt][2 * r + 1]);
-                    }
-                }
-        }
-        lsum = sum;
-        m_log2 = big;
-    }
     if (!q_ok) return;
+    // o[dt][4*j + i] is element 32*dt + 8*j + 4*h + i of query r32
+    if (splits > 1) {
+        const size_t at = (static_cast<size_t>(row0 + wq) * nq + q_head) * splits + split;
+        if (h == 0) {
+            part_ml[at * 2] = m * scale_log2e;     // in the exponent's own unit; -inf stays
+            part_ml[at * 2 + 1] = lsum;
+        }
+        float* arow = part_acc + at * d;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int e0 = 32 * dt + 8 * j + 4 * h;
+                if (e0 < d) *reinterpret_cast<f32x4*>(arow + e0) = f32x4{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
+            }
+        return;
+    }
     float total = lsum, stays = 1.f;
     if (sinks != nullptr) {
         // a sink: one more term of the denominator, unscaled, with no value behind it
         const float sk = sinks[q_head] * 1.4426950408889634f;
-        const float top = fmaxf(m_log2, sk);
-        stays = m_log2 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_log2 - top);
+        const float top = fmaxf(m * scale_log2e, sk);
+        stays = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m * scale_log2e - top);
         total = lsum * stays + __builtin_amdgcn_exp2f(sk - top);
     }
     float inv = total > 0.f ? stays / total : 0.f;
@@ -1062,12 +990,9 @@ template <int DT, int NW, int KS, int FEED, bool GR = false>
 static int launch_prefill(const void* q, int q_stride, void* out, const int* q_start, const int* q_len,
                           const int* ctx_len, int short_limit, int num_seqs, int max_q_len, const int* block_table,
                           int max_blocks, int block_size, const void* k_pool, const void* v_pool, int nq, int nkv,
-                          int d, float scale, int window, int splits, int* arrivals, float* part_acc, float* part_ml,
+                          int d, float scale, int window, int splits, float* part_acc, float* part_ml,
                           int total_rows, int short_rows, const float* sinks, const float* slopes,
                           const PlAttentionMore& more, hipStream_t stream) {
-    // (More shares are left to the second kernel, whose every thread reads all of them for four values, and so are those of
-    // single tokens' groups of heads: 24 tokens at contexts up to 1,500 in three shares gained nothing, 1.431 ms a step and 1.425.)
-    if (GR || splits > AP_MEET_MAX) arrivals = nullptr;
     constexpr int DP = 32 * DT;
     constexpr int BM = 32 * NW;
     const size_t tile_bytes = FEED == 2 ? (2 * ap_direct_ahead(GR) + 3) * static_cast<size_t>(AP_BN) * DP * 2
@@ -1105,12 +1030,12 @@ static int launch_prefill(const void* q, int q_stride, void* out, const int* q_s
         static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out), q_start, q_len, ctx_len, short_limit, tiles,   \
         num_seqs, block_table, max_blocks, block_size, static_cast<const bf16_t*>(k_pool),                                 \
         static_cast<const bf16_t*>(v_pool), nq, nkv, d, scale * 1.4426950408889634f, window, static_cast<int>(total),      \
-        splits, arrivals, part_acc, part_ml, compact, sinks, slopes, WITH)
+        splits, part_acc, part_ml, compact, sinks, slopes, WITH)
     if (pl_has_more(more)) AP_KERNEL(true, ap_more_t<true>{more});
     else AP_KERNEL(false, ap_more_t<false>{});
 #undef AP_KERNEL
     PL_CHECK_LAUNCH("paged_attention_prefill");
-    if (splits > 1 && arrivals == nullptr) {
+    if (splits > 1) {
         const int rows = 256 / (d / 4);
 #define AP_MERGE(SP)                                                                                               \
     paged_attention_prefill_merge_kernel<SP><<<dim3(pl_ceil_div(total_rows, rows), nq), 256, 0, stream>>>(         \
@@ -1130,12 +1055,12 @@ template <int D>
 static int ap_dispatch(bool small, bool uniform_pages, const void* q, int q_stride, void* out, const int* q_start,
                        const int* q_len, const int* ctx_len, int short_limit, int num_seqs, int max_q_len,
                        const int* block_table, int max_blocks, int block_size, const void* k_pool, const void* v_pool,
-                       int nq, int nkv, int d, float scale, int window, int splits, int* arrivals, float* part_acc, float* part_ml,
+                       int nq, int nkv, int d, float scale, int window, int splits, float* part_acc, float* part_ml,
                        int total_rows, const float* sinks, const float* slopes, const PlAttentionMore& more, hipStream_t stream) {
 #define AP_LAUNCH(NW, KS, FEED)                                                                                    \
     launch_prefill<D, NW, KS, FEED>(q, q_stride, out, q_start, q_len, ctx_len, short_limit, num_seqs, max_q_len,    \
                                     block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale, window, \
-                                    splits, arrivals, part_acc, part_ml, total_rows, 0, sinks, slopes, more, stream)
+                                    splits, part_acc, part_ml, total_rows, 0, sinks, slopes, more, stream)
     constexpr bool can_fit = 64 % (4 * D) == 0;
     constexpr int BEST = (D == 2 || D == 4) && AP_KS == 2 && AP_SMALL_KS == 2 ? AP_FEED : 1;   // the feed with uniform pages
     if constexpr (D <= 4) {
@@ -1174,12 +1099,12 @@ static bool ap_more_fits(const PlAttentionMore& more, int nq, int window, float 
 extern "C" int pl_paged_attention_prefill_tile(int max_q_len, int d) {
     return (max_q_len <= 64 && d <= 128) ? 64 : 128;
 }
-// `arrivals`: as for the single-token kernel, n * nq of them.
+
 extern "C" int pl_paged_attention_prefill(const void* q, int q_stride, void* out, const int* q_start,
                                           const int* q_len, const int* ctx_len, int short_limit, int num_seqs,
                                           int max_q_len, const int* block_table, int max_blocks, int block_size,
                                           const void* k_pool, const void* v_pool, int nq, int nkv, int d,
-                                          float scale, int window, int splits, int* arrivals, float* part_acc, float* part_ml,
+                                          float scale, int window, int splits, float* part_acc, float* part_ml,
                                           int total_rows, const float* sinks, const float* slopes, float cap, int keep,
                                           const float* gate, int gate_stride, hipStream_t stream) {
     const PlAttentionMore more{cap, keep, gate, gate_stride};
@@ -1210,7 +1135,7 @@ extern "C" int pl_paged_attention_prefill(const void* q, int q_stride, void* out
     const bool pages_fit = (block_size & (block_size - 1)) == 0 && block_size * 4 * dt >= 64 && 64 % (4 * dt) == 0;
 #define AP_CALL(D)                                                                                                 \
     return ap_dispatch<D>(small, pages_fit, q, q_stride, out, q_start, q_len, ctx_len, short_limit, num_seqs, max_q_len, \
-                          block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale, window, splits, arrivals, \
+                          block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale, window, splits,   \
                           part_acc, part_ml, total_rows, sinks, slopes, more, stream)
     switch (dt) {
         case 1: AP_CALL(1);
@@ -1256,7 +1181,7 @@ static int ap_dispatch_grouped(bool uniform_pages, const void* q, int q_stride, 
 #define AP_GROUPED(FEED)                                                                                           \
     launch_prefill<D, 4, 1, FEED, true>(q, q_stride, out, q_start, q_len, ctx_len, short_limit, num_seqs, max_q_len, \
                                         block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale,    \
-                                        window, splits, nullptr, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream)
+                                        window, splits, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream)
     constexpr bool can_fit = 64 % (4 * D) == 0;
     if constexpr (can_fit) {
         if (uniform_pages) return AP_GROUPED(1);
@@ -1264,6 +1189,7 @@ static int ap_dispatch_grouped(bool uniform_pages, const void* q, int q_stride, 
     return AP_GROUPED(0);
 #undef AP_GROUPED
 }
+
 extern "C" int pl_paged_attention_grouped(const void* q, int q_stride, void* out, const int* q_start,
                                           const int* q_len, const int* ctx_len, int short_limit, int num_seqs,
                                           int max_q_len, const int* block_table, int max_blocks, int block_size,
@@ -1308,8 +1234,8 @@ extern "C" int pl_paged_attention_grouped(const void* q, int q_stride, void* out
     if (d == 64)
         return launch_prefill<2, 1, 2, 2, true>(q, q_stride, out, q_start, q_len, ctx_len, short_limit, num_seqs, max_q_len,
                                                 block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale,
-                                                window, splits, nullptr, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream);
+                                                window, splits, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream);
     return launch_prefill<4, 1, 2, 2, true>(q, q_stride, out, q_start, q_len, ctx_len, short_limit, num_seqs, max_q_len,
                                             block_table, max_blocks, block_size, k_pool, v_pool, nq, nkv, d, scale,
-                                            window, splits, nullptr, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream);
+                                            window, splits, part_acc, part_ml, total_rows, short_rows, sinks, slopes, more, stream);
 }

@@ -80,15 +80,6 @@ __device__ __forceinline__ float block_sum(float v, float* scratch /* >= 16 floa
 // kernel (256 workgroups 9.2 us, against 1.4 us for publishing and reading this way and 4.1 us for a kernel that merges).
 __device__ __forceinline__ void pl_share(float* to, float v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float pl_shared(const float* from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// Two and four values at aligned places.
-__device__ __forceinline__ float2 pl_shared2(const float* from) {
-    return __builtin_bit_cast(float2, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(from), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ void pl_share4(float* to, float a, float b, float c, float d) {
-    unsigned long long* at = reinterpret_cast<unsigned long long*>(to);
-    __hip_atomic_store(at, __builtin_bit_cast(unsigned long long, float2{a, b}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(at + 1, __builtin_bit_cast(unsigned long long, float2{c, d}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // The calling wave's shares are where every workgroup finds them.
 __device__ __forceinline__ void pl_shares_written() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // By one lane: whether all `of` shares are there now, this one the last of them.

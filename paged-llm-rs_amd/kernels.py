@@ -61,7 +61,7 @@ def _signatures(lib) -> None:
         "pl_gemm_finish": [p, p, ctypes.c_longlong, i, i, i, i, i, p],
         "pl_paged_attention_decode": [p, i, p, p, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, i, f, i, i,
                                       i, p, p, i, f, p, p, i, p, p, f, i, p, i, p, p],
-        "pl_paged_attention_prefill": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, p, i, p, p, f, i, p, i, p],
+        "pl_paged_attention_prefill": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped_applies": [i, i, i, i],
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
@@ -647,14 +647,13 @@ def paged_attention_prefill(q: torch.Tensor, q_row_stride: int, out: torch.Tenso
                             scale: float, window: int = 0, short_limit: int = 0, max_ctx: int | None = None,
                             splits: int | None = None, live_seqs: int | None = None,
                             sinks: torch.Tensor | None = None, slopes: torch.Tensor | None = None,
-                            more: AttentionMore | None = None, arrivals: torch.Tensor | None = None) -> torch.Tensor:
+                            more: AttentionMore | None = None) -> torch.Tensor:
     """bfloat16 attention of prompt portions on the matrix cores.  Request s brings the rows
     q_start[s] .. q_start[s]+q_len[s]-1 at the positions ctx_len[s]-q_len[s] .. ctx_len[s]-1;
     requests with fewer than ``short_limit`` tokens are skipped.  ``max_ctx`` (the longest context
     of the step) lets the keys of a token tile be dealt to several workgroups where the tiles alone
     would leave compute units idle; ``splits`` sets their number by hand.  ``live_seqs``: only so many
-    of the requests, the first ones, bring tokens (the rest is padding and gets no workgroups).  ``arrivals``: as for
-    ``paged_attention_decode``."""
+    of the requests, the first ones, bring tokens (the rest is padding and gets no workgroups)."""
     n = q.shape[0]
     S = block_table.shape[0]
     _need(q, "query buffer", None, torch.bfloat16)
@@ -684,7 +683,7 @@ def paged_attention_prefill(q: torch.Tensor, q_row_stride: int, out: torch.Tenso
         q.data_ptr(), q_row_stride, out.data_ptr(), q_start.data_ptr(), q_len.data_ptr(), ctx_len.data_ptr(),
         int(short_limit), live, int(max_q_len), block_table.data_ptr(), block_table.shape[1], block_size,
         k_pool.data_ptr(), v_pool.data_ptr(), nq, nkv, d, float(scale), int(window or 0), int(splits),
-        _arrivals_ptr(arrivals, n * nq), part_acc.data_ptr() if splits > 1 else None, part_ml.data_ptr() if splits > 1 else None, n,
+        part_acc.data_ptr() if splits > 1 else None, part_ml.data_ptr() if splits > 1 else None, n,
         _ptr(_head_numbers(sinks, "sinks", nq)), _ptr(_head_numbers(slopes, "distance slopes", nq)),
         *_more_args(more, nq, n), _stream()))
     return out
@@ -851,8 +850,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
         paged_attention_prefill(qkv, stride, out, batch.q_start, batch.q_len, batch.ctx_len, batch.max_q_len,
                                 kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window,
                                 short_limit=0 if all_tiled else SHORT_PORTION, max_ctx=batch.max_ctx_len,
-                                live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more,
-                                arrivals=_arrivals(batch, nq))
+                                live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more)
         if short_tokens == 0 or all_tiled:
             return out
     mixed = batch.max_q_len >= SHORT_PORTION
