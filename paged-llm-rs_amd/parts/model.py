@@ -192,11 +192,7 @@ class DecoderModel:
                            and getattr(self.embed_transform, "graph_safe", True)
                            and getattr(self.final_transform, "graph_safe", True)
                            and getattr(self.logit_transform, "graph_safe", True))
-        # Mixers that hand requests of few tokens to a kernel of their own say from how many tokens on a
-        # request counts as a long portion; a step reports the tokens of the shorter ones for each such limit.
-        self.portion_limits = tuple(sorted({int(limit) for b in self.blocks
-                                            for limit in [getattr(getattr(b, "mixer", None), "short_portion", None)]
-                                            if limit}))
+        self.portion_limits = portion_limits(self.blocks)
 
     @property
     def _embedding_keeps_state(self) -> bool:
@@ -308,6 +304,18 @@ class DecoderModel:
             top.record(self.spec.head_name.rsplit(".", 1)[0] + ".out", logits)
             top.record("logits", logits)
         return logits
+
+
+def portion_limits(blocks) -> tuple:
+    """Mixers that hand requests of few tokens to a kernel of their own say from how many tokens on a request counts as a long
+    portion (``short_portion``, or ``short_portions`` where they are several mixers); a step reports the tokens of the shorter
+    ones for each such limit.  Whether there are any is part of a captured step's shape, so a limit that is missing here
+    would leave a replayed step without the kernel that its short requests need."""
+    limits = set()
+    for block in blocks:
+        mixer = getattr(block, "mixer", None)
+        limits.update(getattr(mixer, "short_portions", None) or (getattr(mixer, "short_portion", None),))
+    return tuple(sorted(int(limit) for limit in limits if limit))
 
 
 def build_model(config, params: dict, dtype, device) -> DecoderModel:

@@ -56,10 +56,8 @@ class ParallelMixers:
             raise UnsupportedError("more than one of the mixers side by side keeps keys and values in pages")
         self.state_floats = at
         self.graph_safe = all(getattr(m, "graph_safe", True) for m, *_ in self.branches)
-        limits = [getattr(m, "short_portion", None) for m, *_ in self.branches]
-        limits = [x for x in limits if x]
-        if limits:
-            self.short_portion = limits[0]
+        # every branch's own limit: a captured step is laid out for each of them (see ``portion_limits`` in model.py)
+        self.short_portions = tuple(limit for m, *_ in self.branches for limit in [getattr(m, "short_portion", None)] if limit)
 
     def cache_spec(self):
         for mixer, *_ in self.branches:

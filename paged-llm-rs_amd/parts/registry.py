@@ -10,7 +10,8 @@ mixer         ``declare(spec, hidden) -> [ParamDecl]`` (local names);
               ``__init__(spec, hidden, params, dtype, device, shared)``;
               ``cache_spec() -> KVCacheSpec | None``; ``state_spec() -> StateSpec | None``;
               ``forward(x[n,hidden], ctx: LayerContext) -> [n,hidden]``.
-              Optional ``graph_safe = False`` when its forward cannot be captured as a HIP graph.
+              Optional ``graph_safe = False`` when its forward cannot be captured as a HIP graph; ``short_portion`` (or
+              ``short_portions``, several) when its launches go by the tokens of requests that bring fewer than that many.
 feed-forward  ``declare``; ``__init__`` as above; ``forward(x) -> [n,hidden]``.
 norm          ``declare(spec, width)``; ``__init__(spec, width, params, dtype, device)``;
               ``apply(resid, delta, out_dtype, rows=None) -> normed`` which adds

@@ -153,3 +153,27 @@ def test_a_model_without_pages_has_room_without_end_and_still_counts_its_state_s
         steps += 1
         assert steps < 200
     assert seen == {1, 2, 3} and manager.free_state_slots == 2
+
+
+def test_mixers_side_by_side_report_the_limit_of_every_branch(monkeypatch):
+    """A captured step's shape says for every limit whether some request brings fewer tokens: two branches with unlike limits
+    have to be heard both, whichever comes first."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd.parts import parallel
+    from paged_llm_rs_amd.parts.model import portion_limits
+
+    def mixer(limit):
+        def make(*_):
+            return SimpleNamespace(cache_spec=lambda: None, state_spec=lambda: None, **({"short_portion": limit} if limit else {}))
+        return make
+
+    makers = {"few": mixer(4), "more": mixer(16), "none": mixer(None)}
+    monkeypatch.setattr(parallel, "lookup", lambda table, kind, what: makers[kind])
+    blocks = []
+    for kinds in (["none", "more", "few"], ["none"], ["few"]):
+        spec = SimpleNamespace(branches=[(kind, SimpleNamespace(kind=kind), 1.0) for kind in kinds])
+        blocks.append(SimpleNamespace(mixer=parallel.ParallelMixers(spec, 8, {}, torch.float32, "cpu", {})))
+    assert portion_limits(blocks[:1]) == (4, 16)
+    assert portion_limits(blocks[1:2]) == ()
+    assert portion_limits(blocks[1:] + [SimpleNamespace(mixer=makers["more"]()), SimpleNamespace()]) == (4, 16)
