@@ -1290,6 +1290,13 @@ def _step_rows(batch, n: int):
         _need(t, what, (count,), torch.int32)
 
 
+def _brings_short_requests(batch) -> bool:
+    """Whether some request of the step may bring fewer tokens than the kernels in chunks start from.  (A descriptor that does not
+    count them is taken to have such requests: the token-by-token kernel finds none to do and ends.)"""
+    count = getattr(batch, "tokens_of_short_requests", None)
+    return count is None or count(SCAN_CHUNKED_FROM) > 0
+
+
 def scan_state_floats(kind: str, heads: int, dim: int, vdim: int) -> int:
     """32-bit floats a request's state takes: the matrices S [heads, dim, vdim]; for ``mlstm`` also the normaliser n
     and the running maximum m, a copy of each for every tile of 64 columns of vdim (the waves of a head's tiles
@@ -1357,7 +1364,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
               0 if gates is None else gates.shape[1], g1_off, g2_off, _ptr(p1), _ptr(p2), float(cap),
               state.data_ptr(), stride, 0, hdv, hdv + heads * tiles * dim, out.data_ptr(), batch.q_start.data_ptr(),
               batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
-    if not chunked or batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0:
+    if not chunked or _brings_short_requests(batch):
         _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
     if chunked and kind == "delta":
         chunks = (n // SSD_CHUNK + batch.num_seqs + 1) * heads

@@ -491,3 +491,29 @@ def test_the_preparation_of_convolved_heads_in_large_and_in_small_steps(H, G, D,
             m.copy_(torch.where(p != 7.0, p, m))
     for m, p in zip(merged, pools):
         assert torch.equal(m == 7.0, p == 7.0) and close(m, p)
+
+
+@pytest.mark.parametrize("kind", ["lightning", "mlstm", "delta"])
+def test_the_recurrences_over_a_descriptor_that_does_not_count_short_requests(kind):
+    """A step's descriptor need only hold the device's tensors and the longest portion: the same bits as where it also counts the
+    tokens of short requests, in a step with such requests and in one without."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    H, D, V = 2, 32, 64
+    g = torch.Generator().manual_seed(5)
+    for counts in ([70, 3, 1], [40, 90]):
+        b = ScanStep(counts, list(range(len(counts))))
+        bare = SimpleNamespace(**{k: v for k, v in vars(b).items() if k != "counts"})
+        rows = torch.randn((b.num_tokens, H * (V + 2 * D)), generator=g).cuda()
+        gates = None if kind == "lightning" else torch.randn((b.num_tokens, 2 * H), generator=g).cuda()
+        p1, p2 = torch.rand((H,), generator=g).cuda() * 0.4 + 0.5, torch.randn((H,), generator=g).cuda()
+        floats = kernels.scan_state_floats(kind, H, D, V)
+        got = []
+        for step in (b, bare):
+            state = torch.zeros((len(counts), floats)).cuda()
+            out = kernels.recurrent_scan(kind, rows, H * V + H * D, H * V, 0, state, step, H, H, D, V, gates=gates, g1_off=0, g2_off=H, p1=p1,
+                                         p2=None if kind == "lightning" else p2, cap=5.0, chunked=True)
+            got.append((out[:sum(counts)], state))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
