@@ -1816,3 +1816,24 @@ def test_sinks_and_distance_slopes_in_every_attention_kernel(nq, nkv, d, bs, req
                                        q_len=as_i32(q_len), short_limit=limit, sinks=sinks, slopes=slopes)
     for i in range(n):
         assert rel(out[i].float(), plain[i]) < 1.5e-2, f"token {i} (request {seq_of[i]}, position {positions[i]})"
+
+
+def test_32_bit_attention_over_a_descriptor_without_the_requests_rows():
+    """A descriptor that holds each row's position and request only, as the plain kernel reads them, is served by that kernel."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    nq, nkv, d, bs, requests = 4, 2, 64, 16, [(90, 3), (20, 20), (65, 1)]
+    bt, k_pool, v_pool, _, _ = build_paged(nkv, d, bs, [c for c, _ in requests], torch.float32, seed=1)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    positions = i32([c - t + k for c, t in requests for k in range(t)])
+    seq_of = i32([s for s, (_, t) in enumerate(requests) for _ in range(t)])
+    n, stride = positions.numel(), (nq + 2 * nkv) * d
+    q = torch.randn(n, stride, device=DEV)
+    kv = SimpleNamespace(block_table=bt, block_size=bs, k_pool=k_pool, v_pool=v_pool)
+    batch = SimpleNamespace(positions=positions, seq_of=seq_of, num_tokens=n, max_ctx_len=1024)
+    out, plain = (torch.full((n, nq * d), 7.0, device=DEV) for _ in range(2))
+    kernels.paged_attention(q, out, batch, kv, nq, nkv, d, d ** -0.5)
+    kernels.paged_attention_plain(q, stride, plain, positions, seq_of, bt, bs, k_pool, v_pool, nq, nkv, d, d ** -0.5)
+    assert torch.equal(out, plain)
