@@ -449,7 +449,7 @@ struct SsdArgs {
     // the matrix memory's, null for the others
     float* Uk;       // [chunks, H, N]     a chunk's weighted sum of B, for the normaliser
     float* nin;      // [chunks, H, N]     the normaliser before a chunk
-    float* tops;     // [chunks, H, 2]     the largest w_t - b_t of a chunk; the running maximum before it
+    float* tops;     // [chunks, H, 2]     b at the chunk's end plus the largest w_t - b_t; the running maximum before the chunk
 };
 
 // A request's chunks have numbers of their own among all chunks of the step: requests lie one behind the
@@ -536,7 +536,8 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
             for (int off = 32; off > 0; off >>= 1) top = fmax(top, __shfl_xor(top, off, 64));
             weight[lane] = expf(static_cast<float>(dt - top));
             if (vt == 0 && lane == 0) {
-                sa.tops[2 * idx] = static_cast<float>(top);
+                // (their sum: either may be hundreds where it is small, and rounded alone would leave its rounding in the state)
+                sa.tops[2 * idx] = static_cast<float>(end + top);
                 // the maximum that the request's first chunk starts from: the carry reads it here, not in the slot it writes
                 if (c == 0) sa.tops[2 * idx + 1] = a.state[static_cast<size_t>(slot) * a.state_stride + a.m_off + h * tiles];
             }
@@ -626,9 +627,9 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
                 Sin[(c0 + i) * step] = S;
                 if (KIND == PL_SCAN_MLSTM) {
                     if (c0 + i > 0 && e == 0) sa.tops[2 * (first + static_cast<size_t>(c0 + i) * H) + 1] = m;
-                    const float top = fmaxf(m, most[i]);
-                    S = expf(m - top) * S + expf(most[i] - top) * u[i];
-                    m = keep[i] + top;
+                    const float kept = keep[i] + m;
+                    m = fmaxf(kept, most[i]);
+                    S = expf(kept - m) * S + expf(most[i] - m) * u[i];
                 } else {
                     S = expf(keep[i]) * S + u[i];
                 }

@@ -517,3 +517,33 @@ def test_the_recurrences_over_a_descriptor_that_does_not_count_short_requests(ki
                                          p2=None if kind == "lightning" else p2, cap=5.0, chunked=True)
             got.append((out[:sum(counts)], state))
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def test_the_matrix_memory_forgets_hundreds_and_remembers():
+    """Gates that forget nearly all for 60 tokens of a chunk and nothing from then on: the chunk's sum of log gates is some -900 and the
+    largest log weight less that sum as much above zero, while the running maximum is small.  Small inputs let the denominator's
+    floor e^-m decide, so that an error of m would stand in the read-outs.  Chunks, their end and single tokens behind them, against
+    64 bits: some 50 roundings of 2^-24 of the largest read-out behind the first chunk.  (The sum and the maximum rounded one by
+    one: 4e-5 here.)"""
+    from paged_llm_rs_amd import kernels
+
+    H, D, V, T, cap = 8, 32, 32, 133, 15.0
+    g = torch.Generator().manual_seed(3)
+    q, k = (torch.randn((T, H, D), generator=g) for _ in range(2))
+    v = torch.randn((T, H, V), generator=g)
+    at = torch.arange(T)[:, None]
+    x1 = torch.where(at < 64, -2 - torch.rand((T, H), generator=g), torch.full((T, H), -60.0))
+    x2 = torch.where(at < 60, -30 - 20 * torch.rand((T, H), generator=g), torch.full((T, H), 60.0))
+    p1, p2 = torch.zeros(H), torch.zeros(H)
+    want = scan_in_64_bits("mlstm", *(x.double() for x in (q, k, v, x1, x2)), p1.double(), p2.double(), cap).reshape(T, H * V)
+    state = torch.zeros((1, kernels.scan_state_floats("mlstm", H, D, V))).cuda()
+    rows, gates = torch.cat([v.flatten(1), k.flatten(1), q.flatten(1)], -1), torch.cat([x1, x2], -1)
+    pad, got, begin = (lambda x: torch.nn.functional.pad(x, (0, 0, 0, 2)).cuda()), [], 0
+    for count in (130, 1, 2):
+        span = slice(begin, begin + count)
+        out = kernels.recurrent_scan("mlstm", pad(rows[span]), H * V + H * D, H * V, 0, state, ScanStep([count], [0]), H, H, D, V,
+                                     gates=pad(gates[span]), g1_off=0, g2_off=H, p1=p1.cuda(), p2=p2.cuda(), cap=cap, chunked=True)
+        got.append(out[:count].double().cpu())
+        begin += count
+    err = (torch.cat(got) - want)[64:].abs().max() / want[64:].abs().max()
+    assert float(err) < 50 * 2.0 ** -24, float(err)
