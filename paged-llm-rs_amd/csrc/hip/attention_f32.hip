@@ -14,6 +14,8 @@
 // Bound by the matrix cores with many tokens and by the chain of loads with few.  Before this kernel a wave walked all keys
 // of one query head, a key a lane: a step of 8 tokens at contexts up to 512 (16 heads over 8 of 128) 472 us, a prompt of
 // 700 tokens 660 us.
+#include <cfloat>
+
 #include "common.hpp"
 
 typedef float af_f32x4 __attribute__((ext_vector_type(4)));
@@ -214,6 +216,7 @@ attention_f32_kernel(const float* __restrict__ q, int q_stride, float* __restric
                 }
             sum += __shfl_xor(sum, 16, PL_WAVE);
             sum += __shfl_xor(sum, 32, PL_WAVE);
+            if (sum != sum) top = fmaxf(top, -FLT_MAX);     // (scores that are all NaN: not a segment without keys)
             // Values of keys that are not there count as zeros.  Keys that some rows of the tile see and others do not meet
             // weights of zero there, which has to give zero: an infinity or a NaN among such a segment's values stays out
             // of the products and joins the rows that see it one by one.

@@ -1837,3 +1837,38 @@ def test_32_bit_attention_over_a_descriptor_without_the_requests_rows():
     kernels.paged_attention(q, out, batch, kv, nq, nkv, d, d ** -0.5)
     kernels.paged_attention_plain(q, stride, plain, positions, seq_of, bt, bs, k_pool, v_pool, nq, nkv, d, d ** -0.5)
     assert torch.equal(out, plain)
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_32_bit_attention_keeps_what_is_no_number(split):
+    """A query that is NaN, and a NaN in the only key of a segment: the rows that meet it are NaN, also where no other
+    score stands in the segment, and the others keep their bits."""
+    from paged_llm_rs_amd import kernels
+
+    nq, nkv, d, bs, requests = 4, 2, 64, 16, [(65, 1), (130, 4), (20, 20)]
+    ctx, starts = [c for c, _ in requests], [0, 1, 5]
+    bt, k_pool, v_pool, _, _ = build_paged(nkv, d, bs, ctx, torch.float32, seed=2)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    positions = i32([c - t + k for c, t in requests for k in range(t)])
+    n, stride = positions.numel(), (nq + 2 * nkv) * d
+    q = torch.randn(n, stride, device=DEV)
+
+    def run(q, k_pool):
+        out = torch.full((n, nq * d), 7.0, device=DEV)
+        kernels.paged_attention_f32(q, stride, out, positions, i32(starts), i32([t for _, t in requests]), i32(ctx), bt, bs, k_pool, v_pool,
+                                    nq, nkv, d, d ** -0.5, max(ctx), split=split)
+        return out.view(n, nq, d)
+
+    want = run(q, k_pool)
+    assert bool(want.isfinite().all())
+    holed, keys = q.clone(), k_pool.clone()
+    holed[7, d + 3] = math.nan                                          # head 1 of the third request's third token
+    got = run(holed, k_pool)
+    assert bool(got[7, 1].isnan().all())
+    got[7, 1] = want[7, 1]
+    assert torch.equal(got, want)
+    keys[int(bt[0, 64 // bs]) * bs + 64 % bs, d] = math.nan             # key head 1 of position 64, its segment's only key
+    got = run(q, keys)
+    assert bool(got[0, 2:].isnan().all())
+    got[0, 2:] = want[0, 2:]
+    assert torch.equal(got, want)
