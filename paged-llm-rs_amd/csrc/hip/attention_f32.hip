@@ -348,6 +348,11 @@ attention_f32_merge_kernel(float* __restrict__ out, const int* __restrict__ posi
     const int segments = front + pos / AF_SEGMENT - from + 1;
     const size_t base = (static_cast<size_t>(row) * nq + head) * max_segments;
     const int col = threadIdx.x * 4;
+    float* const to = out + (static_cast<size_t>(row) * nq + head) * d + col;
+    if (pos / AF_SEGMENT >= max_segments) {             // (a context longer than the launch was told: there is no room with its last segments)
+        if (col < d) *reinterpret_cast<af_f32x4*>(to) = af_f32x4{NAN, NAN, NAN, NAN};
+        return;
+    }
     float m = -INFINITY, l = 0.f;
     af_f32x4 a = {0.f, 0.f, 0.f, 0.f};
     constexpr int AHEAD = 4;
@@ -372,9 +377,7 @@ attention_f32_merge_kernel(float* __restrict__ out, const int* __restrict__ posi
         }
     }
     const float by = af_finish(m, l, row, head, sinks, more);
-    if (col < d)
-        *reinterpret_cast<af_f32x4*>(out + (static_cast<size_t>(row) * nq + head) * d + col) =
-            by == 0.f ? af_f32x4{0.f, 0.f, 0.f, 0.f} : a * by;
+    if (col < d) *reinterpret_cast<af_f32x4*>(to) = by == 0.f ? af_f32x4{0.f, 0.f, 0.f, 0.f} : a * by;
 }
 
 // Whether the kernel takes heads of this size over these tensors (all rows are then whole groups of four aligned values).
@@ -386,7 +389,7 @@ extern "C" int pl_paged_attention_f32_applies(const void* q, int q_stride, const
 
 // Request s of the first `num_seqs` brings the rows q_start[s] .. q_start[s] + q_len[s] - 1 at the positions that end in
 // ctx_len[s] - 1.  `part_acc` [n, nq, max_segments, d] and `part_ml` [n, nq, max_segments, 2]: room for the segments of every
-// row where they are folded by a second kernel; null: folded in the first.
+// row where they are folded by a second kernel (rows at positions behind them come out as NaN); null: folded in the first.
 extern "C" int pl_paged_attention_f32(const float* q, int q_stride, float* out, const int* positions, const int* q_start,
                                       const int* q_len, const int* ctx_len, int num_seqs, const int* block_table, int max_blocks,
                                       int block_size, const float* k_pool, const float* v_pool, int n, int nq, int nkv, int d,

@@ -418,7 +418,7 @@ def paged_attention_f32(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, p
                         split: bool | None = None) -> torch.Tensor:
     """32-bit attention of any rows on the matrix cores' 32-bit instruction.  Request s brings the rows q_start[s] ..
     q_start[s] + q_len[s] - 1, which end at position ctx_len[s] - 1 (``positions`` says the same row by row); no context
-    is longer than ``max_ctx``.  ``live_seqs``: only so many of the requests, the first ones, bring tokens.  ``split``: whether
+    is longer than ``max_ctx`` (with ``split`` rows of longer ones come out as NaN).  ``live_seqs``: only so many of the requests, the first ones, bring tokens.  ``split``: whether
     a second kernel folds the keys' segments (``f32_splits`` where not given); the result is the same bit for bit.  What is
     left: as for ``paged_attention_plain``."""
     n = positions.numel()

@@ -1872,3 +1872,26 @@ def test_32_bit_attention_keeps_what_is_no_number(split):
     assert bool(got[0, 2:].isnan().all())
     got[0, 2:] = want[0, 2:]
     assert torch.equal(got, want)
+
+
+def test_32_bit_attention_of_contexts_longer_than_the_launch_was_told():
+    """The room for segments is sized by ``max_ctx``: rows at positions behind it are NaN, nothing outside the room is read,
+    and the other rows keep their bits."""
+    from paged_llm_rs_amd import kernels
+
+    nq, nkv, d, bs, requests, told = 4, 2, 64, 16, [(64, 2), (300, 1), (130, 4)], 128
+    ctx, starts = [c for c, _ in requests], [0, 2, 3]
+    bt, k_pool, v_pool, _, _ = build_paged(nkv, d, bs, ctx, torch.float32, seed=3)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    positions = [c - t + k for c, t in requests for k in range(t)]
+    n, stride = len(positions), (nq + 2 * nkv) * d
+    q = torch.randn(n, stride, device=DEV)
+
+    def run(max_ctx):
+        out = torch.full((n, nq * d), 7.0, device=DEV)
+        return kernels.paged_attention_f32(q, stride, out, i32(positions), i32(starts), i32([t for _, t in requests]), i32(ctx), bt, bs,
+                                           k_pool, v_pool, nq, nkv, d, d ** -0.5, max_ctx, split=True)
+
+    want, got = run(max(ctx)), run(told)
+    for row, position in enumerate(positions):
+        assert bool(got[row].isnan().all()) if position >= told else torch.equal(got[row], want[row]), position
