@@ -613,10 +613,18 @@ paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t
             finish(h, dd, big, sum, a);
         } else {
             const size_t pi = (static_cast<size_t>(t) * nq + h) * splits + split;
-            pl_share(part_acc + pi * d + dd, a);
-            if (dd == 0) {
-                pl_share(part_ml + pi * 2, big);
-                pl_share(part_ml + pi * 2 + 1, sum);
+            if (arrivals != nullptr) {
+                pl_share(part_acc + pi * d + dd, a);
+                if (dd == 0) {
+                    pl_share(part_ml + pi * 2, big);
+                    pl_share(part_ml + pi * 2 + 1, sum);
+                }
+            } else {
+                part_acc[pi * d + dd] = a;
+                if (dd == 0) {
+                    part_ml[pi * 2] = big;
+                    part_ml[pi * 2 + 1] = sum;
+                }
             }
         }
     }

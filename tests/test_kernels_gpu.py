@@ -1608,9 +1608,10 @@ def test_a_norm_handed_forward_from_one_product_to_the_next(n, H, deep, N2, swig
 
 @pytest.mark.parametrize("window", [0, 40])
 def test_shares_that_meet_in_the_kernel_and_shares_merged_by_a_second(window):
-    """Single tokens in one to sixteen shares, with room for the workgroups' arrivals and without,
-    over contexts that leave some shares without keys: the same bits, the same again in the next launch, and the room is zeros
-    again behind every one."""
+    """Single tokens in two to eight shares, with room for the workgroups' arrivals and without, over contexts that leave some
+    shares without keys: the same bits, the same again in the next launch, and the room is zeros again behind every one.  The same
+    with only the short requests' tokens served, and in a step of one token a request that prepares its own queries and keys.
+    One share and nine leave the room alone."""
     from paged_llm_rs_amd import kernels
 
     bs, requests = 16, [(300, 1), (9, 1), (700, 3), (70, 40), (1000, 130), (64, 64), (1, 1)]
@@ -1633,12 +1634,32 @@ def test_shares_that_meet_in_the_kernel_and_shares_merged_by_a_second(window):
             out = torch.full((n, nq * d), 7.0, device=DEV).bfloat16()
             return kernels.paged_attention_decode(q, stride, out, positions, seq_of, *paged, splits, sinks=sinks, **more)
 
-        for splits in (1, 2, 3, 4, 8, 16):
+        short = dict(q_len=q_len, short_limit=16, short_rows=8, live_seqs=len(requests))
+        served = torch.tensor([t < 16 for _, t in requests for _ in range(t)], device=DEV)
+        lone_at, lone_of, raw = i32([c - 1 for c in ctx]), i32(list(range(len(ctx)))), torch.randn(len(ctx), stride, device=DEV).bfloat16()
+        gain = (1 + 0.2 * torch.randn(d, device=DEV)).bfloat16()
+        angle = torch.rand(max(ctx), d // 2, device=DEV) * 6
+        fuse = kernels.QkFusion(gain, gain, 1e-5, angle.cos(), angle.sin(), d, True)
+
+        def prepared(splits, **more):
+            k, v, out = k_pool.clone(), v_pool.clone(), torch.full((len(ctx), nq * d), 7.0, device=DEV).bfloat16()
+            kernels.paged_attention_decode(raw, stride, out, lone_at, lone_of, bt, bs, k, v, nq, nkv, d, d ** -0.5, window, splits,
+                                           sinks=sinks, fuse=fuse, **more)
+            return out
+
+        for splits in range(2, 9):
             want = single(splits)
-            got = single(splits, arrivals=arrivals)
-            assert torch.equal(got, want), (nq, d, splits)
-            assert torch.equal(got, single(splits, arrivals=arrivals)), (nq, d, splits)
-            assert not bool(arrivals.any())
+            assert bool(want.isfinite().all())
+            for name, run in (("all", single), ("short", lambda s, **k: single(s, **short, **k)), ("prepared", prepared)):
+                apart, together = run(splits), run(splits, arrivals=arrivals)
+                assert torch.equal(together, apart), (name, nq, d, splits)
+                assert torch.equal(run(splits, arrivals=arrivals), apart), (name, nq, d, splits)
+                assert not bool(arrivals.any()), (name, nq, d, splits)
+                if name == "short":
+                    assert torch.equal(together[served], want[served]) and bool((together[~served] == 7.0).all())
+        arrivals.fill_(5)
+        for splits in (1, 9):
+            assert torch.equal(single(splits, arrivals=arrivals), single(splits)) and bool((arrivals == 5).all())
 
 
 def attention_with_everything(q, keys, values, pos, g, scale, window, sinks, slopes, more, row):
