@@ -836,6 +836,9 @@ static int dispatch_gt(int gt, const void* q, int q_stride, void* out, float* pa
 #undef AD_CALL
 }
 
+// The most shares whose workgroups meet in the kernel.
+extern "C" int pl_paged_attention_decode_meets() { return AD_MERGE_AT_ONCE; }
+
 // bfloat16 only.  With splits > 1 the workspace needs n*nq*splits*d floats (part_acc) and n*nq*splits*2 (part_ml).
 // q_len (may be null) and short_limit leave the tokens of requests with q_len >= short_limit to the tiled kernel.
 // With q_len: num_seqs, the requests whose rows follow each other in q from row 0 on, and short_rows, the most

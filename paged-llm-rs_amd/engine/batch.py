@@ -33,9 +33,9 @@ class StepEntry:
     fed_row: int = -1
 
 
-# Steps of up to so many rows bring room for the arrivals of attention workgroups that share the keys of a row (an int32 a row and
-# query head, up to so many heads); the keys of larger steps' rows are seldom shared out, and a second kernel puts them together.
-ARRIVAL_ROWS, ARRIVAL_HEADS = 1024, 64
+# Steps of up to so many rows have room for the arrivals of attention workgroups that share the keys of a row; the keys of larger
+# steps' rows are seldom shared out, and a second kernel puts them together.
+ARRIVAL_ROWS = 1024
 
 
 class StepBatch:
@@ -60,10 +60,10 @@ class StepBatch:
                             else np.asarray(tokens_each, dtype=np.int64))
         self.padded = padded
         self.short_bounds = dict(short_bounds or {})
-        # Zeros between any two kernels (``kernels.paged_attention_decode``).  They belong to this step alone: steps on other
-        # streams, of this cache or of another, count in their own.
-        self.arrivals = (torch.zeros(num_tokens * ARRIVAL_HEADS, dtype=torch.int32, device=packed.device)
-                         if packed.is_cuda and num_tokens <= ARRIVAL_ROWS else None)
+        # Zeros between any two kernels (``kernels.paged_attention_decode``), once a layer has asked for them.  They belong to this
+        # step alone: steps on other streams, of this cache or of another, count in their own.
+        self._arrivals = None
+        self._stream = torch.cuda.current_stream(packed.device) if packed.is_cuda else None
 
         def view(name, *shape):
             begin, count = layout[name]
@@ -82,6 +82,24 @@ class StepBatch:
         self.state_slots = view("state_slots", num_seqs)
         self.logit_rows = view("logit_rows", num_logit_rows)
         self.block_tables = [view(f"block_table_{g}", num_seqs, mb) for g, mb in enumerate(max_blocks)]
+
+    def arrivals(self, heads: int):
+        """An int32 zero a row and each of ``heads`` query heads (or more of them), or None where the step has none to give.  Made
+        at the first use, on the stream that the step was laid out on: the run before a capture, which is on another, leaves
+        what its capture finds.  None in a capture without such a run: zeros written in a graph would not be there before its replay."""
+        need = self.num_tokens * heads
+        if self._arrivals is not None and self._arrivals.numel() >= need:
+            return self._arrivals
+        if self._stream is None or self.num_tokens > ARRIVAL_ROWS or torch.cuda.is_current_stream_capturing():
+            return None
+        now = torch.cuda.current_stream(self.packed.device)
+        if self._arrivals is not None and now != self._stream:
+            self._stream.wait_stream(now)       # (the smaller room goes, which a kernel on this stream may still count in)
+        with torch.cuda.stream(self._stream):
+            self._arrivals = torch.zeros(need, dtype=torch.int32, device=self.packed.device)
+        if now != self._stream:
+            now.wait_stream(self._stream)
+        return self._arrivals
 
     def tokens_of_short_requests(self, limit: int) -> int:
         """How many tokens the requests that bring fewer than ``limit`` tokens bring together: what a

@@ -61,6 +61,7 @@ def _signatures(lib) -> None:
         "pl_gemm_finish": [p, p, ctypes.c_longlong, i, i, i, i, i, p],
         "pl_paged_attention_decode": [p, i, p, p, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, i, f, i, i,
                                       i, p, p, i, f, p, p, i, p, p, f, i, p, i, p, p],
+        "pl_paged_attention_decode_meets": [],
         "pl_paged_attention_prefill": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped_applies": [i, i, i, i],
@@ -500,10 +501,11 @@ def _arrivals_ptr(arrivals, count: int) -> int:
     return _need(arrivals, "arrivals", None, torch.int32).data_ptr()
 
 
-def _arrivals(batch, nq: int):
-    """The step's room for the arrivals of its shares' workgroups, where it has enough for ``nq`` heads."""
-    room = getattr(batch, "arrivals", None)
-    return room if room is not None and room.numel() >= batch.num_tokens * nq else None
+def _arrivals(batch, nq: int, splits: int):
+    """The step's room for the arrivals of its shares' workgroups, where they count themselves."""
+    if not 1 < splits <= library().pl_paged_attention_decode_meets() or not hasattr(batch, "arrivals"):
+        return None
+    return batch.arrivals(nq)
 
 
 _attention_mode = "kernel"
@@ -811,7 +813,7 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
         splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d)
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
-                                      fuse=prepare, arrivals=_arrivals(batch, nq))
+                                      fuse=prepare, arrivals=_arrivals(batch, nq, splits))
     qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
                           batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
                           nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)
@@ -872,7 +874,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                                   kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                   q_len=batch.q_len if mixed else None, short_limit=SHORT_PORTION if mixed else 0,
                                   live_seqs=getattr(batch, "live_seqs", None), short_rows=short_tokens,
-                                  sinks=sinks, slopes=slopes, more=more, arrivals=_arrivals(batch, nq))
+                                  sinks=sinks, slopes=slopes, more=more, arrivals=_arrivals(batch, nq, splits))
 
 
 class HandedNorm:

@@ -1916,3 +1916,39 @@ def test_32_bit_attention_of_contexts_longer_than_the_launch_was_told():
     want, got = run(max(ctx)), run(told)
     for row, position in enumerate(positions):
         assert bool(got[row].isnan().all()) if position >= told else torch.equal(got[row], want[row]), position
+
+
+def test_a_steps_room_for_arrivals_is_made_where_a_layer_shares_keys_out():
+    """Nothing is allocated for a step before a layer's shares are to meet; any number of heads has room; a capture takes the room
+    that the run before it left, and makes none that would only be cleared in the graph; many rows have none."""
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.engine.batch import ARRIVAL_ROWS, StepBatch
+
+    def step(rows):
+        pieces = [("token_ids", rows), ("positions", rows), ("seq_of", rows), ("q_start", rows), ("q_len", rows), ("ctx_len", rows),
+                  ("state_slots", rows), ("logit_rows", rows)]
+        layout, at = {}, 0
+        for name, count in pieces:
+            layout[name], at = (at, count), at + count
+        return StepBatch(torch.zeros(at, dtype=torch.int32, device=DEV), layout, rows, rows, [], rows, 1, 1024, [])
+
+    most = kernels.library().pl_paged_attention_decode_meets()
+    before = torch.cuda.memory_allocated()
+    batch = step(40)
+    grown = torch.cuda.memory_allocated() - before
+    assert kernels._arrivals(batch, 16, 1) is None and kernels._arrivals(batch, 16, most + 1) is None
+    assert torch.cuda.memory_allocated() - before == grown
+    few = kernels._arrivals(batch, 16, 2)
+    assert few.numel() == 40 * 16 and not bool(few.any()) and kernels._arrivals(batch, 8, 2) is few
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        more = kernels._arrivals(batch, 200, most)
+        assert more.numel() == 40 * 200 and not bool(more.any())
+    torch.cuda.current_stream().wait_stream(side)
+    fresh, graph = step(8), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert kernels._arrivals(batch, 100, 2) is more
+        assert kernels._arrivals(fresh, 100, 2) is None
+        torch.zeros(1, device=DEV)
+    assert kernels._arrivals(fresh, 100, 2).numel() == 800
+    assert kernels._arrivals(step(ARRIVAL_ROWS + 1), 4, 2) is None
