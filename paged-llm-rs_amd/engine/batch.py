@@ -62,6 +62,7 @@ class StepBatch:
         self.short_bounds = dict(short_bounds or {})
         # Zeros between any two kernels (``kernels.paged_attention_decode``), once a layer has asked for them.  They belong to this
         # step alone: steps on other streams, of this cache or of another, count in their own.
+        self.has_arrivals = packed.is_cuda and num_tokens <= ARRIVAL_ROWS
         self._arrivals = None
         self._stream = torch.cuda.current_stream(packed.device) if packed.is_cuda else None
 
@@ -90,7 +91,7 @@ class StepBatch:
         need = self.num_tokens * heads
         if self._arrivals is not None and self._arrivals.numel() >= need:
             return self._arrivals
-        if self._stream is None or self.num_tokens > ARRIVAL_ROWS or torch.cuda.is_current_stream_capturing():
+        if not self.has_arrivals or torch.cuda.is_current_stream_capturing():
             return None
         now = torch.cuda.current_stream(self.packed.device)
         if self._arrivals is not None and now != self._stream:

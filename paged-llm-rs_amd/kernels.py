@@ -501,9 +501,14 @@ def _arrivals_ptr(arrivals, count: int) -> int:
     return _need(arrivals, "arrivals", None, torch.int32).data_ptr()
 
 
+def _has_arrivals(batch) -> bool:
+    """Whether the step gives room for arrivals to a layer that asks (``StepBatch.arrivals``)."""
+    return getattr(batch, "has_arrivals", False)
+
+
 def _arrivals(batch, nq: int, splits: int):
     """The step's room for the arrivals of its shares' workgroups, where they count themselves."""
-    if not 1 < splits <= library().pl_paged_attention_decode_meets() or not hasattr(batch, "arrivals"):
+    if not 1 < splits <= library().pl_paged_attention_decode_meets() or not _has_arrivals(batch):
         return None
     return batch.arrivals(nq)
 
@@ -527,22 +532,26 @@ def set_attention(mode: str) -> None:
     _attention_mode = mode
 
 
-# What a compute unit takes in from memory (bytes a microsecond), what the merge of the shares costs beside the
-# kernel (microseconds), and the compute units: the figures of the estimate below.
+# The figures of the estimate below: what a compute unit takes in from memory (bytes a microsecond); what a workgroup costs it
+# beside that; and what sharing costs the launch, where the shares meet in the kernel, where a second kernel puts them together, and
+# where that one has more than 16 of them, which it fetches in several trips (microseconds).
 DECODE_INTAKE = 22e3
-DECODE_MERGE_US = 4.0
+DECODE_WORKGROUP_US = 0.4
+DECODE_MEET_US, DECODE_MERGE_US, DECODE_MERGE_MANY_US = 4.0, 5.4, 9.0
 
 
-def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128) -> int:
+def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128, meets: bool = True) -> int:
     """Into how many stretches the context is cut for the single-token kernel, each with at least 128 keys
-    (two rounds of loads).
+    (two rounds of loads).  ``meets``: whether the step has counters for the shares to meet in the kernel.
 
     Up to two query heads a key head the kernel waits for memory, and a compute unit takes in only so much:
     the launch is as long as the keys and values of its busiest compute unit take (workgroups are dealt to
-    the compute units in turn), plus the merge's kernel where there are shares; the count with the smallest
-    such estimate is taken.  (Measured, 16 query over 8 key heads of 128, one share against the estimate's
-    choice: 12 tokens at context 2,048, three shares 32.9 us, eight 28.0; 24 tokens, two 50.1, four 45.4; 48
-    tokens at 1,024, one 48.1, two 45.3; 24 tokens at 512, two 20.9, one 18.8.)
+    the compute units in turn), plus what sharing costs; the count with the smallest such estimate is taken.  Over 1 to 64
+    tokens, bounds of 1,024 to 4,096 with contexts at them and far below, 16 over 8 heads of 128, 12 of 96, 4 of 64 and 8 of 128, keys and values
+    of several layers in turn, its choice takes 5% longer than the best count (the estimate before, with a second kernel's 4 us
+    for any number of shares and nothing a workgroup, 11%), and longer than that one's by more than 3% in one of 960.  (16 over 8 of
+    128: one token at 4,096, thirty-two shares 16.8 us, sixteen 14.1; three at 4,096, thirty-two 24.6, ten 20.8; six at 2,048, sixteen
+    19.9, five 19.0; one at 1,536, eight, which meet, 12.2, twelve 11.5.  12 of 96: six at 4,096, thirty-two 39.9, seven 28.3.)
     With more query heads a key head a workgroup has more arithmetic a key and the compute units are what
     is short: none when the tokens and heads alone give about two workgroups a compute unit, else up to
     that many (8 tokens at context 2,048 with four heads a key head: eight shares 24.6 us, four 25.9; 32
@@ -557,11 +566,14 @@ def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128) ->
             return 1
         return max(1, min((target + base - 1) // base, most))
     units = compute_units()
+    meeting = library().pl_paged_attention_decode_meets() if meets else 1
     best, best_us = 1, None
     for splits in range(1, most + 1):
         busiest = -(-base * splits // units)                      # workgroups on one compute unit
         keys = -(-max_ctx // splits)
-        us = busiest * keys * (4 * d) / DECODE_INTAKE + (DECODE_MERGE_US if splits > 1 else 0.0)
+        together = (0.0 if splits == 1 else DECODE_MEET_US if splits <= meeting else DECODE_MERGE_US if splits <= 16
+                    else DECODE_MERGE_MANY_US)
+        us = busiest * (keys * (4 * d) / DECODE_INTAKE + DECODE_WORKGROUP_US) + together
         if best_us is None or us < best_us - 1e-9:
             best, best_us = splits, us
     return best
@@ -810,7 +822,7 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
     any other step runs the stand-alone kernel for the first three and then attention."""
     if (qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and batch.max_q_len == 1
             and prepare.rot % 16 == 0 and not prepare.neighbours and not grouped_applies(nq, nkv, d, kv.block_size)):
-        splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d)
+        splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d, _has_arrivals(batch))
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                       fuse=prepare, arrivals=_arrivals(batch, nq, splits))
@@ -869,7 +881,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                                        short_limit=SHORT_PORTION if mixed else 0, max_ctx=reach,
                                        live_seqs=getattr(batch, "live_seqs", None), tokens=short_tokens,
                                        sinks=sinks, slopes=slopes, more=more)
-    splits = decode_splits(short_tokens, nq, nkv, reach, d)
+    splits = decode_splits(short_tokens, nq, nkv, reach, d, _has_arrivals(batch))
     return paged_attention_decode(qkv, stride, out, batch.positions, batch.seq_of, kv.block_table,
                                   kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                   q_len=batch.q_len if mixed else None, short_limit=SHORT_PORTION if mixed else 0,

@@ -1952,3 +1952,18 @@ def test_a_steps_room_for_arrivals_is_made_where_a_layer_shares_keys_out():
         torch.zeros(1, device=DEV)
     assert kernels._arrivals(fresh, 100, 2).numel() == 800
     assert kernels._arrivals(step(ARRIVAL_ROWS + 1), 4, 2) is None
+
+
+def test_the_number_of_shares_goes_by_what_putting_them_together_costs():
+    """Where the estimate for single tokens leaves one way of putting shares together for another: no more than meet in the kernel
+    where a second kernel costs more than shorter shares give, no more than sixteen where that one would fetch them in several trips,
+    and a step without counters pays for the second kernel from two shares on."""
+    from paged_llm_rs_amd import kernels
+
+    if kernels.compute_units() != 256:
+        pytest.skip("the counts below are for 256 compute units")
+    picked = lambda tokens, nq, nkv, d, bound, **more: kernels.decode_splits(tokens, nq, nkv, bound, d, **more)
+    assert [picked(1, 4, 4, 64, bound) for bound in (128, 1024, 1536, 4096)] == [1, 8, 8, 16]
+    assert [picked(1, 16, 8, 128, bound) for bound in (1024, 1536, 2048, 4096, 16384)] == [8, 12, 16, 16, 32]
+    assert [picked(6, 12, 12, 96, bound) for bound in (1024, 4096)] == [7, 7]
+    assert picked(1, 4, 4, 64, 1536, meets=False) == 12
