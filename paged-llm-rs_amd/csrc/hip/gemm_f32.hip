@@ -166,6 +166,26 @@ gemm_f32_few_kernel(const float* __restrict__ x, const float* __restrict__ w, fl
 #define F32_BK 32
 #define F32_STAGES 4
 
+// The workgroup's tile, of row_tiles x col_tiles.  Workgroups go to the eight XCDs in turn: an XCD gets every eighth column of tiles,
+// the rows of x first, so that a row of w is read into one L2 only; the tiles of the columns left over are dealt out in
+// runs, so that no XCD has more than one of them more than another.  (With those as whole columns too 16 heads of 1,500 rows by 128 by 192,
+// two columns of tiles, ran on two of the eight XCDs: 55 us, 19 so; 64 by 128 24 and 9.9.  With runs of all tiles 400 rows of 8,192 x
+// 4,096 took 257 us, 241 so.)
+__device__ __forceinline__ bool f32_tile(int row_tiles, int col_tiles, int& row_tile, int& col_tile) {
+    const int whole = col_tiles / 8 * 8, in_whole = whole * row_tiles;
+    int at = blockIdx.x;
+    if (at < in_whole) {
+        col_tile = at % 8 + at / 8 / row_tiles * 8;
+        row_tile = at / 8 % row_tiles;
+        return true;
+    }
+    at -= in_whole;             // (a multiple of eight: the XCDs' turns begin anew)
+    at = at % 8 * ((gridDim.x - in_whole) / 8) + at / 8;
+    row_tile = at % row_tiles;
+    col_tile = whole + at / row_tiles;
+    return col_tile < col_tiles;
+}
+
 // 16 bytes a lane from `offset` bytes behind `base` (the same for the wave) to LDS, lane after lane from byte `to` on.  Assembly,
 // so that the compiler does not count the load and make every later read of LDS wait for all of them.
 __device__ __forceinline__ void f32_load_to_lds(const void* base, uint32_t offset, uint32_t to) {
@@ -180,10 +200,8 @@ gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     constexpr int TM = TILE / 32, TN = TM;                      // tiles of 16 a wave: columns, rows
     constexpr int STAGE = 2 * TILE * F32_BK, LOADS = TILE / 16;
     extern __shared__ __attribute__((aligned(16))) float f32_lds[];         // [stage][rows of x, then columns of w][32]
-    // Workgroups go to the eight XCDs in turn: an XCD gets whole columns of tiles, so that a row of w is read into one
-    // L2 only, and walks the rows of x first.
-    const int col_tile = blockIdx.x % 8 + 8 * (blockIdx.x / 8 / row_tiles), row_tile = blockIdx.x / 8 % row_tiles;
-    if (col_tile >= col_tiles) return;      // (the whole workgroup)
+    int row_tile, col_tile;
+    if (!f32_tile(row_tiles, col_tiles, row_tile, col_tile)) return;        // (the whole workgroup)
     const int m0 = row_tile * TILE, n0 = col_tile * TILE;
     const int lane = threadIdx.x % PL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PL_WAVE);
     const int r = lane % 16, c = lane / 16;
@@ -309,7 +327,7 @@ void launch_tiled(const F32Product& g, hipStream_t stream) {
     constexpr size_t lds = sizeof(float) * F32_STAGES * 2 * TILE * F32_BK;
     static_assert(lds <= 64 * 1024, "a workgroup's LDS");
     const int row_tiles = pl_ceil_div(g.n, TILE), col_tiles = pl_ceil_div(g.N, TILE);
-    const dim3 grid(pl_ceil_div(col_tiles, 8) * 8 * row_tiles, 1, g.batch);
+    const dim3 grid(pl_ceil_div(col_tiles * row_tiles, 8) * 8, 1, g.batch);
     gemm_f32_tiled_kernel<TILE><<<grid, 256, lds, stream>>>(g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw, g.sy,
                                                             f32_part_len(g.K), row_tiles, col_tiles);
 }

@@ -1967,3 +1967,22 @@ def test_the_number_of_shares_goes_by_what_putting_them_together_costs():
     assert [picked(1, 16, 8, 128, bound) for bound in (1024, 1536, 2048, 4096, 16384)] == [8, 12, 16, 16, 32]
     assert [picked(6, 12, 12, 96, bound) for bound in (1024, 4096)] == [7, 7]
     assert picked(1, 4, 4, 64, 1536, meets=False) == 12
+
+
+@pytest.mark.parametrize("N", [1, 64, 65, 449, 512, 513, 577, 1100])
+@pytest.mark.parametrize("rows", [40, 65, 300])
+def test_every_tile_of_the_32_bit_product_has_its_workgroup(N, rows):
+    """Fewer columns of tiles than chiplets, whole rounds of them and columns left over, alone and a head at a time: 64-bit
+    arithmetic within a factor of four of what chains of 16 k and 16 parts can be off."""
+    from paged_llm_rs_amd import kernels
+
+    K = 64
+    for heads in (1, 3):
+        x, w = torch.randn(rows, heads, K, device=DEV), torch.randn(heads, N, K, device=DEV)
+        got = torch.full((rows, heads, N), math.nan, device=DEV)
+        if heads == 1:
+            kernels.gemm_plain(x[:, 0], w[0], out=got[:, 0])
+        else:
+            kernels.gemm_heads(x, kernels.head_weights(w), got)
+        want = (x.double().transpose(0, 1) @ w.double().transpose(1, 2).contiguous()).transpose(0, 1)
+        assert rel(got, want) < 4 * math.sqrt(K / 16 + 16) * 2.0 ** -24
