@@ -55,8 +55,8 @@ __device__ __forceinline__ void f32_store4(float* to, f32x4 v, int col, int N, b
 
 // ---- few rows ----------------------------------------------------------------------------------------------------------------
 // Bound by the weights' bytes.  A workgroup of sixteen waves owns 16 columns and TN x 16 rows of x; a wave takes one part
-// of K straight from memory in the instruction's layout, 64 k a round, and the parts meet in LDS.  Also the product of many
-// rows whose rows are not made of aligned groups of four values (VEC false, a row tile a blockIdx.y).
+// of K straight from memory in the instruction's layout, 64 k a round, and the parts meet in LDS (a row tile a blockIdx.y).
+// VEC: rows are made of aligned groups of four values.
 //
 // With at most 8 rows of x half of the instruction's 16 would be copies.  SHARE 2 gives that half to another part of K: a wave takes
 // two parts of 8 columns, rows 0 .. 7 of its operands from one part and 8 .. 15 from the next, and of the result keeps the two
@@ -306,6 +306,112 @@ gemm_f32_tiled_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     }
 }
 
+// ---- many rows, any K ----------------------------------------------------------------------------------------------------------
+// The same where K is no multiple of 64 or rows are not aligned groups of four values: a step's operands come through registers,
+// asked for two steps ahead, into two stages of LDS that take turns.  What lies past K counts as zeros, which leave a chain as it is.
+// Bound by the matrix cores and the barrier a step, and by the loads' issue where they are of one value (VEC false): 1,500 rows of 4,096 x
+// 1,026 81 TFLOP/s, of 4,096 x 4,128 110; the kernel for few rows, which took them before, 21 and 57.
+template <int TILE, bool VEC>
+__global__ void __launch_bounds__(256)
+gemm_f32_ragged_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int n, int N, int K,
+                       int ldx, int ldy, long sx, long sw, long sy, int part_len, int row_tiles, int col_tiles) {
+    constexpr int TM = TILE / 32, TN = TM;                      // tiles of 16 a wave: columns, rows
+    constexpr int STAGE = 2 * TILE * F32_BK, WIDE = VEC ? 4 : 1, LANES = F32_BK / WIDE, LOADS = STAGE / 256 / WIDE;
+    __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];           // [stage][rows of x, then columns of w][32]
+    int row_tile, col_tile;
+    if (!f32_tile(row_tiles, col_tiles, row_tile, col_tile)) return;        // (the whole workgroup)
+    const int m0 = row_tile * TILE, n0 = col_tile * TILE;
+    const int lane = threadIdx.x % PL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PL_WAVE);
+    const int r = lane % 16, c = lane / 16;
+    y += blockIdx.z * sy;
+
+    const int kk = threadIdx.x % LANES * WIDE, first = threadIdx.x / LANES;
+    const float* from[LOADS];                                   // rows first + i * 8 WIDE of the stage
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = first + i * 8 * WIDE;
+        from[i] = i < LOADS / 2 ? x + blockIdx.z * sx + static_cast<size_t>(min(m0 + row, n - 1)) * ldx
+                                : w + blockIdx.z * sw + static_cast<size_t>(min(n0 + row - TILE, N - 1)) * K;
+    }
+    float* const to = lds + first * F32_BK + ((kk / 4) ^ first % 8) * 4 + kk % 4;
+    f32x4 wide[VEC ? LOADS : 1];
+    float narrow[VEC ? 1 : LOADS];
+    auto ask = [&](int step) {
+        const int k = step * F32_BK + kk;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            if (VEC) wide[i] = f32_load4<VEC>(from[i], k, K);
+            else narrow[i] = from[i][min(k, K - 1)];
+        }
+    };
+    auto put = [&](int step) {
+        const int k = step * F32_BK + kk;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            float* at = to + step % 2 * STAGE + i * 8 * WIDE * F32_BK;
+            if (VEC) *reinterpret_cast<f32x4*>(at) = f32_end(wide[i], k, K);
+            else *at = k < K ? narrow[i] : 0.f;
+        }
+    };
+    int a_at[2], b_at[2];                   // this lane's operands in a stage, for either half of a step
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int slot = ((c + 4 * h) ^ r % 8) * 4;
+        a_at[h] = (TILE + wave % 2 * TM * 16 + r) * F32_BK + slot;
+        b_at[h] = (wave / 2 * TN * 16 + r) * F32_BK + slot;
+    }
+    f32x4 acc[TM][TN], total[TM][TN];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) total[i][j] = zero;
+    ask(0);
+    put(0);
+    ask(1);
+    __syncthreads();
+    const int steps = (K + F32_BK - 1) / F32_BK, part_steps = part_len / F32_BK;
+    for (int s0 = 0; s0 < steps; s0 += part_steps) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = zero;
+        const int stop = min(steps, s0 + part_steps);
+        for (int s = s0; s < stop; ++s) {
+            const float* stage = lds + s % 2 * STAGE;
+            f32x4 a[2][TM], b[2][TN];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) a[h][i] = *reinterpret_cast<const f32x4*>(stage + a_at[h] + i * 16 * F32_BK);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[h][j] = *reinterpret_cast<const f32x4*>(stage + b_at[h] + j * 16 * F32_BK);
+            }
+            put(s + 1);                     // (everybody has read that stage before the last barrier)
+            ask(s + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            f32_multiply<TM, TN>(a[0], b[0], acc);
+            f32_multiply<TM, TN>(a[1], b[1], acc);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) total[i][j] += acc[i][j];
+    }
+    const bool whole = N % 4 == 0 && ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int row = m0 + (wave / 2 * TN + j) * 16 + r;
+        if (row >= n) continue;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int col = n0 + (wave % 2 * TM + i) * 16 + c * 4;
+            f32_store4(y + static_cast<size_t>(row) * ldy + col, total[i][j], col, N, whole);
+        }
+    }
+}
+
 namespace {
 
 struct F32Product {
@@ -332,6 +438,14 @@ void launch_tiled(const F32Product& g, hipStream_t stream) {
                                                             f32_part_len(g.K), row_tiles, col_tiles);
 }
 
+template <int TILE, bool VEC>
+void launch_ragged(const F32Product& g, hipStream_t stream) {
+    const int row_tiles = pl_ceil_div(g.n, TILE), col_tiles = pl_ceil_div(g.N, TILE);
+    const dim3 grid(pl_ceil_div(col_tiles * row_tiles, 8) * 8, 1, g.batch);
+    gemm_f32_ragged_kernel<TILE, VEC><<<grid, 256, 0, stream>>>(g.x, g.w, g.y, g.n, g.N, g.K, g.ldx, g.ldy, g.sx, g.sw, g.sy,
+                                                                f32_part_len(g.K), row_tiles, col_tiles);
+}
+
 }  // namespace
 
 // `batch` products, their operands and results sx, sw and sy values apart.  Which kernel: up to 16 rows the one for few rows,
@@ -345,6 +459,13 @@ void launch_tiled(const F32Product& g, hipStream_t stream) {
 // Tiles of 64 rows by 64 columns or of 32 by 32: the shorter estimate for the compute unit with most of them, a small tile
 // costing 1.15 times as much for what it does (700 rows, tiles of 64 / 32: 1,024 x 2,048 43.7 / 34.7, 4,096 x 1,024 62.3 /
 // 59.5; 2,048 rows, 1,024 x 2,048 76.7 / 87.6, 4,096 x 1,024 152 / 178).
+// Where the tiled kernel does not apply: rows of aligned groups stay with the kernel for few rows while its workgroups are no more than the
+// compute units (us, few / ragged tiles of 32: 200 rows, 1,000 x 1,040 12.7 / 15.6, 300 rows 20.5 / 20.0, 700 rows 30.5 / 26.6; 64 rows,
+// 4,096 x 4,128 46.0 / 55.9, 96 rows 77.6 / 67.0; 17 rows, 151,936 x 1,028 240 / 162), others only up to 16 rows (17 rows, 4,096 x
+// 1,026 19.9 / 17.3, 64 rows 29.9 / 17.5, 1,500 rows 610 / 187).  Ragged tiles of 64 cost a small tile's quarter of 0.83, and another
+// quarter of a tile to begin with (tiles of 64 / 32: 200 rows, 4,096 x 1,026 38.5 / 34.6, 700 rows 77.3 / 84.8, 1,500 rows 156 / 187;
+// 700 rows, 3,072 x 1,000 65.2 / 59.5, 1,500 rows 107 / 114).  On the vector units, before the matrix instruction was used: 700 and
+// 1,500 rows of 4,096 x 1,026 189 and 218.
 int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, int ldx, int ldy, int batch, long sx,
                 long sw, long sy, hipStream_t stream) {
     const F32Product g{x, w, y, n, N, K, ldx, ldy, batch, sx, sw, sy};
@@ -356,26 +477,27 @@ int pl_gemm_f32(const float* x, const float* w, float* y, int n, int N, int K, i
     const auto busiest = [&](int tile) {
         return (static_cast<long>(pl_ceil_div(n, tile)) * pl_ceil_div(N, tile) * batch + units - 1) / units * tile * tile;
     };
-    const bool few = n <= 8 || (n <= 16 && N < 32768) || (n <= 32 && N <= 4096);
+    const long few_workgroups = static_cast<long>(pl_ceil_div(n, n <= 32 ? 32 : 64)) * pl_ceil_div(N, 16) * batch;
+    const bool few = n <= 8 || (n <= 16 && N < 32768) || (tiles && n <= 32 && N <= 4096) || (vec && !tiles && few_workgroups <= units);
     PL_REQUIRE(static_cast<long>(pl_ceil_div(n, 32)) * (pl_ceil_div(N, 32) + 8) < (1L << 31) && pl_ceil_div(n, 64) <= 65535,
                "gemm: %d x %d results are more than one launch covers", n, N);
-    if (few || !tiles) {
-        if (vec) {
-            const bool idle = static_cast<long>(pl_ceil_div(N, 16)) * batch * 2 <= units;
-            if (n == 1 || (n <= 4 && idle)) launch_few<1, true, 4>(g, stream);
-            else if (n <= 8 && idle) launch_few<1, true, 2>(g, stream);
-            else if (n <= 16) launch_few<1, true>(g, stream);
-            else if (n <= 32) launch_few<2, true>(g, stream);
-            else launch_few<4, true>(g, stream);
-        } else if (n <= 16) {
-            launch_few<1, false>(g, stream);
-        } else {
-            launch_few<4, false>(g, stream);
-        }
-    } else if (busiest(64) * 20 <= busiest(32) * 23) {
-        launch_tiled<64>(g, stream);
+    if (few) {
+        const bool idle = static_cast<long>(pl_ceil_div(N, 16)) * batch * 2 <= units;
+        if (!vec) launch_few<1, false>(g, stream);          // (up to 16 rows)
+        else if (n == 1 || (n <= 4 && idle)) launch_few<1, true, 4>(g, stream);
+        else if (n <= 8 && idle) launch_few<1, true, 2>(g, stream);
+        else if (n <= 16) launch_few<1, true>(g, stream);
+        else if (n <= 32) launch_few<2, true>(g, stream);
+        else launch_few<4, true>(g, stream);
+    } else if (tiles) {
+        if (busiest(64) * 20 <= busiest(32) * 23) launch_tiled<64>(g, stream);
+        else launch_tiled<32>(g, stream);
+    } else if ((busiest(64) + 1000) * 20 <= busiest(32) * 24) {
+        if (vec) launch_ragged<64, true>(g, stream);
+        else launch_ragged<64, false>(g, stream);
     } else {
-        launch_tiled<32>(g, stream);
+        if (vec) launch_ragged<32, true>(g, stream);
+        else launch_ragged<32, false>(g, stream);
     }
     PL_CHECK_LAUNCH("gemm_f32");
     return 0;

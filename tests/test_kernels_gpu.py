@@ -1986,3 +1986,32 @@ def test_every_tile_of_the_32_bit_product_has_its_workgroup(N, rows):
             kernels.gemm_heads(x, kernels.head_weights(w), got)
         want = (x.double().transpose(0, 1) @ w.double().transpose(1, 2).contiguous()).transpose(0, 1)
         assert rel(got, want) < 4 * math.sqrt(K / 16 + 16) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("N,K", [(1, 3), (5, 33), (33, 66), (64, 100), (65, 1000), (100, 1030), (300, 130), (1100, 1027), (4100, 68)])
+def test_the_32_bit_product_of_many_rows_of_any_k(N, K):
+    """K no multiple of 64 or of 4, rows that are not aligned, apart from each other and a head at a time: on both sides of every rule
+    that chooses the kernel the same bits for a row whatever else is in the batch; 64-bit arithmetic within a factor of four of what chains of
+    K / 16 and 16 parts can be off; infinities and NaNs stay in their rows and columns."""
+    from paged_llm_rs_amd import kernels
+
+    most = 1500 if N * K < 200_000 else 700
+    w = torch.randn(N, K, device=DEV)
+    apart = torch.full((most, K + 5), math.nan, device=DEV)           # (rows further apart than their values, unaligned)
+    x = apart[:, 1:K + 1]
+    x.copy_(torch.randn(most, K, device=DEV))
+    full = torch.full((most, N), math.nan, device=DEV)
+    kernels.gemm_heads(x.unflatten(1, (1, K)), kernels.head_weights(w[None]), full.unflatten(1, (1, N)))
+    assert rel(full, x.double() @ w.double().T) < 4 * math.sqrt(K / 16 + 16) * 2.0 ** -24
+    for n in (1, 8, 9, 16, 17, 32, 33, 64, 65, 130, 300, most):
+        assert torch.equal(kernels.gemm_plain(x[-n:].contiguous(), w), full[-n:]), f"{n} rows"
+    heads = x[:120].contiguous().view(40, 3, K)
+    both = torch.full((40, 3, N), math.nan, device=DEV)
+    kernels.gemm_heads(heads, kernels.head_weights(w[None].expand(3, N, K)), both)
+    assert torch.equal(both.view(120, N), full[:120])
+    x[1, K // 2], w[N // 2, 0] = math.inf, math.nan
+    y = kernels.gemm_plain(x.contiguous(), w)
+    keep = torch.arange(N, device=DEV) != N // 2
+    assert bool(y[:, N // 2].isnan().all()) and not bool(y[1].isfinite().any())
+    y[1], full[1] = 0, 0
+    assert torch.equal(y[:, keep], full[:, keep])
