@@ -521,11 +521,12 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
     const int va = min(vt * 64 + l32, V - 1), vb = min(vt * 64 + 32 + l32, V - 1);
     float xa[SSD_CHUNK / 2], xb[SSD_CHUNK / 2];
     const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
+    // (every load before the first silu: one behind a branch would be waited for alone)
 #pragma unroll
     for (int k = 0; k < SSD_CHUNK / 2; ++k) {
         const float* x = rows + static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.v_off + h * V;
-        xa[k] = ssd_kv<KIND>(x[va]);
-        xb[k] = two ? ssd_kv<KIND>(x[vb]) : 0.f;
+        xa[k] = x[va];
+        xb[k] = x[vb];
     }
     if (wave == 0) {
         double b, dt;
@@ -550,8 +551,8 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
 #pragma unroll
     for (int k = 0; k < SSD_CHUNK / 2; ++k) {
         const float w = weight[2 * k + half];
-        xa[k] *= w;
-        xb[k] *= w;
+        xa[k] = ssd_kv<KIND>(xa[k]) * w;
+        xb[k] = ssd_kv<KIND>(xb[k]) * w;
     }
     float* U = sa.U + idx * N * V;
     for (int n0 = wave * 32; n0 < N; n0 += 128) {
@@ -559,7 +560,11 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
         float ka[SSD_CHUNK / 2];
 #pragma unroll
         for (int k = 0; k < SSD_CHUNK / 2; ++k)
-            ka[k] = ssd_kv<KIND>(rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n]);
+            ka[k] = rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n];
+        if (KIND == PL_SCAN_LIGHTNING) {
+#pragma unroll
+            for (int k = 0; k < SSD_CHUNK / 2; ++k) ka[k] = ssd_kv<KIND>(ka[k]);
+        }
         if (KIND == PL_SCAN_MLSTM && vt == 0) {
             float sum = 0.f;
 #pragma unroll
@@ -710,7 +715,7 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         x[k] = 0.f;
         if (columns && (k < 16 || ti == 1)) {
             const int u = 8 * (k >> 2) + 4 * half + (k & 3);
-            x[k] = ssd_kv<KIND>(rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc]);
+            x[k] = rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc];
         }
     }
     const float* S0 = sa.Sin + idx * N * V + vc;
@@ -814,6 +819,11 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
     }
     if (!columns) return;
     // ---- the weighted scores times x, and D x ----
+    if (KIND == PL_SCAN_LIGHTNING) {
+#pragma unroll
+        for (int k = 0; k < SSD_CHUNK / 2; ++k)
+            if (k < 16 || ti == 1) x[k] = ssd_kv<KIND>(x[k]);
+    }
     {
         const float* sc = As + (32 * ti + l32) * PA + 4 * half;
 #pragma unroll
