@@ -547,3 +547,43 @@ def test_the_matrix_memory_forgets_hundreds_and_remembers():
         begin += count
     err = (torch.cat(got) - want)[64:].abs().max() / want[64:].abs().max()
     assert float(err) < 50 * 2.0 ** -24, float(err)
+
+
+@pytest.mark.parametrize("kind", ["lightning", "mlstm", "delta"])
+@pytest.mark.parametrize("D,V", [(16, 64), (17, 64), (5, 8)])
+def test_requests_of_a_few_tokens_without_chunks(kind, D, V):
+    """Steps in which no request has enough tokens for chunks: several tokens a request (small states by one wave, others by four) and then
+    one, out of the same slots, against 64 bits."""
+    from paged_llm_rs_amd import kernels
+
+    H, T, cap = 2, [15, 3, 1, 9], 5.0
+    g = torch.Generator().manual_seed(D)
+    G = 1 if kind == "delta" else H
+    q, k = ([torch.randn((t + 2, G, D), generator=g) for t in T] for _ in range(2))
+    v = [torch.randn((t + 2, H, V), generator=g) for t in T]
+    x1, x2 = ([2 * torch.randn((t + 2, H), generator=g) for t in T] for _ in range(2))
+    p1 = 1 - 0.5 * torch.rand((H,), generator=g) if kind == "lightning" else 0.5 * torch.randn((H,), generator=g)
+    p2 = 2 + torch.randn((H,), generator=g)
+    want = [scan_in_64_bits(kind, *(x[i].double() for x in (q, k, v, x1, x2)), p1.double(), p2.double(), cap).reshape(-1, H * V)
+            for i in range(len(T))]
+    floats = kernels.scan_state_floats(kind, H, D, V)
+    state, got, at = torch.zeros((5, (floats + 3) // 4 * 4)).cuda(), [[] for _ in T], [0] * len(T)
+    for counts in (T, [1] * len(T), [1] * len(T)):
+        b = ScanStep(counts, [4, 0, 2, 1], padding=1 if max(counts) == 1 else 2)
+        rows, gates = torch.zeros((b.num_tokens, H * V + 2 * G * D)), torch.zeros((b.num_tokens, 2 * H))
+        r = 0
+        for i, c in enumerate(counts):
+            span = slice(at[i], at[i] + c)
+            rows[r:r + c] = torch.cat([v[i][span].flatten(1), k[i][span].flatten(1), q[i][span].flatten(1)], -1)
+            gates[r:r + c] = torch.cat([x1[i][span], x2[i][span]], -1)
+            r, at[i] = r + c, at[i] + c
+        out = kernels.recurrent_scan(kind, rows.cuda(), H * V + G * D, H * V, 0, state[:, :floats], b, H, G, D, V,
+                                     gates=None if kind == "lightning" else gates.cuda(), g1_off=0, g2_off=H, p1=p1.cuda(),
+                                     p2=None if kind == "lightning" else p2.cuda(), cap=cap, chunked=True).double().cpu()
+        r = 0
+        for i, c in enumerate(counts):
+            got[i].append(out[r:r + c])
+            r += c
+    scale = max(float(w.abs().max()) for w in want)
+    for i, pieces in enumerate(got):
+        assert float((torch.cat(pieces) - want[i]).abs().max()) <= 1e-5 * scale, i
