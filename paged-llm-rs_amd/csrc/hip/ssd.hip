@@ -779,9 +779,10 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         for (int r = 0; r < 16; ++r) As[(32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)) * PA + 32 * tj + l32] = acc[r];
     }
     // ---- S_0^T C_t, times e^(b_t) ----
-    ssd_f32x16 y;
+    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size)
+    ssd_f32x16 y, y2;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) y[r] = 0.f;
+    for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;
     if (columns) {
         const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
         for (int n0 = 0; n0 < Np; n0 += 64) {
@@ -794,12 +795,15 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
                 if (n0 + 8 * q < Np) {
                     const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + n0 + 8 * q);   // (zeros past N)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) y = ssd_mfma(cv[e], now[4 * q + e], y);
+                    for (int e = 0; e < 4; ++e) {
+                        if (q % 2 == 0) y = ssd_mfma(cv[e], now[4 * q + e], y);
+                        else y2 = ssd_mfma(cv[e], now[4 * q + e], y2);
+                    }
                 }
             }
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] *= before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
+        for (int r = 0; r < 16; ++r) y[r] = (y[r] + y2[r]) * before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
     }
     __syncthreads();                                                  // the weighted scores are written
     if (KIND == PL_SCAN_MLSTM) {
@@ -824,6 +828,9 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         for (int k = 0; k < SSD_CHUNK / 2; ++k)
             if (k < 16 || ti == 1) x[k] = ssd_kv<KIND>(x[k]);
     }
+    ssd_f32x16 own;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) own[r] = 0.f;
     {
         const float* sc = As + (32 * ti + l32) * PA + 4 * half;
 #pragma unroll
@@ -831,7 +838,7 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             if (q < 4 || ti == 1) {
                 const ssd_f32x4 av = *reinterpret_cast<const ssd_f32x4*>(sc + 8 * q);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) y = ssd_mfma(av[e], x[4 * q + e], y);
+                for (int e = 0; e < 4; ++e) own = ssd_mfma(av[e], x[4 * q + e], own);
             }
         }
     }
@@ -842,7 +849,7 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         const int t = 32 * ti + 8 * (r >> 2) + 4 * half + (r & 3);
         // (token t's own x is the one this lane holds in the same place of its half of the chunk)
         if (t >= L || v >= V) continue;
-        float o = y[r];
+        float o = y[r] + own[r];
         if (KIND == PL_SCAN_SSD) o += skip * (ti == 0 ? x[r] : x[16 + r]);
         if (KIND == PL_SCAN_MLSTM) o *= below[t];
         out[static_cast<size_t>(t) * (H * V) + v] = o;

@@ -430,7 +430,7 @@ def test_the_recurrences_kernels_in_portions(kind, H, D, V):
         assert (state[:, floats:] == 7.0).all(), "nothing beside the state is touched"
         for i, pieces in got.items():
             err = float((torch.cat(pieces) - want[i]).abs().max()) / scale
-            assert err <= 3e-5, (i, err)
+            assert err <= (3e-5 if kind == "mlstm" else 30 * 2.0 ** -24), (i, err)
 
     run([[(i, t) for i, t in enumerate(T)]], [5, 0, 3, 1, 7, 2])
     run([[(0, 15), (1, 16), (2, 1), (4, 63)], [(0, 64), (2, 1), (1, 48), (5, 2)], [(0, 1), (3, 1), (4, 2), (2, 1)], [(0, 114), (5, 31)]],
