@@ -398,16 +398,19 @@ F32_SEGMENT = 64
 F32_SPLIT_BYTES = 64 << 20
 
 
-def f32_splits(rows: int, live_seqs: int, nq: int, nkv: int, d: int, max_ctx: int) -> bool:
+def f32_splits(rows: int, live_seqs: int, nq: int, nkv: int, d: int, max_ctx: int, window: int = 0, keep: int = 0) -> bool:
     """Whether the 32-bit kernel leaves the segments of every row in memory for a second kernel to fold.  It costs that
-    kernel (some 5 us) and the segments' trip, and it pays where the tiles alone leave compute units without work: a few
-    tokens, whose keys a few workgroups would take in at what a compute unit gets from memory (8 tokens at contexts up to 512,
-    16 heads over 8 of 128: 24 us whole, 18.5 split with its second kernel), or few tiles before more than 1,024 keys."""
+    kernel (some 5 us) and the segments' trip, and it pays where the tiles alone leave compute units without work and the four
+    waves of a tile do not take its segments at once: a few tokens, whose keys a few workgroups would take in at what a compute unit
+    gets from memory (8 tokens at contexts up to 512, 16 heads over 8 of 128: 24 us whole, 18.5 split with its second kernel), or few
+    tiles before more than 1,024 keys.  Under a window what counts is what a tile sees (200 tokens behind 2,000 others, a window
+    of 64, 12 over 12 heads of 96: 45 us split, 18 whole)."""
     group = nq // nkv
     tokens, head_tiles = (16 // group, 1) if group <= 16 else (1, -(-group // 16))
     tiles = min(rows, rows // tokens + live_seqs) * nkv * head_tiles
     segments = -(-max_ctx // F32_SEGMENT)
-    return (tiles < compute_units() and segments > 1 and (rows <= 16 or segments > 16)
+    seen = min(segments, -(-(abs(window) + tokens + keep) // F32_SEGMENT) + 1) if window else segments
+    return (tiles < compute_units() and seen > 4 and (rows <= 16 or seen > 16)
             and rows * nq * segments * (d + 2) * 4 <= F32_SPLIT_BYTES)
 
 
@@ -442,7 +445,7 @@ def paged_attention_f32(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, p
         raise TensorError(f"{live} requests with tokens of {S}")
     sinks, slopes = _head_numbers(sinks, "sinks", nq), _head_numbers(slopes, "distance slopes", nq)
     if split is None:
-        split = f32_splits(n, live, nq, nkv, d, int(max_ctx))
+        split = f32_splits(n, live, nq, nkv, d, int(max_ctx), int(window or 0), more.keep if more is not None else 0)
     part_acc = part_ml = None
     segments = -(-int(max_ctx) // F32_SEGMENT)
     if split:

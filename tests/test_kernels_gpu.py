@@ -2015,3 +2015,16 @@ def test_the_32_bit_product_of_many_rows_of_any_k(N, K):
     assert bool(y[:, N // 2].isnan().all()) and not bool(y[1].isfinite().any())
     y[1], full[1] = 0, 0
     assert torch.equal(y[:, keep], full[:, keep])
+
+
+def test_the_32_bit_attention_folds_in_one_kernel_what_a_window_leaves():
+    """Under a window the choice between the two ways to fold goes by the keys that a tile sees, not by the context; what the
+    second kernel needs room for still goes by the context."""
+    from paged_llm_rs_amd import kernels
+
+    if kernels.compute_units() != 256:
+        pytest.skip("the choices below are for 256 compute units")
+    f = lambda rows, seqs, bound, *more: kernels.f32_splits(rows, seqs, 12, 12, 96, bound, *more)
+    assert f(200, 1, 3072) and not f(200, 1, 3072, 64) and not f(200, 1, 3072, -64) and f(200, 1, 3072, 2000)
+    assert f(8, 8, 1024) and not f(8, 8, 1024, 128) and f(8, 8, 1024, 512) and f(8, 8, 1024, 128, 400) and not f(8, 8, 256)
+    assert not f(200, 1, 1 << 20)
