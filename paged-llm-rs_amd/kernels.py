@@ -844,12 +844,12 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                     slopes: torch.Tensor | None = None, more: AttentionMore | None = None) -> torch.Tensor:
     """Attention for every token of a step.  ``qkv`` rows begin with the rotated queries.
     In 32-bit every row goes to the kernel on the matrix cores' 32-bit instruction, where the head size is a multiple of four up
-    to 256 and the step says which rows each request brings (``q_start``, ``q_len``, ``ctx_len``), and otherwise to the plain one,
+    to 256 and the step says which rows each request brings (``q_start``, ``q_len``, ``ctx_len``, ``max_ctx_len``), and otherwise to the plain one,
     which needs each row's position and request only.  In bfloat16 the long portions go to the tiled kernel and the tokens of short ones
     (decoded tokens among them) to the kernel for single tokens, or, where many query heads share a key
     head, to the tiled kernel with a group's heads as its rows; all read the same pages."""
     if qkv.dtype == torch.float32 and _attention_mode == "kernel" and all(
-            getattr(batch, name, None) is not None for name in ("q_start", "q_len", "ctx_len")) and library().pl_paged_attention_f32_applies(
+            getattr(batch, name, None) is not None for name in ("q_start", "q_len", "ctx_len", "max_ctx_len")) and library().pl_paged_attention_f32_applies(
             qkv.data_ptr(), qkv.shape[1], out.data_ptr(), kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), d):
         return paged_attention_f32(qkv, qkv.shape[1], out, batch.positions, batch.q_start, batch.q_len, batch.ctx_len,
                                    kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, batch.max_ctx_len,

@@ -1839,8 +1839,10 @@ def test_sinks_and_distance_slopes_in_every_attention_kernel(nq, nkv, d, bs, req
         assert rel(out[i].float(), plain[i]) < 1.5e-2, f"token {i} (request {seq_of[i]}, position {positions[i]})"
 
 
-def test_32_bit_attention_over_a_descriptor_without_the_requests_rows():
-    """A descriptor that holds each row's position and request only, as the plain kernel reads them, is served by that kernel."""
+@pytest.mark.parametrize("holds", ["positions", "all but the longest context"])
+def test_32_bit_attention_over_a_descriptor_without_the_requests_rows(holds):
+    """A descriptor that holds each row's position and request only, as the plain kernel reads them, is served by that kernel, and so
+    is one that does not say how long contexts are."""
     from types import SimpleNamespace
 
     from paged_llm_rs_amd import kernels
@@ -1853,7 +1855,8 @@ def test_32_bit_attention_over_a_descriptor_without_the_requests_rows():
     n, stride = positions.numel(), (nq + 2 * nkv) * d
     q = torch.randn(n, stride, device=DEV)
     kv = SimpleNamespace(block_table=bt, block_size=bs, k_pool=k_pool, v_pool=v_pool)
-    batch = SimpleNamespace(positions=positions, seq_of=seq_of, num_tokens=n, max_ctx_len=1024)
+    rows = dict(q_start=i32([0, 3, 23]), q_len=i32([t for _, t in requests]), ctx_len=i32([c for c, _ in requests]))
+    batch = SimpleNamespace(positions=positions, seq_of=seq_of, num_tokens=n, **(dict(max_ctx_len=1024) if holds == "positions" else rows))
     out, plain = (torch.full((n, nq * d), 7.0, device=DEV) for _ in range(2))
     kernels.paged_attention(q, out, batch, kv, nq, nkv, d, d ** -0.5)
     kernels.paged_attention_plain(q, stride, plain, positions, seq_of, bt, bs, k_pool, v_pool, nq, nkv, d, d ** -0.5)
