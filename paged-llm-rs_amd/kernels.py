@@ -441,8 +441,10 @@ def paged_attention_f32(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, p
         if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % block_size != 0:
             raise TensorError(f"{what} has shape {tuple(pool.shape)}, expected [pages*{block_size}, {nkv * d}]")
     live = S if live_seqs is None else int(live_seqs)
-    if not 0 < live <= S:
+    if not 0 <= live <= S:
         raise TensorError(f"{live} requests with tokens of {S}")
+    if n == 0 or live == 0:
+        return out
     sinks, slopes = _head_numbers(sinks, "sinks", nq), _head_numbers(slopes, "distance slopes", nq)
     if split is None:
         split = f32_splits(n, live, nq, nkv, d, int(max_ctx), int(window or 0), more.keep if more is not None else 0)

@@ -2031,3 +2031,20 @@ def test_the_32_bit_attention_folds_in_one_kernel_what_a_window_leaves():
     assert f(200, 1, 3072) and not f(200, 1, 3072, 64) and not f(200, 1, 3072, -64) and f(200, 1, 3072, 2000)
     assert f(8, 8, 1024) and not f(8, 8, 1024, 128) and f(8, 8, 1024, 512) and f(8, 8, 1024, 128, 400) and not f(8, 8, 256)
     assert not f(200, 1, 1 << 20)
+
+
+@pytest.mark.parametrize("requests", [0, 2])
+def test_32_bit_attention_of_a_step_without_tokens(requests):
+    """No rows, with or without requests that bring none: nothing to do, and no error."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    nq, nkv, d, bs = 4, 2, 64, 16
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=DEV)
+    pool = torch.zeros(bs, nkv * d, device=DEV)
+    kv = SimpleNamespace(block_table=i32(requests, 4), block_size=bs, k_pool=pool, v_pool=pool)
+    batch = SimpleNamespace(positions=i32(0), seq_of=i32(0), q_start=i32(requests), q_len=i32(requests), ctx_len=i32(requests),
+                            num_tokens=0, max_ctx_len=64)
+    out = torch.empty(0, nq * d, device=DEV)
+    assert kernels.paged_attention(torch.empty(0, (nq + 2 * nkv) * d, device=DEV), out, batch, kv, nq, nkv, d, d ** -0.5) is out
