@@ -213,7 +213,7 @@ extern "C" int pl_recurrent_scan(int kind, const float* qkv, int qkv_stride, int
                                  const float* p1, const float* p2, const float* p3, float cap,
                                  float* state, long state_stride, int s_off, int n_off, int m_off,
                                  float* out, const int* q_start, const int* q_len, const int* state_slots,
-                                 int seqs, int H, int G, int D, int V, int below, int several, hipStream_t stream) {
+                                 int seqs, int H, int G, int D, int V, int below, hipStream_t stream) {
     PL_REQUIRE(kind >= 0 && kind <= PL_SCAN_RETENTION, "recurrent_scan: kind %d", kind);
     PL_REQUIRE(kind != PL_SCAN_SSD || p3 != nullptr, "recurrent_scan: what v counts in its own read-out is missing");
     PL_REQUIRE(H > 0 && G > 0 && H % G == 0, "recurrent_scan: %d heads over %d heads of q and k", H, G);
@@ -226,11 +226,12 @@ extern "C" int pl_recurrent_scan(int kind, const float* qkv, int qkv_stride, int
     if (seqs == 0) return 0;
     ScanArgs a{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, p1, p2, p3, cap,
                state, state_stride, s_off, n_off, m_off, out, q_start, q_len, state_slots, H, G, D, V, below};
-    // The scan kernel is left with states whose columns are no whole aligned quads, and with requests of several tokens whose
-    // states have up to 16 rows: a wave goes through those faster than four waves meet, three times a token for delta (two heads
-    // of 16 by 64, four waves / one: 15 tokens, lightning 15.7 / 13.0 us, mlstm 23.3 / 18.3, delta 26.2 / 15.7; one token 4.9 / 6.5, 5.6 /
-    // 7.4, 5.7 / 7.7; two heads of 40, one wave, 15 tokens 26.1, 30.3, 31.4).
-    if (!(several && D <= 16) && pl_state_step(kind, a, seqs, stream)) {
+    // The scan kernel is left with states whose columns are no whole aligned quads, and with states of up to 16 rows: a wave goes
+    // through several tokens of those faster than four waves meet, three times a token for delta (two heads of 16 by 64, four waves /
+    // one: 15 tokens, lightning 15.7 / 13.0 us, mlstm 23.3 / 18.3, delta 26.2 / 15.7; one token 4.9 / 6.5, 5.6 / 7.4, 5.7 / 7.7; two heads of
+    // 40, one wave, 15 tokens 26.1, 30.3, 31.4).  The state's shape alone decides: the two sum in different orders, and a token's bits
+    // depend neither on how its request was cut into steps nor on what the others bring.
+    if (D > 16 && pl_state_step(kind, a, seqs, stream)) {
         PL_CHECK_LAUNCH("recurrent_scan (step)");
         return 0;
     }

@@ -420,8 +420,7 @@ __global__ __launch_bounds__(256) void state_step_kernel(ScanArgs a) {
 template <int KIND>
 static void launch_step(const ScanArgs& a, int seqs, hipStream_t stream) {
     const dim3 grid(pl_ceil_div(a.V, 64), a.H, seqs);
-    if (a.D <= 16) state_step_kernel<1, KIND><<<grid, 256, 0, stream>>>(a);
-    else if (a.D <= 32) state_step_kernel<2, KIND><<<grid, 256, 0, stream>>>(a);
+    if (a.D <= 32) state_step_kernel<2, KIND><<<grid, 256, 0, stream>>>(a);
     else if (a.D <= 64) state_step_kernel<4, KIND><<<grid, 256, 0, stream>>>(a);
     else if (a.D <= 128) state_step_kernel<8, KIND><<<grid, 256, 0, stream>>>(a);
     else state_step_kernel<16, KIND><<<grid, 256, 0, stream>>>(a);

@@ -66,7 +66,7 @@ def _signatures(lib) -> None:
         "pl_paged_attention_grouped": [p, i, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, f, i, i, p, p, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_grouped_applies": [i, i, i, i],
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
-                              i, i, i, i, i, i, i, p],
+                              i, i, i, i, i, i, p],
         "pl_recurrent_chunked": [i, p, i, i, i, i, p, i, i, i, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
                                  i, i, i, i, i, i, i, p, p, p, p, p, p],
         "pl_ssd_step": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p],
@@ -1386,10 +1386,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
               state.data_ptr(), stride, 0, hdv, hdv + heads * tiles * dim, out.data_ptr(), batch.q_start.data_ptr(),
               batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
     if not chunked or _brings_short_requests(batch):
-        # (beside portions in chunks most short requests bring one token; the step does not say)
-        several = 0 if chunked or batch.max_q_len <= 1 else 1
-        _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0,
-                                           several, _stream()))
+        _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
     if chunked and kind == "delta":
         chunks = (n // SSD_CHUNK + batch.num_seqs + 1) * heads
         f32 = dict(dtype=torch.float32, device=qkv.device)
@@ -1435,7 +1432,7 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
             _check(lib.pl_recurrent_scan(SCAN_KINDS["ssd"], qkv.data_ptr(), qkv.shape[1], q_off, k_off, v_off, gates.data_ptr(),
                                          gates.shape[1], g_off, g_off, *constants, 0.0, state.data_ptr(), stride, 0, 0, 0,
                                          out.data_ptr(), batch.q_start.data_ptr(), batch.q_len.data_ptr(),
-                                         batch.state_slots.data_ptr(), batch.num_seqs, H, G, N, V, below, 0, stream))
+                                         batch.state_slots.data_ptr(), batch.num_seqs, H, G, N, V, below, stream))
     if chunked:
         chunks = n // SSD_CHUNK + batch.num_seqs + 1
         f32 = dict(dtype=torch.float32, device=qkv.device)
@@ -1494,7 +1491,7 @@ def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state
                                      stride, out.data_ptr(), *step, heads, dim, vdim, below, stream))
     elif by_token:
         _check(lib.pl_recurrent_scan(SCAN_KINDS["retention"], *at, 0, 0, 0, 0, decay.data_ptr(), 0, 0, 0.0, state.data_ptr(), stride,
-                                     0, 0, 0, out.data_ptr(), *step, heads, heads, dim, vdim, below, 0, stream))
+                                     0, 0, 0, out.data_ptr(), *step, heads, heads, dim, vdim, below, stream))
     if chunked:
         chunks = n // SSD_CHUNK + batch.num_seqs + 1
         f32 = dict(dtype=torch.float32, device=rows.device)

@@ -552,7 +552,7 @@ def test_the_matrix_memory_forgets_hundreds_and_remembers():
 @pytest.mark.parametrize("kind", ["lightning", "mlstm", "delta"])
 @pytest.mark.parametrize("D,V", [(16, 64), (17, 64), (5, 8)])
 def test_requests_of_a_few_tokens_without_chunks(kind, D, V):
-    """Steps in which no request has enough tokens for chunks: several tokens a request (small states by one wave, others by four) and then
+    """Steps in which no request has enough tokens for chunks: several tokens a request and then
     one, out of the same slots, against 64 bits."""
     from paged_llm_rs_amd import kernels
 
@@ -587,3 +587,32 @@ def test_requests_of_a_few_tokens_without_chunks(kind, D, V):
     scale = max(float(w.abs().max()) for w in want)
     for i, pieces in enumerate(got):
         assert float((torch.cat(pieces) - want[i]).abs().max()) <= 1e-5 * scale, i
+
+
+@pytest.mark.parametrize("kind", ["lightning", "mlstm", "delta"])
+@pytest.mark.parametrize("D,V", [(16, 64), (17, 64), (5, 8), (64, 10)])
+def test_token_by_token_scans_give_the_same_bits_however_the_tokens_are_cut(kind, D, V):
+    """A request's tokens in one step, beside requests of several and of single tokens, and one step a token, alone."""
+    from paged_llm_rs_amd import kernels
+
+    H, counts = 2, [6, 1, 9]
+    g = torch.Generator().manual_seed(D)
+    rows, gates = torch.randn((sum(counts) + 2, 3 * H * max(D, V)), generator=g).cuda(), torch.randn((sum(counts) + 2, 2 * H), generator=g).cuda()
+    p1, p2 = (0.5 + 0.4 * torch.rand((H,), generator=g)).cuda(), torch.randn((H,), generator=g).cuda()
+    floats = kernels.scan_state_floats(kind, H, D, V)
+
+    def run(state, rows, gates, counts, slots):
+        step = ScanStep(counts, slots, padding=len(rows) - sum(counts))
+        return kernels.recurrent_scan(kind, rows, 0, H * max(D, V), 2 * H * max(D, V), state[:, :floats], step, H, H, D, V,
+                                      gates=None if kind == "lightning" else gates, g1_off=0, g2_off=H, p1=p1,
+                                      p2=None if kind == "lightning" else p2, cap=5.0)
+
+    empty = lambda: torch.zeros((3, (floats + 3) // 4 * 4)).cuda()
+    together, state = empty(), empty()
+    want, begin = run(together, rows, gates, counts, [0, 1, 2]), 0
+    for slot, count in enumerate(counts):
+        for t in range(begin, begin + count):
+            at = [t, len(rows) - 1]                                 # (the token and a row of padding)
+            assert torch.equal(run(state, rows[at], gates[at], [1], [slot])[0], want[t]), (slot, t)
+        begin += count
+    assert torch.equal(state[:, :floats], together[:, :floats])
