@@ -9,6 +9,7 @@ GPU, these functions raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_float, c_int, c_void_p
 
 import torch
@@ -113,6 +114,7 @@ def library():
     if _lib is None:
         lib = build.load("hip")
         _signatures(lib)
+        lib.decode_meets = lib.pl_paged_attention_decode_meets()       # (a constant of the library that every layer asks for)
         _lib = lib
     return _lib
 
@@ -511,9 +513,15 @@ def _has_arrivals(batch) -> bool:
     return getattr(batch, "has_arrivals", False)
 
 
+def _says_rows(batch) -> bool:
+    """Whether the step says which rows each request brings and how long contexts are."""
+    return (getattr(batch, "q_start", None) is not None and getattr(batch, "q_len", None) is not None
+            and getattr(batch, "ctx_len", None) is not None and getattr(batch, "max_ctx_len", None) is not None)
+
+
 def _arrivals(batch, nq: int, splits: int):
     """The step's room for the arrivals of its shares' workgroups, where they count themselves."""
-    if not 1 < splits <= library().pl_paged_attention_decode_meets() or not _has_arrivals(batch):
+    if not 1 < splits <= library().decode_meets or not _has_arrivals(batch):
         return None
     return batch.arrivals(nq)
 
@@ -545,6 +553,7 @@ DECODE_WORKGROUP_US = 0.4
 DECODE_MEET_US, DECODE_MERGE_US, DECODE_MERGE_MANY_US = 4.0, 5.4, 9.0
 
 
+@functools.lru_cache(maxsize=512)           # (every layer of a step asks the same)
 def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128, meets: bool = True) -> int:
     """Into how many stretches the context is cut for the single-token kernel, each with at least 128 keys
     (two rounds of loads).  ``meets``: whether the step has counters for the shares to meet in the kernel.
@@ -571,7 +580,7 @@ def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128, me
             return 1
         return max(1, min((target + base - 1) // base, most))
     units = compute_units()
-    meeting = library().pl_paged_attention_decode_meets() if meets else 1
+    meeting = library().decode_meets if meets else 1
     best, best_us = 1, None
     for splits in range(1, most + 1):
         busiest = -(-base * splits // units)                      # workgroups on one compute unit
@@ -850,8 +859,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
     which needs each row's position and request only.  In bfloat16 the long portions go to the tiled kernel and the tokens of short ones
     (decoded tokens among them) to the kernel for single tokens, or, where many query heads share a key
     head, to the tiled kernel with a group's heads as its rows; all read the same pages."""
-    if qkv.dtype == torch.float32 and _attention_mode == "kernel" and all(
-            getattr(batch, name, None) is not None for name in ("q_start", "q_len", "ctx_len", "max_ctx_len")) and library().pl_paged_attention_f32_applies(
+    if qkv.dtype == torch.float32 and _attention_mode == "kernel" and _says_rows(batch) and library().pl_paged_attention_f32_applies(
             qkv.data_ptr(), qkv.shape[1], out.data_ptr(), kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), d):
         return paged_attention_f32(qkv, qkv.shape[1], out, batch.positions, batch.q_start, batch.q_len, batch.ctx_len,
                                    kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, batch.max_ctx_len,
