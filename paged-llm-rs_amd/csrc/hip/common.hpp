@@ -77,7 +77,8 @@ __device__ __forceinline__ float block_sum(float v, float* scratch /* >= 16 floa
 // (pl_arrive); the one that finds all others there before it reads their shares with pl_shared and sets the counter
 // back to zero for the next launch.  Nobody waits for anybody.  Every access is a relaxed atomic of device scope, which goes
 // past the XCD's L2; what a fence of device scope would do on top, write back and drop a whole L2, costs more than a
-// kernel (256 workgroups 9.2 us, against 1.4 us for publishing and reading this way and 4.1 us for a kernel that merges).
+// kernel (a probe of 256 workgroups, 1 KB each: 9.2 us with it, 1.4 us this way, 4.1 us for a kernel that merges).  In the
+// single-token attention it costs 2.2 us of 11.2 (one token, eight shares) to 2.7 of 27.7 (eight tokens of 32 heads), the merging kernel 4.4 to 4.8.
 __device__ __forceinline__ void pl_share(float* to, float v) { __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float pl_shared(const float* from) { return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 // The calling wave's shares are where every workgroup finds them.

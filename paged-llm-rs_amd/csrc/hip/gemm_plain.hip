@@ -1,7 +1,7 @@
 // y[n, N] = x[n, K] . w[N, K]^T with 32-bit products and sums whatever the operands are: 32-bit ones go to gemm_f32.hip,
 // bfloat16 ones (the fallback for shapes that the fast kernels refuse) are multiplied here on the vector units.
 //
-// Each output element is the sum over k in ascending order, whatever n is, so a row's result does not depend on what
+// Each output element here is the sum over k in ascending order, whatever n is, so a row's result does not depend on what
 // else is in the batch.
 #include "common.hpp"
 

@@ -778,7 +778,8 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
         for (int r = 0; r < 16; ++r) As[(32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)) * PA + 32 * tj + l32] = acc[r];
     }
     // ---- S_0^T C_t, times e^(b_t) ----
-    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size)
+    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size.  Linear attention
+    // with heads of 256, against 64 bits: 1.2e-7 to 1.5e-7; everything in one chain 1.5e-7 to 2.5e-7)
     ssd_f32x16 y, y2;
 #pragma unroll
     for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;

@@ -1678,7 +1678,7 @@ def gemm_heads(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Ten
     """A product a head: out[t, h, :N] = x[t, h, :K] . W[h]^T with ``w = head_weights(W)``, W [heads, N, K].  ``x`` [n, heads, >= K] and ``out``
     [n, heads, >= N] may be views whose rows and heads lie further apart than their own sizes (the last axis
     contiguous); a view's values behind K or N are neither read nor written.  In 32-bit by the 32-bit product
-    (sums in ascending k: the true 32-bit path); in bfloat16 the library's batched product on the matrix cores."""
+    (at most 16 parts of K, one chain of the matrix cores' 32-bit instruction each, added in ascending order); in bfloat16 the library's batched product on the matrix cores."""
     _need(w, "weights a head")
     heads, N, K = w.shape if w.dtype == torch.float32 else (w.shape[0], w.shape[2], w.shape[1])
     n = x.shape[0]
