@@ -229,7 +229,8 @@ extern "C" int pl_recurrent_scan(int kind, const float* qkv, int qkv_stride, int
     // The scan kernel is left with states whose columns are no whole aligned quads, and with states of up to 16 rows: a wave goes
     // through several tokens of those faster than four waves meet, three times a token for delta (two heads of 16 by 64, four waves /
     // one: 15 tokens, lightning 15.7 / 13.0 us, mlstm 23.3 / 18.3, delta 26.2 / 15.7; one token 4.9 / 6.5, 5.6 / 7.4, 5.7 / 7.7; two heads of
-    // 40, one wave, 15 tokens 26.1, 30.3, 31.4).  The state's shape alone decides: the two sum in different orders, and a token's bits
+    // 40, one wave, 15 tokens 26.1, 30.3, 31.4; just above the line, two heads of 17 by 64, delta, 15 tokens 25.4 / 21.2, 5 and 3 tokens 10.4 / 11.4, one
+    // 4.5 / 7.6).  The state's shape alone decides: the two sum in different orders, and a token's bits
     // depend neither on how its request was cut into steps nor on what the others bring.
     if (D > 16 && pl_state_step(kind, a, seqs, stream)) {
         PL_CHECK_LAUNCH("recurrent_scan (step)");

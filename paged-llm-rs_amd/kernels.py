@@ -405,7 +405,8 @@ def f32_splits(rows: int, live_seqs: int, nq: int, nkv: int, d: int, max_ctx: in
     kernel (some 5 us) and the segments' trip, and it pays where the tiles alone leave compute units without work and the four
     waves of a tile do not take its segments at once: a few tokens, whose keys a few workgroups would take in at what a compute unit
     gets from memory (8 tokens at contexts up to 512, 16 heads over 8 of 128: 24 us whole, 18.5 split with its second kernel), or few
-    tiles before more than 1,024 keys.  Under a window what counts is what a tile sees (200 tokens behind 2,000 others, a window
+    tiles before more than 1,024 keys.  (A bound is all that is known, and contexts far below one of 1,024 pay for it, one token of 16 heads over 8
+    of 128 / 12 over 12 of 96: at 30 keys 15.5 / 18.9 us split, 13.9 / 16.9 whole, 15.7 / 14.8 by the plain kernel; at 500 18.8 / 21.1, 23.8 / 27.8, 174 / 170.)  Under a window what counts is what a tile sees (200 tokens behind 2,000 others, a window
     of 64, 12 over 12 heads of 96: 45 us split, 18 whole)."""
     group = nq // nkv
     tokens, head_tiles = (16 // group, 1) if group <= 16 else (1, -(-group // 16))
