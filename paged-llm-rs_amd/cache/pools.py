@@ -10,6 +10,7 @@ from dataclasses import dataclass
 
 import torch
 
+from .. import kernels
 from ..errors import ConfigError
 from .layout import CacheLayout
 from .manager import CacheManager, GroupGeometry
@@ -53,6 +54,7 @@ class PagedCache:
             layer: torch.zeros((max_seqs, *spec.shape), dtype=spec.dtype, device=self.device)
             for layer, spec in layout.states.items()
         }
+        self._slot_table = None
 
     @property
     def bytes(self) -> int:
@@ -75,5 +77,18 @@ class PagedCache:
 
     def clear_state_slot(self, slot: int) -> None:
         """A slot is cleared before a new request uses it."""
-        for state in self._states.values():
-            state[slot].zero_()
+        self.clear_state_slots([slot])
+
+    def clear_state_slots(self, slots) -> None:
+        """The slots of all requests that begin with a step, over all layers in one launch."""
+        slots = list(slots)
+        if not slots or not self._states:
+            return
+        if self.device.type != "cuda":
+            for slot in slots:
+                for state in self._states.values():
+                    state[slot].zero_()
+            return
+        if self._slot_table is None:
+            self._slot_table = kernels.SlotTable(self._states.values())
+        kernels.clear_slots(self._slot_table, slots)

@@ -57,12 +57,17 @@ def run_step(model, cache, entries, check_start: bool = True, pad_to: int | None
     batch = build_batch(entries, cache.manager, len(cache.layout.groups), model.spec.vocab_size,
                         model.spec.max_positions, model.device, check_start=check_start, pad_to=pad_to,
                         short_bounds=short_bounds)
-    for e in entries:
-        if e.fresh_state and e.state_slot >= 0:
-            cache.clear_state_slot(e.state_slot)
+    clear_fresh_slots(cache, entries)
     if trace is not None:
         return model.forward(batch, cache, trace=trace)
     return model.forward(batch, cache)
+
+
+def clear_fresh_slots(cache, entries) -> None:
+    """The state slots of the requests that begin with this step."""
+    fresh = [e.state_slot for e in entries if e.fresh_state and e.state_slot >= 0]
+    if fresh:
+        cache.clear_state_slots(fresh)
 
 
 def commit_step(cache, entries) -> None:
@@ -392,9 +397,7 @@ class StepRunner:
                 self._shapes.pop(next(iter(self._shapes)))
             self.eager_steps += 1
             return StepOutput(run_step(self.model, self.cache, entries, pad_to=rows, short_bounds=short_bounds))
-        for e in entries:
-            if e.fresh_state and e.state_slot >= 0:
-                self.cache.clear_state_slot(e.state_slot)
+        clear_fresh_slots(self.cache, entries)
         if graph is not None:
             try:
                 out = graph.run(entries)
@@ -443,9 +446,7 @@ class StepRunner:
             raise ConfigError("a request appears twice in one step")
         if fed and max(e.fed_row for e in entries) >= self._feedable:
             raise CannotFeed(f"the step before chose {self._feedable} tokens")
-        for e in entries:
-            if e.fresh_state and e.state_slot >= 0:
-                self.cache.clear_state_slot(e.state_slot)
+        clear_fresh_slots(self.cache, entries)
         cap = _bucket(len(entries))
         graph = self._graphs.get(cap)
         if graph is not None:

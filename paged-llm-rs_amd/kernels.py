@@ -79,6 +79,7 @@ def _signatures(lib) -> None:
         "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i,
                              p, p, p, p, p, p, p],
         "pl_short_conv": [p, i, i, i, p, i, p, ctypes.c_long, i, p, p, p, p, p, i, p, i, i, p],
+        "pl_clear_slots": [p, i, ctypes.c_longlong, p, i, p],
         "pl_conv_history": [p, i, i, i, i, p, ctypes.c_long, i, p, p, p, i, p],
         "pl_gated_group_norm": [p, i, i, i, p, i, f, p, i, i, i, i, p, i, p],
         "pl_conv_qk_prepare": [p, i, i, p, i, p, ctypes.c_long, i, p, p, f, p, i, p, p, p, p, p, i, i, p, p, p, i,
@@ -1558,6 +1559,33 @@ def conv_history(rows: torch.Tensor, off: int, weight: torch.Tensor, history: to
     _check(library().pl_conv_history(rows.data_ptr(), rows.shape[1], off, channels, taps, history.data_ptr(), stride, 0,
                                      batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.state_slots.data_ptr(),
                                      batch.num_seqs, _stream()))
+
+
+class SlotTable:
+    """Where the slots of every layer's state tensor [slots, ...] lie on the device, for ``clear_slots``: made once, for
+    tensors that live as long as it does (it holds them)."""
+
+    def __init__(self, states):
+        self.states = list(states)
+        for t in self.states:
+            _need(t, "a layer's state")
+        sizes = [t[0].numel() * t.element_size() if t.shape[0] else 0 for t in self.states]
+        self.slots = min([t.shape[0] for t in self.states], default=0)
+        self.largest = max(sizes, default=0)
+        rows = [[t.data_ptr(), size] for t, size in zip(self.states, sizes)]
+        self.table = torch.tensor(rows, dtype=torch.int64, device=self.states[0].device) if rows else None
+
+
+def clear_slots(table: SlotTable, slots) -> None:
+    """Zeros in the given slots of every layer's state, in one launch."""
+    slots = list(slots)
+    for slot in slots:
+        if not 0 <= slot < table.slots:
+            raise IndexError(f"state slot {slot} of {table.slots}")
+    if table.table is None or not slots:
+        return
+    _check(library().pl_clear_slots(table.table.data_ptr(), len(table.states), table.largest, (c_int * len(slots))(*slots), len(slots),
+                                    _stream()))
 
 
 GATES = {None: -1, "sigmoid": 0, "silu": 1}

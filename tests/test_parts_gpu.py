@@ -1314,3 +1314,22 @@ def test_a_context_of_thousands_of_tokens_in_portions_and_decoded(model_dirs, na
     assert len(got) >= 2 * 5 + 40 + 40
     worst, where = ru.worst_error(got, want)
     assert worst <= (1e-5 if dtype == "float32" else 2e-2), f"{worst:.3e} at {where}"
+
+
+# --- state slots of requests that begin --------------------------------------------------------------------------
+
+@pytest.mark.parametrize("shapes", [[(3,), (1024,), (7, 5)], [(16384,)], [(4,), (70001,)]])
+@pytest.mark.parametrize("slots", [[0], [68, 3, 5], list(range(1, 67))])
+def test_clearing_state_slots_touches_these_slots_of_every_layer_only(shapes, slots):
+    """One launch clears the slots of all layers: sizes that are and are not whole groups of 16 bytes, more slots than a
+    launch carries; the slots beside them keep every value."""
+    from paged_llm_rs_amd import kernels
+
+    states = [torch.randn((69, *shape), device=DEV) for shape in shapes]
+    before = [t.clone() for t in states]
+    kernels.clear_slots(kernels.SlotTable(states), slots)
+    for t, b in zip(states, before):
+        b[slots] = 0.0
+        assert torch.equal(t, b)
+    with pytest.raises(IndexError):
+        kernels.clear_slots(kernels.SlotTable(states), [69])
