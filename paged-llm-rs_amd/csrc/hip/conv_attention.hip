@@ -12,7 +12,7 @@ struct ConvQkArgs {
     int stride, off;
     const float* conv_w;      // [taps, H*D + G*D + G*V]: a tap's filter values of all channels side by side
     int taps;
-    const float* state;       // [slots, state_stride], the history at hist_off: [taps - 1][channels]
+    float* state;             // [slots, state_stride], the history at hist_off: [taps - 1][channels]
     long state_stride;
     int hist_off;
     const float* q_gain;      // [D]
@@ -32,7 +32,101 @@ struct ConvQkArgs {
     int H, G, D, V, Dp;
 };
 
-// Few tokens (decode steps): a wave a token and head, all of them at once.
+// A step of one token a request: a wave a token and head, all of them at once.  The wave that convolves a request's channels is the only
+// one that reads their history, and moves it on as well.  Bound by its chain of trips (position, request, slot, history): everything
+// that does not wait for the slot is asked for in front of it, the taps together (TAPS known; otherwise up to 16), and the angles
+// are worked out meanwhile.  Two tokens of 16 over 8 heads of 128, four taps: 4.0 us, and 7.7 with the taps one by one, beside a launch of
+// 3.8 for the history.
+template <typename T, int NI, int TAPS>
+__global__ __launch_bounds__(64) void conv_qk_prepare_single_kernel(ConvQkArgs a) {
+    __shared__ float head[64 * NI];
+    constexpr int MOST = TAPS > 0 ? TAPS : 16;
+    const int t = blockIdx.x, which = blockIdx.y, lane = threadIdx.x;
+    const int pos = a.positions[t];
+    const int s = a.seq_of[t];
+    if (pos < 0) return;
+    const int H = a.H, G = a.G, D = a.D, V = a.V, Dp = a.Dp;
+    const int channels = H * D + G * D + G * V, taps = TAPS > 0 ? TAPS : a.taps;
+    const int kind = which < H ? 0 : (which < H + G ? 1 : 2);               // a query head, a key head or a value head
+    const int index = kind == 0 ? which : (kind == 1 ? which - H : which - H - G);
+    const int width = kind == 2 ? V : D;
+    const int c0 = kind == 0 ? index * D : (kind == 1 ? H * D + index * D : H * D + G * D + index * V);
+    const int half = a.rot / 2;
+    const int slot = a.state_slots[s];
+    const int page = kind == 0 ? 0 : a.block_table[static_cast<size_t>(s) * a.max_blocks + pos / a.block_size];
+    const float* gains = kind == 0 ? a.q_gain : a.k_gain;
+    float u[MOST][NI], w[MOST][NI], gain[NI], turn[NI];
+    int at[NI];                         // (past the head's end: its last value again, which is cleared)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int e = lane + 64 * i;
+        at[i] = c0 + min(e, width - 1);
+        const float now = a.rows[static_cast<size_t>(t) * a.stride + a.off + at[i]];
+#pragma unroll
+        for (int j = 0; j < MOST; ++j)
+            if (j < taps) {
+                w[j][i] = a.conv_w[j * channels + at[i]];
+                if (j == taps - 1) u[j][i] = now;
+            }
+        gain[i] = kind != 2 ? gains[min(e, width - 1)] : 0.f;
+        turn[i] = kind != 2 && e < a.rot ? a.freq[e < half ? e : e - half] : 0.f;
+    }
+    if (slot < 0) return;
+    float* hist = a.state + static_cast<size_t>(slot) * a.state_stride + a.hist_off;
+#pragma unroll
+    for (int j = 0; j + 1 < MOST; ++j)
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+            if (j < taps - 1) u[j][i] = hist[static_cast<size_t>(j) * channels + at[i]];
+    float cs[NI], sn[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        cs[i] = 1.f;
+        sn[i] = 0.f;
+        if (kind != 2 && lane + 64 * i < a.rot) sincosf(static_cast<float>(pos) * turn[i], &sn[i], &cs[i]);
+    }
+    float x[NI], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        x[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < MOST; ++j)
+            if (j < taps) x[i] += w[j][i] * u[j][i];
+        if (lane + 64 * i < width) {
+#pragma unroll
+            for (int j = 0; j + 1 < MOST; ++j)
+                if (j < taps - 1) hist[static_cast<size_t>(j) * channels + at[i]] = u[j + 1][i];
+        } else {
+            x[i] = 0.f;
+        }
+        ss += x[i] * x[i];
+    }
+    if (kind != 2) {
+        ss = wave_sum(ss);
+        const float inv = 1.f / sqrtf(ss / static_cast<float>(D) + a.eps);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) x[i] = x[i] * inv * gain[i];
+        if (a.rot > 0) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) head[lane + 64 * i] = x[i];
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const int e = lane + 64 * i;
+                if (e < a.rot) x[i] = e < half ? x[i] * cs[i] - head[e + half] * sn[i] : x[i] * cs[i] + head[e - half] * sn[i];
+            }
+        }
+    }
+    if (page < 0) return;
+    const size_t row = static_cast<size_t>(page) * a.block_size + pos % a.block_size;
+    T* dst = kind == 0 ? static_cast<T*>(a.q_out) + (static_cast<size_t>(t) * H + index) * Dp
+                       : static_cast<T*>(kind == 1 ? a.k_pool : a.v_pool) + (row * G + index) * Dp;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+        if (lane + 64 * i < Dp) dst[lane + 64 * i] = from_float<T>(x[i]);
+}
+
+// Few tokens of portions: a wave a token and head.
 template <typename T>
 __global__ __launch_bounds__(64) void conv_qk_prepare_heads_kernel(ConvQkArgs a) {
     __shared__ float head[256];
@@ -216,13 +310,27 @@ static void launch_conv_qk(const ConvQkArgs& a, int n, hipStream_t stream) {
     else launch_conv_qk<T, 4>(a, n, stream);
 }
 
+template <typename T, int NI>
+static void launch_conv_qk_single(const ConvQkArgs& a, const dim3& grid, hipStream_t stream) {
+    if (a.taps == 4) conv_qk_prepare_single_kernel<T, NI, 4><<<grid, 64, 0, stream>>>(a);
+    else conv_qk_prepare_single_kernel<T, NI, 0><<<grid, 64, 0, stream>>>(a);
+}
+
+template <typename T>
+static void launch_conv_qk_single(const ConvQkArgs& a, const dim3& grid, hipStream_t stream) {
+    if (a.Dp <= 64) launch_conv_qk_single<T, 1>(a, grid, stream);
+    else if (a.Dp <= 128) launch_conv_qk_single<T, 2>(a, grid, stream);
+    else launch_conv_qk_single<T, 4>(a, grid, stream);
+}
+
+// single: every request of the step brings one token, and the history moves on in the same launch (conv_history is then not called).
 extern "C" int pl_conv_qk_prepare(const float* rows, int stride, int off, const float* conv_w, int taps,
-                                  const float* state, long state_stride, int hist_off,
+                                  float* state, long state_stride, int hist_off,
                                   const float* q_gain, const float* k_gain, float eps, const float* freq, int rot,
                                   const int* positions, const int* seq_of, const int* q_start, const int* state_slots,
                                   const int* block_table, int max_blocks, int block_size,
                                   void* q_out, void* k_pool, void* v_pool, int dtype,
-                                  int n, int H, int G, int D, int V, int Dp, hipStream_t stream) {
+                                  int n, int H, int G, int D, int V, int Dp, int single, hipStream_t stream) {
     PL_REQUIRE(n >= 0 && H > 0 && G > 0 && H % G == 0, "conv_qk_prepare: rows %d, %d query heads over %d key heads", n, H, G);
     PL_REQUIRE(D > 0 && V > 0 && Dp >= D && Dp >= V && Dp <= 256, "conv_qk_prepare: heads of %d and %d in rows of %d (up to 256)", D, V, Dp);
     PL_REQUIRE(taps >= 1 && taps <= 16, "conv_qk_prepare: %d taps", taps);
@@ -236,7 +344,12 @@ extern "C" int pl_conv_qk_prepare(const float* rows, int stride, int off, const 
     // large steps by what they compute and read, where the angles once a token and the heads in rounds pay)
     const bool few = n < 512 && H + 2 * G <= 65535;
     const dim3 grid(n, H + 2 * G);
-    if (dtype == PL_DTYPE_F32) {
+    PL_REQUIRE(!single || H + 2 * G <= 65535, "conv_qk_prepare: %d heads", H + 2 * G);
+    if (single && dtype == PL_DTYPE_F32)
+        launch_conv_qk_single<float>(a, grid, stream);
+    else if (single && dtype == PL_DTYPE_BF16)
+        launch_conv_qk_single<bf16_t>(a, grid, stream);
+    else if (dtype == PL_DTYPE_F32) {
         if (few) conv_qk_prepare_heads_kernel<float><<<grid, 64, 0, stream>>>(a);
         else launch_conv_qk<float>(a, n, stream);
     } else if (dtype == PL_DTYPE_BF16) {

@@ -83,7 +83,7 @@ def _signatures(lib) -> None:
         "pl_conv_history": [p, i, i, i, i, p, ctypes.c_long, i, p, p, p, i, p],
         "pl_gated_group_norm": [p, i, i, i, p, i, f, p, i, i, i, i, p, i, p],
         "pl_conv_qk_prepare": [p, i, i, p, i, p, ctypes.c_long, i, p, p, f, p, i, p, p, p, p, p, i, i, p, p, p, i,
-                               i, i, i, i, i, i, p],
+                               i, i, i, i, i, i, i, p],
         "pl_rmsnorm_onto": [p, p, p, f, p, i, i, i, p],
         "pl_scale": [p, f, ctypes.c_long, p],
         "pl_to_bf16": [p, p, ctypes.c_long, p],
@@ -1620,11 +1620,14 @@ def gated_group_norm(x: torch.Tensor, group: int, gain: torch.Tensor | None, eps
 
 def conv_qk_prepare(rows: torch.Tensor, off: int, weight: torch.Tensor, history: torch.Tensor, q_gain, k_gain,
                     eps: float, freq, rot: int, batch, kv, heads: int, kv_heads: int, dim: int, vdim: int,
-                    padded: int, q_out: torch.Tensor) -> torch.Tensor:
+                    padded: int, q_out: torch.Tensor, move_history: bool = False) -> torch.Tensor:
     """For an attention layer with short convolutions: convolution of the projected q | k | v columns, norm a
     head of q and k, rotation of the first ``rot`` values of a head by position * freq, q into ``q_out``
-    [rows, heads * padded] and k, v into the pages, every head in a row of ``padded`` values."""
+    [rows, heads * padded] and k, v into the pages, every head in a row of ``padded`` values.  ``move_history``: the history is
+    moved on here as well (in the same launch where every request of the step brings one token)."""
+    given = history
     n, channels, taps, history, stride = _conv_args(rows, off, weight, history, batch)
+    single = move_history and batch.max_q_len == 1 and heads + 2 * kv_heads <= 65535
     if channels != heads * dim + kv_heads * dim + kv_heads * vdim:
         raise TensorError(f"{channels} channels for {heads} heads and {kv_heads} key heads of {dim} and {vdim}")
     _need(q_gain, "query norm gain", (dim,), torch.float32)
@@ -1646,7 +1649,9 @@ def conv_qk_prepare(rows: torch.Tensor, off: int, weight: torch.Tensor, history:
         q_gain.data_ptr(), k_gain.data_ptr(), float(eps), _ptr(freq) if rot else 0, rot,
         batch.positions.data_ptr(), batch.seq_of.data_ptr(), batch.q_start.data_ptr(), batch.state_slots.data_ptr(),
         kv.block_table.data_ptr(), kv.block_table.shape[1], kv.block_size, q_out.data_ptr(), kv.k_pool.data_ptr(),
-        kv.v_pool.data_ptr(), _code(q_out, "query buffer"), n, heads, kv_heads, dim, vdim, padded, _stream()))
+        kv.v_pool.data_ptr(), _code(q_out, "query buffer"), n, heads, kv_heads, dim, vdim, padded, 1 if single else 0, _stream()))
+    if move_history and not single and taps > 1:
+        conv_history(rows, off, weight, given, batch)
     return q_out
 
 

@@ -90,9 +90,7 @@ class ConvAttention:
             history = torch.empty((1, 0), dtype=torch.float32, device=rows.device)
         q = torch.empty((n, self.H * self.padded), dtype=self.dtype, device=rows.device)
         kernels.conv_qk_prepare(rows, 0, self.conv_w, history, self.q_gain, self.k_gain, self.eps, self.freq,
-                                self.spec.rotary_dim, batch, kv, self.H, self.G, self.D, self.V, self.padded, q)
-        if self.spec.conv_taps > 1:
-            kernels.conv_history(rows, 0, self.conv_w, history, batch)
+                                self.spec.rotary_dim, batch, kv, self.H, self.G, self.D, self.V, self.padded, q, move_history=True)
         out = torch.empty((n, self.H * self.padded), dtype=self.dtype, device=rows.device)
         kernels.paged_attention(q, out, batch, kv, self.H, self.G, self.padded, self.scale, self.window)
         return self.o_proj.forward(out, out_dtype=torch.float32)

@@ -160,8 +160,7 @@ class GatedDelta(_ScanMixer):
         state = ctx.state()
         history = state[:, self.matrix:]
         rows = self.proj.forward(x, out_dtype=torch.float32)
-        mixed = kernels.short_conv(rows, c["q"], self.conv_w, history, ctx.batch, silu=True)
-        kernels.conv_history(rows, c["q"], self.conv_w, history, ctx.batch)
+        mixed = kernels.short_conv(rows, c["q"], self.conv_w, history, ctx.batch, silu=True, move_history=True)
         read = kernels.recurrent_scan("delta", mixed, 0, G * D, 2 * G * D, state[:, :self.matrix], ctx.batch,
                                       self.H, G, D, self.V, gates=rows, g1_off=c["b"], g2_off=c["a"],
                                       p1=self.a_log, p2=self.dt_bias, chunked=True)

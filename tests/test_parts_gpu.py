@@ -1333,3 +1333,45 @@ def test_clearing_state_slots_touches_these_slots_of_every_layer_only(shapes, sl
         assert torch.equal(t, b)
     with pytest.raises(IndexError):
         kernels.clear_slots(kernels.SlotTable(states), [69])
+
+
+def gpu_randn(*shape, std=1.0, seed=0):
+    return randn(*shape, std=std, seed=seed).to(DEV)
+
+
+# --- the convolutions in front of attention, one token a request ------------------------------------------------------
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps,D,V,padded,rot", [(4, 128, 128, 128, 64), (4, 64, 48, 64, 64), (2, 40, 24, 48, 8), (7, 160, 192, 192, 0), (1, 16, 16, 16, 16)])
+def test_single_tokens_move_their_convolutions_history_in_the_same_launch(dtype, taps, D, V, padded, rot):
+    """The kernel of a step of one token a request against the one that leaves the history to a launch of its own: rows,
+    pages and histories, with a row of padding and slots that are not the rows' numbers."""
+    from paged_llm_rs_amd import kernels
+
+    H, G, block, n = 4, 2, 4, 5
+    channels = H * D + G * D + G * V
+    slots = torch.tensor([3, 0, 6, 1, -1], dtype=torch.int32, device=DEV)
+    positions = torch.tensor([0, 9, 2, 14, -1], dtype=torch.int32, device=DEV)
+    at = torch.arange(n, dtype=torch.int32, device=DEV)
+    table = torch.arange(n * 4, dtype=torch.int32, device=DEV).view(n, 4)
+    batch = types.SimpleNamespace(positions=positions, seq_of=at, q_start=at, q_len=torch.ones_like(at), state_slots=slots, num_seqs=n,
+                                  num_tokens=n, max_q_len=1)
+    rows, weight = gpu_randn(n, channels + 8, seed=1), gpu_randn(taps, channels, seed=2)
+    gains = gpu_randn(D, seed=3), gpu_randn(D, seed=4)
+    freq = gpu_randn(max(rot // 2, 1), seed=5).abs()
+    results = []
+    for moves in (False, True):
+        history = gpu_randn(7, (taps - 1) * channels, seed=6) if taps > 1 else torch.empty((1, 0), device=DEV)
+        kv = types.SimpleNamespace(k_pool=torch.zeros((n * 4 * block, G * padded), dtype=dtype, device=DEV),
+                                   v_pool=torch.zeros((n * 4 * block, G * padded), dtype=dtype, device=DEV), block_table=table, block_size=block)
+        q = torch.zeros((n, H * padded), dtype=dtype, device=DEV)
+        kernels.conv_qk_prepare(rows, 8, weight, history, *gains, 1e-6, freq if rot else None, rot, batch, kv, H, G, D, V, padded, q,
+                                move_history=moves)
+        if not moves and taps > 1:
+            kernels.conv_history(rows, 8, weight, history, batch)
+        results.append((q, kv.k_pool, kv.v_pool, history))
+    for old, new in zip(*results):
+        # (the same sums in the same order; the compiler may contract a product and a sum in one and not in the other)
+        assert torch.allclose(old.float(), new.float(), rtol=1e-5 if dtype == torch.float32 else 2.0 ** -8, atol=1e-5)
+    if taps > 1:
+        assert torch.equal(results[0][3], results[1][3]), "histories are copies"
