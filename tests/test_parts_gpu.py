@@ -1339,6 +1339,26 @@ def gpu_randn(*shape, std=1.0, seed=0):
     return randn(*shape, std=std, seed=seed).to(DEV)
 
 
+# --- a norm of a sublayer's output, added onto the stream -----------------------------------------------------------
+
+@pytest.mark.parametrize("width", [3, 64, 252, 1020, 1024, 1028, 2048, 4100, 8192, 8196])
+@pytest.mark.parametrize("rows", [1, 5])
+def test_rmsnorm_onto_over_widths_of_every_kernel(width, rows):
+    """Widths that a thread's groups of four cover once, twice and four times, with and without a remainder, and those
+    that go value by value (no multiple of four, wider than the registers hold)."""
+    from paged_llm_rs_amd import kernels
+
+    resid, y, gain = gpu_randn(rows, width, seed=1), gpu_randn(rows, width, seed=2, std=3.0), gpu_randn(width, seed=3)
+    want = resid.double() + y.double() / (y.double().pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * gain.double()
+    for rows_dtype in (None, torch.float32, torch.bfloat16):
+        got = resid.clone()
+        out = kernels.rmsnorm_onto(got, y, gain, 1e-5, rows_dtype)
+        # the sum of squares of `width` values in 32 bits, and four more operations behind it
+        assert (got - want).abs().max() <= (8 + width ** 0.5) * 2.0 ** -24 * want.abs().max()
+        if rows_dtype is not None:
+            assert torch.equal(out, got.to(rows_dtype))
+
+
 # --- the convolutions in front of attention, one token a request ------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
