@@ -13,6 +13,7 @@ static int sk_launch_plain(int epilogue, int out_f32, const void* x, const void*
 // x: bfloat16 [n, K], or with a gain the 32-bit residual stream [*, K] whose rows rows[0..n) (or 0..n) are
 // normalised on the way in (the gain is 32-bit).  w: bfloat16 [N_out, K], or [2*N_out, K] with gate rows first for epilogue 1.
 // epilogue 0: y = result, bfloat16 or (out_f32) 32-bit.  1: y = act(gate) * up (act: PL_ACT_*).  2: y, 32-bit, += result.
+// 3: y = act(result), bfloat16 (without a gain).
 // x_stride (with a gain): elements between two rows of x (0: K), a multiple of 4.
 // strips: w holds the same weights in strips (gemm_skinny.hpp has the layout; pl_gemm_skinny_strips_apply says for
 // which products that is read).
@@ -25,7 +26,8 @@ extern "C" int pl_gemm_skinny(const void* x, const void* w, void* y, const float
                "skinny product: rows %d apart for an inner width of %d", x_stride, K);
     PL_REQUIRE(n >= 0 && n <= 64, "skinny product: %d rows, it takes up to 64", n);
     PL_REQUIRE(N_out > 0 && K > 0 && K % 8 == 0, "skinny product: %d columns, inner width %d (a multiple of 8 is needed)", N_out, K);
-    PL_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_ADD, "skinny product: epilogue code %d", epilogue);
+    PL_REQUIRE(epilogue >= EPI_STORE && epilogue <= EPI_ACT, "skinny product: epilogue code %d", epilogue);
+    PL_REQUIRE(epilogue != EPI_ACT || (!gain && !out_f32), "skinny product: an activated product has plain rows and a bfloat16 result");
     PL_REQUIRE(epilogue != EPI_ADD || out_f32, "skinny product: the residual stream is 32-bit");
     PL_REQUIRE(gain || !rows, "skinny product: a row list without a norm");
     PL_REQUIRE(epilogue != EPI_SWIGLU || !out_f32, "skinny product: the activation is stored in bfloat16");

@@ -969,13 +969,14 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch
                 norm_gain: torch.Tensor | None = None, eps: float = 0.0, rows: torch.Tensor | None = None,
                 add_into: torch.Tensor | None = None, activation: str = "silu",
                 handed: "HandedNorm | None" = None, hand: "HandedNorm | None" = None,
-                strips: torch.Tensor | None = None, columns: tuple | None = None) -> torch.Tensor:
+                strips: torch.Tensor | None = None, columns: tuple | None = None, activated: bool = False) -> torch.Tensor:
     """y = x . w^T for up to 64 rows on the matrix cores, the bfloat16 weights streamed once.
 
     ``x`` is bfloat16 [n, K]; or, with ``norm_gain``, the 32-bit residual stream, whose rows
     (``rows[i]`` for output row i when a row list is given) are RMS-normalised on the way in.
     With ``swiglu`` the rows of ``w`` are [gate | up] and y = act(x . gate^T) * (x . up^T), in bfloat16
     (``activation``: silu or a gelu).
+    With ``activated`` y = act(x . w^T), in bfloat16, of the 32-bit sum (plain rows, no norm).
     With ``add_into`` (the 32-bit residual stream, [n, N]) the result is added there and that
     tensor is returned.
     ``handed``: a norm that an earlier product left behind; its rows are the input (``x`` is not looked at)
@@ -1022,6 +1023,10 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch
             raise TensorError(f"matrix product output {out_dtype}" + (" after the activation" if swiglu else ""))
         out = torch.empty((n, N_out), dtype=out_dtype, device=x.device)
         epilogue, out_f32 = (1 if swiglu else 0), (1 if out_dtype == torch.float32 else 0)
+    if activated:
+        if swiglu or add_into is not None or norm_gain is not None or handed is not None or out_f32:
+            raise TensorError("an activated product has plain rows, a bfloat16 result and no gate")
+        epilogue = 3
     in_strips = 0
     if strips is not None and library().pl_gemm_skinny_strips_apply(n, N_out, K):
         _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16)

@@ -92,8 +92,7 @@ class DenseMlp:
         self.down_proj = Linear(params["down"])
 
     def forward(self, x):
-        return self.down_proj.forward(kernels.activation(self.up_proj.forward(x), self.activation),
-                                      out_dtype=torch.float32)
+        return self.down_proj.forward(self.up_proj.forward_activated(x, self.activation), out_dtype=torch.float32)
 
 
 register_feed_forward("dense_mlp", DenseMlp)
