@@ -45,16 +45,17 @@ __device__ __forceinline__ dl_f32x4 dl_multiply(const dl_f32x4& a, const dl_f32x
 // 3 us, the inverse another 2: its diagonal blocks by forward substitution, a column a lane, the others as products,
 // T_ij = -T_ii sum_k M_ik T_kj, a block row after the other.  (On the vector units with the whole inverse a column a thread: 111 us for
 // two prompts of 1,500 tokens and eight heads of 128.)
-__global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp) {
+__global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp, int seqs) {
     const ScanArgs& a = da.a;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int D = a.D, H = a.H;
-    const int c_at = blockIdx.x, h = blockIdx.y, s = blockIdx.z;
-    const int slot = a.state_slots[s], n = a.q_len[s];
-    if (slot < 0 || n < a.below || c_at * DL_C >= n) return;
-    const int L = min(DL_C, n - c_at * DL_C), row0 = a.q_start[s] + c_at * DL_C;
+    const int h = blockIdx.y;
+    ChunkPlace place;
+    if (!find_chunk(a, seqs, blockIdx.x, place)) return;
+    const int c_at = place.c, s = place.s, n = place.count;
+    const int L = min(DL_C, n - c_at * DL_C), row0 = place.first_row + c_at * DL_C;
     const int g = h / (H / a.G);
-    const size_t idx = static_cast<size_t>(delta_chunk_number(a, s, c_at)) * H + h;
+    const size_t idx = static_cast<size_t>(place.first_row / DL_C + s + c_at) * H + h;
     const int P = Dp + 4;
     double* bd = reinterpret_cast<double*>(lds);        // [64] b_t, the sum of log decays
     double* nrm = bd + DL_C;                            // [2][64]
@@ -355,14 +356,14 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs da) {
         }
 }
 
-static int launch_delta(const DeltaArgs& da, int seqs, int max_q_len, hipStream_t stream) {
+static int launch_delta(const DeltaArgs& da, int rows, int seqs, int max_q_len, hipStream_t stream) {
     const ScanArgs& a = da.a;
     const int Dp = pl_ceil_div(a.D, 64) * 64, P = Dp + 4;
     const size_t lds_p = (7 * DL_C + 2 * static_cast<size_t>(DL_C) * (P > DL_T ? P : DL_T)) * sizeof(float);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prepare_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(lds_p));
     PL_REQUIRE(e == hipSuccess, "delta_chunked: %zu bytes of LDS refused: %s", lds_p, hipGetErrorString(e));
-    delta_prepare_kernel<<<dim3(pl_ceil_div(max_q_len, DL_C), a.H, seqs), 256, lds_p, stream>>>(da, Dp);
+    delta_prepare_kernel<<<dim3(chunk_bound(rows, max_q_len, seqs), a.H), 256, lds_p, stream>>>(da, Dp, seqs);
     PL_CHECK_LAUNCH("delta_chunked (prepare)");
     // the workgroups of one head read the same chunks: with heads and requests along x they share a chiplet's cache wherever those are a
     // multiple of the eight chiplets
@@ -382,7 +383,7 @@ extern "C" int pl_delta_chunked(const float* qkv, int qkv_stride, int q_off, int
                                 const float* a_log, const float* dt_bias,
                                 float* state, long state_stride, float* out,
                                 const int* q_start, const int* q_len, const int* state_slots,
-                                int seqs, int max_q_len, int H, int G, int D, int V, int from,
+                                int rows, int seqs, int max_q_len, int H, int G, int D, int V, int from,
                                 float* Kn, float* Qn, float* Kw, float* Tm, float* Aq, float* scal, hipStream_t stream) {
     PL_REQUIRE(H > 0 && G > 0 && H % G == 0 && D > 0 && D <= 256 && V > 0 && from >= 1,
                "delta_chunked: %d heads over %d of q and k, %d by %d, from %d tokens", H, G, D, V, from);
@@ -394,5 +395,5 @@ extern "C" int pl_delta_chunked(const float* qkv, int qkv_stride, int q_off, int
     DeltaArgs da{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, a_log, dt_bias, nullptr, 0.f, state,
                   state_stride, 0, 0, 0, out, q_start, q_len, state_slots, H, G, D, V, from},
                  Kn, Qn, Kw, Tm, Aq, scal};
-    return launch_delta(da, seqs, max_q_len, stream);
+    return launch_delta(da, rows, seqs, max_q_len, stream);
 }

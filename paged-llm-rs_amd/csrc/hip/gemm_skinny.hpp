@@ -20,7 +20,8 @@
 //   EPI_STORE   y = result (bfloat16 or 32-bit).
 //   EPI_SWIGLU  the workgroup owns 16 gate columns and the 16 up columns that belong to
 //               them (rows c and N + c of w) and stores silu(gate) * up.
-//   EPI_ACT     y = act(result), bfloat16: the activation of a feed-forward without a gate, of the 32-bit sum.  (2 rows of 3,072 x 1,024:
+//   EPI_ACT     y = act(bf16(result)), bfloat16: the activation of a feed-forward without a gate, of the rounded sum as the pass behind a
+//               product of many rows takes it, so that a row's bits are the same in steps of either size.  (2 rows of 3,072 x 1,024:
 //               4.9 us with the tanh of a GELU; 4.15 and a launch of 3.4 apart.)
 //   EPI_ADD     the 32-bit residual stream takes the result: resid[r, c] += result.  Every
 //               element has one owner, so the sum does not depend on timing.
@@ -449,7 +450,7 @@ gemm_skinny_kernel(const void* __restrict__ x_, const bf16_t* __restrict__ w, OU
             if (mine) {
                 float r = v[0];
                 if (EPI == EPI_SWIGLU) r = pl_activate<false>(v[0], act) * v[BT - 1];
-                if (EPI == EPI_ACT) r = pl_activate<true>(v[0], act);
+                if (EPI == EPI_ACT) r = pl_activate<true>(to_float(from_float<bf16_t>(v[0])), act);
                 const size_t at = static_cast<size_t>(row) * N_out + col;
                 if (EPI == EPI_ADD) {
                     updated = to_float(y[at]) + r;
@@ -748,7 +749,7 @@ gemm_skinny_rows_kernel(const void* __restrict__ x_, const bf16_t* __restrict__ 
             if (out_row < n && col < N_out) {
                 float r = v[0];
                 if (EPI == EPI_SWIGLU) r = pl_activate<false>(v[0], act) * v[BT - 1];
-                if (EPI == EPI_ACT) r = pl_activate<true>(v[0], act);
+                if (EPI == EPI_ACT) r = pl_activate<true>(to_float(from_float<bf16_t>(v[0])), act);
                 const size_t at = static_cast<size_t>(out_row) * N_out + col;
                 if (EPI == EPI_ADD)
                     y[at] = from_float<OUT>(to_float(y[at]) + r);

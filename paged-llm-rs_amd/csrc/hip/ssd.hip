@@ -500,32 +500,69 @@ __device__ __forceinline__ float ssd_q(float x, float scale) { return KIND == PL
 //     y_t = (sum_{u<=t} e^(w_u - b_u - c_t) (q_t . k_u) v_u + e^(m_0 - c_t) S_0^T q_t) / max(|n . q|, e^(-m_t)),  c_t = m_t - b_t,
 // with n . q the same sum without v_u and S_0.)
 
-// summary: a wave a tile of 32 rows of N (and the tile four further on, where N has more than 128), 64 columns of V.
-// Both operands come straight from memory, a token a row: 128 bytes a half wave.
-template <int KIND>
-__global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
+// summary: W tiles of 64 columns of V a workgroup, four waves each; of a tile, a wave 32 rows of N (and the 32 four further on, where N
+// has more than 128).  Both operands go through LDS, a token a row, so that a value is read and activated once a workgroup; rows there are
+// 16 values longer than they hold.  What it is bound by: the trip to memory, the activation (silu of linear attention: an exponential and a
+// division a value) and the trip back, one behind the other.  42 chunks of 8 heads of 128 by 128: SUMMARY0 us (34.4 with every wave
+// reading and activating all of v and a workgroup for each 64 columns and each chunk that there might be), of 4 heads of 128 by 256
+// (matrix memory) SUMMARY1 (24.5).
+#define SSD_SUMMARY_PAD 16
+template <int KIND, int W>
+__global__ __launch_bounds__(256 * W) void ssd_summary_kernel(SsdArgs sa, int seqs, int aligned) {
     const ScanArgs& a = sa.a;
     __shared__ float weight[SSD_CHUNK];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int T = 256 * W, COLS = 64 * W, XP = COLS + SSD_SUMMARY_PAD;
     const int N = a.D, V = a.V, H = a.H;
-    const int tiles = (V + 63) / 64;
-    const int c = blockIdx.x, h = blockIdx.y / tiles, vt = blockIdx.y % tiles, s = blockIdx.z;
-    const int slot = a.state_slots[s], count = a.q_len[s];
-    if (slot < 0 || count < a.below || c * SSD_CHUNK >= count) return;
-    const int L = min(SSD_CHUNK, count - c * SSD_CHUNK), row0 = a.q_start[s] + c * SSD_CHUNK;
-    const size_t idx = static_cast<size_t>(ssd_chunk(a, s, c)) * H + h;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles = (V + COLS - 1) / COLS;
+    const int h = blockIdx.y / tiles, vt = blockIdx.y % tiles;
+    ChunkPlace place;
+    if (!find_chunk(a, seqs, blockIdx.x, place)) return;
+    const int c = place.c, s = place.s;
+    const int L = min(SSD_CHUNK, place.count - c * SSD_CHUNK), row0 = place.first_row + c * SSD_CHUNK;
+    const size_t idx = static_cast<size_t>(place.first_row / SSD_CHUNK + s + c) * H + h;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const int g = h / (H / a.G);
-    const bool two = vt * 64 + 32 < V;               // whether the second 32 columns exist
-    const int va = min(vt * 64 + l32, V - 1), vb = min(vt * 64 + 32 + l32, V - 1);
-    float xa[SSD_CHUNK / 2], xb[SSD_CHUNK / 2];
+    const int Nq = (N + 31) / 32 * 32, KP = Nq + SSD_SUMMARY_PAD;
+    float* Xs = lds;                                  // [64][XP]
+    float* Ks = lds + SSD_CHUNK * XP;                 // [64][KP]
     const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
-    // (every load before the first silu: one behind a branch would be waited for alone)
+    const float* v_at = rows + a.v_off + h * V;
+    const float* k_at = rows + a.k_off + g * N;
+    // four neighbouring columns from column i on of a row's `width`, zeros past it
+    auto load4 = [&](const float* row, int i, int width) {
+        if (aligned && i + 3 < width) return *reinterpret_cast<const ssd_f32x4*>(row + i);
+        ssd_f32x4 v;
 #pragma unroll
-    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
-        const float* x = rows + static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.v_off + h * V;
-        xa[k] = x[va];
-        xb[k] = x[vb];
+        for (int j = 0; j < 4; ++j) v[j] = i + j < width ? row[i + j] : 0.f;
+        return v;
+    };
+    // (tokens past the chunk: its last again, under a weight of zero)
+    ssd_f32x4 x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = tid + i * T, t = e / (COLS / 4), col = vt * COLS + 4 * (e % (COLS / 4));
+        x[i] = load4(v_at + static_cast<size_t>(min(t, L - 1)) * a.qkv_stride, col, V);
+    }
+    for (int e0 = 0; e0 < SSD_CHUNK * Nq / 4; e0 += 4 * T) {
+        ssd_f32x4 kv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = min(e0 + tid + i * T, SSD_CHUNK * Nq / 4 - 1), t = e / (Nq / 4);
+            kv[i] = load4(k_at + static_cast<size_t>(min(t, L - 1)) * a.qkv_stride, 4 * (e - t * (Nq / 4)), N);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + tid + i * T;
+            if (e >= SSD_CHUNK * Nq / 4) continue;
+            const int t = e / (Nq / 4), n = 4 * (e - t * (Nq / 4));
+            if (KIND == PL_SCAN_LIGHTNING) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) kv[i][j] = ssd_kv<KIND>(kv[i][j]);
+            }
+            *reinterpret_cast<ssd_f32x4*>(Ks + t * KP + n) = kv[i];
+        }
     }
     if (wave == 0) {
         double b, dt;
@@ -539,7 +576,7 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
                 // (their sum: either may be hundreds where it is small, and rounded alone would leave its rounding in the state)
                 sa.tops[2 * idx] = static_cast<float>(end + top);
                 // the maximum that the request's first chunk starts from: the carry reads it here, not in the slot it writes
-                if (c == 0) sa.tops[2 * idx + 1] = a.state[static_cast<size_t>(slot) * a.state_stride + a.m_off + h * tiles];
+                if (c == 0) sa.tops[2 * idx + 1] = a.state[static_cast<size_t>(a.state_slots[s]) * a.state_stride + a.m_off + h * ((V + 63) / 64)];
             }
         } else {
             weight[lane] = expf(static_cast<float>(end - b)) * static_cast<float>(dt);  // (zero past the chunk's tokens)
@@ -548,43 +585,48 @@ __global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
-        const float w = weight[2 * k + half];
-        xa[k] = ssd_kv<KIND>(xa[k]) * w;
-        xb[k] = ssd_kv<KIND>(xb[k]) * w;
+    for (int i = 0; i < 4; ++i) {
+        const int e = tid + i * T, t = e / (COLS / 4), col = 4 * (e % (COLS / 4));
+        const float w = weight[t];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[i][j] = ssd_kv<KIND>(x[i][j]) * w;
+        *reinterpret_cast<ssd_f32x4*>(Xs + t * XP + col) = x[i];
+    }
+    __syncthreads();
+    if (KIND == PL_SCAN_MLSTM && vt == 0) {
+        for (int n = tid; n < N; n += T) {
+            float even = 0.f, odd = 0.f;
+#pragma unroll 8
+            for (int t = 0; t < SSD_CHUNK; t += 2) {
+                even += weight[t] * Ks[t * KP + n];
+                odd += weight[t + 1] * Ks[(t + 1) * KP + n];
+            }
+            sa.Uk[idx * N + n] = even + odd;
+        }
     }
     float* U = sa.U + idx * N * V;
-    for (int n0 = wave * 32; n0 < N; n0 += 128) {
-        const int n = min(n0 + l32, N - 1);
-        float ka[SSD_CHUNK / 2];
-#pragma unroll
-        for (int k = 0; k < SSD_CHUNK / 2; ++k)
-            ka[k] = rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n];
-        if (KIND == PL_SCAN_LIGHTNING) {
-#pragma unroll
-            for (int k = 0; k < SSD_CHUNK / 2; ++k) ka[k] = ssd_kv<KIND>(ka[k]);
-        }
-        if (KIND == PL_SCAN_MLSTM && vt == 0) {
-            float sum = 0.f;
-#pragma unroll
-            for (int k = 0; k < SSD_CHUNK / 2; ++k) sum += weight[2 * k + half] * ka[k];
-            sum += __shfl_xor(sum, 32, 64);
-            if (half == 0 && n0 + l32 < N) sa.Uk[idx * N + n0 + l32] = sum;
-        }
+    const int v0 = 64 * (wave >> 2);                  // the wave's first column of the workgroup's
+    if (vt * COLS + v0 >= V) return;
+    const bool two = vt * COLS + v0 + 32 < V;         // whether its second 32 columns exist
+    for (int n0 = (wave & 3) * 32; n0 < N; n0 += 128) {
         ssd_f32x16 da, db;
 #pragma unroll
         for (int r = 0; r < 16; ++r) da[r] = db[r] = 0.f;
+        const float* kr = Ks + half * KP + n0 + l32;
+        const float* xr = Xs + half * XP + v0 + l32;
 #pragma unroll
         for (int k = 0; k < SSD_CHUNK / 2; ++k) {
-            da = ssd_mfma(ka[k], xa[k], da);
-            if (two) db = ssd_mfma(ka[k], xb[k], db);
+            const float kk = kr[2 * k * KP];
+            da = ssd_mfma(kk, xr[2 * k * XP], da);
+            if (two) db = ssd_mfma(kk, xr[2 * k * XP + 32], db);
         }
+        const int va = vt * COLS + v0 + l32;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = n0 + 8 * (r >> 2) + 4 * half + (r & 3);
             if (row >= N) continue;
-            if (vt * 64 + l32 < V) U[static_cast<size_t>(row) * V + vt * 64 + l32] = da[r];
-            if (vt * 64 + 32 + l32 < V) U[static_cast<size_t>(row) * V + vt * 64 + 32 + l32] = db[r];
+            if (va < V) U[static_cast<size_t>(row) * V + va] = da[r];
+            if (va + 32 < V) U[static_cast<size_t>(row) * V + va + 32] = db[r];
         }
     }
 }
@@ -645,20 +687,25 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
     if (KIND == PL_SCAN_MLSTM && e < tiles) slot_state[a.m_off + h * tiles + e] = m;
 }
 
-// output: the read-outs of one chunk, head and tile of 64 columns.  Four waves; wave 2 ti + j owns the tokens 32 ti .. + 31 and, of the
-// scores, the earlier tokens 32 j .. + 31, of the read-outs, the columns 32 j .. + 31.
+// output: the read-outs of one chunk, head and W tiles of 64 columns.  4 W waves; wave 2 W ti + j owns the tokens 32 ti .. + 31 and, of the
+// scores, the earlier tokens 32 j .. + 31 (j < 2), of the read-outs, the columns 32 j .. + 31.  Bound by its chain (rows, scores, what the
+// state gives, what the chunk gives; three barriers), so waves without scores do the state's part meanwhile, and two workgroups share a
+// compute unit.  Two tiles a workgroup make the scores once for both: 42 chunks of 8 heads of 128 by 128 OUTPUT0 us (50.8 with a tile a
+// workgroup and one for each chunk that there might be), of 4 heads of 128 by 256 (matrix memory) OUTPUT1 (49.3).
 // LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes, two numbers a token.
-template <int KIND>
-__global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int aligned) {
+template <int KIND, int W>
+__global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, int seqs, int aligned) {
     const ScanArgs& a = sa.a;
     extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int T = 256 * W;
     const int N = a.D, V = a.V, H = a.H;
-    const int tiles = (V + 63) / 64;
-    const int c = blockIdx.x, h = blockIdx.y / tiles, vt = blockIdx.y % tiles, s = blockIdx.z;
-    const int slot = a.state_slots[s], count = a.q_len[s];
-    if (slot < 0 || count < a.below || c * SSD_CHUNK >= count) return;
-    const int L = min(SSD_CHUNK, count - c * SSD_CHUNK), row0 = a.q_start[s] + c * SSD_CHUNK;
-    const size_t idx = static_cast<size_t>(ssd_chunk(a, s, c)) * H + h;
+    const int tiles = (V + 64 * W - 1) / (64 * W);
+    const int h = blockIdx.y / tiles, vt = blockIdx.y % tiles;
+    ChunkPlace place;
+    if (!find_chunk(a, seqs, blockIdx.x, place)) return;
+    const int c = place.c, s = place.s;
+    const int L = min(SSD_CHUNK, place.count - c * SSD_CHUNK), row0 = place.first_row + c * SSD_CHUNK;
+    const size_t idx = static_cast<size_t>(place.first_row / SSD_CHUNK + s + c) * H + h;
     const int g = h / (H / a.G);
     const int Np = (N + 7) & ~7, P = Np + 4;
     constexpr int PA = SSD_CHUNK + 4;
@@ -673,13 +720,13 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
     float* As = Bs;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int ti = wave >> 1, tj = wave & 1;
+    const int ti = wave / (2 * W), tj = wave % (2 * W);
     const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
 
     // ---- what waits for nothing: C and B into LDS, the columns of x into registers, the first rows of S_0 ----
     if (aligned) {
         const int quads = Np / 4;
-        for (int e = tid; e < SSD_CHUNK * quads; e += 256) {
+        for (int e = tid; e < SSD_CHUNK * quads; e += T) {
             const int t = e / quads, i = 4 * (e - t * quads);
             ssd_f32x4 cv = {0.f, 0.f, 0.f, 0.f}, bv = cv;
             if (t < L && i < N) {
@@ -698,7 +745,7 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             *reinterpret_cast<ssd_f32x4*>(Bs + t * P + i) = bv;
         }
     } else {
-        for (int e = tid; e < SSD_CHUNK * Np; e += 256) {
+        for (int e = tid; e < SSD_CHUNK * Np; e += T) {
             const int t = e / Np, i = e - t * Np;
             const bool in = t < L && i < N;
             const float* row = rows + static_cast<size_t>(in ? t : 0) * a.qkv_stride + g * N + (in ? i : 0);
@@ -706,8 +753,8 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
             Bs[t * P + i] = in ? ssd_kv<KIND>(row[a.k_off]) : 0.f;
         }
     }
-    const int v = vt * 64 + 32 * tj + l32, vc = min(v, V - 1);
-    const bool columns = vt * 64 + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
+    const int v = vt * 64 * W + 32 * tj + l32, vc = min(v, V - 1);
+    const bool columns = vt * 64 * W + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
     float x[SSD_CHUNK / 2];                                           // x of token 8 q + 4 half + e in x[4 q + e]
 #pragma unroll
     for (int k = 0; k < SSD_CHUNK / 2; ++k) {
@@ -751,6 +798,34 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
 
     // ---- the scores C_t . B_u of a tile of 32 by 32 (the tile of later tokens against earlier ones is all hidden) ----
     const bool scored = tj <= ti && 32 * ti < L;
+    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size.  Linear attention
+    // with heads of 256, against 64 bits: 1.2e-7 to 1.5e-7; everything in one chain 1.5e-7 to 2.5e-7)
+    ssd_f32x16 y, y2;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;
+    auto state_part = [&]() {                                         // S_0^T C_t, times e^(b_t)
+        const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
+        for (int n0 = 0; n0 < Np; n0 += 64) {
+            float now[32];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) now[k] = s0[k];
+            if (n0 + 64 < Np) ask(n0 + 64, s0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                if (n0 + 8 * q < Np) {
+                    const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + n0 + 8 * q);   // (zeros past N)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (q % 2 == 0) y = ssd_mfma(cv[e], now[4 * q + e], y);
+                        else y2 = ssd_mfma(cv[e], now[4 * q + e], y2);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] = (y[r] + y2[r]) * before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
+    };
+    if (columns && !scored) state_part();
     ssd_f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -777,48 +852,21 @@ __global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int alig
 #pragma unroll
         for (int r = 0; r < 16; ++r) As[(32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)) * PA + 32 * tj + l32] = acc[r];
     }
-    // ---- S_0^T C_t, times e^(b_t) ----
-    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size.  Linear attention
-    // with heads of 256, against 64 bits: 1.2e-7 to 1.5e-7; everything in one chain 1.5e-7 to 2.5e-7)
-    ssd_f32x16 y, y2;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;
-    if (columns) {
-        const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
-        for (int n0 = 0; n0 < Np; n0 += 64) {
-            float now[32];
-#pragma unroll
-            for (int k = 0; k < 32; ++k) now[k] = s0[k];
-            if (n0 + 64 < Np) ask(n0 + 64, s0);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (n0 + 8 * q < Np) {
-                    const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + n0 + 8 * q);   // (zeros past N)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (q % 2 == 0) y = ssd_mfma(cv[e], now[4 * q + e], y);
-                        else y2 = ssd_mfma(cv[e], now[4 * q + e], y2);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) y[r] = (y[r] + y2[r]) * before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
-    }
+    if (columns && scored) state_part();
     __syncthreads();                                                  // the weighted scores are written
     if (KIND == PL_SCAN_MLSTM) {
         // n . q of a token, by four lanes: the weighted scores' sum and e^(m_0 - c_t) (n_0 . q_t)
         const int t = tid >> 2, part = tid & 3;
         float sum = 0.f, dot = 0.f;
-        if (t < L) {
+        if (t < L) {                                                  // (of a second tile's threads, none)
             const float* n0 = sa.nin + idx * N;
             for (int u = part; u <= t; u += 4) sum += As[t * PA + u];
             for (int i = part; i < N; i += 4) dot += n0[i] * Cs[t * P + i];
         }
-        sum += before_w[t] * dot;
+        if (t < SSD_CHUNK) sum += before_w[t] * dot;
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);
-        if (part == 0) below[t] = 1.f / (fmaxf(fabsf(sum), expf(below[t])) + 1e-6f);
+        if (part == 0 && t < SSD_CHUNK) below[t] = 1.f / (fmaxf(fabsf(sum), expf(below[t])) + 1e-6f);
         __syncthreads();
     }
     if (!columns) return;
@@ -892,31 +940,42 @@ extern "C" int pl_ssd_step(const float* qkv, int qkv_stride, int q_off, int k_of
     return 0;
 }
 
-template <int KIND>
-static int launch_chunks(const SsdArgs& sa, int seqs, int max_q_len, hipStream_t stream) {
+template <int KIND, int W>
+static int launch_chunks_of(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
     const ScanArgs& a = sa.a;
-    const int N = a.D, V = a.V, tiles = pl_ceil_div(V, 64);
-    const dim3 grid(pl_ceil_div(max_q_len, SSD_CHUNK), a.H * tiles, seqs);
-    ssd_summary_kernel<KIND><<<grid, 256, 0, stream>>>(sa);
+    const int N = a.D, V = a.V;
+    const dim3 grid(chunk_bound(rows, max_q_len, seqs), a.H * pl_ceil_div(V, 64 * W));
+    const auto room = [](const void* kernel, size_t lds) {
+        return lds <= 48 * 1024 ? hipSuccess : hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    };
+    const size_t lds_s = SSD_CHUNK * (64 * W + pl_ceil_div(N, 32) * 32 + 2 * SSD_SUMMARY_PAD) * sizeof(float);
+    hipError_t e = room(reinterpret_cast<const void*>(&ssd_summary_kernel<KIND, W>), lds_s);
+    PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds_s, hipGetErrorString(e));
+    const bool aligned = ssd_aligned(a);
+    ssd_summary_kernel<KIND, W><<<grid, 256 * W, lds_s, stream>>>(sa, seqs, aligned && V % 4 == 0 ? 1 : 0);
     PL_CHECK_LAUNCH("ssd_chunked (summary)");
     ssd_carry_kernel<KIND><<<dim3(pl_ceil_div(N * (KIND == PL_SCAN_MLSTM ? V + 1 : V), 256), a.H, seqs), 256, 0, stream>>>(sa);
     PL_CHECK_LAUNCH("ssd_chunked (carry)");
     const int P = ((N + 7) & ~7) + 4;
     const size_t lds = (6 * SSD_CHUNK + SSD_CHUNK * static_cast<size_t>(P) + SSD_CHUNK * static_cast<size_t>(P > SSD_CHUNK + 4 ? P : SSD_CHUNK + 4)) * sizeof(float);
-    if (lds > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ssd_output_kernel<KIND>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-    }
-    ssd_output_kernel<KIND><<<grid, 256, lds, stream>>>(sa, ssd_aligned(a) ? 1 : 0);
+    e = room(reinterpret_cast<const void*>(&ssd_output_kernel<KIND, W>), lds);
+    PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    ssd_output_kernel<KIND, W><<<grid, 256 * W, lds, stream>>>(sa, seqs, aligned ? 1 : 0);
     PL_CHECK_LAUNCH("ssd_chunked (output)");
     return 0;
 }
 
-// The requests that bring at least `from` tokens, in chunks of 64.  U, Sin: room for (rows / 64 + requests + 1) chunks of
+template <int KIND>
+static int launch_chunks(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
+    return sa.a.V > 64 ? launch_chunks_of<KIND, 2>(sa, rows, seqs, max_q_len, stream) : launch_chunks_of<KIND, 1>(sa, rows, seqs, max_q_len, stream);
+}
+
+// The requests that bring at least `from` tokens, in chunks of 64; `rows`: what the step's requests bring together at most.  U, Sin: room
+// for (rows / 64 + requests + 1) chunks of
 // H * N * V floats; ends: of H.
 extern "C" int pl_ssd_chunked(const float* qkv, int qkv_stride, int q_off, int k_off, int v_off, const float* gates, int gates_stride,
                               int g_off, const float* a_log, const float* dt_bias, const float* skip, float* state, long state_stride,
-                              float* out, const int* q_start, const int* q_len, const int* state_slots, int seqs, int max_q_len, int H,
+                              float* out, const int* q_start, const int* q_len, const int* state_slots, int rows, int seqs, int max_q_len, int H,
                               int G, int N, int V, int from, float* U, float* Sin, float* ends, hipStream_t stream) {
     PL_REQUIRE(H > 0 && G > 0 && H % G == 0 && N > 0 && N <= 256 && V > 0 && from >= 1, "ssd_chunked: %d heads of %d by %d over %d groups, from %d tokens", H, N, V, G, from);
     PL_REQUIRE(gates != nullptr && a_log != nullptr && dt_bias != nullptr && skip != nullptr && U != nullptr && Sin != nullptr && ends != nullptr,
@@ -926,7 +985,7 @@ extern "C" int pl_ssd_chunked(const float* qkv, int qkv_stride, int q_off, int k
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g_off, 0, a_log, dt_bias, skip, 0.f, state, state_stride,
                       0, 0, 0, out, q_start, q_len, state_slots, H, G, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
-    return launch_chunks<PL_SCAN_SSD>(sa, seqs, max_q_len, stream);
+    return launch_chunks<PL_SCAN_SSD>(sa, rows, seqs, max_q_len, stream);
 }
 
 // Retention: S = decay S + k v^T, o = S^T q, q and k turning with their positions (HalfTurn; freq null: not at all).
@@ -968,7 +1027,7 @@ extern "C" int pl_retention_step(const float* qkv, int qkv_stride, int q_off, in
 
 // The requests that bring at least `from` tokens, in chunks of 64, q and k turned already; decays above zero.  Room as in pl_ssd_chunked.
 extern "C" int pl_retention_chunked(const float* qkv, int qkv_stride, int q_off, int k_off, int v_off, const float* decay, float* state,
-                                    long state_stride, float* out, const int* q_start, const int* q_len, const int* state_slots, int seqs,
+                                    long state_stride, float* out, const int* q_start, const int* q_len, const int* state_slots, int rows, int seqs,
                                     int max_q_len, int H, int N, int V, int from, float* U, float* Sin, float* ends, hipStream_t stream) {
     PL_REQUIRE(H > 0 && N > 0 && N <= 256 && V > 0 && from >= 1, "retention_chunked: %d heads of %d by %d, from %d tokens", H, N, V, from);
     PL_REQUIRE(decay != nullptr && U != nullptr && Sin != nullptr && ends != nullptr, "retention_chunked: the decays or room for the chunks' sums are missing");
@@ -976,7 +1035,7 @@ extern "C" int pl_retention_chunked(const float* qkv, int qkv_stride, int q_off,
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, nullptr, 0, 0, 0, decay, nullptr, nullptr, 0.f, state, state_stride,
                       0, 0, 0, out, q_start, q_len, state_slots, H, H, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
-    return launch_chunks<PL_SCAN_RETENTION>(sa, seqs, max_q_len, stream);
+    return launch_chunks<PL_SCAN_RETENTION>(sa, rows, seqs, max_q_len, stream);
 }
 
 // Linear attention with a fixed decay a head and silu on q, k and v (kind lightning), and the matrix memory with exponential gates
@@ -987,7 +1046,7 @@ extern "C" int pl_recurrent_chunked(int kind, const float* qkv, int qkv_stride, 
                                     const float* p1, const float* p2, float cap,
                                     float* state, long state_stride, int s_off, int n_off, int m_off,
                                     float* out, const int* q_start, const int* q_len, const int* state_slots,
-                                    int seqs, int max_q_len, int H, int D, int V, int from, int chunks,
+                                    int rows, int seqs, int max_q_len, int H, int D, int V, int from, int chunks,
                                     float* U, float* Uk, float* Sin, float* nin, float* scal, hipStream_t stream) {
     PL_REQUIRE(kind == PL_SCAN_LIGHTNING || kind == PL_SCAN_MLSTM, "recurrent_chunked: kind %d", kind);
     PL_REQUIRE(H > 0 && D > 0 && D <= 256 && V > 0 && from >= 1, "recurrent_chunked: %d heads of %d by %d, from %d tokens", H, D, V, from);
@@ -1000,6 +1059,6 @@ extern "C" int pl_recurrent_chunked(int kind, const float* qkv, int qkv_stride, 
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, p1, p2, nullptr, cap, state, state_stride,
                       s_off, n_off, m_off, out, q_start, q_len, state_slots, H, H, D, V, from},
                      U, Sin, scal, Uk, nin, scal + static_cast<size_t>(chunks) * H};
-    return kind == PL_SCAN_LIGHTNING ? launch_chunks<PL_SCAN_LIGHTNING>(sa, seqs, max_q_len, stream)
-                                     : launch_chunks<PL_SCAN_MLSTM>(sa, seqs, max_q_len, stream);
+    return kind == PL_SCAN_LIGHTNING ? launch_chunks<PL_SCAN_LIGHTNING>(sa, rows, seqs, max_q_len, stream)
+                                     : launch_chunks<PL_SCAN_MLSTM>(sa, rows, seqs, max_q_len, stream);
 }

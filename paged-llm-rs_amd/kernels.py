@@ -69,14 +69,14 @@ def _signatures(lib) -> None:
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
                               i, i, i, i, i, i, p],
         "pl_recurrent_chunked": [i, p, i, i, i, i, p, i, i, i, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
-                                 i, i, i, i, i, i, i, p, p, p, p, p, p],
+                                 i, i, i, i, i, i, i, i, p, p, p, p, p, p],
         "pl_ssd_step": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p],
         "pl_ssd_step_applies": [i, ctypes.c_long],
-        "pl_ssd_chunked": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p, p, p],
+        "pl_ssd_chunked": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, p, p, p, p],
         "pl_retention_turn": [p, i, i, i, i, i, i, p, i, f, f, p, p],
         "pl_retention_step": [p, i, i, i, i, p, p, i, f, f, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, p],
-        "pl_retention_chunked": [p, i, i, i, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p, p, p, p],
-        "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i,
+        "pl_retention_chunked": [p, i, i, i, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p, p, p],
+        "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i,
                              p, p, p, p, p, p, p],
         "pl_short_conv": [p, i, i, i, p, i, p, ctypes.c_long, i, p, p, p, p, p, i, p, i, i, p],
         "pl_clear_slots": [p, i, ctypes.c_longlong, p, i, p],
@@ -976,7 +976,7 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch
     (``rows[i]`` for output row i when a row list is given) are RMS-normalised on the way in.
     With ``swiglu`` the rows of ``w`` are [gate | up] and y = act(x . gate^T) * (x . up^T), in bfloat16
     (``activation``: silu or a gelu).
-    With ``activated`` y = act(x . w^T), in bfloat16, of the 32-bit sum (plain rows, no norm).
+    With ``activated`` y = act(x . w^T) of the product in bfloat16, as ``activation`` behind it gives it (plain rows, no norm).
     With ``add_into`` (the 32-bit residual stream, [n, N]) the result is added there and that
     tensor is returned.
     ``handed``: a norm that an earlier product left behind; its rows are the input (``x`` is not looked at)
@@ -1412,7 +1412,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
         _check(library().pl_delta_chunked(
             qkv.data_ptr(), width, q_off, k_off, v_off, gates.data_ptr(), gates.shape[1], g1_off, g2_off,
             p1.data_ptr(), p2.data_ptr(), state.data_ptr(), stride, out.data_ptr(), batch.q_start.data_ptr(),
-            batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs, batch.max_q_len, heads, qk_heads, dim,
+            batch.q_len.data_ptr(), batch.state_slots.data_ptr(), n, batch.num_seqs, batch.max_q_len, heads, qk_heads, dim,
             vdim, SCAN_CHUNKED_FROM, unit_k.data_ptr(), unit_q.data_ptr(), weighted_k.data_ptr(), inverse.data_ptr(), masked.data_ptr(),
             scalars.data_ptr(), _stream()))
     elif chunked:
@@ -1422,7 +1422,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
         k_sums, n_before = (torch.empty((chunks, heads * dim), **f32), torch.empty((chunks, heads * dim), **f32)) \
             if kind == "mlstm" else (None, None)
         scalars = torch.empty((chunks, heads * 4), **f32)
-        _check(library().pl_recurrent_chunked(*common, batch.max_q_len, heads, dim, vdim, SCAN_CHUNKED_FROM, chunks,
+        _check(library().pl_recurrent_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, heads, dim, vdim, SCAN_CHUNKED_FROM, chunks,
                                               sums.data_ptr(), _ptr(k_sums), before.data_ptr(), _ptr(n_before),
                                               scalars.data_ptr(), _stream()))
     return out
@@ -1453,7 +1453,7 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
         f32 = dict(dtype=torch.float32, device=qkv.device)
         sums, before = torch.empty((chunks, H * N * V), **f32), torch.empty((chunks, H * N * V), **f32)
         ends = torch.empty((chunks, H), **f32)
-        _check(lib.pl_ssd_chunked(*common, batch.max_q_len, H, G, N, V, SCAN_CHUNKED_FROM, sums.data_ptr(), before.data_ptr(),
+        _check(lib.pl_ssd_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, H, G, N, V, SCAN_CHUNKED_FROM, sums.data_ptr(), before.data_ptr(),
                                   ends.data_ptr(), stream))
     return out
 
@@ -1512,7 +1512,7 @@ def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state
         f32 = dict(dtype=torch.float32, device=rows.device)
         sums, before_chunks = torch.empty((chunks, heads * dim * vdim), **f32), torch.empty((chunks, heads * dim * vdim), **f32)
         ends = torch.empty((chunks, heads), **f32)
-        _check(lib.pl_retention_chunked(*at, decay.data_ptr(), state.data_ptr(), stride, out.data_ptr(), *step, batch.max_q_len, heads,
+        _check(lib.pl_retention_chunked(*at, decay.data_ptr(), state.data_ptr(), stride, out.data_ptr(), *step[:-1], n, batch.num_seqs, batch.max_q_len, heads,
                                         dim, vdim, SCAN_CHUNKED_FROM, sums.data_ptr(), before_chunks.data_ptr(), ends.data_ptr(), stream))
     return out
 

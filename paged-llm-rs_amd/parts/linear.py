@@ -60,7 +60,7 @@ class Linear:
         return self._product(x, out_dtype, add_into, swiglu, activation, hand)
 
     def forward_activated(self, x, activation: str):
-        """act(x . W^T) in the type of ``x``: of few bfloat16 rows the product's last stage, of the 32-bit sums; otherwise a pass behind it."""
+        """act(x . W^T) in the type of ``x``: of few bfloat16 rows the product's last stage; otherwise a pass behind it."""
         if (self.bias is None and isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 == self.weight.dtype
                 and x.shape[1] == self.in_features and kernels.skinny_applies(x, self.weight, self.strips is not None)):
             return kernels.gemm_skinny(x, self.weight, activation=activation, strips=self.strips, activated=True)

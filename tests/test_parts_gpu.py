@@ -1402,7 +1402,8 @@ def test_single_tokens_move_their_convolutions_history_in_the_same_launch(dtype,
 @pytest.mark.parametrize("name", ["gelu_pytorch_tanh", "gelu", "silu", "relu2"])
 @pytest.mark.parametrize("n,N,K", [(1, 3072, 1024), (7, 40, 64), (16, 24, 8), (17, 96, 512), (33, 48, 1000), (64, 272, 2048), (65, 48, 64)])
 def test_activated_product_of_few_rows(name, n, N, K):
-    """Every kernel of the product for few rows and, past 64 rows, the pass behind the library's: act of the product, in bfloat16."""
+    """Every kernel of the product for few rows and, past 64 rows, the pass behind the library's: act of the product in bfloat16,
+    the same bits as product and pass."""
     from paged_llm_rs_amd import kernels
     from paged_llm_rs_amd.parts.linear import Linear
 
@@ -1412,7 +1413,8 @@ def test_activated_product_of_few_rows(name, n, N, K):
     act = {"gelu_pytorch_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"), "gelu": torch.nn.functional.gelu,
            "silu": torch.nn.functional.silu, "relu2": lambda t: torch.relu(t) ** 2}[name]
     assert got.dtype == torch.bfloat16 and got.shape == (n, N)
-    # a rounding of the result and, where the activation is a pass behind the product, one of its input (slopes up to 2 |y|)
+    assert torch.equal(got, kernels.activation(Linear(w).forward(x), name))
+    # a rounding of the result and one of the activation's input (slopes up to 2 |y|)
     assert torch.allclose(got.double(), act(y), rtol=2.0 ** -6, atol=2.0 ** -7)
     with pytest.raises(Exception):
         kernels.gemm_skinny(x[:1], w, torch.float32, activated=True)
