@@ -192,10 +192,12 @@ gemm_tiled_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, vo
                     acc[t][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[set][t][kk], b[set][mb][kk], acc[t][mb], 0, 0, 0);
     };
     // One step: the loads of the step after this one have landed in this wave (two later steps, eight loads,
-    // may be on their way); after the barrier every wave's have, and every wave has read this step's operands,
-    // whose stage is the one asked for next.
+    // may be on their way), and the wave holds this step's operands (lgkmcnt 0: they were asked of LDS a step ago); after the barrier
+    // that is so of every wave, and this step's stage is the one asked for next.  (Without the wait for the operands a load that
+    // a cache answers could reach the stage before another wave's reads of it did: rows of experts whose 32 columns of one wave were off
+    // by a step of the inner width, other ones in every run.)
     auto one_step = [&](int set, int step) {
-        __builtin_amdgcn_s_waitcnt(0x0F70 | 8);
+        __builtin_amdgcn_s_waitcnt(0x0070 | 8);      // vmcnt 8, lgkmcnt 0
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();

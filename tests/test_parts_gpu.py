@@ -1418,3 +1418,43 @@ def test_activated_product_of_few_rows(name, n, N, K):
     assert torch.allclose(got.double(), act(y), rtol=2.0 ** -6, atol=2.0 ** -7)
     with pytest.raises(Exception):
         kernels.gemm_skinny(x[:1], w, torch.float32, activated=True)
+
+
+# --- the tiled product's stages ------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("rows,width,ff", [(1792, 1024, 1536), (300, 512, 192), (2000, 256, 3072)])
+def test_grouped_products_give_a_row_the_same_bits_in_every_run(rows, width, ff):
+    """A stage of LDS is filled again only when every wave holds its operands: every run gives a row the same bits
+    whichever slot it got, and those of the experts it names."""
+    from paged_llm_rs_amd import kernels
+
+    E, top, vocab = 8, 2, 999
+    x = gpu_randn(rows, width, seed=1).bfloat16()
+    w_up, w_down = gpu_randn(E, 2 * ff, width, std=0.02, seed=2).bfloat16(), gpu_randn(E, width, ff, std=0.02, seed=3).bfloat16()
+    table = gpu_randn(vocab, E, seed=4).argsort(1)[:, :top].to(torch.int32).contiguous()
+    ids = torch.arange(rows, dtype=torch.int32, device=DEV) * 7 % vocab
+    batch = types.SimpleNamespace(token_ids=ids, positions=torch.arange(rows, dtype=torch.int32, device=DEV), fed_tokens=None, token_src=None)
+    runs = [kernels.moe_grouped(x, batch, table, w_up, w_down) for _ in range(6)]
+    want = torch.zeros((rows, width), device=DEV)
+    chosen = table[ids.long()]
+    for e in range(E):
+        at, _ = torch.where(chosen == e)
+        both = x[at].float() @ w_up[e].float().T
+        hidden = (torch.nn.functional.silu(both[:, :ff]) * both[:, ff:]).bfloat16().float()
+        want.index_add_(0, at, hidden @ w_down[e].float().T / top)
+    assert all(torch.equal(runs[0], r) for r in runs[1:])
+    # (a step of the inner width off by one moves single values by a tenth of their size and more; roundings of `ff` hidden values to
+    # eight bits, 2^-9 each, by 2^-9 of the root of their squares' sum)
+    assert (runs[0] - want).abs().max() <= 2.0 ** -6 * want.pow(2).mean().sqrt()
+
+
+@pytest.mark.parametrize("rows,columns,width", [(576, 3072, 1024), (1024, 3072, 1024), (130, 64, 2048)])
+def test_tiled_products_give_the_same_bits_in_every_run(rows, columns, width):
+    from paged_llm_rs_amd import kernels
+
+    x, w = gpu_randn(rows, width, seed=1).bfloat16(), gpu_randn(2 * columns, width, std=0.02, seed=2).bfloat16()
+    runs = [kernels.gemm_tiled(x, w, swiglu=True) for _ in range(8)]
+    both = x.float() @ w.float().T
+    want = torch.nn.functional.silu(both[:, :columns]) * both[:, columns:]
+    assert all(torch.equal(runs[0], r) for r in runs[1:])
+    assert torch.allclose(runs[0].float(), want, rtol=2.0 ** -7, atol=1e-4)       # one rounding to bfloat16, the hardware's exponential
