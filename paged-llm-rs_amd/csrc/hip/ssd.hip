@@ -503,9 +503,9 @@ __device__ __forceinline__ float ssd_q(float x, float scale) { return KIND == PL
 // summary: W tiles of 64 columns of V a workgroup, four waves each; of a tile, a wave 32 rows of N (and the 32 four further on, where N
 // has more than 128).  Both operands go through LDS, a token a row, so that a value is read and activated once a workgroup; rows there are
 // 16 values longer than they hold.  What it is bound by: the trip to memory, the activation (silu of linear attention: an exponential and a
-// division a value) and the trip back, one behind the other.  42 chunks of 8 heads of 128 by 128: SUMMARY0 us (34.4 with every wave
+// division a value) and the trip back, one behind the other.  42 chunks of 8 heads of 128 by 128: 26.4 us (34.4 with every wave
 // reading and activating all of v and a workgroup for each 64 columns and each chunk that there might be), of 4 heads of 128 by 256
-// (matrix memory) SUMMARY1 (24.5).
+// (matrix memory) 24.7 (24.5); 25 chunks of the first 17.8 (28.7).
 #define SSD_SUMMARY_PAD 16
 template <int KIND, int W>
 __global__ __launch_bounds__(256 * W) void ssd_summary_kernel(SsdArgs sa, int seqs, int aligned) {
@@ -690,8 +690,9 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
 // output: the read-outs of one chunk, head and W tiles of 64 columns.  4 W waves; wave 2 W ti + j owns the tokens 32 ti .. + 31 and, of the
 // scores, the earlier tokens 32 j .. + 31 (j < 2), of the read-outs, the columns 32 j .. + 31.  Bound by its chain (rows, scores, what the
 // state gives, what the chunk gives; three barriers), so waves without scores do the state's part meanwhile, and two workgroups share a
-// compute unit.  Two tiles a workgroup make the scores once for both: 42 chunks of 8 heads of 128 by 128 OUTPUT0 us (50.8 with a tile a
-// workgroup and one for each chunk that there might be), of 4 heads of 128 by 256 (matrix memory) OUTPUT1 (49.3).
+// compute unit.  Two tiles a workgroup make the scores once for both: 42 chunks of 8 heads of 128 by 128 44.6 us (50.8 with a tile a
+// workgroup and one for each chunk that there might be), of 4 heads of 128 by 256 (matrix memory) 40.8 (49.3), 25 chunks of the first 27.6 (40.7);
+// one tile a workgroup with the same order of loads 56.7, 52.9 and 30.8.
 // LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes, two numbers a token.
 template <int KIND, int W>
 __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, int seqs, int aligned) {
@@ -723,28 +724,52 @@ __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, 
     const int ti = wave / (2 * W), tj = wave % (2 * W);
     const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
 
-    // ---- what waits for nothing: C and B into LDS, the columns of x into registers, the first rows of S_0 ----
+    // ---- what waits for nothing: C and B into LDS, the first rows of S_0 into registers ----
+    // (every load is unconditional, from an address that is valid in any case: one in a branch would be waited for alone)
+    const int v = vt * 64 * W + 32 * tj + l32, vc = min(v, V - 1);
+    const bool columns = vt * 64 * W + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
+    // (32-bit offsets from bases that are the same for the wave: an address a load would take two registers)
+    const char* S0 = reinterpret_cast<const char*>(sa.Sin + idx * N * V);
+    auto ask = [&](int n0, float (&s0)[16]) {                         // rows n0 .. n0 + 31 of S_0, the wave's columns
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int n = n0 + 8 * (k >> 2) + 4 * half + (k & 3);
+            s0[k] = *reinterpret_cast<const float*>(S0 + 4u * static_cast<uint32_t>(min(n, N - 1) * V + vc));
+        }
+    };
+    float s_even[16], s_odd[16];
     if (aligned) {
-        const int quads = Np / 4;
-        for (int e = tid; e < SSD_CHUNK * quads; e += T) {
-            const int t = e / quads, i = 4 * (e - t * quads);
-            ssd_f32x4 cv = {0.f, 0.f, 0.f, 0.f}, bv = cv;
-            if (t < L && i < N) {
-                const float* row = rows + static_cast<size_t>(t) * a.qkv_stride + g * N + i;
-                cv = *reinterpret_cast<const ssd_f32x4*>(row + a.q_off);
-                bv = *reinterpret_cast<const ssd_f32x4*>(row + a.k_off);
+        const int quads = Np / 4, all = SSD_CHUNK * quads;
+        for (int e0 = 0; e0 < all; e0 += 4 * T) {
+            ssd_f32x4 cv[4], bv[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = min(e0 + tid + k * T, all - 1), t = e / quads, i = min(4 * (e - t * quads), N - 4);
+                const float* row = rows + static_cast<size_t>(min(t, L - 1)) * a.qkv_stride + g * N + i;
+                cv[k] = *reinterpret_cast<const ssd_f32x4*>(row + a.q_off);
+                bv[k] = *reinterpret_cast<const ssd_f32x4*>(row + a.k_off);
             }
-            if (KIND == PL_SCAN_LIGHTNING || KIND == PL_SCAN_MLSTM) {
+            if (e0 == 0) {
+                ask(0, s_even);
+                ask(32, s_odd);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int e = e0 + tid + k * T, t = e / quads, i = 4 * (e - t * quads);
+                if (e >= all) continue;
+                const bool in = t < L && i < N;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    cv[j] = ssd_q<KIND>(cv[j], q_scale);
-                    bv[j] = ssd_kv<KIND>(bv[j]);
+                    cv[k][j] = in ? ssd_q<KIND>(cv[k][j], q_scale) : 0.f;
+                    bv[k][j] = in ? ssd_kv<KIND>(bv[k][j]) : 0.f;
                 }
+                *reinterpret_cast<ssd_f32x4*>(Cs + t * P + i) = cv[k];
+                *reinterpret_cast<ssd_f32x4*>(Bs + t * P + i) = bv[k];
             }
-            *reinterpret_cast<ssd_f32x4*>(Cs + t * P + i) = cv;
-            *reinterpret_cast<ssd_f32x4*>(Bs + t * P + i) = bv;
         }
     } else {
+        ask(0, s_even);
+        ask(32, s_odd);
         for (int e = tid; e < SSD_CHUNK * Np; e += T) {
             const int t = e / Np, i = e - t * Np;
             const bool in = t < L && i < N;
@@ -753,27 +778,16 @@ __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, 
             Bs[t * P + i] = in ? ssd_kv<KIND>(row[a.k_off]) : 0.f;
         }
     }
-    const int v = vt * 64 * W + 32 * tj + l32, vc = min(v, V - 1);
-    const bool columns = vt * 64 * W + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
+    const char* x_at = reinterpret_cast<const char*>(rows + a.v_off + h * V);
+    const int last_x = min(L, 32 * ti + 32) - 1;
     float x[SSD_CHUNK / 2];                                           // x of token 8 q + 4 half + e in x[4 q + e]
+    auto ask_x = [&]() {                                              // (behind the scores, whose registers it takes)
 #pragma unroll
-    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
-        x[k] = 0.f;
-        if (columns && (k < 16 || ti == 1)) {
-            const int u = 8 * (k >> 2) + 4 * half + (k & 3);
-            x[k] = rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc];
-        }
-    }
-    const float* S0 = sa.Sin + idx * N * V + vc;
-    auto ask = [&](int n0, float (&s0)[32]) {                         // rows n0 .. n0 + 63 of S_0, the wave's columns
-#pragma unroll
-        for (int k = 0; k < 32; ++k) {
-            const int n = n0 + 8 * (k >> 2) + 4 * half + (k & 3);
-            s0[k] = S0[static_cast<size_t>(min(n, N - 1)) * V];
+        for (int k = 0; k < SSD_CHUNK / 2; ++k) {
+            const int u = 8 * (k >> 2) + 4 * half + (k & 3);          // (the tokens behind its own a wave of the first half does not use)
+            x[k] = *reinterpret_cast<const float*>(x_at + 4u * static_cast<uint32_t>(min(u, last_x) * a.qkv_stride + vc));
         }
     };
-    float s0[32];
-    if (columns) ask(0, s0);
     if (wave == 0) {
         double b, dt;
         ssd_gates<KIND>(a, h, row0, L, lane, b, dt);
@@ -805,27 +819,32 @@ __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, 
     for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;
     auto state_part = [&]() {                                         // S_0^T C_t, times e^(b_t)
         const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
-        for (int n0 = 0; n0 < Np; n0 += 64) {
-            float now[32];
+        auto take = [&](int n0, const float (&s0)[16]) {
 #pragma unroll
-            for (int k = 0; k < 32; ++k) now[k] = s0[k];
-            if (n0 + 64 < Np) ask(n0 + 64, s0);
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < 4; ++q) {
                 if (n0 + 8 * q < Np) {
                     const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + n0 + 8 * q);   // (zeros past N)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        if (q % 2 == 0) y = ssd_mfma(cv[e], now[4 * q + e], y);
-                        else y2 = ssd_mfma(cv[e], now[4 * q + e], y2);
+                        if (q % 2 == 0) y = ssd_mfma(cv[e], s0[4 * q + e], y);
+                        else y2 = ssd_mfma(cv[e], s0[4 * q + e], y2);
                     }
                 }
             }
+        };
+        for (int n0 = 0; n0 < Np; n0 += 64) {                         // (past N the last row again)
+            take(n0, s_even);
+            ask(n0 + 64, s_even);
+            take(n0 + 32, s_odd);
+            ask(n0 + 96, s_odd);
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) y[r] = (y[r] + y2[r]) * before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
     };
-    if (columns && !scored) state_part();
+    if (columns && !scored) {
+        ask_x();
+        state_part();
+    }
     ssd_f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -852,7 +871,10 @@ __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, 
 #pragma unroll
         for (int r = 0; r < 16; ++r) As[(32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)) * PA + 32 * tj + l32] = acc[r];
     }
-    if (columns && scored) state_part();
+    if (columns && scored) {
+        ask_x();
+        state_part();
+    }
     __syncthreads();                                                  // the weighted scores are written
     if (KIND == PL_SCAN_MLSTM) {
         // n . q of a token, by four lanes: the weighted scores' sum and e^(m_0 - c_t) (n_0 . q_t)

@@ -617,3 +617,41 @@ def test_token_by_token_scans_give_the_same_bits_however_the_tokens_are_cut(kind
             assert torch.equal(run(state, rows[at], gates[at], [1], [slot])[0], want[t]), (slot, t)
         begin += count
     assert torch.equal(state[:, :floats], together[:, :floats])
+
+
+# --- chunks of requests dealt to workgroups --------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("kind,H,D,V", [("lightning", 2, 128, 128), ("lightning", 1, 40, 72), ("lightning", 2, 256, 200), ("mlstm", 2, 64, 256),
+                                        ("mlstm", 1, 100, 36), ("delta", 2, 128, 64)])
+def test_chunks_of_many_requests_are_those_of_each_alone(kind, H, D, V):
+    """A step of 70 requests (more than a wave counts at a time), most of them without a chunk, rows of padding behind them: every
+    request's read-out and state are those of a step of its own.  Head sizes on both sides of the tiles of 64 and 128 columns."""
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator().manual_seed(7)
+    counts = [[1, 64, 2, 129, 15, 16][i % 6] if i % 7 == 0 or i in (63, 64, 69) else 1 for i in range(70)]
+    n, pad = sum(counts), 37
+    width = H * (2 * D + V) + 2 * H
+    rows = torch.randn(n + pad, width, generator=g).cuda() * 0.5
+    p1 = torch.linspace(0.9, 0.99, H, device="cuda:0") if kind == "lightning" else torch.linspace(-1.0, 0.5, H, device="cuda:0")
+    p2 = torch.linspace(1.0, 2.0, H, device="cuda:0")
+    floats = kernels.scan_state_floats(kind, H, D, V)
+    before = torch.randn(70, floats, generator=g).cuda() * 0.1 if kind != "mlstm" else torch.zeros(70, floats, device="cuda:0")
+
+    def scan(rows, counts, state, padding=0):
+        step = ScanStep(counts, range(len(counts)), padding)
+        step.max_q_len = step.num_tokens                # (as a padded step says it)
+        return kernels.recurrent_scan(kind, rows, 0, H * D, 2 * H * D, state, step, H, H, D, V, gates=None if kind == "lightning" else rows,
+                                      g1_off=width - 2 * H, g2_off=width - H, p1=p1, p2=None if kind == "lightning" else p2, cap=15.0,
+                                      chunked=True)
+
+    state = before.clone()
+    together = scan(rows, counts, state, pad)[:n]
+    first = 0
+    for s, count in enumerate(counts):
+        if count >= 15 or s in (1, 68):
+            alone = before[s:s + 1].clone()
+            out = scan(rows[first:first + count].contiguous(), [count], alone)
+            assert torch.equal(out, together[first:first + count]), (s, count)
+            assert torch.equal(alone[0], state[s]), (s, count)
+        first += count
