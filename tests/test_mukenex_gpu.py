@@ -628,3 +628,28 @@ def test_the_command_line_generates_with_the_design(tmp_path):
     assert done.returncode == 0, done.stderr[-2000:]
     lines = [json.loads(x) for x in done.stdout.splitlines() if x.startswith("{")]
     assert len(lines) == 2 and all(len(x["tokens"]) == 5 for x in lines), done.stdout
+
+
+# --- several copies of the stream ------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("copies", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("width", [6, 64, 1020, 4096, 4100])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_pass_over_the_copies_for_every_number_and_width(copies, width, dtype):
+    """Numbers of copies with and without an instance of their own, widths of one round and of more, with and without a norm."""
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator().manual_seed(copies * 1000 + width)
+    draw = lambda *shape: torch.randn(*shape, generator=g).cuda()
+    rows, eps = 3, 1e-5
+    streams, y, gain = draw(rows, copies * width), draw(rows, width), draw(width)
+    mix, out, read = draw(copies, copies), draw(copies), draw(copies)
+    x = streams.double().view(rows, copies, width)
+    want = torch.einsum("st,nsw->ntw", mix.double(), x) + out.double()[None, :, None] * y.double()[:, None]
+    u = torch.einsum("s,nsw->nw", read.double(), want)
+    normed = u / (u.pow(2).mean(-1, keepdim=True) + eps).sqrt() * gain.double()
+    got = kernels.hc_step(streams, copies, y=y, mix=mix, out=out, read=read, gain=gain, eps=eps, read_dtype=dtype)
+    # sums of up to nine products, and of `width` squares, in 32 bits
+    bound = (16 + width ** 0.5) * 2.0 ** -24
+    assert (streams.view_as(want) - want).abs().max() <= bound * want.abs().max()
+    assert (got.double() - normed).abs().max() <= (bound + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * normed.abs().max()
