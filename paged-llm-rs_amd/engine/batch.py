@@ -52,6 +52,7 @@ class StepBatch:
         self.num_logit_rows = num_logit_rows
         self.max_q_len = max_q_len
         self.max_ctx_len = max_ctx_len
+        self.near_ctx_len = max_ctx_len  # (``near_context`` where the contexts themselves are known)
         self.seq_ids = seq_ids
         # On the host: the tokens every live request brings; whether the step reports bounds instead of
         # counts (a padded step does); and, for such a step, {limit: the most tokens that requests of fewer
@@ -125,6 +126,17 @@ def context_bound(longest: int) -> int:
             return bound + bound // 2
         bound *= 2
     return bound
+
+
+def near_context(longest: int) -> int:
+    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens.  A fresh prompt of a few
+    dozen tokens has one tile of keys: dealt out by a bound of 1,024 it had four workgroups a tile, three without a key, and a
+    second launch to put them together (0.6B shape, a step: 37 tokens 1,385 to 1,301 us, 256 tokens 2,334 to 2,260; 37 tokens behind 700 others, whose
+    keys are worth sharing, stay as they were).  A step's shape names it, so a captured step is replayed for contexts like its own."""
+    bound = 128
+    while bound < longest and bound < 1024:
+        bound *= 2
+    return bound if bound >= longest else context_bound(longest)
 
 
 class CannotFeed(Exception):
@@ -266,6 +278,7 @@ def build_batch(entries, manager, num_groups: int, vocab_size: int, max_position
         ctx_bound = context_bound(longest)
     if longest > ctx_bound:
         raise ContextTooLong(f"a context of {longest} tokens in a step laid out for {ctx_bound}")
+    near = min(near_context(longest), ctx_bound)
     longest = ctx_bound
     each = q_len[:len(entries)]
     if pad_to is not None:
@@ -278,6 +291,9 @@ def build_batch(entries, manager, num_groups: int, vocab_size: int, max_position
         batch = StepBatch(packed, layout, n, S, max_blocks, len(logit_rows), n, longest,
                           [e.seq_id for e in entries], tokens_each=each, padded=True, short_bounds=short_bounds)
         batch.live_seqs = S - 1
+        batch.near_ctx_len = near
         return batch
-    return StepBatch(packed, layout, n, S, max_blocks, len(logit_rows), int(q_len.max()), longest,
-                     [e.seq_id for e in entries], tokens_each=each)
+    batch = StepBatch(packed, layout, n, S, max_blocks, len(logit_rows), int(q_len.max()), longest,
+                      [e.seq_id for e in entries], tokens_each=each)
+    batch.near_ctx_len = near
+    return batch

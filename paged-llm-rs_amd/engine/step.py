@@ -35,7 +35,7 @@ import torch
 
 from .. import kernels
 from ..errors import ConfigError, PagedLLMError, TensorError
-from .batch import CannotFeed, CaptureOutgrown, StepBatch, TableTooWide, build_batch, context_bound, token_bucket
+from .batch import CannotFeed, CaptureOutgrown, StepBatch, TableTooWide, build_batch, context_bound, near_context, token_bucket
 
 GRAPH_MAX_REQUESTS = 256     # requests a captured step may have (steps of more run kernel by kernel)
 SHAPE_GRAPH_ROWS_KEPT = 32768    # rows over all captured shapes of steps other than plain decoding (the
@@ -312,7 +312,7 @@ class ShapeGraph:
         self.batch = StepBatch(self.device_buf, first.layout, first.num_tokens, first.num_seqs, list(widths),
                                first.num_logit_rows, first.max_q_len, ctx_bound, [],
                                tokens_each=first.tokens_each, padded=True, short_bounds=first.short_bounds)
-        self.batch.live_seqs = first.live_seqs
+        self.batch.live_seqs, self.batch.near_ctx_len = first.live_seqs, first.near_ctx_len
         self.graph = None
         self.logits = None
 
@@ -388,7 +388,9 @@ class StepRunner:
         if not self.use_graphs or rows is None or len(entries) > GRAPH_MAX_REQUESTS:
             self.eager_steps += 1
             return StepOutput(run_step(self.model, self.cache, entries, pad_to=rows, short_bounds=short_bounds))
-        shape = (rows, len(entries), sum(len(e.want) for e in entries), tuple(sorted(short_bounds.items())))
+        longest = max(e.start + len(e.tokens) for e in entries)
+        shape = (rows, len(entries), sum(len(e.want) for e in entries), tuple(sorted(short_bounds.items())),
+                 min(near_context(longest), context_bound(1)))
         known = shape in self._shapes
         graph = self._shapes.pop(shape, None)
         if not known:
@@ -407,7 +409,6 @@ class StepRunner:
             except CaptureOutgrown:
                 pass                            # a request has outgrown the capture: a new one below
         widths = [_bucket(w + 1, 32) for w in self._widths_needed(entries)]
-        longest = max(e.start + len(e.tokens) for e in entries)
         graph = ShapeGraph(self.model, self.cache, entries, widths, context_bound(longest), rows, short_bounds)
         out = graph.run(entries)
         self._shapes[shape] = graph

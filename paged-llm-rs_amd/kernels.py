@@ -880,7 +880,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
                      and not grouped_applies(nq, nkv, d, kv.block_size))   # (grouped, a token reads its keys once for all its heads)
         paged_attention_prefill(qkv, stride, out, batch.q_start, batch.q_len, batch.ctx_len, batch.max_q_len,
                                 kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window,
-                                short_limit=0 if all_tiled else SHORT_PORTION, max_ctx=batch.max_ctx_len,
+                                short_limit=0 if all_tiled else SHORT_PORTION,
+                                max_ctx=getattr(batch, "near_ctx_len", batch.max_ctx_len),
                                 live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more)
         if short_tokens == 0 or all_tiled:
             return out

@@ -88,3 +88,18 @@ def test_steps_of_one_shape_have_one_layout():
     two = build_batch(requests(b, [13, 30], written=[50, 0]), b, 1, 100, 0, "cpu", widths=[32], ctx_bound=1024, pad_to=64)
     assert one.layout == two.layout and one.packed.numel() == two.packed.numel()
     assert (one.max_q_len, one.tokens_of_short_requests(16), one.num_seqs) == (two.max_q_len, two.tokens_of_short_requests(16), two.num_seqs)
+
+
+def test_a_step_says_how_near_its_contexts_are():
+    """Bounds from 128 on for what shares a prompt's keys out, those of ``context_bound`` past 1,024, and never more than the step was
+    laid out for."""
+    from paged_llm_rs_amd.engine.batch import near_context
+
+    assert [near_context(n) for n in (1, 128, 129, 256, 257, 513, 1024, 1025, 1537)] == [128, 128, 256, 256, 512, 1024, 1024, 1536, 2048]
+    m = manager()
+    assert build_batch(requests(m, [5, 1, 20], written=[0, 9, 3]), m, 1, 100, 0, "cpu").near_ctx_len == 128
+    m = manager()
+    padded = build_batch(requests(m, [40, 1], written=[0, 7]), m, 1, 100, 0, "cpu", widths=[32], ctx_bound=1024, pad_to=64)
+    assert (padded.near_ctx_len, padded.max_ctx_len) == (128, 1024)
+    m = manager()
+    assert build_batch(requests(m, [40], written=[0]), m, 1, 100, 0, "cpu", ctx_bound=64).near_ctx_len == 64
