@@ -59,6 +59,7 @@ def _signatures(lib) -> None:
         "pl_gemm_tiled_applies": [i, i, i, i],
         "pl_gemm_stream": [p, p, p, p, i, i, i, i, i, i, i, p],
         "pl_gemm_stream_splits": [i, i, i, i],
+        "pl_gemm_wide": [p, p, p, i, i, i, p],
         "pl_gemm_finish": [p, p, ctypes.c_longlong, i, i, i, i, i, p],
         "pl_paged_attention_decode": [p, i, p, p, p, p, p, p, i, i, i, p, i, i, p, p, i, i, i, i, f, i, i,
                                       i, p, p, i, f, p, p, i, p, p, f, i, p, i, p, p],
@@ -1129,6 +1130,29 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
     return out
 
 
+# Where the product over strips and very many columns beats the others (gemm_wide.hip has the times of both sides).
+WIDE_ROWS, WIDE_FEW_ROWS = 32, 16
+WIDE_K, WIDE_FEW_K = 2048, 4097        # the narrowest streams, with 17 to 32 rows and with fewer
+WIDE_COLUMNS = 131072
+
+
+def wide_wins(rows: int, weight_rows: int, width: int, strips: bool) -> bool:
+    return (strips and 0 < rows <= WIDE_ROWS and weight_rows >= WIDE_COLUMNS and weight_rows % 16 == 0 and width % 32 == 0
+            and WIDE_K <= width <= 1 << 20 and (rows > WIDE_FEW_ROWS or width >= WIDE_FEW_K))
+
+
+def gemm_wide(x: torch.Tensor, strips: torch.Tensor) -> torch.Tensor:
+    """y = x . w^T (32-bit) for up to 32 rows of bfloat16 over very many columns, out of the weights in strips
+    (``weights_in_strips``) alone."""
+    _need(x, "matrix product input", None, torch.bfloat16)
+    _need(strips, "weights in strips", None, torch.bfloat16)
+    if x.dim() != 2 or strips.dim() != 2 or strips.shape[1] != x.shape[1]:
+        raise TensorError(f"weight has shape {tuple(strips.shape)} for an input of shape {tuple(x.shape)}")
+    out = torch.empty((x.shape[0], strips.shape[0]), dtype=torch.float32, device=x.device)
+    _check(library().pl_gemm_wide(x.data_ptr(), strips.data_ptr(), out.data_ptr(), x.shape[0], strips.shape[0], x.shape[1], _stream()))
+    return out
+
+
 STREAM_ROWS = 64
 # Where the streamed product beats both the library and the skinny kernel (each timed over weights from
 # memory, at 8 to 64 rows).  The library cuts a deep product over few columns badly (5,120 x 25,600 at 64
@@ -1285,6 +1309,8 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
     _need(w, "weight", None, torch.bfloat16)
     if out_dtype == torch.float32:
         # the projection onto the vocabulary: 32-bit out of the 32-bit sums, from either product
+        if wide_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
+            return gemm_wide(x, _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16))
         if stream_wins(x.shape[0], w.shape[0], x.shape[1]):
             return gemm_stream(x, w, torch.float32)
         if skinny_applies(x) and x.shape[1] <= (SKINNY_F32_FEW_K if x.shape[0] <= 16 else SKINNY_SHALLOW_K):

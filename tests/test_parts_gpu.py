@@ -1458,3 +1458,25 @@ def test_tiled_products_give_the_same_bits_in_every_run(rows, columns, width):
     want = torch.nn.functional.silu(both[:, :columns]) * both[:, columns:]
     assert all(torch.equal(runs[0], r) for r in runs[1:])
     assert torch.allclose(runs[0].float(), want, rtol=2.0 ** -7, atol=1e-4)       # one rounding to bfloat16, the hardware's exponential
+
+
+# --- few rows over very many columns -----------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("N,K", [(16, 32), (144, 64), (128, 416), (2064, 2080), (131072, 2048)])
+def test_the_wide_product_out_of_strips(N, K):
+    """Fewer steps than waves, a wave without steps, stretches that are no whole rounds, one strip, a last workgroup of one; a row's bits are
+    the same among 1, 16, 17 and 32 rows."""
+    from paged_llm_rs_amd import kernels
+
+    x, w = gpu_randn(32, K, seed=1).bfloat16(), gpu_randn(N, K, std=K ** -0.5, seed=2).bfloat16()
+    strips = kernels.weights_in_strips(w)
+    whole = kernels.gemm_wide(x, strips)
+    want = x.float() @ w.float().T
+    # 32-bit sums of K exact products, in another order
+    assert (whole - want).abs().max() <= 4 * K ** 0.5 * 2.0 ** -24 * want.abs().max()
+    for n in (1, 16, 17):
+        assert torch.equal(kernels.gemm_wide(x[:n].contiguous(), strips), whole[:n])
+        got = kernels.linear_bf16(x[:n].contiguous(), w, torch.float32, strips)
+        assert (got - want[:n]).abs().max() <= 8 * K ** 0.5 * 2.0 ** -24 * want.abs().max()
+    with pytest.raises(Exception):
+        kernels.gemm_wide(torch.cat([x, x]), strips)
