@@ -1610,10 +1610,11 @@ class SlotTable:
 
 def clear_slots(table: SlotTable, slots) -> None:
     """Zeros in the given slots of every layer's state, in one launch."""
-    slots = list(slots)
+    slots = [int(slot) for slot in slots]
     for slot in slots:
-        if not 0 <= slot < table.slots:
+        if not -table.slots <= slot < table.slots:
             raise IndexError(f"state slot {slot} of {table.slots}")
+    slots = [slot % table.slots for slot in slots]        # (a negative one counts from the end, as a tensor's index does)
     if table.table is None or not slots:
         return
     _check(library().pl_clear_slots(table.table.data_ptr(), len(table.states), table.largest, (c_int * len(slots))(*slots), len(slots),

@@ -1319,7 +1319,7 @@ def test_a_context_of_thousands_of_tokens_in_portions_and_decoded(model_dirs, na
 # --- state slots of requests that begin --------------------------------------------------------------------------
 
 @pytest.mark.parametrize("shapes", [[(3,), (1024,), (7, 5)], [(16384,)], [(4,), (70001,)]])
-@pytest.mark.parametrize("slots", [[0], [68, 3, 5], list(range(1, 67))])
+@pytest.mark.parametrize("slots", [[0], [68, 3, 5], [-1, 2], list(range(1, 67))])
 def test_clearing_state_slots_touches_these_slots_of_every_layer_only(shapes, slots):
     """One launch clears the slots of all layers: sizes that are and are not whole groups of 16 bytes, more slots than a
     launch carries; the slots beside them keep every value."""
