@@ -51,7 +51,12 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaArgs da, int Dp
     const int D = a.D, H = a.H;
     const int h = blockIdx.y;
     ChunkPlace place;
-    if (!find_chunk(a, seqs, blockIdx.x, place)) return;
+    if (seqs > 0) {
+        if (!find_chunk(a, seqs, blockIdx.x, place)) return;
+    } else {
+        place = {static_cast<int>(blockIdx.z), static_cast<int>(blockIdx.x), a.q_len[blockIdx.z], a.q_start[blockIdx.z]};
+        if (a.state_slots[place.s] < 0 || place.count < a.below || place.c * DL_C >= place.count) return;
+    }
     const int c_at = place.c, s = place.s, n = place.count;
     const int L = min(DL_C, n - c_at * DL_C), row0 = place.first_row + c_at * DL_C;
     const int g = h / (H / a.G);
@@ -363,7 +368,9 @@ static int launch_delta(const DeltaArgs& da, int rows, int seqs, int max_q_len, 
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prepare_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(lds_p));
     PL_REQUIRE(e == hipSuccess, "delta_chunked: %zu bytes of LDS refused: %s", lds_p, hipGetErrorString(e));
-    delta_prepare_kernel<<<dim3(chunk_bound(rows, max_q_len, seqs), a.H), 256, lds_p, stream>>>(da, Dp, seqs);
+    // (with three requests or more a workgroup for each chunk that there can be; below that the longest's chunks for every request)
+    if (seqs >= 3) delta_prepare_kernel<<<dim3(chunk_bound(rows, max_q_len, seqs), a.H), 256, lds_p, stream>>>(da, Dp, seqs);
+    else delta_prepare_kernel<<<dim3(pl_ceil_div(max_q_len, DL_C), a.H, seqs), 256, lds_p, stream>>>(da, Dp, 0);
     PL_CHECK_LAUNCH("delta_chunked (prepare)");
     // the workgroups of one head read the same chunks: with heads and requests along x they share a chiplet's cache wherever those are a
     // multiple of the eight chiplets

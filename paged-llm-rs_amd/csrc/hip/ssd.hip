@@ -500,19 +500,108 @@ __device__ __forceinline__ float ssd_q(float x, float scale) { return KIND == PL
 //     y_t = (sum_{u<=t} e^(w_u - b_u - c_t) (q_t . k_u) v_u + e^(m_0 - c_t) S_0^T q_t) / max(|n . q|, e^(-m_t)),  c_t = m_t - b_t,
 // with n . q the same sum without v_u and S_0.)
 
-// summary: W tiles of 64 columns of V a workgroup, four waves each; of a tile, a wave 32 rows of N (and the 32 four further on, where N
+// summary: a wave a tile of 32 rows of N (and the tile four further on, where N has more than 128), 64 columns of V.
+// Both operands come straight from memory, a token a row: 128 bytes a half wave.
+template <int KIND>
+__global__ __launch_bounds__(256) void ssd_summary_kernel(SsdArgs sa) {
+    const ScanArgs& a = sa.a;
+    __shared__ float weight[SSD_CHUNK];
+    const int N = a.D, V = a.V, H = a.H;
+    const int tiles = (V + 63) / 64;
+    const int c = blockIdx.x, h = blockIdx.y / tiles, vt = blockIdx.y % tiles, s = blockIdx.z;
+    const int slot = a.state_slots[s], count = a.q_len[s];
+    if (slot < 0 || count < a.below || c * SSD_CHUNK >= count) return;
+    const int L = min(SSD_CHUNK, count - c * SSD_CHUNK), row0 = a.q_start[s] + c * SSD_CHUNK;
+    const size_t idx = static_cast<size_t>(ssd_chunk(a, s, c)) * H + h;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int g = h / (H / a.G);
+    const bool two = vt * 64 + 32 < V;               // whether the second 32 columns exist
+    const int va = min(vt * 64 + l32, V - 1), vb = min(vt * 64 + 32 + l32, V - 1);
+    float xa[SSD_CHUNK / 2], xb[SSD_CHUNK / 2];
+    const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
+    // (every load before the first silu: one behind a branch would be waited for alone)
+#pragma unroll
+    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
+        const float* x = rows + static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.v_off + h * V;
+        xa[k] = x[va];
+        xb[k] = x[vb];
+    }
+    if (wave == 0) {
+        double b, dt;
+        const double end = ssd_gates<KIND>(a, h, row0, L, lane, b, dt);
+        if (KIND == PL_SCAN_MLSTM) {
+            double top = dt;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) top = fmax(top, __shfl_xor(top, off, 64));
+            weight[lane] = expf(static_cast<float>(dt - top));
+            if (vt == 0 && lane == 0) {
+                // (their sum: either may be hundreds where it is small, and rounded alone would leave its rounding in the state)
+                sa.tops[2 * idx] = static_cast<float>(end + top);
+                // the maximum that the request's first chunk starts from: the carry reads it here, not in the slot it writes
+                if (c == 0) sa.tops[2 * idx + 1] = a.state[static_cast<size_t>(slot) * a.state_stride + a.m_off + h * tiles];
+            }
+        } else {
+            weight[lane] = expf(static_cast<float>(end - b)) * static_cast<float>(dt);  // (zero past the chunk's tokens)
+        }
+        if (vt == 0 && lane == 0) sa.ends[idx] = static_cast<float>(end);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
+        const float w = weight[2 * k + half];
+        xa[k] = ssd_kv<KIND>(xa[k]) * w;
+        xb[k] = ssd_kv<KIND>(xb[k]) * w;
+    }
+    float* U = sa.U + idx * N * V;
+    for (int n0 = wave * 32; n0 < N; n0 += 128) {
+        const int n = min(n0 + l32, N - 1);
+        float ka[SSD_CHUNK / 2];
+#pragma unroll
+        for (int k = 0; k < SSD_CHUNK / 2; ++k)
+            ka[k] = rows[static_cast<size_t>(min(2 * k + half, L - 1)) * a.qkv_stride + a.k_off + g * N + n];
+        if (KIND == PL_SCAN_LIGHTNING) {
+#pragma unroll
+            for (int k = 0; k < SSD_CHUNK / 2; ++k) ka[k] = ssd_kv<KIND>(ka[k]);
+        }
+        if (KIND == PL_SCAN_MLSTM && vt == 0) {
+            float sum = 0.f;
+#pragma unroll
+            for (int k = 0; k < SSD_CHUNK / 2; ++k) sum += weight[2 * k + half] * ka[k];
+            sum += __shfl_xor(sum, 32, 64);
+            if (half == 0 && n0 + l32 < N) sa.Uk[idx * N + n0 + l32] = sum;
+        }
+        ssd_f32x16 da, db;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) da[r] = db[r] = 0.f;
+#pragma unroll
+        for (int k = 0; k < SSD_CHUNK / 2; ++k) {
+            da = ssd_mfma(ka[k], xa[k], da);
+            if (two) db = ssd_mfma(ka[k], xb[k], db);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = n0 + 8 * (r >> 2) + 4 * half + (r & 3);
+            if (row >= N) continue;
+            if (vt * 64 + l32 < V) U[static_cast<size_t>(row) * V + vt * 64 + l32] = da[r];
+            if (vt * 64 + 32 + l32 < V) U[static_cast<size_t>(row) * V + vt * 64 + 32 + l32] = db[r];
+        }
+    }
+}
+
+// summary_pair, the same for two tiles of 64 columns of V a workgroup, four waves each; of a tile, a wave 32 rows of N (and the 32 four further on, where N
 // has more than 128).  Both operands go through LDS, a token a row, so that a value is read and activated once a workgroup; rows there are
 // 16 values longer than they hold.  What it is bound by: the trip to memory, the activation (silu of linear attention: an exponential and a
 // division a value) and the trip back, one behind the other.  42 chunks of 8 heads of 128 by 128: 26.4 us (34.4 with every wave
 // reading and activating all of v and a workgroup for each 64 columns and each chunk that there might be), of 4 heads of 128 by 256
 // (matrix memory) 24.7 (24.5); 25 chunks of the first 17.8 (28.7).
 #define SSD_SUMMARY_PAD 16
-template <int KIND, int W>
-__global__ __launch_bounds__(256 * W) void ssd_summary_kernel(SsdArgs sa, int seqs, int aligned) {
+template <int KIND>
+__global__ __launch_bounds__(512) void ssd_summary_pair_kernel(SsdArgs sa, int seqs, int aligned) {
     const ScanArgs& a = sa.a;
     __shared__ float weight[SSD_CHUNK];
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    constexpr int T = 256 * W, COLS = 64 * W, XP = COLS + SSD_SUMMARY_PAD;
+    constexpr int T = 512, COLS = 128, XP = COLS + SSD_SUMMARY_PAD;
     const int N = a.D, V = a.V, H = a.H;
     const int tiles = (V + COLS - 1) / COLS;
     const int h = blockIdx.y / tiles, vt = blockIdx.y % tiles;
@@ -687,20 +776,231 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsdArgs sa) {
     if (KIND == PL_SCAN_MLSTM && e < tiles) slot_state[a.m_off + h * tiles + e] = m;
 }
 
-// output: the read-outs of one chunk, head and W tiles of 64 columns.  4 W waves; wave 2 W ti + j owns the tokens 32 ti .. + 31 and, of the
+// output: the read-outs of one chunk, head and tile of 64 columns.  Four waves; wave 2 ti + j owns the tokens 32 ti .. + 31 and, of the
+// scores, the earlier tokens 32 j .. + 31, of the read-outs, the columns 32 j .. + 31.
+// LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes, two numbers a token.
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void ssd_output_kernel(SsdArgs sa, int aligned) {
+    const ScanArgs& a = sa.a;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int N = a.D, V = a.V, H = a.H;
+    const int tiles = (V + 63) / 64;
+    const int c = blockIdx.x, h = blockIdx.y / tiles, vt = blockIdx.y % tiles, s = blockIdx.z;
+    const int slot = a.state_slots[s], count = a.q_len[s];
+    if (slot < 0 || count < a.below || c * SSD_CHUNK >= count) return;
+    const int L = min(SSD_CHUNK, count - c * SSD_CHUNK), row0 = a.q_start[s] + c * SSD_CHUNK;
+    const size_t idx = static_cast<size_t>(ssd_chunk(a, s, c)) * H + h;
+    const int g = h / (H / a.G);
+    const int Np = (N + 7) & ~7, P = Np + 4;
+    constexpr int PA = SSD_CHUNK + 4;
+    // mlstm: bd holds c_t, dtd the w_u - b_u, before_w what multiplies S_0^T q_t, below what the read-out is divided by
+    double* bd = reinterpret_cast<double*>(lds);
+    double* dtd = bd + SSD_CHUNK;
+    float* before_w = lds + 4 * SSD_CHUNK;
+    float* below = before_w + SSD_CHUNK;
+    float* Cs = below + SSD_CHUNK;
+    const float q_scale = 1.f / sqrtf(static_cast<float>(N));
+    float* Bs = Cs + SSD_CHUNK * P;
+    float* As = Bs;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int ti = wave >> 1, tj = wave & 1;
+    const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
+
+    // ---- what waits for nothing: C and B into LDS, the columns of x into registers, the first rows of S_0 ----
+    if (aligned) {
+        const int quads = Np / 4;
+        for (int e = tid; e < SSD_CHUNK * quads; e += 256) {
+            const int t = e / quads, i = 4 * (e - t * quads);
+            ssd_f32x4 cv = {0.f, 0.f, 0.f, 0.f}, bv = cv;
+            if (t < L && i < N) {
+                const float* row = rows + static_cast<size_t>(t) * a.qkv_stride + g * N + i;
+                cv = *reinterpret_cast<const ssd_f32x4*>(row + a.q_off);
+                bv = *reinterpret_cast<const ssd_f32x4*>(row + a.k_off);
+            }
+            if (KIND == PL_SCAN_LIGHTNING || KIND == PL_SCAN_MLSTM) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    cv[j] = ssd_q<KIND>(cv[j], q_scale);
+                    bv[j] = ssd_kv<KIND>(bv[j]);
+                }
+            }
+            *reinterpret_cast<ssd_f32x4*>(Cs + t * P + i) = cv;
+            *reinterpret_cast<ssd_f32x4*>(Bs + t * P + i) = bv;
+        }
+    } else {
+        for (int e = tid; e < SSD_CHUNK * Np; e += 256) {
+            const int t = e / Np, i = e - t * Np;
+            const bool in = t < L && i < N;
+            const float* row = rows + static_cast<size_t>(in ? t : 0) * a.qkv_stride + g * N + (in ? i : 0);
+            Cs[t * P + i] = in ? ssd_q<KIND>(row[a.q_off], q_scale) : 0.f;
+            Bs[t * P + i] = in ? ssd_kv<KIND>(row[a.k_off]) : 0.f;
+        }
+    }
+    const int v = vt * 64 + 32 * tj + l32, vc = min(v, V - 1);
+    const bool columns = vt * 64 + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
+    float x[SSD_CHUNK / 2];                                           // x of token 8 q + 4 half + e in x[4 q + e]
+#pragma unroll
+    for (int k = 0; k < SSD_CHUNK / 2; ++k) {
+        x[k] = 0.f;
+        if (columns && (k < 16 || ti == 1)) {
+            const int u = 8 * (k >> 2) + 4 * half + (k & 3);
+            x[k] = rows[static_cast<size_t>(min(u, L - 1)) * a.qkv_stride + a.v_off + h * V + vc];
+        }
+    }
+    const float* S0 = sa.Sin + idx * N * V + vc;
+    auto ask = [&](int n0, float (&s0)[32]) {                         // rows n0 .. n0 + 63 of S_0, the wave's columns
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            const int n = n0 + 8 * (k >> 2) + 4 * half + (k & 3);
+            s0[k] = S0[static_cast<size_t>(min(n, N - 1)) * V];
+        }
+    };
+    float s0[32];
+    if (columns) ask(0, s0);
+    if (wave == 0) {
+        double b, dt;
+        ssd_gates<KIND>(a, h, row0, L, lane, b, dt);
+        if (KIND == PL_SCAN_MLSTM) {
+            const double m0 = sa.tops[2 * idx + 1];
+            double top = fmax(m0, dt);
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const double other = __shfl_up(top, off, 64);
+                if (lane >= off) top = fmax(top, other);
+            }
+            before_w[lane] = expf(static_cast<float>(m0 - top));
+            below[lane] = static_cast<float>(-(b + top));               // -m_t, until the weighted scores are there
+            b = top;
+        } else {
+            before_w[lane] = expf(static_cast<float>(b));
+        }
+        bd[lane] = b;
+        dtd[lane] = dt;
+    }
+    __syncthreads();
+
+    // ---- the scores C_t . B_u of a tile of 32 by 32 (the tile of later tokens against earlier ones is all hidden) ----
+    const bool scored = tj <= ti && 32 * ti < L;
+    ssd_f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (scored) {
+        const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
+        const float* ba = Bs + (32 * tj + l32) * P + 4 * half;
+        for (int q = 0; q < Np; q += 8) {
+            const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + q), bv = *reinterpret_cast<const ssd_f32x4*>(ba + q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = ssd_mfma(cv[e], bv[e], acc);
+        }
+        const int u = 32 * tj + l32;
+        const double bu = bd[u], du = dtd[u];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int t = 32 * ti + 8 * (r >> 2) + 4 * half + (r & 3);
+            const float w = KIND == PL_SCAN_MLSTM ? expf(static_cast<float>(du - bd[t]))
+                                                  : expf(static_cast<float>(bd[t] - bu)) * static_cast<float>(du);
+            acc[r] = (u <= t && t < L) ? acc[r] * w : 0.f;
+        }
+    }
+    __syncthreads();                                                  // nobody reads B any more
+    if (scored) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) As[(32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)) * PA + 32 * tj + l32] = acc[r];
+    }
+    // ---- S_0^T C_t, times e^(b_t) ----
+    // (in two chains, and the chunk's own part below in one of its own: half the roundings, each of its part's size.  Linear attention
+    // with heads of 256, against 64 bits: 1.2e-7 to 1.5e-7; everything in one chain 1.5e-7 to 2.5e-7)
+    ssd_f32x16 y, y2;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[r] = y2[r] = 0.f;
+    if (columns) {
+        const float* ca = Cs + (32 * ti + l32) * P + 4 * half;
+        for (int n0 = 0; n0 < Np; n0 += 64) {
+            float now[32];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) now[k] = s0[k];
+            if (n0 + 64 < Np) ask(n0 + 64, s0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                if (n0 + 8 * q < Np) {
+                    const ssd_f32x4 cv = *reinterpret_cast<const ssd_f32x4*>(ca + n0 + 8 * q);   // (zeros past N)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (q % 2 == 0) y = ssd_mfma(cv[e], now[4 * q + e], y);
+                        else y2 = ssd_mfma(cv[e], now[4 * q + e], y2);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] = (y[r] + y2[r]) * before_w[32 * ti + 8 * (r >> 2) + 4 * half + (r & 3)];
+    }
+    __syncthreads();                                                  // the weighted scores are written
+    if (KIND == PL_SCAN_MLSTM) {
+        // n . q of a token, by four lanes: the weighted scores' sum and e^(m_0 - c_t) (n_0 . q_t)
+        const int t = tid >> 2, part = tid & 3;
+        float sum = 0.f, dot = 0.f;
+        if (t < L) {
+            const float* n0 = sa.nin + idx * N;
+            for (int u = part; u <= t; u += 4) sum += As[t * PA + u];
+            for (int i = part; i < N; i += 4) dot += n0[i] * Cs[t * P + i];
+        }
+        sum += before_w[t] * dot;
+        sum += __shfl_xor(sum, 1, 64);
+        sum += __shfl_xor(sum, 2, 64);
+        if (part == 0) below[t] = 1.f / (fmaxf(fabsf(sum), expf(below[t])) + 1e-6f);
+        __syncthreads();
+    }
+    if (!columns) return;
+    // ---- the weighted scores times x, and D x ----
+    if (KIND == PL_SCAN_LIGHTNING) {
+#pragma unroll
+        for (int k = 0; k < SSD_CHUNK / 2; ++k)
+            if (k < 16 || ti == 1) x[k] = ssd_kv<KIND>(x[k]);
+    }
+    ssd_f32x16 own;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) own[r] = 0.f;
+    {
+        const float* sc = As + (32 * ti + l32) * PA + 4 * half;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (q < 4 || ti == 1) {
+                const ssd_f32x4 av = *reinterpret_cast<const ssd_f32x4*>(sc + 8 * q);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) own = ssd_mfma(av[e], x[4 * q + e], own);
+            }
+        }
+    }
+    const float skip = KIND == PL_SCAN_SSD ? a.p3[h] : 0.f;
+    float* out = a.out + static_cast<size_t>(row0) * (H * V) + h * V;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int t = 32 * ti + 8 * (r >> 2) + 4 * half + (r & 3);
+        // (token t's own x is the one this lane holds in the same place of its half of the chunk)
+        if (t >= L || v >= V) continue;
+        float o = y[r] + own[r];
+        if (KIND == PL_SCAN_SSD) o += skip * (ti == 0 ? x[r] : x[16 + r]);
+        if (KIND == PL_SCAN_MLSTM) o *= below[t];
+        out[static_cast<size_t>(t) * (H * V) + v] = o;
+    }
+}
+
+// output_pair: the read-outs of one chunk, head and two tiles of 64 columns.  Eight waves; wave 4 ti + j owns the tokens 32 ti .. + 31 and, of the
 // scores, the earlier tokens 32 j .. + 31 (j < 2), of the read-outs, the columns 32 j .. + 31.  Bound by its chain (rows, scores, what the
 // state gives, what the chunk gives; three barriers), so waves without scores do the state's part meanwhile, and two workgroups share a
 // compute unit.  Two tiles a workgroup make the scores once for both: 42 chunks of 8 heads of 128 by 128 44.6 us (50.8 with a tile a
 // workgroup and one for each chunk that there might be), of 4 heads of 128 by 256 (matrix memory) 40.8 (49.3), 25 chunks of the first 27.6 (40.7);
 // one tile a workgroup with the same order of loads 56.7, 52.9 and 30.8.
 // LDS: C [64][P], B [64][P] (behind the scores' barrier the weighted scores [64][68] lie in its place), b, step sizes, two numbers a token.
-template <int KIND, int W>
-__global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, int seqs, int aligned) {
+template <int KIND>
+__global__ __launch_bounds__(512, 4) void ssd_output_pair_kernel(SsdArgs sa, int seqs, int aligned) {
     const ScanArgs& a = sa.a;
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    constexpr int T = 256 * W;
+    constexpr int T = 512;
     const int N = a.D, V = a.V, H = a.H;
-    const int tiles = (V + 64 * W - 1) / (64 * W);
+    const int tiles = (V + 128 - 1) / (128);
     const int h = blockIdx.y / tiles, vt = blockIdx.y % tiles;
     ChunkPlace place;
     if (!find_chunk(a, seqs, blockIdx.x, place)) return;
@@ -721,13 +1021,13 @@ __global__ __launch_bounds__(256 * W, 2 * W) void ssd_output_kernel(SsdArgs sa, 
     float* As = Bs;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int ti = wave / (2 * W), tj = wave % (2 * W);
+    const int ti = wave / (4), tj = wave % (4);
     const float* rows = a.qkv + static_cast<size_t>(row0) * a.qkv_stride;
 
     // ---- what waits for nothing: C and B into LDS, the first rows of S_0 into registers ----
     // (every load is unconditional, from an address that is valid in any case: one in a branch would be waited for alone)
-    const int v = vt * 64 * W + 32 * tj + l32, vc = min(v, V - 1);
-    const bool columns = vt * 64 * W + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
+    const int v = vt * 128 + 32 * tj + l32, vc = min(v, V - 1);
+    const bool columns = vt * 128 + 32 * tj < V && 32 * ti < L;      // (the same for the wave) it has read-outs to give
     // (32-bit offsets from bases that are the same for the wave: an address a load would take two registers)
     const char* S0 = reinterpret_cast<const char*>(sa.Sin + idx * N * V);
     auto ask = [&](int n0, float (&s0)[16]) {                         // rows n0 .. n0 + 31 of S_0, the wave's columns
@@ -962,34 +1262,54 @@ extern "C" int pl_ssd_step(const float* qkv, int qkv_stride, int q_off, int k_of
     return 0;
 }
 
-template <int KIND, int W>
-static int launch_chunks_of(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
+template <int KIND>
+static int launch_chunk_pairs(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
     const ScanArgs& a = sa.a;
     const int N = a.D, V = a.V;
-    const dim3 grid(chunk_bound(rows, max_q_len, seqs), a.H * pl_ceil_div(V, 64 * W));
+    const dim3 grid(chunk_bound(rows, max_q_len, seqs), a.H * pl_ceil_div(V, 128));
     const auto room = [](const void* kernel, size_t lds) {
         return lds <= 48 * 1024 ? hipSuccess : hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     };
-    const size_t lds_s = SSD_CHUNK * (64 * W + pl_ceil_div(N, 32) * 32 + 2 * SSD_SUMMARY_PAD) * sizeof(float);
-    hipError_t e = room(reinterpret_cast<const void*>(&ssd_summary_kernel<KIND, W>), lds_s);
+    const size_t lds_s = SSD_CHUNK * (128 + pl_ceil_div(N, 32) * 32 + 2 * SSD_SUMMARY_PAD) * sizeof(float);
+    hipError_t e = room(reinterpret_cast<const void*>(&ssd_summary_pair_kernel<KIND>), lds_s);
     PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds_s, hipGetErrorString(e));
     const bool aligned = ssd_aligned(a);
-    ssd_summary_kernel<KIND, W><<<grid, 256 * W, lds_s, stream>>>(sa, seqs, aligned && V % 4 == 0 ? 1 : 0);
+    ssd_summary_pair_kernel<KIND><<<grid, 512, lds_s, stream>>>(sa, seqs, aligned && V % 4 == 0 ? 1 : 0);
     PL_CHECK_LAUNCH("ssd_chunked (summary)");
     ssd_carry_kernel<KIND><<<dim3(pl_ceil_div(N * (KIND == PL_SCAN_MLSTM ? V + 1 : V), 256), a.H, seqs), 256, 0, stream>>>(sa);
     PL_CHECK_LAUNCH("ssd_chunked (carry)");
     const int P = ((N + 7) & ~7) + 4;
     const size_t lds = (6 * SSD_CHUNK + SSD_CHUNK * static_cast<size_t>(P) + SSD_CHUNK * static_cast<size_t>(P > SSD_CHUNK + 4 ? P : SSD_CHUNK + 4)) * sizeof(float);
-    e = room(reinterpret_cast<const void*>(&ssd_output_kernel<KIND, W>), lds);
+    e = room(reinterpret_cast<const void*>(&ssd_output_pair_kernel<KIND>), lds);
     PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
-    ssd_output_kernel<KIND, W><<<grid, 256 * W, lds, stream>>>(sa, seqs, aligned ? 1 : 0);
+    ssd_output_pair_kernel<KIND><<<grid, 512, lds, stream>>>(sa, seqs, aligned ? 1 : 0);
     PL_CHECK_LAUNCH("ssd_chunked (output)");
     return 0;
 }
 
 template <int KIND>
 static int launch_chunks(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
-    return sa.a.V > 64 ? launch_chunks_of<KIND, 2>(sa, rows, seqs, max_q_len, stream) : launch_chunks_of<KIND, 1>(sa, rows, seqs, max_q_len, stream);
+    const ScanArgs& a = sa.a;
+    const int N = a.D, V = a.V, tiles = pl_ceil_div(V, 64);
+    // Two tiles of columns a workgroup, and a workgroup for each chunk that there can be, pay where there are three requests or more (one of
+    // them rows of padding, mostly), whose chunks are counted as those of the longest otherwise.  (Sums, walk and read-outs, us, one / two
+    // tiles: 8 heads of 128 by 128, one request of 2,048 tokens 64 / 78, of 512 37 / 44, two of 1,500 and 1,125 94 / 81, eight of 300 122 / 82;
+    // 4 heads of 128 by 256 (matrix memory) 57 / 74, 33 / 42, 87 / 78, 108 / 74.  The same bits either way.)
+    if (seqs >= 3 && V > 64) return launch_chunk_pairs<KIND>(sa, rows, seqs, max_q_len, stream);
+    const dim3 grid(pl_ceil_div(max_q_len, SSD_CHUNK), a.H * tiles, seqs);
+    ssd_summary_kernel<KIND><<<grid, 256, 0, stream>>>(sa);
+    PL_CHECK_LAUNCH("ssd_chunked (summary)");
+    ssd_carry_kernel<KIND><<<dim3(pl_ceil_div(N * (KIND == PL_SCAN_MLSTM ? V + 1 : V), 256), a.H, seqs), 256, 0, stream>>>(sa);
+    PL_CHECK_LAUNCH("ssd_chunked (carry)");
+    const int P = ((N + 7) & ~7) + 4;
+    const size_t lds = (6 * SSD_CHUNK + SSD_CHUNK * static_cast<size_t>(P) + SSD_CHUNK * static_cast<size_t>(P > SSD_CHUNK + 4 ? P : SSD_CHUNK + 4)) * sizeof(float);
+    if (lds > 48 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ssd_output_kernel<KIND>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        PL_REQUIRE(e == hipSuccess, "ssd_chunked: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    }
+    ssd_output_kernel<KIND><<<grid, 256, lds, stream>>>(sa, ssd_aligned(a) ? 1 : 0);
+    PL_CHECK_LAUNCH("ssd_chunked (output)");
+    return 0;
 }
 
 // The requests that bring at least `from` tokens, in chunks of 64; `rows`: what the step's requests bring together at most.  U, Sin: room

@@ -129,7 +129,8 @@ def context_bound(longest: int) -> int:
 
 
 def near_context(longest: int) -> int:
-    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens.  A fresh prompt of a few
+    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens (in layers whose queries and
+    keys are normed and turned by the kernel in front of attention).  A fresh prompt of a few
     dozen tokens has one tile of keys: dealt out by a bound of 1,024 it had four workgroups a tile, three without a key, and a
     second launch to put them together (0.6B shape, a step: 37 tokens 1,385 to 1,301 us, 256 tokens 2,334 to 2,260; 37 tokens behind 700 others, whose
     keys are worth sharing, stay as they were).  A step's shape names it, so a captured step is replayed for contexts like its own."""

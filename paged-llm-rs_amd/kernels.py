@@ -846,7 +846,7 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
     qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
                           batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
                           nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)
-    return paged_attention(qkv, out, batch, kv, nq, nkv, d, scale, window)
+    return paged_attention(qkv, out, batch, kv, nq, nkv, d, scale, window, near=getattr(batch, "near_ctx_len", None))
 
 
 # Up to this many workgroups (requests times query heads) the tiled kernel takes a mixed step's short requests too.
@@ -855,8 +855,9 @@ TILED_TAKES_SHORT_WORKGROUPS = 512
 
 def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, d: int,
                     scale: float, window: int = 0, sinks: torch.Tensor | None = None,
-                    slopes: torch.Tensor | None = None, more: AttentionMore | None = None) -> torch.Tensor:
-    """Attention for every token of a step.  ``qkv`` rows begin with the rotated queries.
+                    slopes: torch.Tensor | None = None, more: AttentionMore | None = None, near: int | None = None) -> torch.Tensor:
+    """Attention for every token of a step.  ``qkv`` rows begin with the rotated queries.  ``near``: a closer bound on the
+    contexts than the step's, by which the tiled kernel shares keys out (``near_context``).
     In 32-bit every row goes to the kernel on the matrix cores' 32-bit instruction, where the head size is a multiple of four up
     to 256 and the step says which rows each request brings (``q_start``, ``q_len``, ``ctx_len``, ``max_ctx_len``), and otherwise to the plain one,
     which needs each row's position and request only.  In bfloat16 the long portions go to the tiled kernel and the tokens of short ones
@@ -882,7 +883,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
         paged_attention_prefill(qkv, stride, out, batch.q_start, batch.q_len, batch.ctx_len, batch.max_q_len,
                                 kv.block_table, kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window,
                                 short_limit=0 if all_tiled else SHORT_PORTION,
-                                max_ctx=getattr(batch, "near_ctx_len", batch.max_ctx_len),
+                                max_ctx=batch.max_ctx_len if near is None else near,
                                 live_seqs=getattr(batch, "live_seqs", None), sinks=sinks, slopes=slopes, more=more)
         if short_tokens == 0 or all_tiled:
             return out
