@@ -20,66 +20,53 @@ __global__ void rmsnorm_onto_kernel(float* __restrict__ resid, const float* __re
     }
 }
 
-// The same for rows of whole groups of four values: a thread keeps its NV groups of y in registers and asks for the stream and the gains
-// beside them, so that a row is one trip to memory and one sum over the workgroup.  Two rows of 1,024 take 2.7 us (4.8 value by
-// value); 2,816 rows 7.9 (11.3), at the rate that reads and writes side by side reach.
+// The same for rows that fit the registers: a thread keeps its NV values of y and asks for the stream and the gains beside them, so that a
+// row is one trip to memory and one sum over the workgroup.  Which values a thread has, and in which order it squares them, is as above,
+// so the bits are the same.  Two rows of 1,024 take 2.4 us (3.1 value by value); 2,816 rows 9.8 (14.9), at the rate that reads and writes side by
+// side reach.  (With 16 bytes a lane 2.1 and 9.4, but a sum in another order, whose error against 64 bits is up to 2% larger; 16 bytes a
+// lane and the sum from LDS in this order 2.4 and 9.6.)
 template <typename T, int NV>
-__global__ void __launch_bounds__(512) rmsnorm_onto_quads_kernel(float* __restrict__ resid, const float* __restrict__ y,
-                                                                 const float* __restrict__ gain, float eps,
-                                                                 T* __restrict__ rows_out, int H) {
+__global__ void __launch_bounds__(256) rmsnorm_onto_held_kernel(float* __restrict__ resid, const float* __restrict__ y,
+                                                                const float* __restrict__ gain, float eps,
+                                                                T* __restrict__ rows_out, int H) {
     __shared__ float scratch[16];
     const size_t base = static_cast<size_t>(blockIdx.x) * H;
-    float4 v[NV], x[NV], g[NV];
+    float v[NV], x[NV], g[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int c = (k * blockDim.x + threadIdx.x) * 4;
-        const int from = c < H ? c : 0;
-        v[k] = *reinterpret_cast<const float4*>(y + base + from);
-        x[k] = *reinterpret_cast<const float4*>(resid + base + from);
-        g[k] = *reinterpret_cast<const float4*>(gain + from);
+        const int c = k * blockDim.x + threadIdx.x, from = c < H ? c : 0;
+        v[k] = y[base + from];
+        x[k] = resid[base + from];
+        g[k] = gain[from];
     }
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
-        if (static_cast<int>(k * blockDim.x + threadIdx.x) * 4 < H)
-            ss += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+        if (static_cast<int>(k * blockDim.x + threadIdx.x) < H) ss = fmaf(v[k], v[k], ss);
     ss = block_sum(ss, scratch);
     const float inv = 1.f / sqrtf(ss / static_cast<float>(H) + eps);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int c = (k * blockDim.x + threadIdx.x) * 4;
+        const int c = k * blockDim.x + threadIdx.x;
         if (c >= H) continue;
-        x[k].x += v[k].x * inv * g[k].x;
-        x[k].y += v[k].y * inv * g[k].y;
-        x[k].z += v[k].z * inv * g[k].z;
-        x[k].w += v[k].w * inv * g[k].w;
-        *reinterpret_cast<float4*>(resid + base + c) = x[k];
-        if (rows_out == nullptr) continue;
-        if constexpr (sizeof(T) == 4) {
-            *reinterpret_cast<float4*>(rows_out + base + c) = x[k];
-        } else {
-            uint2 w;
-            w.x = static_cast<uint32_t>(bf16_bits_from_float(x[k].x)) | (static_cast<uint32_t>(bf16_bits_from_float(x[k].y)) << 16);
-            w.y = static_cast<uint32_t>(bf16_bits_from_float(x[k].z)) | (static_cast<uint32_t>(bf16_bits_from_float(x[k].w)) << 16);
-            *reinterpret_cast<uint2*>(rows_out + base + c) = w;
-        }
+        const float sum = fmaf(v[k] * inv, g[k], x[k]);
+        resid[base + c] = sum;
+        if (rows_out != nullptr) rows_out[base + c] = from_float<T>(sum);
     }
 }
 
 template <typename T>
 static void launch_rmsnorm_onto(float* resid, const float* y, const float* gain, float eps, T* rows_out, int n, int H, hipStream_t stream) {
-    const uintptr_t at = reinterpret_cast<uintptr_t>(resid) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gain) |
-                         reinterpret_cast<uintptr_t>(rows_out);
-    if (H % 4 == 0 && H <= 512 * 4 * 4 && at % 16 == 0) {       // (wider rows have no registers for it)
-        const int quads = H / 4, threads = quads <= 256 ? pl_ceil_div(quads, 64) * 64 : (quads <= 512 ? 256 : 512);
-        const int each = pl_ceil_div(quads, threads);
-        if (each == 1) rmsnorm_onto_quads_kernel<T, 1><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
-        else if (each == 2) rmsnorm_onto_quads_kernel<T, 2><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
-        else rmsnorm_onto_quads_kernel<T, 4><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
-        return;
-    }
-    const int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64);
-    rmsnorm_onto_kernel<T><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
+    const int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64), each = pl_ceil_div(H, threads);
+#define ONTO_HELD(NV) rmsnorm_onto_held_kernel<T, NV><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H)
+    if (each <= 1) ONTO_HELD(1);
+    else if (each <= 2) ONTO_HELD(2);
+    else if (each <= 4) ONTO_HELD(4);
+    else if (each <= 8) ONTO_HELD(8);
+    else if (each <= 16) ONTO_HELD(16);
+    else if (each <= 32) ONTO_HELD(32);
+    else rmsnorm_onto_kernel<T><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);      // (wider rows have no registers for it)
+#undef ONTO_HELD
 }
 
 // rows_out may be null; its type is `dtype` otherwise.

@@ -1359,6 +1359,34 @@ def test_rmsnorm_onto_over_widths_of_every_kernel(width, rows):
             assert torch.equal(out, got.to(rows_dtype))
 
 
+@pytest.mark.parametrize("width", [3, 64, 255, 256, 640, 1023, 1024, 1100, 4096, 8192, 8196])
+def test_rmsnorm_onto_adds_the_squares_in_one_order_at_every_width(width):
+    """Thread t of the launch squares the columns t, t + threads, ... one onto the other, a wave adds its threads' sums in pairs 32, 16, ... apart,
+    the waves' follow each other: the same bits whichever kernel takes a width."""
+    from paged_llm_rs_amd import kernels
+
+    rows, eps = 6, np.float32(1e-5)
+    resid, y, gain = randn(rows, width, seed=1), randn(rows, width, seed=2, std=3.0), randn(width, seed=3)
+    threads = 256 if width >= 1024 else (128 if width >= 256 else 64)
+    values = np.zeros((rows, -(-width // threads) * threads), np.float64)
+    values[:, :width] = y.numpy()
+    sums = np.zeros((rows, threads), np.float32)
+    for part in np.split(values, values.shape[1] // threads, axis=1):
+        sums = (part * part + sums).astype(np.float32)                  # (a fused product and sum: one rounding)
+    lanes = sums.reshape(rows, threads // 64, 64)
+    for apart in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, :, np.arange(64) ^ apart]
+    total = np.zeros(rows, np.float32)
+    for wave in range(threads // 64):
+        total = total + lanes[:, wave, 0]
+    inv = np.float32(1.0) / np.sqrt(total / np.float32(width) + eps)
+    scaled = (y.numpy() * inv[:, None]).astype(np.float64)
+    want = torch.from_numpy((scaled * gain.numpy() + resid.numpy()).astype(np.float32))
+    got = resid.to(DEV)
+    kernels.rmsnorm_onto(got, y.to(DEV), gain.to(DEV), float(eps), None)
+    assert torch.equal(got.cpu(), want)
+
+
 # --- the convolutions in front of attention, one token a request ------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
