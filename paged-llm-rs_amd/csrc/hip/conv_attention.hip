@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64) void conv_qk_prepare_single_kernel(ConvQkArgs a
         } else {
             x[i] = 0.f;
         }
-        ss += x[i] * x[i];
+        ss = fmaf(x[i], x[i], ss);          // (written out, so that it is rounded as in the kernels of longer portions)
     }
     if (kind != 2) {
         ss = wave_sum(ss);

@@ -1425,6 +1425,31 @@ def test_single_tokens_move_their_convolutions_history_in_the_same_launch(dtype,
         assert torch.equal(results[0][3], results[1][3]), "histories are copies"
 
 
+@pytest.mark.parametrize("taps,D,V,padded,rot", [(4, 128, 128, 128, 64), (2, 40, 24, 48, 8), (7, 160, 192, 192, 0), (3, 256, 256, 256, 256)])
+def test_single_tokens_behind_convolutions_give_the_bits_of_any_portion(taps, D, V, padded, rot):
+    """In 32-bit: the kernel of a step of one token a request against that of portions, head sizes of one to four values a lane."""
+    from paged_llm_rs_amd import kernels
+
+    H, G, block, n = 4, 2, 16, 24
+    channels = H * D + G * D + G * V
+    at = torch.arange(n, dtype=torch.int32, device=DEV)
+    batch = types.SimpleNamespace(positions=at * 41, seq_of=at, q_start=at, q_len=torch.ones_like(at), state_slots=at, num_seqs=n,
+                                  num_tokens=n, max_q_len=1)
+    pages = 41 * n // block + 1
+    table = torch.arange(n * pages, dtype=torch.int32, device=DEV).view(n, pages)
+    rows, weight, before = gpu_randn(n, channels, seed=1), gpu_randn(taps, channels, seed=2), gpu_randn(n, (taps - 1) * channels, seed=6)
+    gains, freq = (gpu_randn(D, seed=3), gpu_randn(D, seed=4)), gpu_randn(max(rot // 2, 1), seed=5).abs()
+    results = []
+    for moves in (False, True):
+        kv = types.SimpleNamespace(k_pool=torch.zeros((n * pages * block, G * padded), device=DEV),
+                                   v_pool=torch.zeros((n * pages * block, G * padded), device=DEV), block_table=table, block_size=block)
+        q = torch.zeros((n, H * padded), device=DEV)
+        kernels.conv_qk_prepare(rows, 0, weight, before.clone(), *gains, 1e-6, freq if rot else None, rot, batch, kv, H, G, D, V, padded, q,
+                                move_history=moves)
+        results.append((q, kv.k_pool, kv.v_pool))
+    assert all(torch.equal(old, new) for old, new in zip(*results))
+
+
 # --- the activation of a feed-forward without a gate, as the product's last stage ---------------------------------------
 
 @pytest.mark.parametrize("name", ["gelu_pytorch_tanh", "gelu", "silu", "relu2"])
