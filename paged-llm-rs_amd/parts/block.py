@@ -453,15 +453,18 @@ class ParallelBlock:
     The stream and every sum into it are 32-bit; sublayers hand back 32-bit rows.  One kernel adds a layer's two outputs
     into the stream and norms the next layer's two rows in the same pass (``kernels.parallel_step``): a layer that is
     followed by another of this arrangement leaves its sums to that layer's pass (``PendingSums``), so a layer is one
-    pass over the stream.  Behind that pass neither sublayer waits for the other: the feed-forward runs on a second stream beside the
-    mixer (``side_by_side``; a captured step keeps the two branches), and the pass behind the layer waits for both.  ``ctx.stream_addend`` (rows the decoder wants added to the stream before this run) joins
+    pass over the stream.  Behind that pass neither sublayer waits for the other: with ``side_by_side`` the feed-forward runs on a second
+    stream beside the mixer (a captured step keeps the two branches), and the pass behind the layer waits for both.  ``ctx.stream_addend`` (rows the decoder wants added to the stream before this run) joins
     that pass too.  Tensor names: the norms' gains under the norms' own names."""
 
     NAMES = {"norm1": "norm1", "mixer": "mix", "norm2": "norm2", "feed_forward": "mlp", "scale1": "ls1", "scale2": "ls2"}
     # the decoder may hand this block rows to add to the stream before it runs (``LayerContext.stream_addend``)
     takes_stream_addend = True
-    # the two sublayers on two streams (False: one behind the other; the same bits)
-    side_by_side = True
+    # The two sublayers on two streams (False: one behind the other; the same bits).  Off: the host process has ended in a segmentation fault
+    # twice where engines of the designs with this arrangement came and went, with captured steps of two branches alive or just
+    # destroyed, and its cause is not known.  What that costs a decoding step at batch 1 to 64: with experts and retention 1,024 wide
+    # 8 to 16% (0.415 to 0.469 ms at batch 8), 4,096 wide 6 to 20%.
+    side_by_side = False
 
     @classmethod
     def names_of(cls, layer) -> dict:

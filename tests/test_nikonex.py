@@ -221,3 +221,32 @@ def test_properties_of_the_plain_router():
           "shared.sg": torch.randn(1, 12, generator=g, dtype=F)}
     want = torch.sigmoid(h @ w2["shared.sg"].T) * (plain.relu_squared(h @ w2["shared.up"].T) @ w2["shared.down"].T)
     assert torch.allclose(plain.feed_forward(h, w2, "", mlp), want)
+
+
+def test_a_parallel_layer_stays_on_one_stream(monkeypatch):
+    """The two sublayers run one behind the other: no second stream is made, and what they give reaches the pass."""
+    import types
+
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.parts.block import ParallelBlock
+
+    def no_stream(*args, **kw):
+        raise AssertionError("a second stream")
+
+    order, passes = [], []
+
+    def step(resid, **kw):
+        passes.append(kw)
+        return resid + 1, resid + 2
+
+    monkeypatch.setattr(torch.cuda, "Stream", no_stream)
+    monkeypatch.setattr(kernels, "parallel_step", step)
+    layer = object.__new__(ParallelBlock)
+    layer.shared, layer.mult, layer.ls1, layer.ls2, layer.dtype = {}, 1.0, None, None, torch.float32
+    layer.norm1 = layer.norm2 = types.SimpleNamespace(eps=1e-5, gain32=None)
+    layer.mixer = types.SimpleNamespace(forward=lambda x, ctx: order.append("mixer") or x * 10)
+    layer.feed_forward = types.SimpleNamespace(forward=lambda x: order.append("feed-forward") or x * 100)
+    ctx = types.SimpleNamespace(trace=None, batch=None)
+    assert layer.forward(torch.ones(2, 3), None, ctx) is None
+    assert order == ["mixer", "feed-forward"] and len(passes) == 2
+    assert torch.equal(passes[1]["a"], torch.full((2, 3), 20.0)) and torch.equal(passes[1]["b"], torch.full((2, 3), 300.0))

