@@ -361,15 +361,15 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs da) {
         }
 }
 
-static int launch_delta(const DeltaArgs& da, int rows, int seqs, int max_q_len, hipStream_t stream) {
+static int launch_delta(const DeltaArgs& da, int rows, int seqs, int max_q_len, int dealt, hipStream_t stream) {
     const ScanArgs& a = da.a;
     const int Dp = pl_ceil_div(a.D, 64) * 64, P = Dp + 4;
     const size_t lds_p = (7 * DL_C + 2 * static_cast<size_t>(DL_C) * (P > DL_T ? P : DL_T)) * sizeof(float);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prepare_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(lds_p));
     PL_REQUIRE(e == hipSuccess, "delta_chunked: %zu bytes of LDS refused: %s", lds_p, hipGetErrorString(e));
-    // (with three requests or more a workgroup for each chunk that there can be; below that the longest's chunks for every request)
-    if (seqs >= 3) delta_prepare_kernel<<<dim3(chunk_bound(rows, max_q_len, seqs), a.H), 256, lds_p, stream>>>(da, Dp, seqs);
+    // (dealt: a workgroup for each chunk that the rows can hold; otherwise the longest's chunks for every request)
+    if (dealt) delta_prepare_kernel<<<dim3(chunk_bound(rows, max_q_len, seqs), a.H), 256, lds_p, stream>>>(da, Dp, seqs);
     else delta_prepare_kernel<<<dim3(pl_ceil_div(max_q_len, DL_C), a.H, seqs), 256, lds_p, stream>>>(da, Dp, 0);
     PL_CHECK_LAUNCH("delta_chunked (prepare)");
     // the workgroups of one head read the same chunks: with heads and requests along x they share a chiplet's cache wherever those are a
@@ -390,7 +390,7 @@ extern "C" int pl_delta_chunked(const float* qkv, int qkv_stride, int q_off, int
                                 const float* a_log, const float* dt_bias,
                                 float* state, long state_stride, float* out,
                                 const int* q_start, const int* q_len, const int* state_slots,
-                                int rows, int seqs, int max_q_len, int H, int G, int D, int V, int from,
+                                int rows, int seqs, int max_q_len, int dealt, int H, int G, int D, int V, int from,
                                 float* Kn, float* Qn, float* Kw, float* Tm, float* Aq, float* scal, hipStream_t stream) {
     PL_REQUIRE(H > 0 && G > 0 && H % G == 0 && D > 0 && D <= 256 && V > 0 && from >= 1,
                "delta_chunked: %d heads over %d of q and k, %d by %d, from %d tokens", H, G, D, V, from);
@@ -402,5 +402,5 @@ extern "C" int pl_delta_chunked(const float* qkv, int qkv_stride, int q_off, int
     DeltaArgs da{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, a_log, dt_bias, nullptr, 0.f, state,
                   state_stride, 0, 0, 0, out, q_start, q_len, state_slots, H, G, D, V, from},
                  Kn, Qn, Kw, Tm, Aq, scal};
-    return launch_delta(da, rows, seqs, max_q_len, stream);
+    return launch_delta(da, rows, seqs, max_q_len, dealt, stream);
 }

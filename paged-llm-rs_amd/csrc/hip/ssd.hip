@@ -1288,14 +1288,11 @@ static int launch_chunk_pairs(const SsdArgs& sa, int rows, int seqs, int max_q_l
 }
 
 template <int KIND>
-static int launch_chunks(const SsdArgs& sa, int rows, int seqs, int max_q_len, hipStream_t stream) {
+static int launch_chunks(const SsdArgs& sa, int rows, int seqs, int max_q_len, int dealt, hipStream_t stream) {
     const ScanArgs& a = sa.a;
     const int N = a.D, V = a.V, tiles = pl_ceil_div(V, 64);
-    // Two tiles of columns a workgroup, and a workgroup for each chunk that there can be, pay where there are three requests or more (one of
-    // them rows of padding, mostly), whose chunks are counted as those of the longest otherwise.  (Sums, walk and read-outs, us, one / two
-    // tiles: 8 heads of 128 by 128, one request of 2,048 tokens 64 / 78, of 512 37 / 44, two of 1,500 and 1,125 94 / 81, eight of 300 122 / 82;
-    // 4 heads of 128 by 256 (matrix memory) 57 / 74, 33 / 42, 87 / 78, 108 / 74.  The same bits either way.)
-    if (seqs >= 3 && V > 64) return launch_chunk_pairs<KIND>(sa, rows, seqs, max_q_len, stream);
+    // (The same bits either way; which steps are dealt, and the times of both, is where the caller chooses.)
+    if (dealt && V > 64) return launch_chunk_pairs<KIND>(sa, rows, seqs, max_q_len, stream);
     const dim3 grid(pl_ceil_div(max_q_len, SSD_CHUNK), a.H * tiles, seqs);
     ssd_summary_kernel<KIND><<<grid, 256, 0, stream>>>(sa);
     PL_CHECK_LAUNCH("ssd_chunked (summary)");
@@ -1313,11 +1310,11 @@ static int launch_chunks(const SsdArgs& sa, int rows, int seqs, int max_q_len, h
 }
 
 // The requests that bring at least `from` tokens, in chunks of 64; `rows`: what the step's requests bring together at most.  U, Sin: room
-// for (rows / 64 + requests + 1) chunks of
-// H * N * V floats; ends: of H.
+// for (rows / 64 + requests + 1) chunks of H * N * V floats; ends: of H.  dealt: a workgroup for each chunk that the rows can hold, two tiles
+// of 64 columns each where V has them, instead of the longest request's chunks for every request.
 extern "C" int pl_ssd_chunked(const float* qkv, int qkv_stride, int q_off, int k_off, int v_off, const float* gates, int gates_stride,
                               int g_off, const float* a_log, const float* dt_bias, const float* skip, float* state, long state_stride,
-                              float* out, const int* q_start, const int* q_len, const int* state_slots, int rows, int seqs, int max_q_len, int H,
+                              float* out, const int* q_start, const int* q_len, const int* state_slots, int rows, int seqs, int max_q_len, int dealt, int H,
                               int G, int N, int V, int from, float* U, float* Sin, float* ends, hipStream_t stream) {
     PL_REQUIRE(H > 0 && G > 0 && H % G == 0 && N > 0 && N <= 256 && V > 0 && from >= 1, "ssd_chunked: %d heads of %d by %d over %d groups, from %d tokens", H, N, V, G, from);
     PL_REQUIRE(gates != nullptr && a_log != nullptr && dt_bias != nullptr && skip != nullptr && U != nullptr && Sin != nullptr && ends != nullptr,
@@ -1327,7 +1324,7 @@ extern "C" int pl_ssd_chunked(const float* qkv, int qkv_stride, int q_off, int k
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g_off, 0, a_log, dt_bias, skip, 0.f, state, state_stride,
                       0, 0, 0, out, q_start, q_len, state_slots, H, G, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
-    return launch_chunks<PL_SCAN_SSD>(sa, rows, seqs, max_q_len, stream);
+    return launch_chunks<PL_SCAN_SSD>(sa, rows, seqs, max_q_len, dealt, stream);
 }
 
 // Retention: S = decay S + k v^T, o = S^T q, q and k turning with their positions (HalfTurn; freq null: not at all).
@@ -1370,14 +1367,14 @@ extern "C" int pl_retention_step(const float* qkv, int qkv_stride, int q_off, in
 // The requests that bring at least `from` tokens, in chunks of 64, q and k turned already; decays above zero.  Room as in pl_ssd_chunked.
 extern "C" int pl_retention_chunked(const float* qkv, int qkv_stride, int q_off, int k_off, int v_off, const float* decay, float* state,
                                     long state_stride, float* out, const int* q_start, const int* q_len, const int* state_slots, int rows, int seqs,
-                                    int max_q_len, int H, int N, int V, int from, float* U, float* Sin, float* ends, hipStream_t stream) {
+                                    int max_q_len, int dealt, int H, int N, int V, int from, float* U, float* Sin, float* ends, hipStream_t stream) {
     PL_REQUIRE(H > 0 && N > 0 && N <= 256 && V > 0 && from >= 1, "retention_chunked: %d heads of %d by %d, from %d tokens", H, N, V, from);
     PL_REQUIRE(decay != nullptr && U != nullptr && Sin != nullptr && ends != nullptr, "retention_chunked: the decays or room for the chunks' sums are missing");
     PL_REQUIRE(static_cast<long long>(H) * pl_ceil_div(V, 64) <= 65535 && seqs >= 0 && seqs <= 65535, "retention_chunked: %d heads of %d columns, %d requests", H, V, seqs);
     if (seqs == 0 || max_q_len < from) return 0;
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, nullptr, 0, 0, 0, decay, nullptr, nullptr, 0.f, state, state_stride,
                       0, 0, 0, out, q_start, q_len, state_slots, H, H, N, V, from}, U, Sin, ends, nullptr, nullptr, nullptr};
-    return launch_chunks<PL_SCAN_RETENTION>(sa, rows, seqs, max_q_len, stream);
+    return launch_chunks<PL_SCAN_RETENTION>(sa, rows, seqs, max_q_len, dealt, stream);
 }
 
 // Linear attention with a fixed decay a head and silu on q, k and v (kind lightning), and the matrix memory with exponential gates
@@ -1388,7 +1385,7 @@ extern "C" int pl_recurrent_chunked(int kind, const float* qkv, int qkv_stride, 
                                     const float* p1, const float* p2, float cap,
                                     float* state, long state_stride, int s_off, int n_off, int m_off,
                                     float* out, const int* q_start, const int* q_len, const int* state_slots,
-                                    int rows, int seqs, int max_q_len, int H, int D, int V, int from, int chunks,
+                                    int rows, int seqs, int max_q_len, int dealt, int H, int D, int V, int from, int chunks,
                                     float* U, float* Uk, float* Sin, float* nin, float* scal, hipStream_t stream) {
     PL_REQUIRE(kind == PL_SCAN_LIGHTNING || kind == PL_SCAN_MLSTM, "recurrent_chunked: kind %d", kind);
     PL_REQUIRE(H > 0 && D > 0 && D <= 256 && V > 0 && from >= 1, "recurrent_chunked: %d heads of %d by %d, from %d tokens", H, D, V, from);
@@ -1401,6 +1398,6 @@ extern "C" int pl_recurrent_chunked(int kind, const float* qkv, int qkv_stride, 
     const SsdArgs sa{{qkv, qkv_stride, q_off, k_off, v_off, gates, gates_stride, g1_off, g2_off, p1, p2, nullptr, cap, state, state_stride,
                       s_off, n_off, m_off, out, q_start, q_len, state_slots, H, H, D, V, from},
                      U, Sin, scal, Uk, nin, scal + static_cast<size_t>(chunks) * H};
-    return kind == PL_SCAN_LIGHTNING ? launch_chunks<PL_SCAN_LIGHTNING>(sa, rows, seqs, max_q_len, stream)
-                                     : launch_chunks<PL_SCAN_MLSTM>(sa, rows, seqs, max_q_len, stream);
+    return kind == PL_SCAN_LIGHTNING ? launch_chunks<PL_SCAN_LIGHTNING>(sa, rows, seqs, max_q_len, dealt, stream)
+                                     : launch_chunks<PL_SCAN_MLSTM>(sa, rows, seqs, max_q_len, dealt, stream);
 }

@@ -70,14 +70,14 @@ def _signatures(lib) -> None:
         "pl_recurrent_scan": [i, p, i, i, i, i, p, i, i, i, p, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
                               i, i, i, i, i, i, p],
         "pl_recurrent_chunked": [i, p, i, i, i, i, p, i, i, i, p, p, f, p, ctypes.c_long, i, i, i, p, p, p, p,
-                                 i, i, i, i, i, i, i, i, p, p, p, p, p, p],
+                                 i, i, i, i, i, i, i, i, i, p, p, p, p, p, p],
         "pl_ssd_step": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, p],
         "pl_ssd_step_applies": [i, ctypes.c_long],
-        "pl_ssd_chunked": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, p, p, p, p],
+        "pl_ssd_chunked": [p, i, i, i, i, p, i, i, p, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, i, p, p, p, p],
         "pl_retention_turn": [p, i, i, i, i, i, i, p, i, f, f, p, p],
         "pl_retention_step": [p, i, i, i, i, p, p, i, f, f, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, p],
-        "pl_retention_chunked": [p, i, i, i, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, p, p, p, p],
-        "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i,
+        "pl_retention_chunked": [p, i, i, i, i, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, p, p, p, p],
+        "pl_delta_chunked": [p, i, i, i, i, p, i, i, i, p, p, p, ctypes.c_long, p, p, p, p, i, i, i, i, i, i, i, i, i,
                              p, p, p, p, p, p, p],
         "pl_short_conv": [p, i, i, i, p, i, p, ctypes.c_long, i, p, p, p, p, p, i, p, i, i, p],
         "pl_clear_slots": [p, i, ctypes.c_longlong, p, i, p],
@@ -1339,6 +1339,43 @@ SCAN_MAX_DIM = 256
 SCAN_CHUNKED_FROM = 16
 
 
+# In front of the chunk kernels a step only knows its rows and requests: launched plainly, every request gets the chunks that the longest could
+# have (in a padded step all rows), most of which are not there.  The other launch deals a workgroup to each chunk that the rows can hold, of
+# two tiles of 64 columns where the state has them; its chain is longer, so it pays where many chunks are there or very many are not.  Sums,
+# walk and read-outs, us, plain / dealt.  Eight heads of 128 by 128 (linear attention): a prompt of 100 tokens beside one decoded token 33 / 40,
+# of 600 beside 63 46 / 66, of 1,950 beside one 63 / 77, of 4,000 beside 63 146 / 95; without decoded tokens 60, 50 and 40 36 / 43, two of
+# 512 45 / 50, 700 and 800 79 / 52, 1,500 and 1,125 93 / 80, four of up to 1,400 128 / 81, eight of 300 124 / 82, sixteen of up to
+# 100 126 / 86, 32 of 64 1,155 / 108; one request is never dealt.  Over steps of 2 to 32 such requests and 384 to 7,168 rows, five kinds and shapes
+# of state, what the lines below deal is faster but for six of 518 (up to 5% slower), by a quarter together.
+DEALT_WORKGROUPS = 192        # whole chunks of rows, times heads and pairs of tiles, that fill the chip
+DEALT_PLAIN = 200             # chunks that a plain launch would have, from which it is the empty ones that cost
+DEALT_PLAIN_BESIDE = 2200     # the same where requests go token by token beside the chunks (how many, the launch does not know)
+DEALT_PLAIN_DELTA = 100       # the delta rule's first kernel, which is the same in either launch
+DEALT_PLAIN_RETENTION = 150   # retention (its scores cost no exponentials), from four requests on
+
+
+def deals_chunks(kind: str, requests: int, seqs: int, rows: int, max_q_len: int, heads: int, vdim: int, beside: bool) -> bool:
+    """Whether the chunk kernels' workgroups are dealt to the chunks there can be.  ``requests`` live ones of ``seqs``, ``beside``: some of them
+    bring too few tokens for a chunk.  All of it is part of a captured step's shape."""
+    plain = -(-max_q_len // SSD_CHUNK) * seqs
+    if requests < 2:
+        return False
+    if kind == "delta":
+        return not beside and plain >= DEALT_PLAIN_DELTA
+    if vdim <= 64:
+        return False
+    if kind == "retention":
+        return not beside and requests >= 4 and plain >= DEALT_PLAIN_RETENTION
+    fills = rows // SSD_CHUNK * heads * (-(-vdim // 128)) >= DEALT_WORKGROUPS
+    return (fills and plain >= DEALT_PLAIN_BESIDE) if beside else (fills or plain >= DEALT_PLAIN)
+
+
+def _dealt(kind: str, batch, rows: int, heads: int, vdim: int, beside: bool, given: bool | None) -> int:
+    if given is None:
+        given = deals_chunks(kind, getattr(batch, "live_seqs", batch.num_seqs), batch.num_seqs, rows, batch.max_q_len, heads, vdim, beside)
+    return 1 if given else 0
+
+
 def _state_view(state: torch.Tensor, what: str):
     """(tensor, floats between two slots): a [slots, floats] 32-bit state, possibly a run of columns of a wider one."""
     if not isinstance(state, torch.Tensor) or not state.is_cuda or state.dtype != torch.float32 or state.dim() != 2 \
@@ -1373,7 +1410,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
                    batch, heads: int, qk_heads: int, dim: int, vdim: int, *, gates: torch.Tensor | None = None,
                    g1_off: int = 0, g2_off: int = 0, p1: torch.Tensor | None = None, p2: torch.Tensor | None = None,
                    p3: torch.Tensor | None = None, cap: float = 0.0, out: torch.Tensor | None = None,
-                   chunked: bool = False) -> torch.Tensor:
+                   chunked: bool = False, dealt: bool | None = None) -> torch.Tensor:
     """The read-out [rows, heads * vdim] (32-bit) of a mixer that carries a [dim, vdim] matrix a head from
     token to token, over the tokens of a step, request by request, from and into the requests' state slots.
 
@@ -1388,7 +1425,8 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
     ``p3`` = D; one gate column a head, from ``g1_off``.
     q and k have ``qk_heads`` heads (head h of v reads head h / (heads / qk_heads)).
     ``chunked`` (lightning only with decays above zero): requests that bring ``SCAN_CHUNKED_FROM`` tokens or more
-    are computed in chunks of tokens, the same sums in another order."""
+    are computed in chunks of tokens, the same sums in another order.  ``dealt``: which launch the chunks get (chosen by
+    ``deals_chunks`` when not given; the same bits)."""
     if kind not in SCAN_KINDS:
         raise TensorError(f"a scan of kind {kind!r}, the kernels know {', '.join(SCAN_KINDS)}")
     n = qkv.shape[0]
@@ -1423,13 +1461,15 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
     hdv = heads * dim * vdim
     chunked = bool(chunked) and batch.max_q_len >= SCAN_CHUNKED_FROM
     if kind == "ssd":
-        return _ssd_scan(qkv, q_off, k_off, v_off, state, stride, batch, heads, qk_heads, dim, vdim, gates, g1_off, p1, p2, p3, out, chunked)
+        return _ssd_scan(qkv, q_off, k_off, v_off, state, stride, batch, heads, qk_heads, dim, vdim, gates, g1_off, p1, p2, p3, out, chunked, dealt)
     common = (SCAN_KINDS[kind], qkv.data_ptr(), width, q_off, k_off, v_off, _ptr(gates),
               0 if gates is None else gates.shape[1], g1_off, g2_off, _ptr(p1), _ptr(p2), float(cap),
               state.data_ptr(), stride, 0, hdv, hdv + heads * tiles * dim, out.data_ptr(), batch.q_start.data_ptr(),
               batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
-    if not chunked or _brings_short_requests(batch):
+    beside = _brings_short_requests(batch)
+    if not chunked or beside:
         _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
+    dealt = _dealt(kind, batch, n, heads, vdim, beside, dealt)
     if chunked and kind == "delta":
         chunks = (n // SSD_CHUNK + batch.num_seqs + 1) * heads
         f32 = dict(dtype=torch.float32, device=qkv.device)
@@ -1440,7 +1480,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
         _check(library().pl_delta_chunked(
             qkv.data_ptr(), width, q_off, k_off, v_off, gates.data_ptr(), gates.shape[1], g1_off, g2_off,
             p1.data_ptr(), p2.data_ptr(), state.data_ptr(), stride, out.data_ptr(), batch.q_start.data_ptr(),
-            batch.q_len.data_ptr(), batch.state_slots.data_ptr(), n, batch.num_seqs, batch.max_q_len, heads, qk_heads, dim,
+            batch.q_len.data_ptr(), batch.state_slots.data_ptr(), n, batch.num_seqs, batch.max_q_len, dealt, heads, qk_heads, dim,
             vdim, SCAN_CHUNKED_FROM, unit_k.data_ptr(), unit_q.data_ptr(), weighted_k.data_ptr(), inverse.data_ptr(), masked.data_ptr(),
             scalars.data_ptr(), _stream()))
     elif chunked:
@@ -1450,7 +1490,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
         k_sums, n_before = (torch.empty((chunks, heads * dim), **f32), torch.empty((chunks, heads * dim), **f32)) \
             if kind == "mlstm" else (None, None)
         scalars = torch.empty((chunks, heads * 4), **f32)
-        _check(library().pl_recurrent_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, heads, dim, vdim, SCAN_CHUNKED_FROM, chunks,
+        _check(library().pl_recurrent_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, dealt, heads, dim, vdim, SCAN_CHUNKED_FROM, chunks,
                                               sums.data_ptr(), _ptr(k_sums), before.data_ptr(), _ptr(n_before),
                                               scalars.data_ptr(), _stream()))
     return out
@@ -1460,7 +1500,7 @@ SSD_CHUNK = 64       # tokens of a chunk of the kernels in chunks
 
 
 def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch, H: int, G: int, N: int, V: int, gates,
-              g_off: int, a_log, dt_bias, skip, out, chunked: bool) -> torch.Tensor:
+              g_off: int, a_log, dt_bias, skip, out, chunked: bool, dealt: bool | None) -> torch.Tensor:
     """``recurrent_scan`` of kind ``ssd``, its arguments checked: requests of few tokens token by token, the others in
     chunks on the matrix cores (32-bit operands and sums)."""
     lib, stream, n = library(), _stream(), qkv.shape[0]
@@ -1468,7 +1508,8 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
     common = (qkv.data_ptr(), qkv.shape[1], q_off, k_off, v_off, gates.data_ptr(), gates.shape[1], g_off, *constants, state.data_ptr(),
               stride, out.data_ptr(), batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
     below = SCAN_CHUNKED_FROM if chunked else 0
-    if not chunked or batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0:
+    beside = batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
+    if not chunked or beside:
         if lib.pl_ssd_step_applies(V, stride) and state.data_ptr() % 16 == 0:
             _check(lib.pl_ssd_step(*common, H, G, N, V, below, stream))
         else:
@@ -1481,20 +1522,20 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
         f32 = dict(dtype=torch.float32, device=qkv.device)
         sums, before = torch.empty((chunks, H * N * V), **f32), torch.empty((chunks, H * N * V), **f32)
         ends = torch.empty((chunks, H), **f32)
-        _check(lib.pl_ssd_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, H, G, N, V, SCAN_CHUNKED_FROM, sums.data_ptr(), before.data_ptr(),
-                                  ends.data_ptr(), stream))
+        _check(lib.pl_ssd_chunked(*common[:-1], n, batch.num_seqs, batch.max_q_len, _dealt("ssd", batch, n, H, V, beside, dealt), H, G, N, V,
+                                  SCAN_CHUNKED_FROM, sums.data_ptr(), before.data_ptr(), ends.data_ptr(), stream))
     return out
 
 
 def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state: torch.Tensor, batch, heads: int, dim: int,
                    vdim: int, decay: torch.Tensor, freq: torch.Tensor | None, amplitude: float, k_scale: float,
-                   chunked: bool = True) -> torch.Tensor:
+                   chunked: bool = True, dealt: bool | None = None) -> torch.Tensor:
     """The read-out [rows, heads * vdim] (32-bit) of linear attention with a fixed decay a head, S = decay S + k v^T, o = S^T q, over
     the tokens of a step from and into the requests' state slots.  ``rows`` (32-bit) hold q, k [heads, dim] and v [heads, vdim] from
     their columns on; of every head of q and k the values i and i + len(freq) turn by position * ``freq``[i] (None: nothing turns),
     cosine and sine times ``amplitude``, and k is multiplied by ``k_scale``.  q and k may be turned in place: the rows are
     nobody else's.  ``chunked`` (decays above zero): requests of ``SCAN_CHUNKED_FROM`` tokens or more in chunks on the matrix
-    cores (32-bit operands and sums), the same sums in another order."""
+    cores (32-bit operands and sums), the same sums in another order; ``dealt`` as for ``recurrent_scan``."""
     n = rows.shape[0]
     _need(rows, "rows of q, k and v", None, torch.float32)
     width = rows.shape[1] if rows.dim() == 2 else -1
@@ -1519,7 +1560,8 @@ def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state
         return out
     lib, stream = library(), _stream()
     chunked = bool(chunked) and batch.max_q_len >= SCAN_CHUNKED_FROM
-    by_token = not chunked or batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
+    beside = batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
+    by_token = not chunked or beside
     steps = lib.pl_ssd_step_applies(vdim, stride) and state.data_ptr() % 16 == 0
     turn = (_ptr(freq), turned, float(amplitude), float(k_scale))
     at = (rows.data_ptr(), width, q_off, k_off, v_off)
@@ -1540,8 +1582,8 @@ def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state
         f32 = dict(dtype=torch.float32, device=rows.device)
         sums, before_chunks = torch.empty((chunks, heads * dim * vdim), **f32), torch.empty((chunks, heads * dim * vdim), **f32)
         ends = torch.empty((chunks, heads), **f32)
-        _check(lib.pl_retention_chunked(*at, decay.data_ptr(), state.data_ptr(), stride, out.data_ptr(), *step[:-1], n, batch.num_seqs, batch.max_q_len, heads,
-                                        dim, vdim, SCAN_CHUNKED_FROM, sums.data_ptr(), before_chunks.data_ptr(), ends.data_ptr(), stream))
+        _check(lib.pl_retention_chunked(*at, decay.data_ptr(), state.data_ptr(), stride, out.data_ptr(), *step[:-1], n, batch.num_seqs, batch.max_q_len,
+                                        _dealt("retention", batch, n, heads, vdim, beside, dealt), heads, dim, vdim, SCAN_CHUNKED_FROM, sums.data_ptr(), before_chunks.data_ptr(), ends.data_ptr(), stream))
     return out
 
 

@@ -177,3 +177,21 @@ def test_mixers_side_by_side_report_the_limit_of_every_branch(monkeypatch):
     assert portion_limits(blocks[:1]) == (4, 16)
     assert portion_limits(blocks[1:2]) == ()
     assert portion_limits(blocks[1:] + [SimpleNamespace(mixer=makers["more"]()), SimpleNamespace()]) == (4, 16)
+
+
+def test_which_steps_have_their_chunks_dealt():
+    """What a launch for every request's longest possible portion costs against one for the chunks there can be: one prompt, few short
+    prompts, and a prompt beside decoded tokens keep the plain launch; many chunks, or very many that are not there, are dealt."""
+    from paged_llm_rs_amd.kernels import deals_chunks
+
+    def step(live, rows, beside=False, kind="lightning", heads=8, vdim=128):
+        return deals_chunks(kind, live, live + 1, rows, rows, heads, vdim, beside)
+
+    for kind in ("lightning", "mlstm", "ssd", "delta", "retention"):
+        assert not step(1, 2048, kind=kind) and not step(3, 192, kind=kind)
+        assert not any(step(1 + k, rows, True, kind) for k, rows in ((1, 128), (1, 640), (63, 704), (1, 1280), (16, 1536), (1, 2048), (4, 2304)))
+        assert step(32, 2048, kind=kind) and step(8, 2560, kind=kind)
+    assert step(2, 2816) and step(2, 1536) and step(4, 3072) and step(64, 4352, True)
+    assert not step(2, 1024) and not step(2, 2816, heads=2) and step(16, 1280, heads=2) and not step(8, 2560, vdim=64)
+    assert not step(2, 5120, kind="retention") and step(6, 1536, kind="retention") and not step(64, 4352, True, "delta")
+    assert not deals_chunks("lightning", 16, 16, 1024, 64, 8, 128, False)             # (not padded: every request has one chunk, all of them there)

@@ -655,3 +655,39 @@ def test_chunks_of_many_requests_are_those_of_each_alone(kind, H, D, V):
             assert torch.equal(out, together[first:first + count]), (s, count)
             assert torch.equal(alone[0], state[s]), (s, count)
         first += count
+
+
+@pytest.mark.parametrize("kind,H,G,D,V", [("lightning", 2, 2, 128, 128), ("lightning", 1, 1, 40, 72), ("lightning", 2, 2, 256, 200), ("mlstm", 2, 2, 64, 256),
+                                          ("mlstm", 1, 1, 100, 36), ("delta", 4, 2, 128, 64), ("ssd", 4, 2, 64, 96), ("ssd", 2, 1, 100, 130),
+                                          ("ssd", 2, 2, 128, 64), ("retention", 2, 2, 48, 128), ("retention", 1, 1, 256, 67)])
+def test_dealt_chunks_give_the_bits_of_a_plain_launch(kind, H, G, D, V):
+    """A workgroup for each chunk that the rows can hold against the longest request's chunks for every request: 70 requests (more than a
+    wave counts at a time), most of them without a chunk, rows of padding behind them; states and read-outs."""
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator().manual_seed(11)
+    counts = [[1, 64, 2, 129, 15, 16][i % 6] if i % 7 == 0 or i in (63, 64, 69) else 1 for i in range(70)]
+    n, pad = sum(counts), 37
+    qk = G * D
+    width = 2 * qk + H * V + 2 * H
+    rows = torch.randn(n + pad, width, generator=g).cuda() * 0.5
+    p1 = torch.linspace(0.9, 0.99, H).cuda() if kind in ("lightning", "retention") else torch.linspace(-1.0, 0.5, H).cuda()
+    p2 = torch.linspace(1.0, 2.0, H).cuda()
+    floats = H * D * V if kind == "retention" else kernels.scan_state_floats(kind, H, D, V)
+    before = torch.zeros(70, floats) if kind == "mlstm" else torch.randn(70, floats, generator=g) * 0.1
+    step = ScanStep(counts, range(70), pad)
+    step.max_q_len = step.num_tokens                # (as a padded step says it)
+
+    def scan(dealt):
+        state = before.cuda()
+        if kind == "retention":
+            out = kernels.retention_scan(rows.clone(), 0, qk, 2 * qk, state, step, H, D, V, p1, None, 1.0, 1.0, dealt=dealt)
+        else:
+            out = kernels.recurrent_scan(kind, rows, 0, qk, 2 * qk, state, step, H, G, D, V, gates=None if kind == "lightning" else rows,
+                                         g1_off=width - 2 * H, g2_off=width - H, p1=p1, p2=None if kind == "lightning" else p2,
+                                         p3=p2 if kind == "ssd" else None, cap=15.0, chunked=True, dealt=dealt)
+        return out[:n], state
+
+    plain, dealt = scan(False), scan(True)
+    assert torch.equal(plain[0], dealt[0]) and torch.equal(plain[1], dealt[1])
+    assert plain[0].isfinite().all() and not torch.equal(plain[1].cpu(), before)
