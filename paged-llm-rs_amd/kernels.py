@@ -1131,15 +1131,33 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
     return out
 
 
-# Where the product over strips and very many columns beats the others (gemm_wide.hip has the times of both sides).
+# Where the product over strips and very many columns beats the others, timed at 1 to 32 rows over 131,072 to 524,288 columns and widths from 2,048
+# to 8,192.  The library cuts a product of up to 16 rows into tiles of 256 columns and one of more rows into tiles of 128: where the
+# last turn of 256 such tiles is partly empty it loses what is missing there, and this kernel, whose workgroups are not tied to
+# turns, gains it (5,120 wide, us, the other product / this one: 24 rows of 135,168 columns 295 / 270, of 151,936 332 / 281, of whole turns,
+# 131,072 and 163,840, 232 / 240 and 286 / 294; 8 rows of 151,936 305 / 262, of 131,072 222 / 222).  At widths of 2,048, 4,096 and
+# 6,144, whose rows begin on the same channels of the memory, it loses at any count (6,144: 24 rows of 131,072 300 / 284, 8 rows 287 /
+# 269; 4,096: 24 rows 232 / 215, while up to 16 rows of it are the product's for few rows, 8 of 151,936 210 / 233; 2,048: 24 rows 123 / 109, streamed).
+# Between 2,048 and 3,072 the rows' trip costs more than is gained at 32 rows (2,560 wide, 147,456 columns: 164 / 173), and from 7,168 on
+# the library's products of whole turns are the faster at most sizes (8,192, 24 rows of 147,456: 419 / 444).
 WIDE_ROWS, WIDE_FEW_ROWS = 32, 16
-WIDE_K, WIDE_FEW_K = 2048, 4097        # the narrowest streams, with 17 to 32 rows and with fewer
 WIDE_COLUMNS = 131072
+WIDE_TURN, WIDE_FEW_TURN = 32768, 65536        # columns of 256 tiles of the library's
+WIDE_FULL = 0.95                               # ... and the share of them from which a turn counts as full
+WIDE_K, WIDE_FEW_K, WIDE_MOST_K = 3072, 4097, 6656
+WIDE_SAME_CHANNELS = 2048
 
 
 def wide_wins(rows: int, weight_rows: int, width: int, strips: bool) -> bool:
-    return (strips and 0 < rows <= WIDE_ROWS and weight_rows >= WIDE_COLUMNS and weight_rows % 16 == 0 and width % 32 == 0
-            and WIDE_K <= width <= 1 << 20 and (rows > WIDE_FEW_ROWS or width >= WIDE_FEW_K))
+    if not (strips and 0 < rows <= WIDE_ROWS and weight_rows >= WIDE_COLUMNS and weight_rows % 16 == 0 and width % 32 == 0):
+        return False
+    few = rows <= WIDE_FEW_ROWS
+    if width > WIDE_MOST_K or (few and width < WIDE_FEW_K):
+        return False
+    if width % WIDE_SAME_CHANNELS == 0:
+        return True
+    turn = WIDE_FEW_TURN if few else WIDE_TURN
+    return width >= WIDE_K and weight_rows <= WIDE_FULL * turn * -(-weight_rows // turn)
 
 
 def gemm_wide(x: torch.Tensor, strips: torch.Tensor) -> torch.Tensor:

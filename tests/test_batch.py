@@ -103,3 +103,19 @@ def test_a_step_says_how_near_its_contexts_are():
     assert (padded.near_ctx_len, padded.max_ctx_len) == (128, 1024)
     m = manager()
     assert build_batch(requests(m, [40], written=[0]), m, 1, 100, 0, "cpu", ctx_bound=64).near_ctx_len == 64
+
+
+def test_the_wide_product_leaves_full_turns_and_narrow_rows_to_the_others():
+    """Which products over very many columns go to the one out of strips: those whose library product would end in a turn of tiles that is
+    partly empty, and widths whose rows share the memory's channels; never without strips, past 32 rows, or where the other is the faster."""
+    from paged_llm_rs_amd.kernels import wide_wins
+
+    assert all(wide_wins(n, 151936, 5120, True) for n in (1, 8, 16, 17, 24, 32))
+    assert not any(wide_wins(n, 131072, w, True) for n in (1, 16, 17, 32) for w in (2560, 3072, 3584, 5120, 7168, 8192))
+    assert not any(wide_wins(n, 262144, w, True) for n in (8, 32) for w in (2560, 3072, 5120, 8192))
+    assert not any(wide_wins(n, 147456, w, True) for n in (8, 32) for w in (2560, 7168, 8192))
+    assert wide_wins(8, 163840, 5120, True) and not wide_wins(24, 163840, 5120, True)          # a turn of few rows' tiles is twice as wide
+    assert wide_wins(24, 131072, 2048, True) and wide_wins(24, 131072, 4096, True) and wide_wins(8, 131072, 6144, True)
+    assert not wide_wins(16, 131072, 2048, True) and not wide_wins(16, 151936, 4096, True)
+    assert not wide_wins(33, 151936, 5120, True) and not wide_wins(24, 151936, 5120, False) and not wide_wins(24, 128256, 5120, True)
+    assert not wide_wins(24, 151937, 5120, True) and not wide_wins(24, 151936, 5112, True) and not wide_wins(0, 151936, 5120, True)
