@@ -129,11 +129,13 @@ def context_bound(longest: int) -> int:
 
 
 def near_context(longest: int) -> int:
-    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens (in layers whose queries and
-    keys are normed and turned by the kernel in front of attention).  A fresh prompt of a few
+    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens.  A fresh prompt of a few
     dozen tokens has one tile of keys: dealt out by a bound of 1,024 it had four workgroups a tile, three without a key, and a
-    second launch to put them together (0.6B shape, a step: 37 tokens 1,385 to 1,301 us, 256 tokens 2,334 to 2,260; 37 tokens behind 700 others, whose
-    keys are worth sharing, stay as they were).  A step's shape names it, so a captured step is replayed for contexts like its own."""
+    second launch to put them together (0.6B shape, a step: 37 tokens 1,411 to 1,314 us, 200 tokens 2,310 to 2,232, 100 tokens beside eight decoded at
+    contexts of 60 2,550 to 2,231; 37 tokens behind 700 others, whose
+    keys are worth sharing, stay as they were).  Past one tile the shares are added up in another order, so the last bits of a context's keys
+    and values depend on the bound that its prompt was dealt by, as they do on ``context_bound`` past 1,024 tokens.  The plain attention
+    layers in bfloat16 go by it (``shares_by_near_context``); where a model has one, a step's shape names it, so a captured step is replayed for contexts like its own."""
     bound = 128
     while bound < longest and bound < 1024:
         bound *= 2

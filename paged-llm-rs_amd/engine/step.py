@@ -389,8 +389,8 @@ class StepRunner:
             self.eager_steps += 1
             return StepOutput(run_step(self.model, self.cache, entries, pad_to=rows, short_bounds=short_bounds))
         longest = max(e.start + len(e.tokens) for e in entries)
-        shape = (rows, len(entries), sum(len(e.want) for e in entries), tuple(sorted(short_bounds.items())),
-                 min(near_context(longest), context_bound(1)))
+        near = min(near_context(longest), context_bound(1)) if getattr(self.model, "shares_by_near_context", False) else None
+        shape = (rows, len(entries), sum(len(e.want) for e in entries), tuple(sorted(short_bounds.items())), near)
         known = shape in self._shapes
         graph = self._shapes.pop(shape, None)
         if not known:

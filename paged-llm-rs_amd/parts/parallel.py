@@ -57,6 +57,7 @@ class ParallelMixers:
         self.state_floats = at
         self.graph_safe = all(getattr(m, "graph_safe", True) for m, *_ in self.branches)
         # every branch's own limit: a captured step is laid out for each of them (see ``portion_limits`` in model.py)
+        self.shares_by_near_context = any(getattr(m, "shares_by_near_context", False) for m, *_ in self.branches)
         self.short_portions = tuple(limit for m, *_ in self.branches for limit in [getattr(m, "short_portion", None)] if limit)
 
     def cache_spec(self):

@@ -119,3 +119,37 @@ def test_the_wide_product_leaves_full_turns_and_narrow_rows_to_the_others():
     assert not wide_wins(16, 131072, 2048, True) and not wide_wins(16, 151936, 4096, True)
     assert not wide_wins(33, 151936, 5120, True) and not wide_wins(24, 151936, 5120, False) and not wide_wins(24, 128256, 5120, True)
     assert not wide_wins(24, 151937, 5120, True) and not wide_wins(24, 151936, 5112, True) and not wide_wins(0, 151936, 5120, True)
+
+
+def test_only_models_whose_layers_go_by_near_contexts_capture_a_shape_for_each(monkeypatch):
+    """One shape with contexts of 40, 100, 300 and 900 tokens: a model without such layers runs it once kernel by kernel and replays one
+    capture from then on; one with them has a capture for each bound that its layers see."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from paged_llm_rs_amd.engine import step
+
+    made = []
+
+    class Graph:
+        def __init__(self, model, cache, entries, widths, ctx_bound, rows, short_bounds):
+            made.append(max(e.start + len(e.tokens) for e in entries))
+
+        def run(self, entries):
+            return "replayed"
+
+    monkeypatch.setattr(step, "run_step", lambda *args, **kw: "eager")
+    monkeypatch.setattr(step, "ShapeGraph", Graph)
+    cache = SimpleNamespace(manager=SimpleNamespace(table=lambda seq, group: []), layout=SimpleNamespace(groups=[]), clear_state_slots=None)
+
+    def play(**model):
+        made.clear()
+        runner = step.StepRunner(SimpleNamespace(device="cpu", portion_limits=(16,), **model), cache)
+        for longest in (40, 100, 300, 900) * 3:
+            runner.run([StepEntry(1, [0] * 20, longest - 20, [19]), StepEntry(2, [0] * 17, 3, [16])])
+        return list(made), runner.eager_steps, runner.graph_steps
+
+    assert play() == ([100], 1, 11)
+    assert play(shares_by_near_context=False) == ([100], 1, 11)
+    assert play(shares_by_near_context=True) == ([100, 300, 900], 3, 9)        # (bounds of 128, 512 and 1,024)

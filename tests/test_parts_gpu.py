@@ -1316,6 +1316,28 @@ def test_a_context_of_thousands_of_tokens_in_portions_and_decoded(model_dirs, na
     assert worst <= (1e-5 if dtype == "float32" else 2e-2), f"{worst:.3e} at {where}"
 
 
+def test_a_capture_made_for_long_contexts_serves_shorter_ones(model_dirs):
+    """Portions of 20 tokens behind 1,100 of one request and then behind 600 of another: the second's are replayed from the capture that the
+    first's brought about, whose keys are dealt out by a wider bound."""
+    from paged_llm_rs_amd.engine.replay import Replayer
+
+    d = model_dirs("L", "bfloat16")
+    prompts = ru.make_prompts(TINY_INIT["L"]["config"]["vocab_size"], [1160, 660], seed=17)
+    want = ru.plain_logits(d, prompts, device="cuda:0")
+    r = Replayer(d, "bfloat16", max_tokens=ru.pool_tokens(prompts, 2), block_size=16)
+    counts, got = [], {}
+    for name, cuts in (("r0", [0, 512, 1024, 1100, 1120, 1140, 1160]), ("r1", [0, 400, 600, 620, 640, 660])):
+        for a, b in zip(cuts, cuts[1:]):
+            step = {"step": len(counts), "entries": [{"id": name, "tokens": prompts[name][a:b], "want": [b - a - 1]}], "end": []}
+            (got[(name, b - 1)],) = ru.collect(r, [step]).values()
+            counts.append((len([g for g in r.runner._shapes.values() if g is not None]), r.runner.graph_steps))
+    captures = [c for c, _ in counts]
+    assert captures[-1] == captures[-4], "the shorter contexts brought no capture of their own"
+    assert counts[-1][1] - counts[-4][1] == 3, "all three of them were replayed"
+    worst, where = ru.worst_error(got, want)
+    assert worst <= 2e-2, f"{worst:.3e} at {where}"
+
+
 # --- state slots of requests that begin --------------------------------------------------------------------------
 
 @pytest.mark.parametrize("shapes", [[(3,), (1024,), (7, 5)], [(16384,)], [(4,), (70001,)]])
