@@ -134,20 +134,23 @@ __global__ __launch_bounds__(1024) void hc_step_kernel(HcArgs a) {
         inv = 1.f / sqrtf(ss / static_cast<float>(W) + a.eps);
     }
     for (int c = mine; c < W; c += step) {            // (every thread reads back what it wrote itself)
-        T value[VEC];
+        float value[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             const float u = c == mine ? first[e] : hc_row[c + e];
             const float g = c == mine ? gain[e] : (normed ? static_cast<const float*>(a.gain)[c + e] : 1.f);
-            value[e] = from_float<T>(normed ? u * inv * g : u);
+            value[e] = normed ? u * inv * g : u;
         }
         if constexpr (VEC == 4 && sizeof(T) == 2) {
-            *reinterpret_cast<uint2*>(o + c) = *reinterpret_cast<const uint2*>(value);
+            uint2 w;
+            w.x = static_cast<uint32_t>(bf16_bits_from_float(value[0])) | (static_cast<uint32_t>(bf16_bits_from_float(value[1])) << 16);
+            w.y = static_cast<uint32_t>(bf16_bits_from_float(value[2])) | (static_cast<uint32_t>(bf16_bits_from_float(value[3])) << 16);
+            *reinterpret_cast<uint2*>(o + c) = w;
         } else if constexpr (VEC == 4) {
-            *reinterpret_cast<float4*>(o + c) = *reinterpret_cast<const float4*>(value);
+            *reinterpret_cast<float4*>(o + c) = make_float4(value[0], value[1], value[2], value[3]);
         } else {
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) o[c + e] = value[e];
+            for (int e = 0; e < VEC; ++e) o[c + e] = from_float<T>(value[e]);
         }
     }
 }
