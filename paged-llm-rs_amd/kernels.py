@@ -1363,13 +1363,15 @@ SCAN_CHUNKED_FROM = 16
 # walk and read-outs, us, plain / dealt.  Eight heads of 128 by 128 (linear attention): a prompt of 100 tokens beside one decoded token 33 / 40,
 # of 600 beside 63 46 / 66, of 1,950 beside one 63 / 77, of 4,000 beside 63 146 / 95; without decoded tokens 60, 50 and 40 36 / 43, two of
 # 512 45 / 50, 700 and 800 79 / 52, 1,500 and 1,125 93 / 80, four of up to 1,400 128 / 81, eight of 300 124 / 82, sixteen of up to
-# 100 126 / 86, 32 of 64 1,155 / 108; one request is never dealt.  Over steps of 2 to 32 such requests and 384 to 7,168 rows, five kinds and shapes
-# of state, what the lines below deal is faster but for six of 518 (up to 5% slower), by a quarter together.
+# 100 126 / 86, 32 of 64 1,155 / 108; one request is never dealt.  Over 159 steps of 1 to 64 requests and 128 to 7,168 rows and eight kinds and
+# shapes of state, what the lines below deal is faster but for 8 of 548 (up to 6% slower).
 DEALT_WORKGROUPS = 192        # whole chunks of rows, times heads and pairs of tiles, that fill the chip
 DEALT_PLAIN = 200             # chunks that a plain launch would have, from which it is the empty ones that cost
 DEALT_PLAIN_BESIDE = 2200     # the same where requests go token by token beside the chunks (how many, the launch does not know)
 DEALT_PLAIN_DELTA = 100       # the delta rule's first kernel, which is the same in either launch
 DEALT_PLAIN_RETENTION = 150   # retention (its scores cost no exponentials), from four requests on
+DEALT_PLAIN_LIGHTNING = 35    # linear attention (its values are activated once a workgroup), from three requests on and
+DEALT_LIGHTNING_TILES = 16    # ... so many heads times tiles of 64 columns: six of up to 250 tokens, eight heads, 57 / 50, two heads 34 / 41
 
 
 def deals_chunks(kind: str, requests: int, seqs: int, rows: int, max_q_len: int, heads: int, vdim: int, beside: bool) -> bool:
@@ -1384,6 +1386,9 @@ def deals_chunks(kind: str, requests: int, seqs: int, rows: int, max_q_len: int,
         return False
     if kind == "retention":
         return not beside and requests >= 4 and plain >= DEALT_PLAIN_RETENTION
+    if (kind == "lightning" and not beside and requests >= 3 and plain >= DEALT_PLAIN_LIGHTNING
+            and heads * (-(-vdim // 64)) >= DEALT_LIGHTNING_TILES):
+        return True
     fills = rows // SSD_CHUNK * heads * (-(-vdim // 128)) >= DEALT_WORKGROUPS
     return (fills and plain >= DEALT_PLAIN_BESIDE) if beside else (fills or plain >= DEALT_PLAIN)
 

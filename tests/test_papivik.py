@@ -194,4 +194,5 @@ def test_which_steps_have_their_chunks_dealt():
     assert step(2, 2816) and step(2, 1536) and step(4, 3072) and step(64, 4352, True)
     assert not step(2, 1024) and not step(2, 2816, heads=2) and step(16, 1280, heads=2) and not step(8, 2560, vdim=64)
     assert not step(2, 5120, kind="retention") and step(6, 1536, kind="retention") and not step(64, 4352, True, "delta")
+    assert step(7, 384) and not step(7, 384, heads=2) and not step(7, 384, kind="mlstm") and not step(2, 768)
     assert not deals_chunks("lightning", 16, 16, 1024, 64, 8, 128, False)             # (not padded: every request has one chunk, all of them there)
