@@ -20,53 +20,73 @@ __global__ void rmsnorm_onto_kernel(float* __restrict__ resid, const float* __re
     }
 }
 
-// The same for rows that fit the registers: a thread keeps its NV values of y and asks for the stream and the gains beside them, so that a
-// row is one trip to memory and one sum over the workgroup.  Which values a thread has, and in which order it squares them, is as above,
-// so the bits are the same.  Two rows of 1,024 take 2.4 us (3.1 value by value); 2,816 rows 9.8 (14.9), at the rate that reads and writes side by
-// side reach.  (With 16 bytes a lane 2.1 and 9.4, but a sum in another order, whose error against 64 bits is up to 2% larger; 16 bytes a
-// lane and the sum from LDS in this order 2.4 and 9.6.)
+// The same for rows of whole groups of four values: a thread asks at once for its NV groups of y, of the stream and of the gains, and for the
+// values of y that the kernel above would give it, whose squares it adds in that order: the bits are the same, a row is one trip to
+// memory (the second reading of y comes from the nearest cache) and one sum over the workgroup, and leaves 16 bytes a lane.  Two rows
+// of 1,024 take 2.2 us (3.1 value by value), 2,816 rows 9.5 (14.9), at the rate that reads and writes side by side reach.  (The squares in groups
+// of four 2.1 and 9.4, in an order whose error against 64 bits is up to 2% larger; y read once, four bytes a lane throughout, 2.4 and 9.8; y
+// exchanged through LDS 2.4 and 9.6.)
 template <typename T, int NV>
-__global__ void __launch_bounds__(256) rmsnorm_onto_held_kernel(float* __restrict__ resid, const float* __restrict__ y,
-                                                                const float* __restrict__ gain, float eps,
-                                                                T* __restrict__ rows_out, int H) {
+__global__ void __launch_bounds__(256) rmsnorm_onto_quads_kernel(float* __restrict__ resid, const float* __restrict__ y,
+                                                                 const float* __restrict__ gain, float eps,
+                                                                 T* __restrict__ rows_out, int H) {
     __shared__ float scratch[16];
     const size_t base = static_cast<size_t>(blockIdx.x) * H;
-    float v[NV], x[NV], g[NV];
+    float one[4 * NV];
+    float4 v[NV], x[NV], g[NV];
+#pragma unroll
+    for (int k = 0; k < 4 * NV; ++k) {
+        const int c = k * blockDim.x + threadIdx.x;
+        one[k] = y[base + (c < H ? c : 0)];
+    }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int c = k * blockDim.x + threadIdx.x, from = c < H ? c : 0;
-        v[k] = y[base + from];
-        x[k] = resid[base + from];
-        g[k] = gain[from];
+        const int c = (k * blockDim.x + threadIdx.x) * 4;
+        const int from = c < H ? c : 0;
+        v[k] = *reinterpret_cast<const float4*>(y + base + from);
+        x[k] = *reinterpret_cast<const float4*>(resid + base + from);
+        g[k] = *reinterpret_cast<const float4*>(gain + from);
     }
     float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < NV; ++k)
-        if (static_cast<int>(k * blockDim.x + threadIdx.x) < H) ss = fmaf(v[k], v[k], ss);
+    for (int k = 0; k < 4 * NV; ++k)
+        if (static_cast<int>(k * blockDim.x + threadIdx.x) < H) ss = fmaf(one[k], one[k], ss);
     ss = block_sum(ss, scratch);
     const float inv = 1.f / sqrtf(ss / static_cast<float>(H) + eps);
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const int c = k * blockDim.x + threadIdx.x;
+        const int c = (k * blockDim.x + threadIdx.x) * 4;
         if (c >= H) continue;
-        const float sum = fmaf(v[k] * inv, g[k], x[k]);
-        resid[base + c] = sum;
-        if (rows_out != nullptr) rows_out[base + c] = from_float<T>(sum);
+        x[k].x = fmaf(v[k].x * inv, g[k].x, x[k].x);
+        x[k].y = fmaf(v[k].y * inv, g[k].y, x[k].y);
+        x[k].z = fmaf(v[k].z * inv, g[k].z, x[k].z);
+        x[k].w = fmaf(v[k].w * inv, g[k].w, x[k].w);
+        *reinterpret_cast<float4*>(resid + base + c) = x[k];
+        if (rows_out == nullptr) continue;
+        if constexpr (sizeof(T) == 4) {
+            *reinterpret_cast<float4*>(rows_out + base + c) = x[k];
+        } else {
+            uint2 w;
+            w.x = static_cast<uint32_t>(bf16_bits_from_float(x[k].x)) | (static_cast<uint32_t>(bf16_bits_from_float(x[k].y)) << 16);
+            w.y = static_cast<uint32_t>(bf16_bits_from_float(x[k].z)) | (static_cast<uint32_t>(bf16_bits_from_float(x[k].w)) << 16);
+            *reinterpret_cast<uint2*>(rows_out + base + c) = w;
+        }
     }
 }
 
 template <typename T>
 static void launch_rmsnorm_onto(float* resid, const float* y, const float* gain, float eps, T* rows_out, int n, int H, hipStream_t stream) {
-    const int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64), each = pl_ceil_div(H, threads);
-#define ONTO_HELD(NV) rmsnorm_onto_held_kernel<T, NV><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H)
-    if (each <= 1) ONTO_HELD(1);
-    else if (each <= 2) ONTO_HELD(2);
-    else if (each <= 4) ONTO_HELD(4);
-    else if (each <= 8) ONTO_HELD(8);
-    else if (each <= 16) ONTO_HELD(16);
-    else if (each <= 32) ONTO_HELD(32);
-    else rmsnorm_onto_kernel<T><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);      // (wider rows have no registers for it)
-#undef ONTO_HELD
+    const uintptr_t at = reinterpret_cast<uintptr_t>(resid) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gain) |
+                         reinterpret_cast<uintptr_t>(rows_out);
+    const int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64), each = pl_ceil_div(H, 4 * threads);
+    if (H % 4 == 0 && each <= 8 && at % 16 == 0) {              // (wider rows have no registers for it)
+        if (each == 1) rmsnorm_onto_quads_kernel<T, 1><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
+        else if (each == 2) rmsnorm_onto_quads_kernel<T, 2><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
+        else if (each <= 4) rmsnorm_onto_quads_kernel<T, 4><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
+        else rmsnorm_onto_quads_kernel<T, 8><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
+        return;
+    }
+    rmsnorm_onto_kernel<T><<<n, threads, 0, stream>>>(resid, y, gain, eps, rows_out, H);
 }
 
 // rows_out may be null; its type is `dtype` otherwise.
