@@ -1132,11 +1132,11 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
 
 
 # Where the product over strips and very many columns beats the others, timed at 1 to 32 rows over 131,072 to 524,288 columns and widths from 2,048
-# to 8,192.  The library cuts a product of up to 16 rows into tiles of 256 columns and one of more rows into tiles of 128: where the
-# last turn of 256 such tiles is partly empty it loses what is missing there, and this kernel, whose workgroups are not tied to
+# to 8,192.  The library's times follow turns of 256 tiles, of 256 columns for up to 16 rows and of 128 for more: where the
+# last turn is partly empty it loses what is missing there, and this kernel, whose workgroups are not tied to
 # turns, gains it (5,120 wide, us, the other product / this one: 24 rows of 135,168 columns 295 / 270, of 151,936 332 / 281, of whole turns,
 # 131,072 and 163,840, 232 / 240 and 286 / 294; 8 rows of 151,936 305 / 262, of 131,072 222 / 222).  At widths of 2,048, 4,096 and
-# 6,144, whose rows begin on the same channels of the memory, it loses at any count (6,144: 24 rows of 131,072 300 / 284, 8 rows 287 /
+# 6,144 (rows of w a multiple of 4 KB apart, which the strips are not) it loses at any count (6,144: 24 rows of 131,072 300 / 284, 8 rows 287 /
 # 269; 4,096: 24 rows 232 / 215, while up to 16 rows of it are the product's for few rows, 8 of 151,936 210 / 233; 2,048: 24 rows 123 / 109, streamed).
 # Between 2,048 and 3,072 the rows' trip costs more than is gained at 32 rows (2,560 wide, 147,456 columns: 164 / 173), and from 7,168 on
 # the library's products of whole turns are the faster at most sizes (8,192, 24 rows of 147,456: 419 / 444).
@@ -1145,7 +1145,7 @@ WIDE_COLUMNS = 131072
 WIDE_TURN, WIDE_FEW_TURN = 32768, 65536        # columns of 256 tiles of the library's
 WIDE_FULL = 0.95                               # ... and the share of them from which a turn counts as full
 WIDE_K, WIDE_FEW_K, WIDE_MOST_K = 3072, 4097, 6656
-WIDE_SAME_CHANNELS = 2048
+WIDE_ALIKE = 2048                              # widths of whole multiples: rows 4 KB, or a multiple, apart
 
 
 def wide_wins(rows: int, weight_rows: int, width: int, strips: bool) -> bool:
@@ -1154,7 +1154,7 @@ def wide_wins(rows: int, weight_rows: int, width: int, strips: bool) -> bool:
     few = rows <= WIDE_FEW_ROWS
     if width > WIDE_MOST_K or (few and width < WIDE_FEW_K):
         return False
-    if width % WIDE_SAME_CHANNELS == 0:
+    if width % WIDE_ALIKE == 0:
         return True
     turn = WIDE_FEW_TURN if few else WIDE_TURN
     return width >= WIDE_K and weight_rows <= WIDE_FULL * turn * -(-weight_rows // turn)
@@ -1489,7 +1489,7 @@ def recurrent_scan(kind: str, qkv: torch.Tensor, q_off: int, k_off: int, v_off: 
               0 if gates is None else gates.shape[1], g1_off, g2_off, _ptr(p1), _ptr(p2), float(cap),
               state.data_ptr(), stride, 0, hdv, hdv + heads * tiles * dim, out.data_ptr(), batch.q_start.data_ptr(),
               batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
-    beside = _brings_short_requests(batch)
+    beside = chunked and _brings_short_requests(batch)
     if not chunked or beside:
         _check(library().pl_recurrent_scan(*common[:12], 0, *common[12:], heads, qk_heads, dim, vdim, SCAN_CHUNKED_FROM if chunked else 0, _stream()))
     dealt = _dealt(kind, batch, n, heads, vdim, beside, dealt)
@@ -1531,7 +1531,7 @@ def _ssd_scan(qkv, q_off: int, k_off: int, v_off: int, state, stride: int, batch
     common = (qkv.data_ptr(), qkv.shape[1], q_off, k_off, v_off, gates.data_ptr(), gates.shape[1], g_off, *constants, state.data_ptr(),
               stride, out.data_ptr(), batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.state_slots.data_ptr(), batch.num_seqs)
     below = SCAN_CHUNKED_FROM if chunked else 0
-    beside = batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
+    beside = chunked and batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
     if not chunked or beside:
         if lib.pl_ssd_step_applies(V, stride) and state.data_ptr() % 16 == 0:
             _check(lib.pl_ssd_step(*common, H, G, N, V, below, stream))
@@ -1583,7 +1583,7 @@ def retention_scan(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, state
         return out
     lib, stream = library(), _stream()
     chunked = bool(chunked) and batch.max_q_len >= SCAN_CHUNKED_FROM
-    beside = batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
+    beside = chunked and batch.tokens_of_short_requests(SCAN_CHUNKED_FROM) > 0
     by_token = not chunked or beside
     steps = lib.pl_ssd_step_applies(vdim, stride) and state.data_ptr() % 16 == 0
     turn = (_ptr(freq), turned, float(amplitude), float(k_scale))

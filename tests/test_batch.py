@@ -107,7 +107,7 @@ def test_a_step_says_how_near_its_contexts_are():
 
 def test_the_wide_product_leaves_full_turns_and_narrow_rows_to_the_others():
     """Which products over very many columns go to the one out of strips: those whose library product would end in a turn of tiles that is
-    partly empty, and widths whose rows share the memory's channels; never without strips, past 32 rows, or where the other is the faster."""
+    partly empty, and widths whose rows are a multiple of 4 KB apart; never without strips, past 32 rows, or where the other is the faster."""
     from paged_llm_rs_amd.kernels import wide_wins
 
     assert all(wide_wins(n, 151936, 5120, True) for n in (1, 8, 16, 17, 24, 32))
