@@ -56,6 +56,8 @@ def _signatures(lib) -> None:
         "pl_gemm_skinny_hand": [p, p, p, i, i, i, i, i, i, p, i, f, p, p, p, i, p],
         "pl_gemm_skinny_hand_applies": [i, i, i, i, i],
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
+        "pl_gemm_strips": [p, p, p, i, i, i, p],
+        "pl_gemm_strips_apply": [i, i, i],
         "pl_gemm_tiled_applies": [i, i, i, i],
         "pl_gemm_stream": [p, p, p, p, i, i, i, i, i, i, i, p],
         "pl_gemm_stream_splits": [i, i, i, i],
@@ -1128,6 +1130,42 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
         out, epilogue = torch.empty((M, N), dtype=torch.bfloat16, device=x.device), (1 if swiglu else 0)
     _check(library().pl_gemm_tiled(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, epilogue,
                                    activation_code(activation), _stream()))
+    return out
+
+
+# Where the product over strips with the gated activation inside beats the others (the library's product and the activation kernel, or
+# ``gemm_tiled``), timed at 65 to 8,192 rows of 13 pairs of widths.  Up to a width of 2,048 it does at every size until the operations are what
+# counts, which the library's tiles of 256 x 256 do at up to 1.4 PFLOP/s and this one's at 1.0 to 1.2 (us, before / this one; 1,024 wide,
+# 3,072 columns: 65 rows 14 / 7, 2,048 36 / 26, 8,192 104 / 102; 8,192 columns: 2,560 rows 115 / 89, 4,096 140 / 151; 2,048 wide, 6,144 columns:
+# 1,024 rows 69 / 45, 1,150 58 / 60).  Beyond, it wins by what the library's turns of 256 such tiles leave empty, and up to 128 rows (12,288 columns of
+# 4,096: 65 rows 59 / 51, 256 83 / 72, turns 0.38 full, 576 124 / 114, 0.56 full; 14,336 of 4,096: 512 rows 105 / 122, 0.88 full; 25,600 of
+# 5,120: 128 rows 128 / 113, 256 166 / 168, 0.78 full).
+STRIPS_WORK = ((1024, 27e9), (2048, 13e9))      # widths up to, and rows x columns x width up to
+STRIPS_WIDE_ROWS = 128
+STRIPS_WIDE_MOST_ROWS = 704
+STRIPS_WIDE_TURNS = 0.6
+
+
+def strips_swiglu_wins(rows: int, columns: int, width: int) -> bool:
+    if rows <= SKINNY_ROWS or not library().pl_gemm_strips_apply(rows, columns, width):
+        return False
+    for most, work in STRIPS_WORK:
+        if width <= most:
+            return rows * columns * width <= work
+    tiles = -(-rows // 256) * -(-2 * columns // 256)
+    return rows <= STRIPS_WIDE_ROWS or (rows <= STRIPS_WIDE_MOST_ROWS and tiles <= STRIPS_WIDE_TURNS * 256 * -(-tiles // 256))
+
+
+def gemm_strips_swiglu(x: torch.Tensor, strips: torch.Tensor) -> torch.Tensor:
+    """silu(x . gate^T) * (x . up^T) for many rows of bfloat16, 32-bit sums; ``strips``: what ``weights_in_strips`` made of
+    the weights [gate | up] stacked."""
+    _need(x, "matrix product input", None, torch.bfloat16)
+    _need(strips, "weights in strips", None, torch.bfloat16)
+    if x.dim() != 2 or strips.dim() != 2 or strips.shape[1] != x.shape[1] or strips.shape[0] % 32:
+        raise TensorError(f"weights in strips of shape {tuple(strips.shape)} for an input of shape {tuple(x.shape)}")
+    M, K = x.shape
+    out = torch.empty((M, strips.shape[0] // 2), dtype=torch.bfloat16, device=x.device)
+    _check(library().pl_gemm_strips(x.data_ptr(), strips.data_ptr(), out.data_ptr(), M, out.shape[1], K, _stream()))
     return out
 
 

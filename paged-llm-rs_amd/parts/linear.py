@@ -112,6 +112,9 @@ class Linear:
                 kernels.gemm_split_library(x, self.weight, splits, add_into=add_into, turned=self.turned)
                 return None
         if swiglu:
+            if (self.strips is not None and kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
+                    and kernels.strips_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features)):
+                return kernels.gemm_strips_swiglu(x, self.strips)
             if kernels.tiled_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features):
                 return kernels.gemm_tiled(x, self.weight, swiglu=True, activation=activation)
             return kernels.swiglu(kernels.linear_bf16(x, self.weight, x.dtype, self.strips, self.turned), activation=activation)

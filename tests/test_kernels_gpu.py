@@ -2048,3 +2048,27 @@ def test_32_bit_attention_of_a_step_without_tokens(requests):
                             num_tokens=0, max_ctx_len=64)
     out = torch.empty(0, nq * d, device=DEV)
     assert kernels.paged_attention(torch.empty(0, (nq + 2 * nkv) * d, device=DEV), out, batch, kv, nq, nkv, d, d ** -0.5) is out
+
+
+@pytest.mark.parametrize("N,K", [(16, 64), (48, 128), (208, 192), (1040, 320), (3072, 1024)])
+def test_the_gated_product_out_of_strips(N, K):
+    """Every shape of tile (the rows and columns choose it), tiles that reach past the rows and the columns, an odd count of stages of 64 k
+    and one alone: 64-bit arithmetic within bfloat16's rounding of the result (2^-9, a factor of two for the 32-bit sums' part), and every
+    row the same whichever rows stand beside it in its tile."""
+    from paged_llm_rs_amd import kernels
+
+    w = (torch.randn(2 * N, K, device=DEV) * 3 / K ** 0.5).bfloat16()
+    strips = kernels.weights_in_strips(w)
+    for n in (65, 96, 129, 300, 520, 700, 1030, 2050):
+        x = torch.randn(n, K, device=DEV).bfloat16()
+        assert kernels.strips_swiglu_wins(n, N, K)
+        both = x.double() @ w.double().T
+        want = torch.nn.functional.silu(both[:, :N]) * both[:, N:]
+        got = kernels.gemm_strips_swiglu(x, strips)
+        assert rel(got, want) < 2.0 ** -8, f"{n} rows"
+        assert float((got.double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max()), f"{n} rows"
+        assert torch.equal(got, kernels.gemm_strips_swiglu(x, strips))
+    x = torch.zeros(130, K, device=DEV, dtype=torch.bfloat16)
+    x[7, 0], x[8, K - 1] = math.inf, math.nan
+    y = kernels.gemm_strips_swiglu(x, strips)
+    assert bool(y[8].isnan().all()) and not bool(y[7].isfinite().all()) and not bool(y[torch.arange(130, device=DEV).sub(7.5).abs() > 1].any())
