@@ -1,0 +1,475 @@
+// y[M, N] = x[M, K] . w[N, K]^T for many rows of bfloat16, 32-bit sums, on the matrix cores, with what stands around the product fused into it:
+// the norm in front of it (what an earlier product left of it), the gated activation, the sum into the residual stream and the norm behind that.
+//
+// A workgroup of four waves owns 32 RT rows of x and 128 CT rows of w; a wave all of the former and a quarter of the latter, as tiles of
+// v_mfma_f32_32x32x16_bf16 with A = w: a lane then holds, for one row of x, groups of four neighbouring columns.  K is walked 64 a stage, two stages
+// and more asked for ahead.  The rows of x go through registers and two stages of LDS, their 16-byte pieces permuted by their row against bank
+// conflicts.  The weights in strips (kernels.weights_in_strips: 16 rows by 32 k as the lanes of a wave take them) go from memory straight into the
+// registers that multiply them, and pass LDS by: it is read once for CT matrix instructions, where a tile whose operands are shared by two waves each
+// (gemm_tiled.hip) reads it once an instruction.  Weights in rows, as they are stored, go through LDS as x does, a wave's through a part of
+// its own (100 and 2,048 rows, 3,072 gated columns of 1,024: 9.8 and 28.3 us, 9.0 and 27.5 in strips).
+//
+// Reads of LDS, loads and stores into LDS are dealt between the matrix instructions one by one: asked for together in front of them
+// they kept the matrix cores waiting for what LDS gives a compute unit in turn (a stage of 64 k by 128 rows by 256 columns 0.71 us, 0.54 so;
+// its instructions alone 0.43).  The loop is bound by the matrix cores at 70 to 85% of their rate while the operands come out of L2, by the
+// 64 bytes a clock that a compute unit takes in at the small tiles, and with few rows before wide weights by the weights' trip from memory.
+// Beside it a workgroup pays some 5 us for its launch, its first loads and its tile's way out.
+//
+// us, before (the library's product and the kernels around it; gemm_tiled for gated columns up to 1,024 rows) / this one.  Gated, 3,072 columns
+// of 1,024: 100 rows 17 / 9.4, 512 17.5 / 12.3, 1,024 25 / 18, 2,048 37 / 28, 4,096 64 / 51; 12,288 of 4,096: 65 rows 57 / 45, 575 125 / 112, and
+// 2,048 294 / 332: the library's.  Added into the stream with the norm behind it, 1,024 columns: of 2,048, 512 rows 13.7 / 13.2, 2,048 22.5 / 16.7; of
+// 3,072, 2,048 rows 26.6 / 21.1.  Plain, 4,096 columns of 1,024: 300 rows 10 / 7.5, 1,024 13.3 / 12.3, 2,048 20.3 / 20.8.
+#include "common.hpp"
+
+typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 gm_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float gm_f32x16 __attribute__((ext_vector_type(16)));
+typedef float gm_f32x4 __attribute__((ext_vector_type(4)));
+typedef float gm_f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t gm_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t gm_u32x2 __attribute__((ext_vector_type(2)));
+
+#define GM_STORE 0         // y (bfloat16) = result
+#define GM_SWIGLU 1        // w is [gate | up], N rows each: y (bfloat16) = silu(gate) * up
+#define GM_ADD 2           // y (32-bit, the residual stream) += result
+#define GM_STORE32 3       // y (32-bit) = result
+
+#define GM_BK 64           // K a stage
+#define GM_STRIPE 64       // columns of the stream whose squares are one number of a norm handed forward
+#define GM_BAND 16         // row tiles that are walked before the next column tile's
+
+// Norms on both sides of a product (kernels.HandedNorm).
+struct GmNorms {
+    const float* taken;        // [M, taken_count]: sums of squares of the rows of the stream that x is bfloat16(row * gain) of; the
+    int taken_count;           // (a multiple of four) result is scaled by 1 / sqrt(their sum / K + eps); null: x is what it is
+    float eps;
+    const float* gain;         // [N] of the norm behind the updated stream (GM_ADD): left behind are
+    bf16_t* rows;              // [M, N] bfloat16(y * gain) and
+    float* sums;               // [M, N / 64] the sums of squares of every 64 columns of y; null: no norm
+};
+#define GM_TAKEN_MOST 64
+
+__device__ __forceinline__ uint32_t gm_pack2(float lo, float hi) {
+    const gm_f32x2 pair = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, gm_bf16x2));
+}
+
+// silu(g), the division by the hardware's reciprocal (1 ulp of 32 bits; what leaves is bfloat16)
+__device__ __forceinline__ float gm_silu(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
+
+template <int V>
+struct GmInt {
+    static constexpr int value = V;
+};
+
+// The workgroup's tile.  Workgroups go to the eight XCDs in turn; an XCD gets tiles that follow each other, the row tiles of one column
+// tile first, so that its L2 reads a row of w once.
+__device__ __forceinline__ void gm_tile(int at, int row_tiles, int col_tiles, int& row_tile, int& col_tile) {
+    const int total = row_tiles * col_tiles, each = total / 8, rest = total % 8;
+    const int xcd = at % 8;
+    const int work = xcd * each + min(xcd, rest) + at / 8;
+    const int band = work / (GM_BAND * col_tiles), in_band = work - band * GM_BAND * col_tiles;
+    const int rows = min(GM_BAND, row_tiles - band * GM_BAND);
+    row_tile = band * GM_BAND + in_band % rows;
+    col_tile = in_band / rows;
+}
+
+// The sum over 16 lanes that stand side by side, by each of them.
+__device__ __forceinline__ float gm_sum16(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));      // quad_perm [1,0,3,2]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));      // quad_perm [2,3,0,1]
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));     // lane i of 8 takes 7 - i
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true));     // lane i of 16 takes 15 - i
+    return v;
+}
+
+constexpr int gm_out_cols(int CT, int epi) { return 4 * (epi == GM_SWIGLU ? 16 : 32) * CT; }
+constexpr bool gm_is_32(int epi) { return epi == GM_ADD || epi == GM_STORE32; }
+// bytes between two rows of the tile on its way out
+constexpr int gm_pitch(int CT, int epi) { return gm_out_cols(CT, epi) * (gm_is_32(epi) ? 4 : 2) + 16; }
+// ... and of the LDS of a workgroup: two stages of x (and of weights in rows), or the tile on its way out, and 1 / rms of its rows
+constexpr int gm_lds_bytes(int CT, int RT, int epi, bool strips) {
+    const int in = 2 * 32 * RT * GM_BK * 2 + (strips ? 0 : 4 * 2 * 32 * CT * GM_BK * 2), out = 32 * RT * gm_pitch(CT, epi);
+    return (in > out ? in : out) + 32 * RT * 4;
+}
+
+// CT, RT: a wave's tiles of 32 rows of w (with GM_SWIGLU 16 of gate, 16 of up) and of 32 rows of x.  N a multiple of 16, K of 64; rows and columns past the
+// matrices are read from their last and not stored.
+// STRIPS: the weights in strips; otherwise in rows as they are stored, which go through registers and LDS as the rows of x do, each wave's
+// through a part of LDS of its own.  The sums are the same, k after k: the layout changes no bit.
+template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS>
+__global__ void __launch_bounds__(256, PER_SIMD)
+gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weights, void* __restrict__ y_, int M, int N, int K,
+                   int row_tiles, int col_tiles, GmNorms norms) {
+    constexpr int ROWS = 32 * RT, STAGE = ROWS * GM_BK * 2;
+    extern __shared__ __attribute__((aligned(16))) char gm_lds[];          // two stages of x [row][64], then the tile on its way out
+    int row_tile, col_tile;
+    gm_tile(blockIdx.x, row_tiles, col_tiles, row_tile, col_tile);
+    const int m0 = row_tile * ROWS;
+    const int tid = threadIdx.x, lane = tid % PL_WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / PL_WAVE);
+    const int r32 = lane % 32, h = lane / 32;
+    constexpr int COLS = gm_out_cols(CT, EPI) / 4;                         // output columns a wave
+    const int n_wave = (col_tile * 4 + wave) * COLS;                       // the wave's first
+
+    const int last_strip = N / 16 - 1;                                     // (of gate alone)
+    auto strip_of = [&](int c, int half) {                                 // the strip of either half of an instruction's 32 rows
+        return EPI == GM_SWIGLU ? min(n_wave / 16 + c, last_strip) + half * (N / 16) : min(n_wave / 16 + 2 * c + half, last_strip);
+    };
+    // bytes from the weights' first: a lane's operands in strips; its pieces of rows 0 .. 7 of either half
+    uint32_t w_at[CT][STRIPS ? 1 : 2];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        if constexpr (STRIPS) {
+            w_at[c][0] = static_cast<uint32_t>(strip_of(c, r32 / 16)) * static_cast<uint32_t>(K) * 32u + h * 256 + r32 % 16 * 16;
+        } else {
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+                w_at[c][half] = (static_cast<uint32_t>(strip_of(c, half)) * 16u + lane / 8) * static_cast<uint32_t>(K) * 2u + lane % 8 * 16;
+        }
+    }
+    uint32_t x_at[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+        x_at[i] = static_cast<uint32_t>(min(m0 + tid / 8 + 32 * i, M - 1)) * static_cast<uint32_t>(K) * 2u + tid % 8 * 16;
+    char* const w_lds = gm_lds + 2 * STAGE + wave * 2 * CT * 4096;         // the wave's weights in rows: two stages of [32 CT][64]
+    char* const put_w_at = w_lds + lane / 8 * 128 + ((lane % 8) ^ (lane / 8)) * 16;
+    char* const put_at = gm_lds + tid / 8 * 128 + ((tid % 8) ^ (tid / 8 % 8)) * 16;
+    int b_at[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) b_at[kk] = r32 * 128 + (((2 * kk + h) ^ (r32 % 8)) * 16);
+
+    const int stages = K / GM_BK;
+    // w: weights on their way or, in strips, the operands [set][k / 16 in the stage][c]; in rows the pieces [set][rows / 8][c], whose operands are a
+    gm_bf16x8 w[2][4][CT], a[2][CT], b[2][RT];
+    gm_u32x4 xr[2][RT];
+    gm_f32x16 acc[CT][RT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[c][t][i] = 0.f;
+
+    // (past the end the last stage is asked for again)
+    auto ask_w = [&](auto set, auto kk, int s, int c) {
+        constexpr int KK = decltype(kk)::value;
+        const char* from = reinterpret_cast<const char*>(weights) + static_cast<size_t>(min(s, stages - 1)) * (STRIPS ? 2048 : 128);
+        if constexpr (STRIPS) w[set.value][KK][c] = *reinterpret_cast<const gm_bf16x8*>(from + KK * 512 + w_at[c][0]);
+        else w[set.value][KK][c] = *reinterpret_cast<const gm_bf16x8*>(from + static_cast<size_t>(KK % 2) * 16 * K + w_at[c][KK / 2]);
+    };
+    auto put_w = [&](auto set, auto kk, int s, int c) {
+        *reinterpret_cast<gm_bf16x8*>(put_w_at + (s % 2) * CT * 4096 + c * 4096 + kk.value * 1024) = w[set.value][kk.value][c];
+    };
+    auto read_a = [&](auto set, int s, int kk, int c) {
+        a[set.value][c] = *reinterpret_cast<const gm_bf16x8*>(w_lds + (s % 2) * CT * 4096 + c * 4096 + b_at[kk]);
+    };
+    auto ask_x = [&](auto set, int s, int i) {
+        const char* from = reinterpret_cast<const char*>(x) + static_cast<size_t>(min(s, stages - 1)) * 128;
+        xr[set.value][i] = *reinterpret_cast<const gm_u32x4*>(from + x_at[i]);
+    };
+    auto put_x = [&](auto set, int s, int i) {
+        *reinterpret_cast<gm_u32x4*>(put_at + (s % 2) * STAGE + i * 32 * 128) = xr[set.value][i];
+    };
+    auto read_b = [&](auto set, int s, int kk, int t) {
+        b[set.value][t] = *reinterpret_cast<const gm_bf16x8*>(gm_lds + (s % 2) * STAGE + b_at[kk] + t * 32 * 128);
+    };
+    auto meet = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // 16 k.  The next 16's operands are read, and what else there is to do is done, an instruction of it between two of the matrix cores'.
+    // (The weights in rows: a stage's are laid down in LDS by the wave that reads them, a quarter a slice, while the stage before is multiplied.)
+    auto slice = [&](auto set, auto kk, int s) {
+        constexpr int KK = decltype(kk)::value, SET = decltype(set)::value;
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                const int m = c * RT + t;
+                if (KK == 3 && m == 1) meet();
+                if (m >= 1 && m <= RT) {
+                    if constexpr (KK < 3) read_b(GmInt<(KK + 1) % 2>{}, s, KK + 1, m - 1);
+                    else read_b(GmInt<0>{}, s + 1, 0, m - 1);
+                }
+                if constexpr (!STRIPS) {
+                    // (the last quarter is written in front of the first read of what it is a part of)
+                    if (t == 0) put_w(GmInt<1 - SET>{}, kk, s + 1, c);
+                    if (c == CT - 1 && t >= RT - CT && t < RT) {
+                        if constexpr (KK < 3) read_a(GmInt<(KK + 1) % 2>{}, s, KK + 1, t - RT + CT);
+                        else read_a(GmInt<0>{}, s + 1, 0, t - RT + CT);
+                    }
+                }
+                if (KK == 1 && c == (CT > 1 ? 1 : 0)) put_x(GmInt<1 - SET>{}, s + 1, t);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (STRIPS) acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[SET][KK][c], b[KK % 2][t], acc[c][t], 0, 0, 0);
+                else acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[KK % 2][c], b[KK % 2][t], acc[c][t], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (KK == 2 && c == 0) ask_x(GmInt<1 - SET>{}, s + 3, t);
+                if (t == RT - 1) {
+                    if constexpr (STRIPS) ask_w(set, kk, s + 2, c);
+                    else ask_w(GmInt<1 - SET>{}, kk, s + 3, c);
+                }
+                if (CT == 1 && t == RT - 1) {
+                    if constexpr (KK < 3) read_b(GmInt<(KK + 1) % 2>{}, s, KK + 1, t);
+                    else read_b(GmInt<0>{}, s + 1, 0, t);
+                }
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stage = [&](auto set, int s) {
+        slice(set, GmInt<0>{}, s);
+        slice(set, GmInt<1>{}, s);
+        slice(set, GmInt<2>{}, s);
+        slice(set, GmInt<3>{}, s);
+    };
+    auto ask_all = [&](auto set, int s) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) ask_x(set, s, i);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            ask_w(set, GmInt<0>{}, s, c);
+            ask_w(set, GmInt<1>{}, s, c);
+            ask_w(set, GmInt<2>{}, s, c);
+            ask_w(set, GmInt<3>{}, s, c);
+        }
+    };
+    // the sums of squares of the tile's rows, four lanes a row, asked for first
+    constexpr int PASSES = (ROWS + 63) / 64;
+    gm_f32x4 sums[TAKES ? PASSES : 1][GM_TAKEN_MOST / 16];
+    if constexpr (TAKES) {
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) {
+            const float* from = norms.taken + static_cast<size_t>(min(m0 + 64 * q + tid / 4, M - 1)) * norms.taken_count + tid % 4 * 4;
+#pragma unroll
+            for (int i = 0; i < GM_TAKEN_MOST / 16; ++i) {
+                sums[q][i] = gm_f32x4{0.f, 0.f, 0.f, 0.f};
+                if (16 * i + tid % 4 * 4 < norms.taken_count) sums[q][i] = *reinterpret_cast<const gm_f32x4*>(from + 16 * i);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    ask_all(GmInt<0>{}, 0);
+    ask_all(GmInt<1>{}, 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) put_x(GmInt<0>{}, 0, i);
+#pragma unroll
+    for (int i = 0; i < RT; ++i) ask_x(GmInt<0>{}, 2, i);
+    if constexpr (!STRIPS) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            put_w(GmInt<0>{}, GmInt<0>{}, 0, c);
+            put_w(GmInt<0>{}, GmInt<1>{}, 0, c);
+            put_w(GmInt<0>{}, GmInt<2>{}, 0, c);
+            put_w(GmInt<0>{}, GmInt<3>{}, 0, c);
+            ask_w(GmInt<0>{}, GmInt<0>{}, 2, c);
+            ask_w(GmInt<0>{}, GmInt<1>{}, 2, c);
+            ask_w(GmInt<0>{}, GmInt<2>{}, 2, c);
+            ask_w(GmInt<0>{}, GmInt<3>{}, 2, c);
+        }
+    }
+    float* const scales = reinterpret_cast<float*>(gm_lds + gm_lds_bytes(CT, RT, EPI, STRIPS) - ROWS * 4);
+    if constexpr (TAKES) {
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) {
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < GM_TAKEN_MOST / 16; ++i) sum += (sums[q][i][0] + sums[q][i][1]) + (sums[q][i][2] + sums[q][i][3]);
+            sum += __shfl_xor(sum, 1, PL_WAVE);
+            sum += __shfl_xor(sum, 2, PL_WAVE);
+            if (tid % 4 == 0 && 64 * q + tid / 4 < ROWS) scales[64 * q + tid / 4] = 1.f / sqrtf(sum / K + norms.eps);
+        }
+    }
+    meet();
+#pragma unroll
+    for (int t = 0; t < RT; ++t) read_b(GmInt<0>{}, 0, 0, t);
+    if constexpr (!STRIPS) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) read_a(GmInt<0>{}, 0, 0, c);
+    }
+    int s = 0;
+    for (; s + 1 < stages; s += 2) {
+        stage(GmInt<0>{}, s);
+        stage(GmInt<1>{}, s + 1);
+    }
+    if (s < stages) stage(GmInt<0>{}, s);
+    constexpr int PITCH = gm_pitch(CT, EPI), OUT_COLS = 4 * COLS;
+    const int n0 = col_tile * OUT_COLS;
+    // (32-bit results: a thread's four columns are the same in all of its rows)
+    constexpr bool IS_32 = gm_is_32(EPI);
+    constexpr int LANES = OUT_COLS / (IS_32 ? 4 : 8), STEP = 256 / LANES, AHEAD = 8;          // lanes of a row, rows a pass
+    const int col = n0 + tid % LANES * 4;
+    gm_f32x4 old[AHEAD];
+    auto ask_old = [&](int r0) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int row = m0 + r0 + i * STEP + tid / LANES;
+            old[i] = *reinterpret_cast<const gm_f32x4*>(static_cast<const float*>(y_) + static_cast<size_t>(min(row, M - 1)) * N + min(col, N - 4));
+        }
+    };
+    if constexpr (EPI == GM_ADD) ask_old(0);
+    __syncthreads();
+
+    // The tile leaves through LDS in whole rows.  acc[c][t][4 j + i]: row 32 t + r32, row of A 8 j + 4 h + i
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        char* at_row = gm_lds + (32 * t + r32) * PITCH + wave * COLS * (IS_32 ? 4 : 2);
+        const float scale = TAKES ? scales[32 * t + r32] : 1.f;
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int j = 0; j < (EPI == GM_SWIGLU ? 2 : 4); ++j) {
+                gm_f32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = acc[c][t][4 * j + i] * scale;
+                    if constexpr (EPI == GM_SWIGLU) v[i] = gm_silu(v[i]) * (acc[c][t][4 * (j + 2) + i] * scale);
+                }
+                const int at = (EPI == GM_SWIGLU ? 16 : 32) * c + 8 * j + 4 * h;
+                if constexpr (IS_32) {
+                    *reinterpret_cast<gm_f32x4*>(at_row + at * 4) = v;
+                } else {
+                    const gm_u32x2 packed = {gm_pack2(v[0], v[1]), gm_pack2(v[2], v[3])};
+                    *reinterpret_cast<gm_u32x2*>(at_row + at * 2) = packed;
+                }
+            }
+    }
+    __syncthreads();
+    if constexpr (!IS_32) {
+        bf16_t* y = static_cast<bf16_t*>(y_);
+        for (int i = tid; i < ROWS * LANES; i += 256) {
+            const int r = i / LANES, piece = i % LANES;
+            if (m0 + r < M && n0 + piece * 8 < N)
+                *reinterpret_cast<gm_u32x4*>(y + static_cast<size_t>(m0 + r) * N + n0 + piece * 8) =
+                    *reinterpret_cast<const gm_u32x4*>(gm_lds + r * PITCH + piece * 16);
+        }
+    } else {
+        static_assert(!IS_32 || (256 % LANES == 0 && LANES % 16 == 0 && ROWS % (STEP * AHEAD) == 0), "whole passes");
+        const bool hands = EPI == GM_ADD && norms.gain != nullptr;
+        gm_f32x4 gain = {0.f, 0.f, 0.f, 0.f};
+        if (hands) gain = *reinterpret_cast<const gm_f32x4*>(norms.gain + min(col, N - 4));
+        for (int r0 = 0; r0 < ROWS; r0 += STEP * AHEAD) {
+            if (EPI == GM_ADD && r0 > 0) ask_old(r0);
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                const int r = r0 + i * STEP + tid / LANES, row = m0 + r;
+                const bool there = row < M && col < N;
+                gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(gm_lds + r * PITCH + tid % LANES * 16);
+                if constexpr (EPI == GM_ADD) v += old[i];
+                const size_t to = static_cast<size_t>(row) * N + col;
+                if (there) *reinterpret_cast<gm_f32x4*>(static_cast<float*>(y_) + to) = v;
+                if (hands) {
+                    const float square = gm_sum16(there ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f);
+                    if (there) {
+                        const gm_u32x2 packed = {gm_pack2(v[0] * gain[0], v[1] * gain[1]), gm_pack2(v[2] * gain[2], v[3] * gain[3])};
+                        *reinterpret_cast<gm_u32x2*>(norms.rows + to) = packed;
+                        if (tid % 16 == 0) norms.sums[static_cast<size_t>(row) * (N / GM_STRIPE) + col / GM_STRIPE] = square;
+                    }
+                }
+            }
+        }
+    }
+}
+
+struct GmProduct {
+    const void *x, *weights;
+    bool strips;
+    void* y;
+    int M, N, K;
+    GmNorms norms;
+};
+
+template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS>
+static int gm_launch_one(const GmProduct& g, hipStream_t stream) {
+    constexpr int lds = gm_lds_bytes(CT, RT, EPI, STRIPS);
+    static_assert(lds <= 160 * 1024, "a workgroup's LDS");
+    const int row_tiles = pl_ceil_div(g.M, 32 * RT), col_tiles = pl_ceil_div(g.N, gm_out_cols(CT, EPI));
+    if constexpr (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_many_kernel<CT, RT, PER_SIMD, EPI, TAKES, STRIPS>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        PL_REQUIRE(e == hipSuccess, "product of many rows: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    }
+    gemm_many_kernel<CT, RT, PER_SIMD, EPI, TAKES, STRIPS><<<row_tiles * col_tiles, 256, lds, stream>>>(
+        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms);
+    PL_CHECK_LAUNCH("gemm_many");
+    return 0;
+}
+
+template <int CT, int RT, int PER_SIMD, int EPI>
+static int gm_launch(const GmProduct& g, hipStream_t stream) {
+    if constexpr (!gm_is_32(EPI)) {
+        if (g.norms.taken != nullptr)
+            return g.strips ? gm_launch_one<CT, RT, PER_SIMD, EPI, true, true>(g, stream) : gm_launch_one<CT, RT, PER_SIMD, EPI, true, false>(g, stream);
+    }
+    return g.strips ? gm_launch_one<CT, RT, PER_SIMD, EPI, false, true>(g, stream) : gm_launch_one<CT, RT, PER_SIMD, EPI, false, false>(g, stream);
+}
+
+// The tiles there are, and what one costs a compute unit: us for 64 k, and for the tile itself by what is done with it, as timed one tile a
+// compute unit (K of 1,024 and of 3,072).  A launch is taken to last as long as the compute unit with most tiles: that is the order of the
+// shapes in all of 40 timed products (65 to 4,096 rows of 1,024, 4,096 and 5,120) but for differences of a few per cent.  (32-bit
+// results of the largest tile would not fit into LDS.)
+struct GmShape {
+    int ct, rt;
+    float stage, tile[4];      // (by epilogue)
+};
+static const GmShape GM_SHAPES[] = {{1, 2, 0.25f, {1.5f, 3.0f, 4.0f, 2.5f}},
+                                    {1, 4, 0.37f, {2.2f, 2.9f, 8.0f, 4.0f}},
+                                    {2, 3, 0.425f, {3.0f, 5.2f, 10.f, 5.0f}},
+                                    {2, 4, 0.54f, {4.0f, 5.8f, 14.f, 6.0f}},
+                                    {3, 4, 0.755f, {6.0f, 9.0f, 0.f, 0.f}}};
+
+static int gm_pick(int M, int N, int K, int epilogue) {
+    int best = 0;
+    float least = 0.f;
+    for (int i = 0; i < (gm_is_32(epilogue) ? 4 : 5); ++i) {
+        const GmShape& s = GM_SHAPES[i];
+        const long tiles = static_cast<long>(pl_ceil_div(M, 32 * s.rt)) * pl_ceil_div(N, gm_out_cols(s.ct, epilogue));
+        const float cost = static_cast<float>((tiles + pl_compute_units() - 1) / pl_compute_units()) * (s.tile[epilogue] + K / GM_BK * s.stage);
+        if (i == 0 || cost < least) best = i, least = cost;
+    }
+    return best;
+}
+
+template <int EPI>
+static int gm_shaped(const GmProduct& g, hipStream_t stream) {
+    switch (gm_pick(g.M, g.N, g.K, EPI)) {
+        case 0: return gm_launch<1, 2, 2, EPI>(g, stream);
+        case 1: return gm_launch<1, 4, 2, EPI>(g, stream);
+        case 2: return gm_launch<2, 3, 2, EPI>(g, stream);
+        case 3: return gm_launch<2, 4, 1, EPI>(g, stream);
+        default:
+            if constexpr (!gm_is_32(EPI)) return gm_launch<3, 4, 1, EPI>(g, stream);
+    }
+    return -1;
+}
+
+// Whether a shape is served: N (of gate alone for epilogue 1) a multiple of 16, K of 64, and offsets of 32 bits into x and into the weights.
+extern "C" int pl_gemm_many_applies(int M, int N, int K, int epilogue) {
+    return M > 0 && N > 0 && K > 0 && N % 16 == 0 && K % GM_BK == 0 && static_cast<long long>(M) * K < (1ll << 31) &&
+           (epilogue == GM_SWIGLU ? 2ll : 1ll) * N * K < (1ll << 31) && static_cast<long long>(pl_ceil_div(M, 64)) * pl_ceil_div(N, 64) < (1ll << 30);
+}
+
+// x: bfloat16 [M, K].  weights: bfloat16 [N, K], or [2 N, K], gate rows first, for epilogue 1; in strips or as they are.
+// epilogue 0: y (bfloat16 [M, N]) = result.  1: y = silu(gate) * up.  2: y (32-bit [M, N]) += result.  3: y (32-bit) = result.  All aligned to 16 bytes.
+// taken [M, taken_count] (epilogues 0 and 1; a multiple of four, up to 64): the sums of a norm handed forward, whose rows x are.  gain [N], rows [M, N],
+// sums [M, N / 64] (epilogue 2, N a multiple of 64): the norm behind the sum, handed forward.
+extern "C" int pl_gemm_many(const void* x, const void* weights, int in_strips, void* y, int M, int N, int K, int epilogue, const float* taken, int taken_count,
+                              float eps, const float* gain, void* rows, float* sums, hipStream_t stream) {
+    PL_REQUIRE(epilogue >= GM_STORE && epilogue <= GM_STORE32 && pl_gemm_many_applies(M, N, K, epilogue),
+               "product of many rows: %d rows, %d columns, inner width %d, epilogue %d", M, N, K, epilogue);
+    PL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weights) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gain) |
+                reinterpret_cast<uintptr_t>(rows)) % 16 == 0, "product of many rows: rows that are not aligned to 16 bytes");
+    PL_REQUIRE(taken == nullptr || (!gm_is_32(epilogue) && taken_count > 0 && taken_count <= GM_TAKEN_MOST && taken_count % 4 == 0 && reinterpret_cast<uintptr_t>(taken) % 16 == 0), "product of many rows: %d sums of a norm, epilogue %d",
+               taken_count, epilogue);
+    PL_REQUIRE((gain == nullptr) == (rows == nullptr) && (gain == nullptr) == (sums == nullptr) && (gain == nullptr || (epilogue == GM_ADD && N % GM_STRIPE == 0)),
+               "product of many rows: a norm handed forward by epilogue %d", epilogue);
+    const GmProduct g{x, weights, in_strips != 0, y, M, N, K, GmNorms{taken, taken_count, eps, gain, static_cast<bf16_t*>(rows), sums}};
+    if (epilogue == GM_STORE) return gm_shaped<GM_STORE>(g, stream);
+    if (epilogue == GM_SWIGLU) return gm_shaped<GM_SWIGLU>(g, stream);
+    if (epilogue == GM_ADD) return gm_shaped<GM_ADD>(g, stream);
+    return gm_shaped<GM_STORE32>(g, stream);
+}

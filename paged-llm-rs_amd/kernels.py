@@ -56,8 +56,8 @@ def _signatures(lib) -> None:
         "pl_gemm_skinny_hand": [p, p, p, i, i, i, i, i, i, p, i, f, p, p, p, i, p],
         "pl_gemm_skinny_hand_applies": [i, i, i, i, i],
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
-        "pl_gemm_strips": [p, p, p, i, i, i, p],
-        "pl_gemm_strips_apply": [i, i, i],
+        "pl_gemm_many": [p, p, i, p, i, i, i, i, p, i, f, p, p, p, p],
+        "pl_gemm_many_applies": [i, i, i, i],
         "pl_gemm_tiled_applies": [i, i, i, i],
         "pl_gemm_stream": [p, p, p, p, i, i, i, i, i, i, i, p],
         "pl_gemm_stream_splits": [i, i, i, i],
@@ -911,19 +911,24 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nk
 
 class HandedNorm:
     """An RMSNorm handed forward by the product that last added into the stream: that product owns whole
-    16-column stripes of the updated stream, so it leaves ``x`` = bfloat16(stream * gain) [n, width] and, for
-    every row, the sum of squares over each stripe, ``ssq`` [n, stripes].  The product that stands behind the
+    stripes of columns of the updated stream (16 of them, or 64 in products of many rows), so it leaves ``x`` = bfloat16(stream * gain)
+    [n, width] and, for every row, the sum of squares over each stripe, ``ssq`` [n, stripes].  The product that stands behind the
     norm then loads ``x`` (half the bytes of the 32-bit stream, nothing to convert or square), adds a row's
     sums in a fixed order and scales its result by 1 / sqrt(sum / width + eps).  ``filled`` says that a
-    product has written both."""
+    product has written both.  (Of many rows there is no room before a product asks for it.)"""
 
     __slots__ = ("gain", "eps", "x", "ssq", "filled")
 
     def __init__(self, gain: torch.Tensor, eps: float, rows: int, width: int, device):
         self.gain, self.eps = gain, float(eps)
-        self.x = torch.empty((rows, width), dtype=torch.bfloat16, device=device)
-        self.ssq = torch.empty((rows, (width + 15) // 16), dtype=torch.float32, device=device)
+        self.x = self.ssq = None
         self.filled = False
+        if rows <= SKINNY_ROWS:
+            self.room(rows, width, 16, device)
+
+    def room(self, rows: int, width: int, stripe: int, device) -> None:
+        self.x = torch.empty((rows, width), dtype=torch.bfloat16, device=device)
+        self.ssq = torch.empty((rows, -(-width // stripe)), dtype=torch.float32, device=device)
 
 
 # From this many rows on a norm is handed forward.  With fewer the product behind the norm normalises the 32-bit
@@ -1133,39 +1138,104 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
     return out
 
 
-# Where the product over strips with the gated activation inside beats the others (the library's product and the activation kernel, or
+# Where the product of many rows with the gated activation inside beats the others (the library's product and the activation kernel, or
 # ``gemm_tiled``), timed at 65 to 8,192 rows of 13 pairs of widths.  Up to a width of 2,048 it does at every size until the operations are what
 # counts, which the library's tiles of 256 x 256 do at up to 1.4 PFLOP/s and this one's at 1.0 to 1.2 (us, before / this one; 1,024 wide,
 # 3,072 columns: 65 rows 14 / 7, 2,048 36 / 26, 8,192 104 / 102; 8,192 columns: 2,560 rows 115 / 89, 4,096 140 / 151; 2,048 wide, 6,144 columns:
 # 1,024 rows 69 / 45, 1,150 58 / 60).  Beyond, it wins by what the library's turns of 256 such tiles leave empty, and up to 128 rows (12,288 columns of
 # 4,096: 65 rows 59 / 51, 256 83 / 72, turns 0.38 full, 576 124 / 114, 0.56 full; 14,336 of 4,096: 512 rows 105 / 122, 0.88 full; 25,600 of
 # 5,120: 128 rows 128 / 113, 256 166 / 168, 0.78 full).
-STRIPS_WORK = ((1024, 27e9), (2048, 13e9))      # widths up to, and rows x columns x width up to
-STRIPS_WIDE_ROWS = 128
-STRIPS_WIDE_MOST_ROWS = 704
-STRIPS_WIDE_TURNS = 0.6
+MANY_STRIPE = 64       # columns of the stream whose squares are one number of a norm that the product hands forward
+MANY_WORK = ((1024, 27e9), (2048, 13e9))      # widths up to, and rows x columns x width up to
+MANY_WIDE_ROWS = 128
+MANY_WIDE_MOST_ROWS = 704
+MANY_WIDE_TURNS = 0.6
 
 
-def strips_swiglu_wins(rows: int, columns: int, width: int) -> bool:
-    if rows <= SKINNY_ROWS or not library().pl_gemm_strips_apply(rows, columns, width):
+def many_swiglu_wins(rows: int, columns: int, width: int) -> bool:
+    if rows <= SKINNY_ROWS or not library().pl_gemm_many_applies(rows, columns, width, 1):
         return False
-    for most, work in STRIPS_WORK:
+    for most, work in MANY_WORK:
         if width <= most:
             return rows * columns * width <= work
     tiles = -(-rows // 256) * -(-2 * columns // 256)
-    return rows <= STRIPS_WIDE_ROWS or (rows <= STRIPS_WIDE_MOST_ROWS and tiles <= STRIPS_WIDE_TURNS * 256 * -(-tiles // 256))
+    return rows <= MANY_WIDE_ROWS or (rows <= MANY_WIDE_MOST_ROWS and tiles <= MANY_WIDE_TURNS * 256 * -(-tiles // 256))
 
 
-def gemm_strips_swiglu(x: torch.Tensor, strips: torch.Tensor) -> torch.Tensor:
-    """silu(x . gate^T) * (x . up^T) for many rows of bfloat16, 32-bit sums; ``strips``: what ``weights_in_strips`` made of
-    the weights [gate | up] stacked."""
+# The plain product, bfloat16 or 32-bit: up to a width of 1,024, as long as the rows and columns of the result are few (us, library / this one:
+# 4,096 columns: 65 rows 9.0 / 7.1, 450 11.1 / 8.1, 1,024 13.3 / 12.3, 1,536 16.8 / 15.7, 2,560 23.8 / 26.3; 1,024 columns: 65 rows 8.4 / 6.9,
+# 4,096 13.4 / 12.4, 8,192 20.5 / 20.7; of 2,048 and wider the library's is as fast at most sizes).
+MANY_STORE_WIDTH = 1024
+MANY_STORE_RESULTS = 6.25e6
+
+
+def many_store_wins(rows: int, columns: int, width: int) -> bool:
+    return (rows > SKINNY_ROWS and width <= MANY_STORE_WIDTH and rows * columns <= MANY_STORE_RESULTS
+            and bool(library().pl_gemm_many_applies(rows, columns, width, 0)))
+
+
+# The product that adds into the stream and hands the norm behind it forward, against the library's product and the norm kernel: a workgroup of the
+# smallest tile (64 rows by 128 columns) walks all of K, so the deeper K the more rows it takes until enough of them stand side by side (us, 1,024
+# columns: K 1,024, 65 rows 11.5 / 8.9, 8,192 38.6 / 31.7; K 2,048, 128 rows 11.9 / 12.5, 450 13.4 / 13.4, 1,024 15.7 / 14.6, 2,048 22.5 /
+# 16.7; K 3,072, 450 rows 16.6 / 17.6, 1,024 19.8 / 18.9, 2,048 26.6 / 21.1; K 4,096, 1,300 rows 27.0 / 22.8; 2,048 columns of 2,048: 4,096 rows 50.6 /
+# 45.2, 6,144 67.3 / 69.8).  The product behind the norm pays 0.6 for the sums.
+MANY_ADD_WIDTH = 4096
+MANY_ADD_ROWS = 0.42          # rows from which, for every k past 1,024
+MANY_ADD_RESULTS = 8.4e6
+
+
+def many_add_wins(rows: int, columns: int, width: int) -> bool:
+    return (rows > SKINNY_ROWS and columns <= FUSED_NORM_MAX_WIDTH and columns % (4 * MANY_STRIPE) == 0 and width <= MANY_ADD_WIDTH
+            and rows >= MANY_ADD_ROWS * (width - 1024) and rows * columns <= MANY_ADD_RESULTS
+            and bool(library().pl_gemm_many_applies(rows, columns, width, 2)))
+
+
+def many_takes(handed, rows: int, columns: int, width: int, swiglu: bool = False) -> bool:
+    """Whether the product of many rows takes this norm, which a product of many rows handed forward: it costs less than the norm as a
+    kernel wherever ``many_add_wins`` had it handed forward (8,192 rows of 1,024 against 4,096 columns 76 us, the library's product 56 and the norm 25)."""
+    return (rows > SKINNY_ROWS and handed.ssq.shape[1] * MANY_STRIPE == width
+            and bool(library().pl_gemm_many_applies(rows, columns, width, 1 if swiglu else 0)))
+
+
+def gemm_many(x: torch.Tensor | None, w: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16, swiglu: bool = False,
+              add_into: torch.Tensor | None = None, handed: "HandedNorm | None" = None, hand: "HandedNorm | None" = None,
+              strips: torch.Tensor | None = None) -> torch.Tensor:
+    """y = x . w^T for many rows of bfloat16, 32-bit sums.  With ``swiglu`` w is [gate | up] stacked and y = silu(x . gate^T) * (x . up^T),
+    in bfloat16.  With ``add_into`` (the 32-bit residual stream) the result is added there and that tensor is returned; ``hand``: the norm
+    that follows the stream is left behind in it.  ``handed``: a norm that an earlier product left behind; its rows are the input and its
+    sums of squares scale the result.  ``strips``: what ``weights_in_strips`` made of ``w``, read instead of it; the same bits."""
+    if handed is not None:
+        if not handed.filled:
+            raise TensorError("a handed norm is the product's input once a product has written it")
+        x = handed.x
     _need(x, "matrix product input", None, torch.bfloat16)
-    _need(strips, "weights in strips", None, torch.bfloat16)
-    if x.dim() != 2 or strips.dim() != 2 or strips.shape[1] != x.shape[1] or strips.shape[0] % 32:
-        raise TensorError(f"weights in strips of shape {tuple(strips.shape)} for an input of shape {tuple(x.shape)}")
+    _need(w, "weight", None, torch.bfloat16)
+    if strips is not None:
+        _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16)
+    if x.dim() != 2 or w.dim() != 2 or w.shape[1] != x.shape[1] or (swiglu and w.shape[0] % 2):
+        raise TensorError(f"weight has shape {tuple(w.shape)} for an input of shape {tuple(x.shape)}")
     M, K = x.shape
-    out = torch.empty((M, strips.shape[0] // 2), dtype=torch.bfloat16, device=x.device)
-    _check(library().pl_gemm_strips(x.data_ptr(), strips.data_ptr(), out.data_ptr(), M, out.shape[1], K, _stream()))
+    N = w.shape[0] // 2 if swiglu else w.shape[0]
+    if add_into is not None:
+        if swiglu or handed is not None:
+            raise TensorError("a product that adds into the residual stream has a plain input and no activation")
+        out, epilogue = _need(add_into, "residual stream", (M, N), torch.float32), 2
+    else:
+        if out_dtype not in (torch.bfloat16, torch.float32) or (out_dtype == torch.float32 and (swiglu or handed is not None)):
+            raise TensorError(f"matrix product output {out_dtype}" + (" after the activation" if swiglu else " behind a handed norm"))
+        out, epilogue = torch.empty((M, N), dtype=out_dtype, device=x.device), (1 if swiglu else 3 if out_dtype == torch.float32 else 0)
+    if hand is not None:
+        if add_into is None:
+            raise TensorError("a norm is handed forward by a product that adds into the stream")
+        _need(hand.gain, "gain of the norm handed forward", (N,), torch.float32)
+        hand.room(M, N, MANY_STRIPE, x.device)
+    _check(library().pl_gemm_many(
+        x.data_ptr(), (w if strips is None else strips).data_ptr(), 0 if strips is None else 1, out.data_ptr(), M, N, K, epilogue,
+        _ptr(handed.ssq if handed is not None else None), handed.ssq.shape[1] if handed is not None else 0,
+        float(handed.eps if handed is not None else 0.0), _ptr(hand.gain if hand is not None else None),
+        _ptr(hand.x if hand is not None else None), _ptr(hand.ssq if hand is not None else None), _stream()))
+    if hand is not None:
+        hand.filled = True
     return out
 
 
@@ -1372,6 +1442,8 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
             return gemm_stream(x, w, torch.float32)
         if skinny_applies(x) and x.shape[1] <= (SKINNY_F32_FEW_K if x.shape[0] <= 16 else SKINNY_SHALLOW_K):
             return gemm_skinny(x, w, torch.float32, strips=strips)
+        if many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
+            return gemm_many(x, w, torch.float32, strips=strips)
         if x.shape[1] % 8 == 0:
             return torch.mm(x, w.t(), out_dtype=torch.float32)
         return gemm_plain(x, w, out_dtype=torch.float32)
@@ -1379,6 +1451,8 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
         return gemm_skinny(x, w, out_dtype, strips=strips)
     if stream_wins(x.shape[0], w.shape[0], x.shape[1]):
         return gemm_stream(x, w, out_dtype)
+    if many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
+        return gemm_many(x, w, strips=strips)
     splits = library_splits(x.shape[0], w.shape[0], x.shape[1])
     if splits > 1 and turned is not None:
         return gemm_split_library(x, w, splits, out_dtype, turned=turned)

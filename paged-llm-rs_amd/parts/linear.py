@@ -76,6 +76,11 @@ class Linear:
                     and kernels.takes_handed_norm(x.num_rows, columns, self.in_features, swiglu)):
                 return kernels.gemm_skinny(None, self.weight, out_dtype or x.out_dtype, swiglu=swiglu,
                                            activation=activation, handed=x.handed, strips=self.strips)
+            silu = kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
+            if (x.handed is not None and add_into is None and self.weight.dtype == torch.bfloat16 and (silu or not swiglu)
+                    and (out_dtype or x.out_dtype) == torch.bfloat16
+                    and kernels.many_takes(x.handed, x.num_rows, columns, self.in_features, swiglu)):
+                return kernels.gemm_many(None, self.weight, swiglu=swiglu, handed=x.handed, strips=self.strips)
             if (getattr(x.norm, "fuses_into_product", False) and add_into is None
                     and kernels.fused_norm_applies(x.num_rows, self.in_features, self.weight)
                     and self.out_features <= kernels.FUSED_NORM_MAX_COLUMNS):
@@ -107,14 +112,17 @@ class Linear:
                 return None
             return kernels.gemm_stream(x, self.weight, out_dtype, swiglu=swiglu, activation=activation)
         if add_into is not None and not swiglu:
+            if kernels.many_add_wins(x.shape[0], self.out_features, self.in_features):
+                kernels.gemm_many(x, self.weight, add_into=add_into, hand=hand, strips=self.strips)
+                return None
             splits = kernels.library_splits(x.shape[0], self.out_features, self.in_features)
             if splits > 1 and self.turned is not None:
                 kernels.gemm_split_library(x, self.weight, splits, add_into=add_into, turned=self.turned)
                 return None
         if swiglu:
-            if (self.strips is not None and kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
-                    and kernels.strips_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features)):
-                return kernels.gemm_strips_swiglu(x, self.strips)
+            if (kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
+                    and kernels.many_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features)):
+                return kernels.gemm_many(x, self.weight, swiglu=True, strips=self.strips)
             if kernels.tiled_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features):
                 return kernels.gemm_tiled(x, self.weight, swiglu=True, activation=activation)
             return kernels.swiglu(kernels.linear_bf16(x, self.weight, x.dtype, self.strips, self.turned), activation=activation)

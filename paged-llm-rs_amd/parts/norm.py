@@ -89,8 +89,8 @@ class RmsNorm:
 
     def handoff(self, rows: int, device):
         """Room for this norm handed forward by a product that adds into the stream (``kernels.HandedNorm``),
-        or None where no product would take it: many rows, a wide stream."""
-        if rows > kernels.SKINNY_ROWS or self.width > kernels.FUSED_NORM_MAX_WIDTH or self.width % 8:
+        or None where no product would take it: a wide stream."""
+        if self.width > kernels.FUSED_NORM_MAX_WIDTH or self.width % 8:
             return None
         return kernels.HandedNorm(self.gain32, self.eps, rows, self.width, device)
 

@@ -2051,24 +2051,76 @@ def test_32_bit_attention_of_a_step_without_tokens(requests):
 
 
 @pytest.mark.parametrize("N,K", [(16, 64), (48, 128), (208, 192), (1040, 320), (3072, 1024)])
-def test_the_gated_product_out_of_strips(N, K):
+def test_the_gated_product_of_many_rows(N, K):
     """Every shape of tile (the rows and columns choose it), tiles that reach past the rows and the columns, an odd count of stages of 64 k
-    and one alone: 64-bit arithmetic within bfloat16's rounding of the result (2^-9, a factor of two for the 32-bit sums' part), and every
-    row the same whichever rows stand beside it in its tile."""
+    and one alone: 64-bit arithmetic within bfloat16's rounding of the result (2^-9, a factor of two for the 32-bit sums' part); the same bits
+    out of weights in strips and in rows; infinities and NaNs stay in their rows."""
     from paged_llm_rs_amd import kernels
 
     w = (torch.randn(2 * N, K, device=DEV) * 3 / K ** 0.5).bfloat16()
     strips = kernels.weights_in_strips(w)
     for n in (65, 96, 129, 300, 520, 700, 1030, 2050):
         x = torch.randn(n, K, device=DEV).bfloat16()
-        assert kernels.strips_swiglu_wins(n, N, K)
+        assert kernels.many_swiglu_wins(n, N, K)
         both = x.double() @ w.double().T
         want = torch.nn.functional.silu(both[:, :N]) * both[:, N:]
-        got = kernels.gemm_strips_swiglu(x, strips)
+        got = kernels.gemm_many(x, w, swiglu=True, strips=strips)
         assert rel(got, want) < 2.0 ** -8, f"{n} rows"
         assert float((got.double() - want).abs().max()) < 2.0 ** -8 * float(want.abs().max()), f"{n} rows"
-        assert torch.equal(got, kernels.gemm_strips_swiglu(x, strips))
+        assert torch.equal(got, kernels.gemm_many(x, w, swiglu=True)), f"{n} rows"
     x = torch.zeros(130, K, device=DEV, dtype=torch.bfloat16)
     x[7, 0], x[8, K - 1] = math.inf, math.nan
-    y = kernels.gemm_strips_swiglu(x, strips)
-    assert bool(y[8].isnan().all()) and not bool(y[7].isfinite().all()) and not bool(y[torch.arange(130, device=DEV).sub(7.5).abs() > 1].any())
+    for s in (strips, None):
+        y = kernels.gemm_many(x, w, swiglu=True, strips=s)
+        others = torch.arange(130, device=DEV).sub(7.5).abs() > 1
+        assert bool(y[8].isnan().all()) and not bool(y[7].isfinite().all()) and not bool(y[others].any())
+
+
+@pytest.mark.parametrize("N,K", [(256, 64), (1024, 192), (1024, 1024), (768, 2048)])
+def test_products_of_many_rows_and_the_norms_between_them(N, K):
+    """The plain product, 32-bit and bfloat16; the sum into the stream, which hands the norm behind it forward; and the products that take
+    it: against 64-bit arithmetic, bfloat16 results within their rounding (2^-9 and half of it for an input's), 32-bit ones within a factor of four of
+    what a chain of K / 16 sums can be off; the same bits out of weights in strips and in rows."""
+    from paged_llm_rs_amd import kernels
+
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).bfloat16()
+    strips, chain = kernels.weights_in_strips(w), 4 * math.sqrt(K / 16 + 1) * 2.0 ** -24
+    after = (torch.randn(2 * 208, N, device=DEV) * 2 / N ** 0.5).bfloat16()
+    gain, eps = 1 + 0.3 * torch.randn(N, device=DEV), 1e-3
+    for n in (65, 129, 300, 520, 700, 1300):
+        x = torch.randn(n, K, device=DEV).bfloat16()
+        want = x.double() @ w.double().T
+        for dtype, most in ((torch.float32, chain), (torch.bfloat16, 2.0 ** -8)):
+            got = kernels.gemm_many(x, w, dtype, strips=strips)
+            assert rel(got, want) < most and torch.equal(got, kernels.gemm_many(x, w, dtype))
+        before = torch.randn(n, N, device=DEV)
+        stream, alone, summed = before.clone(), before.clone(), before.double() + want
+        hand, again = kernels.HandedNorm(gain, eps, n, N, DEV), kernels.HandedNorm(gain, eps, n, N, DEV)
+        assert hand.x is None and kernels.gemm_many(x, w, add_into=stream, hand=hand, strips=strips) is stream and hand.filled
+        assert rel(stream, summed) < chain and torch.equal(kernels.gemm_many(x, w, add_into=alone, hand=again), stream)
+        assert torch.equal(hand.x, again.x) and torch.equal(hand.ssq, again.ssq)
+        assert torch.equal(kernels.gemm_many(x, w, add_into=before, strips=strips), stream)
+        assert rel(hand.x, summed * gain.double()) < 2.0 ** -8
+        assert rel(hand.ssq, (summed * summed).view(n, -1, 64).sum(2)) < 2 * chain + 2.0 ** -20
+        normed = summed / torch.sqrt((summed * summed).mean(1, keepdim=True) + eps) * gain.double()
+        plain = normed @ after.double().T
+        assert kernels.many_takes(hand, n, 208, N, swiglu=True) and kernels.many_takes(hand, n, 416, N)
+        assert rel(kernels.gemm_many(None, after, handed=hand), plain) < 1.5 * 2.0 ** -8
+        gated = torch.nn.functional.silu(plain[:, :208]) * plain[:, 208:]
+        assert rel(kernels.gemm_many(None, after, swiglu=True, handed=hand, strips=kernels.weights_in_strips(after)), gated) < 3 * 2.0 ** -8
+
+
+def test_products_of_many_rows_refuse_what_they_do_not_take():
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.errors import TensorError
+
+    x, w = torch.randn(70, 64, device=DEV).bfloat16(), torch.randn(96, 64, device=DEV).bfloat16()
+    stream = torch.zeros(70, 96, device=DEV)
+    hand = kernels.HandedNorm(torch.ones(96, device=DEV), 1e-6, 70, 96, DEV)
+    for call in (lambda: kernels.gemm_many(x[:, :32].contiguous(), w), lambda: kernels.gemm_many(x, w, swiglu=True, add_into=stream),
+                 lambda: kernels.gemm_many(x, w, hand=hand), lambda: kernels.gemm_many(None, w, handed=hand),
+                 lambda: kernels.gemm_many(x, w, add_into=stream, hand=hand), lambda: kernels.gemm_many(x, w, add_into=stream[:, :48].contiguous()),
+                 lambda: kernels.gemm_many(x, w, torch.float16), lambda: kernels.gemm_many(x, w, torch.float32, swiglu=True),
+                 lambda: kernels.gemm_many(x, w, strips=w[:48].contiguous())):
+        with pytest.raises(TensorError):
+            call()
