@@ -49,6 +49,18 @@ struct GmNorms {
 };
 #define GM_TAKEN_MOST 64
 
+// Grouped: the rows are dealt to groups (experts), every group with a weight matrix of its own, one behind the other in w.  A tile of 128 rows belongs to one
+// group (`tile_group`; the tiles in use come first, and how many they are stands behind the last of all); row r of the tiles reads row gather[r] of x (null: row r itself; negative: a row of
+// padding, which reads row 0 and whose result nobody looks at) and writes row r of y.
+struct GmGroups {
+    const int* tile_group;     // [row tiles + 1]
+    const int* gather;         // [row tiles * 128] or null
+    long long w_stride;        // elements between two groups' matrices
+    int x_pitch, y_pitch;      // elements between two rows of x and of y
+    int last, N_last, K_last;  // one group, `last` (-1: none), may have a matrix of other sizes: w_last, [N_last (2 N_last with GM_SWIGLU), K_last]
+    const bf16_t* w_last;
+};
+
 __device__ __forceinline__ uint32_t gm_pack2(float lo, float hi) {
     const gm_f32x2 pair = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, gm_bf16x2));
@@ -97,13 +109,18 @@ constexpr int gm_lds_bytes(int CT, int RT, int epi, bool strips) {
 // matrices are read from their last and not stored.
 // STRIPS: the weights in strips; otherwise in rows as they are stored, which go through registers and LDS as the rows of x do, each wave's
 // through a part of LDS of its own.  The sums are the same, k after k: the layout changes no bit.
-template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS>
+template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS, bool GROUPED = false>
 __global__ void __launch_bounds__(256, PER_SIMD)
 gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weights, void* __restrict__ y_, int M, int N, int K,
-                   int row_tiles, int col_tiles, GmNorms norms) {
+                   int row_tiles, int col_tiles, GmNorms norms, GmGroups groups) {
+    static_assert(!GROUPED || (RT == 4 && !TAKES && !STRIPS && EPI != GM_ADD), "groups' tiles are of 128 rows");
     constexpr int ROWS = 32 * RT, STAGE = ROWS * GM_BK * 2;
     extern __shared__ __attribute__((aligned(16))) char gm_lds[];          // two stages of x [row][64], then the tile on its way out
     int row_tile, col_tile;
+    if constexpr (GROUPED) {
+        row_tiles = groups.tile_group[row_tiles];                          // those that are used: the XCDs share them evenly
+        if (static_cast<int>(blockIdx.x) >= row_tiles * col_tiles) return; // (the whole workgroup)
+    }
     gm_tile(blockIdx.x, row_tiles, col_tiles, row_tile, col_tile);
     const int m0 = row_tile * ROWS;
     const int tid = threadIdx.x, lane = tid % PL_WAVE;
@@ -111,6 +128,20 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
     const int r32 = lane % 32, h = lane / 32;
     constexpr int COLS = gm_out_cols(CT, EPI) / 4;                         // output columns a wave
     const int n_wave = (col_tile * 4 + wave) * COLS;                       // the wave's first
+    int x_pitch = K, y_pitch = N;
+    if constexpr (GROUPED) {
+        const int group = groups.tile_group[row_tile];
+        if (group == groups.last) {
+            weights = groups.w_last;
+            N = groups.N_last;
+            K = groups.K_last;
+        } else {
+            weights += static_cast<long long>(group) * groups.w_stride;
+        }
+        if (col_tile * 4 * COLS >= N) return;                              // (this group has fewer columns than another)
+        x_pitch = groups.x_pitch;
+        y_pitch = groups.y_pitch;
+    }
 
     const int last_strip = N / 16 - 1;                                     // (of gate alone)
     auto strip_of = [&](int c, int half) {                                 // the strip of either half of an instruction's 32 rows
@@ -130,8 +161,13 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
     }
     uint32_t x_at[RT];
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
-        x_at[i] = static_cast<uint32_t>(min(m0 + tid / 8 + 32 * i, M - 1)) * static_cast<uint32_t>(K) * 2u + tid % 8 * 16;
+    for (int i = 0; i < RT; ++i) {
+        int row = min(m0 + tid / 8 + 32 * i, M - 1);
+        if constexpr (GROUPED) {
+            if (groups.gather != nullptr) row = max(groups.gather[row], 0);
+        }
+        x_at[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(x_pitch) * 2u + tid % 8 * 16;
+    }
     char* const w_lds = gm_lds + 2 * STAGE + wave * 2 * CT * 4096;         // the wave's weights in rows: two stages of [32 CT][64]
     char* const put_w_at = w_lds + lane / 8 * 128 + ((lane % 8) ^ (lane / 8)) * 16;
     char* const put_at = gm_lds + tid / 8 * 128 + ((tid % 8) ^ (tid / 8 % 8)) * 16;
@@ -344,7 +380,7 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
         for (int i = tid; i < ROWS * LANES; i += 256) {
             const int r = i / LANES, piece = i % LANES;
             if (m0 + r < M && n0 + piece * 8 < N)
-                *reinterpret_cast<gm_u32x4*>(y + static_cast<size_t>(m0 + r) * N + n0 + piece * 8) =
+                *reinterpret_cast<gm_u32x4*>(y + static_cast<size_t>(m0 + r) * y_pitch + n0 + piece * 8) =
                     *reinterpret_cast<const gm_u32x4*>(gm_lds + r * PITCH + piece * 16);
         }
     } else {
@@ -360,7 +396,7 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
                 const bool there = row < M && col < N;
                 gm_f32x4 v = *reinterpret_cast<const gm_f32x4*>(gm_lds + r * PITCH + tid % LANES * 16);
                 if constexpr (EPI == GM_ADD) v += old[i];
-                const size_t to = static_cast<size_t>(row) * N + col;
+                const size_t to = static_cast<size_t>(row) * y_pitch + col;
                 if (there) *reinterpret_cast<gm_f32x4*>(static_cast<float*>(y_) + to) = v;
                 if (hands) {
                     const float square = gm_sum16(there ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f);
@@ -394,7 +430,7 @@ static int gm_launch_one(const GmProduct& g, hipStream_t stream) {
         PL_REQUIRE(e == hipSuccess, "product of many rows: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
     }
     gemm_many_kernel<CT, RT, PER_SIMD, EPI, TAKES, STRIPS><<<row_tiles * col_tiles, 256, lds, stream>>>(
-        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms);
+        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, GmGroups{});
     PL_CHECK_LAUNCH("gemm_many");
     return 0;
 }
@@ -472,4 +508,61 @@ extern "C" int pl_gemm_many(const void* x, const void* weights, int in_strips, v
     if (epilogue == GM_SWIGLU) return gm_shaped<GM_SWIGLU>(g, stream);
     if (epilogue == GM_ADD) return gm_shaped<GM_ADD>(g, stream);
     return gm_shaped<GM_STORE32>(g, stream);
+}
+
+template <int CT, int PER_SIMD, int EPI>
+static int gm_launch_grouped(const GmProduct& g, const GmGroups& groups, int row_tiles, int columns, hipStream_t stream) {
+    constexpr int lds = gm_lds_bytes(CT, 4, EPI, false);
+    static_assert(lds <= 160 * 1024, "a workgroup's LDS");
+    const int col_tiles = pl_ceil_div(columns, gm_out_cols(CT, EPI));
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_many_kernel<CT, 4, PER_SIMD, EPI, false, false, true>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    PL_REQUIRE(e == hipSuccess, "grouped product of many rows: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
+    gemm_many_kernel<CT, 4, PER_SIMD, EPI, false, false, true><<<row_tiles * col_tiles, 256, lds, stream>>>(
+        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, groups);
+    PL_CHECK_LAUNCH("gemm_many_grouped");
+    return 0;
+}
+
+// Whether the grouped form takes these sizes (those of the last group too, where it has its own).
+extern "C" int pl_gemm_many_grouped_applies(int row_tiles, int x_rows, int N, int K, int x_pitch) {
+    return row_tiles > 0 && row_tiles <= (1 << 22) && x_rows > 0 && N > 0 && K > 0 && N % 16 == 0 && K % GM_BK == 0 && 2ll * N * K < (1ll << 31) &&
+           static_cast<long long>(x_rows) * x_pitch < (1ll << 31) && static_cast<long long>(row_tiles) * pl_ceil_div(N, 64) < (1ll << 30);
+}
+
+// The product over rows dealt to groups (see GmGroups).  x: bfloat16 [x_rows, x_pitch], read through `gather` ([row_tiles * 128]) or, with gather null, in
+// place (x_rows >= row_tiles * 128).  w: bfloat16, group g's matrix at w + g * w_stride: [N, K], or [2 N, K] with the gate rows first for epilogue 1.
+// y: [row_tiles * 128, y_pitch], bfloat16 for epilogue 1 (silu(gate) * up), 32-bit for epilogue 3.  last >= 0: that group's matrix is w_last, of N_last and
+// K_last in the places of N and K, under the same rules.  likely_tiles: how many of the tiles will likely be used (the shape goes by it).
+// us, gemm_tiled / this one, 28 tiles of 36 used: 1,536 gated columns of 1,024 50 / 32, 1,024 of 1,536 in 32 bits 26.6 / 22.6.
+extern "C" int pl_gemm_many_grouped(const void* x, const void* w, void* y, const int* tile_group, const int* gather, long long w_stride, int row_tiles,
+                                    int likely_tiles, int x_rows, int N, int K, int epilogue, int x_pitch, int y_pitch, int last, const void* w_last, int N_last,
+                                    int K_last, hipStream_t stream) {
+    PL_REQUIRE((epilogue == GM_SWIGLU || epilogue == GM_STORE32) && pl_gemm_many_grouped_applies(row_tiles, x_rows, N, K, x_pitch) &&
+                   (last < 0 || (w_last != nullptr && pl_gemm_many_grouped_applies(row_tiles, x_rows, N_last, K_last, x_pitch))),
+               "grouped product of many rows: %d tiles, %d columns, inner width %d, epilogue %d", row_tiles, N, K, epilogue);
+    PL_REQUIRE(x_pitch >= K && y_pitch >= N && x_pitch % 8 == 0 && y_pitch % 8 == 0 && (last < 0 || (x_pitch >= K_last && y_pitch >= N_last)),
+               "grouped product of many rows: rows of %d and %d for an inner width of %d and %d columns", x_pitch, y_pitch, K, N);
+    PL_REQUIRE(tile_group != nullptr && (gather != nullptr || x_rows >= row_tiles * 128), "grouped product of many rows: %d rows for %d tiles", x_rows, row_tiles);
+    PL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w_last)) % 16 == 0 &&
+                   w_stride % 8 == 0, "grouped product of many rows: rows that are not aligned to 16 bytes");
+    const GmProduct g{x, w, false, y, row_tiles * 128, N, K, GmNorms{}};
+    const GmGroups groups{tile_group, gather, w_stride, x_pitch, y_pitch, last, N_last, K_last, static_cast<const bf16_t*>(w_last)};
+    const int columns = last >= 0 && N_last > N ? N_last : N;
+    int best = 0;
+    float least = 0.f;
+    for (int i = 1; i < (epilogue == GM_STORE32 ? 4 : 5); ++i) {
+        const GmShape& s = GM_SHAPES[i];
+        if (s.rt != 4) continue;
+        const long tiles = static_cast<long>(likely_tiles) * pl_ceil_div(columns, gm_out_cols(s.ct, epilogue));
+        const float cost = static_cast<float>((tiles + pl_compute_units() - 1) / pl_compute_units()) * (s.tile[epilogue] + K / GM_BK * s.stage);
+        if (best == 0 || cost < least) best = i, least = cost;
+    }
+    if (epilogue == GM_SWIGLU) {
+        if (best == 1) return gm_launch_grouped<1, 2, GM_SWIGLU>(g, groups, row_tiles, columns, stream);
+        if (best == 3) return gm_launch_grouped<2, 1, GM_SWIGLU>(g, groups, row_tiles, columns, stream);
+        return gm_launch_grouped<3, 1, GM_SWIGLU>(g, groups, row_tiles, columns, stream);
+    }
+    if (best == 1) return gm_launch_grouped<1, 2, GM_STORE32>(g, groups, row_tiles, columns, stream);
+    return gm_launch_grouped<2, 1, GM_STORE32>(g, groups, row_tiles, columns, stream);
 }

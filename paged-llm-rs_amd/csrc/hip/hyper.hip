@@ -412,6 +412,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* ids, const in
             for (int i = 0; i < mine && at + i < tiles; ++i) tile_group[at + i] = e;
             at += mine;
         }
+        tile_group[tiles] = at < tiles ? at : tiles;  // (those in use)
         for (; at < tiles; ++at) tile_group[at] = -1;
     }
     __syncthreads();
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* ids, const in
     }
 }
 
-// tiles: what the caller has room for, at least ceil(n * top / tile) + min(E, n * top).
+// tiles: what the caller has room for, at least ceil(n * top / tile) + min(E, n * top).  tile_group: [tiles + 1], the last how many tiles are in use.
 extern "C" int pl_moe_sort(const int* ids, const int* src, const int* fed, const int* positions, const int* table,
                            const int* choice, int n, int top, int E, int vocab, int shared_at, int tile, int tiles, int* gather, int* slot_of,
                            int* tile_group, hipStream_t stream) {

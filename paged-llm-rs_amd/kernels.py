@@ -58,6 +58,8 @@ def _signatures(lib) -> None:
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
         "pl_gemm_many": [p, p, i, p, i, i, i, i, p, i, f, p, p, p, p],
         "pl_gemm_many_applies": [i, i, i, i],
+        "pl_gemm_many_grouped": [p, p, p, p, p, ctypes.c_longlong, i, i, i, i, i, i, i, i, i, p, i, i, p],
+        "pl_gemm_many_grouped_applies": [i, i, i, i, i],
         "pl_gemm_tiled_applies": [i, i, i, i],
         "pl_gemm_stream": [p, p, p, p, i, i, i, i, i, i, i, p],
         "pl_gemm_stream_splits": [i, i, i, i],
@@ -2296,7 +2298,7 @@ def moe_grouped(x: torch.Tensor, batch, table, w_gate_up: torch.Tensor, w_down: 
     tiles = -(-pairs // MOE_TILE) + min(dealt, pairs)
     slots = tiles * MOE_TILE
     lib, stream = library(), _stream()
-    ints = torch.empty((slots + pairs + tiles,), dtype=torch.int32, device=x.device)
+    ints = torch.empty((slots + pairs + tiles + 1,), dtype=torch.int32, device=x.device)
     gather, slot_of, tile_group = ints[:slots], ints[slots:slots + pairs], ints[slots + pairs:]
     _check(lib.pl_moe_sort(batch.token_ids.data_ptr(), _ptr(src), _ptr(fed), batch.positions.data_ptr(), _ptr(table),
                            _ptr(choice), n, top, dealt, vocab, E + int(identity) if size else -1, MOE_TILE, tiles,
@@ -2304,13 +2306,25 @@ def moe_grouped(x: torch.Tensor, batch, table, w_gate_up: torch.Tensor, w_down: 
     longest = max(F, size)
     last, shared_up, shared_down = (E, shared[0].data_ptr(), shared[1].data_ptr()) if size else (-1, 0, 0)
     hidden = torch.empty((slots, longest), dtype=torch.bfloat16, device=x.device)
-    _check(lib.pl_gemm_tiled_grouped(x.data_ptr(), w_gate_up.data_ptr(), hidden.data_ptr(), tile_group.data_ptr(),
-                                     gather.data_ptr(), w_gate_up.stride(0), tiles, n, F, W, 1 if gated else 4, act, 1, bound,
-                                     W, longest, last, shared_up, size, W, stream))
+    # (as if every expert had as many pairs; a shared one has every row)
+    own = pairs - n if size else pairs
+    likely = min(tiles, E * -(-max(own, 1) // (E * MOE_TILE)) + (-(-n // MOE_TILE) if size else 0))
+    many = lambda rows, N, K, pitch: lib.pl_gemm_many_grouped_applies(tiles, rows, N, K, pitch)
+    if gated and act == ACTIVATIONS["silu"] and many(n, F, W, W) and (not size or many(n, size, W, W)):
+        _check(lib.pl_gemm_many_grouped(x.data_ptr(), w_gate_up.data_ptr(), hidden.data_ptr(), tile_group.data_ptr(), gather.data_ptr(),
+                                        w_gate_up.stride(0), tiles, likely, n, F, W, 1, W, longest, last, shared_up, size, W, stream))
+    else:
+        _check(lib.pl_gemm_tiled_grouped(x.data_ptr(), w_gate_up.data_ptr(), hidden.data_ptr(), tile_group.data_ptr(),
+                                         gather.data_ptr(), w_gate_up.stride(0), tiles, n, F, W, 1 if gated else 4, act, 1, bound,
+                                         W, longest, last, shared_up, size, W, stream))
     splits = moe_down_splits(tiles, W, min(F, size) if size else F)
     y = torch.empty((splits, slots, W), dtype=torch.float32, device=x.device)
-    _check(lib.pl_gemm_tiled_grouped(hidden.data_ptr(), w_down.data_ptr(), y.data_ptr(), tile_group.data_ptr(), 0,
-                                     W * F, tiles, slots, W, F, 3, 0, splits, 0.0, longest, W, last, shared_down, W, size, stream))
+    if splits == 1 and many(slots, W, F, longest) and (not size or many(slots, W, size, longest)):
+        _check(lib.pl_gemm_many_grouped(hidden.data_ptr(), w_down.data_ptr(), y.data_ptr(), tile_group.data_ptr(), 0, W * F, tiles, likely, slots, W, F, 3,
+                                        longest, W, last, shared_down, W, size, stream))
+    else:
+        _check(lib.pl_gemm_tiled_grouped(hidden.data_ptr(), w_down.data_ptr(), y.data_ptr(), tile_group.data_ptr(), 0,
+                                         W * F, tiles, slots, W, F, 3, 0, splits, 0.0, longest, W, last, shared_down, W, size, stream))
     sums = ExpertSums(y, slot_of, choice, weight, n, top, splits, x, E, int(identity), batch.positions)
     return sums.total() if summed else sums
 

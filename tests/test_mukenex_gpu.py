@@ -653,3 +653,10 @@ def test_the_pass_over_the_copies_for_every_number_and_width(copies, width, dtyp
     bound = (16 + width ** 0.5) * 2.0 ** -24
     assert (streams.view_as(want) - want).abs().max() <= bound * want.abs().max()
     assert (got.double() - normed).abs().max() <= (bound + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * normed.abs().max()
+
+
+@pytest.mark.parametrize("experts,top,ff,width,rows", [(8, 2, 1536, 1024, 1800), (2, 1, 64, 64, 400), (5, 2, 448, 192, 900), (70, 2, 128, 128, 2300), (3, 2, 960, 320, 5000)])
+def test_experts_dealt_to_tiles_of_every_shape(experts, top, ff, width, rows):
+    """The same at sizes at which the grouped product takes each of its shapes of tile, with columns and groups that end inside a tile, more than 64 experts (the
+    tiles of 64 are counted at a time) and more pairs than the sorting threads take at once."""
+    test_experts_by_table_dealt_to_their_experts(experts, top, ff, width, rows)
