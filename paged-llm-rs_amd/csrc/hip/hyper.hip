@@ -384,46 +384,74 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* ids, const in
     for (int s = threadIdx.x; s < tiles * tile; s += blockDim.x) gather[s] = -1;
     __syncthreads();
     const int pairs = n * top;
-    auto expert_of = [&](int p) -> int {
-        const int t = p / top;
-        if (positions[t] < 0) return -1;
-        int e;
-        if (choice != nullptr) {
-            e = choice[p];                            // (an identity expert, at the given experts' count or beyond, takes no slot)
-            if (shared_at >= 0) e = e == shared_at ? E - 1 : (e < E - 1 ? e : -1);
-        } else {
-            const int id = moe_token(ids, src, fed, t);
-            if (id < 0 || id >= vocab) return -1;
-            e = table[static_cast<size_t>(id) * top + (p - t * top)];
+    // Four pairs a thread at a time: what a pair's expert follows from is asked for together, a trip for all four (one pair after the
+    // other 3,584 pairs over 8 experts took 12.6 us, 9.3 so).
+    constexpr int EACH = 4;
+    for (int p0 = threadIdx.x; p0 < pairs; p0 += EACH * blockDim.x) {
+        int position[EACH], named[EACH], e[EACH];
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            const int p = min(p0 + u * static_cast<int>(blockDim.x), pairs - 1);
+            position[u] = positions[p / top];
+            named[u] = choice != nullptr ? choice[p] : moe_token(ids, src, fed, p / top);
         }
-        return (e >= 0 && e < E) ? e : -1;
-    };
-    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-        const int e = expert_of(p);
-        slot_of[p] = e;                               // (kept for the second pass, which the same thread makes)
-        if (e >= 0) atomicAdd(&count[e], 1);
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            const int p = min(p0 + u * static_cast<int>(blockDim.x), pairs - 1);
+            e[u] = named[u];
+            if (choice != nullptr) {                  // (an identity expert, at the given experts' count or beyond, takes no slot)
+                if (shared_at >= 0) e[u] = e[u] == shared_at ? E - 1 : (e[u] < E - 1 ? e[u] : -1);
+            } else {
+                e[u] = named[u] < 0 || named[u] >= vocab ? -1 : table[static_cast<size_t>(named[u]) * top + p % top];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            const int p = p0 + u * static_cast<int>(blockDim.x);
+            if (p >= pairs) continue;
+            if (position[u] < 0 || e[u] < 0 || e[u] >= E) e[u] = -1;
+            slot_of[p] = e[u];                        // (kept for the second pass, which the same thread makes)
+            if (e[u] >= 0) atomicAdd(&count[e[u]], 1);
+        }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < PL_WAVE) {                      // the first tile of every expert, 64 of them at a time
         int at = 0;                                   // in tiles
-        for (int e = 0; e < E; ++e) {
-            base[e] = at * tile;
-            const int mine = (count[e] + tile - 1) / tile;
-            for (int i = 0; i < mine && at + i < tiles; ++i) tile_group[at + i] = e;
-            at += mine;
+        for (int e0 = 0; e0 < E; e0 += PL_WAVE) {
+            const int e = e0 + threadIdx.x, mine = e < E ? (count[e] + tile - 1) / tile : 0;
+            int through = mine;
+#pragma unroll
+            for (int off = 1; off < PL_WAVE; off <<= 1) {
+                const int other = __shfl_up(through, off, PL_WAVE);
+                if (static_cast<int>(threadIdx.x) >= off) through += other;
+            }
+            const int first = at + through - mine;
+            if (e < E) base[e] = first * tile;
+            for (int i = 0; i < mine && first + i < tiles; ++i) tile_group[first + i] = e;
+            at += __shfl(through, PL_WAVE - 1, PL_WAVE);
         }
-        tile_group[tiles] = at < tiles ? at : tiles;  // (those in use)
-        for (; at < tiles; ++at) tile_group[at] = -1;
+        if (threadIdx.x == 0) tile_group[tiles] = at < tiles ? at : tiles;        // (those in use)
+        for (int i = at + threadIdx.x; i < tiles; i += PL_WAVE) tile_group[i] = -1;
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
-        const int e = slot_of[p];
-        int slot = -1;
-        if (e >= 0) {
-            slot = base[e] + atomicAdd(&cursor[e], 1);
-            gather[slot] = p / top;
+    for (int p0 = threadIdx.x; p0 < pairs; p0 += EACH * blockDim.x) {
+        int e[EACH];
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            const int p = p0 + u * static_cast<int>(blockDim.x);
+            e[u] = p < pairs ? slot_of[p] : -1;
         }
-        slot_of[p] = slot;
+#pragma unroll
+        for (int u = 0; u < EACH; ++u) {
+            const int p = p0 + u * static_cast<int>(blockDim.x);
+            if (p >= pairs) continue;
+            int slot = -1;
+            if (e[u] >= 0) {
+                slot = base[e[u]] + atomicAdd(&cursor[e[u]], 1);
+                gather[slot] = p / top;
+            }
+            slot_of[p] = slot;
+        }
     }
 }
 
