@@ -41,6 +41,7 @@ def _signatures(lib) -> None:
         "pl_paged_attention_plain": [p, i, p, p, p, p, i, i, p, p, i, i, i, i, f, i, i, p, p, f, i, p, i, p],
         "pl_paged_attention_f32_applies": [p, i, p, p, p, i],
         "pl_paged_attention_f32": [p, i, p, p, p, p, p, i, p, i, i, p, p, i, i, i, i, f, i, p, p, f, i, p, i, p, p, i, p],
+        "pl_attention_near": [p, p, p, p, i, f, p, p, p, p, p, i, p, i, i, p, p, i, i, f, p],
         "pl_gemm_heads": [p, p, p, i, i, i, i, i, ctypes.c_long, i, ctypes.c_long, i, i, p],
         "pl_head_prepare": [p, p, i, i, i, f, p, p, p, p, i, i, i, i, f, i, p, p, p, i, i, i, p, p, p, i, i, i, i, i, i, i,
                             p, i, p, f, p],
@@ -835,6 +836,47 @@ def prefill_splits(requests: int, max_q_len: int, nq: int, d: int, max_ctx: int,
     return best
 
 
+# A step whose contexts are all as near as one workgroup holds them runs preparation and attention as one kernel, a workgroup a request and query head,
+# while those are no more than two a compute unit; beyond, requests of a token or two keep a workgroup each for little (us, two kernels / one: 32 heads, 8
+# requests of 10 tokens at 120 20.1 / 11.5, 16 28.7 / 21.1, 32 48 / 40, but one of 40 beside 31 single tokens 27.4 / 27.9, beside 63 24.8 / 50.3).
+NEAR_KEYS = 128
+NEAR_HEAD = 128
+NEAR_WORKGROUPS = 512
+
+
+def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, scale: float, prepare: QkFusion) -> torch.Tensor:
+    """Everything between the fused q/k/v projection and the output projection for a step whose contexts are no longer than 128 tokens
+    (``NEAR_KEYS``; rows of longer ones come out as NaN): heads of 128 rotated whole or not at all, in bfloat16."""
+    n, d, S = qkv.shape[0], NEAR_HEAD, kv.block_table.shape[0]
+    _need(qkv, "fused q/k/v projection", (n, (nq + 2 * nkv) * d), torch.bfloat16)
+    _need(out, "attention output", (n, nq * d), torch.bfloat16)
+    _need(kv.block_table, "block table", None, torch.int32)
+    for t, what in ((batch.q_start, "first row of each request"), (batch.q_len, "tokens of each request"), (batch.ctx_len, "context length of each request")):
+        _need(t, what, (S,), torch.int32)
+    for pool, what in ((kv.k_pool, "key pool"), (kv.v_pool, "value pool")):
+        _need(pool, what, None, torch.bfloat16)
+        if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % kv.block_size != 0:
+            raise TensorError(f"{what} has shape {tuple(pool.shape)}, expected [pages*{kv.block_size}, {nkv * d}]")
+    if kv.k_pool.shape[0] >= 2 ** 31:
+        raise TensorError("a pool of 2^31 slots or more is not addressed by these kernels")
+    gain_code = F32
+    if prepare.q_gain is not None:
+        _need(prepare.q_gain, "query norm gain", (d,))
+        _need(prepare.k_gain, "key norm gain", (d,), prepare.q_gain.dtype)
+        gain_code = _code(prepare.q_gain, "query norm gain")
+    if prepare.cos is not None:
+        _need(prepare.cos, "cosine table", None, torch.float32)
+        _need(prepare.sin, "sine table", tuple(prepare.cos.shape), torch.float32)
+        if prepare.cos.dim() != 2 or prepare.cos.shape[1] != d // 2:
+            raise TensorError(f"rotary tables have shape {tuple(prepare.cos.shape)}, expected [positions, {d // 2}]")
+    live = getattr(batch, "live_seqs", None)
+    _check(library().pl_attention_near(
+        qkv.data_ptr(), out.data_ptr(), _ptr(prepare.q_gain), _ptr(prepare.k_gain), gain_code, float(prepare.eps), _ptr(prepare.cos), _ptr(prepare.sin),
+        batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.ctx_len.data_ptr(), S if live is None else int(live), kv.block_table.data_ptr(),
+        kv.block_table.shape[1], kv.block_size, kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), nq, nkv, float(scale), _stream()))
+    return out
+
+
 def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, d: int, scale: float,
                    window: int, prepare: QkFusion) -> torch.Tensor:
     """Everything between the fused q/k/v projection and the output projection for the tokens of a step:
@@ -847,6 +889,11 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                       fuse=prepare, arrivals=_arrivals(batch, nq, splits))
+    near = getattr(batch, "near_ctx_len", None)
+    if (qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and near is not None and near <= NEAR_KEYS and _says_rows(batch)
+            and d == NEAR_HEAD and prepare.rot in (0, d) and not prepare.neighbours and prepare.write_kv and not window
+            and (getattr(batch, "live_seqs", None) or batch.num_seqs) * nq <= NEAR_WORKGROUPS):
+        return attention_near(qkv, out, batch, kv, nq, nkv, scale, prepare)
     qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
                           batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
                           nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)

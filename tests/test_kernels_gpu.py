@@ -2124,3 +2124,62 @@ def test_products_of_many_rows_refuse_what_they_do_not_take():
                  lambda: kernels.gemm_many(x, w, strips=w[:48].contiguous())):
         with pytest.raises(TensorError):
             call()
+
+
+@pytest.mark.parametrize("nq,nkv,bs,norm,turned", [(16, 8, 16, True, True), (4, 1, 1, False, True), (3, 3, 128, True, False), (8, 2, 7, False, False)])
+def test_attention_of_near_contexts_in_one_kernel(nq, nkv, bs, norm, turned):
+    """Fresh portions, portions behind others, single tokens and requests without tokens in one step, contexts of 1 to 128 on both sides of every tile of 32:
+    the pages get the bits that the stand-alone kernel writes and nothing else is written, the read-outs are those of 64-bit arithmetic over the same
+    rounded q and k within what bfloat16 leaves of weights and results (the tolerance of the tiled kernel's tests), a key whose page is missing is not
+    seen, what free rows hold does not enter, and a context longer than told gives NaN."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    d, eps, scale = 128, 1e-6, 128 ** -0.5
+    requests = [(37, 37), (1, 1), (128, 128), (65, 97), (0, 0), (1, 64), (16, 33), (64, 128), (33, 34), (96, 96)]      # (tokens, context)
+    S, per = len(requests), 128 // bs if 128 % bs == 0 else 128 // bs + 1
+    n = sum(t for t, _ in requests)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    table = torch.randperm(S * per, device=DEV).reshape(S, per).to(torch.int32)
+    if bs <= 32:
+        table[7, 20 // bs] = -1             # (a hole among the keys that were there before)
+    starts = [sum(t for t, _ in requests[:s]) for s in range(S)]
+    positions = i32([c - t + i for t, c in requests for i in range(t)])
+    seq_of = i32([s for s, (t, _) in enumerate(requests) for _ in range(t)])
+    qkv = torch.randn(n, (nq + 2 * nkv) * d, device=DEV).bfloat16()
+    q_gain, k_gain = ((torch.rand(d, device=DEV) + 0.5).bfloat16(), (torch.rand(d, device=DEV) + 0.5).bfloat16()) if norm else (None, None)
+    cos, sin = tables(128, d, 1e4) if turned else (None, None)
+    pools = [torch.full((S * per * bs, nkv * d), math.nan, device=DEV).bfloat16() for _ in range(2)]
+    slots = lambda s, keys: torch.tensor([int(table[s, k // bs]) * bs + k % bs for k in keys], device=DEV)
+    for s, (t, c) in enumerate(requests):
+        old = [k for k in range(c - t) if int(table[s, k // bs]) >= 0]
+        for pool in pools:
+            if old:
+                pool[slots(s, old)] = torch.randn(len(old), nkv * d, device=DEV).bfloat16()
+    kp, vp = (pool.clone() for pool in pools)
+    prepare = kernels.QkFusion(q_gain, k_gain, eps, cos, sin, d if turned else 0, True)
+    batch = SimpleNamespace(positions=positions, seq_of=seq_of, q_start=i32(starts), q_len=i32([t for t, _ in requests]), ctx_len=i32([c for _, c in requests]),
+                            num_seqs=S, num_tokens=n, max_ctx_len=1024, near_ctx_len=128, max_q_len=128)
+    kv = SimpleNamespace(block_table=table, block_size=bs, k_pool=kp, v_pool=vp)
+    assert S * nq <= kernels.NEAR_WORKGROUPS
+    out = torch.full((n, nq * d), 7.0, device=DEV).bfloat16()
+    kernels.attention_step(qkv.clone(), out, batch, kv, nq, nkv, d, scale, 0, prepare)
+    rows, k_want, v_want = qkv.clone(), pools[0].clone(), pools[1].clone()
+    kernels.qk_norm_rope_kv_write(rows, q_gain, k_gain, eps, cos, sin, prepare.rot, positions, seq_of, table, bs, k_want, v_want, nq, nkv, d)
+    bits = lambda x: x.view(torch.int16)
+    assert torch.equal(bits(kp), bits(k_want)) and torch.equal(bits(vp), bits(v_want))
+    for s, (t, c) in enumerate(requests):
+        if t == 0:
+            continue
+        there = [k for k in range(c) if int(table[s, k // bs]) >= 0]
+        k = kp[slots(s, there)].double().view(-1, nkv, d).repeat_interleave(nq // nkv, 1)
+        v = vp[slots(s, there)].double().view(-1, nkv, d).repeat_interleave(nq // nkv, 1)
+        q = rows[starts[s]:starts[s] + t, :nq * d].double().view(t, nq, d)
+        score = torch.einsum("thd,khd->htk", q, k) * scale
+        hidden = i32(there)[None, :] > torch.arange(c - t, c, device=DEV)[:, None]
+        want = torch.einsum("htk,khd->thd", torch.softmax(score.masked_fill(hidden[None], -math.inf), -1), v).reshape(t, nq * d)
+        assert rel(out[starts[s]:starts[s] + t], want) < 6e-3, (s, t, c)
+    batch.ctx_len[2] = 129
+    kernels.attention_near(qkv, out, batch, kv, nq, nkv, scale, prepare)
+    assert bool(out[starts[2]:starts[2] + 128].isnan().all()) and not bool(out[:38].isnan().any())
