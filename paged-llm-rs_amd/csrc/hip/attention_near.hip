@@ -12,80 +12,16 @@
 // cycles.  us, the two kernels before / this one, 16 heads over 8: 37 fresh tokens 12.2 / 8.6, 128 16.8 / 13.9, eight requests of 10 17.6 / 7.0,
 // 10 tokens behind 110 12.5 / 10.7.
 #include "common.hpp"
+#include "head_rows.hpp"
 
 typedef __bf16 an_bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 an_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float an_f32x16 __attribute__((ext_vector_type(16)));
-typedef float an_f32x4 __attribute__((ext_vector_type(4)));
-typedef float an_f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t an_u32x4 __attribute__((ext_vector_type(4)));
+typedef hr_u32x4 an_u32x4;
 typedef uint32_t an_u32x2 __attribute__((ext_vector_type(2)));
 
 #define AN_KEYS 128                // of a context, at most
 #define AN_D 128
 #define AN_V_PITCH (AN_KEYS * 2 + 8)   // bytes between two columns of values
-
-__device__ __forceinline__ uint32_t an_pack2(float lo, float hi) {
-    const an_f32x2 pair = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, an_bf16x2));
-}
-template <int CONTROL>
-__device__ __forceinline__ float an_dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CONTROL, 0xf, 0xf, true));
-}
-
-// Eight values of a head's row of 128, of which 16 lanes side by side hold all: normed with the gains g (GAIN) and turned by c and sn (TURN), and rounded.
-// The order of the sums is that of qk_norm_rope_kv_write_128_kernel.
-__device__ __forceinline__ an_u32x4 an_prepare(an_u32x4 raw, bool gain, const float (&g)[8], float eps, bool turn, const float (&c)[8], const float (&sn)[8], bool low) {
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        x[2 * e] = __uint_as_float(raw[e] << 16);
-        x[2 * e + 1] = __uint_as_float(raw[e] & 0xffff0000u);
-    }
-    if (gain) {
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
-        ss += an_dpp<0xB1>(ss);        // quad_perm [1,0,3,2]
-        ss += an_dpp<0x4E>(ss);        // quad_perm [2,3,0,1]
-        ss += an_dpp<0x141>(ss);       // lane i of 8 takes 7 - i
-        ss += an_dpp<0x140>(ss);       // lane i of 16 takes 15 - i
-        const float rinv = 1.f / sqrtf(ss / static_cast<float>(AN_D) + eps);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = x[e] * rinv * g[e];
-    }
-    if (turn) {
-        float px[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) px[e] = an_dpp<0x128>(x[e]);       // lane i of 16 takes i ^ 8
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = low ? x[e] * c[e] - px[e] * sn[e] : x[e] * c[e] + px[e] * sn[e];
-    }
-    return an_u32x4{an_pack2(x[0], x[1]), an_pack2(x[2], x[3]), an_pack2(x[4], x[5]), an_pack2(x[6], x[7])};
-}
-
-__device__ __forceinline__ void an_load8(const float* from, float (&to)[8]) {
-    const an_f32x4 a = *reinterpret_cast<const an_f32x4*>(from), b = *reinterpret_cast<const an_f32x4*>(from + 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        to[e] = a[e];
-        to[4 + e] = b[e];
-    }
-}
-
-__device__ __forceinline__ void an_load_gain(const void* gain, int dtype, int chunk, float (&to)[8]) {
-    if (dtype == PL_DTYPE_F32) {
-        an_load8(static_cast<const float*>(gain) + chunk * 8, to);
-    } else {
-        const an_u32x4 raw = *reinterpret_cast<const an_u32x4*>(static_cast<const bf16_t*>(gain) + chunk * 8);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            to[2 * e] = __uint_as_float(raw[e] << 16);
-            to[2 * e + 1] = __uint_as_float(raw[e] & 0xffff0000u);
-        }
-    }
-}
 
 __global__ void __launch_bounds__(512, 1)
 attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, const void* __restrict__ q_gain, const void* __restrict__ k_gain,
@@ -112,8 +48,8 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
     float gq[8], gk[8];
     const bool gain = q_gain != nullptr;
     if (gain) {
-        an_load_gain(q_gain, gain_dtype, chunk, gq);
-        an_load_gain(k_gain, gain_dtype, chunk, gk);
+        hr_load_gain(q_gain, gain_dtype, chunk, gq);
+        hr_load_gain(k_gain, gain_dtype, chunk, gk);
     }
     if (count <= 0 || ctx <= 0) return;                                // (padding; the whole workgroup)
     const size_t stride = static_cast<size_t>(nq + 2 * nkv) * AN_D;
@@ -159,16 +95,16 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
             k[u] = *reinterpret_cast<const an_u32x4*>(row + (nq + kvh) * AN_D);
             if (cos_table != nullptr) {
                 const size_t at = static_cast<size_t>(start + t) * (AN_D / 2) + (chunk & 7) * 8;
-                an_load8(cos_table + at, c[u]);
-                an_load8(sin_table + at, sn[u]);
+                hr_load8(cos_table + at, c[u]);
+                hr_load8(sin_table + at, sn[u]);
             }
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             if (first + 32 * u + wave * 4 >= count) continue;
             const int t = first + 32 * u + slot, key = start + t, at = place(key);
-            q[u] = an_prepare(q[u], gain, gq, eps, cos_table != nullptr, c[u], sn[u], low);
-            k[u] = an_prepare(k[u], gain, gk, eps, cos_table != nullptr, c[u], sn[u], low);
+            q[u] = hr_prepare(q[u], gain, gq, eps, cos_table != nullptr, c[u], sn[u], low);
+            k[u] = hr_prepare(k[u], gain, gk, eps, cos_table != nullptr, c[u], sn[u], low);
             if (t < count) {
                 *reinterpret_cast<an_u32x4*>(q_lds + t * 256 + (chunk ^ (t % 16)) * 16) = q[u];
                 *reinterpret_cast<an_u32x4*>(k_lds + key * 256 + (chunk ^ (key % 16)) * 16) = k[u];
@@ -244,8 +180,8 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const an_u32x4 packed = {an_pack2(s[kt][8 * u], s[kt][8 * u + 1]), an_pack2(s[kt][8 * u + 2], s[kt][8 * u + 3]),
-                                     an_pack2(s[kt][8 * u + 4], s[kt][8 * u + 5]), an_pack2(s[kt][8 * u + 6], s[kt][8 * u + 7])};
+            const an_u32x4 packed = {hr_pack2(s[kt][8 * u], s[kt][8 * u + 1]), hr_pack2(s[kt][8 * u + 2], s[kt][8 * u + 3]),
+                                     hr_pack2(s[kt][8 * u + 4], s[kt][8 * u + 5]), hr_pack2(s[kt][8 * u + 6], s[kt][8 * u + 7])};
             p[kt][u] = __builtin_bit_cast(an_bf16x8, packed);
         }
     }
@@ -270,7 +206,7 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
             bf16_t* to = out + static_cast<size_t>(row0 + token) * nq * AN_D + head * AN_D + d * 32 + 4 * h;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                *reinterpret_cast<an_u32x2*>(to + 8 * j) = an_u32x2{an_pack2(o[4 * j] * by, o[4 * j + 1] * by), an_pack2(o[4 * j + 2] * by, o[4 * j + 3] * by)};
+                *reinterpret_cast<an_u32x2*>(to + 8 * j) = an_u32x2{hr_pack2(o[4 * j] * by, o[4 * j + 1] * by), hr_pack2(o[4 * j + 2] * by, o[4 * j + 3] * by)};
         }
     }
 }

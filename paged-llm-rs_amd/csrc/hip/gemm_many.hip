@@ -20,6 +20,7 @@
 // 2,048 294 / 332: the library's.  Added into the stream with the norm behind it, 1,024 columns: of 2,048, 512 rows 13.7 / 13.2, 2,048 22.5 / 16.7; of
 // 3,072, 2,048 rows 26.6 / 21.1.  Plain, 4,096 columns of 1,024: 300 rows 10 / 7.5, 1,024 13.3 / 12.3, 2,048 20.3 / 20.8.
 #include "common.hpp"
+#include "head_rows.hpp"
 
 typedef __bf16 gm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 gm_bf16x2 __attribute__((ext_vector_type(2)));
@@ -33,6 +34,7 @@ typedef uint32_t gm_u32x2 __attribute__((ext_vector_type(2)));
 #define GM_SWIGLU 1        // w is [gate | up], N rows each: y (bfloat16) = silu(gate) * up
 #define GM_ADD 2           // y (32-bit, the residual stream) += result
 #define GM_STORE32 3       // y (32-bit) = result
+#define GM_HEADS 4         // rows [q | k | v] of heads of 128: q normed and turned into y (bfloat16 [M, N]), k (the same) and v into the pages (GmHeads)
 
 #define GM_BK 64           // K a stage
 #define GM_STRIPE 64       // columns of the stream whose squares are one number of a norm handed forward
@@ -48,6 +50,18 @@ struct GmNorms {
     float* sums;               // [M, N / 64] the sums of squares of every 64 columns of y; null: no norm
 };
 #define GM_TAKEN_MOST 64
+
+// What GM_HEADS does with its rows: qk_norm_rope_kv_write_128_kernel's work, on the tile on its way out (heads of 128 rotated whole or not at all).
+struct GmHeads {
+    const void *q_gain, *k_gain;       // [128] or null
+    int gain_dtype;
+    float eps;
+    const float *cos_table, *sin_table;        // [positions, 64] or null
+    const int *positions, *seq_of, *block_table;
+    int max_blocks, block_size;
+    bf16_t *k_pool, *v_pool;
+    int nq, nkv;
+};
 
 // Grouped: the rows are dealt to groups (experts), every group with a weight matrix of its own, one behind the other in w.  A tile of 128 rows belongs to one
 // group (`tile_group`; the tiles in use come first, and how many they are stands behind the last of all); row r of the tiles reads row gather[r] of x (null: row r itself; negative: a row of
@@ -99,10 +113,11 @@ constexpr int gm_out_cols(int CT, int epi) { return 4 * (epi == GM_SWIGLU ? 16 :
 constexpr bool gm_is_32(int epi) { return epi == GM_ADD || epi == GM_STORE32; }
 // bytes between two rows of the tile on its way out
 constexpr int gm_pitch(int CT, int epi) { return gm_out_cols(CT, epi) * (gm_is_32(epi) ? 4 : 2) + 16; }
-// ... and of the LDS of a workgroup: two stages of x (and of weights in rows), or the tile on its way out, and 1 / rms of its rows
+// ... and of the LDS of a workgroup: two stages of x (and of weights in rows), or the tile on its way out, and 1 / rms of its rows (with GM_HEADS also
+// their positions and places in the pages)
 constexpr int gm_lds_bytes(int CT, int RT, int epi, bool strips) {
     const int in = 2 * 32 * RT * GM_BK * 2 + (strips ? 0 : 4 * 2 * 32 * CT * GM_BK * 2), out = 32 * RT * gm_pitch(CT, epi);
-    return (in > out ? in : out) + 32 * RT * 4;
+    return (in > out ? in : out) + 32 * RT * (epi == GM_HEADS ? 12 : 4);
 }
 
 // CT, RT: a wave's tiles of 32 rows of w (with GM_SWIGLU 16 of gate, 16 of up) and of 32 rows of x.  N a multiple of 16, K of 64; rows and columns past the
@@ -112,7 +127,7 @@ constexpr int gm_lds_bytes(int CT, int RT, int epi, bool strips) {
 template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS, bool GROUPED = false>
 __global__ void __launch_bounds__(256, PER_SIMD)
 gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weights, void* __restrict__ y_, int M, int N, int K,
-                   int row_tiles, int col_tiles, GmNorms norms, GmGroups groups) {
+                   int row_tiles, int col_tiles, GmNorms norms, GmGroups groups, GmHeads heads) {
     static_assert(!GROUPED || (RT == 4 && !TAKES && !STRIPS && EPI != GM_ADD), "groups' tiles are of 128 rows");
     constexpr int ROWS = 32 * RT, STAGE = ROWS * GM_BK * 2;
     extern __shared__ __attribute__((aligned(16))) char gm_lds[];          // two stages of x [row][64], then the tile on its way out
@@ -273,6 +288,14 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
             ask_w(set, GmInt<3>{}, s, c);
         }
     };
+    // where the tile's rows stand, a thread a row (its page is asked for behind the first stages and looked at when the tile leaves)
+    int row_pos = -1, row_seq = 0, row_page = -1;
+    if constexpr (EPI == GM_HEADS) {
+        if (tid < ROWS && m0 + tid < M) {
+            row_pos = heads.positions[m0 + tid];
+            row_seq = heads.seq_of[m0 + tid];
+        }
+    }
     // the sums of squares of the tile's rows, four lanes a row, asked for first
     constexpr int PASSES = (ROWS + 63) / 64;
     gm_f32x4 sums[TAKES ? PASSES : 1][GM_TAKEN_MOST / 16];
@@ -291,6 +314,9 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
     ask_all(GmInt<0>{}, 0);
     ask_all(GmInt<1>{}, 1);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (EPI == GM_HEADS) {
+        if (row_pos >= 0) row_page = heads.block_table[static_cast<size_t>(row_seq) * heads.max_blocks + row_pos / heads.block_size];
+    }
 #pragma unroll
     for (int i = 0; i < RT; ++i) put_x(GmInt<0>{}, 0, i);
 #pragma unroll
@@ -309,6 +335,7 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
         }
     }
     float* const scales = reinterpret_cast<float*>(gm_lds + gm_lds_bytes(CT, RT, EPI, STRIPS) - ROWS * 4);
+    int* const places = reinterpret_cast<int*>(scales) - 2 * ROWS;         // (GM_HEADS) [row]: its position and its row of the pages, or -1
     if constexpr (TAKES) {
 #pragma unroll
         for (int q = 0; q < PASSES; ++q) {
@@ -348,6 +375,12 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
         }
     };
     if constexpr (EPI == GM_ADD) ask_old(0);
+    if constexpr (EPI == GM_HEADS) {
+        if (tid < ROWS) {
+            places[2 * tid] = row_pos;
+            places[2 * tid + 1] = row_page >= 0 ? row_page * heads.block_size + row_pos % heads.block_size : -1;
+        }
+    }
     __syncthreads();
 
     // The tile leaves through LDS in whole rows.  acc[c][t][4 j + i]: row 32 t + r32, row of A 8 j + 4 h + i
@@ -375,7 +408,46 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
             }
     }
     __syncthreads();
-    if constexpr (!IS_32) {
+    if constexpr (EPI == GM_HEADS) {
+        // 16 lanes a head's row; the angles of four rows are asked for together.  Bound by the vector instructions, some 140 a row and 9 cycles apart where a wave
+        // is alone on its SIMD (128 rows by 256 columns 8 us, 128 by 128 two a compute unit 5): the shapes are chosen with that.  us, the product and the
+        // stand-alone kernel / this one, 16 heads over 8 of a width of 1,024: 300 rows 12.3 / 10.3, 1,024 21.8 / 17.0, 2,048 30.3 / 27.2.
+        static_assert(EPI != GM_HEADS || (ROWS * LANES) % (4 * 256) == 0, "whole groups of four rows a thread");
+        const int chunk = tid % 16;
+        const bool gain = heads.q_gain != nullptr, turn = heads.cos_table != nullptr;
+        float gq[8], gk[8];
+        if (gain) {
+            hr_load_gain(heads.q_gain, heads.gain_dtype, chunk, gq);
+            hr_load_gain(heads.k_gain, heads.gain_dtype, chunk, gk);
+        }
+        for (int i0 = tid; i0 < ROWS * LANES; i0 += 4 * 256) {
+            float cs[4][8], sn[4][8];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = (i0 + 256 * u) / LANES;
+                if (turn) {
+                    const size_t at = static_cast<size_t>(max(places[2 * r], 0)) * 64 + (chunk & 7) * 8;
+                    hr_load8(heads.cos_table + at, cs[u]);
+                    hr_load8(heads.sin_table + at, sn[u]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = (i0 + 256 * u) / LANES, head = n0 / 128 + (i0 + 256 * u) % LANES / 16;
+                const bool is_q = head < heads.nq, is_k = !is_q && head < heads.nq + heads.nkv;
+                hr_u32x4 v = *reinterpret_cast<const hr_u32x4*>(gm_lds + r * PITCH + (i0 + 256 * u) % LANES * 16);
+                if (is_q || is_k) v = hr_prepare(v, gain, is_q ? gq : gk, heads.eps, turn, cs[u], sn[u], chunk < 8);
+                const int place = places[2 * r + 1];
+                bf16_t* to = static_cast<bf16_t*>(y_) + static_cast<size_t>(m0 + r) * N + head * 128;
+                bool there = m0 + r < M && places[2 * r] >= 0 && head * 128 < N;
+                if (!is_q) {
+                    there = there && place >= 0;               // (never written through a hole in the table)
+                    to = (is_k ? heads.k_pool : heads.v_pool) + (static_cast<size_t>(max(place, 0)) * heads.nkv + head - heads.nq - (is_k ? 0 : heads.nkv)) * 128;
+                }
+                if (there) *reinterpret_cast<hr_u32x4*>(to + chunk * 8) = v;
+            }
+        }
+    } else if constexpr (!IS_32) {
         bf16_t* y = static_cast<bf16_t*>(y_);
         for (int i = tid; i < ROWS * LANES; i += 256) {
             const int r = i / LANES, piece = i % LANES;
@@ -417,6 +489,7 @@ struct GmProduct {
     void* y;
     int M, N, K;
     GmNorms norms;
+    GmHeads heads;
 };
 
 template <int CT, int RT, int PER_SIMD, int EPI, bool TAKES, bool STRIPS>
@@ -430,7 +503,7 @@ static int gm_launch_one(const GmProduct& g, hipStream_t stream) {
         PL_REQUIRE(e == hipSuccess, "product of many rows: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
     }
     gemm_many_kernel<CT, RT, PER_SIMD, EPI, TAKES, STRIPS><<<row_tiles * col_tiles, 256, lds, stream>>>(
-        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, GmGroups{});
+        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, GmGroups{}, g.heads);
     PL_CHECK_LAUNCH("gemm_many");
     return 0;
 }
@@ -450,13 +523,13 @@ static int gm_launch(const GmProduct& g, hipStream_t stream) {
 // results of the largest tile would not fit into LDS.)
 struct GmShape {
     int ct, rt;
-    float stage, tile[4];      // (by epilogue)
+    float stage, tile[5];      // (by epilogue)
 };
-static const GmShape GM_SHAPES[] = {{1, 2, 0.25f, {1.5f, 3.0f, 4.0f, 2.5f}},
-                                    {1, 4, 0.37f, {2.2f, 2.9f, 8.0f, 4.0f}},
-                                    {2, 3, 0.425f, {3.0f, 5.2f, 10.f, 5.0f}},
-                                    {2, 4, 0.54f, {4.0f, 5.8f, 14.f, 6.0f}},
-                                    {3, 4, 0.755f, {6.0f, 9.0f, 0.f, 0.f}}};
+static const GmShape GM_SHAPES[] = {{1, 2, 0.25f, {1.5f, 3.0f, 4.0f, 2.5f, 4.0f}},
+                                    {1, 4, 0.37f, {2.2f, 2.9f, 8.0f, 4.0f, 7.0f}},
+                                    {2, 3, 0.425f, {3.0f, 5.2f, 10.f, 5.0f, 10.f}},
+                                    {2, 4, 0.54f, {4.0f, 5.8f, 14.f, 6.0f, 18.f}},
+                                    {3, 4, 0.755f, {6.0f, 9.0f, 0.f, 0.f, 22.f}}};
 
 static int gm_pick(int M, int N, int K, int epilogue) {
     int best = 0;
@@ -503,11 +576,33 @@ extern "C" int pl_gemm_many(const void* x, const void* weights, int in_strips, v
                taken_count, epilogue);
     PL_REQUIRE((gain == nullptr) == (rows == nullptr) && (gain == nullptr) == (sums == nullptr) && (gain == nullptr || (epilogue == GM_ADD && N % GM_STRIPE == 0)),
                "product of many rows: a norm handed forward by epilogue %d", epilogue);
-    const GmProduct g{x, weights, in_strips != 0, y, M, N, K, GmNorms{taken, taken_count, eps, gain, static_cast<bf16_t*>(rows), sums}};
+    const GmProduct g{x, weights, in_strips != 0, y, M, N, K, GmNorms{taken, taken_count, eps, gain, static_cast<bf16_t*>(rows), sums}, GmHeads{}};
     if (epilogue == GM_STORE) return gm_shaped<GM_STORE>(g, stream);
     if (epilogue == GM_SWIGLU) return gm_shaped<GM_SWIGLU>(g, stream);
     if (epilogue == GM_ADD) return gm_shaped<GM_ADD>(g, stream);
     return gm_shaped<GM_STORE32>(g, stream);
+}
+
+// The projection [q | k | v] of heads of 128 and what stands between it and attention (see GmHeads).  x, weights: as pl_gemm_many, N = (nq + 2 nkv) 128.  y: bfloat16
+// [M, N], of which the queries are written; rows at negative positions are not.  taken: as pl_gemm_many.
+extern "C" int pl_gemm_many_heads(const void* x, const void* weights, int in_strips, void* y, int M, int K, const float* taken, int taken_count,
+                                  float taken_eps, const void* q_gain, const void* k_gain, int gain_dtype, float eps, const float* cos_table,
+                                  const float* sin_table, const int* positions, const int* seq_of, const int* block_table, int max_blocks, int block_size,
+                                  void* k_pool, void* v_pool, int nq, int nkv, hipStream_t stream) {
+    const int N = (nq + 2 * nkv) * 128;
+    PL_REQUIRE(nq > 0 && nkv > 0 && nq <= (1 << 16) && nkv <= (1 << 16) && pl_gemm_many_applies(M, N, K, GM_STORE), "heads of many rows: %d rows, %d and %d heads, inner width %d",
+               M, nq, nkv, K);
+    PL_REQUIRE(block_size > 0 && max_blocks > 0, "heads of many rows: block size %d, %d blocks a row", block_size, max_blocks);
+    PL_REQUIRE((q_gain == nullptr) == (k_gain == nullptr) && (cos_table == nullptr) == (sin_table == nullptr), "heads of many rows: one of the two gains or tables is missing");
+    PL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weights) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(k_pool) |
+                reinterpret_cast<uintptr_t>(v_pool) | reinterpret_cast<uintptr_t>(q_gain) | reinterpret_cast<uintptr_t>(k_gain) |
+                reinterpret_cast<uintptr_t>(cos_table) | reinterpret_cast<uintptr_t>(sin_table)) % 16 == 0, "heads of many rows: rows that are not aligned to 16 bytes");
+    PL_REQUIRE(taken == nullptr || (taken_count > 0 && taken_count <= GM_TAKEN_MOST && taken_count % 4 == 0 && reinterpret_cast<uintptr_t>(taken) % 16 == 0),
+               "heads of many rows: %d sums of a norm", taken_count);
+    const GmProduct g{x, weights, in_strips != 0, y, M, N, K, GmNorms{taken, taken_count, taken_eps, nullptr, nullptr, nullptr},
+                      GmHeads{q_gain, k_gain, gain_dtype, eps, cos_table, sin_table, positions, seq_of, block_table, max_blocks, block_size,
+                              static_cast<bf16_t*>(k_pool), static_cast<bf16_t*>(v_pool), nq, nkv}};
+    return gm_shaped<GM_HEADS>(g, stream);
 }
 
 template <int CT, int PER_SIMD, int EPI>
@@ -519,7 +614,7 @@ static int gm_launch_grouped(const GmProduct& g, const GmGroups& groups, int row
                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     PL_REQUIRE(e == hipSuccess, "grouped product of many rows: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
     gemm_many_kernel<CT, 4, PER_SIMD, EPI, false, false, true><<<row_tiles * col_tiles, 256, lds, stream>>>(
-        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, groups);
+        static_cast<const bf16_t*>(g.x), static_cast<const bf16_t*>(g.weights), g.y, g.M, g.N, g.K, row_tiles, col_tiles, g.norms, groups, GmHeads{});
     PL_CHECK_LAUNCH("gemm_many_grouped");
     return 0;
 }
@@ -546,7 +641,7 @@ extern "C" int pl_gemm_many_grouped(const void* x, const void* w, void* y, const
     PL_REQUIRE(tile_group != nullptr && (gather != nullptr || x_rows >= row_tiles * 128), "grouped product of many rows: %d rows for %d tiles", x_rows, row_tiles);
     PL_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w_last)) % 16 == 0 &&
                    w_stride % 8 == 0, "grouped product of many rows: rows that are not aligned to 16 bytes");
-    const GmProduct g{x, w, false, y, row_tiles * 128, N, K, GmNorms{}};
+    const GmProduct g{x, w, false, y, row_tiles * 128, N, K, GmNorms{}, GmHeads{}};
     const GmGroups groups{tile_group, gather, w_stride, x_pitch, y_pitch, last, N_last, K_last, static_cast<const bf16_t*>(w_last)};
     const int columns = last >= 0 && N_last > N ? N_last : N;
     int best = 0;

@@ -59,6 +59,7 @@ def _signatures(lib) -> None:
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
         "pl_gemm_many": [p, p, i, p, i, i, i, i, p, i, f, p, p, p, p],
         "pl_gemm_many_applies": [i, i, i, i],
+        "pl_gemm_many_heads": [p, p, i, p, i, i, p, i, f, p, p, i, f, p, p, p, p, p, i, i, p, p, i, i, p],
         "pl_gemm_many_grouped": [p, p, p, p, p, ctypes.c_longlong, i, i, i, i, i, i, i, i, i, p, i, i, p],
         "pl_gemm_many_grouped_applies": [i, i, i, i, i],
         "pl_gemm_tiled_applies": [i, i, i, i],
@@ -844,15 +845,21 @@ NEAR_HEAD = 128
 NEAR_WORKGROUPS = 512
 
 
-def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, scale: float, prepare: QkFusion) -> torch.Tensor:
-    """Everything between the fused q/k/v projection and the output projection for a step whose contexts are no longer than 128 tokens
-    (``NEAR_KEYS``; rows of longer ones come out as NaN): heads of 128 rotated whole or not at all, in bfloat16."""
-    n, d, S = qkv.shape[0], NEAR_HEAD, kv.block_table.shape[0]
-    _need(qkv, "fused q/k/v projection", (n, (nq + 2 * nkv) * d), torch.bfloat16)
-    _need(out, "attention output", (n, nq * d), torch.bfloat16)
-    _need(kv.block_table, "block table", None, torch.int32)
-    for t, what in ((batch.q_start, "first row of each request"), (batch.q_len, "tokens of each request"), (batch.ctx_len, "context length of each request")):
-        _need(t, what, (S,), torch.int32)
+def near_applies(batch, nq: int, d: int, window: int, prepare: QkFusion) -> bool:
+    """Whether a step of bfloat16 rows goes to ``attention_near``."""
+    near = getattr(batch, "near_ctx_len", None)
+    return (_attention_mode == "kernel" and near is not None and near <= NEAR_KEYS and _says_rows(batch) and prepares_whole_heads(d, prepare)
+            and not window and (getattr(batch, "live_seqs", None) or batch.num_seqs) * nq <= NEAR_WORKGROUPS)
+
+
+def prepares_whole_heads(d: int, prepare: QkFusion) -> bool:
+    """Heads of 128 rotated whole, by halves, or not at all, whose keys and values go into the pages."""
+    return d == NEAR_HEAD and prepare.rot in (0, d) and not prepare.neighbours and prepare.write_kv
+
+
+def _heads_code(kv, nkv: int, prepare: QkFusion) -> int:
+    """The code of the gains' type, once pages, gains and tables are what the kernels for whole heads of 128 take."""
+    d = NEAR_HEAD
     for pool, what in ((kv.k_pool, "key pool"), (kv.v_pool, "value pool")):
         _need(pool, what, None, torch.bfloat16)
         if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % kv.block_size != 0:
@@ -869,6 +876,19 @@ def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
         _need(prepare.sin, "sine table", tuple(prepare.cos.shape), torch.float32)
         if prepare.cos.dim() != 2 or prepare.cos.shape[1] != d // 2:
             raise TensorError(f"rotary tables have shape {tuple(prepare.cos.shape)}, expected [positions, {d // 2}]")
+    return gain_code
+
+
+def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, scale: float, prepare: QkFusion) -> torch.Tensor:
+    """Everything between the fused q/k/v projection and the output projection for a step whose contexts are no longer than 128 tokens
+    (``NEAR_KEYS``; rows of longer ones come out as NaN): heads of 128 rotated whole or not at all, in bfloat16."""
+    n, d, S = qkv.shape[0], NEAR_HEAD, kv.block_table.shape[0]
+    _need(qkv, "fused q/k/v projection", (n, (nq + 2 * nkv) * d), torch.bfloat16)
+    _need(out, "attention output", (n, nq * d), torch.bfloat16)
+    _need(kv.block_table, "block table", None, torch.int32)
+    for t, what in ((batch.q_start, "first row of each request"), (batch.q_len, "tokens of each request"), (batch.ctx_len, "context length of each request")):
+        _need(t, what, (S,), torch.int32)
+    gain_code = _heads_code(kv, nkv, prepare)
     live = getattr(batch, "live_seqs", None)
     _check(library().pl_attention_near(
         qkv.data_ptr(), out.data_ptr(), _ptr(prepare.q_gain), _ptr(prepare.k_gain), gain_code, float(prepare.eps), _ptr(prepare.cos), _ptr(prepare.sin),
@@ -878,25 +898,23 @@ def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
 
 
 def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, d: int, scale: float,
-                   window: int, prepare: QkFusion) -> torch.Tensor:
+                   window: int, prepare: QkFusion, prepared: bool = False) -> torch.Tensor:
     """Everything between the fused q/k/v projection and the output projection for the tokens of a step:
     per-head norm and rotation of q and k, the write of k and v into the pages, attention.  A step in
     which every request brings one token (in bfloat16) does all of it in the attention kernel;
-    any other step runs the stand-alone kernel for the first three and then attention."""
-    if (qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and batch.max_q_len == 1
+    any other step runs the stand-alone kernel for the first three (or its projection has done it: ``prepared``) and then attention."""
+    if (not prepared and qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and batch.max_q_len == 1
             and prepare.rot % 16 == 0 and not prepare.neighbours and not grouped_applies(nq, nkv, d, kv.block_size)):
         splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d, _has_arrivals(batch))
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                       fuse=prepare, arrivals=_arrivals(batch, nq, splits))
-    near = getattr(batch, "near_ctx_len", None)
-    if (qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and near is not None and near <= NEAR_KEYS and _says_rows(batch)
-            and d == NEAR_HEAD and prepare.rot in (0, d) and not prepare.neighbours and prepare.write_kv and not window
-            and (getattr(batch, "live_seqs", None) or batch.num_seqs) * nq <= NEAR_WORKGROUPS):
+    if not prepared and qkv.dtype == torch.bfloat16 and near_applies(batch, nq, d, window, prepare):
         return attention_near(qkv, out, batch, kv, nq, nkv, scale, prepare)
-    qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
-                          batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
-                          nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)
+    if not prepared:
+        qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
+                              batch.positions, batch.seq_of, kv.block_table, kv.block_size, kv.k_pool, kv.v_pool,
+                              nq, nkv, d, write_kv=prepare.write_kv, neighbours=prepare.neighbours)
     return paged_attention(qkv, out, batch, kv, nq, nkv, d, scale, window, near=getattr(batch, "near_ctx_len", None))
 
 
@@ -1285,6 +1303,36 @@ def gemm_many(x: torch.Tensor | None, w: torch.Tensor, out_dtype: torch.dtype = 
         _ptr(hand.x if hand is not None else None), _ptr(hand.ssq if hand is not None else None), _stream()))
     if hand is not None:
         hand.filled = True
+    return out
+
+
+def gemm_many_heads(x: torch.Tensor | None, w: torch.Tensor, batch, kv, nq: int, nkv: int, prepare: QkFusion,
+                    handed: "HandedNorm | None" = None, strips: torch.Tensor | None = None) -> torch.Tensor:
+    """The projection [q | k | v] of many bfloat16 rows (``gemm_many``) with what ``qk_norm_rope_kv_write`` does behind it as its last stage, to the same
+    bits: the rows that come back hold the queries, normed and turned; keys and values are in the pages.  Heads of 128 (``prepares_whole_heads``)."""
+    if handed is not None:
+        if not handed.filled:
+            raise TensorError("a handed norm is the product's input once a product has written it")
+        x = handed.x
+    _need(x, "matrix product input", None, torch.bfloat16)
+    M, K = x.shape
+    N = (nq + 2 * nkv) * NEAR_HEAD
+    _need(w, "weight", (N, K), torch.bfloat16)
+    if strips is not None:
+        _need(strips, "weights in strips", (N, K), torch.bfloat16)
+    _need(batch.positions, "positions", (M,), torch.int32)
+    _need(batch.seq_of, "request index of each token", (M,), torch.int32)
+    _need(kv.block_table, "block table", None, torch.int32)
+    if not prepares_whole_heads(NEAR_HEAD, prepare) or kv.block_table.dim() != 2:
+        raise TensorError(f"heads prepared by their projection: a rotation of {prepare.rot}, block table of shape {tuple(kv.block_table.shape)}")
+    gain_code = _heads_code(kv, nkv, prepare)
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _check(library().pl_gemm_many_heads(
+        x.data_ptr(), (w if strips is None else strips).data_ptr(), 0 if strips is None else 1, out.data_ptr(), M, K,
+        _ptr(handed.ssq if handed is not None else None), handed.ssq.shape[1] if handed is not None else 0, float(handed.eps if handed is not None else 0.0),
+        _ptr(prepare.q_gain), _ptr(prepare.k_gain), gain_code, float(prepare.eps), _ptr(prepare.cos), _ptr(prepare.sin), batch.positions.data_ptr(),
+        batch.seq_of.data_ptr(), kv.block_table.data_ptr(), kv.block_table.shape[1], kv.block_size, kv.k_pool.data_ptr(), kv.v_pool.data_ptr(),
+        nq, nkv, _stream()))
     return out
 
 

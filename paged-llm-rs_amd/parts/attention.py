@@ -87,16 +87,23 @@ class PagedAttention:
         projection can add into it, None comes back."""
         batch = ctx.batch
         kv = ctx.kv()
-        qkv = self.qkv_proj.forward(x)
         cos = self.rotary.cos if self.rotary is not None else None
         sin = self.rotary.sin if self.rotary is not None else None
         rot = self.rotary.dim if self.rotary is not None else 0
         prepare = kernels.QkFusion(self.q_gain, self.k_gain, self.eps, cos, sin, rot, ctx.writes_cache,
                                    neighbours=bool(getattr(self.rotary, "neighbours", False)))
+        # (many rows: the projection may do what stands between it and attention, unless one kernel does that and the attention)
+        qkv = None
+        if (ctx.trace is None and batch.max_q_len > 1 and kernels.prepares_whole_heads(self.d, prepare)
+                and not kernels.near_applies(batch, self.nq, self.d, self.window, prepare)):
+            qkv = self.qkv_proj.forward_heads(x, batch, kv, self.nq, self.nkv, prepare)
+        prepared = qkv is not None
+        if not prepared:
+            qkv = self.qkv_proj.forward(x)
         out = torch.empty((qkv.shape[0], self.nq * self.d), dtype=qkv.dtype, device=qkv.device)
         if ctx.trace is not None:
             self._record_projections(qkv, batch, kv, ctx.trace)
-        kernels.attention_step(qkv, out, batch, kv, self.nq, self.nkv, self.d, self.scale, self.window, prepare)
+        kernels.attention_step(qkv, out, batch, kv, self.nq, self.nkv, self.d, self.scale, self.window, prepare, prepared=prepared)
         if ctx.trace is not None:
             ctx.trace.record("o_proj.in", out)
             out = self.o_proj.forward(out)

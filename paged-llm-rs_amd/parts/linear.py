@@ -66,6 +66,23 @@ class Linear:
             return kernels.gemm_skinny(x, self.weight, activation=activation, strips=self.strips, activated=True)
         return kernels.activation(self.forward(x), activation)
 
+    def forward_heads(self, x, batch, kv, nq: int, nkv: int, prepare):
+        """The projection [q | k | v] with norm, rotation and page write behind it in one kernel (``kernels.gemm_many_heads``), or None where the product
+        of so many rows is not that kernel's."""
+        if self.bias is not None or self.weight.dtype != torch.bfloat16:
+            return None
+        handed = None
+        if isinstance(x, PendingNorm):
+            if x.out_dtype != torch.bfloat16 or x.width != self.in_features:
+                return None
+            if x.handed is not None and kernels.many_takes(x.handed, x.num_rows, self.out_features, self.in_features):
+                handed = x.handed
+        if handed is None and not kernels.many_store_wins(x.num_rows if isinstance(x, PendingNorm) else x.shape[0], self.out_features, self.in_features):
+            return None
+        if handed is None and isinstance(x, PendingNorm):
+            x = x.materialize()
+        return kernels.gemm_many_heads(None if handed is not None else x, self.weight, batch, kv, nq, nkv, prepare, handed=handed, strips=self.strips)
+
     def _product(self, x, out_dtype: torch.dtype | None = None, add_into: torch.Tensor | None = None,
                  swiglu: bool = False, activation: str = "silu", hand=None):
         if isinstance(x, PendingNorm):

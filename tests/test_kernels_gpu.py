@@ -2183,3 +2183,45 @@ def test_attention_of_near_contexts_in_one_kernel(nq, nkv, bs, norm, turned):
     batch.ctx_len[2] = 129
     kernels.attention_near(qkv, out, batch, kv, nq, nkv, scale, prepare)
     assert bool(out[starts[2]:starts[2] + 128].isnan().all()) and not bool(out[:38].isnan().any())
+
+
+@pytest.mark.parametrize("nq,nkv,K,norm,turned", [(16, 8, 1024, True, True), (4, 1, 128, False, True), (3, 3, 192, True, False), (5, 1, 64, False, False)])
+def test_the_projection_of_many_rows_prepares_its_heads(nq, nkv, K, norm, turned):
+    """Queries and pages have the bits that the product and the stand-alone kernel behind it give, at every shape of tile, with tiles that end inside the rows
+    and the heads, rows of padding, a page that is missing, out of rows, out of strips and behind a handed norm; nothing else is written."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    d, eps, bs, pages = 128, 1e-6, 16, 200
+    N = (nq + 2 * nkv) * d
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).bfloat16()
+    strips = kernels.weights_in_strips(w)
+    gains = [(torch.rand(d, device=DEV) + 0.5).to(torch.bfloat16 if nq % 2 else torch.float32) for _ in range(2)] if norm else [None, None]
+    cos, sin = tables(2200, d, 1e4) if turned else (None, None)
+    prepare = kernels.QkFusion(*gains, eps, cos, sin, d if turned else 0, True)
+    bits = lambda t: t.view(torch.int16)
+    for n in (65, 130, 300, 700, 1100, 2100):
+        x = torch.randn(n, K, device=DEV).bfloat16()
+        positions = torch.arange(n, dtype=torch.int32, device=DEV)
+        positions[n // 2] = -1
+        positions[n - 1] = -1
+        table = torch.randperm(pages, device=DEV)[:(n + bs - 1) // bs].to(torch.int32)[None].contiguous()
+        table[0, 1] = -1
+        seq_of = torch.zeros(n, dtype=torch.int32, device=DEV)
+        batch = SimpleNamespace(positions=positions, seq_of=seq_of)
+        fresh = lambda: SimpleNamespace(block_table=table, block_size=bs, k_pool=torch.full((pages * bs, nkv * d), 3.0, device=DEV).bfloat16(),
+                                        v_pool=torch.full((pages * bs, nkv * d), 5.0, device=DEV).bfloat16())
+        hand = None
+        if K % 256 == 0:
+            hand = kernels.HandedNorm(torch.ones(K, device=DEV), eps, n, K, DEV)
+            kernels.gemm_many(torch.randn(n, 64, device=DEV).bfloat16(), torch.randn(K, 64, device=DEV).bfloat16(), add_into=torch.randn(n, K, device=DEV), hand=hand)
+        for handed in (None, hand) if hand is not None else (None,):
+            want_kv, rows = fresh(), kernels.gemm_many(None if handed else x, w, handed=handed)
+            kernels.qk_norm_rope_kv_write(rows, *gains, eps, cos, sin, prepare.rot, positions, seq_of, table, bs, want_kv.k_pool, want_kv.v_pool, nq, nkv, d)
+            for s in (None, strips):
+                kv = fresh()
+                got = kernels.gemm_many_heads(None if handed else x, w, batch, kv, nq, nkv, prepare, handed=handed, strips=s)
+                live = positions >= 0
+                assert torch.equal(bits(got[live][:, :nq * d]), bits(rows[live][:, :nq * d])), (n, handed is None, s is None)
+                assert torch.equal(bits(kv.k_pool), bits(want_kv.k_pool)) and torch.equal(bits(kv.v_pool), bits(want_kv.v_pool)), (n, handed is None, s is None)
