@@ -1231,14 +1231,22 @@ def many_swiglu_wins(rows: int, columns: int, width: int) -> bool:
 
 # The plain product, bfloat16 or 32-bit: up to a width of 1,024, as long as the rows and columns of the result are few (us, library / this one:
 # 4,096 columns: 65 rows 9.0 / 7.1, 450 11.1 / 8.1, 1,024 13.3 / 12.3, 1,536 16.8 / 15.7, 2,560 23.8 / 26.3; 1,024 columns: 65 rows 8.4 / 6.9,
-# 4,096 13.4 / 12.4, 8,192 20.5 / 20.7; of 2,048 and wider the library's is as fast at most sizes).
+# 4,096 13.4 / 12.4, 8,192 20.5 / 20.7); and up to 3,072 where its smallest tiles (64 by 128) are one a compute unit, or a little less (1,024 columns: K 2,048,
+# 1,024 rows, 128 tiles, 11.2 / 11.8, 1,152 13.5 / 11.8, 2,048 15.6 / 12.6; K 3,072, 1,152 rows 17.6 / 16.8, 2,048 20.9 / 18.4; 2,048 columns of 2,048:
+# 640 rows 13.6 / 11.6, 1,024 15.6 / 12.8).
 MANY_STORE_WIDTH = 1024
 MANY_STORE_RESULTS = 6.25e6
+MANY_STORE_WIDE = 3072
+MANY_STORE_WIDE_TILES = (0.56, 1.0)     # of the compute units
 
 
 def many_store_wins(rows: int, columns: int, width: int) -> bool:
-    return (rows > SKINNY_ROWS and width <= MANY_STORE_WIDTH and rows * columns <= MANY_STORE_RESULTS
-            and bool(library().pl_gemm_many_applies(rows, columns, width, 0)))
+    if rows <= SKINNY_ROWS or width > MANY_STORE_WIDE or not library().pl_gemm_many_applies(rows, columns, width, 0):
+        return False
+    if width <= MANY_STORE_WIDTH:
+        return rows * columns <= MANY_STORE_RESULTS
+    low, high = MANY_STORE_WIDE_TILES
+    return low * compute_units() <= -(-rows // 64) * -(-columns // 128) <= high * compute_units()
 
 
 # The product that adds into the stream and hands the norm behind it forward, against the library's product and the norm kernel: a workgroup of the
