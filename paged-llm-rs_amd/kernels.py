@@ -1249,6 +1249,24 @@ def many_store_wins(rows: int, columns: int, width: int) -> bool:
     return low * compute_units() <= -(-rows // 64) * -(-columns // 128) <= high * compute_units()
 
 
+# The projection onto a vocabulary, 32-bit out: a workgroup takes 128 columns and all of up to 64 rows, so the weights are read once and the rows out of L2.  Timed at 1 to
+# 200 rows over 12 vocabularies (us, before / this one, out of strips; in rows in brackets): from 17 rows on it wins at all of them (151,936 columns of 1,024:
+# 17 rows 63 / 57 (63 / 61), 64 77 / 68 (78 / 75), 65 89 / 74; of 4,096: 24 rows 259 / 236 (274 / 248), 64 274 / 252; of 5,120: 24 rows 297 / 289 (348 / 290); 100,352 of 1,536:
+# 40 rows 128 / 68; 32,768 of 1,024: 32 rows 48 / 16; the least, 131,072 of 4,096, 200 rows 300 / 303).  With fewer the kernels for few rows are as
+# fast or faster (4,096: 8 rows 219 / 223; 2,048: 115 / 115; 65,536 of 2,048, 8 rows 51 / 53 (56 / 70)) but for widths about 1,024 (151,936 columns: 1 row 55 /
+# 53 (55 / 55), 8 60 / 55 (61 / 58); 768 loses: 50,304 columns, 1 row 17 / 19).
+MANY_VOCABULARY = 32768
+MANY_VOCABULARY_ROWS = (17, 200)
+MANY_VOCABULARY_FEW_WIDTHS = (896, 1024)
+
+
+def many_vocabulary_wins(rows: int, columns: int, width: int) -> bool:
+    low, most = MANY_VOCABULARY_ROWS
+    narrow, wide = MANY_VOCABULARY_FEW_WIDTHS
+    return (columns >= MANY_VOCABULARY and 0 < rows <= most and (rows >= low or narrow <= width <= wide)
+            and bool(library().pl_gemm_many_applies(rows, columns, width, 3)))
+
+
 # The product that adds into the stream and hands the norm behind it forward, against the library's product and the norm kernel: a workgroup of the
 # smallest tile (64 rows by 128 columns) walks all of K, so the deeper K the more rows it takes until enough of them stand side by side (us, 1,024
 # columns: K 1,024, 65 rows 11.5 / 8.9, 8,192 38.6 / 31.7; K 2,048, 128 rows 11.9 / 12.5, 450 13.4 / 13.4, 1,024 15.7 / 14.6, 2,048 22.5 /
@@ -1540,7 +1558,9 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
     _need(x, "matrix product input", None, torch.bfloat16)
     _need(w, "weight", None, torch.bfloat16)
     if out_dtype == torch.float32:
-        # the projection onto the vocabulary: 32-bit out of the 32-bit sums, from either product
+        # the projection onto the vocabulary: 32-bit out of the 32-bit sums, whichever product it is
+        if many_vocabulary_wins(x.shape[0], w.shape[0], x.shape[1]):
+            return gemm_many(x, w, torch.float32, strips=strips)
         if wide_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
             return gemm_wide(x, _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16))
         if stream_wins(x.shape[0], w.shape[0], x.shape[1]):

@@ -2225,3 +2225,20 @@ def test_the_projection_of_many_rows_prepares_its_heads(nq, nkv, K, norm, turned
                 live = positions >= 0
                 assert torch.equal(bits(got[live][:, :nq * d]), bits(rows[live][:, :nq * d])), (n, handed is None, s is None)
                 assert torch.equal(bits(kv.k_pool), bits(want_kv.k_pool)) and torch.equal(bits(kv.v_pool), bits(want_kv.v_pool)), (n, handed is None, s is None)
+
+
+@pytest.mark.parametrize("N,K", [(32768, 64), (32784, 192), (40000, 1024)])
+def test_the_projection_onto_a_vocabulary_of_few_and_of_many_rows(N, K):
+    """Row counts on both sides of what the product of many rows takes of a vocabulary, columns that end inside a tile: 64-bit arithmetic within a factor of four of what
+    chains of K / 16 sums can be off, the same bits out of rows and out of strips, and of a row whatever rows stand beside it in that kernel."""
+    from paged_llm_rs_amd import kernels
+
+    w = (torch.randn(N, K, device=DEV) / K ** 0.5).bfloat16()
+    strips, x = kernels.weights_in_strips(w), torch.randn(201, K, device=DEV).bfloat16()
+    full = kernels.gemm_many(x, w, torch.float32)
+    assert rel(full, x.double() @ w.double().T) < 4 * math.sqrt(K / 16 + 1) * 2.0 ** -24
+    for n in (1, 8, 16, 17, 63, 64, 65, 200, 201):
+        taken = kernels.many_vocabulary_wins(n, N, K)
+        assert taken == (17 <= n <= 200 or (K == 1024 and n < 17))
+        if taken:
+            assert torch.equal(kernels.linear_bf16(x[:n], w, torch.float32, strips), full[:n]) and torch.equal(kernels.linear_bf16(x[:n], w, torch.float32), full[:n])
