@@ -2242,3 +2242,27 @@ def test_the_projection_onto_a_vocabulary_of_few_and_of_many_rows(N, K):
         assert taken == (17 <= n <= 200 or (K == 1024 and n < 17))
         if taken:
             assert torch.equal(kernels.linear_bf16(x[:n], w, torch.float32, strips), full[:n]) and torch.equal(kernels.linear_bf16(x[:n], w, torch.float32), full[:n])
+
+
+@pytest.mark.parametrize("lens,nq,nkv,d,splits", [([1100, 1030], 16, 8, 128, 1), ([1100, 1030], 16, 8, 128, 2), ([130] * 12, 16, 4, 64, 1),
+                                                  ([130] * 12, 12, 4, 128, 1), ([1030, 1025, 1100, 1030], 8, 8, 256, 1), ([300] * 3, 40, 8, 64, 2)])
+def test_the_order_of_the_token_tiles_changes_no_bit(lens, nq, nkv, d, splits):
+    """More token tiles than are taken at once, of up to eight heads an XCD, of more (a request's at a time) and of numbers that no XCD shares evenly:
+    every request comes out to the bit as it does alone, where the chip takes all tiles at once."""
+    from paged_llm_rs_amd import kernels
+
+    bs, stride = 16, (nq + 2 * nkv) * d
+    assert sum(-(-n // 128) for n in lens) * nq > 256 and max(-(-n // 128) for n in lens) * nq <= 256
+    bt, k_pool, v_pool, _, _ = build_paged(nkv, d, bs, [n + 40 for n in lens], torch.bfloat16, seed=5)
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(sum(lens), stride, generator=g).to(torch.bfloat16).to(DEV)
+    as_i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    starts = [sum(lens[:i]) for i in range(len(lens))]
+    together = torch.full((sum(lens), nq * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    kernels.paged_attention_prefill(q, stride, together, as_i32(starts), as_i32(lens), as_i32([n + 40 for n in lens]), max(lens), bt, bs, k_pool, v_pool,
+                                    nq, nkv, d, d ** -0.5, splits=splits)
+    for s, (at, n) in enumerate(zip(starts, lens)):
+        alone = torch.full((n, nq * d), 9.0, dtype=torch.bfloat16, device=DEV)
+        kernels.paged_attention_prefill(q[at:at + n].contiguous(), stride, alone, as_i32([0]), as_i32([n]), as_i32([n + 40]), n, bt[s:s + 1].contiguous(), bs,
+                                        k_pool, v_pool, nq, nkv, d, d ** -0.5, splits=splits)
+        assert torch.equal(together[at:at + n], alone), s
