@@ -805,18 +805,24 @@ def paged_attention_grouped(q: torch.Tensor, q_row_stride: int, out: torch.Tenso
     return out
 
 
+# What a tile of 64 keys costs a workgroup of 128 tokens in us: alone on its compute unit where few are at work, and with all of them at work; heads of
+# more than 128 go through registers, by half as many waves.
+PREFILL_TILE_US = {False: (1.04, 1.3), True: (3.7, 3.7)}
+
+
 def prefill_splits(requests: int, max_q_len: int, nq: int, d: int, max_ctx: int, rows: int | None = None,
                    short_limit: int = 0) -> int:
     """Into how many shares the keys of a token tile are cut.  A share more costs a trip of the
     unnormalised outputs through memory (rows * nq * d floats written and read) and one launch;
     it pays where few token tiles stand before a long context, as in a late portion of a long
-    prompt.  The shares that make the estimate below smallest are taken: a workgroup spends about
-    1.5 us on 64 keys, memory moves about 3 TB/s for this."""
+    prompt.  The shares that make the estimate below smallest are taken: a launch ends no sooner than its longest share of keys, nor than its shares
+    laid in turns on the compute units take on average (the last tokens of a prompt read all keys, the first ones few); memory moves about 3 TB/s for
+    the outputs.  ``max_ctx`` bounds the longest context, and may exceed it twofold up to 1,024 and by half beyond: where the longest portion alone could have
+    that bound, a whole prompt is meant.  (us, one share / two: 700 fresh tokens of 16 heads of 128 23 / 28, 3,000 66 / 92, 512 behind 3,500 79 / 54 and in four 43.)"""
     if max_ctx <= 0:
         return 1
     tile = library().pl_paged_attention_prefill_tile(max_q_len, d)
     base = max(1, -(-max_q_len // tile) * nq * requests)
-    key_tiles = -(-max_ctx // 64)
     rows = rows if rows is not None else requests * max_q_len
     # Where the rows cannot fill that many token tiles the kernel deals its workgroups to the tiles there can
     # be; most of those are empty too when the step is one portion beside single tokens, so the portion's
@@ -824,14 +830,19 @@ def prefill_splits(requests: int, max_q_len: int, nq: int, d: int, max_ctx: int,
     served = min(requests, rows // short_limit) if short_limit > 0 else requests
     if (rows + served * (tile - 1)) // tile < -(-max_q_len // tile) * requests:
         base = (rows // tile + 1) * nq
+    fresh = 2 * max_q_len > max_ctx if max_ctx <= 1024 else 3 * max_q_len > 2 * max_ctx
+    key_tiles = -(-(max_q_len if fresh else max_ctx) // 64)
+    first = -(-min(tile, max_q_len) // 64) if fresh else max(1, -(-(max_ctx - max_q_len + min(tile, max_q_len)) // 64))
+    mean = (first + key_tiles) / 2
+    alone, busy = PREFILL_TILE_US[d > 128]
     best, best_cost = 1, None
     for s in (1, 2, 3, 4, 6, 8, 12, 16):
         if s > 1 and key_tiles // s < 4:
             break
         turns = -(-base * s // compute_units())
-        cost = turns * -(-key_tiles // s) * 1.5
+        cost = max(-(-key_tiles // s) * alone, turns * mean / s * busy)
         if s > 1:
-            cost += 3.0 + rows * nq * d * 8.0 * s / 3e6
+            cost += 5.0 + rows * nq * d * 8.0 * s / 3e6
         if best_cost is None or cost < best_cost:
             best, best_cost = s, cost
     return best

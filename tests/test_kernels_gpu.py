@@ -2266,3 +2266,15 @@ def test_the_order_of_the_token_tiles_changes_no_bit(lens, nq, nkv, d, splits):
         kernels.paged_attention_prefill(q[at:at + n].contiguous(), stride, alone, as_i32([0]), as_i32([n]), as_i32([n + 40]), n, bt[s:s + 1].contiguous(), bs,
                                         k_pool, v_pool, nq, nkv, d, d ** -0.5, splits=splits)
         assert torch.equal(together[at:at + n], alone), s
+
+
+def test_the_shares_of_a_prompts_keys():
+    """One share where it measured fastest and several where they did: fresh prompts, whose bound is their own, and portions behind long contexts."""
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.engine.batch import near_context
+
+    pick = lambda q, behind, nq, d: kernels.prefill_splits(1, q, nq, d, near_context(q + behind), q)
+    for q in (37, 300, 700, 1100, 2048, 3000, 8192):
+        assert pick(q, 0, 16, 128) == pick(q, 0, 32, 128) == 1, q
+    assert pick(512, 3500, 16, 128) == 4 and pick(512, 3500, 32, 128) == 2 and pick(1024, 7000, 16, 128) == 2 and pick(1024, 7000, 32, 128) == 1
+    assert pick(1500, 0, 16, 256) == 2 and pick(512, 1500, 16, 256) == 4
