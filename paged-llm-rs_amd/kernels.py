@@ -1036,7 +1036,7 @@ def weights_in_strips(w: torch.Tensor) -> torch.Tensor | None:
     rows, a strip a run of K/32 tiles of 1 KB, a tile stored as [4 groups of 8 elements][16 rows][8 elements], so
     that a wave's stretch of K of a strip is one contiguous stretch of memory, which the memory serves faster
     than 64 bytes from each of 16 rows that lie K elements apart.  The result has the shape of ``w`` and is
-    read by ``gemm_skinny(..., strips=...)`` only.  None where the layout is not defined: rows that are no
+    read by ``gemm_skinny``, ``gemm_wide``, ``gemm_many`` and the grouped product of experts.  None where the layout is not defined: rows that are no
     multiple of 16, a K that is no multiple of 32."""
     if w.dim() != 2 or w.dtype != torch.bfloat16 or not w.is_cuda:
         return None
@@ -1183,7 +1183,8 @@ def gemm_tiled_applies(rows: int, columns: int, width: int, swiglu: bool = False
 # 0.7 PFLOP/s, below the library's best; what it saves is the trip of gate and up through memory and a
 # launch.  That wins for the gated feed-forward of a narrow model in portions of a prompt (512 rows of
 # width 1,024: 12.6 us against 20 for product plus activation; 2,048 rows: 38 against 39, no better inside
-# a step), and loses from a width of 4,096 on, as do the plain and the adding product at every size measured.
+# a step), and loses from a width of 4,096 on, as do the plain and the adding product at every size measured.  (``gemm_many`` takes the SiLU-gated
+# ones of widths that are multiples of 64 before they come here; what is left are other activations and widths.)
 TILED_SWIGLU_MAX_ROWS = 1024
 TILED_SWIGLU_MAX_WIDTH = 2048
 
@@ -1373,6 +1374,7 @@ def gemm_many_heads(x: torch.Tensor | None, w: torch.Tensor, batch, kv, nq: int,
     return out
 
 
+# (Reached with up to 16 rows, and with more only where the width is no multiple of 64, which the kernel for many rows asks for: ``many_vocabulary_wins`` goes first.)
 # Where the product over strips and very many columns beats the others, timed at 1 to 32 rows over 131,072 to 524,288 columns and widths from 2,048
 # to 8,192.  The library's times follow turns of 256 tiles, of 256 columns for up to 16 rows and of 128 for more: where the
 # last turn is partly empty it loses what is missing there, and this kernel, whose workgroups are not tied to
@@ -1419,8 +1421,8 @@ STREAM_ROWS = 64
 # memory, at 8 to 64 rows).  The library cuts a deep product over few columns badly (5,120 x 25,600 at 64
 # rows: 158 us against 67 here), and from 17 rows on it is slower over very many columns of a narrow stream
 # (the vocabulary of 151,936 over a width of 1,024, 32-bit out, 17 to 64 rows: 74 to 84 us against 62 to
-# 77; over widths of 4,096 and 5,120 the two are within a tenth of each other, either way, and the
-# library keeps them).  A wide product of moderate depth (51,200 x 5,120) stays the
+# 77; over widths of 4,096 and 5,120 the two are within a tenth of each other, either way.  Vocabularies of widths that are multiples of 64
+# are ``many_vocabulary_wins``'s before they come here).  A wide product of moderate depth (51,200 x 5,120) stays the
 # library's: its columns give too few workgroups for an even share a compute unit, and cutting K there
 # costs more in partial results than it gains.
 STREAM_DEEP = 1.5            # K / N from which the product counts as deep, with more than 16 rows
