@@ -1275,20 +1275,19 @@ def many_store_wins(rows: int, columns: int, width: int) -> bool:
 
 
 # The projection onto a vocabulary, 32-bit out: a workgroup takes 128 columns and all of up to 64 rows, so the weights are read once and the rows out of L2.  Timed at 1 to
-# 200 rows over 12 vocabularies (us, before / this one, out of strips; in rows in brackets): from 17 rows on it wins at all of them (151,936 columns of 1,024:
-# 17 rows 63 / 57 (63 / 61), 64 77 / 68 (78 / 75), 65 89 / 74; of 4,096: 24 rows 259 / 236 (274 / 248), 64 274 / 252; of 5,120: 24 rows 297 / 289 (348 / 290); 100,352 of 1,536:
-# 40 rows 128 / 68; 32,768 of 1,024: 32 rows 48 / 16; the least, 131,072 of 4,096, 200 rows 300 / 303).  With fewer the kernels for few rows are as
-# fast or faster (4,096: 8 rows 219 / 223; 2,048: 115 / 115; 65,536 of 2,048, 8 rows 51 / 53 (56 / 70)) but for widths about 1,024 (151,936 columns: 1 row 55 /
-# 53 (55 / 55), 8 60 / 55 (61 / 58); 768 loses: 50,304 columns, 1 row 17 / 19).
+# 256 rows over 12 vocabularies, out of strips and in rows (us, before / this one, out of strips).  From 17 rows on, where the kernels for few rows take a second tile of them, it
+# wins at all of them (151,936 columns of 1,024: 17 rows 68 / 61, 64 82 / 71, 128 96 / 90; of 4,096: 24 rows 251 / 235, 64 276 / 250, 128 296 / 281; 200,064 of 3,072: 64 rows
+# 293 / 264; 100,352 of 1,536: 48 rows 137 / 75; 32,768 of 1,024: 32 rows 48 / 16), in rows a little less and up to 64 of them (151,936 of 1,024: 17 rows 67 / 66; 65,536 of 2,048: 64
+# 122 / 79, 65 76 / 79, 128 83 / 86; 200,064 of 3,072: 128 rows 305 / 315).  Beyond 128 rows its third tile of them is paid by the columns, and it wins at some vocabularies and loses at
+# others (160 rows: 65,536 of 2,048 85 / 76, 151,936 of 4,096 319 / 337, 200,064 of 3,072 329 / 351).  With fewer than 17 neither the width nor the size says which is the
+# faster, and it is a matter of a few per cent (8 rows: 151,936 columns of 1,024 60 / 55, of 4,096 219 / 223; 32,768 of 4,096 55 / 50; 65,536 of 2,048 51 / 53; 50,304 of 768 19 / 19).
 MANY_VOCABULARY = 32768
-MANY_VOCABULARY_ROWS = (17, 200)
-MANY_VOCABULARY_FEW_WIDTHS = (896, 1024)
+MANY_VOCABULARY_FROM_ROWS = 17
+MANY_VOCABULARY_ROWS = {True: 128, False: 64}         # at most, out of strips and in rows
 
 
-def many_vocabulary_wins(rows: int, columns: int, width: int) -> bool:
-    low, most = MANY_VOCABULARY_ROWS
-    narrow, wide = MANY_VOCABULARY_FEW_WIDTHS
-    return (columns >= MANY_VOCABULARY and 0 < rows <= most and (rows >= low or narrow <= width <= wide)
+def many_vocabulary_wins(rows: int, columns: int, width: int, strips: bool) -> bool:
+    return (columns >= MANY_VOCABULARY and MANY_VOCABULARY_FROM_ROWS <= rows <= MANY_VOCABULARY_ROWS[strips]
             and bool(library().pl_gemm_many_applies(rows, columns, width, 3)))
 
 
@@ -1585,7 +1584,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
     _need(w, "weight", None, torch.bfloat16)
     if out_dtype == torch.float32:
         # the projection onto the vocabulary: 32-bit out of the 32-bit sums, whichever product it is
-        if many_vocabulary_wins(x.shape[0], w.shape[0], x.shape[1]):
+        if many_vocabulary_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
             return gemm_many(x, w, torch.float32, strips=strips)
         if wide_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
             return gemm_wide(x, _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16))
@@ -1593,7 +1592,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
             return gemm_stream(x, w, torch.float32)
         if skinny_applies(x) and x.shape[1] <= (SKINNY_F32_FEW_K if x.shape[0] <= 16 else SKINNY_SHALLOW_K):
             return gemm_skinny(x, w, torch.float32, strips=strips)
-        if many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
+        if w.shape[0] < MANY_VOCABULARY and many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
             return gemm_many(x, w, torch.float32, strips=strips)
         if x.shape[1] % 8 == 0:
             return torch.mm(x, w.t(), out_dtype=torch.float32)

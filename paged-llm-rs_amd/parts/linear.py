@@ -116,7 +116,7 @@ class Linear:
                 return kernels.gemm_plain_gated(x, self.weight, activation)
             return kernels.gemm_plain(x, self.weight, out_dtype=torch.float32)
         if (out_dtype == torch.float32 and add_into is None and not swiglu
-                and kernels.many_vocabulary_wins(x.shape[0], self.out_features, self.in_features)):
+                and kernels.many_vocabulary_wins(x.shape[0], self.out_features, self.in_features, self.strips is not None)):
             return kernels.gemm_many(x, self.weight, torch.float32, strips=self.strips)
         if kernels.skinny_applies(x, self.weight, self.strips is not None):
             if add_into is not None and not swiglu:

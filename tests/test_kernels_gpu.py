@@ -2237,11 +2237,12 @@ def test_the_projection_onto_a_vocabulary_of_few_and_of_many_rows(N, K):
     strips, x = kernels.weights_in_strips(w), torch.randn(201, K, device=DEV).bfloat16()
     full = kernels.gemm_many(x, w, torch.float32)
     assert rel(full, x.double() @ w.double().T) < 4 * math.sqrt(K / 16 + 1) * 2.0 ** -24
-    for n in (1, 8, 16, 17, 63, 64, 65, 200, 201):
-        taken = kernels.many_vocabulary_wins(n, N, K)
-        assert taken == (17 <= n <= 200 or (K == 1024 and n < 17))
-        if taken:
-            assert torch.equal(kernels.linear_bf16(x[:n], w, torch.float32, strips), full[:n]) and torch.equal(kernels.linear_bf16(x[:n], w, torch.float32), full[:n])
+    for n in (1, 8, 16, 17, 63, 64, 65, 128, 129, 200, 201):
+        for layout in (strips, None):
+            taken = kernels.many_vocabulary_wins(n, N, K, layout is not None)
+            assert taken == (17 <= n <= (64 if layout is None else 128))
+            if taken:
+                assert torch.equal(kernels.linear_bf16(x[:n], w, torch.float32, layout), full[:n])
 
 
 @pytest.mark.parametrize("lens,nq,nkv,d,splits", [([1100, 1030], 16, 8, 128, 1), ([1100, 1030], 16, 8, 128, 2), ([130] * 12, 16, 4, 64, 1),

@@ -31,3 +31,13 @@ def test_the_shares_of_several_prompts_keys(requests, nq, d, good):
     assert kernels.prefill_splits(len(requests), rows, nq, d, near, rows, 0) in good
     # (never a share of less than four tiles of keys, as many requests as there may be)
     assert kernels.prefill_splits(len(requests), rows, nq, d, near, rows, 0) * 4 * 64 <= max(near, 256)
+
+
+@pytest.mark.parametrize("columns", [32768, 50304, 151936, 262144])
+def test_a_vocabulary_of_few_rows_goes_by_no_width(columns):
+    """The product of many rows takes a vocabulary by the rows and by how the weights lie, whatever the width."""
+    for width in (768, 896, 960, 1024, 1088, 1536, 2048, 4096, 5120):
+        if columns * width < 2 ** 31:
+            assert [kernels.many_vocabulary_wins(n, columns, width, True) for n in (1, 8, 16, 17, 64, 128, 129, 200)] == [False] * 3 + [True] * 3 + [False] * 2
+            assert [kernels.many_vocabulary_wins(n, columns, width, False) for n in (1, 16, 17, 64, 65, 128)] == [False, False, True, True, False, False]
+    assert not kernels.many_vocabulary_wins(32, columns, 1000, True) and not kernels.many_vocabulary_wins(32, 32752, 1024, True)
