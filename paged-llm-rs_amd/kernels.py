@@ -1254,24 +1254,35 @@ def many_swiglu_wins(rows: int, columns: int, width: int) -> bool:
     return rows <= MANY_WIDE_ROWS or (rows <= MANY_WIDE_MOST_ROWS and tiles <= MANY_WIDE_TURNS * 256 * -(-tiles // 256))
 
 
-# The plain product, bfloat16 or 32-bit: up to a width of 1,024, as long as the rows and columns of the result are few (us, library / this one:
-# 4,096 columns: 65 rows 9.0 / 7.1, 450 11.1 / 8.1, 1,024 13.3 / 12.3, 1,536 16.8 / 15.7, 2,560 23.8 / 26.3; 1,024 columns: 65 rows 8.4 / 6.9,
-# 4,096 13.4 / 12.4, 8,192 20.5 / 20.7); and up to 3,072 where its smallest tiles (64 by 128) are one a compute unit, or a little less (1,024 columns: K 2,048,
-# 1,024 rows, 128 tiles, 11.2 / 11.8, 1,152 13.5 / 11.8, 2,048 15.6 / 12.6; K 3,072, 1,152 rows 17.6 / 16.8, 2,048 20.9 / 18.4; 2,048 columns of 2,048:
-# 640 rows 13.6 / 11.6, 1,024 15.6 / 12.8).
+# The plain product, bfloat16 or 32-bit, timed with weights that come from memory (us, library / this one out of strips / in rows).  Up to a width of 1,024, as long as the rows and
+# columns of the result are few: this one's tiles pass LDS on their way out, and in rows its weights do too (4,096 columns: 65 rows 11.6 / 8.3 / 9.3, 448 12.9 / 9.1 / 9.9, 1,024 14.9 / 13.0 / 14.2,
+# 1,408 20.9 / 16.1 / 17.9, 2,048 21.4 / 21.4 / 23.3; 1,024 columns: 65 rows 10.8 / 8.1 / 9.1, 4,096 15.0 / 12.9 / 14.5, 5,120 16.4 / 15.2 / 17.0; 3,072 of 768: 1,408 rows 13.5 / 13.4 / 14.4).  Beyond,
+# where its smallest tiles (64 by 128) are one a compute unit or less, a workgroup walks all of K alone, and what it wins by is the library's turns: up to a width of 1,536 that is from
+# a little more than half of the compute units on (1,024 columns of 1,536: 1,024 rows, 128 tiles, 10.6 / 12.0 / 12.9, 1,216 15.8 / 12.0 / 12.8; of 1,152: 1,089 13.6 / 9.6 / 10.0), as for
+# 5,120 columns and more of up to 3,072 (5,120 of 2,048: 256 rows, 160 tiles, 24.0 / 15.8 / 16.7; 8,192 of 3,072: 192 28.5 / 23.9 / 25.7), and otherwise from four fifths on (2,048 columns
+# of 2,048: 704 rows, 176 tiles, 14.1 / 15.1 / 15.7, 832 16.2 / 15.2 / 15.9; 1,024 of 3,072: 1,216, 152, 19.9 / 20.8 / 22.2, 1,792 22.0 / 20.7 / 22.4; 4,096 of 2,560: 384, 192, 18.4 / 19.5 / 21.8,
+# 448 22.0 / 19.6 / 21.7).
 MANY_STORE_WIDTH = 1024
-MANY_STORE_RESULTS = 6.25e6
-MANY_STORE_WIDE = 3072
-MANY_STORE_WIDE_TILES = (0.56, 1.0)     # of the compute units
+MANY_STORE_RESULTS = {True: 6.25e6, False: 4.2e6}         # out of strips, in rows
+MANY_STORE_WIDE = {True: 3072, False: 2560}
+MANY_HALF_WIDTH = 1536
+MANY_HALF_COLUMNS = 5120
+MANY_HALF = 0.53         # of the compute units
+MANY_MOST = 0.8
 
 
-def many_store_wins(rows: int, columns: int, width: int) -> bool:
-    if rows <= SKINNY_ROWS or width > MANY_STORE_WIDE or not library().pl_gemm_many_applies(rows, columns, width, 0):
+def many_store_wins(rows: int, columns: int, width: int, strips: bool) -> bool:
+    if rows <= SKINNY_ROWS or width > MANY_STORE_WIDE[strips] or not library().pl_gemm_many_applies(rows, columns, width, 0):
         return False
     if width <= MANY_STORE_WIDTH:
-        return rows * columns <= MANY_STORE_RESULTS
-    low, high = MANY_STORE_WIDE_TILES
-    return low * compute_units() <= -(-rows // 64) * -(-columns // 128) <= high * compute_units()
+        return rows * columns <= MANY_STORE_RESULTS[strips]
+    low = MANY_HALF if width <= MANY_HALF_WIDTH or columns >= MANY_HALF_COLUMNS else MANY_MOST
+    return low * compute_units() <= many_tiles(rows, columns) <= compute_units()
+
+
+def many_tiles(rows: int, columns: int) -> int:
+    """The smallest tiles of a product of many rows."""
+    return -(-rows // 64) * -(-columns // 128)
 
 
 # The projection onto a vocabulary, 32-bit out: a workgroup takes 128 columns and all of up to 64 rows, so the weights are read once and the rows out of L2.  Timed at 1 to
@@ -1592,7 +1603,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
             return gemm_stream(x, w, torch.float32)
         if skinny_applies(x) and x.shape[1] <= (SKINNY_F32_FEW_K if x.shape[0] <= 16 else SKINNY_SHALLOW_K):
             return gemm_skinny(x, w, torch.float32, strips=strips)
-        if w.shape[0] < MANY_VOCABULARY and many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
+        if w.shape[0] < MANY_VOCABULARY and many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
             return gemm_many(x, w, torch.float32, strips=strips)
         if x.shape[1] % 8 == 0:
             return torch.mm(x, w.t(), out_dtype=torch.float32)
@@ -1601,7 +1612,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
         return gemm_skinny(x, w, out_dtype, strips=strips)
     if stream_wins(x.shape[0], w.shape[0], x.shape[1]):
         return gemm_stream(x, w, out_dtype)
-    if many_store_wins(x.shape[0], w.shape[0], x.shape[1]):
+    if many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
         return gemm_many(x, w, strips=strips)
     splits = library_splits(x.shape[0], w.shape[0], x.shape[1])
     if splits > 1 and turned is not None:

@@ -77,7 +77,8 @@ class Linear:
                 return None
             if x.handed is not None and kernels.many_takes(x.handed, x.num_rows, self.out_features, self.in_features):
                 handed = x.handed
-        if handed is None and not kernels.many_store_wins(x.num_rows if isinstance(x, PendingNorm) else x.shape[0], self.out_features, self.in_features):
+        if handed is None and not kernels.many_store_wins(x.num_rows if isinstance(x, PendingNorm) else x.shape[0], self.out_features, self.in_features,
+                                                          self.strips is not None):
             return None
         if handed is None and isinstance(x, PendingNorm):
             x = x.materialize()

@@ -41,3 +41,19 @@ def test_a_vocabulary_of_few_rows_goes_by_no_width(columns):
             assert [kernels.many_vocabulary_wins(n, columns, width, True) for n in (1, 8, 16, 17, 64, 128, 129, 200)] == [False] * 3 + [True] * 3 + [False] * 2
             assert [kernels.many_vocabulary_wins(n, columns, width, False) for n in (1, 16, 17, 64, 65, 128)] == [False, False, True, True, False, False]
     assert not kernels.many_vocabulary_wins(32, columns, 1000, True) and not kernels.many_vocabulary_wins(32, 32752, 1024, True)
+
+
+# (columns, width): {rows: whether the product of many rows measured at most as long as the library's, out of strips and in rows}, a twenty-fifth either way let pass
+PLAIN = {
+    (4096, 1024): {65: "yy", 576: "yy", 1024: "yy", 2048: "nn"}, (1024, 1024): {65: "yy", 4096: "yy", 5120: "yn", 8192: "nn"}, (3072, 768): {1024: "yy", 1408: "yn"},
+    (1024, 1536): {832: "nn", 1024: "nn", 1216: "yy", 1984: "yy"}, (2048, 1536): {512: "nn", 576: "yy", 1024: "yy"}, (1024, 1152): {321: "nn", 1089: "yy"},
+    (2048, 2048): {576: "nn", 704: "nn", 832: "yy", 1024: "yy"}, (3072, 2048): {384: "nn", 576: "yy"}, (4096, 2048): {384: "nn", 448: "yy"},
+    (1024, 3072): {1216: "nn", 1408: "nn", 1792: "yn"}, (3072, 3072): {448: "nn", 512: "nn", 576: "yn"}, (4096, 2560): {384: "nn", 448: "yy"}, (4096, 3072): {384: "nn", 512: "yn"},
+    (5120, 2048): {65: "nn", 256: "yy", 384: "yy"}, (8192, 3072): {65: "nn", 192: "yn"}, (6144, 3072): {256: "yn"}, (1024, 4096): {1024: "nn", 2048: "nn"},
+}
+
+
+@pytest.mark.parametrize("columns,width", list(PLAIN))
+def test_the_plain_product_of_many_rows_is_taken_where_it_measured_faster(columns, width):
+    for rows, wanted in PLAIN[columns, width].items():
+        assert [kernels.many_store_wins(rows, columns, width, strips) for strips in (True, False)] == [w == "y" for w in wanted], rows
