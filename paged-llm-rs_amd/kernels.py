@@ -1231,27 +1231,38 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, swiglu: bool = False, add_into:
 
 
 # Where the product of many rows with the gated activation inside beats the others (the library's product and the activation kernel, or
-# ``gemm_tiled``), timed at 65 to 8,192 rows of 13 pairs of widths.  Up to a width of 2,048 it does at every size until the operations are what
-# counts, which the library's tiles of 256 x 256 do at up to 1.4 PFLOP/s and this one's at 1.0 to 1.2 (us, before / this one; 1,024 wide,
-# 3,072 columns: 65 rows 14 / 7, 2,048 36 / 26, 8,192 104 / 102; 8,192 columns: 2,560 rows 115 / 89, 4,096 140 / 151; 2,048 wide, 6,144 columns:
-# 1,024 rows 69 / 45, 1,150 58 / 60).  Beyond, it wins by what the library's turns of 256 such tiles leave empty, and up to 128 rows (12,288 columns of
-# 4,096: 65 rows 59 / 51, 256 83 / 72, turns 0.38 full, 576 124 / 114, 0.56 full; 14,336 of 4,096: 512 rows 105 / 122, 0.88 full; 25,600 of
-# 5,120: 128 rows 128 / 113, 256 166 / 168, 0.78 full).
+# ``gemm_tiled``), timed at 65 to 8,192 rows of 16 pairs of widths with weights that come from memory (us, before / this one out of strips / in rows).  Up to a width of 2,048 it does at
+# every size until the operations are what counts, which the library's tiles of 256 x 256 do at up to 1.4 PFLOP/s and this one's at 1.0 to 1.2, in rows 0.9 to 1.0 (1,024 wide, 3,072
+# columns: 65 rows 16.7 / 9.0 / 9.7, 2,048 38 / 28 / 30, 8,192 112 / 106 / 114; 8,192 columns: 1,536 rows 67 / 58 / 63, 3,072 116 / 111 / 121, 4,096 154 / 159; 2,048 wide, 6,144
+# columns: 1,024 rows 71 / 47 / 51; 4,096 columns: 1,536 rows 53 / 52 / 59).  In rows it still wins there while its largest tiles are one turn of the compute units (6,144 columns of
+# 2,048: 1,024 rows).  Beyond, it wins by what the library's turns of 256 such tiles leave empty, and up to 128 rows (12,288 columns of 4,096: 65 rows 58 / 48 / 52, 256 74 / 72 / 71,
+# turns 0.38 full, 576 125 / 117 / 127, 0.56 full; 14,336 of 4,096: 512 rows 109 / 120 / 137, 0.88 full; 25,600 of 5,120: 128 rows 126 / 111 / 117, 256 166 / 167 / 179, 0.78 full; 9,728 of
+# 2,560: 160 rows 45 / 39 / 45, 448 62 / 54 / 60).  But a second tile of 128 rows that is less than half full costs a wide one as much as a full one (12,288 of 4,096: 160 rows
+# 62 / 68 / 65, 14,336 of 4,096 69 / 71 / 74), and wide weights in rows lose what more rows would gain.
 MANY_STRIPE = 64       # columns of the stream whose squares are one number of a norm that the product hands forward
-MANY_WORK = ((1024, 27e9), (2048, 13e9))      # widths up to, and rows x columns x width up to
+MANY_WORK = {True: ((1024, 27e9), (2048, 13e9)), False: ((1024, 13e9), (2048, 10.5e9))}      # out of strips, in rows: widths up to, and rows x columns x width up to
+MANY_WORK_TURN = 13e9        # in rows, in one turn
 MANY_WIDE_ROWS = 128
 MANY_WIDE_MOST_ROWS = 704
 MANY_WIDE_TURNS = 0.6
+MANY_DEEP = 2560             # wider ones: none of 129 to MANY_DEEP_ROWS rows and, in rows, none of more than MANY_DEEP_MOST_ROWS
+MANY_DEEP_ROWS = 192
+MANY_DEEP_MOST_ROWS = 256
 
 
-def many_swiglu_wins(rows: int, columns: int, width: int) -> bool:
+def many_swiglu_wins(rows: int, columns: int, width: int, strips: bool) -> bool:
     if rows <= SKINNY_ROWS or not library().pl_gemm_many_applies(rows, columns, width, 1):
         return False
-    for most, work in MANY_WORK:
+    work = rows * columns * width
+    for most, limit in MANY_WORK[strips]:
         if width <= most:
-            return rows * columns * width <= work
+            return work <= limit or (not strips and work <= MANY_WORK_TURN and -(-rows // 128) * -(-columns // 192) <= compute_units())
+    if rows <= MANY_WIDE_ROWS:
+        return True
+    if width > MANY_DEEP and (rows <= MANY_DEEP_ROWS or (not strips and rows > MANY_DEEP_MOST_ROWS)):
+        return False
     tiles = -(-rows // 256) * -(-2 * columns // 256)
-    return rows <= MANY_WIDE_ROWS or (rows <= MANY_WIDE_MOST_ROWS and tiles <= MANY_WIDE_TURNS * 256 * -(-tiles // 256))
+    return rows <= MANY_WIDE_MOST_ROWS and tiles <= MANY_WIDE_TURNS * 256 * -(-tiles // 256)
 
 
 # The plain product, bfloat16 or 32-bit, timed with weights that come from memory (us, library / this one out of strips / in rows).  Up to a width of 1,024, as long as the rows and

@@ -142,7 +142,7 @@ class Linear:
                 return None
         if swiglu:
             if (kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
-                    and kernels.many_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features)):
+                    and kernels.many_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features, self.strips is not None)):
                 return kernels.gemm_many(x, self.weight, swiglu=True, strips=self.strips)
             if kernels.tiled_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features):
                 return kernels.gemm_tiled(x, self.weight, swiglu=True, activation=activation)

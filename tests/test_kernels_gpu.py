@@ -2061,7 +2061,7 @@ def test_the_gated_product_of_many_rows(N, K):
     strips = kernels.weights_in_strips(w)
     for n in (65, 96, 129, 300, 520, 700, 1030, 2050):
         x = torch.randn(n, K, device=DEV).bfloat16()
-        assert kernels.many_swiglu_wins(n, N, K)
+        assert kernels.many_swiglu_wins(n, N, K, True) and kernels.many_swiglu_wins(n, N, K, False)
         both = x.double() @ w.double().T
         want = torch.nn.functional.silu(both[:, :N]) * both[:, N:]
         got = kernels.gemm_many(x, w, swiglu=True, strips=strips)

@@ -57,3 +57,17 @@ PLAIN = {
 def test_the_plain_product_of_many_rows_is_taken_where_it_measured_faster(columns, width):
     for rows, wanted in PLAIN[columns, width].items():
         assert [kernels.many_store_wins(rows, columns, width, strips) for strips in (True, False)] == [w == "y" for w in wanted], rows
+
+
+GATED = {
+    (3072, 1024): {65: "yy", 2048: "yy", 4096: "yy", 8192: "yn"}, (8192, 1024): {1024: "yy", 1536: "yy", 2048: "yn", 3072: "yn", 4096: "nn"},
+    (4096, 2048): {65: "yy", 1024: "yy", 1536: "yn", 2048: "nn"}, (6144, 2048): {200: "yy", 1024: "yy"}, (9728, 2560): {128: "yy", 160: "yy", 192: "yy", 384: "yy"},
+    (12288, 4096): {65: "yy", 128: "yy", 160: "nn", 192: "nn", 256: "yy", 320: "nn", 576: "yn", 704: "yn"}, (14336, 4096): {128: "yy", 160: "nn", 256: "yy", 512: "nn"},
+    (25600, 5120): {128: "yy", 160: "nn", 256: "nn", 512: "nn"}, (11008, 4096): {160: "nn", 256: "yy", 640: "yn"},
+}
+
+
+@pytest.mark.parametrize("columns,width", list(GATED))
+def test_the_gated_product_of_many_rows_is_taken_where_it_measured_faster(columns, width):
+    for rows, wanted in GATED[columns, width].items():
+        assert [kernels.many_swiglu_wins(rows, columns, width, strips) for strips in (True, False)] == [w == "y" for w in wanted], rows
