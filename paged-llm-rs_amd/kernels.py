@@ -1313,25 +1313,47 @@ def many_vocabulary_wins(rows: int, columns: int, width: int, strips: bool) -> b
             and bool(library().pl_gemm_many_applies(rows, columns, width, 3)))
 
 
-# The product that adds into the stream and hands the norm behind it forward, against the library's product and the norm kernel: a workgroup of the
-# smallest tile (64 rows by 128 columns) walks all of K, so the deeper K the more rows it takes until enough of them stand side by side (us, 1,024
-# columns: K 1,024, 65 rows 11.5 / 8.9, 8,192 38.6 / 31.7; K 2,048, 128 rows 11.9 / 12.5, 450 13.4 / 13.4, 1,024 15.7 / 14.6, 2,048 22.5 /
-# 16.7; K 3,072, 450 rows 16.6 / 17.6, 1,024 19.8 / 18.9, 2,048 26.6 / 21.1; K 4,096, 1,300 rows 27.0 / 22.8; 2,048 columns of 2,048: 4,096 rows 50.6 /
-# 45.2, 6,144 67.3 / 69.8).  The product behind the norm pays 0.6 for the sums.
-MANY_ADD_WIDTH = 4096
-MANY_ADD_ROWS = 0.42          # rows from which, for every k past 1,024
+# The product that adds into the stream and hands the norm behind it forward.  Alone it is slower than the library's product, whose result the norm kernel adds (the stream makes a
+# trip more: 1,024 columns of 2,048, 2,048 rows with the norm 22.4 / 24.8 us out of strips, 27.2 in rows); what it saves is that kernel, where the product behind the norm takes what
+# it left.  Timed as the three of them, weights from memory (us, library and norm kernel, then the product behind the norm by its own rule / this way): it wins from the first row on
+# up to a width of 1,024 (1,024 columns, then 2,048 gated: 65 rows 19.9 / 19.2, 4,096 62.5 / 60.9) and beyond from a little more than half a smallest tile a compute unit on, since a
+# workgroup walks all of K alone (1,024 columns of 2,048, then 3,072 gated: 704 rows 31.9 / 33.2, 1,024, 128 tiles, 35.8 / 36.6, 1,088, 136, 38.5 / 36.7, 2,048 50.0 / 47.4; of 3,072, then
+# 4,096: 1,024 35.4 / 37.4, 1,536 43.8 / 41.8; 2,048 columns of 2,048, then 6,144 gated: 448 45.7 / 47.0, 576 52.7 / 51.8; of 4,096, then 4,096: 576 53.7 / 49.3), until the results are many
+# (8,192 x 2,048 of 2,048, then 6,144 gated 442 / 463).  In rows it ends at a width of 2,048 (1,024 of 3,072, then 4,096: 1,024 rows 36.1 / 39.8, 3,072 63 / 73).
+MANY_ADD_WIDTH = {True: 4096, False: 2048}         # out of strips, in rows
+MANY_ADD_ALONE_WIDTH = 1024
 MANY_ADD_RESULTS = 8.4e6
 
 
-def many_add_wins(rows: int, columns: int, width: int) -> bool:
-    return (rows > SKINNY_ROWS and columns <= FUSED_NORM_MAX_WIDTH and columns % (4 * MANY_STRIPE) == 0 and width <= MANY_ADD_WIDTH
-            and rows >= MANY_ADD_ROWS * (width - 1024) and rows * columns <= MANY_ADD_RESULTS
+def many_add_wins(rows: int, columns: int, width: int, strips: bool) -> bool:
+    """Of a norm that the product behind it takes (``many_takes_wins``)."""
+    return (rows > SKINNY_ROWS and columns <= FUSED_NORM_MAX_WIDTH and columns % (4 * MANY_STRIPE) == 0 and width <= MANY_ADD_WIDTH[strips]
+            and (width <= MANY_ADD_ALONE_WIDTH or many_tiles(rows, columns) >= MANY_HALF * compute_units()) and rows * columns <= MANY_ADD_RESULTS
             and bool(library().pl_gemm_many_applies(rows, columns, width, 2)))
 
 
+# Where the product behind a norm of many rows takes it as an earlier product left it (which then is this kernel's as well) and the two ways above are as fast or faster: the norm kernel's
+# time grows with the rows alone, what the library's large tiles are ahead by with the columns too (us as above; plain, 1,024 wide, 4,096 columns: 3,072 rows 47.0 / 47.1, 4,096
+# 55 / 62; 2,048 wide: 3,072 rows 89 / 89, 4,096 105 / 118).  Where it prepares its heads the pass behind it is saved as well (1,024 wide, 4,096 columns: 4,096 rows 84 / 78, 8,192
+# 160 / 151; 2,048 wide: 3,072 rows 123 / 116, 4,096 155 / 158).  Gated: 6,144 columns of 2,048, 4,096 rows 239 / 233, 8,192 442 / 463.  In rows a gated
+# one is asked for by its own rule, and others end sooner (1,024 wide, 4,096 columns: 2,048 rows 37.9 / 37.3, 3,072 48 / 55, with heads 70 / 75).
+MANY_TAKES_RESULTS = {True: 13e6, False: 8.4e6}
+MANY_TAKES_HEADS_WIDTH = 1024
+MANY_TAKES_GATED = 26e6
+
+
+def many_takes_wins(rows: int, columns: int, width: int, swiglu: bool, strips: bool, heads: bool = False) -> bool:
+    """Whether the product behind the norm of a stream of ``width`` columns should be left that norm (``many_takes`` says whether it can take one).
+    ``heads``: it prepares its heads (``gemm_many_heads``)."""
+    if rows <= SKINNY_ROWS or not library().pl_gemm_many_applies(rows, columns, width, 1 if swiglu else 0):
+        return False
+    if swiglu:
+        return rows * columns <= MANY_TAKES_GATED if strips else many_swiglu_wins(rows, columns, width, False)
+    return rows * columns <= MANY_TAKES_RESULTS[strips] or (strips and heads and width <= MANY_TAKES_HEADS_WIDTH)
+
+
 def many_takes(handed, rows: int, columns: int, width: int, swiglu: bool = False) -> bool:
-    """Whether the product of many rows takes this norm, which a product of many rows handed forward: it costs less than the norm as a
-    kernel wherever ``many_add_wins`` had it handed forward (8,192 rows of 1,024 against 4,096 columns 76 us, the library's product 56 and the norm 25)."""
+    """Whether the product of many rows can take this norm, which a product of many rows handed forward."""
     return (rows > SKINNY_ROWS and handed.ssq.shape[1] * MANY_STRIPE == width
             and bool(library().pl_gemm_many_applies(rows, columns, width, 1 if swiglu else 0)))
 

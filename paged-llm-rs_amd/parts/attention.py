@@ -87,11 +87,7 @@ class PagedAttention:
         projection can add into it, None comes back."""
         batch = ctx.batch
         kv = ctx.kv()
-        cos = self.rotary.cos if self.rotary is not None else None
-        sin = self.rotary.sin if self.rotary is not None else None
-        rot = self.rotary.dim if self.rotary is not None else 0
-        prepare = kernels.QkFusion(self.q_gain, self.k_gain, self.eps, cos, sin, rot, ctx.writes_cache,
-                                   neighbours=bool(getattr(self.rotary, "neighbours", False)))
+        prepare = self._prepare(ctx.writes_cache)
         # (many rows: the projection may do what stands between it and attention, unless one kernel does that and the attention)
         qkv = None
         if (ctx.trace is None and batch.max_q_len > 1 and kernels.prepares_whole_heads(self.d, prepare)
@@ -111,6 +107,20 @@ class PagedAttention:
             return out
         return self.o_proj.forward(out, add_into=ctx.residual,
                                    hand=getattr(ctx, "hand", None) if ctx.residual is not None else None)
+
+    def _prepare(self, writes_cache: bool):
+        cos = self.rotary.cos if self.rotary is not None else None
+        sin = self.rotary.sin if self.rotary is not None else None
+        rot = self.rotary.dim if self.rotary is not None else 0
+        return kernels.QkFusion(self.q_gain, self.k_gain, self.eps, cos, sin, rot, writes_cache,
+                                neighbours=bool(getattr(self.rotary, "neighbours", False)))
+
+    def takes_norm(self, rows: int, batch) -> bool:
+        """Whether the norm in front of this mixer, of many rows, is worth leaving to its projection."""
+        prepare = self._prepare(True)
+        heads = (batch.max_q_len > 1 and kernels.prepares_whole_heads(self.d, prepare)
+                 and not kernels.near_applies(batch, self.nq, self.d, self.window, prepare))
+        return self.qkv_proj.takes_norm(rows, heads=heads)
 
     def _record_projections(self, qkv, batch, kv, trace) -> None:
         """q, k and v as projected, and q and k after their per-head norm (before the rotation).  The

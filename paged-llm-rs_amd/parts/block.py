@@ -65,11 +65,22 @@ class PreNormBlock:
         """The norm this block applies to the stream first: the block before may leave its work behind."""
         return self.norm1
 
+    @property
+    def first_taker(self):
+        """The part that takes that norm as an earlier product left it, where it is one that does."""
+        return self.mixer if getattr(self.mixer, "fuses", False) else None
+
     @staticmethod
-    def _room(norm, resid):
-        """Room for ``norm`` handed forward over the rows of ``resid``, where the norm has such a thing."""
+    def _room(norm, resid, taker, batch):
+        """Room for ``norm`` handed forward over the rows of ``resid``, where the norm has such a thing and, of many rows, the part behind it (``taker``)
+        says that it takes it: the product that fills the room is the slower one where nobody does."""
         make = getattr(norm, "handoff", None)
-        return make(resid.shape[0], resid.device) if make is not None else None
+        if make is None:
+            return None
+        rows = resid.shape[0]
+        if rows > kernels.SKINNY_ROWS and not (hasattr(taker, "takes_norm") and taker.takes_norm(rows, batch)):
+            return None
+        return make(rows, resid.device)
 
     def forward(self, resid, delta, ctx):
         """``delta``: what the block before has not added to the stream yet, or None.  Returns this
@@ -86,7 +97,7 @@ class PreNormBlock:
             x = self.norm1.apply(resid, delta, self.dtype)
         ctx.residual = resid if mixer_fuses else None
         # a mixer that adds into the stream may leave the second norm's work behind ...
-        ctx.hand = self._room(self.norm2, resid) if half and mixer_fuses and ffn_fuses else None
+        ctx.hand = self._room(self.norm2, resid, self.feed_forward, ctx.batch) if half and mixer_fuses and ffn_fuses else None
         mixed = self.mixer.forward(x, ctx)
         left, ctx.residual, ctx.hand = ctx.hand, None, None
         if mixed is None and ffn_fuses:
@@ -97,7 +108,7 @@ class PreNormBlock:
             # ... and a feed-forward that does, the next layer's first norm's
             after = getattr(ctx, "norm_after", None)
             if half and after is not None and getattr(self.feed_forward, "hands_forward", False):
-                room = self._room(after, resid)
+                room = self._room(after, resid, getattr(ctx, "taker_after", None), ctx.batch)
                 out = self.feed_forward.forward(x, residual=resid, hand=room)
                 ctx.handed_out = room if out is None and room is not None and room.filled else None
                 return out

@@ -84,6 +84,13 @@ class Linear:
             x = x.materialize()
         return kernels.gemm_many_heads(None if handed is not None else x, self.weight, batch, kv, nq, nkv, prepare, handed=handed, strips=self.strips)
 
+    def takes_norm(self, rows: int, swiglu: bool = False, activation: str = "silu", heads: bool = False) -> bool:
+        """Whether a norm of many rows in front of this product is worth leaving to it (``kernels.many_takes_wins``)."""
+        if self.bias is not None or self.weight.dtype != torch.bfloat16 or (swiglu and kernels.ACTIVATIONS[activation] != kernels.ACTIVATIONS["silu"]):
+            return False
+        columns = self.out_features // 2 if swiglu else self.out_features
+        return kernels.many_takes_wins(rows, columns, self.in_features, swiglu, self.strips is not None, heads)
+
     def _product(self, x, out_dtype: torch.dtype | None = None, add_into: torch.Tensor | None = None,
                  swiglu: bool = False, activation: str = "silu", hand=None):
         if isinstance(x, PendingNorm):
@@ -133,7 +140,7 @@ class Linear:
                 return None
             return kernels.gemm_stream(x, self.weight, out_dtype, swiglu=swiglu, activation=activation)
         if add_into is not None and not swiglu:
-            if kernels.many_add_wins(x.shape[0], self.out_features, self.in_features):
+            if hand is not None and kernels.many_add_wins(x.shape[0], self.out_features, self.in_features, self.strips is not None):
                 kernels.gemm_many(x, self.weight, add_into=add_into, hand=hand, strips=self.strips)
                 return None
             splits = kernels.library_splits(x.shape[0], self.out_features, self.in_features)

@@ -60,6 +60,10 @@ class GatedMlp:
             return out
         return self.finish(self.begin(x), residual=residual, hand=hand, out_dtype=out_dtype)
 
+    def takes_norm(self, rows: int, batch) -> bool:
+        """Whether the norm in front of this feed-forward, of many rows, is worth leaving to its first product."""
+        return self.gate_up_proj.takes_norm(rows, swiglu=True, activation=self.activation)
+
     def begin(self, x):
         """The first half, act(gate x) * (up x): all that reads the feed-forward's input.  A layer whose mixer
         adds into the stream that ``x`` is a norm of may run this half before the mixer and ``finish`` behind it."""

@@ -106,7 +106,7 @@ class LayerContext:
     the pages of the layer it reads from) and its state slots."""
 
     __slots__ = ("batch", "cache", "layer", "cache_layer", "writes_cache", "residual", "trace", "hand", "handed",
-                 "norm_after", "handed_out", "stream_rows", "stream_addend", "carried")
+                 "norm_after", "taker_after", "handed_out", "stream_rows", "stream_addend", "carried")
 
     def __init__(self, batch, cache, layer: int, cache_layer: int, writes_cache: bool):
         # ``layer`` and ``cache_layer`` are the keys under which the cache keeps this run's state and the pages it
@@ -124,10 +124,12 @@ class LayerContext:
         # Norms handed forward (``kernels.HandedNorm``; all optional, a part that knows nothing of them loses
         # nothing).  ``hand``: while a mixer that adds its own output runs, room for the norm that follows the
         # stream then.  ``handed``: what the layer before left of this layer's first norm.  ``norm_after``: the
-        # norm that the next layer applies to the stream first; a block that can leaves its work in ``handed_out``.
+        # norm that the next layer applies to the stream first; a block that can leaves its work in ``handed_out``.  ``taker_after``: the part
+        # of the next layer that would take it.
         self.hand = None
         self.handed = None
         self.norm_after = None
+        self.taker_after = None
         self.handed_out = None
         # The rows of the stream in the model's type, where the part that last updated the stream left them
         # (a block that normalises sublayer outputs does; any block may read, replace or clear them).
@@ -272,7 +274,8 @@ class DecoderModel:
                     kernels.residual_add(resid, began_with)
                     ctx.handed = ctx.stream_rows = None
             if at + 1 < len(schedule):
-                ctx.norm_after = getattr(self.blocks[schedule[at + 1].layer], "first_norm", None)
+                behind = self.blocks[schedule[at + 1].layer]
+                ctx.norm_after, ctx.taker_after = getattr(behind, "first_norm", None), getattr(behind, "first_taker", None)
             delta = self.blocks[entry.layer].forward(resid, delta, ctx)
             handed = ctx.handed_out if delta is None else None
             stream_rows = ctx.stream_rows if delta is None else None

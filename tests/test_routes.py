@@ -1,9 +1,15 @@
 """Which kernel a call goes to, as far as sizes alone decide it: the rules, asked as the engine asks them (no GPU; a chip of 256 compute units)."""
 
+from types import SimpleNamespace
+
 import pytest
+import torch
 
 from paged_llm_rs_amd import kernels
 from paged_llm_rs_amd.engine.batch import near_context, token_bucket
+from paged_llm_rs_amd.parts.block import PreNormBlock
+from paged_llm_rs_amd.parts.linear import Linear
+from paged_llm_rs_amd.parts.mlp import GatedMlp
 
 
 @pytest.fixture(autouse=True)
@@ -71,3 +77,56 @@ GATED = {
 def test_the_gated_product_of_many_rows_is_taken_where_it_measured_faster(columns, width):
     for rows, wanted in GATED[columns, width].items():
         assert [kernels.many_swiglu_wins(rows, columns, width, strips) for strips in (True, False)] == [w == "y" for w in wanted], rows
+
+
+# (columns of the stream, width before them, columns behind, how): {rows: whether handing the norm forward measured at most as long, out of strips and in rows}
+HANDED = {
+    (1024, 2048, 3072, "gated"): {448: "nn", 704: "nn", 1024: "nn", 1088: "yy", 2048: "yy", 4096: "yy", 8192: "yn"}, (1024, 1024, 2048, "gated"): {65: "yy", 1024: "yy", 8192: "yn"},
+    (1024, 3072, 4096, "plain"): {448: "nn", 1024: "nn", 1536: "yn", 3072: "yn", 4096: "nn", 8192: "nn"}, (1024, 3072, 4096, "heads"): {1024: "nn", 1536: "yn", 4096: "yn", 8192: "yn"},
+    (2048, 2048, 6144, "gated"): {448: "nn", 576: "yy", 1024: "yy", 4096: "yn", 8192: "nn"}, (2048, 2048, 4096, "plain"): {300: "nn", 576: "yy", 2048: "yy", 3072: "yn", 4096: "nn"},
+    (2048, 4096, 4096, "heads"): {576: "yn", 3072: "yn", 4096: "nn"}, (1024, 1024, 4096, "plain"): {300: "yy", 2048: "yy", 3072: "yn", 4096: "nn"}, (2048, 6144, 4096, "plain"): {2048: "nn"},
+}
+
+
+@pytest.mark.parametrize("columns,width,behind,how", list(HANDED))
+def test_a_norm_of_many_rows_is_handed_forward_where_that_measured_faster(columns, width, behind, how):
+    for rows, wanted in HANDED[columns, width, behind, how].items():
+        got = [kernels.many_add_wins(rows, columns, width, strips) and kernels.many_takes_wins(rows, behind, columns, how == "gated", strips, how == "heads") for strips in (True, False)]
+        assert got == [w == "y" for w in wanted], rows
+
+
+@pytest.fixture
+def products(monkeypatch):
+    """Which products a layer's parts call, without running them."""
+    called = []
+    monkeypatch.setattr(kernels, "gemm_many", lambda x, w, *a, **k: called.append("many") or k.get("add_into", torch.empty(0)))
+    monkeypatch.setattr(kernels, "linear_bf16", lambda x, *a: called.append("library") or x)
+    monkeypatch.setattr(kernels, "gemm_split_library", lambda *a, **k: called.append("library"))
+    return called
+
+
+def test_a_sum_whose_norm_nobody_takes_is_left_to_the_library(products):
+    """With no room for the norm behind it the product of many rows that adds is the slower one."""
+    down = Linear(torch.zeros(1024, 1024, dtype=torch.bfloat16))
+    down.strips = down.weight
+    x, stream = torch.zeros(700, 1024, dtype=torch.bfloat16), torch.zeros(700, 1024)
+    room = kernels.HandedNorm(torch.ones(1024), 1e-6, 700, 1024, "cpu")
+    assert down.forward(x, add_into=stream) is not None and products == ["library"]
+    assert down.forward(x, add_into=stream, hand=room) is None and products == ["library", "many"]
+
+
+def test_room_for_a_norm_of_many_rows_is_made_for_a_part_that_takes_it():
+    """A projection with a bias, a gate that is no SiLU and a part that knows nothing of it get the norm's rows from the norm itself."""
+    asked, batch = [], SimpleNamespace(max_q_len=700, num_seqs=1)
+    norm = SimpleNamespace(handoff=lambda rows, device: asked.append(rows) or "room")
+    mlp = lambda act: GatedMlp(SimpleNamespace(activation=act, names=None, intermediate_size=128),
+                               1024, {"gate_proj.weight": torch.zeros(128, 1024, dtype=torch.bfloat16), "up_proj.weight": torch.zeros(128, 1024, dtype=torch.bfloat16),
+                                      "down_proj.weight": torch.zeros(1024, 128, dtype=torch.bfloat16)}, torch.bfloat16, "cpu", {})
+    with_bias = SimpleNamespace(takes_norm=lambda rows, batch: Linear(torch.zeros(128, 1024, dtype=torch.bfloat16), torch.zeros(128)).takes_norm(rows))
+    stream = torch.zeros(700, 1024)
+    assert PreNormBlock._room(norm, stream, mlp("silu"), batch) == "room"
+    for taker in (mlp("gelu"), with_bias, SimpleNamespace(), None):
+        assert PreNormBlock._room(norm, stream, taker, batch) is None
+    assert asked == [700]
+    assert PreNormBlock._room(norm, stream[:64], None, batch) == "room"        # (few rows: as their products decide)
+    assert PreNormBlock._room(SimpleNamespace(), stream, mlp("silu"), batch) is None
