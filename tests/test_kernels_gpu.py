@@ -2185,6 +2185,58 @@ def test_attention_of_near_contexts_in_one_kernel(nq, nkv, bs, norm, turned):
     assert bool(out[starts[2]:starts[2] + 128].isnan().all()) and not bool(out[:38].isnan().any())
 
 
+@pytest.mark.parametrize("nq,nkv", [(16, 8), (8, 1), (64, 8)])
+def test_values_that_are_not_finite_reach_the_tokens_that_see_them(nq, nkv):
+    """Contexts of up to 128 in one kernel: infinite and NaN values of a request's own tokens and of keys that were there before.  A token that stands before such a key, and every other
+    column, has the bits that it has without; a token at or behind it does not come out finite in that column.  Pages get the values as they are."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    d, bs, eps, scale = 128, 16, 1e-6, 128 ** -0.5
+    requests = [(37, 37), (10, 10), (1, 64), (16, 33), (100, 120), (128, 128)]
+    S, per, n = len(requests), 8, sum(t for t, _ in requests)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    starts = [sum(t for t, _ in requests[:s]) for s in range(S)]
+    table = torch.randperm(S * per, device=DEV).reshape(S, per).to(torch.int32)
+    positions, seq_of = i32([c - t + i for t, c in requests for i in range(t)]), i32([s for s, (t, _) in enumerate(requests) for _ in range(t)])
+    clean = torch.randn(n, (nq + 2 * nkv) * d, device=DEV).bfloat16()
+    k_pool, v_pool = (torch.randn(S * per * bs, nkv * d, device=DEV).bfloat16() for _ in range(2))
+    q_gain, k_gain = torch.ones(d, device=DEV), torch.ones(d, device=DEV)
+    cos, sin = tables(128, d, 1e4)
+    prepare = kernels.QkFusion(q_gain, k_gain, eps, cos, sin, d, True)
+    batch = SimpleNamespace(positions=positions, seq_of=seq_of, q_start=i32(starts), q_len=i32([t for t, _ in requests]), ctx_len=i32([c for _, c in requests]),
+                            num_seqs=S, num_tokens=n, max_ctx_len=1024, near_ctx_len=128, max_q_len=128)
+    assert kernels.near_applies(batch, nq, d, 0, prepare)
+    # (request, key, key head, column, value)
+    wild = [(0, 5, 0, 3, math.inf), (0, 5, 0, 70, math.nan), (0, 36, nkv - 1, 127, -math.inf), (1, 9, 0, 0, math.nan), (2, 63, 0, 64, math.inf), (3, 20, 0, 33, math.inf),
+            (3, 4, nkv - 1, 5, math.nan), (4, 119, 0, 99, math.inf), (4, 19, 0, 31, -math.inf), (4, 70, nkv - 1, 32, math.nan), (5, 0, 0, 1, math.inf), (5, 127, 0, 2, math.nan), (5, 64, 0, 1, -math.inf)]
+
+    def run(with_them):
+        qkv, kv = clean.clone(), SimpleNamespace(block_table=table, block_size=bs, k_pool=k_pool.clone(), v_pool=v_pool.clone())
+        for s, key, head, column, value in wild if with_them else ():
+            t, c = requests[s]
+            if key >= c - t:
+                qkv[starts[s] + key - (c - t), (nq + nkv + head) * d + column] = value
+            else:
+                kv.v_pool[int(table[s, key // bs]) * bs + key % bs, head * d + column] = value
+        rows, pages = qkv.clone(), (kv.k_pool.clone(), kv.v_pool.clone())
+        out = torch.full((n, nq * d), 7.0, device=DEV).bfloat16()
+        kernels.attention_step(qkv, out, batch, kv, nq, nkv, d, scale, 0, prepare)
+        kernels.qk_norm_rope_kv_write(rows, q_gain, k_gain, eps, cos, sin, d, positions, seq_of, table, bs, *pages, nq, nkv, d)
+        assert torch.equal(kv.k_pool.view(torch.int16), pages[0].view(torch.int16)) and torch.equal(kv.v_pool.view(torch.int16), pages[1].view(torch.int16))
+        return out
+
+    want, got = run(False), run(True)
+    reached = torch.zeros(n, nq * d, dtype=torch.bool, device=DEV)
+    for s, key, head, column, _ in wild:
+        t, c = requests[s]
+        for h in range(head * (nq // nkv), (head + 1) * (nq // nkv)):
+            reached[starts[s] + max(0, key - (c - t)):starts[s] + t, h * d + column] = True
+    assert bool(want.isfinite().all()) and not bool(got[reached].isfinite().any())
+    assert torch.equal(got[~reached].view(torch.int16), want[~reached].view(torch.int16))
+
+
 @pytest.mark.parametrize("nq,nkv,K,norm,turned", [(16, 8, 1024, True, True), (4, 1, 128, False, True), (3, 3, 192, True, False), (5, 1, 64, False, False)])
 def test_the_projection_of_many_rows_prepares_its_heads(nq, nkv, K, norm, turned):
     """Queries and pages have the bits that the product and the stand-alone kernel behind it give, at every shape of tile, with tiles that end inside the rows
