@@ -863,7 +863,9 @@ def prefill_splits(requests: int, max_q_len: int, nq: int, d: int, max_ctx: int,
 
 # A step whose contexts are all as near as one workgroup holds them runs preparation and attention as one kernel, a workgroup a request and query head,
 # while those are no more than two a compute unit; beyond, requests of a token or two keep a workgroup each for little (us, two kernels / one: 32 heads, 8
-# requests of 10 tokens at 120 20.1 / 11.5, 16 28.7 / 21.1, 32 48 / 40, but one of 40 beside 31 single tokens 27.4 / 27.9, beside 63 24.8 / 50.3).
+# requests of 10 tokens at 120 20.3 / 12.0, 16 28 / 21, 32 48 / 40, but one of 40 beside 31 single tokens 27.4 / 27.9, beside 63 24.8 / 50.3).  So do steps of single tokens alone, which come
+# here where eight query heads and more share a key head: no more than one a compute unit (64 heads over 8: one token at 40 15.6 / 8.4, four at 120 16.0 / 11.5, eight 18.1 / 20.7; two
+# of three tokens at 100 17.9 / 11.1, eight 19.2 / 20.0).
 NEAR_KEYS = 128
 NEAR_HEAD = 128
 NEAR_WORKGROUPS = 512
@@ -873,7 +875,7 @@ def near_applies(batch, nq: int, d: int, window: int, prepare: QkFusion) -> bool
     """Whether a step of bfloat16 rows goes to ``attention_near``."""
     near = getattr(batch, "near_ctx_len", None)
     return (_attention_mode == "kernel" and near is not None and near <= NEAR_KEYS and _says_rows(batch) and prepares_whole_heads(d, prepare)
-            and not window and (getattr(batch, "live_seqs", None) or batch.num_seqs) * nq <= NEAR_WORKGROUPS)
+            and not window and (getattr(batch, "live_seqs", None) or batch.num_seqs) * nq <= (NEAR_WORKGROUPS if batch.max_q_len > 1 else compute_units()))
 
 
 def prepares_whole_heads(d: int, prepare: QkFusion) -> bool:

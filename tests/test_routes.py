@@ -130,3 +130,16 @@ def test_room_for_a_norm_of_many_rows_is_made_for_a_part_that_takes_it():
     assert asked == [700]
     assert PreNormBlock._room(norm, stream[:64], None, batch) == "room"        # (few rows: as their products decide)
     assert PreNormBlock._room(SimpleNamespace(), stream, mlp("silu"), batch) is None
+
+
+def test_near_contexts_go_to_one_kernel_while_the_workgroups_are_few():
+    """Two workgroups a compute unit, one in steps of single tokens; no window, heads of 128 turned whole, a step that says which rows its requests bring."""
+    prepare = kernels.QkFusion(None, None, 1e-6, None, None, 128, True)
+
+    def takes(requests, nq, longest=10, near=128, d=128, window=0, prepare=prepare, **more):
+        return kernels.near_applies(SimpleNamespace(q_start=0, q_len=0, ctx_len=0, max_ctx_len=1024, near_ctx_len=near, max_q_len=longest, num_seqs=requests, **more), nq, d, window, prepare)
+
+    assert takes(16, 32) and not takes(17, 32) and takes(8, 64) and not takes(9, 64)
+    assert takes(4, 64, longest=1) and not takes(5, 64, longest=1) and not takes(8, 64, longest=1)
+    assert takes(17, 32, live_seqs=16) and not takes(1, 16, near=256) and not takes(1, 16, near=None) and not takes(1, 16, window=64) and not takes(1, 16, d=64)
+    assert not takes(1, 16, prepare=kernels.QkFusion(None, None, 1e-6, None, None, 64, True)) and not takes(1, 16, prepare=kernels.QkFusion(None, None, 1e-6, None, None, 128, False))
