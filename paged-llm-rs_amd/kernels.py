@@ -890,8 +890,12 @@ def _heads_code(kv, nkv: int, prepare: QkFusion) -> int:
         _need(pool, what, None, torch.bfloat16)
         if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % kv.block_size != 0:
             raise TensorError(f"{what} has shape {tuple(pool.shape)}, expected [pages*{kv.block_size}, {nkv * d}]")
+    if kv.k_pool.shape != kv.v_pool.shape:
+        raise TensorError("key and value pools differ in shape")
     if kv.k_pool.shape[0] >= 2 ** 31:
         raise TensorError("a pool of 2^31 slots or more is not addressed by these kernels")
+    if kv.block_table.dim() != 2:
+        raise TensorError(f"block table has shape {tuple(kv.block_table.shape)}, expected [requests, pages]")
     gain_code = F32
     if prepare.q_gain is not None:
         _need(prepare.q_gain, "query norm gain", (d,))
@@ -908,17 +912,26 @@ def _heads_code(kv, nkv: int, prepare: QkFusion) -> int:
 def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, scale: float, prepare: QkFusion) -> torch.Tensor:
     """Everything between the fused q/k/v projection and the output projection for a step whose contexts are no longer than 128 tokens
     (``NEAR_KEYS``; rows of longer ones come out as NaN): heads of 128 rotated whole or not at all, in bfloat16."""
-    n, d, S = qkv.shape[0], NEAR_HEAD, kv.block_table.shape[0]
+    n, d = qkv.shape[0], NEAR_HEAD
     _need(qkv, "fused q/k/v projection", (n, (nq + 2 * nkv) * d), torch.bfloat16)
     _need(out, "attention output", (n, nq * d), torch.bfloat16)
     _need(kv.block_table, "block table", None, torch.int32)
+    gain_code = _heads_code(kv, nkv, prepare)
+    S = kv.block_table.shape[0]
     for t, what in ((batch.q_start, "first row of each request"), (batch.q_len, "tokens of each request"), (batch.ctx_len, "context length of each request")):
         _need(t, what, (S,), torch.int32)
-    gain_code = _heads_code(kv, nkv, prepare)
-    live = getattr(batch, "live_seqs", None)
+    _need(batch.positions, "positions", (n,), torch.int32)
+    _need(batch.seq_of, "request index of each token", (n,), torch.int32)
+    if not 0 < batch.max_q_len <= n:
+        raise TensorError(f"the longest portion is said to have {batch.max_q_len} of the step's {n} tokens")
+    live = S if getattr(batch, "live_seqs", None) is None else int(batch.live_seqs)
+    if not 0 < live <= S:
+        raise TensorError(f"{live} requests with tokens of {S}")
+    if not prepares_whole_heads(d, prepare):
+        raise TensorError(f"near contexts: a rotation of {prepare.rot} of heads of {d}")
     _check(library().pl_attention_near(
         qkv.data_ptr(), out.data_ptr(), _ptr(prepare.q_gain), _ptr(prepare.k_gain), gain_code, float(prepare.eps), _ptr(prepare.cos), _ptr(prepare.sin),
-        batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.ctx_len.data_ptr(), S if live is None else int(live), kv.block_table.data_ptr(),
+        batch.q_start.data_ptr(), batch.q_len.data_ptr(), batch.ctx_len.data_ptr(), live, kv.block_table.data_ptr(),
         kv.block_table.shape[1], kv.block_size, kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), nq, nkv, float(scale), _stream()))
     return out
 
@@ -1419,8 +1432,8 @@ def gemm_many_heads(x: torch.Tensor | None, w: torch.Tensor, batch, kv, nq: int,
     _need(batch.positions, "positions", (M,), torch.int32)
     _need(batch.seq_of, "request index of each token", (M,), torch.int32)
     _need(kv.block_table, "block table", None, torch.int32)
-    if not prepares_whole_heads(NEAR_HEAD, prepare) or kv.block_table.dim() != 2:
-        raise TensorError(f"heads prepared by their projection: a rotation of {prepare.rot}, block table of shape {tuple(kv.block_table.shape)}")
+    if not prepares_whole_heads(NEAR_HEAD, prepare):
+        raise TensorError(f"heads prepared by their projection: a rotation of {prepare.rot}")
     gain_code = _heads_code(kv, nkv, prepare)
     out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _check(library().pl_gemm_many_heads(

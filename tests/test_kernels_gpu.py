@@ -2237,6 +2237,41 @@ def test_values_that_are_not_finite_reach_the_tokens_that_see_them(nq, nkv):
     assert torch.equal(got[~reached].view(torch.int16), want[~reached].view(torch.int16))
 
 
+def test_kernels_that_write_pages_refuse_what_the_stand_alone_one_refuses():
+    """Pools of unlike sizes, a table that is no table, more requests than the step has, positions of another count: an error on the host, for the near contexts' kernel and for the
+    projection that prepares its heads."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.errors import TensorError
+
+    nq, nkv, d, bs, n, K = 4, 2, 128, 16, 70, 64
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    pool = lambda pages, cols=nkv * d: torch.zeros(pages * bs, cols, device=DEV).bfloat16()
+    prepare = kernels.QkFusion(None, None, 1e-6, None, None, 0, True)
+    x, w = torch.zeros(n, K, device=DEV).bfloat16(), torch.zeros((nq + 2 * nkv) * d, K, device=DEV).bfloat16()
+    qkv, out = torch.zeros(n, (nq + 2 * nkv) * d, device=DEV).bfloat16(), torch.zeros(n, nq * d, device=DEV).bfloat16()
+    batch = lambda **more: SimpleNamespace(**{**dict(positions=torch.arange(n, device=DEV).int(), seq_of=torch.zeros(n, device=DEV).int(), q_start=i32([0]), q_len=i32([n]), ctx_len=i32([n]),
+                                                     num_seqs=1, num_tokens=n, max_ctx_len=1024, near_ctx_len=128, max_q_len=n), **more})
+    kv = lambda **more: SimpleNamespace(**{**dict(block_table=i32([list(range(8))]), block_size=bs, k_pool=pool(8), v_pool=pool(8)), **more})
+    kernels.attention_near(qkv, out, batch(), kv(), nq, nkv, 0.1, prepare)
+    kernels.gemm_many_heads(x, w, batch(), kv(), nq, nkv, prepare)
+    for b, c in ((batch(), kv(v_pool=pool(4))), (batch(), kv(k_pool=pool(4))), (batch(), kv(block_table=i32(list(range(8))))), (batch(), kv(v_pool=pool(8, d))),
+                 (batch(positions=i32([0])), kv()), (batch(seq_of=i32([0])), kv())):
+        with pytest.raises(TensorError):
+            kernels.attention_near(qkv, out, b, c, nq, nkv, 0.1, prepare)
+        with pytest.raises(TensorError):
+            kernels.gemm_many_heads(x, w, b, c, nq, nkv, prepare)
+    for b in (batch(live_seqs=2), batch(live_seqs=0), batch(max_q_len=n + 1), batch(ctx_len=i32([n, n]))):
+        with pytest.raises(TensorError):
+            kernels.attention_near(qkv, out, b, kv(), nq, nkv, 0.1, prepare)
+    for p in (kernels.QkFusion(None, None, 1e-6, None, None, 64, True), kernels.QkFusion(None, None, 1e-6, None, None, 128, False)):
+        with pytest.raises(TensorError):
+            kernels.attention_near(qkv, out, batch(), kv(), nq, nkv, 0.1, p)
+        with pytest.raises(TensorError):
+            kernels.gemm_many_heads(x, w, batch(), kv(), nq, nkv, p)
+
+
 @pytest.mark.parametrize("nq,nkv,K,norm,turned", [(16, 8, 1024, True, True), (4, 1, 128, False, True), (3, 3, 192, True, False), (5, 1, 64, False, False)])
 def test_the_projection_of_many_rows_prepares_its_heads(nq, nkv, K, norm, turned):
     """Queries and pages have the bits that the product and the stand-alone kernel behind it give, at every shape of tile, with tiles that end inside the rows
