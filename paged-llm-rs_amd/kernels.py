@@ -160,6 +160,12 @@ def _need(t: torch.Tensor, what: str, shape=None, dtype=None) -> torch.Tensor:
     return t
 
 
+def in_pieces(*tensors) -> bool:
+    """Whether all of them (None: not there) begin at whole 16 bytes, which the kernels of many rows and of near contexts ask of what they read and write 16 bytes a lane.  A tensor that is
+    part of another may not; it goes to the kernels that took it before those were there."""
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -948,7 +954,8 @@ def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
                                       fuse=prepare, arrivals=_arrivals(batch, nq, splits))
-    if not prepared and qkv.dtype == torch.bfloat16 and near_applies(batch, nq, d, window, prepare):
+    if (not prepared and qkv.dtype == torch.bfloat16 and near_applies(batch, nq, d, window, prepare)
+            and in_pieces(qkv, out, kv.k_pool, kv.v_pool, prepare.q_gain, prepare.k_gain, prepare.cos, prepare.sin)):
         return attention_near(qkv, out, batch, kv, nq, nkv, scale, prepare)
     if not prepared:
         qk_norm_rope_kv_write(qkv, prepare.q_gain, prepare.k_gain, prepare.eps, prepare.cos, prepare.sin, prepare.rot,
@@ -1643,7 +1650,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
     _need(w, "weight", None, torch.bfloat16)
     if out_dtype == torch.float32:
         # the projection onto the vocabulary: 32-bit out of the 32-bit sums, whichever product it is
-        if many_vocabulary_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
+        if many_vocabulary_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None) and in_pieces(x, w if strips is None else strips):
             return gemm_many(x, w, torch.float32, strips=strips)
         if wide_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
             return gemm_wide(x, _need(strips, "weights in strips", tuple(w.shape), torch.bfloat16))
@@ -1651,7 +1658,8 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
             return gemm_stream(x, w, torch.float32)
         if skinny_applies(x) and x.shape[1] <= (SKINNY_F32_FEW_K if x.shape[0] <= 16 else SKINNY_SHALLOW_K):
             return gemm_skinny(x, w, torch.float32, strips=strips)
-        if w.shape[0] < MANY_VOCABULARY and many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
+        if (w.shape[0] < MANY_VOCABULARY and many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None)
+                and in_pieces(x, w if strips is None else strips)):
             return gemm_many(x, w, torch.float32, strips=strips)
         if x.shape[1] % 8 == 0:
             return torch.mm(x, w.t(), out_dtype=torch.float32)
@@ -1660,7 +1668,7 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
         return gemm_skinny(x, w, out_dtype, strips=strips)
     if stream_wins(x.shape[0], w.shape[0], x.shape[1]):
         return gemm_stream(x, w, out_dtype)
-    if many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None):
+    if many_store_wins(x.shape[0], w.shape[0], x.shape[1], strips is not None) and in_pieces(x, w if strips is None else strips):
         return gemm_many(x, w, strips=strips)
     splits = library_splits(x.shape[0], w.shape[0], x.shape[1])
     if splits > 1 and turned is not None:
@@ -2517,7 +2525,8 @@ def moe_grouped(x: torch.Tensor, batch, table, w_gate_up: torch.Tensor, w_down: 
     own = pairs - n if size else pairs
     likely = min(tiles, E * -(-max(own, 1) // (E * MOE_TILE)) + (-(-n // MOE_TILE) if size else 0))
     many = lambda rows, N, K, pitch: lib.pl_gemm_many_grouped_applies(tiles, rows, N, K, pitch)
-    if gated and act == ACTIVATIONS["silu"] and many(n, F, W, W) and (not size or many(n, size, W, W)):
+    whole = in_pieces(x, w_gate_up, w_down, *(shared or ()))
+    if gated and act == ACTIVATIONS["silu"] and whole and many(n, F, W, W) and (not size or many(n, size, W, W)):
         _check(lib.pl_gemm_many_grouped(x.data_ptr(), w_gate_up.data_ptr(), hidden.data_ptr(), tile_group.data_ptr(), gather.data_ptr(),
                                         w_gate_up.stride(0), tiles, likely, n, F, W, 1, W, longest, last, shared_up, size, W, stream))
     else:
@@ -2526,7 +2535,7 @@ def moe_grouped(x: torch.Tensor, batch, table, w_gate_up: torch.Tensor, w_down: 
                                          W, longest, last, shared_up, size, W, stream))
     splits = moe_down_splits(tiles, W, min(F, size) if size else F)
     y = torch.empty((splits, slots, W), dtype=torch.float32, device=x.device)
-    if splits == 1 and many(slots, W, F, longest) and (not size or many(slots, W, size, longest)):
+    if splits == 1 and whole and many(slots, W, F, longest) and (not size or many(slots, W, size, longest)):
         _check(lib.pl_gemm_many_grouped(hidden.data_ptr(), w_down.data_ptr(), y.data_ptr(), tile_group.data_ptr(), 0, W * F, tiles, likely, slots, W, F, 3,
                                         longest, W, last, shared_down, W, size, stream))
     else:

@@ -69,7 +69,8 @@ class Linear:
     def forward_heads(self, x, batch, kv, nq: int, nkv: int, prepare):
         """The projection [q | k | v] with norm, rotation and page write behind it in one kernel (``kernels.gemm_many_heads``), or None where the product
         of so many rows is not that kernel's."""
-        if self.bias is not None or self.weight.dtype != torch.bfloat16:
+        if self.bias is not None or self.weight.dtype != torch.bfloat16 or not kernels.in_pieces(
+                self._read, kv.k_pool, kv.v_pool, prepare.q_gain, prepare.k_gain, prepare.cos, prepare.sin):
             return None
         handed = None
         if isinstance(x, PendingNorm):
@@ -77,6 +78,8 @@ class Linear:
                 return None
             if x.handed is not None and kernels.many_takes(x.handed, x.num_rows, self.out_features, self.in_features):
                 handed = x.handed
+        elif x.dim() != 2 or x.dtype != torch.bfloat16 or x.shape[1] != self.in_features or not kernels.in_pieces(x):
+            return None
         if handed is None and not kernels.many_store_wins(x.num_rows if isinstance(x, PendingNorm) else x.shape[0], self.out_features, self.in_features,
                                                           self.strips is not None):
             return None
@@ -84,9 +87,15 @@ class Linear:
             x = x.materialize()
         return kernels.gemm_many_heads(None if handed is not None else x, self.weight, batch, kv, nq, nkv, prepare, handed=handed, strips=self.strips)
 
+    @property
+    def _read(self) -> torch.Tensor:
+        """What a product of many rows reads for the weight."""
+        return self.weight if self.strips is None else self.strips
+
     def takes_norm(self, rows: int, swiglu: bool = False, activation: str = "silu", heads: bool = False) -> bool:
         """Whether a norm of many rows in front of this product is worth leaving to it (``kernels.many_takes_wins``)."""
-        if self.bias is not None or self.weight.dtype != torch.bfloat16 or (swiglu and kernels.ACTIVATIONS[activation] != kernels.ACTIVATIONS["silu"]):
+        if (self.bias is not None or self.weight.dtype != torch.bfloat16 or (swiglu and kernels.ACTIVATIONS[activation] != kernels.ACTIVATIONS["silu"])
+                or not kernels.in_pieces(self._read)):
             return False
         columns = self.out_features // 2 if swiglu else self.out_features
         return kernels.many_takes_wins(rows, columns, self.in_features, swiglu, self.strips is not None, heads)
@@ -104,7 +113,7 @@ class Linear:
             silu = kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
             if (x.handed is not None and add_into is None and self.weight.dtype == torch.bfloat16 and (silu or not swiglu)
                     and (out_dtype or x.out_dtype) == torch.bfloat16
-                    and kernels.many_takes(x.handed, x.num_rows, columns, self.in_features, swiglu)):
+                    and kernels.many_takes(x.handed, x.num_rows, columns, self.in_features, swiglu) and kernels.in_pieces(self._read)):
                 return kernels.gemm_many(None, self.weight, swiglu=swiglu, handed=x.handed, strips=self.strips)
             if (getattr(x.norm, "fuses_into_product", False) and add_into is None
                     and kernels.fused_norm_applies(x.num_rows, self.in_features, self.weight)
@@ -123,7 +132,8 @@ class Linear:
             if swiglu:
                 return kernels.gemm_plain_gated(x, self.weight, activation)
             return kernels.gemm_plain(x, self.weight, out_dtype=torch.float32)
-        if (out_dtype == torch.float32 and add_into is None and not swiglu
+        whole = kernels.in_pieces(x, self._read)
+        if (out_dtype == torch.float32 and add_into is None and not swiglu and whole
                 and kernels.many_vocabulary_wins(x.shape[0], self.out_features, self.in_features, self.strips is not None)):
             return kernels.gemm_many(x, self.weight, torch.float32, strips=self.strips)
         if kernels.skinny_applies(x, self.weight, self.strips is not None):
@@ -140,7 +150,8 @@ class Linear:
                 return None
             return kernels.gemm_stream(x, self.weight, out_dtype, swiglu=swiglu, activation=activation)
         if add_into is not None and not swiglu:
-            if hand is not None and kernels.many_add_wins(x.shape[0], self.out_features, self.in_features, self.strips is not None):
+            if (hand is not None and kernels.many_add_wins(x.shape[0], self.out_features, self.in_features, self.strips is not None)
+                    and whole and kernels.in_pieces(add_into, hand.gain)):
                 kernels.gemm_many(x, self.weight, add_into=add_into, hand=hand, strips=self.strips)
                 return None
             splits = kernels.library_splits(x.shape[0], self.out_features, self.in_features)
@@ -148,7 +159,7 @@ class Linear:
                 kernels.gemm_split_library(x, self.weight, splits, add_into=add_into, turned=self.turned)
                 return None
         if swiglu:
-            if (kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"]
+            if (kernels.ACTIVATIONS[activation] == kernels.ACTIVATIONS["silu"] and whole
                     and kernels.many_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features, self.strips is not None)):
                 return kernels.gemm_many(x, self.weight, swiglu=True, strips=self.strips)
             if kernels.tiled_swiglu_wins(x.shape[0], self.out_features // 2, self.in_features):

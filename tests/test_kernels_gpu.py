@@ -2272,6 +2272,59 @@ def test_kernels_that_write_pages_refuse_what_the_stand_alone_one_refuses():
             kernels.gemm_many_heads(x, w, batch(), kv(), nq, nkv, p)
 
 
+def test_rows_that_begin_in_the_middle_of_16_bytes_go_where_they_went():
+    """Inputs, weights, gains and streams that are parts of other tensors, 8 bytes into a piece of 16: not refused, and what 64-bit arithmetic says (a bfloat16 result within its rounding
+    and that of an input's, 2^-8)."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.parts.linear import Linear
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 16, dtype=t.dtype, device=DEV)
+        at = room[8 // t.element_size():][:t.numel()].view(t.shape)
+        assert at.data_ptr() % 16 == 8 and at.is_contiguous()
+        return at.copy_(t)
+
+    x, w = torch.randn(300, 1024, device=DEV).bfloat16(), (torch.randn(1024, 1024, device=DEV) / 32).bfloat16()
+    want = x.double() @ w.double().T
+    assert kernels.many_store_wins(300, 1024, 1024, False)
+    for a, b in ((shifted(x), w), (x, shifted(w))):
+        assert rel(kernels.linear_bf16(a, b, torch.bfloat16), want) < 2.0 ** -8 and rel(kernels.linear_bf16(a, b, torch.float32), want) < 1e-5
+    both = (torch.randn(2 * 3072, 1024, device=DEV) / 32).bfloat16()
+    tall = torch.randn(1100, 1024, device=DEV).bfloat16()
+    gate_up = tall.double() @ both.double().T
+    gated = torch.nn.functional.silu(gate_up[:, :3072]) * gate_up[:, 3072:]
+    keep, Linear.keep_strips = Linear.keep_strips, False
+    try:
+        for a, b in ((shifted(tall), both), (tall, shifted(both))):
+            assert kernels.many_swiglu_wins(1100, 3072, 1024, False) and rel(Linear(b).forward(a, swiglu=True), gated) < 2.0 ** -7
+        stream, room = torch.randn(300, 1024, device=DEV), kernels.HandedNorm(torch.ones(1024, device=DEV), 1e-6, 300, 1024, DEV)
+        for a, b, into, gain in ((shifted(x), w, stream, room.gain), (x, shifted(w), stream, room.gain), (x, w, shifted(stream), room.gain), (x, w, stream, shifted(room.gain))):
+            room.gain = gain
+            y = Linear(b).forward(a, add_into=into, hand=room)
+            assert y is not None and not room.filled and rel(y, want) < 2.0 ** -8
+    finally:
+        Linear.keep_strips = keep
+    # gains of the heads, in a step of near contexts and behind the projection
+    nq, nkv, d, bs, n = 4, 2, 128, 16, 100
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    gains = [torch.rand(d, device=DEV) + 0.5 for _ in range(2)]
+    cos, sin = tables(128, d, 1e4)
+    heads, y = Linear((torch.randn((nq + 2 * nkv) * d, 1024, device=DEV) / 32).bfloat16()), torch.randn(n, 1024, device=DEV).bfloat16()
+    batch = SimpleNamespace(positions=torch.arange(n, device=DEV).int(), seq_of=torch.zeros(n, device=DEV).int(), q_start=i32([0]), q_len=i32([n]), ctx_len=i32([n]), num_seqs=1, num_tokens=n,
+                            max_ctx_len=1024, near_ctx_len=128, max_q_len=n, tokens_of_short_requests=lambda limit: 0)
+    outs = []
+    for g in (gains, [shifted(t) for t in gains]):
+        kv = SimpleNamespace(block_table=i32([list(range(8))]), block_size=bs, **{p: torch.zeros(8 * bs, nkv * d, device=DEV).bfloat16() for p in ("k_pool", "v_pool")})
+        prepare = kernels.QkFusion(*g, 1e-6, cos, sin, d, True)
+        assert (heads.forward_heads(y, batch, kv, nq, nkv, prepare) is None) == (g is not gains)
+        out = torch.empty(n, nq * d, device=DEV).bfloat16()
+        kernels.attention_step(heads.forward(y), out, batch, kv, nq, nkv, d, d ** -0.5, 0, prepare)
+        outs.append((out, kv.k_pool, kv.v_pool))
+    assert rel(outs[1][0], outs[0][0].double()) < 6e-3 and all(torch.equal(a, b) for a, b in zip(outs[0][1:], outs[1][1:]))
+
+
 @pytest.mark.parametrize("nq,nkv,K,norm,turned", [(16, 8, 1024, True, True), (4, 1, 128, False, True), (3, 3, 192, True, False), (5, 1, 64, False, False)])
 def test_the_projection_of_many_rows_prepares_its_heads(nq, nkv, K, norm, turned):
     """Queries and pages have the bits that the product and the stand-alone kernel behind it give, at every shape of tile, with tiles that end inside the rows
