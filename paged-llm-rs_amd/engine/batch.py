@@ -52,7 +52,7 @@ class StepBatch:
         self.num_logit_rows = num_logit_rows
         self.max_q_len = max_q_len
         self.max_ctx_len = max_ctx_len
-        self.near_ctx_len = max_ctx_len  # (``near_context`` where the contexts themselves are known)
+        self.near_ctx_len = max_ctx_len  # (``near_context`` where the contexts themselves are known; never less than the longest)
         self.seq_ids = seq_ids
         # On the host: the tokens every live request brings; whether the step reports bounds instead of
         # counts (a padded step does); and, for such a step, {limit: the most tokens that requests of fewer
@@ -129,13 +129,15 @@ def context_bound(longest: int) -> int:
 
 
 def near_context(longest: int) -> int:
-    """The same, from 128 on, for what only chooses how many workgroups share the keys of a prompt's tokens.  A fresh prompt of a few
+    """The same, from 128 on, for what chooses how many workgroups share the keys of a prompt's tokens and, up to 128, the kernel that takes preparation and attention
+    together: that one holds no more keys, and rows of longer contexts come out of it as NaN.  So no step may be run by a nearer bound than its contexts' own.  A fresh prompt of a few
     dozen tokens has one tile of keys: dealt out by a bound of 1,024 it had four workgroups a tile, three without a key, and a
     second launch to put them together (0.6B shape, a step: 37 tokens 1,411 to 1,314 us, 200 tokens 2,310 to 2,232, 100 tokens beside eight decoded at
     contexts of 60 2,550 to 2,231; 37 tokens behind 700 others, whose
     keys are worth sharing, stay as they were).  Past one tile the shares are added up in another order, so the last bits of a context's keys
     and values depend on the bound that its prompt was dealt by, as they do on ``context_bound`` past 1,024 tokens.  The plain attention
-    layers in bfloat16 go by it (``shares_by_near_context``); where a model has one, a step's shape names it, so a captured step is replayed for contexts like its own."""
+    layers in bfloat16 go by it, and a mixer that does says so (``shares_by_near_context``); where a model has one, a step's shape names it, so a captured step is replayed for contexts
+    like its own, and where it has none, a captured step's bound is ``context_bound`` (``ShapeGraph``, which also refuses steps that are not as near as its own)."""
     bound = 128
     while bound < longest and bound < 1024:
         bound *= 2
@@ -161,6 +163,10 @@ class TableTooWide(CaptureOutgrown):
 
 class ContextTooLong(CaptureOutgrown):
     """A request's context is longer than the bound the step was to report."""
+
+
+class NotNear(CaptureOutgrown):
+    """A request's context is longer than the near bound that the step's kernels were chosen by."""
 
 
 class ShortTokensOutgrown(CaptureOutgrown):

@@ -35,7 +35,7 @@ import torch
 
 from .. import kernels
 from ..errors import ConfigError, PagedLLMError, TensorError
-from .batch import CannotFeed, CaptureOutgrown, StepBatch, TableTooWide, build_batch, context_bound, near_context, token_bucket
+from .batch import CannotFeed, CaptureOutgrown, NotNear, StepBatch, TableTooWide, build_batch, context_bound, near_context, token_bucket
 
 GRAPH_MAX_REQUESTS = 256     # requests a captured step may have (steps of more run kernel by kernel)
 SHAPE_GRAPH_ROWS_KEPT = 32768    # rows over all captured shapes of steps other than plain decoding (the
@@ -312,7 +312,9 @@ class ShapeGraph:
         self.batch = StepBatch(self.device_buf, first.layout, first.num_tokens, first.num_seqs, list(widths),
                                first.num_logit_rows, first.max_q_len, ctx_bound, [],
                                tokens_each=first.tokens_each, padded=True, short_bounds=first.short_bounds)
-        self.batch.live_seqs, self.batch.near_ctx_len = first.live_seqs, first.near_ctx_len
+        self.batch.live_seqs = first.live_seqs
+        # (How near the contexts are decides which kernel a layer's attention is: a shape that does not name it is captured for any context that fits.)
+        self.batch.near_ctx_len = first.near_ctx_len if getattr(model, "shares_by_near_context", False) else ctx_bound
         self.graph = None
         self.logits = None
 
@@ -340,6 +342,8 @@ class ShapeGraph:
             batch = self._lay_out(entries)
             if batch.packed.numel() != self.size:
                 raise ConfigError("a step of another shape than the captured one")
+            if batch.near_ctx_len > self.batch.near_ctx_len:
+                raise NotNear(f"contexts within {batch.near_ctx_len} tokens in a step captured for {self.batch.near_ctx_len}")
             self.ring.advance()
             self.ring.host.copy_(batch.packed)
         else:

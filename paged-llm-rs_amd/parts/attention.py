@@ -55,7 +55,7 @@ class PagedAttention:
         self.nq, self.nkv, self.d = spec.num_heads, spec.num_kv_heads, spec.head_dim
         self.scale = spec.scale if spec.scale is not None else 1.0 / math.sqrt(spec.head_dim)
         self.window = int(spec.window or 0)
-        # (in bfloat16 the tiled kernel cuts keys into shares by ``StepBatch.near_ctx_len``)
+        # (in bfloat16 ``StepBatch.near_ctx_len`` chooses the kernel, and the tiled one cuts keys into shares by it: a captured step's shape has to name it)
         self.shares_by_near_context = dtype == torch.bfloat16
         # one product for q, k and v: the output row is [q | k | v]
         self.qkv_proj = Linear.fused([params["q_proj.weight"], params["k_proj.weight"], params["v_proj.weight"]],

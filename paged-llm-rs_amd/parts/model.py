@@ -195,8 +195,8 @@ class DecoderModel:
                            and getattr(self.final_transform, "graph_safe", True)
                            and getattr(self.logit_transform, "graph_safe", True))
         self.portion_limits = portion_limits(self.blocks)
-        # Whether some mixer's launches follow how near the step's contexts are (``StepBatch.near_ctx_len``), which is then part of a
-        # captured step's shape.
+        # Whether some mixer's kernels and launches follow how near the step's contexts are (``StepBatch.near_ctx_len``), which is then part of a
+        # captured step's shape.  (A mixer that does and does not say so gets the bound of any context in captured steps.)
         self.shares_by_near_context = any(getattr(getattr(b, "mixer", None), "shares_by_near_context", False) for b in self.blocks)
 
     @property

@@ -153,3 +153,48 @@ def test_only_models_whose_layers_go_by_near_contexts_capture_a_shape_for_each(m
     assert play() == ([100], 1, 11)
     assert play(shares_by_near_context=False) == ([100], 1, 11)
     assert play(shares_by_near_context=True) == ([100, 300, 900], 3, 9)        # (bounds of 128, 512 and 1,024)
+
+
+def test_a_captured_step_is_not_replayed_for_contexts_past_its_near_bound(monkeypatch):
+    """The near bound chooses a kernel that holds no longer contexts.  A model whose layers do not say that they go by it has none in its captured steps; one whose layers do is refused
+    a replay for contexts past the captured ones, whatever the shape says."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from paged_llm_rs_amd.engine import step
+    from paged_llm_rs_amd.engine.batch import CaptureOutgrown, NotNear
+
+    class Ring:
+        def __init__(self, size):
+            self.host = torch.zeros(size, dtype=torch.int32)
+
+        advance = sent = lambda self: None
+
+    monkeypatch.setattr(step, "_DescriptorRing", Ring)
+    replayed = []
+
+    def graph(**model):
+        m = manager(blocks=512)
+        entries = requests(m, [20, 17], written=[30, 0])
+        model = SimpleNamespace(device="cpu", spec=SimpleNamespace(vocab_size=100, max_positions=0), **model)
+        made = step.ShapeGraph(model, SimpleNamespace(manager=m, layout=SimpleNamespace(groups=[0])), entries, [64], 1024, 64, {})
+        made.graph = SimpleNamespace(replay=lambda: replayed.append(made))
+        return made, m
+
+    def longer(m, written):
+        for seq in (1, 2):
+            m.free_sequence(seq)
+        return requests(m, [20, 17], written=[written, 0])
+
+    for flag in ({}, {"shares_by_near_context": False}):
+        made, m = graph(**flag)
+        assert made.batch.near_ctx_len == 1024
+        made.run(longer(m, 200))
+    made, m = graph(shares_by_near_context=True)
+    assert made.batch.near_ctx_len == 128
+    made.run(longer(m, 100))
+    assert len(replayed) == 3
+    with pytest.raises(NotNear):
+        made.run(longer(m, 109))
+    assert issubclass(NotNear, CaptureOutgrown) and len(replayed) == 3
