@@ -1034,10 +1034,10 @@ static int launch_prefill(const void* q, int q_stride, void* out, const int* q_s
     // that take them end late; with the tiles of all of an XCD's heads in order of their lengths what remains gets ever shorter.  (us, before and
     // after, heads of 128: 2,048 tokens of 24 heads 70.0 / 55.3, 32 83.8 / 63.4, 64 142.6 / 120.7, 1,500 of 32 57.5 / 45.8, four prompts of 1,024
     // of 16 57.8 / 45.5, 8,192 of 32 688 / 672.)  More than eight heads an XCD: those of one request at a time, whose keys its L2 holds longer.
-    // Workgroups that a chip of 256 compute units takes all at once have no order to keep.
+    // Workgroups that the compute units take all at once have no order to keep.
     const int units = (GR ? nkv : nq) * num_seqs;
     int meet = 0;
-    if (!GR && !compact && whole > 256 && units % 8 == 0) {
+    if (!GR && !compact && whole > pl_compute_units() && units % 8 == 0) {
         if (units <= 64) meet = units / 8;
         else if (nq % 8 == 0) meet = nq / 8;
     }

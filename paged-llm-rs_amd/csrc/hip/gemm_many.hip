@@ -521,6 +521,11 @@ static int gm_launch(const GmProduct& g, hipStream_t stream) {
 // compute unit (K of 1,024 and of 3,072).  A launch is taken to last as long as the compute unit with most tiles: that is the order of the
 // shapes in all of 40 timed products (65 to 4,096 rows of 1,024, 4,096 and 5,120) but for differences of a few per cent.  (32-bit
 // results of the largest tile would not fit into LDS.)
+//
+// The order is the same for weights in rows, which take more LDS: {2, 3} then has a compute unit to itself, as its 32-bit results have out of strips, where it and the smaller
+// ones are two a unit otherwise.  Over 68 products (65 to 3,072 rows of 1,024 to 4,096, weights from memory) the shape taken lost 0.7% to the fastest on average and 4% at most out
+// of strips, 1.0% and 4% in rows; 32-bit results of very many columns 7% and, past 64 rows in rows, 14% at most (65,536 columns of 2,048, 65 rows out of strips: 60 us, 56 with {1, 4}).
+// More registers for a {2, 3} that is alone changed nothing (29 products within 2.5% either way).
 struct GmShape {
     int ct, rt;
     float stage, tile[5];      // (by epilogue)
