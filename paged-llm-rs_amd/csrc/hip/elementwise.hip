@@ -2,6 +2,7 @@
 // write, SwiGLU.  Statistics, rotation and the residual sum are 32-bit whatever
 // the activation type is; a result is rounded once, when it is stored.
 #include "common.hpp"
+#include "head_rows.hpp"
 
 // ---------------------------------------------------------------------------
 // Embedding: out[t, :] = table[ids[t], :] as the 32-bit residual stream.
@@ -502,23 +503,7 @@ qk_norm_rope_kv_write_wide_kernel(
 
 // Heads of 128 elements that are rotated whole: a head is a row of 16 lanes, so the sum of squares
 // and the exchange with the rotation's partner (8 lanes further on or back) go through the lanes'
-// own data paths (DPP) instead of LDS.  One wave works on four heads of a token, a workgroup on 16.
-__device__ __forceinline__ float qk_dpp_quad_xor1(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));   // quad_perm [1,0,3,2]
-}
-__device__ __forceinline__ float qk_dpp_quad_xor2(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));   // quad_perm [2,3,0,1]
-}
-__device__ __forceinline__ float qk_dpp_half_mirror(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));  // lane i of 8 takes 7-i
-}
-__device__ __forceinline__ float qk_dpp_mirror(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true));  // lane i of 16 takes 15-i
-}
-__device__ __forceinline__ float qk_dpp_ror8(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));  // lane i of 16 takes i^8
-}
-
+// own data paths (DPP; head_rows.hpp) instead of LDS.  One wave works on four heads of a token, a workgroup on 16.
 template <typename T>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_kv_write_128_kernel(
@@ -554,28 +539,8 @@ qk_norm_rope_kv_write_128_kernel(
         qk_vec<float>::load(sin_table + at, sn);
     }
 
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
-    ss += qk_dpp_quad_xor1(ss);
-    ss += qk_dpp_quad_xor2(ss);
-    ss += qk_dpp_half_mirror(ss);
-    ss += qk_dpp_mirror(ss);
     const bool is_v = !is_q && !is_k;
-    if (gain && !is_v) {
-        const float rinv = 1.f / sqrtf(ss / static_cast<float>(D) + eps);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = x[e] * rinv * g[e];
-    }
-    if (cos_table) {
-        float px[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) px[e] = qk_dpp_ror8(x[e]);
-        if (!is_v) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = low ? x[e] * c[e] - px[e] * sn[e] : x[e] * c[e] + px[e] * sn[e];
-        }
-    }
+    hr_norm_turn(x, gain != nullptr && !is_v, g, eps, cos_table != nullptr && !is_v, c, sn, low);
     T* dst = src;
     if (!is_q) {
         const size_t slot = static_cast<size_t>(blk < 0 ? 0 : blk) * block_size + pos % block_size;

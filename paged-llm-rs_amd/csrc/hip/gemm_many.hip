@@ -100,15 +100,6 @@ __device__ __forceinline__ void gm_tile(int at, int row_tiles, int col_tiles, in
     col_tile = in_band / rows;
 }
 
-// The sum over 16 lanes that stand side by side, by each of them.
-__device__ __forceinline__ float gm_sum16(float v) {
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));      // quad_perm [1,0,3,2]
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));      // quad_perm [2,3,0,1]
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));     // lane i of 8 takes 7 - i
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true));     // lane i of 16 takes 15 - i
-    return v;
-}
-
 constexpr int gm_out_cols(int CT, int epi) { return 4 * (epi == GM_SWIGLU ? 16 : 32) * CT; }
 constexpr bool gm_is_32(int epi) { return epi == GM_ADD || epi == GM_STORE32; }
 // bytes between two rows of the tile on its way out
@@ -471,7 +462,7 @@ gemm_many_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ weight
                 const size_t to = static_cast<size_t>(row) * y_pitch + col;
                 if (there) *reinterpret_cast<gm_f32x4*>(static_cast<float*>(y_) + to) = v;
                 if (hands) {
-                    const float square = gm_sum16(there ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f);
+                    const float square = hr_sum16(there ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f);
                     if (there) {
                         const gm_u32x2 packed = {gm_pack2(v[0] * gain[0], v[1] * gain[1]), gm_pack2(v[2] * gain[2], v[3] * gain[3])};
                         *reinterpret_cast<gm_u32x2*>(norms.rows + to) = packed;
