@@ -885,8 +885,10 @@ def near_applies(batch, nq: int, d: int, window: int, prepare: QkFusion) -> bool
 
 
 def prepares_whole_heads(d: int, prepare: QkFusion) -> bool:
-    """Heads of 128 rotated whole, by halves, or not at all, whose keys and values go into the pages."""
-    return d == NEAR_HEAD and prepare.rot in (0, d) and not prepare.neighbours and prepare.write_kv
+    """Heads of 128 rotated whole, by halves, or not at all, whose keys and values go into the pages.  Tables of another width than the rotation's, or one without the other, are
+    left to the stand-alone kernel, which says what it takes of them."""
+    return (d == NEAR_HEAD and prepare.rot in (0, d) and not prepare.neighbours and prepare.write_kv
+            and (prepare.cos is None) == (prepare.sin is None) and (prepare.cos is None or prepare.rot == d))
 
 
 def _heads_code(kv, nkv: int, prepare: QkFusion) -> int:

@@ -143,3 +143,14 @@ def test_near_contexts_go_to_one_kernel_while_the_workgroups_are_few():
     assert takes(4, 64, longest=1) and not takes(5, 64, longest=1) and not takes(8, 64, longest=1)
     assert takes(17, 32, live_seqs=16) and not takes(1, 16, near=256) and not takes(1, 16, near=None) and not takes(1, 16, window=64) and not takes(1, 16, d=64)
     assert not takes(1, 16, prepare=kernels.QkFusion(None, None, 1e-6, None, None, 64, True)) and not takes(1, 16, prepare=kernels.QkFusion(None, None, 1e-6, None, None, 128, False))
+
+
+def test_tables_that_are_not_the_rotations_go_to_the_kernel_that_says_so():
+    """Tables beside a rotation over nothing were refused, or ignored where they are empty, and one table without the other was ignored or refused: by the stand-alone kernel, as now."""
+    table, empty = torch.zeros(128, 64), torch.zeros(128, 0)
+
+    def whole(cos, sin, rot):
+        return kernels.prepares_whole_heads(128, kernels.QkFusion(None, None, 1e-6, cos, sin, rot, True))
+
+    assert whole(table, table, 128) and whole(None, None, 128) and whole(None, None, 0)
+    assert not whole(table, table, 0) and not whole(empty, empty, 0) and not whole(table, None, 128) and not whole(None, table, 128) and not whole(table, table, 64)
