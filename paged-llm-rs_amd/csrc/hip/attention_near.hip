@@ -8,13 +8,13 @@
 // keys of a step of the second in the order in which a lane holds them.  Every query head prepares its key head's keys again; the first of a group
 // writes them.
 //
-// A weight of zero does not hide an infinite or NaN value, and the second product multiplies a tile's tokens with keys behind them.  Such values are taken out of
-// LDS as they are laid there and added value by value to the tokens that see their key, so a token is what it is with only the keys up to itself.
+// A weight of zero does not hide an infinite or NaN value, and the second product multiplies a tile's tokens with keys behind them: what comes out is then not finite, which is what a
+// wave looks for.  It then takes the product again without such values and adds them value by value to the tokens that see their key, so a token is what it is with only the keys up to itself.
 //
 // Bound by its chain of trips (the request's numbers and pages; its rows) and the arithmetic of preparing rows, a vector instruction a wave every 4 to 5
-// cycles.  us, the two kernels before / this one, 16 heads over 8: 37 fresh tokens 12.1 / 8.9, 128 16.7 / 14.2, eight requests of 10 17.6 / 7.3,
-// 10 tokens behind 110 12.6 / 11.0; 64 heads over 8: 37 fresh tokens 12.3 / 9.1, eight requests of 10 20.9 / 12.2.  (0.2 to 0.4 of it look for values that are
-// not finite.)
+// cycles.  us, a hundred in a row in a captured graph, the two kernels before / this one, 16 heads over 8: 37 fresh tokens 10.4 / 7.3, 128 15.1 / 12.7, eight requests of
+// 10 15.6 / 5.6, 10 tokens behind 110 10.8 / 9.3; 64 heads over 8: 37 fresh tokens 10.6 / 7.4, eight requests of 10 19.1 / 10.1.  (0.1 to 0.2 of it look whether the result is
+// finite; looking through the values as they are laid in LDS took 0.2 to 0.4.)
 #include "common.hpp"
 #include "head_rows.hpp"
 
@@ -26,9 +26,6 @@ typedef uint32_t an_u32x2 __attribute__((ext_vector_type(2)));
 #define AN_KEYS 128                // of a context, at most
 #define AN_D 128
 #define AN_V_PITCH (AN_KEYS * 2 + 8)   // bytes between two columns of values
-#define AN_V_END (2 * AN_KEYS * 256 + AN_D * AN_V_PITCH)
-
-typedef uint16_t an_u16x2 __attribute__((ext_vector_type(2)));
 
 // Whether a value, its low 16 bits, is infinite or NaN.
 __device__ __forceinline__ bool an_wild(uint32_t value) { return (value & 0x7f80u) == 0x7f80u; }
@@ -43,7 +40,6 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
     char* const q_lds = an_lds;                                        // [token][128]
     char* const k_lds = an_lds + AN_KEYS * 256;                        // [key][128]
     char* const v_lds = an_lds + 2 * AN_KEYS * 256;                    // [column][key]
-    uint32_t* const wild_lds = reinterpret_cast<uint32_t*>(an_lds + AN_V_END);     // [wave]: its eight keys of either half with values that are not finite
     const int seq = blockIdx.x, head = blockIdx.y, group = nq / nkv, kvh = head / group;
     const int tid = threadIdx.x, lane = tid % PL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / PL_WAVE);
     const int chunk = tid % 16, slot = tid / 16;                       // eight values of one of 32 rows
@@ -130,31 +126,6 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
         if (key < start && at >= 0) k = *reinterpret_cast<const an_u32x4*>(k_pool + (static_cast<size_t>(at) * nkv + kvh) * AN_D + chunk * 8);
         if (key < start) *reinterpret_cast<an_u32x4*>(k_lds + key * 256 + (chunk ^ (key % 16)) * 16) = k;
     }
-    // values that are not finite: mostly there are none, as the largest of a lane's without their signs says
-    an_u16x2 largest = {0, 0};
-#pragma unroll
-    for (int w = 0; w < 2; ++w)
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(an_u16x2, v[w][u][e] & 0x7fff7fffu));
-    const bool has_wild = __ballot(largest[0] >= 0x7f80u || largest[1] >= 0x7f80u) != 0;        // (of the wave)
-    uint32_t wild = 0;
-    if (has_wild) {
-#pragma unroll
-        for (int w = 0; w < 2; ++w)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                bool mine = false;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) mine = mine || an_wild(v[w][u][e]) || an_wild(v[w][u][e] >> 16);
-                const unsigned long long lanes = __ballot(mine);
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (lanes >> (16 * j) & 0xffffu) wild |= 1u << (8 * w + 2 * j + u);
-            }
-    }
-    if (lane == 0) wild_lds[wave] = wild;
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
         const int pair = slot + 32 * w;
@@ -164,15 +135,6 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
             if (writes && key >= start && at >= 0) *reinterpret_cast<an_u32x4*>(v_pool + (static_cast<size_t>(at) * nkv + kvh) * AN_D + chunk * 8) = v[w][u];
         }
         if (pair >= key_tiles * 16) continue;
-        if (has_wild) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (an_wild(v[w][u][e])) v[w][u][e] &= 0xffff0000u;
-                    if (an_wild(v[w][u][e] >> 16)) v[w][u][e] &= 0xffffu;
-                }
-        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const uint32_t a = e % 2 ? v[w][0][e / 2] >> 16 : v[w][0][e / 2] & 0xffffu, b = e % 2 ? v[w][1][e / 2] >> 16 : v[w][1][e / 2] & 0xffffu;
@@ -180,7 +142,6 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
         }
     }
     __syncthreads();
-    const uint32_t told = wild_lds[lane % 8];
 
     // a wave's 32 tokens and columns: two tiles of tokens by four of columns, or four by two pairs
     const bool many = count > 64;
@@ -232,16 +193,6 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
         }
     }
     sum += __shfl_xor(sum, 32, PL_WAVE);
-    unsigned long long wild0 = 0, wild1 = 0;                           // one bit a key, as `there0` and `there1`
-    const bool any_wild = __ballot(told != 0) != 0;
-    if (any_wild) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t of = __shfl(told, i, PL_WAVE);
-            wild0 |= static_cast<unsigned long long>(of & 0xffu) << (8 * i);
-            wild1 |= static_cast<unsigned long long>(of >> 8 & 0xffu) << (8 * i);
-        }
-    }
     const float by = sum > 0.f || sum != sum ? 1.f / sum : 0.f;
     for (int d = many ? wave % 2 * 2 : wave % 4, last = many ? d + 2 : d + 1; d < last; ++d) {
         an_f32x16 o;
@@ -258,26 +209,52 @@ attention_near_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ out, 
                 o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(an_bf16x8, an_u32x4{a[0], a[1], b[0], b[1]}), p[kt][u], o, 0, 0, 0);
             }
         }
-        // the values that were taken out, key by key, by the tokens that see it
-        for (int half = 0; any_wild && half < 2; ++half)
-            for (unsigned long long left = half == 0 ? wild0 : wild1; left != 0; left &= left - 1) {
-                const int key = 64 * half + __ffsll(left) - 1, of = key % 32;
-                float weight = 0.f;                                    // (held by one of the token's two lanes)
+        // values that are not finite: taken out, and added key by key by the tokens that see it
+        float finite = 0.f;                                            // (or NaN)
 #pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
+        for (int i = 0; i < 16; ++i) finite = fmaf(o[i], 0.f, finite);
+        if (__ballot(token < count && finite != finite) != 0) {
+            unsigned long long wild[2] = {0, 0};                       // one bit a key, as `there0` and `there1`
 #pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        if (kt < seen_tiles && kt == key / 32 && 8 * (i / 4) + 4 * h + i % 4 == of) weight = s[kt][i];
-                weight += __shfl_xor(weight, 32, PL_WAVE);
-                const int at = place(key);
-                const bf16_t* from = key >= start ? qkv + (row0 + key - start) * stride + static_cast<size_t>(nq + nkv + kvh) * AN_D
-                                                  : v_pool + (static_cast<size_t>(max(at, 0)) * nkv + kvh) * AN_D;
+            for (int i = 0; i < 16; ++i) o[i] = 0.f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t value = reinterpret_cast<const uint16_t*>(from)[d * 32 + 8 * (i / 4) + 4 * h + i % 4];
-                    if (key <= pos && an_wild(value)) o[i] += weight * __uint_as_float(value << 16);
+            for (int kt = 0; kt < 4; ++kt) {
+                if (kt >= seen_tiles) continue;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const char* from = v_lds + (d * 32 + r32) * AN_V_PITCH + (kt * 32 + u * 16 + 4 * h) * 2;
+                    const an_u32x2 a = *reinterpret_cast<const an_u32x2*>(from), b = *reinterpret_cast<const an_u32x2*>(from + 16);
+                    an_u32x4 kept = {a[0], a[1], b[0], b[1]};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {                      // (both halves of the wave: keys 4 apart)
+                        const bool mine = an_wild(kept[e / 2] >> (e % 2 * 16));
+                        const unsigned long long lanes = __ballot(mine);
+                        const int key = kt % 2 * 32 + u * 16 + e / 4 * 8 + e % 4;
+                        if (lanes & 0xffffffffull) wild[kt / 2] |= 1ull << key;
+                        if (lanes >> 32) wild[kt / 2] |= 1ull << (key + 4);
+                        if (mine) kept[e / 2] &= e % 2 ? 0xffffu : 0xffff0000u;
+                    }
+                    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(an_bf16x8, kept), p[kt][u], o, 0, 0, 0);
                 }
             }
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+                for (unsigned long long left = wild[half]; left != 0; left &= left - 1) {
+                    const int key = 64 * half + __ffsll(left) - 1, of = key % 32;
+                    float weight = 0.f;                                // (held by one of the token's two lanes)
+#pragma unroll
+                    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i)
+                            if (kt < seen_tiles && kt == key / 32 && 8 * (i / 4) + 4 * h + i % 4 == of) weight = s[kt][i];
+                    weight += __shfl_xor(weight, 32, PL_WAVE);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const uint32_t value = *reinterpret_cast<const uint16_t*>(v_lds + (d * 32 + 8 * (i / 4) + 4 * h + i % 4) * AN_V_PITCH + key * 2);
+                        if (key <= pos && an_wild(value)) o[i] += weight * __uint_as_float(value << 16);
+                    }
+                }
+        }
         if (token < count) {
             bf16_t* to = out + static_cast<size_t>(row0 + token) * nq * AN_D + head * AN_D + d * 32 + 4 * h;
 #pragma unroll
@@ -298,7 +275,7 @@ extern "C" int pl_attention_near(const void* qkv, void* out, const void* q_gain,
     PL_REQUIRE((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool) |
                 reinterpret_cast<uintptr_t>(cos_table) | reinterpret_cast<uintptr_t>(sin_table) | reinterpret_cast<uintptr_t>(q_gain) | reinterpret_cast<uintptr_t>(k_gain)) % 16 == 0, "near attention: rows that are not aligned to 16 bytes");
     if (num_seqs == 0) return 0;
-    constexpr int lds = AN_V_END + 8 * 4;
+    constexpr int lds = 2 * AN_KEYS * 256 + AN_D * AN_V_PITCH;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_near_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     PL_REQUIRE(e == hipSuccess, "near attention: %d bytes of LDS refused: %s", lds, hipGetErrorString(e));
     attention_near_kernel<<<dim3(num_seqs, nq), 512, lds, stream>>>(

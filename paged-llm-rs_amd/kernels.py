@@ -868,10 +868,10 @@ def prefill_splits(requests: int, max_q_len: int, nq: int, d: int, max_ctx: int,
 
 
 # A step whose contexts are all as near as one workgroup holds them runs preparation and attention as one kernel, a workgroup a request and query head,
-# while those are no more than two a compute unit; beyond, requests of a token or two keep a workgroup each for little (us, two kernels / one: 32 heads, 8
-# requests of 10 tokens at 120 20.3 / 12.0, 16 28 / 21, 32 48 / 40, but one of 40 beside 31 single tokens 27.4 / 27.9, beside 63 24.8 / 50.3).  So do steps of single tokens alone, which come
-# here where eight query heads and more share a key head: no more than one a compute unit (64 heads over 8: one token at 40 15.6 / 8.4, four at 120 16.0 / 11.5, eight 18.1 / 20.7; two
-# of three tokens at 100 17.9 / 11.1, eight 19.2 / 20.0).
+# while those are no more than two a compute unit; beyond, requests of a token or two keep a workgroup each for little (us, two kernels / one, in a captured graph: 32
+# heads, 8 requests of 10 tokens at 120 17.2 / 9.5, 16 24.4 / 18.0, 32 41.9 / 34.1, but one of 40 beside 31 single tokens 26.5 / 38.0, beside 63 27.4 / 72.5).  So do steps of single tokens alone,
+# which come here where eight query heads and more share a key head: no more than one a compute unit (64 heads over 8: one token at 40 14.0 / 6.6, four at 120 14.5 / 9.4, eight
+# 16.0 / 17.5; two of three tokens at 100 16.1 / 9.2, eight 17.5 / 17.6).
 NEAR_KEYS = 128
 NEAR_HEAD = 128
 NEAR_WORKGROUPS = 512
