@@ -1325,9 +1325,11 @@ def many_tiles(rows: int, columns: int) -> int:
 # wins at all of them (151,936 columns of 1,024: 17 rows 68 / 61, 64 82 / 71, 128 96 / 90; of 4,096: 24 rows 251 / 235, 64 276 / 250, 128 296 / 281; 200,064 of 3,072: 64 rows
 # 293 / 264; 100,352 of 1,536: 48 rows 137 / 75; 32,768 of 1,024: 32 rows 48 / 16), in rows a little less and up to 64 of them (151,936 of 1,024: 17 rows 67 / 66; 65,536 of 2,048: 64
 # 122 / 79, 65 76 / 79, 128 83 / 86; 200,064 of 3,072: 128 rows 305 / 315).  Beyond 128 rows its third tile of them is paid by the columns, and it wins at some vocabularies and loses at
-# others (160 rows: 65,536 of 2,048 85 / 76, 151,936 of 4,096 319 / 337, 200,064 of 3,072 329 / 351).  With fewer than 17 neither the width nor the size alone says which
-# is the faster, and it is mostly a few per cent (over 104 vocabularies of 512 to 2,048; 1 row: 151,936 columns of 1,024 57 / 54, 65,536 of 896 22.9 / 26.5, 100,352 of 1,024 39 / 41; 8 rows: 151,936 of
-# 1,024 62 / 57, 49,152 of 1,024 21.8 / 21.8, 128,256 of 768 39 / 42; of 4,096, 151,936 columns 219 / 223, 32,768 55 / 50).
+# others (160 rows: 65,536 of 2,048 85 / 76, 151,936 of 4,096 319 / 337, 200,064 of 3,072 329 / 351).
+# With fewer than 17 every row adds to the kernel for few rows, whose waves lay their shares of it together, and none to this one, whose tile is 64 rows anyway: out of strips, over 226 vocabularies (16
+# widths of 512 to 3,072, 19 counts of 32,768 to 262,144 columns), it takes 1.02 times the other's time at 1 row from a width of 1,024 on (geometric mean; 1.14 at worst), 0.94 (1.06) at 8 and 0.89 (1.00)
+# at 16; at narrower ones 1.10, 1.02 and 0.96 (1.08); wider ones lose (200,064 of 4,096: 8 rows 276 / 307).  But in rows it loses there too (8 rows: 151,936 of 1,024 58 / 58, 128,256 of 1,024 49 / 51, 65,536 of 2,048
+# 49 / 69), and the two sum in different orders: a rule that asks for strips would give steps of few rows other bits by how the weights lie, which so far they have not.  They stay with the kernel for few rows.
 MANY_VOCABULARY = 32768
 MANY_VOCABULARY_FROM_ROWS = 17
 MANY_VOCABULARY_ROWS = {True: 128, False: 64}         # at most, out of strips and in rows
