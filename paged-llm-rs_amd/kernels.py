@@ -1328,7 +1328,7 @@ def many_tiles(rows: int, columns: int) -> int:
 # others (160 rows: 65,536 of 2,048 85 / 76, 151,936 of 4,096 319 / 337, 200,064 of 3,072 329 / 351).
 # With fewer than 17 every row adds to the kernel for few rows, whose waves lay their shares of it together, and none to this one, whose tile is 64 rows anyway: out of strips, over 226 vocabularies (16
 # widths of 512 to 3,072, 19 counts of 32,768 to 262,144 columns), it takes 1.02 times the other's time at 1 row from a width of 1,024 on (geometric mean; 1.14 at worst), 0.94 (1.06) at 8 and 0.89 (1.00)
-# at 16; at narrower ones 1.10, 1.02 and 0.96 (1.08); wider ones lose (200,064 of 4,096: 8 rows 276 / 307).  But in rows it loses there too (8 rows: 151,936 of 1,024 58 / 58, 128,256 of 1,024 49 / 51, 65,536 of 2,048
+# at 16; at narrower ones 1.10, 1.02 and 0.96 (1.08); wider ones lose (200,064 of 4,096: 8 rows 276 / 307).  But in rows it loses there too (8 rows: 151,936 of 1,024 59 / 58, 128,256 of 1,024 49 / 51, 65,536 of 2,048
 # 49 / 69), and the two sum in different orders: a rule that asks for strips would give steps of few rows other bits by how the weights lie, which so far they have not.  They stay with the kernel for few rows.
 MANY_VOCABULARY = 32768
 MANY_VOCABULARY_FROM_ROWS = 17
