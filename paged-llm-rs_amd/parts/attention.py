@@ -85,21 +85,7 @@ class PagedAttention:
     def forward(self, x, ctx):
         """``x``: normalised rows, or a PendingNorm.  Where ``ctx.residual`` is given and the output
         projection can add into it, None comes back."""
-        batch = ctx.batch
-        kv = ctx.kv()
-        prepare = self._prepare(ctx.writes_cache)
-        # (many rows: the projection may do what stands between it and attention, unless one kernel does that and the attention)
-        qkv = None
-        if (ctx.trace is None and batch.max_q_len > 1 and kernels.prepares_whole_heads(self.d, prepare)
-                and not kernels.near_applies(batch, self.nq, self.d, self.window, prepare)):
-            qkv = self.qkv_proj.forward_heads(x, batch, kv, self.nq, self.nkv, prepare)
-        prepared = qkv is not None
-        if not prepared:
-            qkv = self.qkv_proj.forward(x)
-        out = torch.empty((qkv.shape[0], self.nq * self.d), dtype=qkv.dtype, device=qkv.device)
-        if ctx.trace is not None:
-            self._record_projections(qkv, batch, kv, ctx.trace)
-        kernels.attention_step(qkv, out, batch, kv, self.nq, self.nkv, self.d, self.scale, self.window, prepare, prepared=prepared)
+        out = self.attend(x, ctx)
         if ctx.trace is not None:
             ctx.trace.record("o_proj.in", out)
             out = self.o_proj.forward(out)
@@ -107,6 +93,31 @@ class PagedAttention:
             return out
         return self.o_proj.forward(out, add_into=ctx.residual,
                                    hand=getattr(ctx, "hand", None) if ctx.residual is not None else None)
+
+    def attend(self, x, ctx, projected=None):
+        """Everything before the output projection.  ``projected``: the rows of q, k and v, where the layer before has worked them out."""
+        batch = ctx.batch
+        kv = ctx.kv()
+        prepare = self._prepare(ctx.writes_cache)
+        # (many rows: the projection may do what stands between it and attention, unless one kernel does that and the attention)
+        qkv = None
+        if (projected is None and ctx.trace is None and batch.max_q_len > 1 and kernels.prepares_whole_heads(self.d, prepare)
+                and not kernels.near_applies(batch, self.nq, self.d, self.window, prepare)):
+            qkv = self.qkv_proj.forward_heads(x, batch, kv, self.nq, self.nkv, prepare)
+        prepared = qkv is not None
+        if not prepared:
+            qkv = projected if projected is not None else self.qkv_proj.forward(x)
+        out = torch.empty((qkv.shape[0], self.nq * self.d), dtype=qkv.dtype, device=qkv.device)
+        if ctx.trace is not None:
+            self._record_projections(qkv, batch, kv, ctx.trace)
+        kernels.attention_step(qkv, out, batch, kv, self.nq, self.nkv, self.d, self.scale, self.window, prepare, prepared=prepared)
+        return out
+
+    @property
+    def chain_products(self):
+        """(first projection, output projection) of a mixer whose middle is ``attend``: what stands behind it may run in one launch with the
+        products around it (``kernels.gemm_chain``).  None for a class with a ``forward`` of its own."""
+        return (self.qkv_proj, self.o_proj) if type(self).forward is PagedAttention.forward else None
 
     def _prepare(self, writes_cache: bool):
         cos = self.rotary.cos if self.rotary is not None else None

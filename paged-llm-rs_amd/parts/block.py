@@ -82,11 +82,40 @@ class PreNormBlock:
             return None
         return make(rows, resid.device)
 
+    @property
+    def chain_sizes(self):
+        """(stream, output projection's inner width, feed-forward, first projection's columns) of a layer whose products may run as one launch a
+        layer (``kernels.gemm_chain``), or None: attention and a gated feed-forward without biases, norms that products take as their first stage,
+        bfloat16 weights in strips."""
+        ours, theirs = getattr(self.mixer, "chain_products", None), getattr(self.feed_forward, "chain_products", None)
+        if self.dtype != torch.bfloat16 or ours is None or theirs is None or type(self).forward is not PreNormBlock.forward:
+            return None
+        if not all(getattr(n, "fuses_into_product", False) for n in (self.norm1, self.norm2)):
+            return None
+        linears = (*ours, *theirs[:2])
+        if any(l.bias is not None or l.strips is None for l in linears) or not kernels.in_pieces(
+                *(l.strips for l in linears), self.norm1.gain32, self.norm2.gain32):
+            return None
+        first, out = ours
+        return out.out_features, out.in_features, theirs[1].in_features, first.out_features
+
+    def _forward_chained(self, resid, delta, ctx):
+        """The layer as two parts: what stands before the output projection, and one launch from there to the next layer's first projection."""
+        chain, x = ctx.chain, None
+        if chain.projected is None:
+            x = PendingNorm(self.norm1, resid, self.dtype) if delta is None else self.norm1.apply(resid, delta, self.dtype)
+        rows = self.mixer.attend(x, ctx, projected=chain.projected)
+        gate_up, down, activation = self.feed_forward.chain_products
+        chain.run(resid, rows, self.mixer.chain_products[1].strips, gate_up.strips, down.strips, self.norm2, activation)
+        return None
+
     def forward(self, resid, delta, ctx):
         """``delta``: what the block before has not added to the stream yet, or None.  Returns this
         block's own unadded output, or None when the feed-forward added it itself."""
         if ctx.trace is not None:
             return self._forward_recorded(resid, delta, ctx)
+        if getattr(ctx, "chain", None) is not None:
+            return self._forward_chained(resid, delta, ctx)
         mixer_fuses = getattr(self.mixer, "fuses", False)
         ffn_fuses = getattr(self.feed_forward, "fuses", False)
         half = self.dtype == torch.bfloat16

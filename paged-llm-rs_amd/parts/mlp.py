@@ -60,6 +60,13 @@ class GatedMlp:
             return out
         return self.finish(self.begin(x), residual=residual, hand=hand, out_dtype=out_dtype)
 
+    @property
+    def chain_products(self):
+        """(gate and up, down, activation): all there is of this feed-forward, for a launch that runs it beside other products.
+        None for a class with a ``forward``, ``begin`` or ``finish`` of its own."""
+        own = all(getattr(type(self), name) is getattr(GatedMlp, name) for name in ("forward", "begin", "finish"))
+        return (self.gate_up_proj, self.down_proj, self.activation) if own else None
+
     def takes_norm(self, rows: int, batch) -> bool:
         """Whether the norm in front of this feed-forward, of many rows, is worth leaving to its first product."""
         return self.gate_up_proj.takes_norm(rows, swiglu=True, activation=self.activation)

@@ -106,7 +106,7 @@ class LayerContext:
     the pages of the layer it reads from) and its state slots."""
 
     __slots__ = ("batch", "cache", "layer", "cache_layer", "writes_cache", "residual", "trace", "hand", "handed",
-                 "norm_after", "taker_after", "handed_out", "stream_rows", "stream_addend", "carried")
+                 "norm_after", "taker_after", "handed_out", "stream_rows", "stream_addend", "carried", "chain")
 
     def __init__(self, batch, cache, layer: int, cache_layer: int, writes_cache: bool):
         # ``layer`` and ``cache_layer`` are the keys under which the cache keeps this run's state and the pages it
@@ -141,6 +141,8 @@ class LayerContext:
         # What one layer of a pass leaves for later layers of the same pass, by name (the values that later layers mix
         # into theirs, say): one dict for all runs of a pass, empty at its start.
         self.carried: dict = {}
+        # a ``Chain`` for a block that runs the products behind its attention as one launch in this step; None otherwise
+        self.chain = None
 
     def kv(self):
         return self.cache.layer_view(self.cache_layer, self.batch)
@@ -148,6 +150,25 @@ class LayerContext:
     def state(self):
         """[slots, ...] state tensor of this layer; ``batch.state_slots`` says which slot each request has."""
         return self.cache.layer_state(self.layer)
+
+
+class Chain:
+    """One layer's launch of the products behind its attention, and what it passes on: the updated stream (a tensor of its own, which only the next
+    chain can read where there is a ``following`` layer: (norm, first projection)), and that layer's first projection.
+    ``projected`` and ``laid`` say what the layer before left of this kind."""
+
+    __slots__ = ("room", "following", "projected", "laid", "stream", "passed")
+
+    def __init__(self, room, following, before):
+        self.room, self.following = room, following
+        self.projected = before.passed if before is not None else None
+        self.laid = before is not None and before.following is not None
+        self.stream = self.passed = None
+
+    def run(self, stream, rows, w_out, w_gated, w_down, norm, activation: str) -> None:
+        following = None if self.following is None else (self.following[1].strips, self.following[0].gain32, self.following[0].eps)
+        self.stream, self.passed = kernels.gemm_chain(stream, self.laid, rows, self.room, w_out, w_gated, w_down, norm.gain32, norm.eps, activation,
+                                                      following)
 
 
 class DecoderModel:
@@ -218,6 +239,25 @@ class DecoderModel:
                     strips += t.numel() * t.element_size()
         return stored, strips
 
+    def _chains(self, rows: int) -> dict:
+        """{place in the schedule: (room for its chain of products, (norm, first projection) of the layer behind it or None)} of a step of ``rows``."""
+        if rows > kernels.CHAIN_ROWS:
+            return {}
+        schedule = self.spec.schedule
+        sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
+        places = [at for at, s in enumerate(sizes) if s is not None and kernels.chain_applies(rows, *s[:3])]
+        if not places:
+            return {}
+        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2]) for at in places], self.device)
+        found = {}
+        for at, layer_room in zip(places, room.layers):
+            behind = None
+            if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3]):
+                block = self.blocks[schedule[at + 1].layer]
+                behind = block.norm1, block.mixer.chain_products[0]
+            found[at] = layer_room, behind
+        return found
+
     # -- the forward pass of one step -------------------------------------------------
 
     def forward(self, batch, cache, trace: dict | None = None) -> torch.Tensor:
@@ -248,6 +288,8 @@ class DecoderModel:
         schedule = self.spec.schedule
         # (kept only where a run of the schedule adds it to the stream again)
         began_with = resid.clone() if any(e.add_embedding for e in schedule) else None
+        chains = self._chains(resid.shape[0]) if trace is None else {}
+        chain = None
         for at, entry in enumerate(schedule):
             own = entry.cache_from is None
             key = entry.layer if entry.cache_key is None else entry.cache_key
@@ -276,7 +318,10 @@ class DecoderModel:
             if at + 1 < len(schedule):
                 behind = self.blocks[schedule[at + 1].layer]
                 ctx.norm_after, ctx.taker_after = getattr(behind, "first_norm", None), getattr(behind, "first_taker", None)
+            chain = ctx.chain = Chain(*chains[at], chain) if at in chains else None
             delta = self.blocks[entry.layer].forward(resid, delta, ctx)
+            if chain is not None:
+                resid = chain.stream
             handed = ctx.handed_out if delta is None else None
             stream_rows = ctx.stream_rows if delta is None else None
             if top is not None:

@@ -1,0 +1,102 @@
+"""The launch that runs the products behind a layer's attention, against the same products a launch each: the same bits, whether
+every workgroup finds its rows in time or has to work them out itself."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _operands(n, width, inner, ff, after):
+    g = torch.Generator(device=DEV).manual_seed(n * 7919 + width + inner + ff + after)
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=g, device=DEV)
+
+    weights = [(draw(rows, cols) * cols ** -0.5).bfloat16() for rows, cols in ((width, inner), (2 * ff, width), (width, ff), (after or 16, width))]
+    gains = [1 + 0.1 * draw(width) for _ in range(2)]
+    return draw(n, width), draw(n, inner).bfloat16(), weights, gains
+
+
+def _apart(stream, rows, weights, strips, gains, activation):
+    from paged_llm_rs_amd import kernels
+
+    stream = stream.clone()
+    kernels.gemm_skinny(rows, weights[0], add_into=stream, strips=strips[0])
+    hidden = kernels.gemm_skinny(stream, weights[1], swiglu=True, norm_gain=gains[0], eps=1e-6, activation=activation, strips=strips[1])
+    kernels.gemm_skinny(hidden, weights[2], add_into=stream, strips=strips[2])
+    return stream, kernels.gemm_skinny(stream, weights[3], norm_gain=gains[1], eps=1e-5, strips=strips[3])
+
+
+# Inner widths of 1 to 96 K steps, at the edges where the stretches of K change (32 and 33, 64 and 65 steps); few columns and many.
+@pytest.mark.parametrize("looks", [None, 0])
+@pytest.mark.parametrize("n,width,inner,ff,after", [
+    (1, 1024, 2048, 3072, 4096), (8, 1024, 2048, 3072, 4096), (15, 1024, 2048, 3072, 4096), (3, 32, 32, 32, 16), (15, 64, 1024, 1056, 80),
+    (2, 992, 2080, 2048, 48), (7, 512, 3072, 1088, 0), (13, 96, 3040, 64, 112)])
+def test_a_chain_gives_the_bits_of_its_products(n, width, inner, ff, after, looks):
+    from paged_llm_rs_amd import kernels
+
+    activation = "silu" if n % 2 else "gelu_tanh"
+    stream, rows, weights, gains = _operands(n, width, inner, ff, after)
+    strips = [kernels.weights_in_strips(w) for w in weights]
+    assert kernels.chain_applies(n, width, inner, ff, after)
+    room = kernels.ChainRoom(n, [(width, ff)] * 3, DEV)
+    following = (strips[3], gains[1], 1e-5) if after else None
+    want = got = stream
+    laid = False
+    for layer in room.layers:
+        before = got.clone()
+        apart = _apart(want, rows, weights, strips, gains, activation)
+        chain = kernels.gemm_chain(got, laid, rows, layer, strips[0], strips[1], strips[2], gains[0], 1e-6, activation, following, looks=looks)
+        assert torch.equal(got, before), "the stream that goes in stays as it is"
+        (want, projected), got, laid = apart, chain[0], bool(after)
+        if after:
+            assert torch.equal(chain[1], projected)
+        else:
+            assert torch.equal(got, want)
+    assert torch.isfinite(want).all()
+    # (without a projection behind it, a chain leaves its stream in rows)
+    last = kernels.ChainRoom(n, [(width, ff)], DEV).layers[0]
+    got, none = kernels.gemm_chain(got, laid, rows, last, strips[0], strips[1], strips[2], gains[0], 1e-6, activation, looks=looks)
+    assert none is None and torch.equal(got, _apart(want, rows, weights, strips, gains, activation)[0])
+
+
+def test_values_that_are_not_finite_stay_in_their_rows():
+    """All ones is how a stage sees that a value is not there; a NaN of these bits among the inputs, and infinities in the weights past a
+    stretch's end, change neither another row nor whether the chain ends."""
+    from paged_llm_rs_amd import kernels
+
+    n, width, inner, ff = 5, 96, 1056, 96
+    stream, rows, weights, gains = _operands(n, width, inner, ff, 48)
+    clean = _apart(stream, rows, weights, [kernels.weights_in_strips(w) for w in weights], gains, "silu")
+    stream.view(torch.int32)[1, 3] = -1
+    rows.view(torch.int16)[3, 10] = -1
+    weights[3][5, 7] = float("inf")
+    strips = [kernels.weights_in_strips(w) for w in weights]
+    want = _apart(stream, rows, weights, strips, gains, "silu")
+    for looks in (None, 0):
+        got = kernels.gemm_chain(stream, False, rows, kernels.ChainRoom(n, [(width, ff)], DEV).layers[0], strips[0], strips[1], strips[2], gains[0], 1e-6,
+                                 "silu", (strips[3], gains[1], 1e-5), looks=looks)[1]
+        assert torch.equal(torch.isnan(got), torch.isnan(want[1]))
+        assert torch.equal(got.nan_to_num(0.0), want[1].nan_to_num(0.0))
+    assert torch.isnan(want[1]).all(dim=1).tolist() == [False, True, False, True, False]
+    assert torch.isinf(want[1][[0, 2, 4], 5]).all() and torch.isfinite(clean[1]).all()
+
+
+def test_what_a_chain_does_not_take_is_refused():
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.errors import TensorError
+
+    for shape in ((16, 1024, 2048, 3072, 0), (0, 1024, 2048, 3072, 0), (1, 1056, 2048, 3072, 0), (1, 1024, 3104, 3072, 0), (1, 1024, 2048, 3104, 0),
+                  (1, 1000, 2048, 3072, 0), (1, 1024, 2040, 3072, 0), (1, 1024, 2048, 3072, 8)):
+        assert not kernels.chain_applies(*shape)
+    stream, rows, weights, gains = _operands(16, 64, 64, 64, 16)
+    strips = [kernels.weights_in_strips(w) for w in weights]
+    with pytest.raises(TensorError, match="16 rows"):
+        kernels.gemm_chain(stream, False, rows, kernels.ChainRoom(16, [(64, 64)], DEV).layers[0], strips[0], strips[1], strips[2], gains[0], 1e-6, "silu")
+    with pytest.raises(TensorError, match="strips"):
+        kernels.gemm_chain(stream[:2], False, rows[:2], kernels.ChainRoom(2, [(64, 64)], DEV).layers[0], strips[0][:32], strips[1], strips[2], gains[0], 1e-6, "silu")
