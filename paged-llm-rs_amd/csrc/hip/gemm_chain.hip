@@ -1,4 +1,4 @@
-// The products behind a layer's attention for few rows (n <= 15), bfloat16 weights in strips, as ONE launch:
+// The products behind a layer's attention for few rows (n <= 64), bfloat16 weights in strips, as ONE launch:
 //
 //   stage 0  mid    = stream + rows . w_out^T                 (the mixer's output projection)
 //   stage 1  hidden = act(norm2(mid) . gate^T) * (norm2(mid) . up^T)
@@ -9,15 +9,18 @@
 // 0.8 to 2.3 us): the boundary between two kernels, weights that are asked for only then, and the drain.  Here the
 // workgroups of all stages are in one grid, 16 columns each.  A workgroup asks for its weights first, into registers, and
 // then looks for its input; so the weights of a stage travel while the stages before it work, and what is left between
-// two stages is one trip of the rows through memory.  Four products of the 0.6B shape, 28 layers, weights from memory, us
-// a layer, four launches / one: 1 row 20.8 / 14.7, 8 rows 22.9 / 15.6, 15 rows 25.3 / 18.3.
+// two stages is one trip of the rows through memory.  It keeps its weights for all its tiles of 16 rows, and a stage begins with a
+// tile as soon as the stage before is done with that tile; from 17 rows on the tiles of rows are dealt to two workgroups
+// (one / two, us a layer: 24 rows 23.2 / 21.2, 64 rows 36.3 / 30.5; one for each tile of rows 64 rows 33.1).  Four products of the 0.6B shape, 28
+// layers, weights from memory, us a layer, four launches / one: 1 row 20.8 / 15.0, 8 rows 22.8 / 15.9, 15 rows 25.3 / 18.5, 16 rows 24.8 / 18.4,
+// 32 rows 26.2 / 21.4, 48 rows 29.2 / 27.3, 64 rows 31.0 / 28.6.
 //
-// How a stage learns that its rows are there.  mid, out and hidden begin as words of all ones (PL_MISSING), and every word
+// How a stage learns that its rows are there.  What the stages leave begins as words of all ones (PL_MISSING), and every word
 // is written once, past the XCD's L2 (relaxed atomics of device scope, as in pl_share): a word that differs is the value.
 // A result that happens to be all ones (a NaN, or a pair of them) is written as another NaN.  There is no counter: one that all
 // workgroups of a stage add to costs 2 us a stage (20.8 us a layer, no gain at all).
-// mid, hidden and out lie in the order in which the next stage's lanes load them ("laid", see cn_laid): 8 rows as
-// [row][column] cost 18.5 us a layer, since a load then touches a line a row twice.
+// The rows between stages lie in the order in which the next stage's lanes load them ("laid", see cn_laid): 8 rows as
+// [row][column] cost 18.5 us a layer where 15.6 were taken laid, since a load then touches a line a row twice.
 //
 // Nothing waits for ever.  A workgroup looks `looks` times; if its rows are not there by then (workgroups are started in the order
 // of their numbers, earlier stages first, but another launch may hold the compute units they need), it works out all
@@ -25,7 +28,9 @@
 // them first.  What it wrote itself it takes without a look, so that way ends whatever anybody else does.
 //
 // The arithmetic is gemm_skinny's for one tile of rows, to the same bits: K in as many stretches as that launch has waves (a
-// wave here takes up to three of them, each an accumulator of its own), the stretches' tiles added in their order.
+// wave here takes up to four of them, each an accumulator of its own), the stretches' tiles added in their order.  As there, the norms in front
+// of stages 1 and 3 are taken from the 32-bit stream below CN_HANDED rows, and from there on handed forward: the stage that adds
+// into the stream leaves bf16(stream * gain) and the sums of squares of its 16 columns.
 #include "common.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -34,28 +39,39 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define CN_ADD 0        // y = old + x . w^T, 32-bit
-#define CN_GATED 1      // y = act(norm(x) . gate^T) * (norm(x) . up^T), bfloat16
-#define CN_STORE 2      // y = norm(x) . w^T, bfloat16
+#define CN_ADD_HANDS 1  // the same, and what the next norm's product takes of it
+#define CN_GATED 2      // y = act(norm(x) . gate^T) * (norm(x) . up^T), bfloat16
+#define CN_STORE 3      // y = norm(x) . w^T, bfloat16
+#define CN_GATED_TAKES 4    // the same of rows that a CN_ADD_HANDS left
+#define CN_STORE_TAKES 5
 #define CN_STAGES 4
 #define CN_WAVES 4
-#define CN_STEPS 8      // K steps of 32 that a stretch of K has at most
-#define CN_STRETCHES 3  // stretches a wave takes at most
-#define CN_ROWS 15
+#define CN_STRETCHES 16     // of K, at most
+#define CN_ROWS 64
+#define CN_HANDED 16        // rows from which on norms are handed forward
+#define CN_RUN 4            // sums of squares a lane adds up: sixteen lanes a row, a stream of 1,024
 #define PL_MISSING 0xffffffffu
-#define CN_PAST_L2 16   // cache policy of a buffer load: device scope (sc1)
 #define CN_NOWHERE 0x7ff00000u
 
+// Cache policies of a buffer load: device scope (sc1), and none.
+struct cn_past_l2_t { static constexpr int value = 16; };
+struct cn_cached_t { static constexpr int value = 0; };
+
 struct cn_stage_t {
-    const void* x;          // CN_ADD: bfloat16 rows; otherwise the 32-bit stream, laid
+    const void* x;          // CN_ADD*: bfloat16 rows; CN_GATED, CN_STORE: the 32-bit stream, laid; *_TAKES: bfloat16 rows, laid
     const bf16_t* w;        // in strips
     void* y;
-    const float* old;       // CN_ADD
-    const float* gain;
+    const float* old;       // CN_ADD*
+    const float* gain;      // of the norm in front (CN_GATED, CN_STORE) or behind (CN_ADD_HANDS)
+    const float* squares;   // *_TAKES: [n, K / 16]
+    bf16_t* hand_x;         // CN_ADD_HANDS: [n, N], laid, ...
+    float* hand_squares;    // ... and [n, N / 16]
     float eps;
     int N, K;               // columns of y
     int per, stretches;     // K steps of a stretch; stretches of K
     int kind;
-    int first, tiles;       // its workgroups
+    int first, tiles;       // its workgroups: tiles of 16 columns times parts
+    int parts;              // workgroups that the tiles of 16 rows are dealt to
     int x_laid, old_laid, y_laid;
 };
 struct cn_chain_t {
@@ -63,191 +79,257 @@ struct cn_chain_t {
     int stages, n, act, looks;
 };
 
-// Where value (row, col) of a laid [n, width] tensor stands: K step by K step of 32 columns, in the order of the lanes that load
-// it (8 columns a group, 16 bytes a load: 32-bit rows in two halves).
-__host__ __device__ static inline size_t cn_laid(int row, int col, int n, bool wide) {
-    const size_t step = col / 32, group = col % 32 / 8;
-    return wide ? ((step * 8 + col % 8 / 4 * 4 + group) * n + row) * 4 + col % 4 : ((step * 4 + group) * n + row) * 8 + col % 8;
+// Where value (row, col) of a laid [n, width] tensor stands: 16 rows after 16 rows, in these K step by K step of 32 columns, in the order of the
+// lanes that load it (8 columns a group, 16 bytes a load: 32-bit rows in two halves).
+__device__ __forceinline__ uint32_t cn_laid(int row, int col, int n, int width, bool wide) {
+    const int begin = row / 16 * 16, rows = min(16, n - begin);
+    const int step = col / 32, group = col % 32 / 8;
+    return begin * width
+           + (wide ? ((step * 8 + col % 8 / 4 * 4 + group) * rows + row % 16) * 4 + col % 4 : ((step * 4 + group) * rows + row % 16) * 8 + col % 8);
 }
 
-// One tile of 16 columns of one stage.  trust: the rows were written by this workgroup.  Returns whether the tile is done
-// (false: its rows were not there in time), the same for all threads.
-template <int KIND, int V>
-__device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s, int stage, int tile, bool trust, float* red, float* ssq_lds,
+__device__ __forceinline__ uint32_t cn_word(const float* p) {
+    return __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void cn_leave(void* p, uint32_t word) {
+    __hip_atomic_store(static_cast<uint32_t*>(p), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A value is never the word that says that there is none.
+__device__ __forceinline__ uint32_t cn_value(float f) {
+    const uint32_t bits = __float_as_uint(f);
+    return bits == PL_MISSING ? 0x7fc00000u : bits;
+}
+// Two neighbouring columns' values, four lanes apart, as the even column's word.
+__device__ __forceinline__ uint32_t cn_pair(float f) {
+    const uint32_t half = bf16_bits_from_float(f);
+    return half | static_cast<uint32_t>(__shfl_down(half, 4, PL_WAVE)) << 16;
+}
+
+// One tile of 16 columns of one stage, all rows.  V stretches of K a wave, of at most S K steps of 32.  trust: the rows were written by this
+// workgroup.  FULL: every stretch of the 4 V has S steps (asking that of each load costs 8 rows 1.4 us a layer).  Returns whether the tile is done (false: its rows were not there in time), the same for
+// all threads.
+template <int KIND, int V, int S, bool FULL>
+__device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s, int stage, int place, bool trust, float* red, float* ssq_lds,
                                         int* late) {
-    constexpr int BT = KIND == CN_GATED ? 2 : 1;
-    constexpr bool NORM = KIND != CN_ADD;
+    const int tile = s.parts == 1 ? place : place / s.parts, part = place - tile * s.parts;
+    constexpr bool ADD = KIND == CN_ADD || KIND == CN_ADD_HANDS;
+    constexpr bool GATED = KIND == CN_GATED || KIND == CN_GATED_TAKES;
+    constexpr bool NORM = KIND == CN_GATED || KIND == CN_STORE;
+    constexpr bool TAKES = KIND == CN_GATED_TAKES || KIND == CN_STORE_TAKES;
+    constexpr int BT = GATED ? 2 : 1;
     constexpr int PARTS = NORM ? 2 : 1;        // loads of 16 bytes for a lane's 8 values
     const int lane = threadIdx.x % PL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PL_WAVE);
     const int c = lane % 16, g = lane / 16;
     const int K = s.K, steps = K / 32;
     const bool asks = stage > 0 && !trust;
 
-    // the weights first: they come from memory and depend on nothing
-    int step[V * CN_STEPS];                    // (-1: none)
-    bf16x8 w[BT][V * CN_STEPS];
-    float gn[NORM ? CN_STEPS : 1][8];
-#pragma unroll
-    for (int u = 0; u < V * CN_STEPS; ++u) {
-        const int at = (wave * V + u / CN_STEPS) * s.per + u % CN_STEPS;
-        step[u] = u % CN_STEPS < s.per && at < steps ? at : -1;
-    }
+    // the weights first: they come from memory and depend on nothing (steps that a stretch does not have are read past a
+    // buffer's end, which gives zeros, and so are rows that are not there)
+    auto step_of = [&](int u) { return FULL ? wave * V * S + u : (wave * V + u / S) * s.per + u % S; };
+    auto is_step = [&](int u) { return FULL || (u % S < s.per && step_of(u) < steps); };
+    bf16x8 w[BT][V * S];
+    float gn[NORM ? S : 1][8];
 #pragma unroll
     for (int b = 0; b < BT; ++b) {
-        const bf16_t* strip = s.w + static_cast<size_t>(b * (s.N / 16) + tile) * 16 * K + lane * 8;
+        const __amdgpu_buffer_rsrc_t strip =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(s.w) + static_cast<size_t>(b * (s.N / 16) + tile) * 16 * K, 0, 32u * K, 0x00027000);
 #pragma unroll
-        for (int u = 0; u < V * CN_STEPS; ++u) w[b][u] = *reinterpret_cast<const bf16x8*>(strip + static_cast<size_t>(max(step[u], 0)) * 512);
+        for (int u = 0; u < V * S; ++u)
+            w[b][u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(strip, is_step(u) ? lane * 16u : CN_NOWHERE, is_step(u) ? step_of(u) * 1024 : 0, 0));
     }
     if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < CN_STEPS; ++u) {
-            const f32x8 v = *reinterpret_cast<const f32x8*>(s.gain + max(step[u], 0) * 32 + g * 8);
+        for (int u = 0; u < S; ++u) {
+            const f32x8 v = *reinterpret_cast<const f32x8*>(s.gain + (is_step(u) ? step_of(u) : 0) * 32 + g * 8);
 #pragma unroll
             for (int e = 0; e < 8; ++e) gn[u][e] = v[e];
         }
     }
-
-    // where the lane's values of each step stand (rows and steps that are not there: past the buffer's end, which gives zeros)
-    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.x), 0, static_cast<uint32_t>(a.n) * K * (NORM ? 4 : 2), 0x00027000);
-    const uint32_t second = NORM ? 4 * 16 * a.n : 0;
-    uint32_t at[V * CN_STEPS];
-#pragma unroll
-    for (int u = 0; u < V * CN_STEPS; ++u)
-        at[u] = c >= a.n || step[u] < 0 ? CN_NOWHERE
-                : !s.x_laid             ? (static_cast<uint32_t>(c) * K + step[u] * 32 + g * 8) * 2
-                                        : ((static_cast<uint32_t>(step[u]) * (NORM ? 8 : 4) + g) * a.n + c) * 16;
-
-    // the element that this thread finishes
+    // the element of a tile that this thread finishes
     const int t = threadIdx.x;
-    const int row = t / 64 * 4 + t % 4, col = tile * 16 + t / 4 % 16;
-    const bool mine = row < a.n;
+    const int tile_row = t / 64 * 4 + t % 4, col = tile * 16 + t / 4 % 16;
+    float hand_gain = 0.f;
+    if constexpr (KIND == CN_ADD_HANDS) hand_gain = s.gain[col];
 
-    // One piece of the wave's rows is looked at until it is there (all of them would be n KB a look, by every workgroup), then
-    // all are loaded and looked at.
-    bool there = true;
-    if (asks) {
-        there = false;
-        for (int look = 0; look < a.looks && !there; ++look) {
-            asm volatile("" ::: "memory");
-            const u32x4 p = __builtin_amdgcn_raw_buffer_load_b128(rows, at[0], 0, CN_PAST_L2);
-            there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
-            if (!there) __builtin_amdgcn_s_sleep(1);
-        }
-    }
-    u32x4 raw[V * CN_STEPS][PARTS];
-    uint32_t old = 0;
-    for (int look = 0; look <= a.looks; ++look) {
-        asm volatile("" ::: "memory");
-        if (KIND == CN_ADD)
-            old = mine ? __hip_atomic_load(reinterpret_cast<const uint32_t*>(s.old) + (s.old_laid ? cn_laid(row, col, a.n, true) : static_cast<size_t>(row) * s.N + col),
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                       : 0u;
-        // (the first time through L2, which the workgroups of an XCD share: what a load that came too early has left there is
-        // seen to be missing, and then read past L2)
-        if (stage == 0 || (asks && look == 0)) {
-#pragma unroll
-            for (int u = 0; u < V * CN_STEPS; ++u)
-#pragma unroll
-                for (int h = 0; h < PARTS; ++h) raw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rows, at[u] + h * second, 0, 0);
-        } else {
-#pragma unroll
-            for (int u = 0; u < V * CN_STEPS; ++u)
-#pragma unroll
-                for (int h = 0; h < PARTS; ++h) raw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rows, at[u] + h * second, 0, CN_PAST_L2);
-        }
-        if (!asks) break;
-        uint32_t most = old;
-#pragma unroll
-        for (int u = 0; u < V * CN_STEPS; ++u)
-#pragma unroll
-            for (int e = 0; e < 4 * PARTS; ++e) most = max(most, raw[u][e / 4][e % 4]);
-        there = __all(most != PL_MISSING);
-        if (there) break;
-        __builtin_amdgcn_s_sleep(1);
-    }
-    if (!there && lane == 0) *late = 1;
+    const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.x), 0, static_cast<uint32_t>(a.n) * K * (NORM ? 4 : 2), 0x00027000);
 
-    f32x4 acc[BT][V];
-#pragma unroll
-    for (int b = 0; b < BT; ++b)
-#pragma unroll
-        for (int v = 0; v < V; ++v) acc[b][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float ssq = 0.f;
-#pragma unroll
-    for (int u = 0; u < CN_STEPS; ++u)
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            const int k = v * CN_STEPS + u;
-            bf16x8 x;
-            if constexpr (NORM) {
-                f32x8 scaled;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float xv = __uint_as_float(raw[k][e / 4][e % 4]);
-                    ssq = fmaf(xv, xv, ssq);
-                    scaled[e] = xv * gn[u][e];
-                }
-                x = __builtin_convertvector(scaled, bf16x8);
-            } else {
-                x = __builtin_bit_cast(bf16x8, raw[k][0]);
+    for (int row0 = part * 16, turn = 0; row0 < a.n; row0 += s.parts * 16, turn ^= 1) {
+        const int tile_rows = min(16, a.n - row0);
+        const int row = row0 + tile_row;
+        const bool mine = row < a.n;
+        float* const tiles = red + turn * (CN_STRETCHES * 256);        // (two of them in turn: a barrier a tile of rows)
+        float* const squares = ssq_lds + turn * (CN_WAVES * 16);
+        // where the lane's values of K step k stand: at `lane_at` + begin + k * stride
+        const uint32_t begin = row0 * K * (NORM ? 4 : 2), second = NORM ? 64 * tile_rows : 0;
+        const uint32_t stride = s.x_laid ? (NORM ? 128 : 64) * tile_rows : 64;
+        const uint32_t lane_at = c >= tile_rows ? CN_NOWHERE : s.x_laid ? (g * tile_rows + c) * 16 : (c * K + g * 8) * 2;
+        auto load = [&](int u, int h, auto policy) {
+            return __builtin_amdgcn_raw_buffer_load_b128(rows, is_step(u) ? lane_at : CN_NOWHERE, begin + h * second + (is_step(u) ? step_of(u) * stride : 0),
+                                                         decltype(policy)::value);
+        };
+
+        // One piece of the wave's rows is looked at until it is there (all of them would be KBs a look, by every workgroup), then
+        // all are loaded and looked at.
+        bool there = true;
+        if (asks) {
+            there = false;
+            for (int look = 0; look < a.looks && !there; ++look) {
+                asm volatile("" ::: "memory");
+                const u32x4 p = load(0, 0, cn_past_l2_t{});
+                there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
+                if (!there) __builtin_amdgcn_s_sleep(1);
             }
-            // (a step past the stretch multiplies nothing, whatever the weights in its place are)
-#pragma unroll
-            for (int b = 0; b < BT; ++b)
-                acc[b][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, step[k] >= 0 ? w[b][k] : bf16x8{}, acc[b][v], 0, 0, 0);
         }
+        u32x4 raw[V * S][PARTS];
+        uint32_t old = 0, sums[TAKES ? CN_RUN : 1];
+        for (int look = 0; look <= a.looks; ++look) {
+            asm volatile("" ::: "memory");
+            if constexpr (ADD) old = mine ? cn_word(s.old + (s.old_laid ? cn_laid(row, col, a.n, s.N, true) : row * s.N + col)) : 0u;
+            if constexpr (TAKES) {
+                // the sixteen threads of a row add up a run of its sums of squares each
+                const int count = K / 16, run = pl_ceil_div(count, 16), from = t / 4 % 16 * run;
 #pragma unroll
-    for (int b = 0; b < BT; ++b)
+                for (int j = 0; j < CN_RUN; ++j)
+                    sums[j] = mine && j < run && from + j < count ? cn_word(s.squares + static_cast<size_t>(row) * count + from + j) : 0u;
+            }
+            // (the first time through L2, which the workgroups of an XCD share: what a load that came too early has left there is
+            // seen to be missing, and then read past L2)
+            if (stage == 0 || (asks && look == 0)) {
 #pragma unroll
-        for (int v = 0; v < V; ++v) *reinterpret_cast<f32x4*>(red + ((wave * V + v) * BT + b) * 256 + lane * 4) = acc[b][v];
-    if constexpr (NORM) {
-        ssq += __shfl_xor(ssq, 16, PL_WAVE);
-        ssq += __shfl_xor(ssq, 32, PL_WAVE);
-        if (g == 0) ssq_lds[wave * 16 + c] = ssq;
-    }
-    __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(*late)) return false;
+                for (int u = 0; u < V * S; ++u)
+#pragma unroll
+                    for (int h = 0; h < PARTS; ++h) raw[u][h] = load(u, h, cn_cached_t{});
+            } else {
+#pragma unroll
+                for (int u = 0; u < V * S; ++u)
+#pragma unroll
+                    for (int h = 0; h < PARTS; ++h) raw[u][h] = load(u, h, cn_past_l2_t{});
+            }
+            if (!asks) break;
+            uint32_t most = old;
+            if constexpr (TAKES)
+#pragma unroll
+                for (int j = 0; j < CN_RUN; ++j) most = max(most, sums[j]);
+#pragma unroll
+            for (int u = 0; u < V * S; ++u)
+#pragma unroll
+                for (int e = 0; e < 4 * PARTS; ++e) most = max(most, raw[u][e / 4][e % 4]);
+            there = __all(most != PL_MISSING);
+            if (there) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (!there && lane == 0) *late = 1;
 
-    float val[BT];
+        f32x4 acc[BT][V];
 #pragma unroll
-    for (int b = 0; b < BT; ++b) {
-        val[b] = 0.f;
+        for (int b = 0; b < BT; ++b)
 #pragma unroll
-        for (int k = 0; k < CN_WAVES * V; ++k)
-            if (k < s.stretches) val[b] += red[(k * BT + b) * 256 + t];
-    }
-    if constexpr (NORM) {
-        float total = 0.f;
+            for (int v = 0; v < V; ++v) acc[b][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float ssq = 0.f;
 #pragma unroll
-        for (int k = 0; k < CN_WAVES; ++k) total += ssq_lds[k * 16 + row];
-        const float rinv = 1.f / sqrtf(total / static_cast<float>(K) + s.eps);
+        for (int u = 0; u < S; ++u)
 #pragma unroll
-        for (int b = 0; b < BT; ++b) val[b] *= rinv;
-    }
-    if constexpr (KIND == CN_ADD) {
-        uint32_t bits = __float_as_uint(__uint_as_float(old) + val[0]);
-        bits = bits == PL_MISSING ? 0x7fc00000u : bits;
-        if (mine)
-            __hip_atomic_store(static_cast<uint32_t*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, true) : static_cast<size_t>(row) * s.N + col), bits,
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        const float r = KIND == CN_GATED ? pl_activate<false>(val[0], a.act) * val[BT - 1] : val[0];
-        // two neighbouring columns, four lanes apart, are a word
-        const uint32_t half = bf16_bits_from_float(r);
-        uint32_t pair = half | static_cast<uint32_t>(__shfl_down(half, 4, PL_WAVE)) << 16;
-        if (s.y_laid && pair == PL_MISSING) pair = 0x7fff7fffu;
-        if (mine && col % 2 == 0)
-            __hip_atomic_store(reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, false) : static_cast<size_t>(row) * s.N + col)),
-                               pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int v = 0; v < V; ++v) {
+                const int k = v * S + u;
+                bf16x8 x;
+                if constexpr (NORM) {
+                    f32x8 scaled;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float xv = __uint_as_float(raw[k][e / 4][e % 4]);
+                        ssq = fmaf(xv, xv, ssq);
+                        scaled[e] = xv * gn[u][e];
+                    }
+                    x = __builtin_convertvector(scaled, bf16x8);
+                } else {
+                    x = __builtin_bit_cast(bf16x8, raw[k][0]);
+                }
+#pragma unroll
+                for (int b = 0; b < BT; ++b)
+                    acc[b][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, w[b][k], acc[b][v], 0, 0, 0);
+            }
+#pragma unroll
+        for (int b = 0; b < BT; ++b)
+#pragma unroll
+            for (int v = 0; v < V; ++v) *reinterpret_cast<f32x4*>(tiles + ((wave * V + v) * BT + b) * 256 + lane * 4) = acc[b][v];
+        if constexpr (NORM) {
+            ssq += __shfl_xor(ssq, 16, PL_WAVE);
+            ssq += __shfl_xor(ssq, 32, PL_WAVE);
+            if (g == 0) squares[wave * 16 + c] = ssq;
+        }
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(*late)) return false;
+
+        float val[BT];
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+            val[b] = 0.f;
+#pragma unroll
+            for (int k = 0; k < CN_WAVES * V; ++k)
+                if (FULL || k < s.stretches) val[b] += tiles[(k * BT + b) * 256 + t];
+        }
+        if constexpr (NORM || TAKES) {
+            float total = 0.f;
+            if constexpr (NORM) {
+#pragma unroll
+                for (int k = 0; k < CN_WAVES; ++k) total += squares[k * 16 + tile_row];
+            } else {
+#pragma unroll
+                for (int j = 0; j < CN_RUN; ++j) total += __uint_as_float(sums[j]);
+                total += __shfl_xor(total, 4, PL_WAVE);
+                total += __shfl_xor(total, 8, PL_WAVE);
+                total += __shfl_xor(total, 16, PL_WAVE);
+                total += __shfl_xor(total, 32, PL_WAVE);
+            }
+            const float rinv = 1.f / sqrtf(total / static_cast<float>(K) + s.eps);
+#pragma unroll
+            for (int b = 0; b < BT; ++b) val[b] *= rinv;
+        }
+        if constexpr (ADD) {
+            float updated = 0.f;
+            if (mine) updated = __uint_as_float(old) + val[0];
+            if (mine) cn_leave(static_cast<float*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, s.N, true) : row * s.N + col), cn_value(updated));
+            if constexpr (KIND == CN_ADD_HANDS) {
+                uint32_t pair = cn_pair(updated * hand_gain);
+                pair = pair == PL_MISSING ? 0x7fff7fffu : pair;
+                if (mine && col % 2 == 0) cn_leave(s.hand_x + cn_laid(row, col, a.n, s.N, false), pair);
+                float sq = updated * updated;
+                sq += __shfl_xor(sq, 4, PL_WAVE);
+                sq += __shfl_xor(sq, 8, PL_WAVE);
+                sq += __shfl_xor(sq, 16, PL_WAVE);
+                sq += __shfl_xor(sq, 32, PL_WAVE);
+                if (mine && col % 16 == 0) cn_leave(s.hand_squares + static_cast<size_t>(row) * (s.N / 16) + tile, cn_value(sq));
+            }
+        } else {
+            uint32_t pair = cn_pair(GATED ? pl_activate<false>(val[0], a.act) * val[BT - 1] : val[0]);
+            if (s.y_laid && pair == PL_MISSING) pair = 0x7fff7fffu;
+            if (mine && col % 2 == 0)
+                cn_leave(static_cast<bf16_t*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, s.N, false) : row * s.N + col), pair);
+        }
     }
     return true;
 }
 
+template <int KIND, int V, int S>
+__device__ __forceinline__ bool cn_form(const cn_chain_t& a, const cn_stage_t& s, int stage, int place, bool trust, float* red, float* ssq_lds, int* late) {
+    if (s.per == S && s.K == CN_WAVES * V * S * 32) return cn_tile<KIND, V, S, true>(a, s, stage, place, trust, red, ssq_lds, late);
+    return cn_tile<KIND, V, S, false>(a, s, stage, place, trust, red, ssq_lds, late);
+}
+// Stretches of K in the kernel's unrolled forms (cn_stretches has how many there are).
+template <int KIND>
+__device__ __forceinline__ bool cn_add(const cn_chain_t& a, const cn_stage_t& s, int stage, int place, bool trust, float* red, float* ssq_lds, int* late) {
+    if (s.stretches <= CN_WAVES) return cn_form<KIND, 1, 8>(a, s, stage, place, trust, red, ssq_lds, late);
+    if (s.stretches <= CN_WAVES * 2) return cn_form<KIND, 2, 8>(a, s, stage, place, trust, red, ssq_lds, late);
+    if constexpr (KIND == CN_ADD) return cn_form<KIND, 3, 8>(a, s, stage, place, trust, red, ssq_lds, late);
+    return cn_form<KIND, 4, 6>(a, s, stage, place, trust, red, ssq_lds, late);
+}
+
 // 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
 // first three stages of the 0.6B shape and most of the 256 of the last).
+template <bool HANDED>
 __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a) {
-    __shared__ float red[CN_WAVES * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
-    __shared__ float ssq_lds[CN_WAVES * 16];
+    __shared__ float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
+    __shared__ float ssq_lds[2 * CN_WAVES * 16];
     __shared__ int late;
     int stage = 0;
     while (stage + 1 < a.stages && static_cast<int>(blockIdx.x) >= a.s[stage + 1].first) ++stage;
@@ -261,14 +343,15 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
         q = __builtin_amdgcn_readfirstlane(q);
         const cn_stage_t& s = a.s[p];
         bool done;
-        if (s.kind == CN_ADD) {
-            if (s.stretches <= CN_WAVES) done = cn_tile<CN_ADD, 1>(a, s, p, q, trust, red, ssq_lds, &late);
-            else if (s.stretches <= CN_WAVES * 2) done = cn_tile<CN_ADD, 2>(a, s, p, q, trust, red, ssq_lds, &late);
-            else done = cn_tile<CN_ADD, 3>(a, s, p, q, trust, red, ssq_lds, &late);
-        } else if (s.kind == CN_GATED) {
-            done = cn_tile<CN_GATED, 1>(a, s, p, q, trust, red, ssq_lds, &late);
+        if constexpr (HANDED) {
+            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
+            else if (s.kind == CN_ADD_HANDS) done = cn_add<CN_ADD_HANDS>(a, s, p, q, trust, red, ssq_lds, &late);
+            else if (s.kind == CN_GATED_TAKES) done = cn_form<CN_GATED_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
+            else done = cn_form<CN_STORE_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
         } else {
-            done = cn_tile<CN_STORE, 1>(a, s, p, q, trust, red, ssq_lds, &late);
+            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
+            else if (s.kind == CN_GATED) done = cn_form<CN_GATED, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
+            else done = cn_form<CN_STORE, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
         }
         if (done && p == stage && q == tile) return;
         // The rows were not there in time: all tiles of the earlier stages, then the workgroup's own once more.  (What the
@@ -289,62 +372,104 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
     }
 }
 
-// How gemm_skinny's launch for up to 16 rows cuts K (launch_unr in gemm_skinny.hpp): the stretches, 0 where they are more
-// than this kernel takes.
-static int cn_stretches(int K, bool norm) {
+// How gemm_skinny's launches for one tile of rows cut K (launch_unr and launch_one in gemm_skinny.hpp): the stretches, 0 where they are
+// more, or longer, than this kernel takes.
+static int cn_stretches(int K, int kind) {
     const int steps = K / 32;
-    if (steps <= CN_WAVES * CN_STEPS) return CN_WAVES;
-    if (norm) return 0;
-    const int least = pl_ceil_div(steps, CN_STEPS);
+    if (steps <= CN_WAVES * 8) return CN_WAVES;
+    if (kind != CN_ADD && kind != CN_ADD_HANDS) return 0;
+    const int least = pl_ceil_div(steps, 8);
     if (least <= 8) return least < 5 ? 5 : least;
-    const int many = least < 9 ? 9 : least;
-    return many <= CN_WAVES * CN_STRETCHES ? many : 0;
+    const int many = max(9, kind == CN_ADD_HANDS ? pl_ceil_div(steps, 6) : least);
+    return many <= (kind == CN_ADD_HANDS ? 16 : 12) ? many : 0;
 }
 
 // Whether the products of so many rows are this launch's: a stream of `width`, an output projection of inner width `inner`, a feed-forward of `ff`,
 // and (0: none) `after` columns behind the next norm.
 extern "C" int pl_gemm_chain_applies(int n, int width, int inner, int ff, int after) {
     return n > 0 && n <= CN_ROWS && width > 0 && width % 32 == 0 && inner > 0 && inner % 32 == 0 && ff > 0 && ff % 32 == 0 && after >= 0 && after % 16 == 0
-           && width <= (1 << 20) && ff <= (1 << 20) && after <= (1 << 20)
-           && cn_stretches(width, true) && cn_stretches(inner, false) && cn_stretches(ff, false);
+           && ff <= (1 << 20) && after <= (1 << 20) && width / 16 <= 16 * CN_RUN
+           && cn_stretches(width, CN_STORE) && cn_stretches(inner, CN_ADD) && cn_stretches(ff, CN_ADD);
+}
+
+// The 32-bit words that one launch leaves between its stages, all ones before it: mid [n, width], hidden [n, ff] in bfloat16, out [n, width], and, from CN_HANDED
+// rows on, the two norms handed forward, rows [n, width] in bfloat16 and sums [n, width / 16] each.  `out` begins at word out_at.
+static size_t cn_room(int n, int width, int ff, size_t* out_at) {
+    const size_t stream = static_cast<size_t>(n) * width, handed = n >= CN_HANDED ? stream / 2 + stream / 16 : 0;
+    if (out_at) *out_at = stream + static_cast<size_t>(n) * ff / 2;
+    return 2 * stream + static_cast<size_t>(n) * ff / 2 + 2 * handed;
+}
+extern "C" long pl_gemm_chain_room(int n, int width, int ff) { return static_cast<long>(cn_room(n, width, ff, nullptr)); }
+extern "C" long pl_gemm_chain_out(int n, int width, int ff) {
+    size_t at = 0;
+    cn_room(n, width, ff, &at);
+    return static_cast<long>(at);
 }
 
 // stream: [n, width] 32-bit, rows or (stream_laid) as an earlier chain left it.  rows: bfloat16 [n, inner].  The weights in strips: w_out [width, inner],
-// w_gated [2 ff, width] (gate rows first), w_down [width, ff], w_next [after, width] or null.  mid [n, width] and out [n, width] 32-bit and hidden [n, ff]
-// bfloat16 are all ones before; out comes laid with a w_next and in rows without.  next: bfloat16 [n, after].  looks: how often a workgroup
-// looks for its rows before it works them out itself.
-extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* rows, float* mid, void* hidden, float* out, void* next, const void* w_out,
+// w_gated [2 ff, width] (gate rows first), w_down [width, ff], w_next [after, width] or null.  room: cn_room words of all ones; its `out`
+// [n, width] takes the updated stream, laid with a w_next and in rows without.  next: bfloat16 [n, after].  looks: how often a
+// workgroup looks for its rows before it works them out itself.
+extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* rows, void* room, void* next, const void* w_out,
                              const void* w_gated, const void* w_down, const void* w_next, const float* gain2, float eps2, const float* gain_next,
                              float eps_next, int n, int width, int inner, int ff, int after, int act, int looks, hipStream_t stream_) {
     if (n == 0) return 0;
     PL_REQUIRE(pl_gemm_chain_applies(n, width, inner, ff, after), "chain of products: %d rows, a stream of %d, inner widths %d and %d, %d columns behind it", n, width, inner, ff, after);
-    PL_REQUIRE(stream && rows && mid && hidden && out && w_out && w_gated && w_down && gain2, "chain of products: an operand is missing");
+    PL_REQUIRE(stream && rows && room && w_out && w_gated && w_down && gain2, "chain of products: an operand is missing");
     PL_REQUIRE((w_next != nullptr) == (after > 0) && (next != nullptr) == (after > 0) && (gain_next != nullptr) == (after > 0),
                "chain of products: %d columns behind the chain", after);
     PL_REQUIRE(act >= PL_ACT_SILU && act <= PL_ACT_RELU2, "chain of products: activation code %d", act);
     PL_REQUIRE(looks >= 0, "chain of products: %d looks", looks);
-    for (const void* p : {static_cast<const void*>(stream), rows, static_cast<const void*>(mid), static_cast<const void*>(hidden), static_cast<const void*>(out), w_out, w_gated,
-                          w_down, w_next, static_cast<const void*>(gain2), static_cast<const void*>(gain_next), static_cast<const void*>(next)})
+    for (const void* p : {static_cast<const void*>(stream), rows, static_cast<const void*>(room), w_out, w_gated, w_down, w_next, static_cast<const void*>(gain2),
+                          static_cast<const void*>(gain_next), static_cast<const void*>(next)})
         PL_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "chain of products: an operand begins in the middle of 16 bytes");
+    const bool handed = n >= CN_HANDED, follows = after > 0;
+    size_t out_at = 0;
+    cn_room(n, width, ff, &out_at);
+    const size_t words = static_cast<size_t>(n) * width;
+    float* const mid = static_cast<float*>(room);
+    float* const hidden = mid + words;
+    float* const out = mid + out_at;
+    // (only there with handed norms)
+    bf16_t* const mid_x = reinterpret_cast<bf16_t*>(out + words);
+    float* const mid_squares = out + words + words / 2;
+    bf16_t* const out_x = reinterpret_cast<bf16_t*>(mid_squares + words / 16);
+    float* const out_squares = mid_squares + words / 16 + words / 2;
     cn_chain_t a{};
     a.n = n;
     a.act = act;
     a.looks = looks;
-    a.s[0] = {rows, static_cast<const bf16_t*>(w_out), mid, stream, nullptr, 0.f, width, inner, 0, 0, CN_ADD, 0, 0, 0, stream_laid ? 1 : 0, 1};
-    a.s[1] = {mid, static_cast<const bf16_t*>(w_gated), hidden, nullptr, gain2, eps2, ff, width, 0, 0, CN_GATED, 0, 0, 1, 0, 1};
-    a.s[2] = {hidden, static_cast<const bf16_t*>(w_down), out, mid, nullptr, 0.f, width, ff, 0, 0, CN_ADD, 0, 0, 1, 1, after > 0 ? 1 : 0};
-    a.s[3] = {out, static_cast<const bf16_t*>(w_next), next, nullptr, gain_next, eps_next, after, width, 0, 0, CN_STORE, 0, 0, 1, 0, 0};
-    a.stages = after > 0 ? 4 : 3;
+    a.stages = follows ? 4 : 3;
+    cn_stage_t& project = a.s[0];
+    project.x = rows; project.w = static_cast<const bf16_t*>(w_out); project.y = mid; project.old = stream;
+    project.N = width; project.K = inner; project.kind = handed ? CN_ADD_HANDS : CN_ADD;
+    project.old_laid = stream_laid ? 1 : 0; project.y_laid = 1;
+    project.gain = gain2; project.hand_x = mid_x; project.hand_squares = mid_squares;
+    cn_stage_t& gated = a.s[1];
+    gated.x = handed ? static_cast<const void*>(mid_x) : mid; gated.w = static_cast<const bf16_t*>(w_gated); gated.y = hidden; gated.gain = gain2; gated.eps = eps2;
+    gated.squares = mid_squares; gated.N = ff; gated.K = width; gated.kind = handed ? CN_GATED_TAKES : CN_GATED;
+    gated.x_laid = 1; gated.y_laid = 1;
+    cn_stage_t& down = a.s[2];
+    down.x = hidden; down.w = static_cast<const bf16_t*>(w_down); down.y = out; down.old = mid;
+    down.N = width; down.K = ff; down.kind = handed && follows ? CN_ADD_HANDS : CN_ADD;
+    down.x_laid = 1; down.old_laid = 1; down.y_laid = follows ? 1 : 0;
+    down.gain = gain_next; down.hand_x = out_x; down.hand_squares = out_squares;
+    cn_stage_t& last = a.s[3];
+    last.x = handed ? static_cast<const void*>(out_x) : out; last.w = static_cast<const bf16_t*>(w_next); last.y = next; last.gain = gain_next; last.eps = eps_next;
+    last.squares = out_squares; last.N = after; last.K = width; last.kind = handed ? CN_STORE_TAKES : CN_STORE;
+    last.x_laid = 1;
     int grid = 0;
     for (int i = 0; i < a.stages; ++i) {
         cn_stage_t& s = a.s[i];
-        s.stretches = cn_stretches(s.K, s.kind != CN_ADD);
+        s.stretches = cn_stretches(s.K, s.kind);
         s.per = pl_ceil_div(s.K / 32, s.stretches);
         s.first = grid;
-        s.tiles = s.N / 16;
+        s.parts = n > 16 ? 2 : 1;
+        s.tiles = s.N / 16 * s.parts;
         grid += s.tiles;
     }
-    gemm_chain_kernel<<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a);
+    if (handed) gemm_chain_kernel<true><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a);
+    else gemm_chain_kernel<false><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a);
     PL_CHECK_LAUNCH("gemm_chain");
     return 0;
 }

@@ -57,7 +57,9 @@ def _signatures(lib) -> None:
         "pl_gemm_skinny_hand": [p, p, p, i, i, i, i, i, i, p, i, f, p, p, p, i, p],
         "pl_gemm_skinny_hand_applies": [i, i, i, i, i],
         "pl_gemm_chain_applies": [i, i, i, i, i],
-        "pl_gemm_chain": [p, i, p, p, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
+        "pl_gemm_chain_room": [i, i, i],
+        "pl_gemm_chain_out": [i, i, i],
+        "pl_gemm_chain": [p, i, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
         "pl_gemm_many": [p, p, i, p, i, i, i, i, p, i, f, p, p, p, p],
         "pl_gemm_many_applies": [i, i, i, i],
@@ -1184,7 +1186,7 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = torch
 
 # How often a workgroup of a chain of products looks for its rows (some 0.7 us a look) before it works them out itself.
 CHAIN_LOOKS = 2048
-CHAIN_ROWS = 15
+CHAIN_ROWS = 64
 
 
 def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0) -> bool:
@@ -1194,23 +1196,18 @@ def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0) ->
 
 
 class ChainRoom:
-    """Where the stages of a step's chains of products leave their rows: for each of ``sizes`` (stream width, feed-forward width) a layer's stream behind
-    its mixer and behind its feed-forward and the feed-forward's inner rows, all words ones, which is how a stage sees what is not there yet.
-    One launch fills them for all layers of a step."""
+    """Where the stages of a step's chains of products leave their rows, for each of ``sizes`` (stream width, feed-forward width) a layer's: all words
+    ones, which is how a stage sees what is not there yet.  One launch fills them for all layers of a step."""
 
     def __init__(self, rows: int, sizes: list, device):
-        self.rows = rows
-        per_layer = [(2 * rows * width, rows * ff // 2) for width, ff in sizes]
-        words = torch.full((sum(a + b for a, b in per_layer),), -1, dtype=torch.int32, device=device)
-        self.layers, at = [], 0
-        for (width, ff), (streams, inner) in zip(sizes, per_layer):
-            both = words[at:at + streams].view(torch.float32).view(2, rows, width)
-            hidden = words[at + streams:at + streams + inner].view(torch.bfloat16).view(rows, ff)
-            self.layers.append((both[0], hidden, both[1]))
-            at += streams + inner
+        lib = library()
+        words = [lib.pl_gemm_chain_room(rows, width, ff) for width, ff in sizes]
+        begins = [sum(-(-w // 4) * 4 for w in words[:i]) for i in range(len(words) + 1)]
+        room = torch.full((begins[-1],), -1, dtype=torch.int32, device=device)
+        self.layers = [room[at:at + count] for at, count in zip(begins, words)]
 
 
-def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: tuple, w_out: torch.Tensor, w_gated: torch.Tensor, w_down: torch.Tensor,
+def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch.Tensor, w_out: torch.Tensor, w_gated: torch.Tensor, w_down: torch.Tensor,
                gain: torch.Tensor, eps: float, activation: str, following: tuple | None = None, looks: int | None = None) -> tuple:
     """The products behind a layer's attention in one launch, all weights in strips (``weights_in_strips``): the mixer's output projection of ``rows`` joins
     ``stream`` (which stays as it is), the gated feed-forward behind the norm of ``gain`` and ``eps`` joins that, and, with ``following`` =
@@ -1218,14 +1215,14 @@ def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: tuple
     ``laid``: ``stream`` is one that a chain with a ``following`` gave: its values lie in the order the next chain loads them.
     ``room``: one layer's of a ``ChainRoom`` that no chain has used.  ``looks``: how often a workgroup looks for its rows before it works
     them out itself."""
-    mid, hidden, out = room
+    lib = library()
     n, width = stream.shape
-    inner, ff = rows.shape[1], hidden.shape[1]
+    inner, ff = rows.shape[1], w_down.shape[1]
     _need(stream, "residual stream", (n, width), torch.float32)
     _need(rows, "mixer output", (n, inner), torch.bfloat16)
-    _need(mid, "room for the stream", (n, width), torch.float32)
-    _need(out, "room for the stream", (n, width), torch.float32)
-    _need(hidden, "room for the feed-forward", (n, ff), torch.bfloat16)
+    _need(room, "room for a chain", (lib.pl_gemm_chain_room(n, width, ff),), torch.int32)
+    at = lib.pl_gemm_chain_out(n, width, ff)
+    out = room[at:at + n * width].view(torch.float32).view(n, width)
     _need(w_out, "output projection in strips", (width, inner), torch.bfloat16)
     _need(w_gated, "gate and up projections in strips", (2 * ff, width), torch.bfloat16)
     _need(w_down, "down projection in strips", (width, ff), torch.bfloat16)
@@ -1238,9 +1235,8 @@ def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: tuple
         _need(w_next, "next projection in strips", (after, width), torch.bfloat16)
         _need(gain_next, "norm gain", (width,), torch.float32)
         projected = torch.empty((n, after), dtype=torch.bfloat16, device=stream.device)
-    _check(library().pl_gemm_chain(
-        stream.data_ptr(), 1 if laid else 0, rows.data_ptr(), mid.data_ptr(), hidden.data_ptr(), out.data_ptr(), _ptr(projected), w_out.data_ptr(),
-        w_gated.data_ptr(), w_down.data_ptr(), _ptr(w_next), gain.data_ptr(), float(eps), _ptr(gain_next), float(eps_next), n, width, inner, ff, after,
+    _check(lib.pl_gemm_chain(
+        stream.data_ptr(), 1 if laid else 0, rows.data_ptr(), room.data_ptr(), _ptr(projected), w_out.data_ptr(), w_gated.data_ptr(), w_down.data_ptr(), _ptr(w_next), gain.data_ptr(), float(eps), _ptr(gain_next), float(eps_next), n, width, inner, ff, after,
         activation_code(activation), CHAIN_LOOKS if looks is None else looks, _stream()))
     return out, projected
 
