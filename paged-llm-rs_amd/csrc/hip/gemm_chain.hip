@@ -31,12 +31,11 @@
 // wave here takes up to four of them, each an accumulator of its own), the stretches' tiles added in their order.  As there, the norms in front
 // of stages 1 and 3 are taken from the 32-bit stream below CN_HANDED rows, and from there on handed forward: the stage that adds
 // into the stream leaves bf16(stream * gain) and the sums of squares of its 16 columns.
-#include "common.hpp"
+#include "gemm_chain.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define CN_ADD 0        // y = old + x . w^T, 32-bit
 #define CN_ADD_HANDS 1  // the same, and what the next norm's product takes of it
@@ -50,12 +49,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #define CN_ROWS 64
 #define CN_HANDED 16        // rows from which on norms are handed forward
 #define CN_RUN 4            // sums of squares a lane adds up: sixteen lanes a row, a stream of 1,024
-#define PL_MISSING 0xffffffffu
-#define CN_NOWHERE 0x7ff00000u
-
-// Cache policies of a buffer load: device scope (sc1), and none.
-struct cn_past_l2_t { static constexpr int value = 16; };
-struct cn_cached_t { static constexpr int value = 0; };
 
 struct cn_stage_t {
     const void* x;          // CN_ADD*: bfloat16 rows; CN_GATED, CN_STORE: the 32-bit stream, laid; *_TAKES: bfloat16 rows, laid
@@ -88,17 +81,6 @@ __device__ __forceinline__ uint32_t cn_laid(int row, int col, int n, int width, 
            + (wide ? ((step * 8 + col % 8 / 4 * 4 + group) * rows + row % 16) * 4 + col % 4 : ((step * 4 + group) * rows + row % 16) * 8 + col % 8);
 }
 
-__device__ __forceinline__ uint32_t cn_word(const float* p) {
-    return __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void cn_leave(void* p, uint32_t word) {
-    __hip_atomic_store(static_cast<uint32_t*>(p), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// A value is never the word that says that there is none.
-__device__ __forceinline__ uint32_t cn_value(float f) {
-    const uint32_t bits = __float_as_uint(f);
-    return bits == PL_MISSING ? 0x7fc00000u : bits;
-}
 // Two neighbouring columns' values, four lanes apart, as the even column's word.
 __device__ __forceinline__ uint32_t cn_pair(float f) {
     const uint32_t half = bf16_bits_from_float(f);

@@ -60,6 +60,10 @@ def _signatures(lib) -> None:
         "pl_gemm_chain_room": [i, i, i],
         "pl_gemm_chain_out": [i, i, i],
         "pl_gemm_chain": [p, i, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
+        "pl_gemm_chain_f32_applies": [i, i, i, i, i],
+        "pl_gemm_chain_f32_room": [i, i, i],
+        "pl_gemm_chain_f32_out": [i, i, i],
+        "pl_gemm_chain_f32": [p, i, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
         "pl_gemm_tiled": [p, p, p, i, i, i, i, i, p],
         "pl_gemm_many": [p, p, i, p, i, i, i, i, p, i, f, p, p, p, p],
         "pl_gemm_many_applies": [i, i, i, i],
@@ -1189,19 +1193,23 @@ CHAIN_LOOKS = 2048
 CHAIN_ROWS = 64
 
 
-def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0) -> bool:
+def _chain(name: str, dtype: torch.dtype):
+    """The entry point ``name`` of the chains of products over operands of this type."""
+    return getattr(library(), f"pl_gemm_chain{'_f32' if dtype == torch.float32 else ''}{name}")
+
+
+def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0, dtype: torch.dtype = torch.bfloat16) -> bool:
     """Whether the products behind a layer's attention, of so many rows, are one launch (``gemm_chain``): a stream of ``width``, an output projection of
     inner width ``inner``, a feed-forward of ``ff`` and, with ``after``, so many columns behind the next norm."""
-    return bool(library().pl_gemm_chain_applies(rows, width, inner, ff, after))
+    return bool(_chain("_applies", dtype)(rows, width, inner, ff, after))
 
 
 class ChainRoom:
     """Where the stages of a step's chains of products leave their rows, for each of ``sizes`` (stream width, feed-forward width) a layer's: all words
     ones, which is how a stage sees what is not there yet.  One launch fills them for all layers of a step."""
 
-    def __init__(self, rows: int, sizes: list, device):
-        lib = library()
-        words = [lib.pl_gemm_chain_room(rows, width, ff) for width, ff in sizes]
+    def __init__(self, rows: int, sizes: list, device, dtype: torch.dtype = torch.bfloat16):
+        words = [_chain("_room", dtype)(rows, width, ff) for width, ff in sizes]
         begins = [sum(-(-w // 4) * 4 for w in words[:i]) for i in range(len(words) + 1)]
         room = torch.full((begins[-1],), -1, dtype=torch.int32, device=device)
         self.layers = [room[at:at + count] for at, count in zip(begins, words)]
@@ -1209,33 +1217,36 @@ class ChainRoom:
 
 def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch.Tensor, w_out: torch.Tensor, w_gated: torch.Tensor, w_down: torch.Tensor,
                gain: torch.Tensor, eps: float, activation: str, following: tuple | None = None, looks: int | None = None) -> tuple:
-    """The products behind a layer's attention in one launch, all weights in strips (``weights_in_strips``): the mixer's output projection of ``rows`` joins
-    ``stream`` (which stays as it is), the gated feed-forward behind the norm of ``gain`` and ``eps`` joins that, and, with ``following`` =
-    (weights, gain, eps), the next layer's first projection behind its norm.  (stream, projection or None) comes back.
+    """The products behind a layer's attention in one launch, bfloat16 weights in strips (``weights_in_strips``) or 32-bit ones as stored: the mixer's
+    output projection of ``rows`` joins ``stream`` (which stays as it is), the gated feed-forward behind the norm of ``gain`` and ``eps`` joins that, and,
+    with ``following`` = (weights, gain, eps), the next layer's first projection behind its norm.  (stream, projection or None) comes back.
     ``laid``: ``stream`` is one that a chain with a ``following`` gave: its values lie in the order the next chain loads them.
     ``room``: one layer's of a ``ChainRoom`` that no chain has used.  ``looks``: how often a workgroup looks for its rows before it works
     them out itself."""
-    lib = library()
+    dtype = rows.dtype
+    if dtype not in (torch.bfloat16, torch.float32):
+        raise TensorError(f"mixer output {dtype} for a chain of products")
     n, width = stream.shape
     inner, ff = rows.shape[1], w_down.shape[1]
     _need(stream, "residual stream", (n, width), torch.float32)
-    _need(rows, "mixer output", (n, inner), torch.bfloat16)
-    _need(room, "room for a chain", (lib.pl_gemm_chain_room(n, width, ff),), torch.int32)
-    at = lib.pl_gemm_chain_out(n, width, ff)
+    _need(rows, "mixer output", (n, inner), dtype)
+    _need(room, "room for a chain", (_chain("_room", dtype)(n, width, ff),), torch.int32)
+    at = _chain("_out", dtype)(n, width, ff)
     out = room[at:at + n * width].view(torch.float32).view(n, width)
-    _need(w_out, "output projection in strips", (width, inner), torch.bfloat16)
-    _need(w_gated, "gate and up projections in strips", (2 * ff, width), torch.bfloat16)
-    _need(w_down, "down projection in strips", (width, ff), torch.bfloat16)
+    how = " in strips" if dtype == torch.bfloat16 else ""
+    _need(w_out, "output projection" + how, (width, inner), dtype)
+    _need(w_gated, "gate and up projections" + how, (2 * ff, width), dtype)
+    _need(w_down, "down projection" + how, (width, ff), dtype)
     _need(gain, "norm gain", (width,), torch.float32)
     w_next = gain_next = projected = None
     after, eps_next = 0, 0.0
     if following is not None:
         w_next, gain_next, eps_next = following
         after = w_next.shape[0]
-        _need(w_next, "next projection in strips", (after, width), torch.bfloat16)
+        _need(w_next, "next projection" + how, (after, width), dtype)
         _need(gain_next, "norm gain", (width,), torch.float32)
-        projected = torch.empty((n, after), dtype=torch.bfloat16, device=stream.device)
-    _check(lib.pl_gemm_chain(
+        projected = torch.empty((n, after), dtype=dtype, device=stream.device)
+    _check(_chain("", dtype)(
         stream.data_ptr(), 1 if laid else 0, rows.data_ptr(), room.data_ptr(), _ptr(projected), w_out.data_ptr(), w_gated.data_ptr(), w_down.data_ptr(), _ptr(w_next), gain.data_ptr(), float(eps), _ptr(gain_next), float(eps_next), n, width, inner, ff, after,
         activation_code(activation), CHAIN_LOOKS if looks is None else looks, _stream()))
     return out, projected

@@ -86,15 +86,15 @@ class PreNormBlock:
     def chain_sizes(self):
         """(stream, output projection's inner width, feed-forward, first projection's columns) of a layer whose products may run as one launch a
         layer (``kernels.gemm_chain``), or None: attention and a gated feed-forward without biases, norms that products take as their first stage,
-        bfloat16 weights in strips."""
+        weights that a chain reads (``Linear.chain_weight``)."""
         ours, theirs = getattr(self.mixer, "chain_products", None), getattr(self.feed_forward, "chain_products", None)
-        if self.dtype != torch.bfloat16 or ours is None or theirs is None or type(self).forward is not PreNormBlock.forward:
+        if ours is None or theirs is None or type(self).forward is not PreNormBlock.forward:
             return None
         if not all(getattr(n, "fuses_into_product", False) for n in (self.norm1, self.norm2)):
             return None
         linears = (*ours, *theirs[:2])
-        if any(l.bias is not None or l.strips is None for l in linears) or not kernels.in_pieces(
-                *(l.strips for l in linears), self.norm1.gain32, self.norm2.gain32):
+        if any(l.bias is not None or l.chain_weight is None for l in linears) or not kernels.in_pieces(
+                *(l.chain_weight for l in linears), self.norm1.gain32, self.norm2.gain32):
             return None
         first, out = ours
         return out.out_features, out.in_features, theirs[1].in_features, first.out_features
@@ -106,7 +106,7 @@ class PreNormBlock:
             x = PendingNorm(self.norm1, resid, self.dtype) if delta is None else self.norm1.apply(resid, delta, self.dtype)
         rows = self.mixer.attend(x, ctx, projected=chain.projected)
         gate_up, down, activation = self.feed_forward.chain_products
-        chain.run(resid, rows, self.mixer.chain_products[1].strips, gate_up.strips, down.strips, self.norm2, activation)
+        chain.run(resid, rows, self.mixer.chain_products[1].chain_weight, gate_up.chain_weight, down.chain_weight, self.norm2, activation)
         return None
 
     def forward(self, resid, delta, ctx):

@@ -92,6 +92,11 @@ class Linear:
         """What a product of many rows reads for the weight."""
         return self.weight if self.strips is None else self.strips
 
+    @property
+    def chain_weight(self) -> torch.Tensor | None:
+        """What a chain of products (``kernels.gemm_chain``) reads for the weight: the strips, or a 32-bit matrix as stored."""
+        return self.weight if self.weight.dtype == torch.float32 else self.strips
+
     def takes_norm(self, rows: int, swiglu: bool = False, activation: str = "silu", heads: bool = False) -> bool:
         """Whether a norm of many rows in front of this product is worth leaving to it (``kernels.many_takes_wins``)."""
         if (self.bias is not None or self.weight.dtype != torch.bfloat16 or (swiglu and kernels.ACTIVATIONS[activation] != kernels.ACTIVATIONS["silu"])

@@ -166,7 +166,7 @@ class Chain:
         self.stream = self.passed = None
 
     def run(self, stream, rows, w_out, w_gated, w_down, norm, activation: str) -> None:
-        following = None if self.following is None else (self.following[1].strips, self.following[0].gain32, self.following[0].eps)
+        following = None if self.following is None else (self.following[1].chain_weight, self.following[0].gain32, self.following[0].eps)
         self.stream, self.passed = kernels.gemm_chain(stream, self.laid, rows, self.room, w_out, w_gated, w_down, norm.gain32, norm.eps, activation,
                                                       following)
 
@@ -245,14 +245,14 @@ class DecoderModel:
             return {}
         schedule = self.spec.schedule
         sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
-        places = [at for at, s in enumerate(sizes) if s is not None and kernels.chain_applies(rows, *s[:3])]
+        places = [at for at, s in enumerate(sizes) if s is not None and kernels.chain_applies(rows, *s[:3], dtype=self.dtype)]
         if not places:
             return {}
-        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2]) for at in places], self.device)
+        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2]) for at in places], self.device, self.dtype)
         found = {}
         for at, layer_room in zip(places, room.layers):
             behind = None
-            if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3]):
+            if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3], dtype=self.dtype):
                 block = self.blocks[schedule[at + 1].layer]
                 behind = block.norm1, block.mixer.chain_products[0]
             found[at] = layer_room, behind

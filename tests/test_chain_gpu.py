@@ -127,3 +127,61 @@ def test_what_a_chain_does_not_take_is_refused():
         kernels.gemm_chain(stream, False, rows, kernels.ChainRoom(65, [(64, 64)], DEV).layers[0], strips[0], strips[1], strips[2], gains[0], 1e-6, "silu")
     with pytest.raises(TensorError, match="strips"):
         kernels.gemm_chain(stream[:2], False, rows[:2], kernels.ChainRoom(2, [(64, 64)], DEV).layers[0], strips[0][:32], strips[1], strips[2], gains[0], 1e-6, "silu")
+
+
+def _apart_f32(stream, rows, weights, gains, activation, follows):
+    """The 32-bit products, norms and sums a launch each."""
+    from paged_llm_rs_amd import kernels
+
+    stream = stream.clone()
+    normed = kernels.add_rmsnorm(stream, kernels.gemm_plain(rows, weights[0]), gains[0], 1e-6, torch.empty_like(stream))
+    down = kernels.gemm_plain(kernels.gemm_plain_gated(normed, weights[1], activation), weights[2])
+    normed = kernels.add_rmsnorm(stream, down, gains[1], 1e-5, torch.empty_like(stream))
+    return stream, kernels.gemm_plain(normed, weights[3]) if follows else None
+
+
+# Parts of K of one, two and three lengths (64, 128 and 192 values), whole and not, fewer of them than sixteen; both tiles of 8 rows.
+@pytest.mark.parametrize("looks", [None, 0])
+@pytest.mark.parametrize("n,width,inner,ff,after", [
+    (1, 1024, 2048, 3072, 4096), (8, 1024, 2048, 3072, 4096), (9, 1024, 2048, 3072, 4096), (16, 1024, 2048, 3072, 4096), (3, 512, 64, 64, 16),
+    (7, 576, 960, 1088, 80), (5, 960, 2112, 2048, 0), (13, 1024, 3072, 1024, 48), (12, 640, 1984, 3008, 0)])
+def test_a_chain_of_32_bit_products_gives_their_bits(n, width, inner, ff, after, looks):
+    from paged_llm_rs_amd import kernels
+
+    g = torch.Generator(device=DEV).manual_seed(n * 7919 + width + inner + ff + after)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    weights = [draw(a, b) * b ** -0.5 for a, b in ((width, inner), (2 * ff, width), (width, ff), (after or 16, width))]
+    gains = [1 + 0.1 * draw(width) for _ in range(2)]
+    stream, rows = draw(n, width), draw(n, inner)
+    if n > 2:       # what is no number, and what is next to none, stays in its row (all ones is how a stage sees that a value is not there)
+        stream.view(torch.int32)[1, 3] = -1
+        rows[2, 10] = float("inf")
+        stream[0, :5], rows[0, :5] = 1e-41, 1e-30
+    activation = "silu" if n % 2 else "gelu"
+    assert kernels.chain_applies(n, width, inner, ff, after, dtype=torch.float32)
+    room = kernels.ChainRoom(n, [(width, ff)] * 3, DEV, torch.float32)
+    want = got = stream
+    laid = False
+    for at, layer in enumerate(room.layers):
+        following = (weights[3], gains[1], 1e-5) if after and at < 2 else None
+        before = got.clone()
+        chain = kernels.gemm_chain(got, laid, rows, layer, weights[0], weights[1], weights[2], gains[0], 1e-6, activation, following, looks=looks)
+        assert torch.equal(got.view(torch.int32), before.view(torch.int32)), "the stream that goes in stays as it is"
+        (want, projected), got, laid = _apart_f32(want, rows, weights, gains, activation, following is not None), chain[0], following is not None
+        for a, b in ((got, want),) if following is None else ((chain[1], projected),):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+    finite = want.isfinite().all(dim=1).tolist()
+    assert finite == [n <= 2 or r not in (1, 2) for r in range(n)]
+
+
+def test_what_a_chain_of_32_bit_products_does_not_take_is_refused():
+    from paged_llm_rs_amd import kernels
+    from paged_llm_rs_amd.errors import TensorError
+
+    for shape in ((17, 1024, 2048, 3072, 0), (0, 1024, 2048, 3072, 0), (1, 1088, 2048, 3072, 0), (1, 448, 2048, 3072, 0), (1, 1024, 3136, 3072, 0),
+                  (1, 1024, 2048, 3136, 0), (1, 1000, 2048, 3072, 0), (1, 1024, 2080, 3072, 0), (1, 1024, 2048, 3072, 8)):
+        assert not kernels.chain_applies(*shape, dtype=torch.float32)
+    draw = lambda *shape: torch.randn(*shape, device=DEV)
+    room = kernels.ChainRoom(17, [(512, 64)], DEV, torch.float32).layers[0]
+    with pytest.raises(TensorError, match="17 rows"):
+        kernels.gemm_chain(draw(17, 512), False, draw(17, 64), room, draw(512, 64), draw(128, 512), draw(512, 64), draw(512), 1e-6, "silu")
