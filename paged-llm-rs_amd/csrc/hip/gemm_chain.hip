@@ -4,6 +4,7 @@
 //   stage 1  hidden = act(norm2(mid) . gate^T) * (norm2(mid) . up^T)
 //   stage 2  out    = mid + hidden . w_down^T
 //   stage 3  after  = norm1'(out) . w_after^T                 (the next layer's first projection; optional)
+//   stage 4  the next layer's attention of single tokens over it (optional, for few workgroups; attention_decode.hpp)
 //
 // A launch of its own takes a stage 5.2 us (one row of a stream of 1,024; weights of 4 to 12 MB that memory gives in
 // 0.8 to 2.3 us): the boundary between two kernels, weights that are asked for only then, and the drain.  Here the
@@ -31,7 +32,7 @@
 // wave here takes up to four of them, each an accumulator of its own), the stretches' tiles added in their order.  As there, the norms in front
 // of stages 1 and 3 are taken from the 32-bit stream below CN_HANDED rows, and from there on handed forward: the stage that adds
 // into the stream leaves bf16(stream * gain) and the sums of squares of its 16 columns.
-#include "gemm_chain.hpp"
+#include "attention_decode.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -43,7 +44,8 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 #define CN_STORE 3      // y = norm(x) . w^T, bfloat16
 #define CN_GATED_TAKES 4    // the same of rows that a CN_ADD_HANDS left
 #define CN_STORE_TAKES 5
-#define CN_STAGES 4
+#define CN_ATTEND 6     // the next layer's attention of single tokens, over the rows that CN_STORE left
+#define CN_STAGES 5
 #define CN_WAVES 4
 #define CN_STRETCHES 16     // of K, at most
 #define CN_ROWS 64
@@ -66,11 +68,34 @@ struct cn_stage_t {
     int first, tiles;       // its workgroups: tiles of 16 columns times parts
     int parts;              // workgroups that the tiles of 16 rows are dealt to
     int x_laid, old_laid, y_laid;
+    int y_missing;          // rows that another stage waits for, but not laid
 };
 struct cn_chain_t {
     cn_stage_t s[CN_STAGES];
     int stages, n, act, looks;
 };
+// The next layer's attention (ad_attend's arguments).
+struct cn_attend_t {
+    const bf16_t* q;
+    int q_stride;
+    bf16_t* out;
+    float *part_acc, *part_ml;
+    const int *positions, *seq_of, *block_table;
+    int max_blocks, block_size;
+    bf16_t *k_pool, *v_pool;
+    int nq, nkv, d;
+    float scale_log2e;
+    int window, splits, g;
+    uint32_t splits_magic;
+    ad_fuse_t fuse;
+    int* arrivals;
+};
+struct cn_nothing_t {};
+template <bool ATTENDS>
+using cn_attend_of = typename std::conditional<ATTENDS, cn_attend_t, cn_nothing_t>::type;
+// (where a kernel's second argument stands)
+constexpr size_t CN_ATTEND_AT = (sizeof(cn_chain_t) + alignof(cn_attend_t) - 1) / alignof(cn_attend_t) * alignof(cn_attend_t);
+#define CN_HEADS 2          // query heads a workgroup of the attention
 
 // Where value (row, col) of a laid [n, width] tensor stands: 16 rows after 16 rows, in these K step by K step of 32 columns, in the order of the
 // lanes that load it (8 columns a group, 16 bytes a load: 32-bit rows in two halves).
@@ -157,12 +182,12 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
             there = false;
             for (int look = 0; look < a.looks && !there; ++look) {
                 asm volatile("" ::: "memory");
-                const u32x4 p = load(0, 0, cn_past_l2_t{});
+                const cn_words4 p = load(0, 0, cn_past_l2_t{});
                 there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
                 if (!there) __builtin_amdgcn_s_sleep(1);
             }
         }
-        u32x4 raw[V * S][PARTS];
+        cn_words4 raw[V * S][PARTS];
         uint32_t old = 0, sums[TAKES ? CN_RUN : 1];
         for (int look = 0; look <= a.looks; ++look) {
             asm volatile("" ::: "memory");
@@ -284,7 +309,7 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
             }
         } else {
             uint32_t pair = cn_pair(GATED ? pl_activate<false>(val[0], a.act) * val[BT - 1] : val[0]);
-            if (s.y_laid && pair == PL_MISSING) pair = 0x7fff7fffu;
+            if ((s.y_laid || s.y_missing) && pair == PL_MISSING) pair = 0x7fff7fffu;
             if (mine && col % 2 == 0)
                 cn_leave(static_cast<bf16_t*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, s.N, false) : row * s.N + col), pair);
         }
@@ -306,15 +331,32 @@ __device__ __forceinline__ bool cn_add(const cn_chain_t& a, const cn_stage_t& s,
     return cn_form<KIND, 4, 6>(a, s, stage, place, trust, red, ssq_lds, late);
 }
 
+// A word of every line of the kernel's arguments, asked for at once: which of the lines a workgroup reads it learns from the first of them, and a
+// second trip for another costs every workgroup some 0.5 us before it asks for its weights.
+__device__ __forceinline__ void cn_touch_arguments(int bytes) {
+    const __attribute__((address_space(4))) uint32_t* args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t words[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) words[i] = i * 64 < bytes ? args[i * 16] : 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) asm volatile("" ::"s"(words[i]));
+}
+
 // 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
 // first three stages of the 0.6B shape and most of the 256 of the last).
-template <bool HANDED>
-__global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a) {
-    __shared__ float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
+// KEYS > 0: the attention is the last stage, so many keys a lane group asks for at once.
+template <bool HANDED, int KEYS>
+__global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a, cn_attend_of<(KEYS > 0)>) {
+    __shared__ __attribute__((aligned(16))) float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
     __shared__ float ssq_lds[2 * CN_WAVES * 16];
     __shared__ int late;
+    cn_touch_arguments(sizeof(cn_chain_t) + (KEYS > 0 ? sizeof(cn_attend_t) : 0));
     int stage = 0;
-    while (stage + 1 < a.stages && static_cast<int>(blockIdx.x) >= a.s[stage + 1].first) ++stage;
+#pragma unroll
+    for (int i = 1; i < CN_STAGES; ++i) {
+        const int at = static_cast<int>(blockIdx.x) - a.s[i].first;
+        if (i < a.stages && at >= 0 && at < a.s[i].tiles) stage = i;
+    }
     const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
     if (threadIdx.x == 0) late = 0;
     __syncthreads();
@@ -325,7 +367,21 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
         q = __builtin_amdgcn_readfirstlane(q);
         const cn_stage_t& s = a.s[p];
         bool done;
-        if constexpr (HANDED) {
+        if (KEYS > 0 && s.kind == CN_ATTEND) {
+            if constexpr (KEYS > 0) {
+                // (read here, where they are needed: as values kept from the kernel's beginning on they spill)
+                const __attribute__((address_space(4))) char* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(args));
+                cn_attend_t next;
+                __builtin_memcpy(&next, (const void*)(args + CN_ATTEND_AT), sizeof(next));
+                const int token = q / next.nkv, split = token / a.n;
+                done = ad_attend<16, CN_HEADS, KEYS, CN_WAVES, 0, true>(
+                    next.q, next.q_stride, next.out, next.part_acc, next.part_ml, next.positions, next.seq_of, nullptr, 0, 0, next.block_table,
+                    next.max_blocks, next.block_size, next.k_pool, next.v_pool, next.nq, next.nkv, next.d, next.scale_log2e, next.window, next.splits, 1,
+                    next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * a.n, split, red,
+                    ad_rows_t{!trust, a.looks, &late});
+            }
+        } else if constexpr (HANDED) {
             if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
             else if (s.kind == CN_ADD_HANDS) done = cn_add<CN_ADD_HANDS>(a, s, p, q, trust, red, ssq_lds, &late);
             else if (s.kind == CN_GATED_TAKES) done = cn_form<CN_GATED_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
@@ -374,31 +430,39 @@ extern "C" int pl_gemm_chain_applies(int n, int width, int inner, int ff, int af
            && cn_stretches(width, CN_STORE) && cn_stretches(inner, CN_ADD) && cn_stretches(ff, CN_ADD);
 }
 
-// The 32-bit words that one launch leaves between its stages, all ones before it: mid [n, width], hidden [n, ff] in bfloat16, out [n, width], and, from CN_HANDED
-// rows on, the two norms handed forward, rows [n, width] in bfloat16 and sums [n, width / 16] each.  `out` begins at word out_at.
-static size_t cn_room(int n, int width, int ff, size_t* out_at) {
+// The 32-bit words that one launch leaves between its stages, all ones before it: mid [n, width], hidden [n, ff] in bfloat16, out [n, width], from CN_HANDED
+// rows on the two norms handed forward, rows [n, width] in bfloat16 and sums [n, width / 16] each, and, where the launch goes on to the next layer's
+// attention, the rows [n, after] in bfloat16 in between.  `out` begins at word out_at.
+static size_t cn_room(int n, int width, int ff, int attended, size_t* out_at) {
     const size_t stream = static_cast<size_t>(n) * width, handed = n >= CN_HANDED ? stream / 2 + stream / 16 : 0;
     if (out_at) *out_at = stream + static_cast<size_t>(n) * ff / 2;
-    return 2 * stream + static_cast<size_t>(n) * ff / 2 + 2 * handed;
+    return 2 * stream + static_cast<size_t>(n) * ff / 2 + 2 * handed + static_cast<size_t>(n) * attended / 2;
 }
-extern "C" long pl_gemm_chain_room(int n, int width, int ff) { return static_cast<long>(cn_room(n, width, ff, nullptr)); }
+extern "C" long pl_gemm_chain_room(int n, int width, int ff, int attended) { return static_cast<long>(cn_room(n, width, ff, attended, nullptr)); }
 extern "C" long pl_gemm_chain_out(int n, int width, int ff) {
     size_t at = 0;
-    cn_room(n, width, ff, &at);
+    cn_room(n, width, ff, 0, &at);
     return static_cast<long>(at);
+}
+
+// Whether a step's attention of single tokens (one a request, nq over nkv heads of d, so many shares of the context) may be the last stage of a chain: the
+// form of the kernel for single tokens that such a step gets, at most the workgroups that the chip holds at once.
+extern "C" int pl_gemm_chain_attends(int n, int nq, int nkv, int d, int splits) {
+    return n > 0 && n < CN_HANDED && nkv > 0 && nq % nkv == 0 && nq / nkv <= CN_HEADS && d > 64 && d <= 128 && d % 16 == 0 && splits >= 1
+           && splits <= AD_MERGE_AT_ONCE && static_cast<long>(nkv) * n * splits <= 2L * pl_compute_units();
 }
 
 // stream: [n, width] 32-bit, rows or (stream_laid) as an earlier chain left it.  rows: bfloat16 [n, inner].  The weights in strips: w_out [width, inner],
 // w_gated [2 ff, width] (gate rows first), w_down [width, ff], w_next [after, width] or null.  room: cn_room words of all ones; its `out`
 // [n, width] takes the updated stream, laid with a w_next and in rows without.  next: bfloat16 [n, after].  looks: how often a
-// workgroup looks for its rows before it works them out itself.
-extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* rows, void* room, void* next, const void* w_out,
+// workgroup looks for its rows before it works them out itself.  attend: the next layer's attention, or null.
+static int chain_launch(const float* stream, int stream_laid, const void* rows, void* room, void* next, const void* w_out,
                              const void* w_gated, const void* w_down, const void* w_next, const float* gain2, float eps2, const float* gain_next,
-                             float eps_next, int n, int width, int inner, int ff, int after, int act, int looks, hipStream_t stream_) {
+                             float eps_next, int n, int width, int inner, int ff, int after, int act, int looks, cn_attend_t* attend, hipStream_t stream_) {
     if (n == 0) return 0;
     PL_REQUIRE(pl_gemm_chain_applies(n, width, inner, ff, after), "chain of products: %d rows, a stream of %d, inner widths %d and %d, %d columns behind it", n, width, inner, ff, after);
     PL_REQUIRE(stream && rows && room && w_out && w_gated && w_down && gain2, "chain of products: an operand is missing");
-    PL_REQUIRE((w_next != nullptr) == (after > 0) && (next != nullptr) == (after > 0) && (gain_next != nullptr) == (after > 0),
+    PL_REQUIRE((w_next != nullptr) == (after > 0) && (next != nullptr) == (after > 0 && !attend) && (!attend || after > 0) && (gain_next != nullptr) == (after > 0),
                "chain of products: %d columns behind the chain", after);
     PL_REQUIRE(act >= PL_ACT_SILU && act <= PL_ACT_RELU2, "chain of products: activation code %d", act);
     PL_REQUIRE(looks >= 0, "chain of products: %d looks", looks);
@@ -407,7 +471,7 @@ extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* r
         PL_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "chain of products: an operand begins in the middle of 16 bytes");
     const bool handed = n >= CN_HANDED, follows = after > 0;
     size_t out_at = 0;
-    cn_room(n, width, ff, &out_at);
+    const size_t room_words = cn_room(n, width, ff, 0, &out_at);
     const size_t words = static_cast<size_t>(n) * width;
     float* const mid = static_cast<float*>(room);
     float* const hidden = mid + words;
@@ -421,7 +485,7 @@ extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* r
     a.n = n;
     a.act = act;
     a.looks = looks;
-    a.stages = follows ? 4 : 3;
+    a.stages = attend ? 5 : follows ? 4 : 3;
     cn_stage_t& project = a.s[0];
     project.x = rows; project.w = static_cast<const bf16_t*>(w_out); project.y = mid; project.old = stream;
     project.N = width; project.K = inner; project.kind = handed ? CN_ADD_HANDS : CN_ADD;
@@ -440,9 +504,23 @@ extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* r
     last.x = handed ? static_cast<const void*>(out_x) : out; last.w = static_cast<const bf16_t*>(w_next); last.y = next; last.gain = gain_next; last.eps = eps_next;
     last.squares = out_squares; last.N = after; last.K = width; last.kind = handed ? CN_STORE_TAKES : CN_STORE;
     last.x_laid = 1;
+    if (attend) {
+        last.y = mid + room_words;
+        last.y_missing = 1;
+        attend->q = reinterpret_cast<const bf16_t*>(last.y);
+        attend->q_stride = after;
+    }
     int grid = 0;
-    for (int i = 0; i < a.stages; ++i) {
+    for (int i = 0; i < (follows ? 4 : 3); ++i) {
         cn_stage_t& s = a.s[i];
+        if (i == 3 && attend) {
+            // The attention's workgroups before those of the projection that they wait for: behind them they began 9 us into the launch and were
+            // still asking for pages, keys and values when their rows came (at 14 us; see the figures above).
+            a.s[4].kind = CN_ATTEND;
+            a.s[4].first = grid;
+            a.s[4].tiles = attend->nkv * n * attend->splits;
+            grid += a.s[4].tiles;
+        }
         s.stretches = cn_stretches(s.K, s.kind);
         s.per = pl_ceil_div(s.K / 32, s.stretches);
         s.first = grid;
@@ -450,8 +528,52 @@ extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* r
         s.tiles = s.N / 16 * s.parts;
         grid += s.tiles;
     }
-    if (handed) gemm_chain_kernel<true><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a);
-    else gemm_chain_kernel<false><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a);
+    if (attend) {
+        // (as many keys at once as in the launch of its own, to the same bits)
+        if (a.s[4].tiles <= pl_compute_units()) gemm_chain_kernel<false, 8><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, *attend);
+        else gemm_chain_kernel<false, 4><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, *attend);
+    } else if (handed) {
+        gemm_chain_kernel<true, 0><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
+    } else {
+        gemm_chain_kernel<false, 0><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
+    }
     PL_CHECK_LAUNCH("gemm_chain");
     return 0;
+}
+
+extern "C" int pl_gemm_chain(const float* stream, int stream_laid, const void* rows, void* room, void* next, const void* w_out,
+                             const void* w_gated, const void* w_down, const void* w_next, const float* gain2, float eps2, const float* gain_next,
+                             float eps_next, int n, int width, int inner, int ff, int after, int act, int looks, hipStream_t stream_) {
+    return chain_launch(stream, stream_laid, rows, room, next, w_out, w_gated, w_down, w_next, gain2, eps2, gain_next, eps_next, n, width, inner, ff, after, act,
+                        looks, nullptr, stream_);
+}
+
+// The same, and behind the next layer's projection [q | k | v] of `after` = (nq + 2 nkv) d columns, which stays in the room, that layer's attention: as
+// pl_paged_attention_decode with fuse_mode 1 or 2 and no lengths, extras or second kernel (splits > 1: with arrivals).
+extern "C" int pl_gemm_chain_attend(const float* stream, int stream_laid, const void* rows, void* room, const void* w_out, const void* w_gated,
+                                    const void* w_down, const void* w_next, const float* gain2, float eps2, const float* gain_next, float eps_next, int n,
+                                    int width, int inner, int ff, int after, int act, int looks, void* out, float* part_acc, float* part_ml,
+                                    const int* positions, const int* seq_of, const int* block_table, int max_blocks, int block_size, void* k_pool,
+                                    void* v_pool, int nq, int nkv, int d, float scale, int window, int splits, int fuse_mode, const void* q_gain,
+                                    const void* k_gain, int gain_dtype, float eps, const float* cos_table, const float* sin_table, int rot, int* arrivals,
+                                    hipStream_t stream_) {
+    if (n == 0) return 0;
+    PL_REQUIRE(pl_gemm_chain_attends(n, nq, nkv, d, splits), "chain with attention: %d tokens, %d over %d heads of %d, %d shares", n, nq, nkv, d, splits);
+    PL_REQUIRE(after == (nq + 2 * nkv) * d && out && positions && seq_of && block_table && k_pool && v_pool && block_size > 0 && max_blocks > 0,
+               "chain with attention: rows of %d values, block size %d, %d blocks a row", after, block_size, max_blocks);
+    PL_REQUIRE(splits == 1 || (part_acc && part_ml && arrivals), "chain with attention: %d shares without a workspace", splits);
+    PL_REQUIRE(fuse_mode == 1 || fuse_mode == 2, "chain with attention: fuse mode %d", fuse_mode);
+    PL_REQUIRE(rot >= 0 && rot <= d && rot % 16 == 0, "chain with attention: a rotated width of %d of a head of %d is not fused", rot, d);
+    PL_REQUIRE((q_gain == nullptr) == (k_gain == nullptr), "chain with attention: one of the two gains is missing");
+    PL_REQUIRE(!q_gain || gain_dtype == PL_DTYPE_F32 || gain_dtype == PL_DTYPE_BF16, "chain with attention: gain dtype code %d", gain_dtype);
+    PL_REQUIRE((cos_table == nullptr) == (sin_table == nullptr) && (cos_table || rot == 0), "chain with attention: rotation tables");
+    for (const void* p : {static_cast<const void*>(k_pool), static_cast<const void*>(v_pool), q_gain, k_gain, static_cast<const void*>(cos_table),
+                          static_cast<const void*>(sin_table)})
+        PL_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0, "chain with attention: an operand begins in the middle of 16 bytes");
+    cn_attend_t attend{nullptr, 0, static_cast<bf16_t*>(out), part_acc, part_ml, positions, seq_of, block_table, max_blocks, block_size,
+                       static_cast<bf16_t*>(k_pool), static_cast<bf16_t*>(v_pool), nq, nkv, d, scale * 1.4426950408889634f, window, splits, nq / nkv,
+                       static_cast<uint32_t>((0x100000000ull + splits - 1) / static_cast<unsigned>(splits)),
+                       ad_fuse_t{q_gain, k_gain, gain_dtype, eps, cos_table, sin_table, rot, fuse_mode}, arrivals};
+    return chain_launch(stream, stream_laid, rows, room, nullptr, w_out, w_gated, w_down, w_next, gain2, eps2, gain_next, eps_next, n, width, inner, ff, after,
+                        act, looks, &attend, stream_);
 }

@@ -2,7 +2,7 @@
 #pragma once
 #include "common.hpp"
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t cn_words4 __attribute__((ext_vector_type(4)));
 
 #define PL_MISSING 0xffffffffu      // a word that nobody has written yet
 #define CN_NOWHERE 0x7ff00000u      // an offset past every buffer's end: loads give zeros there

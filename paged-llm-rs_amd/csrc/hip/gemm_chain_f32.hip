@@ -89,7 +89,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
     const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s.w) + static_cast<size_t>(n0) * K, 0,
                                                                             4u * ((GATED ? s.N : 0) + OUT) * K, 0x00027000);
     const uint32_t w_at = 4u * (wr * K + k_of(0, 0));
-    u32x4 w[V][S];
+    cn_words4 w[V][S];
 #pragma unroll
     for (int v = 0; v < V; ++v)
 #pragma unroll
@@ -114,7 +114,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
             there = false;
             for (int look = 0; look < a.looks && !there; ++look) {
                 asm volatile("" ::: "memory");
-                const u32x4 p = load(0, 0, cn_past_l2_t{});
+                const cn_words4 p = load(0, 0, cn_past_l2_t{});
                 there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
                 if (!there) __builtin_amdgcn_s_sleep(1);
             }
@@ -125,7 +125,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
         uint32_t old = 0;
 #pragma unroll
         for (int half = 0; half < S / STEPS; ++half) {
-            u32x4 x[V][STEPS];
+            cn_words4 x[V][STEPS];
             for (int look = 0; look <= a.looks; ++look) {
                 asm volatile("" ::: "memory");
                 if (ADD && half == 0) old = mine ? cn_word(s.old + cf_place(row0 + at_row, col, n, s.N, s.old_laid)) : 0u;

@@ -57,9 +57,12 @@ def _signatures(lib) -> None:
         "pl_gemm_skinny_hand": [p, p, p, i, i, i, i, i, i, p, i, f, p, p, p, i, p],
         "pl_gemm_skinny_hand_applies": [i, i, i, i, i],
         "pl_gemm_chain_applies": [i, i, i, i, i],
-        "pl_gemm_chain_room": [i, i, i],
+        "pl_gemm_chain_room": [i, i, i, i],
         "pl_gemm_chain_out": [i, i, i],
         "pl_gemm_chain": [p, i, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
+        "pl_gemm_chain_attends": [i, i, i, i, i],
+        "pl_gemm_chain_attend": [p, i, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p, p, p, p, p, p, i, i, p, p, i, i, i, f, i, i, i, p, p, i, f, p,
+                                 p, i, p, p],
         "pl_gemm_chain_f32_applies": [i, i, i, i, i],
         "pl_gemm_chain_f32_room": [i, i, i],
         "pl_gemm_chain_f32_out": [i, i, i],
@@ -616,6 +619,26 @@ def decode_splits(tokens: int, nq: int, nkv: int, max_ctx: int, d: int = 128, me
     return best
 
 
+def _fusion_args(fuse, q_row_stride: int, nq: int, nkv: int, d: int) -> tuple:
+    """What the kernels that normalise and rotate raw rows [q | k | v] themselves are told of ``fuse`` (a ``QkFusion`` or None)."""
+    mode, q_gain, k_gain, gain_code, eps, cos, sin, rot = 0, None, None, F32, 0.0, None, None, 0
+    if fuse is not None:
+        mode = 2 if fuse.write_kv else 1
+        q_gain, k_gain, eps, cos, sin, rot = fuse.q_gain, fuse.k_gain, fuse.eps, fuse.cos, fuse.sin, fuse.rot
+        if q_gain is not None:
+            _need(q_gain, "query norm gain", (d,))
+            _need(k_gain, "key norm gain", (d,), q_gain.dtype)
+            gain_code = _code(q_gain, "query norm gain")
+        if cos is not None:
+            _need(cos, "cosine table", None, torch.float32)
+            _need(sin, "sine table", tuple(cos.shape), torch.float32)
+            if cos.dim() != 2 or cos.shape[1] != rot // 2:
+                raise TensorError(f"rotary tables have shape {tuple(cos.shape)}, expected [positions, {rot // 2}]")
+        if mode == 2 and q_row_stride != (nq + 2 * nkv) * d:
+            raise TensorError(f"rows of {q_row_stride} values are not [q | k | v] of {nq}+2*{nkv} heads of {d}")
+    return mode, _ptr(q_gain), _ptr(k_gain), gain_code, float(eps), _ptr(cos), _ptr(sin), int(rot)
+
+
 def paged_attention_decode(q: torch.Tensor, q_row_stride: int, out: torch.Tensor, positions: torch.Tensor,
                            seq_of: torch.Tensor, block_table: torch.Tensor, block_size: int,
                            k_pool: torch.Tensor, v_pool: torch.Tensor, nq: int, nkv: int, d: int, scale: float,
@@ -652,30 +675,16 @@ def paged_attention_decode(q: torch.Tensor, q_row_stride: int, out: torch.Tensor
     if splits > 1:
         part_acc = torch.empty((n * nq * splits * d,), dtype=torch.float32, device=q.device)
         part_ml = torch.empty((n * nq * splits * 2,), dtype=torch.float32, device=q.device)
-    mode, q_gain, k_gain, gain_code, eps, cos, sin, rot = 0, None, None, F32, 0.0, None, None, 0
-    if fuse is not None:
-        if q_len is not None:
-            raise TensorError("the fused norm, rotation and cache write are for steps of one token a request")
-        mode = 2 if fuse.write_kv else 1
-        q_gain, k_gain, eps, cos, sin, rot = fuse.q_gain, fuse.k_gain, fuse.eps, fuse.cos, fuse.sin, fuse.rot
-        if q_gain is not None:
-            _need(q_gain, "query norm gain", (d,))
-            _need(k_gain, "key norm gain", (d,), q_gain.dtype)
-            gain_code = _code(q_gain, "query norm gain")
-        if cos is not None:
-            _need(cos, "cosine table", None, torch.float32)
-            _need(sin, "sine table", tuple(cos.shape), torch.float32)
-            if cos.dim() != 2 or cos.shape[1] != rot // 2:
-                raise TensorError(f"rotary tables have shape {tuple(cos.shape)}, expected [positions, {rot // 2}]")
-        if mode == 2 and q_row_stride != (nq + 2 * nkv) * d:
-            raise TensorError(f"rows of {q_row_stride} values are not [q | k | v] of {nq}+2*{nkv} heads of {d}")
+    if fuse is not None and q_len is not None:
+        raise TensorError("the fused norm, rotation and cache write are for steps of one token a request")
+    mode, q_gain, k_gain, gain_code, eps, cos, sin, rot = _fusion_args(fuse, q_row_stride, nq, nkv, d)
     _check(library().pl_paged_attention_decode(
         q.data_ptr(), q_row_stride, out.data_ptr(), _ptr(part_acc), _ptr(part_ml), positions.data_ptr(),
         seq_of.data_ptr(), _ptr(q_len), int(short_limit),
         int(block_table.shape[0] if live_seqs is None else live_seqs), int(short_rows if q_len is not None else 0),
         block_table.data_ptr(), block_table.shape[1], block_size,
         k_pool.data_ptr(), v_pool.data_ptr(), n, nq, nkv, d, float(scale), int(window or 0), int(splits),
-        mode, _ptr(q_gain), _ptr(k_gain), gain_code, float(eps), _ptr(cos), _ptr(sin), int(rot), _ptr(sinks),
+        mode, q_gain, k_gain, gain_code, eps, cos, sin, rot, _ptr(sinks),
         _ptr(slopes), *_more_args(more, nq, n), _arrivals_ptr(arrivals, n * nq), _stream()))
     return out
 
@@ -952,14 +961,19 @@ def attention_near(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv
     return out
 
 
+def _attends_single(batch, nq: int, nkv: int, d: int, kv, prepare: QkFusion) -> bool:
+    """Whether a bfloat16 step's attention is one kernel over the raw projection: every request brings one token."""
+    return (_attention_mode == "kernel" and batch.max_q_len == 1 and prepare.rot % 16 == 0 and not prepare.neighbours
+            and not grouped_applies(nq, nkv, d, kv.block_size))
+
+
 def attention_step(qkv: torch.Tensor, out: torch.Tensor, batch, kv, nq: int, nkv: int, d: int, scale: float,
                    window: int, prepare: QkFusion, prepared: bool = False) -> torch.Tensor:
     """Everything between the fused q/k/v projection and the output projection for the tokens of a step:
     per-head norm and rotation of q and k, the write of k and v into the pages, attention.  A step in
     which every request brings one token (in bfloat16) does all of it in the attention kernel;
     any other step runs the stand-alone kernel for the first three (or its projection has done it: ``prepared``) and then attention."""
-    if (not prepared and qkv.dtype == torch.bfloat16 and _attention_mode == "kernel" and batch.max_q_len == 1
-            and prepare.rot % 16 == 0 and not prepare.neighbours and not grouped_applies(nq, nkv, d, kv.block_size)):
+    if not prepared and qkv.dtype == torch.bfloat16 and _attends_single(batch, nq, nkv, d, kv, prepare):
         splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d, _has_arrivals(batch))
         return paged_attention_decode(qkv, qkv.shape[1], out, batch.positions, batch.seq_of, kv.block_table,
                                       kv.block_size, kv.k_pool, kv.v_pool, nq, nkv, d, scale, window, splits,
@@ -1204,23 +1218,71 @@ def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0, dt
     return bool(_chain("_applies", dtype)(rows, width, inner, ff, after))
 
 
+def _room_words(rows: int, dtype: torch.dtype, width: int, ff: int, attended: int = 0) -> int:
+    return _chain("_room", dtype)(rows, width, ff, *(() if dtype == torch.float32 else (attended,)))
+
+
+class ChainAttention:
+    """The next layer's attention as the last stage of a chain of products: what ``attention_step`` is told of it.  ``of`` makes one where such a step's
+    attention is that stage's (``pl_gemm_chain_attends``), and None otherwise."""
+
+    __slots__ = ("batch", "kv", "nq", "nkv", "d", "scale", "window", "prepare", "splits")
+
+    @classmethod
+    def of(cls, batch, kv, nq: int, nkv: int, d: int, scale: float, window: int, prepare: QkFusion):
+        if not _attends_single(batch, nq, nkv, d, kv, prepare) or not in_pieces(kv.k_pool, kv.v_pool, prepare.q_gain, prepare.k_gain, prepare.cos, prepare.sin):
+            return None
+        splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d, _has_arrivals(batch))
+        if not library().pl_gemm_chain_attends(batch.num_tokens, nq, nkv, d, splits) or (splits > 1 and _arrivals(batch, nq, splits) is None):
+            return None
+        self = cls()
+        self.batch, self.kv, self.nq, self.nkv, self.d = batch, kv, nq, nkv, d
+        self.scale, self.window, self.prepare, self.splits = scale, window, prepare, splits
+        return self
+
+    @property
+    def columns(self) -> int:
+        return (self.nq + 2 * self.nkv) * self.d
+
+    def arguments(self, device) -> tuple:
+        """(attended rows, the arguments of ``pl_gemm_chain_attend`` from its output on, what has to live until the launch is queued)."""
+        batch, kv, nq, nkv, d, splits = self.batch, self.kv, self.nq, self.nkv, self.d, self.splits
+        n = batch.num_tokens
+        _need(batch.positions, "positions", (n,), torch.int32)
+        _need(batch.seq_of, "request index of each token", (n,), torch.int32)
+        _need(kv.block_table, "block table", None, torch.int32)
+        for pool, what in ((kv.k_pool, "key pool"), (kv.v_pool, "value pool")):
+            _need(pool, what, None, torch.bfloat16)
+            if pool.dim() != 2 or pool.shape[1] != nkv * d or pool.shape[0] % kv.block_size != 0:
+                raise TensorError(f"{what} has shape {tuple(pool.shape)}, expected [pages*{kv.block_size}, {nkv * d}]")
+        out = torch.empty((n, nq * d), dtype=torch.bfloat16, device=device)
+        room = [torch.empty((n * nq * splits * each,), dtype=torch.float32, device=device) if splits > 1 else None for each in (d, 2)]
+        arrivals = _arrivals(batch, nq, splits)
+        mode, *fusion = _fusion_args(self.prepare, self.columns, nq, nkv, d)
+        return out, (out.data_ptr(), *map(_ptr, room), batch.positions.data_ptr(), batch.seq_of.data_ptr(), kv.block_table.data_ptr(),
+                     kv.block_table.shape[1], kv.block_size, kv.k_pool.data_ptr(), kv.v_pool.data_ptr(), nq, nkv, d, float(self.scale),
+                     int(self.window or 0), splits, mode, *fusion, _arrivals_ptr(arrivals, n * nq)), (room, arrivals)
+
+
 class ChainRoom:
-    """Where the stages of a step's chains of products leave their rows, for each of ``sizes`` (stream width, feed-forward width) a layer's: all words
-    ones, which is how a stage sees what is not there yet.  One launch fills them for all layers of a step."""
+    """Where the stages of a step's chains of products leave their rows, for each of ``sizes`` (stream width, feed-forward width, and, of a chain
+    that goes on to the next layer's attention, the columns of its projection) a layer's: all words ones, which is how a stage sees what is not there yet.  One launch fills them for all layers of a step."""
 
     def __init__(self, rows: int, sizes: list, device, dtype: torch.dtype = torch.bfloat16):
-        words = [_chain("_room", dtype)(rows, width, ff) for width, ff in sizes]
+        words = [_room_words(rows, dtype, *size) for size in sizes]
         begins = [sum(-(-w // 4) * 4 for w in words[:i]) for i in range(len(words) + 1)]
         room = torch.full((begins[-1],), -1, dtype=torch.int32, device=device)
         self.layers = [room[at:at + count] for at, count in zip(begins, words)]
 
 
 def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch.Tensor, w_out: torch.Tensor, w_gated: torch.Tensor, w_down: torch.Tensor,
-               gain: torch.Tensor, eps: float, activation: str, following: tuple | None = None, looks: int | None = None) -> tuple:
+               gain: torch.Tensor, eps: float, activation: str, following: tuple | None = None, looks: int | None = None,
+               attention: "ChainAttention | None" = None) -> tuple:
     """The products behind a layer's attention in one launch, bfloat16 weights in strips (``weights_in_strips``) or 32-bit ones as stored: the mixer's
     output projection of ``rows`` joins ``stream`` (which stays as it is), the gated feed-forward behind the norm of ``gain`` and ``eps`` joins that, and,
     with ``following`` = (weights, gain, eps), the next layer's first projection behind its norm.  (stream, projection or None) comes back.
     ``laid``: ``stream`` is one that a chain with a ``following`` gave: its values lie in the order the next chain loads them.
+    ``attention`` (a bfloat16 chain with a ``following``): the next layer's attention over that projection, whose rows then come back in its place.
     ``room``: one layer's of a ``ChainRoom`` that no chain has used.  ``looks``: how often a workgroup looks for its rows before it works
     them out itself."""
     dtype = rows.dtype
@@ -1230,7 +1292,9 @@ def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch
     inner, ff = rows.shape[1], w_down.shape[1]
     _need(stream, "residual stream", (n, width), torch.float32)
     _need(rows, "mixer output", (n, inner), dtype)
-    _need(room, "room for a chain", (_chain("_room", dtype)(n, width, ff),), torch.int32)
+    if attention is not None and (dtype != torch.bfloat16 or following is None):
+        raise TensorError("a chain that goes on to attention has bfloat16 rows and a following projection")
+    _need(room, "room for a chain", (_room_words(n, dtype, width, ff, attention.columns if attention is not None else 0),), torch.int32)
     at = _chain("_out", dtype)(n, width, ff)
     out = room[at:at + n * width].view(torch.float32).view(n, width)
     how = " in strips" if dtype == torch.bfloat16 else ""
@@ -1245,6 +1309,15 @@ def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch
         after = w_next.shape[0]
         _need(w_next, "next projection" + how, (after, width), dtype)
         _need(gain_next, "norm gain", (width,), torch.float32)
+        if attention is not None:
+            if after != attention.columns or attention.batch.num_tokens != n:
+                raise TensorError(f"{n} rows of {after} columns before attention over {attention.batch.num_tokens} of {attention.columns}")
+            attended, arguments, kept = attention.arguments(stream.device)
+            _check(library().pl_gemm_chain_attend(
+                stream.data_ptr(), 1 if laid else 0, rows.data_ptr(), room.data_ptr(), w_out.data_ptr(), w_gated.data_ptr(), w_down.data_ptr(), w_next.data_ptr(),
+                gain.data_ptr(), float(eps), gain_next.data_ptr(), float(eps_next), n, width, inner, ff, after, activation_code(activation),
+                CHAIN_LOOKS if looks is None else looks, *arguments, _stream()))
+            return out, attended
         projected = torch.empty((n, after), dtype=dtype, device=stream.device)
     _check(_chain("", dtype)(
         stream.data_ptr(), 1 if laid else 0, rows.data_ptr(), room.data_ptr(), _ptr(projected), w_out.data_ptr(), w_gated.data_ptr(), w_down.data_ptr(), _ptr(w_next), gain.data_ptr(), float(eps), _ptr(gain_next), float(eps_next), n, width, inner, ff, after,

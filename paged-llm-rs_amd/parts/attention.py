@@ -119,6 +119,12 @@ class PagedAttention:
         products around it (``kernels.gemm_chain``).  None for a class with a ``forward`` of its own."""
         return (self.qkv_proj, self.o_proj) if type(self).forward is PagedAttention.forward else None
 
+    def chain_attention(self, batch, kv, writes_cache: bool):
+        """This layer's attention as the last stage of the launch before it (``kernels.ChainAttention``), where it may be that."""
+        if type(self).attend is not PagedAttention.attend:
+            return None
+        return kernels.ChainAttention.of(batch, kv, self.nq, self.nkv, self.d, self.scale, self.window, self._prepare(writes_cache))
+
     def _prepare(self, writes_cache: bool):
         cos = self.rotary.cos if self.rotary is not None else None
         sin = self.rotary.sin if self.rotary is not None else None

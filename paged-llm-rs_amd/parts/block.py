@@ -101,10 +101,11 @@ class PreNormBlock:
 
     def _forward_chained(self, resid, delta, ctx):
         """The layer as two parts: what stands before the output projection, and one launch from there to the next layer's first projection."""
-        chain, x = ctx.chain, None
-        if chain.projected is None:
-            x = PendingNorm(self.norm1, resid, self.dtype) if delta is None else self.norm1.apply(resid, delta, self.dtype)
-        rows = self.mixer.attend(x, ctx, projected=chain.projected)
+        chain, rows, x = ctx.chain, ctx.chain.attended, None
+        if rows is None:
+            if chain.projected is None:
+                x = PendingNorm(self.norm1, resid, self.dtype) if delta is None else self.norm1.apply(resid, delta, self.dtype)
+            rows = self.mixer.attend(x, ctx, projected=chain.projected)
         gate_up, down, activation = self.feed_forward.chain_products
         chain.run(resid, rows, self.mixer.chain_products[1].chain_weight, gate_up.chain_weight, down.chain_weight, self.norm2, activation)
         return None

@@ -154,21 +154,26 @@ class LayerContext:
 
 class Chain:
     """One layer's launch of the products behind its attention, and what it passes on: the updated stream (a tensor of its own, which only the next
-    chain can read where there is a ``following`` layer: (norm, first projection)), and that layer's first projection.
-    ``projected`` and ``laid`` say what the layer before left of this kind."""
+    chain can read where there is a ``following`` layer: (norm, first projection, attention or None)), and that layer's first projection or, with its
+    attention, the attended rows.  ``projected``, ``attended`` and ``laid`` say what the layer before left of this kind."""
 
-    __slots__ = ("room", "following", "projected", "laid", "stream", "passed")
+    __slots__ = ("room", "following", "projected", "attended", "laid", "stream", "passed")
 
     def __init__(self, room, following, before):
         self.room, self.following = room, following
-        self.projected = before.passed if before is not None else None
+        attends = before is not None and before.following is not None and before.following[2] is not None
+        self.projected = before.passed if before is not None and not attends else None
+        self.attended = before.passed if attends else None
         self.laid = before is not None and before.following is not None
         self.stream = self.passed = None
 
     def run(self, stream, rows, w_out, w_gated, w_down, norm, activation: str) -> None:
-        following = None if self.following is None else (self.following[1].chain_weight, self.following[0].gain32, self.following[0].eps)
+        following = attention = None
+        if self.following is not None:
+            behind, projection, attention = self.following
+            following = projection.chain_weight, behind.gain32, behind.eps
         self.stream, self.passed = kernels.gemm_chain(stream, self.laid, rows, self.room, w_out, w_gated, w_down, norm.gain32, norm.eps, activation,
-                                                      following)
+                                                      following, attention=attention)
 
 
 class DecoderModel:
@@ -239,24 +244,34 @@ class DecoderModel:
                     strips += t.numel() * t.element_size()
         return stored, strips
 
-    def _chains(self, rows: int) -> dict:
-        """{place in the schedule: (room for its chain of products, (norm, first projection) of the layer behind it or None)} of a step of ``rows``."""
+    @staticmethod
+    def _cache_keys(entry) -> tuple:
+        """(key of a run's state, key of the pages that it reads, whether these are its own)."""
+        key = entry.layer if entry.cache_key is None else entry.cache_key
+        return key, key if entry.cache_from is None else entry.cache_from, entry.cache_from is None
+
+    def _chains(self, rows: int, batch, cache) -> dict:
+        """{place in the schedule: (room for its chain of products, (norm, first projection, attention or None) of the layer behind it or None)} of a
+        step of ``rows``."""
         if rows > kernels.CHAIN_ROWS:
             return {}
         schedule = self.spec.schedule
         sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
         places = [at for at, s in enumerate(sizes) if s is not None and kernels.chain_applies(rows, *s[:3], dtype=self.dtype)]
-        if not places:
-            return {}
-        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2]) for at in places], self.device, self.dtype)
-        found = {}
-        for at, layer_room in zip(places, room.layers):
-            behind = None
+        behind: dict = {}
+        for at in places:
             if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3], dtype=self.dtype):
                 block = self.blocks[schedule[at + 1].layer]
-                behind = block.norm1, block.mixer.chain_products[0]
-            found[at] = layer_room, behind
-        return found
+                attention = None
+                if self.dtype == torch.bfloat16:
+                    _, pages, own = self._cache_keys(schedule[at + 1])
+                    attention = block.mixer.chain_attention(batch, cache.layer_view(pages, batch), own)
+                behind[at] = block.norm1, block.mixer.chain_products[0], attention
+        if not places:
+            return {}
+        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2], *((behind[at][2].columns,) if at in behind and behind[at][2] is not None else ()))
+                                        for at in places], self.device, self.dtype)
+        return {at: (layer_room, behind.get(at)) for at, layer_room in zip(places, room.layers)}
 
     # -- the forward pass of one step -------------------------------------------------
 
@@ -288,12 +303,10 @@ class DecoderModel:
         schedule = self.spec.schedule
         # (kept only where a run of the schedule adds it to the stream again)
         began_with = resid.clone() if any(e.add_embedding for e in schedule) else None
-        chains = self._chains(resid.shape[0]) if trace is None else {}
+        chains = self._chains(resid.shape[0], batch, cache) if trace is None else {}
         chain = None
         for at, entry in enumerate(schedule):
-            own = entry.cache_from is None
-            key = entry.layer if entry.cache_key is None else entry.cache_key
-            ctx = LayerContext(batch, cache, key, key if own else entry.cache_from, own)
+            ctx = LayerContext(batch, cache, *self._cache_keys(entry))
             if top is not None:
                 # (a layer that runs again records under its prefix with ``.run<k>`` behind it, k = 1 for its second run)
                 again = sum(1 for e in schedule[:at] if e.layer == entry.layer)

@@ -185,3 +185,60 @@ def test_what_a_chain_of_32_bit_products_does_not_take_is_refused():
     room = kernels.ChainRoom(17, [(512, 64)], DEV, torch.float32).layers[0]
     with pytest.raises(TensorError, match="17 rows"):
         kernels.gemm_chain(draw(17, 512), False, draw(17, 64), room, draw(512, 64), draw(128, 512), draw(512, 64), draw(512), 1e-6, "silu")
+
+
+# One request and many, contexts of no key but the own one and over several rounds of 64, one share and eight; heads of 80 to 128, one and two a key head;
+# a window, no rotation, pages of another layer (no write), a row of padding.
+@pytest.mark.parametrize("looks", [None, 0])
+@pytest.mark.parametrize("nq,nkv,d,rot,contexts,bound,window,writes", [
+    (16, 8, 128, 128, [512], 1024, 0, True), (16, 8, 128, 128, [1, 2, 511, 300, 64, 65, 512, 17], 1024, 0, True),
+    (16, 8, 128, 128, [1000] * 14, 1024, 0, True), (8, 8, 80, 0, [33, 129], 2048, 100, True), (4, 2, 96, 32, [700, 3, 1], 1024, 0, False),
+    (2, 1, 112, 112, [1000], 1024, 0, True)])
+def test_a_chain_goes_on_to_the_next_layers_attention(nq, nkv, d, rot, contexts, bound, window, writes, looks):
+    """The bits of the chain and then the kernel for single tokens: the stream, the pages, the attended rows."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    width, inner, ff, bs, columns = 256, 128, 192, 16, (nq + 2 * nkv) * d
+    n = len(contexts) + 1
+    stream, rows, weights, gains = _operands(n, width, inner, ff, columns)
+    strips = [kernels.weights_in_strips(w) for w in weights]
+    blocks = -(-bound // bs)
+    g = torch.Generator(device=DEV).manual_seed(n + d)
+    table = torch.randperm(len(contexts) * blocks, generator=g, device=DEV).to(torch.int32).view(len(contexts), blocks)
+    pools = [torch.randn(table.numel() * bs, nkv * d, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    positions = torch.tensor([c - 1 for c in contexts] + [-1], dtype=torch.int32, device=DEV)
+    seq_of = torch.tensor([*range(len(contexts)), 0], dtype=torch.int32, device=DEV)
+    counters = torch.zeros(n * nq, dtype=torch.int32, device=DEV)
+    batch = SimpleNamespace(num_tokens=n, max_q_len=1, max_ctx_len=bound, positions=positions, seq_of=seq_of, has_arrivals=True, arrivals=lambda heads: counters)
+    q_gain, k_gain = ((1 + 0.2 * torch.randn(d, generator=g, device=DEV)).bfloat16() for _ in range(2))
+    angle = torch.arange(bound, device=DEV)[:, None] * 10000.0 ** (-torch.arange(max(rot // 2, 1), device=DEV) / max(rot // 2, 1))
+    prepare = kernels.QkFusion(q_gain, k_gain, 1e-6, angle.cos() if rot else None, angle.sin() if rot else None, rot, writes)
+    results = []
+    for attends in (False, True):
+        kv = SimpleNamespace(k_pool=pools[0].clone(), v_pool=pools[1].clone(), block_table=table, block_size=bs)
+        attention = kernels.ChainAttention.of(batch, kv, nq, nkv, d, d ** -0.5, window, prepare) if attends else None
+        assert (attention is not None) == attends
+        room = kernels.ChainRoom(n, [(width, ff, *((columns,) if attends else ()))], DEV).layers[0]
+        out, behind = kernels.gemm_chain(stream, False, rows, room, strips[0], strips[1], strips[2], gains[0], 1e-6, "silu", (strips[3], gains[1], 1e-5),
+                                         looks=looks, attention=attention)
+        if not attends:
+            projected, behind = behind, torch.empty(n, nq * d, dtype=torch.bfloat16, device=DEV)
+            kernels.attention_step(projected, behind, batch, kv, nq, nkv, d, d ** -0.5, window, prepare)
+        assert not counters.any()
+        results.append((out, kv.k_pool, kv.v_pool, behind[:-1]))
+    for want, got in zip(*results):
+        assert torch.equal(want, got)
+    assert torch.equal(results[0][1], pools[0]) != writes
+
+
+def test_which_attention_a_chain_goes_on_to():
+    """Up to two workgroups a compute unit, two query heads a key head and eight shares; heads of whole 16 values that sixteen lanes hold."""
+    from paged_llm_rs_amd import kernels
+
+    attends, units = kernels.library().pl_gemm_chain_attends, kernels.compute_units()
+    assert attends(1, 16, 8, 128, 8) and attends(1, 8, 8, 80, 1) and attends(1, units, units // 2, 128, 4)
+    for n, nq, nkv, d, splits in ((1, 32, 8, 128, 4), (1, 16, 8, 64, 4), (1, 16, 8, 136, 4), (1, 16, 8, 120, 4), (16, 16, 8, 128, 1), (1, 16, 8, 128, 9),
+                                  (0, 16, 8, 128, 1), (1, 2 * units + 1, 2 * units + 1, 128, 1), (15, units // 2, units // 4, 128, 1)):
+        assert not attends(n, nq, nkv, d, splits)
