@@ -96,6 +96,8 @@ using cn_attend_of = typename std::conditional<ATTENDS, cn_attend_t, cn_nothing_
 // (where a kernel's second argument stands)
 constexpr size_t CN_ATTEND_AT = (sizeof(cn_chain_t) + alignof(cn_attend_t) - 1) / alignof(cn_attend_t) * alignof(cn_attend_t);
 #define CN_HEADS 2          // query heads a workgroup of the attention
+#define CN_KEYS 8           // keys a lane group asks for at once (as in a launch of its own of at most a workgroup a compute unit, to the same bits)
+#define CN_SHARE 256        // keys of a share of the context, at most: two rounds
 
 // Where value (row, col) of a laid [n, width] tensor stands: 16 rows after 16 rows, in these K step by K step of 32 columns, in the order of the
 // lanes that load it (8 columns a group, 16 bytes a load: 32-bit rows in two halves).
@@ -344,13 +346,12 @@ __device__ __forceinline__ void cn_touch_arguments(int bytes) {
 
 // 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
 // first three stages of the 0.6B shape and most of the 256 of the last).
-// KEYS > 0: the attention is the last stage, so many keys a lane group asks for at once.
-template <bool HANDED, int KEYS>
-__global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a, cn_attend_of<(KEYS > 0)>) {
+template <bool HANDED, bool ATTENDS>
+__global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a, cn_attend_of<ATTENDS>) {
     __shared__ __attribute__((aligned(16))) float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
     __shared__ float ssq_lds[2 * CN_WAVES * 16];
     __shared__ int late;
-    cn_touch_arguments(sizeof(cn_chain_t) + (KEYS > 0 ? sizeof(cn_attend_t) : 0));
+    cn_touch_arguments(sizeof(cn_chain_t) + (ATTENDS ? sizeof(cn_attend_t) : 0));
     int stage = 0;
 #pragma unroll
     for (int i = 1; i < CN_STAGES; ++i) {
@@ -367,15 +368,15 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
         q = __builtin_amdgcn_readfirstlane(q);
         const cn_stage_t& s = a.s[p];
         bool done;
-        if (KEYS > 0 && s.kind == CN_ATTEND) {
-            if constexpr (KEYS > 0) {
+        if (ATTENDS && s.kind == CN_ATTEND) {
+            if constexpr (ATTENDS) {
                 // (read here, where they are needed: as values kept from the kernel's beginning on they spill)
                 const __attribute__((address_space(4))) char* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
                 asm volatile("" : "+s"(args));
                 cn_attend_t next;
                 __builtin_memcpy(&next, (const void*)(args + CN_ATTEND_AT), sizeof(next));
                 const int token = q / next.nkv, split = token / a.n;
-                done = ad_attend<16, CN_HEADS, KEYS, CN_WAVES, 0, true>(
+                done = ad_attend<16, CN_HEADS, CN_KEYS, CN_WAVES, 0, true>(
                     next.q, next.q_stride, next.out, next.part_acc, next.part_ml, next.positions, next.seq_of, nullptr, 0, 0, next.block_table,
                     next.max_blocks, next.block_size, next.k_pool, next.v_pool, next.nq, next.nkv, next.d, next.scale_log2e, next.window, next.splits, 1,
                     next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * a.n, split, red,
@@ -445,11 +446,16 @@ extern "C" long pl_gemm_chain_out(int n, int width, int ff) {
     return static_cast<long>(at);
 }
 
-// Whether a step's attention of single tokens (one a request, nq over nkv heads of d, so many shares of the context) may be the last stage of a chain: the
-// form of the kernel for single tokens that such a step gets, at most the workgroups that the chip holds at once.
-extern "C" int pl_gemm_chain_attends(int n, int nq, int nkv, int d, int splits) {
+// Whether a step's attention of single tokens (one a request, nq over nkv heads of d, so many shares of a context of up to `bound`) may be the last stage of
+// a chain.  At most a workgroup a compute unit: they stand in the grid before the workgroups that they wait for, and so leave these half of the
+// chip.  (512 of them filled it, and none of those began before all looks were in vain.)  At most two rounds of keys a workgroup: it has one in
+// registers when its rows come, and asks for a further one only when that is taken (us a step, last stage / a launch of its own, 0.6B shape: 1 token at a
+// context of 512 693 / 785, 4 tokens 728 / 815, 8 tokens 815 / 871, at contexts up to 1,000 958 / 972; 16 tokens, four rounds, at 512 1,044 / 1,072, at
+// 1,000 1,321 / 1,263; 32 tokens, eight rounds, 1,524 / 1,309).
+extern "C" int pl_gemm_chain_attends(int n, int nq, int nkv, int d, int splits, int bound) {
     return n > 0 && n < CN_HANDED && nkv > 0 && nq % nkv == 0 && nq / nkv <= CN_HEADS && d > 64 && d <= 128 && d % 16 == 0 && splits >= 1
-           && splits <= AD_MERGE_AT_ONCE && static_cast<long>(nkv) * n * splits <= 2L * pl_compute_units();
+           && splits <= AD_MERGE_AT_ONCE && bound > 0 && pl_ceil_div(bound, splits) <= CN_SHARE
+           && static_cast<long>(nkv) * n * splits <= pl_compute_units();
 }
 
 // stream: [n, width] 32-bit, rows or (stream_laid) as an earlier chain left it.  rows: bfloat16 [n, inner].  The weights in strips: w_out [width, inner],
@@ -529,13 +535,11 @@ static int chain_launch(const float* stream, int stream_laid, const void* rows, 
         grid += s.tiles;
     }
     if (attend) {
-        // (as many keys at once as in the launch of its own, to the same bits)
-        if (a.s[4].tiles <= pl_compute_units()) gemm_chain_kernel<false, 8><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, *attend);
-        else gemm_chain_kernel<false, 4><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, *attend);
+        gemm_chain_kernel<false, true><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, *attend);
     } else if (handed) {
-        gemm_chain_kernel<true, 0><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
+        gemm_chain_kernel<true, false><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
     } else {
-        gemm_chain_kernel<false, 0><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
+        gemm_chain_kernel<false, false><<<grid, PL_WAVE * CN_WAVES, 0, stream_>>>(a, cn_nothing_t{});
     }
     PL_CHECK_LAUNCH("gemm_chain");
     return 0;
@@ -558,7 +562,7 @@ extern "C" int pl_gemm_chain_attend(const float* stream, int stream_laid, const 
                                     const void* k_gain, int gain_dtype, float eps, const float* cos_table, const float* sin_table, int rot, int* arrivals,
                                     hipStream_t stream_) {
     if (n == 0) return 0;
-    PL_REQUIRE(pl_gemm_chain_attends(n, nq, nkv, d, splits), "chain with attention: %d tokens, %d over %d heads of %d, %d shares", n, nq, nkv, d, splits);
+    PL_REQUIRE(pl_gemm_chain_attends(n, nq, nkv, d, splits, 1), "chain with attention: %d tokens, %d over %d heads of %d, %d shares", n, nq, nkv, d, splits);
     PL_REQUIRE(after == (nq + 2 * nkv) * d && out && positions && seq_of && block_table && k_pool && v_pool && block_size > 0 && max_blocks > 0,
                "chain with attention: rows of %d values, block size %d, %d blocks a row", after, block_size, max_blocks);
     PL_REQUIRE(splits == 1 || (part_acc && part_ml && arrivals), "chain with attention: %d shares without a workspace", splits);

@@ -60,7 +60,7 @@ def _signatures(lib) -> None:
         "pl_gemm_chain_room": [i, i, i, i],
         "pl_gemm_chain_out": [i, i, i],
         "pl_gemm_chain": [p, i, p, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p],
-        "pl_gemm_chain_attends": [i, i, i, i, i],
+        "pl_gemm_chain_attends": [i, i, i, i, i, i],
         "pl_gemm_chain_attend": [p, i, p, p, p, p, p, p, p, f, p, f, i, i, i, i, i, i, i, p, p, p, p, p, p, i, i, p, p, i, i, i, f, i, i, i, p, p, i, f, p,
                                  p, i, p, p],
         "pl_gemm_chain_f32_applies": [i, i, i, i, i],
@@ -1233,7 +1233,7 @@ class ChainAttention:
         if not _attends_single(batch, nq, nkv, d, kv, prepare) or not in_pieces(kv.k_pool, kv.v_pool, prepare.q_gain, prepare.k_gain, prepare.cos, prepare.sin):
             return None
         splits = decode_splits(batch.num_tokens, nq, nkv, batch.max_ctx_len, d, _has_arrivals(batch))
-        if not library().pl_gemm_chain_attends(batch.num_tokens, nq, nkv, d, splits) or (splits > 1 and _arrivals(batch, nq, splits) is None):
+        if not library().pl_gemm_chain_attends(batch.num_tokens, nq, nkv, d, splits, batch.max_ctx_len) or (splits > 1 and _arrivals(batch, nq, splits) is None):
             return None
         self = cls()
         self.batch, self.kv, self.nq, self.nkv, self.d = batch, kv, nq, nkv, d

@@ -191,8 +191,8 @@ def test_what_a_chain_of_32_bit_products_does_not_take_is_refused():
 # a window, no rotation, pages of another layer (no write), a row of padding.
 @pytest.mark.parametrize("looks", [None, 0])
 @pytest.mark.parametrize("nq,nkv,d,rot,contexts,bound,window,writes", [
-    (16, 8, 128, 128, [512], 1024, 0, True), (16, 8, 128, 128, [1, 2, 511, 300, 64, 65, 512, 17], 1024, 0, True),
-    (16, 8, 128, 128, [1000] * 14, 1024, 0, True), (8, 8, 80, 0, [33, 129], 2048, 100, True), (4, 2, 96, 32, [700, 3, 1], 1024, 0, False),
+    (16, 8, 128, 128, [512], 1024, 0, True), (16, 8, 128, 128, [1, 2, 511, 300, 64, 65, 17], 1024, 0, True),
+    (16, 8, 128, 128, [1000] * 7, 1024, 0, True), (8, 8, 80, 0, [33, 129], 2048, 100, True), (4, 2, 96, 32, [700, 3, 1], 1024, 0, False),
     (2, 1, 112, 112, [1000], 1024, 0, True)])
 def test_a_chain_goes_on_to_the_next_layers_attention(nq, nkv, d, rot, contexts, bound, window, writes, looks):
     """The bits of the chain and then the kernel for single tokens: the stream, the pages, the attended rows."""
@@ -234,11 +234,12 @@ def test_a_chain_goes_on_to_the_next_layers_attention(nq, nkv, d, rot, contexts,
 
 
 def test_which_attention_a_chain_goes_on_to():
-    """Up to two workgroups a compute unit, two query heads a key head and eight shares; heads of whole 16 values that sixteen lanes hold."""
+    """Up to a workgroup a compute unit, two query heads a key head, eight shares and 256 keys a share; heads of whole 16 values that sixteen lanes hold."""
     from paged_llm_rs_amd import kernels
 
     attends, units = kernels.library().pl_gemm_chain_attends, kernels.compute_units()
-    assert attends(1, 16, 8, 128, 8) and attends(1, 8, 8, 80, 1) and attends(1, units, units // 2, 128, 4)
-    for n, nq, nkv, d, splits in ((1, 32, 8, 128, 4), (1, 16, 8, 64, 4), (1, 16, 8, 136, 4), (1, 16, 8, 120, 4), (16, 16, 8, 128, 1), (1, 16, 8, 128, 9),
-                                  (0, 16, 8, 128, 1), (1, 2 * units + 1, 2 * units + 1, 128, 1), (15, units // 2, units // 4, 128, 1)):
-        assert not attends(n, nq, nkv, d, splits)
+    assert attends(1, 16, 8, 128, 8, 2048) and attends(1, 8, 8, 80, 1, 256) and attends(1, units, units // 2, 128, 2, 512)
+    for n, nq, nkv, d, splits, bound in ((1, 32, 8, 128, 4, 256), (1, 16, 8, 64, 4, 256), (1, 16, 8, 136, 4, 256), (1, 16, 8, 120, 4, 256), (16, 2, 1, 128, 1, 256),
+                                         (1, 16, 8, 128, 9, 256), (0, 16, 8, 128, 1, 256), (1, units + 1, units + 1, 128, 1, 256), (1, 16, 8, 128, 4, 1025),
+                                         (1, 16, 8, 128, 4, 0), (15, units // 4, units // 8, 128, 4, 256)):
+        assert not attends(n, nq, nkv, d, splits, bound)
