@@ -405,18 +405,13 @@ ad_attend(const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
     }
 
     if constexpr (WAITS) {
-        // the rows of q, which another stage of the launch leaves past L2: one head's piece until it is there, then all
+        // the rows of q, which another stage of the launch leaves past L2
         const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(q) + static_cast<size_t>(t) * q_stride, 0, 2u * q_stride, 0x00027000);
         auto load = [&](size_t at) {
             return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, static_cast<uint32_t>(at) * 2, 0, cn_past_l2_t::value));
         };
         auto most = [](const u32x4& p) { return max(max(p.v[0], p.v[1]), max(p.v[2], p.v[3])); };
-        bool there = !rows_of.asks;
-        for (int look = 0; look < rows_of.looks && !there; ++look) {
-            asm volatile("" ::: "memory");
-            there = __all(most(load(head_at(0))) != PL_MISSING);
-            if (!there) __builtin_amdgcn_s_sleep(2);
-        }
+        bool there = false;
         for (int look = 0; look <= rows_of.looks; ++look) {
             asm volatile("" ::: "memory");
             uint32_t all = 0;

@@ -333,17 +333,6 @@ __device__ __forceinline__ bool cn_add(const cn_chain_t& a, const cn_stage_t& s,
     return cn_form<KIND, 4, 6>(a, s, stage, place, trust, red, ssq_lds, late);
 }
 
-// A word of every line of the kernel's arguments, asked for at once: which of the lines a workgroup reads it learns from the first of them, and a
-// second trip for another costs every workgroup some 0.5 us before it asks for its weights.
-__device__ __forceinline__ void cn_touch_arguments(int bytes) {
-    const __attribute__((address_space(4))) uint32_t* args = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
-    uint32_t words[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) words[i] = i * 64 < bytes ? args[i * 16] : 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) asm volatile("" ::"s"(words[i]));
-}
-
 // 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
 // first three stages of the 0.6B shape and most of the 256 of the last).
 template <bool HANDED, bool ATTENDS>

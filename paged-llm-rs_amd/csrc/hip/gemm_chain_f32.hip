@@ -239,8 +239,11 @@ __device__ __forceinline__ bool cf_form(const cf_chain_t& a, const cf_stage_t& s
 // 128 registers a lane: two workgroups a compute unit, half of a layer's weights in registers at once.
 __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(cf_chain_t a) {
     __shared__ __attribute__((aligned(16))) cf_lds_t lds;
+    cn_touch_arguments(sizeof(cf_chain_t));
     int stage = 0;
-    while (stage + 1 < a.stages && static_cast<int>(blockIdx.x) >= a.s[stage + 1].first) ++stage;
+#pragma unroll
+    for (int i = 1; i < CF_STAGES; ++i)
+        if (i < a.stages && static_cast<int>(blockIdx.x) >= a.s[i].first) stage = i;
     const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
     if (threadIdx.x == 0) lds.late = 0;
     __syncthreads();
