@@ -16,6 +16,12 @@
 // layers, weights from memory, us a layer, four launches / one: 1 row 20.8 / 15.0, 8 rows 22.8 / 15.9, 15 rows 25.3 / 18.5, 16 rows 24.8 / 18.4,
 // 32 rows 26.2 / 21.4, 48 rows 29.2 / 27.3, 64 rows 31.0 / 28.6.
 //
+// With the next layer's attention as the last stage, what is left of its launch (11.5 us of one token, 12.3 of eight, positions, pages and keys one
+// behind the other, and the boundary) is what stands behind its rows of q: one trip, the arithmetic of keys that are there, the meeting of the shares.
+// When a stage's workgroups have their rows and end, us from the launch's begin (one token, medians): output projection 4.2, 5.7; gate/up 7.5, 8.9;
+// down 10.7, 11.3; q/k/v 12.5, 13.8; attention 15.2, 19.4 (keys weighed 17.1, shares written 18.6).  A layer of a step, chain and attention apart /
+// together: one token at 512 26.2 / 21, eight 28.2 / 25.
+//
 // How a stage learns that its rows are there.  What the stages leave begins as words of all ones (PL_MISSING), and every word
 // is written once, past the XCD's L2 (relaxed atomics of device scope, as in pl_share): a word that differs is the value.
 // A result that happens to be all ones (a NaN, or a pair of them) is written as another NaN.  There is no counter: one that all
@@ -24,7 +30,7 @@
 // [row][column] cost 18.5 us a layer where 15.6 were taken laid, since a load then touches a line a row twice.
 //
 // Nothing waits for ever.  A workgroup looks `looks` times; if its rows are not there by then (workgroups are started in the order
-// of their numbers, earlier stages first, but another launch may hold the compute units they need), it works out all
+// of their numbers, what they wait for before them or, where the attention stands in front, beside them on the other half of the chip; but another launch may hold the compute units they need), it works out all
 // earlier stages' tiles itself, in their order, and then its own: the same arithmetic, so the same bits to the same words, whoever writes
 // them first.  What it wrote itself it takes without a look, so that way ends whatever anybody else does.
 //
@@ -97,6 +103,7 @@ using cn_attend_of = typename std::conditional<ATTENDS, cn_attend_t, cn_nothing_
 constexpr size_t CN_ATTEND_AT = (sizeof(cn_chain_t) + alignof(cn_attend_t) - 1) / alignof(cn_attend_t) * alignof(cn_attend_t);
 #define CN_HEADS 2          // query heads a workgroup of the attention
 #define CN_KEYS 8           // keys a lane group asks for at once (as in a launch of its own of at most a workgroup a compute unit, to the same bits)
+#define CN_ATTEND_LOOKS 128 // after which a workgroup of the attention works its own heads' rows out (some 0.15 ms)
 #define CN_SHARE 256        // keys of a share of the context, at most: two rounds
 
 // Where value (row, col) of a laid [n, width] tensor stands: 16 rows after 16 rows, in these K step by K step of 32 columns, in the order of the
@@ -352,6 +359,7 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
     __syncthreads();
     int p = stage, q = tile;
     bool trust = false;
+    int own = -1;       // (the attention's) which tile of its own heads' rows is being worked out, behind the last: all are
     while (true) {
         p = __builtin_amdgcn_readfirstlane(p);
         q = __builtin_amdgcn_readfirstlane(q);
@@ -369,7 +377,7 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
                     next.q, next.q_stride, next.out, next.part_acc, next.part_ml, next.positions, next.seq_of, nullptr, 0, 0, next.block_table,
                     next.max_blocks, next.block_size, next.k_pool, next.v_pool, next.nq, next.nkv, next.d, next.scale_log2e, next.window, next.splits, 1,
                     next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * a.n, split, red,
-                    ad_rows_t{!trust, a.looks, &late});
+                    ad_rows_t{!trust, own < 0 ? min(a.looks, CN_ATTEND_LOOKS) : a.looks, &late});
             }
         } else if constexpr (HANDED) {
             if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
@@ -388,6 +396,27 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
         __syncthreads();
         if (threadIdx.x == 0) late = 0;
         __syncthreads();
+        if constexpr (ATTENDS) {
+            // The attention's own part of the projection first, where what that reads may be there: workgroups of the attention stand in the grid
+            // before the projection's, and two launches of them side by side can fill the chip.
+            if (stage == CN_STAGES - 1 && !trust && (own < 0 || done)) {
+                const __attribute__((address_space(4))) char* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+                asm volatile("" : "+s"(args));
+                cn_attend_t next;
+                __builtin_memcpy(&next, (const void*)(args + CN_ATTEND_AT), sizeof(next));
+                const int head = next.d / 16, heads = next.g * head, kvh = tile % next.nkv;      // (tiles of a head, of its query heads)
+                if (++own < heads + 2 * head) {
+                    p = stage - 1;
+                    q = own < heads ? kvh * heads + own : own < heads + head ? (next.nq + kvh) * head + own - heads : (next.nq + next.nkv + kvh) * head + own - heads - head;
+                    continue;
+                }
+                if (p != stage) {
+                    p = stage;
+                    q = tile;
+                    continue;
+                }
+            }
+        }
         if (!trust) {
             trust = true;
             p = 0;
@@ -510,7 +539,7 @@ static int chain_launch(const float* stream, int stream_laid, const void* rows, 
         cn_stage_t& s = a.s[i];
         if (i == 3 && attend) {
             // The attention's workgroups before those of the projection that they wait for: behind them they began 9 us into the launch and were
-            // still asking for pages, keys and values when their rows came (at 14 us; see the figures above).
+            // still asking for pages, keys and values when their rows came, at 14 (a step of one token 785 us, so 693).
             a.s[4].kind = CN_ATTEND;
             a.s[4].first = grid;
             a.s[4].tiles = attend->nkv * n * attend->splits;

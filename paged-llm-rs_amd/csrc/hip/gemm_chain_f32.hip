@@ -6,8 +6,10 @@
 //   stage 2  out    = mid + hidden . w_down^T
 //   stage 3  after  = norm1'(out) . w_after^T                 (the next layer's first projection; optional)
 //
-// Bound by the weights' bytes (63 MB a layer of the 0.6B shape, which memory gives in some 12 us) once the launches are gone: apart they are six, two norms
-// among them, CF_MEASURED
+// Bound by the weights' bytes (63 MB a layer of the 0.6B shape, which memory gives in some 12 us) and by three trips of the rows between the stages.
+// Apart the stages are six launches, two norms among them: 42.5 us a layer at 8 rows of the 0.6B shape, this one 29; a decoding step of 8 tokens
+// 1,860 us before, 1,624 now.  Half of a layer's weights fit into the registers of the workgroups that the chip holds, and those of the last two stages are asked for
+// when earlier workgroups leave; stage 2's workgroups in the grid before stage 1's, so that theirs are among the first half, took 1,647.
 //
 // The arithmetic is that of the launches apart, to the same bits: K in the parts of gemm_f32.hip (at most 16, by K alone), a part one chain of matrix
 // instructions, the parts added in ascending order; a norm's squares in the order of add_rmsnorm_quads_kernel.

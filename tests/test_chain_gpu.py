@@ -187,9 +187,11 @@ def test_what_a_chain_of_32_bit_products_does_not_take_is_refused():
         kernels.gemm_chain(draw(17, 512), False, draw(17, 64), room, draw(512, 64), draw(128, 512), draw(512, 64), draw(512), 1e-6, "silu")
 
 
+# Looks that are over before the attention's rows can be there, and, with a few, not before what the stages in front read: a workgroup then works its
+# own heads' rows out, and everything where these have to wait as well.
 # One request and many, contexts of no key but the own one and over several rounds of 64, one share and eight; heads of 80 to 128, one and two a key head;
 # a window, no rotation, pages of another layer (no write), a row of padding.
-@pytest.mark.parametrize("looks", [None, 0])
+@pytest.mark.parametrize("looks", [None, 0, 1, 4, 8, 16])
 @pytest.mark.parametrize("nq,nkv,d,rot,contexts,bound,window,writes", [
     (16, 8, 128, 128, [512], 1024, 0, True), (16, 8, 128, 128, [1, 2, 511, 300, 64, 65, 17], 1024, 0, True),
     (16, 8, 128, 128, [1000] * 7, 1024, 0, True), (8, 8, 80, 0, [33, 129], 2048, 100, True), (4, 2, 96, 32, [700, 3, 1], 1024, 0, False),
