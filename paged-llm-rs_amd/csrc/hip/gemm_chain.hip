@@ -173,7 +173,8 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
         const int tile_rows = min(16, a.n - row0);
         const int row = row0 + tile_row;
         const bool mine = row < a.n;
-        float* const tiles = red + turn * (CN_STRETCHES * 256);        // (two of them in turn: a barrier a tile of rows)
+        float* const tiles = red + turn * (CN_STRETCHES * 256);        // (two of them in turn, and of `late`: a barrier a tile of rows, behind which a
+                                                                       // wave may be in the next tile while another has not read this one's)
         float* const squares = ssq_lds + turn * (CN_WAVES * 16);
         // where the lane's values of K step k stand: at `lane_at` + begin + k * stride
         const uint32_t begin = row0 * K * (NORM ? 4 : 2), second = NORM ? 64 * tile_rows : 0;
@@ -234,7 +235,7 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
             if (there) break;
             __builtin_amdgcn_s_sleep(1);
         }
-        if (!there && lane == 0) *late = 1;
+        if (!there && lane == 0) late[turn] = 1;
 
         f32x4 acc[BT][V];
 #pragma unroll
@@ -274,7 +275,7 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
             if (g == 0) squares[wave * 16 + c] = ssq;
         }
         __syncthreads();
-        if (__builtin_amdgcn_readfirstlane(*late)) return false;
+        if (__builtin_amdgcn_readfirstlane(late[turn])) return false;
 
         float val[BT];
 #pragma unroll
@@ -346,7 +347,7 @@ template <bool HANDED, bool ATTENDS>
 __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a, cn_attend_of<ATTENDS>) {
     __shared__ __attribute__((aligned(16))) float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles
     __shared__ float ssq_lds[2 * CN_WAVES * 16];
-    __shared__ int late;
+    __shared__ int late[2];     // (one a turn of cn_tile; the attention takes the first)
     cn_touch_arguments(sizeof(cn_chain_t) + (ATTENDS ? sizeof(cn_attend_t) : 0));
     int stage = 0;
 #pragma unroll
@@ -355,7 +356,7 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
         if (i < a.stages && at >= 0 && at < a.s[i].tiles) stage = i;
     }
     const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
-    if (threadIdx.x == 0) late = 0;
+    if (threadIdx.x < 2) late[threadIdx.x] = 0;
     __syncthreads();
     int p = stage, q = tile;
     bool trust = false;
@@ -377,24 +378,24 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
                     next.q, next.q_stride, next.out, next.part_acc, next.part_ml, next.positions, next.seq_of, nullptr, 0, 0, next.block_table,
                     next.max_blocks, next.block_size, next.k_pool, next.v_pool, next.nq, next.nkv, next.d, next.scale_log2e, next.window, next.splits, 1,
                     next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * a.n, split, red,
-                    ad_rows_t{!trust, own < 0 ? min(a.looks, CN_ATTEND_LOOKS) : a.looks, &late});
+                    ad_rows_t{!trust, own < 0 ? min(a.looks, CN_ATTEND_LOOKS) : a.looks, late});
             }
         } else if constexpr (HANDED) {
-            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
-            else if (s.kind == CN_ADD_HANDS) done = cn_add<CN_ADD_HANDS>(a, s, p, q, trust, red, ssq_lds, &late);
-            else if (s.kind == CN_GATED_TAKES) done = cn_form<CN_GATED_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
-            else done = cn_form<CN_STORE_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
+            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, late);
+            else if (s.kind == CN_ADD_HANDS) done = cn_add<CN_ADD_HANDS>(a, s, p, q, trust, red, ssq_lds, late);
+            else if (s.kind == CN_GATED_TAKES) done = cn_form<CN_GATED_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
+            else done = cn_form<CN_STORE_TAKES, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
         } else {
-            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, &late);
-            else if (s.kind == CN_GATED) done = cn_form<CN_GATED, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
-            else done = cn_form<CN_STORE, 1, 8>(a, s, p, q, trust, red, ssq_lds, &late);
+            if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, late);
+            else if (s.kind == CN_GATED) done = cn_form<CN_GATED, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
+            else done = cn_form<CN_STORE, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
         }
         if (done && p == stage && q == tile) return;
         // The rows were not there in time: all tiles of the earlier stages, then the workgroup's own once more.  (What the
         // workgroup has written is where its loads past L2 find it before the next tile begins.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (threadIdx.x == 0) late = 0;
+        if (threadIdx.x < 2) late[threadIdx.x] = 0;
         __syncthreads();
         if constexpr (ATTENDS) {
             // The attention's own part of the projection first, where what that reads may be there: workgroups of the attention stand in the grid

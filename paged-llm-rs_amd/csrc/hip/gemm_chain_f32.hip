@@ -67,7 +67,7 @@ struct cf_lds_t {
     float parts[2][CF_PARTS][CF_ROWS * 16];         // [turn][part][row][column of w]
     float gain[CF_WIDEST];
     float denom[CF_ROWS];
-    int late;
+    int late[2];        // (by turn as the parts: behind a tile's barrier a wave may be in the next tile while another has not read this one's)
 };
 
 // One tile of one stage, all rows; S steps of 16 k a part at most, FULL: every part has them.  trust: the rows were written by this workgroup.  Returns
@@ -155,7 +155,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
                 if (there) break;
                 __builtin_amdgcn_s_sleep(1);
             }
-            if (!there && lane == 0) lds.late = 1;
+            if (!there && lane == 0) lds.late[turn] = 1;
 
             if constexpr (!ADD) {
                 // x / sqrt(mean of squares + eps) * gain: sums of four squares to LDS, a wave a row adds them up as the norm kernel's workgroup does
@@ -173,7 +173,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
                         if (is_step(v, u)) fours[r * CF_FOURS + k_of(v, u) / 4] = four;
                     }
                 __syncthreads();
-                if (__builtin_amdgcn_readfirstlane(lds.late)) return false;
+                if (__builtin_amdgcn_readfirstlane(lds.late[turn])) return false;
                 for (int row = wave; row < n; row += CF_WAVES) {
                     float total = 0.f;
 #pragma unroll
@@ -211,7 +211,7 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
                 *reinterpret_cast<f32x4*>(&lds.parts[turn][wave * 2 + (ADD ? r / 8 : v)][r % ROWS * COLS + c * 4 % COLS]) = acc[v];
         }
         __syncthreads();
-        if (ADD && __builtin_amdgcn_readfirstlane(lds.late)) return false;
+        if (ADD && __builtin_amdgcn_readfirstlane(lds.late[turn])) return false;
 
         if (mine) {
             const int used = FULL ? CF_PARTS : pl_ceil_div(K, s.part_len);
@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(c
     for (int i = 1; i < CF_STAGES; ++i)
         if (i < a.stages && static_cast<int>(blockIdx.x) >= a.s[i].first) stage = i;
     const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
-    if (threadIdx.x == 0) lds.late = 0;
+    if (threadIdx.x < 2) lds.late[threadIdx.x] = 0;
     __syncthreads();
     int p = stage, q = tile;
     bool trust = false;
@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(c
         // its loads past L2 find it before the next tile begins.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (threadIdx.x == 0) lds.late = 0;
+        if (threadIdx.x < 2) lds.late[threadIdx.x] = 0;
         __syncthreads();
         if (!trust) {
             trust = true;

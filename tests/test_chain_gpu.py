@@ -245,3 +245,28 @@ def test_which_attention_a_chain_goes_on_to():
                                          (1, 16, 8, 128, 9, 256), (0, 16, 8, 128, 1, 256), (1, units + 1, units + 1, 128, 1, 256), (1, 16, 8, 128, 4, 1025),
                                          (1, 16, 8, 128, 4, 0), (15, units // 4, units // 8, 128, 4, 256)):
         assert not attends(n, nq, nkv, d, splits, bound)
+
+
+# Workgroups with two tiles of rows whose looks are over now in the first and now in the second of them, while the stage before is writing: what a
+# wave says of one tile must not reach another wave that is still at the other.
+@pytest.mark.parametrize("looks", [0, 1, 2, 4, 8])
+@pytest.mark.parametrize("n,dtype,ff", [(33, torch.bfloat16, 2048), (64, torch.bfloat16, 2048), (9, torch.float32, 3072), (16, torch.float32, 3072)])
+def test_rows_that_come_in_time_for_one_tile_and_not_for_the_next(n, dtype, ff, looks):
+    from paged_llm_rs_amd import kernels
+
+    width, inner, after = 1024, 2048, 2048
+    stream, rows, weights, gains = _operands(n, width, inner, ff, after)
+    weights, rows = [w.to(dtype) for w in weights], rows.to(dtype)
+    strips = weights if dtype == torch.float32 else [kernels.weights_in_strips(w) for w in weights]
+    results = []
+    for tries in (None, looks):
+        room = kernels.ChainRoom(n, [(width, ff)] * 12, DEV, dtype)
+        got, laid = stream, False
+        for layer in room.layers:
+            got, projected = kernels.gemm_chain(got, laid, rows, layer, strips[0], strips[1], strips[2], gains[0], 1e-6, "silu", (strips[3], gains[1], 1e-5),
+                                                looks=tries)
+            laid = True
+            results.append((tries, got.clone(), projected))
+    for (_, want, want_after), (_, got, got_after) in zip(results[:12], results[12:]):
+        assert torch.equal(want, got) and torch.equal(want_after, got_after)
+    assert torch.isfinite(results[11][1]).all()
