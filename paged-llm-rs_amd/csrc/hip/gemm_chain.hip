@@ -29,7 +29,7 @@
 // The rows between stages lie in the order in which the next stage's lanes load them ("laid", see cn_laid): 8 rows as
 // [row][column] cost 18.5 us a layer where 15.6 were taken laid, since a load then touches a line a row twice.
 //
-// Nothing waits for ever.  A workgroup looks `looks` times; if its rows are not there by then (workgroups are started in the order
+// Nothing waits for ever.  A workgroup looks `looks` times for a tile of rows, and once more at all of them; if its rows are not there by then (workgroups are started in the order
 // of their numbers, what they wait for before them or, where the attention stands in front, beside them on the other half of the chip; but another launch may hold the compute units they need), it works out all
 // earlier stages' tiles itself, in their order, and then its own: the same arithmetic, so the same bits to the same words, whoever writes
 // them first.  What it wrote itself it takes without a look, so that way ends whatever anybody else does.
@@ -186,11 +186,12 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
         };
 
         // One piece of the wave's rows is looked at until it is there (all of them would be KBs a look, by every workgroup), then
-        // all are loaded and looked at.
+        // all are loaded and looked at: once in any case, and as often again as looks are left.
         bool there = true;
+        int left = a.looks;
         if (asks) {
             there = false;
-            for (int look = 0; look < a.looks && !there; ++look) {
+            for (; left > 0 && !there; --left) {
                 asm volatile("" ::: "memory");
                 const cn_words4 p = load(0, 0, cn_past_l2_t{});
                 there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
@@ -199,7 +200,7 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
         }
         cn_words4 raw[V * S][PARTS];
         uint32_t old = 0, sums[TAKES ? CN_RUN : 1];
-        for (int look = 0; look <= a.looks; ++look) {
+        for (int again = 0; again <= left; ++again) {
             asm volatile("" ::: "memory");
             if constexpr (ADD) old = mine ? cn_word(s.old + (s.old_laid ? cn_laid(row, col, a.n, s.N, true) : row * s.N + col)) : 0u;
             if constexpr (TAKES) {
@@ -211,7 +212,7 @@ __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s
             }
             // (the first time through L2, which the workgroups of an XCD share: what a load that came too early has left there is
             // seen to be missing, and then read past L2)
-            if (stage == 0 || (asks && look == 0)) {
+            if (stage == 0 || (asks && again == 0)) {
 #pragma unroll
                 for (int u = 0; u < V * S; ++u)
 #pragma unroll

@@ -112,9 +112,10 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
             return __builtin_amdgcn_raw_buffer_load_b128(rows, is_step(v, u) ? x_at : CN_NOWHERE, (v * s.part_len + u * 16) * each, decltype(policy)::value);
         };
         bool there = true;
-        if (asks) {         // (one piece of the wave's rows until it is there, then all of them)
+        int left = a.looks;
+        if (asks) {         // (one piece of the wave's rows until it is there, then all of them: once in any case, and as often again as looks are left)
             there = false;
-            for (int look = 0; look < a.looks && !there; ++look) {
+            for (; left > 0 && !there; --left) {
                 asm volatile("" ::: "memory");
                 const cn_words4 p = load(0, 0, cn_past_l2_t{});
                 there = __all(max(max(p[0], p[1]), max(p[2], p[3])) != PL_MISSING);
@@ -128,11 +129,11 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
 #pragma unroll
         for (int half = 0; half < S / STEPS; ++half) {
             cn_words4 x[V][STEPS];
-            for (int look = 0; look <= a.looks; ++look) {
+            for (int again = 0; again <= left; ++again) {
                 asm volatile("" ::: "memory");
                 if (ADD && half == 0) old = mine ? cn_word(s.old + cf_place(row0 + at_row, col, n, s.N, s.old_laid)) : 0u;
                 // (the first time through L2, which the workgroups of an XCD share; what a load that came too early has left there is seen to be missing)
-                if (stage == 0 || (asks && look == 0)) {
+                if (stage == 0 || (asks && again == 0)) {
 #pragma unroll
                     for (int v = 0; v < V; ++v)
 #pragma unroll
@@ -155,7 +156,10 @@ __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s
                 if (there) break;
                 __builtin_amdgcn_s_sleep(1);
             }
-            if (!there && lane == 0) lds.late[turn] = 1;
+            if (!there) {
+                left = 0;       // (of the second half too)
+                if (lane == 0) lds.late[turn] = 1;
+            }
 
             if constexpr (!ADD) {
                 // x / sqrt(mean of squares + eps) * gain: sums of four squares to LDS, a wave a row adds them up as the norm kernel's workgroup does
