@@ -30,9 +30,17 @@
 // [row][column] cost 18.5 us a layer where 15.6 were taken laid, since a load then touches a line a row twice.
 //
 // Nothing waits for ever.  A workgroup looks `looks` times for a tile of rows, and once more at all of them; if its rows are not there by then (workgroups are started in the order
-// of their numbers, what they wait for before them or, where the attention stands in front, beside them on the other half of the chip; but another launch may hold the compute units they need), it works out all
-// earlier stages' tiles itself, in their order, and then its own: the same arithmetic, so the same bits to the same words, whoever writes
-// them first.  What it wrote itself it takes without a look, so that way ends whatever anybody else does.
+// of their numbers, what they wait for before them or, where the attention stands in front, beside them on the other half of the chip; but another launch may hold the compute units they need), it finds
+// out which places of the earlier stages are missing, stage by stage, works them out, and then its own: the same arithmetic, so the same bits to the same words, whoever writes
+// them first.  Workgroups that miss the same begin at unlike places and look again behind each, so what is missing is dealt out among them (us a
+// launch in which nobody may wait, 0.6B shape: 1 row 48, 8 rows 100; each by itself working all earlier stages out 1,250).  What is known to be there is taken without a
+// look, so that way ends whatever anybody else does.
+//
+// Beside others on the chip (us a step of eight tokens at a context of 512, launches apart / chains): alone 1,093 / 811, two streams 1,365 / 1,060, three
+// 1,665 / 1,662, four 2,010 / 3,000, where the attention's workgroups wait on half of the chip for each of them (chains without attention 2,080); one
+// token alone 985 / 676, four streams 1,475 / 1,300; two prompts of 64 rows in two processes 1,690 / 1,890, where one alone is 1,208 / 1,107.  From three processes on
+// the hardware gives the chip, compute die by compute die, to some of them at a time: then chains wait for workgroups that are not on it (four processes of eight
+// tokens each, all their steps in two seconds 1,575 / 1,240 to 1,770; three of 64 rows 1,845 / 700).
 //
 // The arithmetic is gemm_skinny's for one tile of rows, to the same bits: K in as many stretches as that launch has waves (a
 // wave here takes up to four of them, each an accumulator of its own), the stretches' tiles added in their order.  As there, the norms in front
@@ -103,7 +111,7 @@ using cn_attend_of = typename std::conditional<ATTENDS, cn_attend_t, cn_nothing_
 constexpr size_t CN_ATTEND_AT = (sizeof(cn_chain_t) + alignof(cn_attend_t) - 1) / alignof(cn_attend_t) * alignof(cn_attend_t);
 #define CN_HEADS 2          // query heads a workgroup of the attention
 #define CN_KEYS 8           // keys a lane group asks for at once (as in a launch of its own of at most a workgroup a compute unit, to the same bits)
-#define CN_ATTEND_LOOKS 128 // after which a workgroup of the attention works its own heads' rows out (some 0.15 ms)
+#define CN_ATTEND_LOOKS 128 // after which a workgroup of the attention sees to its token's row itself (some 0.15 ms; with 64 and 256 four streams took the same or more)
 #define CN_SHARE 256        // keys of a share of the context, at most: two rounds
 
 // Where value (row, col) of a laid [n, width] tensor stands: 16 rows after 16 rows, in these K step by K step of 32 columns, in the order of the
@@ -121,8 +129,8 @@ __device__ __forceinline__ uint32_t cn_pair(float f) {
     return half | static_cast<uint32_t>(__shfl_down(half, 4, PL_WAVE)) << 16;
 }
 
-// One tile of 16 columns of one stage, all rows.  V stretches of K a wave, of at most S K steps of 32.  trust: the rows were written by this
-// workgroup.  FULL: every stretch of the 4 V has S steps (asking that of each load costs 8 rows 1.4 us a layer).  Returns whether the tile is done (false: its rows were not there in time), the same for
+// One tile of 16 columns of one stage, all rows.  V stretches of K a wave, of at most S K steps of 32.  trust: this workgroup knows that the rows
+// are there.  FULL: every stretch of the 4 V has S steps (asking that of each load costs 8 rows 1.4 us a layer).  Returns whether the tile is done (false: its rows were not there in time), the same for
 // all threads.
 template <int KIND, int V, int S, bool FULL>
 __device__ __forceinline__ bool cn_tile(const cn_chain_t& a, const cn_stage_t& s, int stage, int place, bool trust, float* red, float* ssq_lds,
@@ -342,6 +350,46 @@ __device__ __forceinline__ bool cn_add(const cn_chain_t& a, const cn_stage_t& s,
     return cn_form<KIND, 4, 6>(a, s, stage, place, trust, red, ssq_lds, late);
 }
 
+// A place of a stage (tile of columns, part of the rows) whose results in rows row0 to row1 are not all there, the first from `from` on, so that workgroups
+// that miss the same begin with unlike ones; -1: all are there.
+template <bool HANDED>
+__device__ __forceinline__ int cn_missing_place(const __attribute__((address_space(4))) cn_chain_t& a, int stage, int from, int row0, int row1, float* lds) {
+    const auto& s = a.s[stage];
+    const int tiles = s.N / 16;
+    int first = INT_MAX;
+    // (`each` words of a tile's row; a look is a trip to memory, so eight are on their way together)
+    auto look = [&](int each, auto at) {
+        const int step = PL_WAVE * CN_WAVES / each, turns = pl_ceil_div(tiles, step);
+#pragma unroll 8
+        for (int i = 0; i < (row1 - row0) * turns; ++i) {
+            const int row = row0 + i / turns, tile = min(i % turns * step + static_cast<int>(threadIdx.x) / each, tiles - 1);
+            const uint32_t word = cn_word(reinterpret_cast<const float*>(at(row, tile, threadIdx.x % each)));
+            const int turned = tile * s.parts + row / 16 % s.parts - from;
+            first = word == PL_MISSING ? min(first, turned < 0 ? turned + s.tiles : turned) : first;
+        }
+    };
+    if (s.kind == CN_ADD || s.kind == CN_ADD_HANDS) {
+        look(16, [&](int row, int tile, int i) { return static_cast<const float*>(s.y) + cn_laid(row, tile * 16 + i, a.n, s.N, true); });
+    } else {
+        look(8, [&](int row, int tile, int i) {
+            const int col = tile * 16 + i * 2;
+            return static_cast<const bf16_t*>(s.y) + (s.y_laid ? cn_laid(row, col, a.n, s.N, false) : row * s.N + col);
+        });
+    }
+    if (HANDED && s.kind == CN_ADD_HANDS) {
+        look(8, [&](int row, int tile, int i) { return s.hand_x + cn_laid(row, tile * 16 + i * 2, a.n, s.N, false); });
+        look(1, [&](int row, int tile, int) { return s.hand_squares + static_cast<size_t>(row) * tiles + tile; });
+    }
+    int* const least = reinterpret_cast<int*>(lds);
+    if (threadIdx.x == 0) *least = INT_MAX;
+    __syncthreads();
+    if (first != INT_MAX) atomicMin(least, first);
+    __syncthreads();
+    const int found = __builtin_amdgcn_readfirstlane(*least);
+    __syncthreads();
+    return found == INT_MAX ? -1 : (found + from) % s.tiles;
+}
+
 // 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
 // first three stages of the 0.6B shape and most of the 256 of the last).
 template <bool HANDED, bool ATTENDS>
@@ -350,18 +398,19 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
     __shared__ float ssq_lds[2 * CN_WAVES * 16];
     __shared__ int late[2];     // (one a turn of cn_tile; the attention takes the first)
     cn_touch_arguments(sizeof(cn_chain_t) + (ATTENDS ? sizeof(cn_attend_t) : 0));
-    int stage = 0;
+    auto stage_of = [](const auto& a) {
+        int stage = 0;
 #pragma unroll
-    for (int i = 1; i < CN_STAGES; ++i) {
-        const int at = static_cast<int>(blockIdx.x) - a.s[i].first;
-        if (i < a.stages && at >= 0 && at < a.s[i].tiles) stage = i;
-    }
-    const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
-    if (threadIdx.x < 2) late[threadIdx.x] = 0;
+        for (int i = 1; i < CN_STAGES; ++i) {
+            const int at = static_cast<int>(blockIdx.x) - a.s[i].first;
+            if (i < a.stages && at >= 0 && at < a.s[i].tiles) stage = i;
+        }
+        return stage;
+    };
+    if (threadIdx.x == 0) late[0] = late[1] = 0;
     __syncthreads();
-    int p = stage, q = tile;
-    bool trust = false;
-    int own = -1;       // (the attention's) which tile of its own heads' rows is being worked out, behind the last: all are
+    int p = stage_of(a), q = static_cast<int>(blockIdx.x) - a.s[p].first;
+    bool trust = false, own = true;     // (own: place q of stage p is the workgroup's, and not one that it works out because it is missing)
     while (true) {
         p = __builtin_amdgcn_readfirstlane(p);
         q = __builtin_amdgcn_readfirstlane(q);
@@ -374,12 +423,13 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
                 asm volatile("" : "+s"(args));
                 cn_attend_t next;
                 __builtin_memcpy(&next, (const void*)(args + CN_ATTEND_AT), sizeof(next));
-                const int token = q / next.nkv, split = token / a.n;
+                const int n = ((const __attribute__((address_space(4))) cn_chain_t*)args)->n;
+                const int token = q / next.nkv, split = token / n;
                 done = ad_attend<16, CN_HEADS, CN_KEYS, CN_WAVES, 0, true>(
                     next.q, next.q_stride, next.out, next.part_acc, next.part_ml, next.positions, next.seq_of, nullptr, 0, 0, next.block_table,
                     next.max_blocks, next.block_size, next.k_pool, next.v_pool, next.nq, next.nkv, next.d, next.scale_log2e, next.window, next.splits, 1,
-                    next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * a.n, split, red,
-                    ad_rows_t{!trust, own < 0 ? min(a.looks, CN_ATTEND_LOOKS) : a.looks, late});
+                    next.g, next.splits_magic, next.fuse, next.arrivals, ad_extras_t<0>{}, q - token * next.nkv, token - split * n, split, red,
+                    ad_rows_t{!trust, min(a.looks, CN_ATTEND_LOOKS), late});
             }
         } else if constexpr (HANDED) {
             if (s.kind == CN_ADD) done = cn_add<CN_ADD>(a, s, p, q, trust, red, ssq_lds, late);
@@ -391,43 +441,38 @@ __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_ch
             else if (s.kind == CN_GATED) done = cn_form<CN_GATED, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
             else done = cn_form<CN_STORE, 1, 8>(a, s, p, q, trust, red, ssq_lds, late);
         }
-        if (done && p == stage && q == tile) return;
-        // The rows were not there in time: all tiles of the earlier stages, then the workgroup's own once more.  (What the
-        // workgroup has written is where its loads past L2 find it before the next tile begins.)
+        if (done && own) return;
+        // The rows were not there in time: what the earlier stages have not left yet, stage by stage, then the workgroup's own once more.  (What the
+        // workgroup has written is where its loads past L2 find it before it goes on.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (threadIdx.x < 2) late[threadIdx.x] = 0;
-        __syncthreads();
-        if constexpr (ATTENDS) {
-            // The attention's own part of the projection first, where what that reads may be there: workgroups of the attention stand in the grid
-            // before the projection's, and two launches of them side by side can fill the chip.
-            if (stage == CN_STAGES - 1 && !trust && (own < 0 || done)) {
-                const __attribute__((address_space(4))) char* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
-                asm volatile("" : "+s"(args));
-                cn_attend_t next;
-                __builtin_memcpy(&next, (const void*)(args + CN_ATTEND_AT), sizeof(next));
-                const int head = next.d / 16, heads = next.g * head, kvh = tile % next.nkv;      // (tiles of a head, of its query heads)
-                if (++own < heads + 2 * head) {
-                    p = stage - 1;
-                    q = own < heads ? kvh * heads + own : own < heads + head ? (next.nq + kvh) * head + own - heads : (next.nq + next.nkv + kvh) * head + own - heads - head;
-                    continue;
-                }
-                if (p != stage) {
-                    p = stage;
-                    q = tile;
-                    continue;
-                }
-            }
+        if (threadIdx.x == 0) {
+            int zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero));       // (as a constant it is kept through the kernel, and something else spilt)
+            late[0] = late[1] = zero;
         }
-        if (!trust) {
+        __syncthreads();
+        // (its arguments read here, where they are needed: as values kept from the kernel's beginning on they spill)
+        const __attribute__((address_space(4))) cn_chain_t* args = (const __attribute__((address_space(4))) cn_chain_t*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(args));
+        const int stage = stage_of(*args), place = static_cast<int>(blockIdx.x) - args->s[stage].first;
+        int row0 = 0, row1 = args->n;
+        if (ATTENDS && stage == CN_STAGES - 1 && !trust && (own || done)) {
+            // The attention begins with its token's row of the projection, for which what that reads may be there: its workgroups stand in the grid
+            // before the projection's, and several launches of them side by side can fill the chip.
+            p = stage - 1;
+            row0 = place / ((const __attribute__((address_space(4))) cn_attend_t*)((const __attribute__((address_space(4))) char*)args + CN_ATTEND_AT))->nkv % row1;
+            row1 = row0 + 1;
+        } else if (!trust) {
             trust = true;
             p = 0;
-            q = 0;
-        } else if (++q == s.tiles) {
-            ++p;
-            q = 0;
         }
-        if (p == stage) q = tile;
+        for (q = -1; p < stage; ++p) {
+            q = cn_missing_place<HANDED>(*args, p, place % args->s[p].tiles, row0, row1, red);
+            if (q >= 0) break;
+        }
+        own = q < 0;
+        if (own) q = place;
     }
 }
 

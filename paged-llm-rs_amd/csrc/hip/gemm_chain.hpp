@@ -1,5 +1,7 @@
 // What the two chains of products (gemm_chain.hip, bfloat16; gemm_chain_f32.hip) share: how a stage of a launch leaves values for the next.
 #pragma once
+#include <climits>
+
 #include "common.hpp"
 
 typedef uint32_t cn_words4 __attribute__((ext_vector_type(4)));

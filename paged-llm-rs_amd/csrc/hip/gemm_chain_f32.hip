@@ -1,5 +1,6 @@
 // The products behind a layer's attention for few rows (n <= 16) of the 32-bit path as ONE launch: the stages of gemm_chain.hip, and its way for a stage
-// to learn that its rows are there (values that all ones words wait for, bounded looks, a workgroup whose rows do not come works them out itself).
+// to learn that its rows are there (values that all ones words wait for, bounded looks, workgroups whose rows do not come share what is missing: 108 us a launch
+// of 8 rows in which nobody may wait, 5,800 when each worked all of it out).
 //
 //   stage 0  mid    = stream + rows . w_out^T
 //   stage 1  hidden = act(norm2(mid) . gate^T) * (norm2(mid) . up^T)
@@ -67,10 +68,11 @@ struct cf_lds_t {
     float parts[2][CF_PARTS][CF_ROWS * 16];         // [turn][part][row][column of w]
     float gain[CF_WIDEST];
     float denom[CF_ROWS];
+    int least;
     int late[2];        // (by turn as the parts: behind a tile's barrier a wave may be in the next tile while another has not read this one's)
 };
 
-// One tile of one stage, all rows; S steps of 16 k a part at most, FULL: every part has them.  trust: the rows were written by this workgroup.  Returns
+// One tile of one stage, all rows; S steps of 16 k a part at most, FULL: every part has them.  trust: this workgroup knows that the rows are there.  Returns
 // whether the tile is done (false: its rows were not there in time), the same for all threads.
 template <int KIND, int S, bool FULL>
 __device__ __forceinline__ bool cf_tile(const cf_chain_t& a, const cf_stage_t& s, int stage, int tile, bool trust, cf_lds_t& lds) {
@@ -242,19 +244,45 @@ __device__ __forceinline__ bool cf_form(const cf_chain_t& a, const cf_stage_t& s
     return cf_tile<KIND, S, false>(a, s, stage, tile, trust, lds);
 }
 
+// A tile of a stage whose results are not all there, the first from `from` on, so that workgroups that miss the same begin with unlike ones; -1: all are
+// there.
+__device__ __forceinline__ int cf_missing_tile(const __attribute__((address_space(4))) cf_chain_t& a, int stage, int from, cf_lds_t& lds) {
+    const auto& s = a.s[stage];
+    const int shift = s.kind == CF_STORE ? 4 : 3;       // (columns of a tile)
+    int first = INT_MAX;
+    const int turns = pl_ceil_div(s.N, CF_WAVES * PL_WAVE);
+#pragma unroll 8        // (a look is a trip to memory: eight are on their way together)
+    for (int i = 0; i < a.n * turns; ++i) {
+        const int row = i / turns, col = min(i % turns * (CF_WAVES * PL_WAVE) + static_cast<int>(threadIdx.x), s.N - 1);
+        const uint32_t word = cn_word(s.y + cf_place(row, col, a.n, s.N, s.y_laid));
+        const int turned = (col >> shift) - from;
+        first = word == PL_MISSING ? min(first, turned < 0 ? turned + s.tiles : turned) : first;
+    }
+    int* const least = &lds.least;
+    if (threadIdx.x == 0) *least = INT_MAX;
+    __syncthreads();
+    if (first != INT_MAX) atomicMin(least, first);
+    __syncthreads();
+    const int found = __builtin_amdgcn_readfirstlane(*least);
+    __syncthreads();
+    return found == INT_MAX ? -1 : (found + from) % s.tiles;
+}
+
 // 128 registers a lane: two workgroups a compute unit, half of a layer's weights in registers at once.
 __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(cf_chain_t a) {
     __shared__ __attribute__((aligned(16))) cf_lds_t lds;
     cn_touch_arguments(sizeof(cf_chain_t));
-    int stage = 0;
+    auto stage_of = [](const auto& a) {
+        int stage = 0;
 #pragma unroll
-    for (int i = 1; i < CF_STAGES; ++i)
-        if (i < a.stages && static_cast<int>(blockIdx.x) >= a.s[i].first) stage = i;
-    const int tile = static_cast<int>(blockIdx.x) - a.s[stage].first;
-    if (threadIdx.x < 2) lds.late[threadIdx.x] = 0;
+        for (int i = 1; i < CF_STAGES; ++i)
+            if (i < a.stages && static_cast<int>(blockIdx.x) >= a.s[i].first) stage = i;
+        return stage;
+    };
+    if (threadIdx.x == 0) lds.late[0] = lds.late[1] = 0;
     __syncthreads();
-    int p = stage, q = tile;
-    bool trust = false;
+    int p = stage_of(a), q = static_cast<int>(blockIdx.x) - a.s[p].first;
+    bool trust = false, own = true;     // (own: tile q of stage p is the workgroup's, and not one that it works out because it is missing)
     while (true) {
         p = __builtin_amdgcn_readfirstlane(p);
         q = __builtin_amdgcn_readfirstlane(q);
@@ -265,22 +293,31 @@ __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(c
         else if (s.part_len <= 64) done = cf_form<CF_ADD, 4>(a, s, p, q, trust, lds);
         else if (s.part_len <= 128) done = cf_form<CF_ADD, 8>(a, s, p, q, trust, lds);
         else done = cf_form<CF_ADD, 12>(a, s, p, q, trust, lds);
-        if (done && p == stage && q == tile) return;
-        // The rows were not there in time: all tiles of the earlier stages, then the workgroup's own once more.  (What the workgroup has written is where
-        // its loads past L2 find it before the next tile begins.)
+        if (done && own) return;
+        // The rows were not there in time: what the earlier stages have not left yet, stage by stage, then the workgroup's own tile once more.  (What the
+        // workgroup has written is where its loads past L2 find it before it goes on.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (threadIdx.x < 2) lds.late[threadIdx.x] = 0;
+        if (threadIdx.x == 0) {
+            int zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero));       // (as a constant it is kept through the kernel, and something else spilt)
+            lds.late[0] = lds.late[1] = zero;
+        }
         __syncthreads();
+        // (its arguments read here, where they are needed: as values kept from the kernel's beginning on they spill)
+        const __attribute__((address_space(4))) cf_chain_t* args = (const __attribute__((address_space(4))) cf_chain_t*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(args));
+        const int stage = stage_of(*args), tile = static_cast<int>(blockIdx.x) - args->s[stage].first;
         if (!trust) {
             trust = true;
             p = 0;
-            q = 0;
-        } else if (++q == s.tiles) {
-            ++p;
-            q = 0;
         }
-        if (p == stage) q = tile;
+        for (q = -1; p < stage; ++p) {
+            q = cf_missing_tile(*args, p, tile % args->s[p].tiles, lds);
+            if (q >= 0) break;
+        }
+        own = q < 0;
+        if (own) q = tile;
     }
 }
 

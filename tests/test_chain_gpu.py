@@ -270,3 +270,82 @@ def test_rows_that_come_in_time_for_one_tile_and_not_for_the_next(n, dtype, ff, 
     for (_, want, want_after), (_, got, got_after) in zip(results[:12], results[12:]):
         assert torch.equal(want, got) and torch.equal(want_after, got_after)
     assert torch.isfinite(results[11][1]).all()
+
+
+def _time(launch) -> float:
+    """Microseconds of ``launch(i)``, the median of nine (the first of which bring the code in)."""
+    times = []
+    for i in range(9):
+        torch.cuda.synchronize()
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        launch(i)
+        end.record()
+        end.synchronize()
+        times.append(begin.elapsed_time(end) * 1e3)
+    return sorted(times)[4]
+
+
+@pytest.mark.parametrize("n,dtype", [(1, torch.bfloat16), (8, torch.bfloat16), (8, torch.float32)])
+def test_workgroups_without_their_rows_share_what_is_missing(n, dtype):
+    """Where no workgroup may wait, each works out what it finds missing and begins with another piece than the next: 45 to 110 us a launch, and 27
+    to 44 where they wait.  Each by itself working out all that stands before it took 1,250 (in 32 bits 5,800), so a tenfold tells them apart."""
+    from paged_llm_rs_amd import kernels
+
+    stream, rows, weights, gains = _operands(n, 1024, 2048, 3072, 4096)
+    weights, rows = [w.to(dtype) for w in weights], rows.to(dtype)
+    strips = weights if dtype == torch.float32 else [kernels.weights_in_strips(w) for w in weights]
+
+    def chain(looks):
+        rooms = kernels.ChainRoom(n, [(1024, 3072)] * 9, DEV, dtype).layers
+        return lambda i: kernels.gemm_chain(stream, False, rows, rooms[i], strips[0], strips[1], strips[2], gains[0], 1e-6, "silu",
+                                            (strips[3], gains[1], 1e-5), looks=looks)
+
+    assert _time(chain(0)) < 10 * _time(chain(None))
+
+
+def test_chains_on_several_streams_give_the_bits_they_give_alone():
+    """Four streams whose chains go on to attention, a workgroup a compute unit each: together they fill the chip before any of their projections can begin."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd import kernels
+
+    n, nq, nkv, d, bs, layers, splits = 8, 16, 8, 128, 16, 12, 4
+    width, inner, ff, columns = 1024, 2048, 3072, (nq + 2 * nkv) * d
+    stream, rows, weights, gains = _operands(n, width, inner, ff, columns)
+    strips = [kernels.weights_in_strips(w) for w in weights]
+    g = torch.Generator(device=DEV).manual_seed(11)
+    table = torch.randperm(n * 64, generator=g, device=DEV).to(torch.int32).view(n, 64)
+    pools = [torch.randn(n * 64 * bs, nkv * d, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    positions, seq_of = torch.arange(505, 505 + n, dtype=torch.int32, device=DEV), torch.arange(n, dtype=torch.int32, device=DEV)
+    prepare = kernels.QkFusion(None, None, 1e-6, None, None, 0, False)
+
+    def user():
+        counters = torch.zeros(n * nq, dtype=torch.int32, device=DEV)
+        batch = SimpleNamespace(num_tokens=n, max_q_len=1, max_ctx_len=1024, positions=positions, seq_of=seq_of, has_arrivals=True, arrivals=lambda heads: counters)
+        kv = SimpleNamespace(k_pool=pools[0], v_pool=pools[1], block_table=table, block_size=bs)
+        attention = kernels.ChainAttention.of(batch, kv, nq, nkv, d, d ** -0.5, 0, prepare)
+        assert attention is not None and attention.splits == splits
+        return attention, kernels.ChainRoom(n, [(width, ff, columns)] * layers, DEV), counters
+
+    def run(attention, room):
+        got, laid, given = stream, False, []
+        for layer in room.layers:
+            got, attended = kernels.gemm_chain(got, laid, rows, layer, strips[0], strips[1], strips[2], gains[0], 1e-6, "silu", (strips[3], gains[1], 1e-5),
+                                               attention=attention)
+            laid = True
+            given += [got, attended]
+        return given
+
+    alone = run(*user()[:2])
+    users = [user() for _ in range(4)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in users]
+    given = []
+    for side, (attention, room, _) in zip(streams, users):
+        with torch.cuda.stream(side):
+            given.append(run(attention, room))
+    torch.cuda.synchronize()
+    for each, (_, _, counters) in zip(given, users):
+        assert all(torch.equal(a, b) for a, b in zip(each, alone)) and not counters.any()
+    assert torch.isfinite(alone[-1].float()).all()
