@@ -104,7 +104,9 @@ class PreNormBlock:
         chain, rows, x = ctx.chain, ctx.chain.attended, None
         if rows is None:
             if chain.projected is None:
-                x = PendingNorm(self.norm1, resid, self.dtype) if delta is None else self.norm1.apply(resid, delta, self.dtype)
+                # (a layer that is no chain may stand in front, and its last product may have left this norm's work, as in `forward`)
+                x = (PendingNorm(self.norm1, resid, self.dtype, handed=getattr(ctx, "handed", None)) if delta is None
+                     else self.norm1.apply(resid, delta, self.dtype))
             rows = self.mixer.attend(x, ctx, projected=chain.projected)
         gate_up, down, activation = self.feed_forward.chain_products
         chain.run(resid, rows, self.mixer.chain_products[1].chain_weight, gate_up.chain_weight, down.chain_weight, self.norm2, activation)
