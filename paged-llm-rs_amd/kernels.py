@@ -1219,6 +1219,27 @@ def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0, dt
     return bool(_chain("_applies", dtype)(rows, width, inner, ff, after))
 
 
+# Where a chain beats the same products a launch each, timed as decoding steps and short prompts of 28 layers (products apart over a chain, 16 shapes of
+# streams of 32 to 1,024).  In bfloat16 at all of them, from 1 row (1.15 to 1.24, with the attention behind it up to 1.52) to 64 (1.03 to 1.36).  In 32 bits from 8 rows on
+# (1.00 to 1.30; 512 wide with 1,536, 12 tokens of a prompt, 0.99 to 1.01).  With fewer a launch apart has little to do, and a chain gains on wider streams and where a feed-forward's
+# parts of K are 64 or 128 values long (1 row: 576 with 1,536 1.01, 960 with 2,048 1.03, 1,024 with 1,024 1.06) or all whole (1,024 with 3,072 1.03);
+# in parts of 192 that are not it loses at 1 and 2 rows (704 with 2,560 0.95, 960 with 2,560 0.95 and 0.99, 1,024 with 2,560 0.97 and 1.01) and at 4 on streams
+# below 768 (704 0.99, 768 1.01, 960 1.02), and at 512 wide up to 4 rows (0.95 to 1.01).
+CHAIN_F32_ROWS = 8
+CHAIN_F32_NARROW = 512
+CHAIN_F32_LONG = 2048           # the feed-forward beyond which parts are 192 values
+CHAIN_F32_LONG_ROWS, CHAIN_F32_LONG_WIDTH = 4, 768
+
+
+def chain_wins(rows: int, width: int, ff: int, dtype: torch.dtype = torch.bfloat16) -> bool:
+    """Whether a layer's products that can be a chain are faster as one."""
+    if dtype == torch.bfloat16 or rows >= CHAIN_F32_ROWS:
+        return True
+    if width <= CHAIN_F32_NARROW:
+        return False
+    return ff <= CHAIN_F32_LONG or (width, ff) == (1024, 3072) or (rows >= CHAIN_F32_LONG_ROWS and width >= CHAIN_F32_LONG_WIDTH)
+
+
 def _room_words(rows: int, dtype: torch.dtype, width: int, ff: int, attended: int = 0) -> int:
     return _chain("_room", dtype)(rows, width, ff, *(() if dtype == torch.float32 else (attended,)))
 

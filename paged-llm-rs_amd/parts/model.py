@@ -257,7 +257,8 @@ class DecoderModel:
             return {}
         schedule = self.spec.schedule
         sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
-        places = [at for at, s in enumerate(sizes) if s is not None and kernels.chain_applies(rows, *s[:3], dtype=self.dtype)]
+        places = [at for at, s in enumerate(sizes)
+                  if s is not None and kernels.chain_applies(rows, *s[:3], dtype=self.dtype) and kernels.chain_wins(rows, s[0], s[2], self.dtype)]
         behind: dict = {}
         for at in places:
             if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3], dtype=self.dtype):

@@ -170,3 +170,23 @@ def test_chains_beside_layers_that_are_none(toys, dtype, monkeypatch):
         assert got.keys() == apart.keys()
         other = [key for key, row in got.items() if not (row == apart[key]).all()]
         assert not same or not other, f"other bits at {other}"
+
+
+@pytest.mark.parametrize("hidden,inter,chained", [(1024, 192, True), (1024, 3072, True), (1024, 2560, False), (960, 2048, True), (512, 192, False)])
+def test_which_32_bit_steps_of_one_token_are_chains(tmp_path, monkeypatch, hidden, inter, chained):
+    """Of a single row a chain is not the faster way at every size that it takes (``kernels.chain_wins``); of eight it is.  Same bits."""
+    from paged_llm_rs_amd import kernels, write_random_model
+    from conftest import TINY_A
+
+    cfg = dict(TINY_A, hidden_size=hidden, intermediate_size=inter, num_attention_heads=4, num_key_value_heads=2, head_dim=16, num_hidden_layers=2)
+    folder = write_random_model(tmp_path / "model", cfg, seed=5, std=0.02, gain_std=0.1, dtype="float32")
+    prompts = ru.make_prompts(cfg["vocab_size"], [8], seed=3)
+    for steps, expected in ((ru.tail_decoded(prompts, 7), chained), (ru.whole(prompts), True)):
+        with monkeypatch.context() as m:
+            seen = _watch(m)
+            got = _replay(folder, "float32", steps, prompts, 1)
+            assert bool(seen["chains"]) == expected
+        with monkeypatch.context() as m:
+            m.setattr(kernels, "chain_applies", lambda *args, **kwargs: False)
+            apart = _replay(folder, "float32", steps, prompts, 1)
+        assert all((row == apart[key]).all() for key, row in got.items())
