@@ -85,19 +85,24 @@ class PreNormBlock:
     @property
     def chain_sizes(self):
         """(stream, output projection's inner width, feed-forward, first projection's columns) of a layer whose products may run as one launch a
-        layer (``kernels.gemm_chain``), or None: attention and a gated feed-forward without biases, norms that products take as their first stage,
-        weights that a chain reads (``Linear.chain_weight``)."""
+        layer (``kernels.gemm_chain``), or None: attention and a gated feed-forward, norms that products take as their first stage.  Whether the
+        layer's tensors are as a chain reads them is ``chain_ready``, which is asked only of layers whose sizes a chain takes."""
+        if type(self).forward is not PreNormBlock.forward:
+            return None
         ours, theirs = getattr(self.mixer, "chain_products", None), getattr(self.feed_forward, "chain_products", None)
-        if ours is None or theirs is None or type(self).forward is not PreNormBlock.forward:
-            return None
-        if not all(getattr(n, "fuses_into_product", False) for n in (self.norm1, self.norm2)):
-            return None
-        linears = (*ours, *theirs[:2])
-        if any(l.bias is not None or l.chain_weight is None for l in linears) or not kernels.in_pieces(
-                *(l.chain_weight for l in linears), self.norm1.gain32, self.norm2.gain32):
+        if ours is None or theirs is None:
             return None
         first, out = ours
         return out.out_features, out.in_features, theirs[1].in_features, first.out_features
+
+    @property
+    def chain_ready(self) -> bool:
+        """Of a layer with ``chain_sizes``: no biases, and weights and gains that a chain reads (``Linear.chain_weight``)."""
+        if not all(getattr(n, "fuses_into_product", False) for n in (self.norm1, self.norm2)):
+            return False
+        linears = (*self.mixer.chain_products, *self.feed_forward.chain_products[:2])
+        return all(l.bias is None and l.chain_weight is not None for l in linears) and kernels.in_pieces(
+            *(l.chain_weight for l in linears), self.norm1.gain32, self.norm2.gain32)
 
     def _forward_chained(self, resid, delta, ctx):
         """The layer as two parts: what stands before the output projection, and one launch from there to the next layer's first projection."""

@@ -257,22 +257,29 @@ class DecoderModel:
             return {}
         schedule = self.spec.schedule
         sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
-        places = [at for at, s in enumerate(sizes)
-                  if s is not None and kernels.chain_applies(rows, *s[:3], dtype=self.dtype) and kernels.chain_wins(rows, s[0], s[2], self.dtype)]
+        # (layers are of few sizes, and an eager step pays for whatever is asked of each)
+        takes = {s: kernels.chain_applies(rows, *s[:3], dtype=self.dtype) and kernels.chain_wins(rows, s[0], s[2], self.dtype) for s in set(sizes) - {None}}
+        places = {at for at, s in enumerate(sizes) if s is not None and takes[s] and self.blocks[schedule[at].layer].chain_ready}
+        if not places:
+            return {}
+        follows = {}
         behind: dict = {}
-        for at in places:
-            if at + 1 in places and not schedule[at + 1].add_embedding and kernels.chain_applies(rows, *sizes[at][:3], sizes[at + 1][3], dtype=self.dtype):
+        for at in sorted(places):
+            if at + 1 not in places or schedule[at + 1].add_embedding:
+                continue
+            pair = (*sizes[at][:3], sizes[at + 1][3])
+            if pair not in follows:
+                follows[pair] = kernels.chain_applies(rows, *pair, dtype=self.dtype)
+            if follows[pair]:
                 block = self.blocks[schedule[at + 1].layer]
                 attention = None
                 if self.dtype == torch.bfloat16:
                     _, pages, own = self._cache_keys(schedule[at + 1])
                     attention = block.mixer.chain_attention(batch, cache.layer_view(pages, batch), own)
                 behind[at] = block.norm1, block.mixer.chain_products[0], attention
-        if not places:
-            return {}
         room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2], *((behind[at][2].columns,) if at in behind and behind[at][2] is not None else ()))
-                                        for at in places], self.device, self.dtype)
-        return {at: (layer_room, behind.get(at)) for at, layer_room in zip(places, room.layers)}
+                                        for at in sorted(places)], self.device, self.dtype)
+        return {at: (layer_room, behind.get(at)) for at, layer_room in zip(sorted(places), room.layers)}
 
     # -- the forward pass of one step -------------------------------------------------
 
