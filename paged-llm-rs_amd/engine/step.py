@@ -40,6 +40,8 @@ from .batch import CannotFeed, CaptureOutgrown, NotNear, StepBatch, TableTooWide
 GRAPH_MAX_REQUESTS = 256     # requests a captured step may have (steps of more run kernel by kernel)
 SHAPE_GRAPH_ROWS_KEPT = 32768    # rows over all captured shapes of steps other than plain decoding (the
                                  # least recently used go first): their buffers stay allocated
+SHAPE_GRAPH_ROOM_KEPT = 2 << 30  # and bytes over them of what their layers' launches leave for each other (``step_room_bytes`` of the
+                                 # model: some 0.5 MB a row of the 0.6B shape, an order more than a row costs otherwise)
 SHAPE_GRAPH_MAX_TOKENS = 8192
 
 
@@ -417,12 +419,15 @@ class StepRunner:
         out = graph.run(entries)
         self._shapes[shape] = graph
         live = [k for k, g in self._shapes.items() if g is not None]
-        held = sum(k[0] for k in live)
+        room_of = getattr(self.model, "step_room_bytes", lambda rows: 0)
+        rooms = {rows: room_of(rows) for rows in {k[0] for k in live}}
+        held, room = sum(k[0] for k in live), sum(rooms[k[0]] for k in live)
         for k in live[:-1]:
-            if held <= SHAPE_GRAPH_ROWS_KEPT:
+            if held <= SHAPE_GRAPH_ROWS_KEPT and room <= SHAPE_GRAPH_ROOM_KEPT:
                 break
-            held -= k[0]
-            del self._shapes[k]
+            if held > SHAPE_GRAPH_ROWS_KEPT or rooms[k[0]]:
+                held, room = held - k[0], room - rooms[k[0]]
+                del self._shapes[k]
         self.graph_steps += 1
         return out
 

@@ -1240,7 +1240,8 @@ def chain_wins(rows: int, width: int, ff: int, dtype: torch.dtype = torch.bfloat
     return ff <= CHAIN_F32_LONG or (width, ff) == (1024, 3072) or (rows >= CHAIN_F32_LONG_ROWS and width >= CHAIN_F32_LONG_WIDTH)
 
 
-def _room_words(rows: int, dtype: torch.dtype, width: int, ff: int, attended: int = 0) -> int:
+def chain_room_words(rows: int, dtype: torch.dtype, width: int, ff: int, attended: int = 0) -> int:
+    """32-bit words that a layer's chain leaves between its stages (``attended``: columns of the projection whose attention it goes on to)."""
     return _chain("_room", dtype)(rows, width, ff, *(() if dtype == torch.float32 else (attended,)))
 
 
@@ -1291,7 +1292,7 @@ class ChainRoom:
     that goes on to the next layer's attention, the columns of its projection) a layer's: all words ones, which is how a stage sees what is not there yet.  One launch fills them for all layers of a step."""
 
     def __init__(self, rows: int, sizes: list, device, dtype: torch.dtype = torch.bfloat16):
-        words = [_room_words(rows, dtype, *size) for size in sizes]
+        words = [chain_room_words(rows, dtype, *size) for size in sizes]
         begins = [sum(-(-w // 4) * 4 for w in words[:i]) for i in range(len(words) + 1)]
         room = torch.full((begins[-1],), -1, dtype=torch.int32, device=device)
         self.layers = [room[at:at + count] for at, count in zip(begins, words)]
@@ -1316,7 +1317,7 @@ def gemm_chain(stream: torch.Tensor, laid: bool, rows: torch.Tensor, room: torch
     _need(rows, "mixer output", (n, inner), dtype)
     if attention is not None and (dtype != torch.bfloat16 or following is None):
         raise TensorError("a chain that goes on to attention has bfloat16 rows and a following projection")
-    _need(room, "room for a chain", (_room_words(n, dtype, width, ff, attention.columns if attention is not None else 0),), torch.int32)
+    _need(room, "room for a chain", (chain_room_words(n, dtype, width, ff, attention.columns if attention is not None else 0),), torch.int32)
     at = _chain("_out", dtype)(n, width, ff)
     out = room[at:at + n * width].view(torch.float32).view(n, width)
     how = " in strips" if dtype == torch.bfloat16 else ""

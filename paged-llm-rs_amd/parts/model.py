@@ -250,24 +250,33 @@ class DecoderModel:
         key = entry.layer if entry.cache_key is None else entry.cache_key
         return key, key if entry.cache_from is None else entry.cache_from, entry.cache_from is None
 
+    def _chain_places(self, rows: int) -> dict:
+        """{place in the schedule: sizes} of the layers whose products are a chain in a step of ``rows``."""
+        if rows > kernels.CHAIN_ROWS:
+            return {}
+        blocks = [self.blocks[e.layer] for e in self.spec.schedule]
+        sizes = [getattr(block, "chain_sizes", None) for block in blocks]
+        # (layers are of few sizes, and an eager step pays for whatever is asked of each)
+        takes = {s: kernels.chain_applies(rows, *s[:3], dtype=self.dtype) and kernels.chain_wins(rows, s[0], s[2], self.dtype) for s in set(sizes) - {None}}
+        return {at: s for at, s in enumerate(sizes) if s is not None and takes[s] and blocks[at].chain_ready}
+
+    def step_room_bytes(self, rows: int) -> int:
+        """What the chains of a step of ``rows`` leave for each other, all layers' at once (``kernels.ChainRoom``): a captured step keeps it."""
+        return 4 * sum(kernels.chain_room_words(rows, self.dtype, s[0], s[2]) for s in self._chain_places(rows).values())
+
     def _chains(self, rows: int, batch, cache) -> dict:
         """{place in the schedule: (room for its chain of products, (norm, first projection, attention or None) of the layer behind it or None)} of a
         step of ``rows``."""
-        if rows > kernels.CHAIN_ROWS:
-            return {}
         schedule = self.spec.schedule
-        sizes = [getattr(self.blocks[e.layer], "chain_sizes", None) for e in schedule]
-        # (layers are of few sizes, and an eager step pays for whatever is asked of each)
-        takes = {s: kernels.chain_applies(rows, *s[:3], dtype=self.dtype) and kernels.chain_wins(rows, s[0], s[2], self.dtype) for s in set(sizes) - {None}}
-        places = {at for at, s in enumerate(sizes) if s is not None and takes[s] and self.blocks[schedule[at].layer].chain_ready}
+        places = self._chain_places(rows)
         if not places:
             return {}
         follows = {}
         behind: dict = {}
-        for at in sorted(places):
+        for at in places:
             if at + 1 not in places or schedule[at + 1].add_embedding:
                 continue
-            pair = (*sizes[at][:3], sizes[at + 1][3])
+            pair = (*places[at][:3], places[at + 1][3])
             if pair not in follows:
                 follows[pair] = kernels.chain_applies(rows, *pair, dtype=self.dtype)
             if follows[pair]:
@@ -277,9 +286,9 @@ class DecoderModel:
                     _, pages, own = self._cache_keys(schedule[at + 1])
                     attention = block.mixer.chain_attention(batch, cache.layer_view(pages, batch), own)
                 behind[at] = block.norm1, block.mixer.chain_products[0], attention
-        room = kernels.ChainRoom(rows, [(sizes[at][0], sizes[at][2], *((behind[at][2].columns,) if at in behind and behind[at][2] is not None else ()))
-                                        for at in sorted(places)], self.device, self.dtype)
-        return {at: (layer_room, behind.get(at)) for at, layer_room in zip(sorted(places), room.layers)}
+        room = kernels.ChainRoom(rows, [(s[0], s[2], *((behind[at][2].columns,) if at in behind and behind[at][2] is not None else ()))
+                                        for at, s in places.items()], self.device, self.dtype)
+        return {at: (layer_room, behind.get(at)) for at, layer_room in zip(places, room.layers)}
 
     # -- the forward pass of one step -------------------------------------------------
 

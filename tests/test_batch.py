@@ -155,6 +155,40 @@ def test_only_models_whose_layers_go_by_near_contexts_capture_a_shape_for_each(m
     assert play(shares_by_near_context=True) == ([100, 300, 900], 3, 9)        # (bounds of 128, 512 and 1,024)
 
 
+def test_captured_shapes_are_given_back_by_the_room_that_their_chains_keep(monkeypatch):
+    """Steps of few rows may each keep hundreds of kilobytes a row (``step_room_bytes``): the captures that have gone longest without a step go when all of them hold more
+    than SHAPE_GRAPH_ROOM_KEPT, those without such room only for their rows."""
+    from types import SimpleNamespace
+
+    from paged_llm_rs_amd.engine import step
+
+    class Graph:
+        def __init__(self, model, cache, entries, widths, ctx_bound, rows, short_bounds):
+            self.rows = rows
+
+        def run(self, entries):
+            return "replayed"
+
+    monkeypatch.setattr(step, "run_step", lambda *args, **kw: "eager")
+    monkeypatch.setattr(step, "ShapeGraph", Graph)
+    cache = SimpleNamespace(manager=SimpleNamespace(table=lambda seq, group: []), layout=SimpleNamespace(groups=[]), clear_state_slots=None)
+
+    def kept(counts, **model):
+        runner = step.StepRunner(SimpleNamespace(device="cpu", portion_limits=(), **model), cache)
+        for count in counts:
+            for _ in range(2):
+                runner.run([StepEntry(i + 1, [0] * 2, 0, [1]) for i in range(count)])
+        return [(k[0], k[1]) for k, g in runner._shapes.items() if g is not None]
+
+    many = [(16 if 2 * n <= 16 else 32 if 2 * n <= 32 else 64, n) for n in range(1, 33)]
+    assert kept(range(1, 33)) == many
+    # (room for eight captures of 64 rows)
+    monkeypatch.setattr(step, "SHAPE_GRAPH_ROOM_KEPT", 8 * 64 * 1000)
+    assert kept(range(1, 33), step_room_bytes=lambda rows: 1000 * rows) == many[-8:]
+    assert kept([40, *range(1, 33)], step_room_bytes=lambda rows: 1000 * rows if rows <= 64 else 0) == [(128, 40), *many[-8:]]
+    assert kept(range(1, 33), step_room_bytes=lambda rows: 10 ** 9) == many[-1:]
+
+
 def test_a_captured_step_is_not_replayed_for_contexts_past_its_near_bound(monkeypatch):
     """The near bound chooses a kernel that holds no longer contexts.  A model whose layers do not say that they go by it has none in its captured steps; one whose layers do is refused
     a replay for contexts past the captured ones, whatever the shape says."""
