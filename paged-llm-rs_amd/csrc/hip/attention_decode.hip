@@ -29,9 +29,12 @@ paged_attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, bf16_t
                               int nkv, int d, float scale_log2e, int window, int splits, int tiles, int g,
                               uint32_t splits_magic, ad_fuse_t fuse, int* __restrict__ arrivals, ad_extras_t<EX> extras) {
     extern __shared__ float lds[];
-    ad_attend<LPK, GT, U, WV, EX, false>(q, q_stride, out, part_acc, part_ml, positions, seq_of, q_len, short_limit, num_seqs, block_table, max_blocks,
-                                         block_size, k_pool, v_pool, nq, nkv, d, scale_log2e, window, splits, tiles, g, splits_magic, fuse, arrivals,
-                                         extras, blockIdx.x, blockIdx.y, blockIdx.z, lds, ad_rows_t{false, 0, nullptr});
+    constexpr bool WAITS = false;
+    constexpr ad_rows_t rows_of{false, 0, nullptr};
+    const int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+#define AD_DONE(done) return
+#include "attention_decode_body.hpp"
+#undef AD_DONE
 }
 
 // Merges the splits of one (token, query head): out = sum_s a_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).
