@@ -181,6 +181,10 @@ class DecoderModel:
     # a row of the step before: the runner and the engine may then queue a decoding step before the host has read
     # the tokens of the one before.  (A model class without the attribute, or with False, is stepped the ordinary way.)
     takes_fed_tokens = True
+    # Whether layers run as chains of products where those are the faster way (``_chain_places``).  A chain's workgroups hold the chip while they wait for
+    # each other, so a program that keeps several engines busy on one card may set its models' to False, before their first step (a captured
+    # step stays as it was captured).
+    chains = True
 
     def __init__(self, spec, params: dict, dtype: torch.dtype, device):
         self.spec = spec
@@ -252,7 +256,7 @@ class DecoderModel:
 
     def _chain_places(self, rows: int) -> dict:
         """{place in the schedule: sizes} of the layers whose products are a chain in a step of ``rows``."""
-        if rows > kernels.CHAIN_ROWS:
+        if not self.chains or rows > kernels.CHAIN_ROWS:
             return {}
         blocks = [self.blocks[e.layer] for e in self.spec.schedule]
         sizes = [getattr(block, "chain_sizes", None) for block in blocks]

@@ -172,6 +172,28 @@ def test_chains_beside_layers_that_are_none(toys, dtype, monkeypatch):
         assert not same or not other, f"other bits at {other}"
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_model_without_chains_gives_the_same_bits(toys, dtype, monkeypatch):
+    """Told not to, a model runs no chain, eagerly or captured; nor does one in bfloat16 that keeps no strips."""
+    from paged_llm_rs_amd.engine.replay import Replayer
+
+    cfg, folder = toys(dtype)
+    prompts = ru.make_prompts(cfg["vocab_size"], [30], seed=2)
+    steps = ru.tail_decoded(prompts, 12)
+    want = _replay(folder, dtype, steps, prompts, 1)
+    with monkeypatch.context() as m:
+        seen = _watch(m)
+        r = Replayer(folder, dtype, max_tokens=64, block_size=8, max_live=2)
+        r.model.chains = False
+        got = ru.collect(r, steps)
+        assert not seen["chains"] and r.model.step_room_bytes(16) == 0
+        assert got.keys() == want.keys() and all((row == want[key]).all() for key, row in got.items())
+        if dtype == "bfloat16":
+            _replay(folder, dtype, steps, prompts, 1, strips=False)
+            assert not seen["chains"]
+    assert Replayer(folder, dtype, max_tokens=64, block_size=8, max_live=2).model.step_room_bytes(16) > 0
+
+
 @pytest.mark.parametrize("hidden,inter,chained", [(1024, 192, True), (1024, 3072, True), (1024, 2560, False), (960, 2048, True), (512, 192, False)])
 def test_which_32_bit_steps_of_one_token_are_chains(tmp_path, monkeypatch, hidden, inter, chained):
     """Of a single row a chain is not the faster way at every size that it takes (``kernels.chain_wins``); of eight it is.  Same bits."""
