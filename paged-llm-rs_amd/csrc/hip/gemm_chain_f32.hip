@@ -279,7 +279,7 @@ __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(c
             if (i < a.stages && static_cast<int>(blockIdx.x) >= a.s[i].first) stage = i;
         return stage;
     };
-    if (threadIdx.x == 0) lds.late[0] = lds.late[1] = 0;
+    if (threadIdx.x < 2) lds.late[threadIdx.x] = 0;
     __syncthreads();
     int p = stage_of(a), q = static_cast<int>(blockIdx.x) - a.s[p].first;
     bool trust = false, own = true;     // (own: tile q of stage p is the workgroup's, and not one that it works out because it is missing)
