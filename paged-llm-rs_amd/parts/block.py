@@ -15,7 +15,8 @@ import torch
 
 from .. import kernels
 from ..errors import ConfigError
-from .norm import PendingNorm, bare_decls, bare_params
+from .linear import Linear
+from .norm import PendingNorm, RmsNorm, bare_decls, bare_params
 from .registry import (BLOCKS, FEED_FORWARDS, MIXERS, NORMS, lookup, prefixed, register_block, scoped)
 
 
@@ -93,12 +94,15 @@ class PreNormBlock:
         if ours is None or theirs is None:
             return None
         first, out = ours
+        # (a chain reads their weights and never calls them: a product of another class keeps its own way)
+        if not type(first) is type(out) is type(theirs[0]) is type(theirs[1]) is Linear:
+            return None
         return out.out_features, out.in_features, theirs[1].in_features, first.out_features
 
     @property
     def chain_ready(self) -> bool:
         """Of a layer with ``chain_sizes``: no biases, and weights and gains that a chain reads (``Linear.chain_weight``)."""
-        if not all(getattr(n, "fuses_into_product", False) for n in (self.norm1, self.norm2)):
+        if not all(getattr(n, "fuses_into_product", False) and type(n).apply is RmsNorm.apply for n in (self.norm1, self.norm2)):
             return False
         linears = (*self.mixer.chain_products, *self.feed_forward.chain_products[:2])
         return all(l.bias is None and l.chain_weight is not None for l in linears) and kernels.in_pieces(
