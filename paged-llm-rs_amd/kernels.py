@@ -1221,14 +1221,17 @@ def chain_applies(rows: int, width: int, inner: int, ff: int, after: int = 0, dt
 
 # Where a chain beats the same products a launch each, timed as decoding steps and short prompts of 28 layers (products apart over a chain, 16 shapes of
 # streams of 32 to 1,024).  In bfloat16 at all of them, from 1 row (1.15 to 1.24, with the attention behind it up to 1.52) to 64 (1.03 to 1.36).  In 32 bits from 8 rows on
-# (1.00 to 1.30; 512 wide with 1,536, 12 tokens of a prompt, 0.99 to 1.01).  With fewer a launch apart has little to do, and a chain gains on wider streams and where a feed-forward's
-# parts of K are 64 or 128 values long (1 row: 576 with 1,536 1.01, 960 with 2,048 1.03, 1,024 with 1,024 1.06) or all whole (1,024 with 3,072 1.03);
-# in parts of 192 that are not it loses at 1 and 2 rows (704 with 2,560 0.95, 960 with 2,560 0.95 and 0.99, 1,024 with 2,560 0.97 and 1.01) and at 4 on streams
-# below 768 (704 0.99, 768 1.01, 960 1.02), and at 512 wide up to 4 rows (0.95 to 1.01).
+# (1.00 to 1.30; 512 wide with 1,536, 12 tokens of a prompt, 0.99 to 1.01).  With fewer a launch apart has little to do, and a chain gains on wider streams and where a
+# feed-forward's parts of K (sixteen, in steps of 64 values) are 64 or 128 values long (from 576 wide on, feed-forwards of 1,024 to 2,048: 1 row 0.98 to 1.06, 2 rows 1.01
+# to 1.03, 4 rows 1.02 to 1.05), or where stream and feed-forward are whole parts, which the kernel's forms without bounds take (1,024 with 3,072, rows 1, 2, 4: 1.02, 1.07, 1.09).
+# In parts of 192 beside a stream that is not whole parts, or not whole themselves, it loses at 1 and 2 rows (576 to 960 with 3,072 0.94 to 0.98 and 0.98 to 1.01; with
+# 2,560 0.95 to 0.99 and 0.98 to 1.04; 1,024 with 2,560 and 2,816 0.97 and 1.01 to 1.03), at 4 rows on streams below 768 (0.99 to 1.00; from there on 0.98 to 1.07,
+# at 6 rows 1.07 to 1.14), and at 512 wide up to 4 rows (0.95 to 1.01).
 CHAIN_F32_ROWS = 8
 CHAIN_F32_NARROW = 512
 CHAIN_F32_LONG = 2048           # the feed-forward beyond which parts are 192 values
 CHAIN_F32_LONG_ROWS, CHAIN_F32_LONG_WIDTH = 4, 768
+CHAIN_F32_WHOLE = 1024          # sixteen parts of 64
 
 
 def chain_wins(rows: int, width: int, ff: int, dtype: torch.dtype = torch.bfloat16) -> bool:
@@ -1237,7 +1240,8 @@ def chain_wins(rows: int, width: int, ff: int, dtype: torch.dtype = torch.bfloat
         return True
     if width <= CHAIN_F32_NARROW:
         return False
-    return ff <= CHAIN_F32_LONG or (width, ff) == (1024, 3072) or (rows >= CHAIN_F32_LONG_ROWS and width >= CHAIN_F32_LONG_WIDTH)
+    whole = width % CHAIN_F32_WHOLE == 0 and ff % CHAIN_F32_WHOLE == 0
+    return ff <= CHAIN_F32_LONG or whole or (rows >= CHAIN_F32_LONG_ROWS and width >= CHAIN_F32_LONG_WIDTH)
 
 
 def chain_room_words(rows: int, dtype: torch.dtype, width: int, ff: int, attended: int = 0) -> int:
