@@ -45,7 +45,8 @@
 // The arithmetic is gemm_skinny's for one tile of rows, to the same bits: K in as many stretches as that launch has waves (a
 // wave here takes up to four of them, each an accumulator of its own), the stretches' tiles added in their order.  As there, the norms in front
 // of stages 1 and 3 are taken from the 32-bit stream below CN_HANDED rows, and from there on handed forward: the stage that adds
-// into the stream leaves bf16(stream * gain) and the sums of squares of its 16 columns.
+// into the stream leaves bf16(stream * gain) and the sums of squares of its 16 columns.  (Of more than 32 rows over many columns the launches apart are
+// another kernel, which adds its sums in another order: then a result here is the neighbouring bfloat16 now and then.)
 #include "attention_decode.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -390,8 +391,9 @@ __device__ __forceinline__ int cn_missing_place(const __attribute__((address_spa
     return found == INT_MAX ? -1 : (found + from) % s.tiles;
 }
 
-// 256 registers a lane, two workgroups a compute unit: the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
-// first three stages of the 0.6B shape and most of the 256 of the last).
+// 256 registers a lane, two workgroups a compute unit: without attention the first 512 workgroups hold their weights at once (64 + 192 + 64 of the
+// first three stages of the 0.6B shape and most of the 256 of the last).  With it, its workgroups have those places before the last stage's: one token's
+// 64 leave 128 of the 256 a place, the 256 of four or eight tokens none until earlier workgroups end.
 template <bool HANDED, bool ATTENDS>
 __global__ void __launch_bounds__(PL_WAVE * CN_WAVES, 2) gemm_chain_kernel(cn_chain_t a, cn_attend_of<ATTENDS>) {
     __shared__ __attribute__((aligned(16))) float red[2 * CN_STRETCHES * 256];      // [stretch][gate, up][256] partial tiles

@@ -268,7 +268,8 @@ __device__ __forceinline__ int cf_missing_tile(const __attribute__((address_spac
     return found == INT_MAX ? -1 : (found + from) % s.tiles;
 }
 
-// 128 registers a lane: two workgroups a compute unit, half of a layer's weights in registers at once.
+// 128 registers a lane: two workgroups a compute unit, half of a layer's weights in registers at once.  (Two values do not fit: 12 bytes of
+// scratch a lane.)
 __global__ void __launch_bounds__(PL_WAVE * CF_WAVES, 4) gemm_chain_f32_kernel(cf_chain_t a) {
     __shared__ __attribute__((aligned(16))) cf_lds_t lds;
     cn_touch_arguments(sizeof(cf_chain_t));
